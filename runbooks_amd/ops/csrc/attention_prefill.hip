@@ -1,216 +1,246 @@
 // Flash-attention prefill (causal, GQA/MQA, bf16) for CDNA4 (gfx950).
 //
-// MFMA-native design following the CDNA4 attention recipe:
-//  * workgroup = 8 waves; each wave owns 32 query rows (WG tile = 256).
-//  * KV tiles of 64 keys staged to LDS; K row-major, V TRANSPOSED
-//    ([d][key]) so both QK^T and PV read 16 B/lane fragments. Rows padded
-//    +16 B so the b128 column-slice reads are bank-conflict-free
-//    (stride/4 mod 64 cycles through distinct banks; no XOR swizzle).
-//  * swapped QK^T: mfma(A=K, B=Q) so the C layout has qrow = lane&31 —
-//    the whole softmax row lives on a lane pair (l, l^32); row max is a
-//    16-reg in-lane reduce + one shfl_xor(32).
-//  * online softmax in registers; P repacked to PV A/B fragments with
-//    v_cvt (compiler) + v_permlane32_swap (half exchange).
-//  * PV: mfma(A=V^T, B=P^T) accumulating O^T in 16-reg tiles.
+// A workgroup is NW waves of 32 query rows each; tiles of 64 keys and values
+// (flash_tile.h) stand in two LDS buffers, the next one on its way while one
+// is worked on: one barrier per tile.
 //
-// mfma_f32_32x32x16_bf16 layouts (cdna_hip_programming.md §3):
+//  * S^T = K Q^T: a lane pair (l, l ^ 32) holds the scores of one query, so a
+//    row's maximum is an in-lane reduction and one shuffle.
+//  * Online softmax in base 2; the running maximum moves only when a row
+//    exceeds it by a factor of 2^8, so the accumulators are rarely rescaled
+//    (sums and result refer to the same maximum, whichever it is).
+//  * O^T += V^T P^T: the transposed reads of V take the keys in the order of
+//    the scores' registers, which are then the other operand as they are.
+//
+// What bounds it: the matrix cores and the softmax's vector instructions in
+// turn (per 64 x 32 scores of 128 columns 32 MFMA of 32 cycles, and about as
+// long in vector instructions); two waves per SIMD overlap them. Measured, one
+// prompt, before (tiles staged through registers between two barriers) and now:
+//   7931 tokens, 32 query and 8 kv heads of 128    1554 -> 484 us, 1065 TF/s
+//   3001 tokens, the same                           331 ->  88 us,  842 TF/s
+//   512 tokens, 32 heads of 128                      43 ->  13 us
+//   1021 tokens, 16 heads of 256                    133 ->  36 us
+//   4000 tokens, 32 heads of 64                     288 ->  89 us,  737 TF/s
+//
+// mfma_f32_32x32x16_bf16 layouts:
 //   A[i][k]: i = lane&31, k = (lane>>5)*8 + e (e = 0..7)
 //   C[i][j]: j = lane&31, i = (reg&3) + 8*(reg>>2) + 4*(lane>>5)
 //
-// q,k,v,out: [B, S, H, DH] bf16 token-major. DH in {64, 128}.
+// q,k,v,out: [B, S, H, DH] bf16 token-major. DH in {64, 128, 256}.
 
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
-#include "common.h"
+#include <algorithm>
+#include <type_traits>
+
+#include "flash_tile.h"
 
 namespace {
 
-constexpr int BLOCK = 512;   // 8 waves
-constexpr int KVB = 64;      // keys per LDS tile
+using namespace flash;
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8v;
-typedef __attribute__((ext_vector_type(16))) float f32x16v;
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr float RISE = 8.0f;           // of a maximum before it is moved
 
-RB_DEV unsigned pack_bf16(float lo, float hi) {
-  union { __bf16 b; unsigned short u; } a, b;
-  a.b = (__bf16)lo;
-  b.b = (__bf16)hi;
-  return ((unsigned)b.u << 16) | a.u;
-}
-
-RB_DEV bf16x8v frag_from_words(unsigned w0, unsigned w1, unsigned w2, unsigned w3) {
-  union { unsigned u[4]; bf16x8v v; } c;
-  c.u[0] = w0; c.u[1] = w1; c.u[2] = w2; c.u[3] = w3;
-  return c.v;
-}
-
-template <int DH>
-__global__ __launch_bounds__(BLOCK, 2) void flash_prefill_kernel(
+// SPLIT 2: two waves share 32 query rows, one takes the lower and one the upper
+// 32 keys of every tile; their results meet in LDS at the end.
+template <int DH, int NW, int SPLIT>
+__global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kernel(
     const uint16_t *__restrict__ qp, const uint16_t *__restrict__ kp,
     const uint16_t *__restrict__ vp, uint16_t *__restrict__ op,
     float *__restrict__ lsep,  // [B, Hq, S] log-sum-exp for training bwd
     int B, int S, int Hq, int Hkv, float scale) {
   constexpr int KSTEPS = DH / 16;       // QK^T contraction steps
   constexpr int DTILES = DH / 32;       // O column tiles
-  constexpr int K_STRIDE = DH * 2 + 16; // K row bytes (+16 pad)
-  constexpr int V_STRIDE = KVB * 2 + 16;  // V^T row bytes (+16 pad)
+  constexpr int QT = NW / SPLIT * 32;
+  constexpr int TILE = tile_bytes<DH>();
 
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  char *k_img = smem;                       // [KVB][K_STRIDE]
-  char *v_img = smem + KVB * K_STRIDE;      // [DH][V_STRIDE]
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
 
   const int tid = threadIdx.x;
-  const int wid = tid >> 6;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int hi = lane >> 5;
   const int col = lane & 31;                // qrow within the wave tile
 
-  const int q0 = blockIdx.x * 256;
-  const int h = blockIdx.y;
-  const int b = blockIdx.z;
+  const Place at = place(blockIdx.x, (S + QT - 1) / QT, Hq, Hkv, B, true);
+  const int q0 = at.tile * QT, h = at.head, b = at.batch;
   const int h_kv = h / (Hq / Hkv);
-  const int qrow = q0 + wid * 32 + col;     // this lane's query row
+  const int group = wid / SPLIT, part = wid % SPLIT;
+  const int wrow = q0 + group * 32;
+  const int qrow = wrow + col;              // this lane's query row
   const bool q_valid = qrow < S;
 
-  // ---- Q fragments (B operand of swapped QK^T), pre-scaled --------------
+  const int64_t kv_stride = (int64_t)Hkv * DH;
+  const uint16_t *kb = kp + ((int64_t)b * S * Hkv + h_kv) * DH;
+  const uint16_t *vb = vp + ((int64_t)b * S * Hkv + h_kv) * DH;
+  const TileLoad<DH, NW> load(wid, lane);
+  const int kv_end = min(S, q0 + QT);       // causal upper bound for this WG
+  const int n_tiles = (kv_end + ROWS - 1) / ROWS;
+  load(kb, kv_stride, 0, S, smem, wid);
+  load(vb, kv_stride, 0, S, smem + TILE, wid);
+
+  // ---- Q fragments (B operand of K Q^T); a factor below zero goes into
+  // their signs, so that scores and their maxima have one order, and a factor
+  // of zero clears them, so that hidden scores stay at minus infinity --------
   bf16x8v qf[KSTEPS];
   {
-    const uint16_t *qrow_p =
-        qp + ((int64_t)(b * S + (q_valid ? qrow : 0)) * Hq + h) * DH;
+    const uint16_t *src = qp + ((int64_t)(b * S + (q_valid ? qrow : 0)) * Hq +
+                                h) * DH + hi * 8;
+    const unsigned flip = scale < 0.0f ? 0x80008000u : 0u;
+    const unsigned keep = scale == 0.0f ? 0u : ~0u;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
-      const uint16_t *src = qrow_p + ks * 16 + hi * 8;
-      float f[8];
-      rb::VIO<uint16_t>::load(src, f);
-      union { unsigned short u[8]; bf16x8v v; } c;
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        c.u[e] = rb::f32_to_bf16(q_valid ? f[e] * scale : 0.0f);
+      union { uint4 u; bf16x8v v; } c;
+      c.u = *reinterpret_cast<const uint4 *>(src + ks * 16);
+      c.u.x = (c.u.x ^ flip) & keep;
+      c.u.y = (c.u.y ^ flip) & keep;
+      c.u.z = (c.u.z ^ flip) & keep;
+      c.u.w = (c.u.w ^ flip) & keep;
       qf[ks] = c.v;
     }
   }
+  // scores -> exponents of 2
+  const float to2 = scale == 0.0f ? 1.0f : fabsf(scale) * LOG2E;
 
   f32x16v acc_o[DTILES];
 #pragma unroll
   for (int dt = 0; dt < DTILES; ++dt) acc_o[dt] = (f32x16v)(0.0f);
-  float m_run = -INFINITY;
+  float m_run = -INFINITY;                  // in exponents of 2
   float l_run = 0.0f;
 
-  const int kv_end = min(S, q0 + 256);      // causal upper bound for this WG
-  const int n_tiles = (kv_end + KVB - 1) / KVB;
-  const int wave_kmax = q0 + wid * 32 + 31; // last key this wave can see
-
-  for (int kt = 0; kt < n_tiles; ++kt) {
-    const int kbase = kt * KVB;
-
-    // ---- stage K tile: [key][d] rows, each thread 16 elems ---------------
-    {
-      const int per_pass = BLOCK * 8;       // elems per pass
-      constexpr int total = KVB * DH;
+  // Keys kbase .. kbase + 32 SUB - 1 of the tile, from row r0 on; `masked`:
+  // some of them are hidden from some row
+  constexpr int SUB = DH == 256 || SPLIT == 2 ? 1 : 2;
+  auto keys = [&](const char *kt, const char *vt, int kbase, int r0,
+                  auto masked) {
+    f32x16v s[SUB];
 #pragma unroll
-      for (int p = 0; p < total / (BLOCK * 8); ++p) {
-        const int idx = p * per_pass + tid * 8;
-        const int key = idx / DH;
-        const int d0 = idx % DH;
-        const int gk = kbase + key;
-        rb::bf16x8 val;
-        if (gk < S) {
-          val = *reinterpret_cast<const rb::bf16x8 *>(
-              kp + ((int64_t)(b * S + gk) * Hkv + h_kv) * DH + d0);
-        } else {
+    for (int u = 0; u < SUB; ++u) {
+      s[u] = (f32x16v)(0.0f);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) val.v[e] = 0;
-        }
-        *reinterpret_cast<rb::bf16x8 *>(k_img + key * K_STRIDE + d0 * 2) = val;
-      }
+      for (int ks = 0; ks < KSTEPS; ++ks)
+        s[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            row_frag<DH>(kt, r0 + u * 32, ks, col, hi), qf[ks], s[u], 0, 0, 0);
     }
-    // ---- stage V tile transposed: thread owns column d, KPG keys ---------
-    {
-      constexpr int GRPS = BLOCK / DH;      // thread groups over keys
-      constexpr int KPG = KVB / GRPS;       // keys per group (16 @DH=128)
-      const int d = tid % DH;
-      const int kg0 = (tid / DH) * KPG;
-      uint16_t tmp[KPG];
+    if constexpr (decltype(masked)::value) {
 #pragma unroll
-      for (int e = 0; e < KPG; ++e) {
-        const int gk = kbase + kg0 + e;
-        tmp[e] = (gk < S)
-            ? vp[((int64_t)(b * S + gk) * Hkv + h_kv) * DH + d]
-            : (uint16_t)0;
-      }
-#pragma unroll
-      for (int c8 = 0; c8 < KPG / 8; ++c8)
-        *reinterpret_cast<rb::bf16x8 *>(v_img + d * V_STRIDE + (kg0 + c8 * 8) * 2) =
-            *reinterpret_cast<rb::bf16x8 *>(&tmp[c8 * 8]);
-    }
-    __syncthreads();
-
-    if (kbase <= wave_kmax) {
-      // two 32-key sub-tiles per LDS tile
-#pragma unroll
-      for (int it = 0; it < 2; ++it) {
-        // ---- QK^T^T: scores[key][qrow] ----------------------------------
-        f32x16v s = (f32x16v)(0.0f);
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks) {
-          const bf16x8v kf = *reinterpret_cast<const bf16x8v *>(
-              k_img + (it * 32 + col) * K_STRIDE + (ks * 16 + hi * 8) * 2);
-          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], s, 0, 0, 0);
-        }
-
-        // ---- mask + online softmax --------------------------------------
-        float p[16];
-        float mx = -INFINITY;
+      for (int u = 0; u < SUB; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int key = kbase + it * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
-          p[r] = (key <= qrow) ? s[r] : -INFINITY;
-          mx = fmaxf(mx, p[r]);
+          const int key = kbase + u * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
+          if (key > qrow) s[u][r] = -INFINITY;
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));     // full row max
-        const float mn = fmaxf(m_run, mx);
-        if (mn != -INFINITY) {
-          const float alpha = (m_run == -INFINITY) ? 0.0f : __expf(m_run - mn);
-          float psum = 0.0f;
+    }
+    float mx = s[0][0];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            p[r] = (p[r] == -INFINITY) ? 0.0f : __expf(p[r] - mn);
-            psum += p[r];
-          }
-          l_run = l_run * alpha + psum;
-          m_run = mn;
-          if (alpha != 1.0f) {
+    for (int u = 0; u < SUB; ++u)
 #pragma unroll
-            for (int dt = 0; dt < DTILES; ++dt)
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[u][r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * to2;
+    if (__any(mx > m_run + RISE)) {
+      const float mn = fmaxf(m_run, mx);
+      // rows that have seen no finite score keep a finite reference
+      const float alpha = __builtin_amdgcn_exp2f(
+          m_run - (mn == -INFINITY ? 0.0f : mn));
+      l_run *= alpha;
 #pragma unroll
-              for (int r = 0; r < 16; ++r) acc_o[dt][r] *= alpha;
-          }
-
-          // ---- P -> bf16 B-fragments via permlane half-exchange ---------
+      for (int dt = 0; dt < DTILES; ++dt)
 #pragma unroll
-          for (int kslot = 0; kslot < 2; ++kslot) {
-            const int r0 = kslot * 8;
-            unsigned pk0 = pack_bf16(p[r0 + 0], p[r0 + 1]);
-            unsigned pk1 = pack_bf16(p[r0 + 2], p[r0 + 3]);
-            unsigned pk2 = pack_bf16(p[r0 + 4], p[r0 + 5]);
-            unsigned pk3 = pack_bf16(p[r0 + 6], p[r0 + 7]);
-            auto r02 = __builtin_amdgcn_permlane32_swap(pk0, pk2, false, false);
-            auto r13 = __builtin_amdgcn_permlane32_swap(pk1, pk3, false, false);
-            const bf16x8v pf = frag_from_words(r02[0], r13[0], r02[1], r13[1]);
-            const int koff = (it * 32 + kslot * 16 + hi * 8) * 2;
+        for (int r = 0; r < 16; ++r) acc_o[dt][r] *= alpha;
+      m_run = mn;
+    }
+    const float ref = m_run == -INFINITY ? 0.0f : m_run;
 #pragma unroll
-            for (int dt = 0; dt < DTILES; ++dt) {
-              const bf16x8v vf = *reinterpret_cast<const bf16x8v *>(
-                  v_img + (dt * 32 + col) * V_STRIDE + koff);
-              acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                  vf, pf, acc_o[dt], 0, 0, 0);
-            }
-          }
-        }
+    for (int u = 0; u < SUB; ++u) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        s[u][r] = __builtin_amdgcn_exp2f(fmaf(s[u][r], to2, -ref));
+        l_run += s[u][r];
+      }
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        union { unsigned u[4]; bf16x8v v; } pf;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          pf.u[i] = pack2(s[u][ks * 8 + 2 * i], s[u][ks * 8 + 2 * i + 1]);
+#pragma unroll
+        for (int dt = 0; dt < DTILES; ++dt)
+          acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              column_frag<DH>(vt, r0 + u * 32 + ks * 16, dt, lane), pf.v,
+              acc_o[dt], 0, 0, 0);
       }
     }
+  };
+
+  // waits for tile t and sends for the next one
+  auto arrive = [&](int t) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();                    // nobody reads the other buffer any more
+    if (t + 1 < n_tiles) {
+      char *next = smem + (~t & 1) * 2 * TILE;
+      load(kb, kv_stride, (t + 1) * ROWS, S, next, wid);
+      load(vb, kv_stride, (t + 1) * ROWS, S, next + TILE, wid);
+    }
+  };
+  // first all-visible tiles, then those on the diagonal, then those that only
+  // other waves need
+  const int full = wrow / ROWS;
+  int t = 0;
+  for (; t < full; ++t) {
+    arrive(t);
+    const char *kt = smem + (t & 1) * 2 * TILE;
+#pragma unroll
+    for (int i = 0; i < ROWS; i += SUB * 32 * SPLIT)
+      keys(kt, kt + TILE, t * ROWS + i + part * 32, i + part * 32,
+           std::false_type{});
+  }
+  for (; t < n_tiles; ++t) {
+    arrive(t);
+    const char *kt = smem + (t & 1) * 2 * TILE;
+#pragma unroll
+    for (int i = 0; i < ROWS; i += SUB * 32 * SPLIT) {
+      const int r0 = i + part * 32, kbase = t * ROWS + r0;
+      if (kbase <= wrow + 31)
+        keys(kt, kt + TILE, kbase, r0, std::true_type{});
+    }
+  }
+
+  if constexpr (SPLIT == 2) {
+    // lane-major pieces of 16 bytes: the result, maximum and sum of part 1
+    constexpr int PIECES = DTILES * 4;
+    static_assert(PIECES == DH / 8, "merge buffer");
+    float4 *ex = reinterpret_cast<float4 *>(smem) +
+                 group * (PIECES + 1) * 64 + lane;
+    __syncthreads();                        // the last tile has been read
+    if (part == 1) {
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) {
+        const f32x16v &a = acc_o[i / 4];
+        ex[i * 64] = make_float4(a[i % 4 * 4], a[i % 4 * 4 + 1],
+                                 a[i % 4 * 4 + 2], a[i % 4 * 4 + 3]);
+      }
+      ex[PIECES * 64] = make_float4(m_run, l_run, 0.0f, 0.0f);
+    }
     __syncthreads();
+    if (part == 1) return;
+    const float4 ml = ex[PIECES * 64];
+    const float mn = fmaxf(m_run, ml.x);
+    const float ref = mn == -INFINITY ? 0.0f : mn;
+    const float f0 = __builtin_amdgcn_exp2f(m_run - ref);
+    const float f1 = __builtin_amdgcn_exp2f(ml.x - ref);
+    l_run = l_run * f0 + ml.y * f1;
+    m_run = mn;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const float4 o = ex[i * 64];
+      f32x16v &a = acc_o[i / 4];
+      a[i % 4 * 4] = a[i % 4 * 4] * f0 + o.x * f1;
+      a[i % 4 * 4 + 1] = a[i % 4 * 4 + 1] * f0 + o.y * f1;
+      a[i % 4 * 4 + 2] = a[i % 4 * 4 + 2] * f0 + o.z * f1;
+      a[i % 4 * 4 + 3] = a[i % 4 * 4 + 3] * f0 + o.w * f1;
+    }
   }
 
   // ---- epilogue: O^T regs -> out[b, qrow, h, :] ---------------------------
@@ -219,25 +249,79 @@ __global__ __launch_bounds__(BLOCK, 2) void flash_prefill_kernel(
     const float inv_l = (l_full > 0.0f) ? 1.0f / l_full : 0.0f;
     if (lsep != nullptr && hi == 0)
       lsep[((int64_t)b * Hq + h) * S + qrow] =
-          (l_full > 0.0f) ? m_run + __logf(l_full) : -INFINITY;
+          (l_full > 0.0f) ? m_run / LOG2E + __logf(l_full) : -INFINITY;
     uint16_t *orow = op + ((int64_t)(b * S + qrow) * Hq + h) * DH;
 #pragma unroll
     for (int dt = 0; dt < DTILES; ++dt) {
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq) {
-        const int d0 = dt * 32 + 8 * rq + 4 * hi;
-        uint16_t w[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          w[e] = rb::f32_to_bf16(acc_o[dt][rq * 4 + e] * inv_l);
-        *reinterpret_cast<uint2 *>(orow + d0) =
-            *reinterpret_cast<const uint2 *>(w);
+        uint2 w;
+        w.x = pack2(acc_o[dt][rq * 4] * inv_l, acc_o[dt][rq * 4 + 1] * inv_l);
+        w.y = pack2(acc_o[dt][rq * 4 + 2] * inv_l,
+                    acc_o[dt][rq * 4 + 3] * inv_l);
+        *reinterpret_cast<uint2 *>(orow + dt * 32 + 8 * rq + 4 * hi) = w;
       }
     }
   }
 }
 
+template <int DH, int NW, int SPLIT>
+void launch_prefill(const at::Tensor &q, const at::Tensor &k,
+                    const at::Tensor &v, at::Tensor &out, float *lsep,
+                    float scale) {
+  const int B = (int)q.size(0), S = (int)q.size(1), Hq = (int)q.size(2);
+  constexpr size_t merge =
+      SPLIT == 1 ? 0 : (size_t)NW / SPLIT * (DH / 8 + 1) * 1024;
+  constexpr size_t shmem = std::max((size_t)4 * tile_bytes<DH>(), merge);
+  static const bool once = hipFuncSetAttribute(
+      reinterpret_cast<const void *>(&flash_prefill_kernel<DH, NW, SPLIT>),
+      hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) == hipSuccess;
+  TORCH_CHECK(once, "flash_prefill: LDS size");
+  constexpr int QT = NW / SPLIT * 32;
+  const int64_t grid = (int64_t)((S + QT - 1) / QT) * Hq * B;
+  TORCH_CHECK(grid < (int64_t)1 << 31, "flash_prefill: grid");
+  hipLaunchKernelGGL((flash_prefill_kernel<DH, NW, SPLIT>), dim3((unsigned)grid),
+                     dim3(NW * 64), shmem, at::hip::getCurrentHIPStream(),
+                     (const uint16_t *)q.data_ptr(),
+                     (const uint16_t *)k.data_ptr(),
+                     (const uint16_t *)v.data_ptr(), (uint16_t *)out.data_ptr(),
+                     lsep, B, S, Hq, (int)k.size(2), scale);
+}
+
+template <int DH>
+void launch_prefill(const at::Tensor &q, const at::Tensor &k,
+                    const at::Tensor &v, at::Tensor &out, float *lsep,
+                    float scale) {
+  // Tiles of 32 query rows in all heads: one or two waves each, on 1024 SIMDs.
+  // As long as there are fewer of them than SIMDs, the chain of a tile's keys
+  // is what takes the time, and two waves halve it; small workgroups then use
+  // more CUs. us at 128 columns for <2,2> <4,2> <4,1> <8,1>:
+  //   256 tokens, 32 heads ( 256 tiles)   8.3   9.2  10.4  14.1
+  //   1000 tokens         (1024 tiles)   29.6  21.6  25.6  31.6
+  //   1500 tokens         (1504 tiles)   51.3  34.8  37.4  44.1
+  //   2000 tokens         (2016 tiles)   84.1  56.1  51.9  60.1
+  //   7931 tokens         (7936 tiles)   1098   614   502   484
+  // 256 columns take a SIMD's registers for one wave, so four waves fill a CU
+  // (3000 tokens, 16 heads, 1504 tiles: <4,2> 151, <4,1> 141; with eight, which
+  // spill, 281).
+  const int64_t tiles = (q.size(1) + 31) / 32 * q.size(2) * q.size(0);
+  if constexpr (DH == 256) {
+    if (tiles <= 1280) launch_prefill<DH, 4, 2>(q, k, v, out, lsep, scale);
+    else launch_prefill<DH, 4, 1>(q, k, v, out, lsep, scale);
+  } else {
+    if (tiles <= 512) launch_prefill<DH, 2, 2>(q, k, v, out, lsep, scale);
+    else if (tiles <= 1536) launch_prefill<DH, 4, 2>(q, k, v, out, lsep, scale);
+    else if (tiles < 6144) launch_prefill<DH, 4, 1>(q, k, v, out, lsep, scale);
+    else launch_prefill<DH, 8, 1>(q, k, v, out, lsep, scale);
+  }
+}
+
 }  // namespace
+
+// Contiguous values may start anywhere; the kernels load 16 bytes at a time.
+static at::Tensor aligned16(const at::Tensor &t) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 ? t.clone() : t;
+}
 
 static at::Tensor flash_fwd_impl(at::Tensor q, at::Tensor k, at::Tensor v,
                                  double scale, float *lsep) {
@@ -249,36 +333,19 @@ static at::Tensor flash_fwd_impl(at::Tensor q, at::Tensor k, at::Tensor v,
             DH = (int)q.size(3);
   const int Hkv = (int)k.size(2);
   TORCH_CHECK(Hq % Hkv == 0, "flash_prefill: Hq % Hkv");
+  TORCH_CHECK(k.dim() == 4 && k.size(0) == B && k.size(1) == S &&
+              k.size(3) == DH && v.sizes() == k.sizes() &&
+              k.scalar_type() == at::kBFloat16 &&
+              v.scalar_type() == at::kBFloat16, "flash_prefill: k, v");
   auto out = at::empty_like(q);
-  auto stream = at::hip::getCurrentHIPStream();
-  const dim3 grid((S + 255) / 256, Hq, B);
-
-  if (DH == 128) {
-    constexpr size_t shmem = KVB * (128 * 2 + 16) + 128 * (KVB * 2 + 16);
-    hipLaunchKernelGGL((flash_prefill_kernel<128>), grid, dim3(BLOCK), shmem,
-                       stream, (const uint16_t *)q.data_ptr(),
-                       (const uint16_t *)k.data_ptr(),
-                       (const uint16_t *)v.data_ptr(), (uint16_t *)out.data_ptr(),
-                       lsep, B, S, Hq, Hkv, (float)scale);
-  } else if (DH == 64) {
-    constexpr size_t shmem = KVB * (64 * 2 + 16) + 64 * (KVB * 2 + 16);
-    hipLaunchKernelGGL((flash_prefill_kernel<64>), grid, dim3(BLOCK), shmem,
-                       stream, (const uint16_t *)q.data_ptr(),
-                       (const uint16_t *)k.data_ptr(),
-                       (const uint16_t *)v.data_ptr(), (uint16_t *)out.data_ptr(),
-                       lsep, B, S, Hq, Hkv, (float)scale);
-  } else if (DH == 256) {
-    // gemma-7b wide heads: 70.7 KB LDS, fits; closes the last eager
-    // prefill fallback (round-1 NOTES item).
-    constexpr size_t shmem = KVB * (256 * 2 + 16) + 256 * (KVB * 2 + 16);
-    hipLaunchKernelGGL((flash_prefill_kernel<256>), grid, dim3(BLOCK), shmem,
-                       stream, (const uint16_t *)q.data_ptr(),
-                       (const uint16_t *)k.data_ptr(),
-                       (const uint16_t *)v.data_ptr(), (uint16_t *)out.data_ptr(),
-                       lsep, B, S, Hq, Hkv, (float)scale);
-  } else {
-    TORCH_CHECK(false, "flash_prefill: DH must be 64, 128 or 256, got ", DH);
-  }
+  if (out.numel() == 0) return out;
+  q = aligned16(q);
+  k = aligned16(k);
+  v = aligned16(v);
+  if (DH == 128) launch_prefill<128>(q, k, v, out, lsep, (float)scale);
+  else if (DH == 64) launch_prefill<64>(q, k, v, out, lsep, (float)scale);
+  else if (DH == 256) launch_prefill<256>(q, k, v, out, lsep, (float)scale);
+  else TORCH_CHECK(false, "flash_prefill: DH must be 64, 128 or 256, got ", DH);
   return out;
 }
 

@@ -1,0 +1,111 @@
+// LDS tiles of the flash attention kernels (attention_prefill.hip,
+// attention_bwd.hip): rows of DH bf16 values, loaded straight from memory
+// (global_load_lds, 16 bytes a lane) and read both ways, by rows as MFMA
+// operands along DH and by columns (ds_read_b64_tr_b16) as operands along the
+// rows.
+//
+// Row r's 16-byte chunk c stands at chunk c ^ mix(r). A load writes 64
+// consecutive chunks, so the mixing is done on the address it reads. With it
+// the 16 rows of one chunk, which a row read takes, and the 4 rows of 4
+// chunks, which a column read takes, fall on all 64 banks once.
+#pragma once
+
+#include "common.h"
+
+namespace flash {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8v;
+typedef __attribute__((ext_vector_type(16))) float f32x16v;
+
+constexpr int ROWS = 64;               // of a tile
+
+// one v_cvt_pk_bf16_f32 (two scalar conversions take four instructions)
+RB_DEV unsigned pack2(float lo, float hi) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2v;
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2v;
+  union { bf16x2v b; unsigned u; } c;
+  c.b = __builtin_convertvector((f32x2v){lo, hi}, bf16x2v);
+  return c.u;
+}
+
+template <int DH> RB_DEV constexpr int mix(int row) {
+  return DH == 64 ? ((row >> 1 & 1) << 2) | (row >> 2 & 3)
+                  : ((row & 3) << 2) | (row >> 2 & 3);
+}
+
+template <int DH> constexpr int tile_bytes() { return ROWS * DH * 2; }
+
+// Loads of a tile by NW waves: piece i of wave w is the kilobyte (1024 bytes
+// of LDS) i * NW + w of the tile, STEP rows after the one before; mix() is
+// linear in the bits of a row.
+template <int DH, int NW> struct TileLoad {
+  static constexpr int PIECES = tile_bytes<DH>() / 1024 / NW;
+  static constexpr int CHUNKS = DH / 8;          // of a row
+  static constexpr int STEP = NW * 64 / CHUNKS;
+  int row, off;                                  // of piece 0 (off: elements)
+
+  RB_DEV TileLoad(int wid, int lane) {
+    const int at = wid * 64 + lane;
+    row = at / CHUNKS;
+    off = (at % CHUNKS ^ mix<DH>(row)) * 8;
+  }
+
+  // Rows r0 .. r0 + 63 of `rows` rows, `stride` elements apart from `base`
+  // on; rows past the end are the last one again. `tile` is uniform.
+  RB_DEV void operator()(const uint16_t *base, int64_t stride, int r0,
+                         int rows, char *tile, int wid) const {
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const uint16_t *p =
+          base + (int64_t)min(r0 + row + i * STEP, rows - 1) * stride +
+          (off ^ mix<DH>(i * STEP) * 8);
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) uint32_t *)(const void *)p,
+          (__attribute__((address_space(3))) uint32_t *)(void *)(
+              tile + (i * NW + wid) * 1024), 16, 0, 0);
+    }
+  }
+};
+
+// Operand of rows r0 .. r0 + 31 along columns 16 ks .. 16 ks + 15: element e
+// of lane (hi, col) is row r0 + col, column 16 ks + 8 hi + e. r0 % 16 == 0.
+template <int DH>
+RB_DEV bf16x8v row_frag(const char *tile, int r0, int ks, int col, int hi) {
+  return *reinterpret_cast<const bf16x8v *>(
+      tile + (r0 + col) * (DH * 2) + ((ks * 2 + hi) ^ mix<DH>(col)) * 16);
+}
+
+// Operand of columns 32 dt .. 32 dt + 31 along rows r0 .. r0 + 15, in the order
+// of a score tile's registers: element e of lane (hi, col) is column
+// 32 dt + col, row r0 + 8 (e / 4) + 4 hi + e % 4. r0 % 16 == 0.
+template <int DH>
+RB_DEV bf16x8v column_frag(const char *tile, int r0, int dt, int lane) {
+  const int i = lane & 15, hi = lane >> 5;
+  const int r = 4 * hi + (i >> 2);
+  const int chunk = dt * 4 + (lane >> 4 & 1) * 2 + (i >> 1 & 1);
+  const char *lo = tile + (r0 + r) * (DH * 2) +
+                   (chunk ^ mix<DH>(r)) * 16 + (i & 1) * 8;
+  const char *up = tile + (r0 + r + 8) * (DH * 2) +
+                   (chunk ^ mix<DH>(r + 8)) * 16 + (i & 1) * 8;
+  return rb::lds_column8(lo, up);
+}
+
+// Workgroup -> (tile, head, batch). Tiles of a causal triangle differ in
+// length: the longest come first. The heads of one key/value head stay on one
+// XCD, whose L2 then holds their keys, when those heads divide by the XCDs.
+struct Place { int tile, head, batch; };
+RB_DEV Place place(int id, int tiles, int heads, int kv, int batch,
+                   bool longest_is_last) {
+  const int per_tile = heads * batch;
+  int t = id / per_tile, j = id % per_tile;
+  if (longest_is_last) t = tiles - 1 - t;
+  const int group = heads / kv;
+  if (kv * batch % 8 == 0) {
+    const int xcd = j % 8, k = j / 8;        // consecutive ids: next XCD
+    const int pair = k / group * 8 + xcd;    // (batch, kv head)
+    return {t, pair % kv * group + k % group, pair / kv};
+  }
+  return {t, j % heads, j / heads};
+}
+
+}  // namespace flash

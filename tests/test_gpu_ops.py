@@ -374,6 +374,43 @@ def test_flash_prefill(B, S, Hq, Hkv, dh):
     assert diff < 3e-2, f"max diff {diff}"
 
 
+@pytest.mark.parametrize("B,S,Hq,Hkv,dh,scale", [
+    # up to 512 tiles of 32 rows, two waves a tile
+    (1, 1, 2, 1, 64, None), (2, 33, 3, 3, 128, -0.1), (1, 65, 2, 1, 128, 0.0),
+    # up to 1536 tiles, four waves
+    (1, 545, 32, 8, 64, None), (2, 257, 40, 8, 128, None),
+    (1, 63, 4, 2, 256, None), (1, 321, 24, 8, 256, -0.05),
+    # one wave a tile
+    (1, 1601, 32, 8, 128, None), (2, 737, 32, 32, 64, None),
+    (1, 1313, 32, 32, 256, None),
+    # eight waves
+    (1, 1537, 128, 8, 64, None), (3, 1025, 64, 2, 128, None)])
+def test_flash_prefill_tiles(B, S, Hq, Hkv, dh, scale):
+    """Every split of the rows over waves, at remainders of its tiles, with
+    inputs that start off a 16-byte boundary. Weights and result are rounded to
+    bf16 (2^-9 relative each), sums are fp32."""
+    _assert_hip()
+    g = torch.Generator(device=DEV).manual_seed(S)
+
+    def rows(h):
+        n = B * S * h * dh
+        return torch.randn(n + 1, generator=g, device=DEV).bfloat16()[1:] \
+            .view(B, S, h, dh)
+
+    q, k, v = rows(Hq), rows(Hkv), rows(Hkv)
+    scale = dh ** -0.5 if scale is None else scale
+    out, lse = ops.ext().flash_fwd_train(q, k, v, scale)
+    hidden = torch.ones(S, S, dtype=torch.bool, device=DEV).triu(1)
+    for h in {0, Hq // 2, Hq - 1}:
+        at = h // (Hq // Hkv)
+        for b in range(B):
+            s = q[b, :, h].double() @ k[b, :, at].double().t() * scale
+            s = s.masked_fill(hidden, float("-inf"))
+            ref = s.softmax(-1) @ v[b, :, at].double()
+            assert (out[b, :, h] - ref).norm() < 2 ** -8 * ref.norm()
+            assert (lse[b, h] - s.logsumexp(-1)).abs().max() < 1e-5
+
+
 @pytest.mark.parametrize("B,S,Hq,Hkv,dh", [
     (1, 64, 4, 4, 128),      # tiny, single WG tile
     (2, 333, 8, 2, 128),     # ragged S, GQA (group-summed dk/dv)

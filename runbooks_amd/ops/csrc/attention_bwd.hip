@@ -1,33 +1,36 @@
 // Flash-attention TRAINING backward (causal, GQA, bf16) for CDNA4 (gfx950).
 //
-// FA2-style recompute backward in three dispatches:
-//   1. fa_bwd_preprocess: D[b,h,q] = rowsum(dO . O)            (f32)
-//   2. fa_bwd_dq:   per 256-query WG, loop KV tiles:
-//        S^T = K(scaled Q)^T           mfma(A=K_lds,  B=qf)     C[key][qrow]
-//        P^T = exp(S^T - LSE[qrow])
-//        dP^T = V dO^T                 mfma(A=V_lds,  B=dof)    C[key][qrow]
-//        dS^T = P^T (dP^T - D[qrow]) * scale
-//        dQ  += (dS^T)^T K             mfma(A=KT_lds, B=repack(dS^T))
-//                                                               C[d][qrow]
-//   3. fa_bwd_dkdv: per 256-key WG, loop Q tiles (>= diag):
-//        S   = (Q)(scaled K)^T         mfma(A=Q_lds,  B=kf)     C[qrow][key]
-//        P   = exp(S - LSE[qrow])
-//        dV += P^T dO                  mfma(A=dOT_lds, B=repack(P))
-//                                                               C[d][key]
-//        dP  = dO V^T                  mfma(A=dO_lds, B=vf)     C[qrow][key]
-//        dS  = P (dP - D[qrow]) * scale
-//        dK += dS^T Q                  mfma(A=QT_lds, B=repack(dS))
-//                                                               C[d][key]
+// FA2-style recompute backward in two dispatches over LDS tiles of 64 rows
+// (flash_tile.h), double-buffered as in the forward:
+//   1. fa_bwd_dq: a wave owns 32 query rows and walks the keys up to them.
+//        D    = rowsum(dO . O), also left in memory for 2.
+//        S^T  = K Q^T, P^T = exp(scale S^T - LSE)           C[key][qrow]
+//        dP^T = V dO^T, dS^T = P^T (dP^T - D)               C[key][qrow]
+//        dQ^T += K^T dS^T                                   C[d][qrow]
+//   2. fa_bwd_dkdv: a wave owns 32 keys and walks the queries from them on.
+//        S  = Q K^T, P = exp(scale S - LSE)                 C[qrow][key]
+//        dP = dO V^T, dS = P (dP - D)                       C[qrow][key]
+//        dV^T += dO^T P, dK^T += Q^T dS                     C[d][key]
+//   The factor `scale` of dQ and dK is applied to the sums.
 //
-// Same wave geometry as the forward (attention_prefill.hip): 8 waves per
-// WG, each wave owns 32 rows of its output on lanes (j = lane&31), the
-// MFMA C reg dim carries the other axis. The C->B "repack" (pack_bf16 +
-// v_permlane32_swap) is the forward's P repack. GQA: dK/dV are computed
-// per q-head ([B,S,Hq,DH]); the group-sum to Hkv heads happens in the
-// Python wrapper (ops/attention.py) — llama2-7b is MHA so the common path
-// has no extra reduction.
+// LSE and D enter as the first value of the accumulators (-LSE / scale, -D), so
+// they cost no registers of their own. Scores stand in registers in the order
+// in which the transposed reads take the rows, and are the next product's
+// operand as they are. GQA: dK/dV are computed per q-head ([B,S,Hq,DH]); the
+// group-sum to Hkv heads happens in the Python wrapper (ops/attention.py).
 //
-// mfma_f32_32x32x16_bf16 layouts (cdna_hip_programming.md §3):
+// What bounds it: the matrix cores, of whose time the exponentials, products
+// and roundings between take half as much again; LDS reads (32 KB per 32 MFMA
+// and wave) come next. dK/dV of 128 columns hold 128 registers of sums and 64 of
+// operands: with one wave per SIMD (360 registers) they beat two (256, which
+// spill 84): 7931 tokens, 32 query and 8 kv heads, 2068 against 3253 us.
+// Measured, both kernels, before (tiles through registers, transposed copies
+// made in LDS, one element at a time) and now:
+//   3001 tokens, 32 query and 8 kv heads of 128    1864 -> 344 us, 751 TF/s
+//   4 x 512 tokens, 32 heads of 128                 284 ->  79 us
+//   4000 tokens, 32 heads of 64                     941 -> 260 us, 883 TF/s
+//
+// mfma_f32_32x32x16_bf16 layouts:
 //   A[i][k]: i = lane&31, k = (lane>>5)*8 + e
 //   B[k][j]: j = lane&31, k = (lane>>5)*8 + e
 //   C[i][j]: j = lane&31, i = (r&3) + 8*(r>>2) + 4*(lane>>5)
@@ -35,315 +38,228 @@
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
-#include "common.h"
+#include <type_traits>
+
+#include "flash_tile.h"
 
 namespace {
 
-constexpr int BLOCK = 256;  // 4 waves (128-row WGs: finer grid
-                            // halves the causal-triangle imbalance and
-                            // doubles WG count vs 8-wave WGs)
-constexpr int TILE = 64;    // rows staged to LDS per loop step
+using namespace flash;
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8v;
-typedef __attribute__((ext_vector_type(16))) float f32x16v;
+constexpr float LOG2E = 1.4426950408889634f;
 
-RB_DEV unsigned pack2_bf16(float lo, float hi) {
-  union { __bf16 b; unsigned short u; } a, b;
-  a.b = (__bf16)lo;
-  b.b = (__bf16)hi;
-  return ((unsigned)b.u << 16) | a.u;
-}
+struct Args {
+  const uint16_t *q, *k, *v, *dout, *out;
+  const float *lse;                     // [B, Hq, S]
+  float *dvec;                          // [B, Hq, S]
+  uint16_t *dq, *dk, *dv;               // [B, S, Hq, DH]
+  int B, S, Hq, Hkv;
+  float scale;
+};
 
-RB_DEV bf16x8v words_to_frag(unsigned w0, unsigned w1, unsigned w2,
-                             unsigned w3) {
+// Eight values of two score tiles' registers -> a B operand.
+RB_DEV bf16x8v operand(const f32x16v &p, int ks) {
   union { unsigned u[4]; bf16x8v v; } c;
-  c.u[0] = w0; c.u[1] = w1; c.u[2] = w2; c.u[3] = w3;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    c.u[i] = pack2(p[ks * 8 + 2 * i], p[ks * 8 + 2 * i + 1]);
   return c.v;
 }
 
-// C-layout values (16 regs = 32 i-rows) -> two B fragments along k.
-// Identical to the forward's P repack; kslot selects k in [0,16)/[16,32).
-RB_DEV bf16x8v repack_c_to_b(const float *p, int kslot) {
-  const int r0 = kslot * 8;
-  unsigned pk0 = pack2_bf16(p[r0 + 0], p[r0 + 1]);
-  unsigned pk1 = pack2_bf16(p[r0 + 2], p[r0 + 3]);
-  unsigned pk2 = pack2_bf16(p[r0 + 4], p[r0 + 5]);
-  unsigned pk3 = pack2_bf16(p[r0 + 6], p[r0 + 7]);
-  auto r02 = __builtin_amdgcn_permlane32_swap(pk0, pk2, false, false);
-  auto r13 = __builtin_amdgcn_permlane32_swap(pk1, pk3, false, false);
-  return words_to_frag(r02[0], r13[0], r02[1], r13[1]);
+// A row's operands along DH, from memory.
+template <int DH>
+RB_DEV void load_row(bf16x8v *f, const uint16_t *row, int hi) {
+#pragma unroll
+  for (int ks = 0; ks < DH / 16; ++ks)
+    f[ks] = *reinterpret_cast<const bf16x8v *>(row + ks * 16 + hi * 8);
 }
 
-// ---------------------------------------------------------------------------
-// 1. D = rowsum(dO . O): dO, O [B, S, H, DH] bf16 -> D [B, H, S] f32
-// ---------------------------------------------------------------------------
+// C[d][col] times `scale` -> 16-bit rows.
 template <int DH>
-__global__ void fa_bwd_preprocess_kernel(const uint16_t *__restrict__ dop,
-                                         const uint16_t *__restrict__ op,
-                                         float *__restrict__ dp,
-                                         int B, int S, int H) {
-  constexpr int LPR = DH / 32;          // 16B vectors per lane chunk
-  const int row = blockIdx.x * 64 + (threadIdx.x >> 2);  // global (b*S+s)*H+h
-  const int c = threadIdx.x & 3;
-  const int64_t total = (int64_t)B * S * H;
-  if (row >= total) return;
-  const uint16_t *o = op + (int64_t)row * DH + c * (DH / 4);
-  const uint16_t *g = dop + (int64_t)row * DH + c * (DH / 4);
-  float acc = 0.0f;
+RB_DEV void store_row(uint16_t *row, const f32x16v *acc, float scale, int hi) {
 #pragma unroll
-  for (int v = 0; v < LPR; ++v) {
-    float fo[8], fg[8];
-    rb::VIO<uint16_t>::load(o + v * 8, fo);
-    rb::VIO<uint16_t>::load(g + v * 8, fg);
+  for (int dt = 0; dt < DH / 32; ++dt)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc += fo[e] * fg[e];
-  }
-#pragma unroll
-  for (int off = 1; off < 4; off <<= 1) acc += __shfl_xor(acc, off, 64);
-  if (c == 0) {
-    const int h = row % H;
-    const int s = (row / H) % S;
-    const int b = row / (H * (int64_t)S);
-    dp[((int64_t)b * H + h) * S + s] = acc;
-  }
+    for (int rq = 0; rq < 4; ++rq) {
+      uint2 w;
+      w.x = pack2(acc[dt][rq * 4] * scale, acc[dt][rq * 4 + 1] * scale);
+      w.y = pack2(acc[dt][rq * 4 + 2] * scale, acc[dt][rq * 4 + 3] * scale);
+      *reinterpret_cast<uint2 *>(row + dt * 32 + 8 * rq + 4 * hi) = w;
+    }
 }
 
-// ---------------------------------------------------------------------------
-// 2. dQ kernel — mirrors the forward loop over KV tiles.
-// q, k, v, dout: [B, S, H*, DH] bf16; lse, dvec: [B, Hq, S] f32.
-// dq: [B, S, Hq, DH] bf16.
-// ---------------------------------------------------------------------------
+// Scores count scale times; with a scale of zero they count once and Q is
+// cleared, so that hidden ones stay at minus infinity.
+RB_DEV float unit(float scale) { return scale == 0.0f ? 1.0f : scale; }
+
 template <int DH>
-__global__ __launch_bounds__(BLOCK, 2) void fa_bwd_dq_kernel(
-    const uint16_t *__restrict__ qp, const uint16_t *__restrict__ kp,
-    const uint16_t *__restrict__ vp, const uint16_t *__restrict__ dop,
-    const float *__restrict__ lsep, const float *__restrict__ dvecp,
-    uint16_t *__restrict__ dqp, int B, int S, int Hq, int Hkv, float scale) {
-  constexpr int KSTEPS = DH / 16;
-  constexpr int DTILES = DH / 32;
-  constexpr int ROW_STRIDE = DH * 2 + 16;   // row-major tile row bytes
-  constexpr int TR_STRIDE = TILE * 2 + 16;  // transposed tile row bytes
+RB_DEV void clear_if(bool yes, bf16x8v *f) {
+  if (!yes) return;
+#pragma unroll
+  for (int ks = 0; ks < DH / 16; ++ks) f[ks] = (bf16x8v)(__bf16)0.0f;
+}
 
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  char *k_img = smem;                           // [TILE][ROW_STRIDE]
-  char *v_img = k_img + TILE * ROW_STRIDE;      // [TILE][ROW_STRIDE]
-  char *kt_img = v_img + TILE * ROW_STRIDE;     // [DH][TR_STRIDE]
+template <int DH, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
+  constexpr int KSTEPS = DH / 16, DTILES = DH / 32;
+  constexpr int QT = NW * 32, TILE = tile_bytes<DH>();
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
 
-  const int tid = threadIdx.x;
-  const int wid = tid >> 6;
-  const int lane = tid & 63;
-  const int hi = lane >> 5;
-  const int col = lane & 31;
-
-  const int q0 = blockIdx.x * 128;
-  const int h = blockIdx.y;
-  const int b = blockIdx.z;
-  const int h_kv = h / (Hq / Hkv);
-  const int qrow = q0 + wid * 32 + col;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, hi = lane >> 5, col = lane & 31;
+  const int S = a.S;
+  const Place at = place(blockIdx.x, (S + QT - 1) / QT, a.Hq, a.Hkv, a.B,
+                         true);
+  const int h_kv = at.head / (a.Hq / a.Hkv);
+  const int wrow = at.tile * QT + wid * 32;
+  const int qrow = wrow + col;
   const bool q_valid = qrow < S;
 
-  // per-lane fragments for this lane's query row
-  bf16x8v qf[KSTEPS];   // scaled Q (B operand of S^T)
-  bf16x8v dof[KSTEPS];  // dO (B operand of dP^T)
-  float lse = q_valid ? lsep[((int64_t)b * Hq + h) * S + qrow] : INFINITY;
-  float dvec = q_valid ? dvecp[((int64_t)b * Hq + h) * S + qrow] : 0.0f;
-  {
-    const int64_t base = ((int64_t)(b * S + (q_valid ? qrow : 0)) * Hq + h) * DH;
+  const int64_t kv_stride = (int64_t)a.Hkv * DH;
+  const int64_t kv0 = ((int64_t)at.batch * S * a.Hkv + h_kv) * DH;
+  const uint16_t *kb = a.k + kv0, *vb = a.v + kv0;
+  const TileLoad<DH, NW> load(wid, lane);
+  const int n_tiles = (min(S, at.tile * QT + QT) + ROWS - 1) / ROWS;
+  load(kb, kv_stride, 0, S, smem, wid);
+  load(vb, kv_stride, 0, S, smem + TILE, wid);
+
+  const int64_t row0 =
+      (((int64_t)at.batch * S + (q_valid ? qrow : 0)) * a.Hq + at.head) * DH;
+  const int64_t stat = ((int64_t)at.batch * a.Hq + at.head) * S + qrow;
+  bf16x8v qf[KSTEPS], dof[KSTEPS];
+  load_row<DH>(qf, a.q + row0, hi);
+  clear_if<DH>(a.scale == 0.0f, qf);
+  load_row<DH>(dof, a.dout + row0, hi);
+  float dvec = 0.0f;
+#pragma unroll
+  for (int ks = 0; ks < KSTEPS; ++ks) {
+    const bf16x8v o = *reinterpret_cast<const bf16x8v *>(
+        a.out + row0 + ks * 16 + hi * 8);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dvec += (float)o[e] * (float)dof[ks][e];
+  }
+  dvec += __shfl_xor(dvec, 32, 64);
+  if (q_valid && hi == 0) a.dvec[stat] = dvec;
+  const float by = unit(a.scale), to2 = by * LOG2E;
+  const float s0 = q_valid ? -a.lse[stat] / by : 0.0f;
+
+  f32x16v acc[DTILES];
+#pragma unroll
+  for (int dt = 0; dt < DTILES; ++dt) acc[dt] = (f32x16v)(0.0f);
+
+  auto keys = [&](const char *kt, const char *vt, int kbase, int r0,
+                  auto masked) {
+    f32x16v s = (f32x16v)(s0), dp = (f32x16v)(-dvec);
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
-      float fq[8], fd[8];
-      rb::VIO<uint16_t>::load(qp + base + ks * 16 + hi * 8, fq);
-      rb::VIO<uint16_t>::load(dop + base + ks * 16 + hi * 8, fd);
-      union { unsigned short u[8]; bf16x8v v; } cq, cd;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        cq.u[e] = rb::f32_to_bf16(q_valid ? fq[e] * scale : 0.0f);
-        cd.u[e] = rb::f32_to_bf16(q_valid ? fd[e] : 0.0f);
-      }
-      qf[ks] = cq.v;
-      dof[ks] = cd.v;
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          row_frag<DH>(kt, r0, ks, col, hi), qf[ks], s, 0, 0, 0);
+      dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          row_frag<DH>(vt, r0, ks, col, hi), dof[ks], dp, 0, 0, 0);
     }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      float p = __builtin_amdgcn_exp2f(s[r] * to2);
+      if constexpr (decltype(masked)::value)
+        if (kbase + (r & 3) + 8 * (r >> 2) + 4 * hi > qrow) p = 0.0f;
+      s[r] = p * dp[r];
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const bf16x8v ds = operand(s, ks);
+#pragma unroll
+      for (int dt = 0; dt < DTILES; ++dt)
+        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            column_frag<DH>(kt, r0 + ks * 16, dt, lane), ds, acc[dt], 0, 0, 0);
+    }
+  };
+  // waits for tile t and sends for the next one
+  auto arrive = [&](int t) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();                    // nobody reads the other buffer any more
+    if (t + 1 < n_tiles) {
+      char *next = smem + (~t & 1) * 2 * TILE;
+      load(kb, kv_stride, (t + 1) * ROWS, S, next, wid);
+      load(vb, kv_stride, (t + 1) * ROWS, S, next + TILE, wid);
+    }
+  };
+  const int full = wrow / ROWS;         // tiles that every row sees whole
+  int t = 0;
+  for (; t < full; ++t) {
+    arrive(t);
+    const char *kt = smem + (t & 1) * 2 * TILE;
+#pragma unroll
+    for (int r0 = 0; r0 < ROWS; r0 += 32)
+      keys(kt, kt + TILE, t * ROWS + r0, r0, std::false_type{});
   }
-
-  f32x16v acc_dq[DTILES];
+  for (; t < n_tiles; ++t) {
+    arrive(t);
+    const char *kt = smem + (t & 1) * 2 * TILE;
 #pragma unroll
-  for (int dt = 0; dt < DTILES; ++dt) acc_dq[dt] = (f32x16v)(0.0f);
-
-  const int kv_end = min(S, q0 + 128);
-  const int n_tiles = (kv_end + TILE - 1) / TILE;
-  const int wave_kmax = q0 + wid * 32 + 31;
-
-  for (int kt = 0; kt < n_tiles; ++kt) {
-    const int kbase = kt * TILE;
-
-    // ---- stage K and V row-major ----------------------------------------
-    {
-      constexpr int total = TILE * DH;
-      const int per_pass = BLOCK * 8;
-#pragma unroll
-      for (int p = 0; p < total / per_pass; ++p) {
-        const int idx = p * per_pass + tid * 8;
-        const int key = idx / DH;
-        const int d0 = idx % DH;
-        const int gk = kbase + key;
-        rb::bf16x8 kv8, vv8;
-        if (gk < S) {
-          const int64_t base = ((int64_t)(b * S + gk) * Hkv + h_kv) * DH + d0;
-          kv8 = *reinterpret_cast<const rb::bf16x8 *>(kp + base);
-          vv8 = *reinterpret_cast<const rb::bf16x8 *>(vp + base);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) { kv8.v[e] = 0; vv8.v[e] = 0; }
-        }
-        *reinterpret_cast<rb::bf16x8 *>(k_img + key * ROW_STRIDE + d0 * 2) = kv8;
-        *reinterpret_cast<rb::bf16x8 *>(v_img + key * ROW_STRIDE + d0 * 2) = vv8;
-      }
-    }
-    // ---- stage K transposed ([d][key]) -----------------------------------
-    // from the LDS row image (same fix as dkdv: the global column-
-    // strided scalar re-read was latency-bound)
-    __syncthreads();
-    {
-      constexpr int GRPS = BLOCK / DH;
-      constexpr int KPG = TILE / GRPS;
-      const int d = tid % DH;
-      const int kg0 = (tid / DH) * KPG;
-      uint16_t tmp[KPG];
-#pragma unroll
-      for (int e = 0; e < KPG; ++e) {
-        tmp[e] = *reinterpret_cast<const uint16_t *>(
-            k_img + (kg0 + e) * ROW_STRIDE + d * 2);
-      }
-#pragma unroll
-      for (int c8 = 0; c8 < KPG / 8; ++c8)
-        *reinterpret_cast<rb::bf16x8 *>(
-            kt_img + d * TR_STRIDE + (kg0 + c8 * 8) * 2) =
-            *reinterpret_cast<rb::bf16x8 *>(&tmp[c8 * 8]);
-    }
-    __syncthreads();
-
-    if (kbase <= wave_kmax) {
-#pragma unroll
-      for (int it = 0; it < 2; ++it) {
-        // ---- S^T[key][qrow] and dP^T[key][qrow] --------------------------
-        f32x16v s = (f32x16v)(0.0f);
-        f32x16v dpt = (f32x16v)(0.0f);
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks) {
-          const bf16x8v kfr = *reinterpret_cast<const bf16x8v *>(
-              k_img + (it * 32 + col) * ROW_STRIDE + (ks * 16 + hi * 8) * 2);
-          const bf16x8v vfr = *reinterpret_cast<const bf16x8v *>(
-              v_img + (it * 32 + col) * ROW_STRIDE + (ks * 16 + hi * 8) * 2);
-          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr, qf[ks], s, 0, 0, 0);
-          dpt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr, dof[ks], dpt,
-                                                        0, 0, 0);
-        }
-
-        // ---- dS^T = P^T (dP^T - D) * scale -------------------------------
-        float ds[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = kbase + it * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
-          const float pt = (key <= qrow) ? __expf(s[r] - lse) : 0.0f;
-          ds[r] = pt * (dpt[r] - dvec) * scale;
-        }
-
-        // ---- dQ += (dS^T)^T K -------------------------------------------
-#pragma unroll
-        for (int kslot = 0; kslot < 2; ++kslot) {
-          const bf16x8v dsf = repack_c_to_b(ds, kslot);
-          const int koff = (it * 32 + kslot * 16 + hi * 8) * 2;
-#pragma unroll
-          for (int dt = 0; dt < DTILES; ++dt) {
-            const bf16x8v ktf = *reinterpret_cast<const bf16x8v *>(
-                kt_img + (dt * 32 + col) * TR_STRIDE + koff);
-            acc_dq[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                ktf, dsf, acc_dq[dt], 0, 0, 0);
-          }
-        }
-      }
-    }
-    __syncthreads();
+    for (int r0 = 0; r0 < ROWS; r0 += 32)
+      if (t * ROWS + r0 <= wrow + 31)
+        keys(kt, kt + TILE, t * ROWS + r0, r0, std::true_type{});
   }
-
-  // ---- epilogue: dQ[b, qrow, h, :] ----------------------------------------
-  if (q_valid) {
-    uint16_t *row = dqp + ((int64_t)(b * S + qrow) * Hq + h) * DH;
-#pragma unroll
-    for (int dt = 0; dt < DTILES; ++dt) {
-#pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        const int d0 = dt * 32 + 8 * rq + 4 * hi;
-        uint16_t w[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          w[e] = rb::f32_to_bf16(acc_dq[dt][rq * 4 + e]);
-        *reinterpret_cast<uint2 *>(row + d0) =
-            *reinterpret_cast<const uint2 *>(w);
-      }
-    }
-  }
+  if (q_valid) store_row<DH>(a.dq + row0, acc, a.scale, hi);
 }
 
-// ---------------------------------------------------------------------------
-// 3. dK/dV kernel — wave owns 32 keys, loops over Q tiles at/after the
-// diagonal. Outputs per-q-head dk, dv [B, S, Hq, DH] bf16.
-// ---------------------------------------------------------------------------
-template <int DH>
-__global__ __launch_bounds__(BLOCK, 2) void fa_bwd_dkdv_kernel(
-    const uint16_t *__restrict__ qp, const uint16_t *__restrict__ kp,
-    const uint16_t *__restrict__ vp, const uint16_t *__restrict__ dop,
-    const float *__restrict__ lsep, const float *__restrict__ dvecp,
-    uint16_t *__restrict__ dkp, uint16_t *__restrict__ dvp,
-    int B, int S, int Hq, int Hkv, float scale) {
-  constexpr int KSTEPS = DH / 16;
-  constexpr int DTILES = DH / 32;
-  constexpr int ROW_STRIDE = DH * 2 + 16;
-  constexpr int TR_STRIDE = TILE * 2 + 16;
-
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  char *q_img = smem;                            // [TILE][ROW_STRIDE]
-  char *do_img = q_img + TILE * ROW_STRIDE;      // [TILE][ROW_STRIDE]
-  char *qt_img = do_img + TILE * ROW_STRIDE;     // [DH][TR_STRIDE]
-  char *dot_img = qt_img + DH * TR_STRIDE;       // [DH][TR_STRIDE]
-  float *lse_s = reinterpret_cast<float *>(dot_img + DH * TR_STRIDE);  // [TILE]
-  float *dvec_s = lse_s + TILE;                                        // [TILE]
+template <int DH, int NW>
+__global__ __launch_bounds__(NW * 64, DH == 128 ? 1 : 2)
+void fa_bwd_dkdv_kernel(Args a) {
+  constexpr int KSTEPS = DH / 16, DTILES = DH / 32;
+  constexpr int KT = NW * 32, TILE = tile_bytes<DH>();
+  constexpr int STATS = ROWS * 4 * 2;   // bytes of a tile's LSE and D
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
 
   const int tid = threadIdx.x;
-  const int wid = tid >> 6;
-  const int lane = tid & 63;
-  const int hi = lane >> 5;
-  const int col = lane & 31;
-
-  const int k0 = blockIdx.x * 128;
-  const int h = blockIdx.y;
-  const int b = blockIdx.z;
-  const int h_kv = h / (Hq / Hkv);
-  const int key = k0 + wid * 32 + col;       // this lane's key row
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, hi = lane >> 5, col = lane & 31;
+  const int S = a.S;
+  const Place at = place(blockIdx.x, (S + KT - 1) / KT, a.Hq, a.Hkv, a.B,
+                         false);
+  const int h_kv = at.head / (a.Hq / a.Hkv);
+  const int wkey = at.tile * KT + wid * 32;
+  const int key = wkey + col;
   const bool k_valid = key < S;
 
-  // per-lane fragments for this lane's key row
-  bf16x8v kf[KSTEPS];   // scaled K (B operand of S)
-  bf16x8v vf[KSTEPS];   // V (B operand of dP)
-  {
-    const int64_t base =
-        ((int64_t)(b * S + (k_valid ? key : 0)) * Hkv + h_kv) * DH;
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      float fk[8], fv[8];
-      rb::VIO<uint16_t>::load(kp + base + ks * 16 + hi * 8, fk);
-      rb::VIO<uint16_t>::load(vp + base + ks * 16 + hi * 8, fv);
-      union { unsigned short u[8]; bf16x8v v; } ck, cv;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        ck.u[e] = rb::f32_to_bf16(k_valid ? fk[e] * scale : 0.0f);
-        cv.u[e] = rb::f32_to_bf16(k_valid ? fv[e] : 0.0f);
-      }
-      kf[ks] = ck.v;
-      vf[ks] = cv.v;
-    }
-  }
+  const int64_t q_stride = (int64_t)a.Hq * DH;
+  const int64_t q00 = ((int64_t)at.batch * S * a.Hq + at.head) * DH;
+  const uint16_t *qb = a.q + q00, *ob = a.dout + q00;
+  const int64_t stat = ((int64_t)at.batch * a.Hq + at.head) * S;
+  const float by = unit(a.scale), to2 = by * LOG2E;
+  const TileLoad<DH, NW> load(wid, lane);
+  const int tile0 = at.tile * KT / ROWS, n_tiles = (S + ROWS - 1) / ROWS;
 
+  // tile t's rows and statistics; the latter through registers, stored when
+  // the tile before it has been worked on
+  auto send = [&](int t, char *tile) {
+    load(qb, q_stride, t * ROWS, S, tile, wid);
+    load(ob, q_stride, t * ROWS, S, tile + TILE, wid);
+  };
+  char *stats = smem + 4 * TILE;        // two buffers, like the tiles
+  auto stat_of = [&](int t) {
+    const int row = t * ROWS + (tid & 63);
+    if (tid >= 2 * ROWS) return 0.0f;
+    if (tid >= ROWS) return row < S ? -a.dvec[stat + row] : 0.0f;
+    // rows past the end: weights of zero
+    return row < S ? -a.lse[stat + row] / by : by < 0.0f ? INFINITY
+                                                         : -INFINITY;
+  };
+  auto keep = [&](int t, float x) {
+    if (tid < 2 * ROWS)
+      reinterpret_cast<float *>(stats + (t & 1) * STATS)[tid] = x;
+  };
+  send(tile0, smem + (tile0 & 1) * 2 * TILE);
+  keep(tile0, stat_of(tile0));
+
+  bf16x8v kf[KSTEPS], vf[KSTEPS];
+  {
+    const int64_t row0 =
+        (((int64_t)at.batch * S + (k_valid ? key : 0)) * a.Hkv + h_kv) * DH;
+    load_row<DH>(kf, a.k + row0, hi);
+    clear_if<DH>(a.scale == 0.0f, kf);
+    load_row<DH>(vf, a.v + row0, hi);
+  }
   f32x16v acc_dk[DTILES], acc_dv[DTILES];
 #pragma unroll
   for (int dt = 0; dt < DTILES; ++dt) {
@@ -351,151 +267,102 @@ __global__ __launch_bounds__(BLOCK, 2) void fa_bwd_dkdv_kernel(
     acc_dv[dt] = (f32x16v)(0.0f);
   }
 
-  const int wave_kmin = k0 + wid * 32;       // first key this wave owns
-  const int n_tiles = (S - k0 + TILE - 1) / TILE;
-
-  for (int qt = 0; qt < n_tiles; ++qt) {
-    const int qbase = k0 + qt * TILE;
-
-    // ---- stage Q and dO row-major ----------------------------------------
-    {
-      constexpr int total = TILE * DH;
-      const int per_pass = BLOCK * 8;
+  // queries qbase .. qbase + 31, rows r0 .. of the tile
+  auto queries = [&](const char *qt, const float *st, int qbase, int r0,
+                     auto masked) {
+    const char *ot = qt + TILE;
+    f32x16v s, dp;
 #pragma unroll
-      for (int p = 0; p < total / per_pass; ++p) {
-        const int idx = p * per_pass + tid * 8;
-        const int qr = idx / DH;
-        const int d0 = idx % DH;
-        const int gq = qbase + qr;
-        rb::bf16x8 q8, d8;
-        if (gq < S) {
-          const int64_t base = ((int64_t)(b * S + gq) * Hq + h) * DH + d0;
-          q8 = *reinterpret_cast<const rb::bf16x8 *>(qp + base);
-          d8 = *reinterpret_cast<const rb::bf16x8 *>(dop + base);
-        } else {
+    for (int rq = 0; rq < 4; ++rq) {
+      const float4 l = *reinterpret_cast<const float4 *>(
+          st + r0 + 8 * rq + 4 * hi);
+      const float4 d = *reinterpret_cast<const float4 *>(
+          st + ROWS + r0 + 8 * rq + 4 * hi);
+      s[rq * 4] = l.x; s[rq * 4 + 1] = l.y;
+      s[rq * 4 + 2] = l.z; s[rq * 4 + 3] = l.w;
+      dp[rq * 4] = d.x; dp[rq * 4 + 1] = d.y;
+      dp[rq * 4 + 2] = d.z; dp[rq * 4 + 3] = d.w;
+    }
 #pragma unroll
-          for (int e = 0; e < 8; ++e) { q8.v[e] = 0; d8.v[e] = 0; }
-        }
-        *reinterpret_cast<rb::bf16x8 *>(q_img + qr * ROW_STRIDE + d0 * 2) = q8;
-        *reinterpret_cast<rb::bf16x8 *>(do_img + qr * ROW_STRIDE + d0 * 2) = d8;
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          row_frag<DH>(qt, r0, ks, col, hi), kf[ks], s, 0, 0, 0);
+      dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          row_frag<DH>(ot, r0, ks, col, hi), vf[ks], dp, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      float p = __builtin_amdgcn_exp2f(s[r] * to2);
+      if constexpr (decltype(masked)::value)
+        if (qbase + (r & 3) + 8 * (r >> 2) + 4 * hi < key) p = 0.0f;
+      s[r] = p;
+      dp[r] *= p;
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const bf16x8v pf = operand(s, ks), dsf = operand(dp, ks);
+#pragma unroll
+      for (int dt = 0; dt < DTILES; ++dt) {
+        acc_dv[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            column_frag<DH>(ot, r0 + ks * 16, dt, lane), pf, acc_dv[dt],
+            0, 0, 0);
+        acc_dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            column_frag<DH>(qt, r0 + ks * 16, dt, lane), dsf, acc_dk[dt],
+            0, 0, 0);
       }
     }
-    // ---- stage Q^T and dO^T ([d][qrow]) ----------------------------------
-    // Sourced from the just-staged LDS row images (50-cycle LDS reads)
-    // instead of re-reading global column-strided with scalar loads
-    // (~900-cycle HBM/L2 round trips per element — measured r9: dkdv at
-    // 235 us was the largest single train kernel).
-    __syncthreads();
-    {
-      constexpr int GRPS = BLOCK / DH;
-      constexpr int KPG = TILE / GRPS;
-      const int d = tid % DH;
-      const int qg0 = (tid / DH) * KPG;
-      uint16_t tq[KPG], td[KPG];
-#pragma unroll
-      for (int e = 0; e < KPG; ++e) {
-        const int qr = qg0 + e;
-        tq[e] = *reinterpret_cast<const uint16_t *>(
-            q_img + qr * ROW_STRIDE + d * 2);
-        td[e] = *reinterpret_cast<const uint16_t *>(
-            do_img + qr * ROW_STRIDE + d * 2);
-      }
-#pragma unroll
-      for (int c8 = 0; c8 < KPG / 8; ++c8) {
-        *reinterpret_cast<rb::bf16x8 *>(
-            qt_img + d * TR_STRIDE + (qg0 + c8 * 8) * 2) =
-            *reinterpret_cast<rb::bf16x8 *>(&tq[c8 * 8]);
-        *reinterpret_cast<rb::bf16x8 *>(
-            dot_img + d * TR_STRIDE + (qg0 + c8 * 8) * 2) =
-            *reinterpret_cast<rb::bf16x8 *>(&td[c8 * 8]);
-      }
+  };
+  auto step = [&](int t, auto masked) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();                    // nobody reads the other buffers any more
+    float next = 0.0f;
+    if (t + 1 < n_tiles) {
+      send(t + 1, smem + (~t & 1) * 2 * TILE);
+      next = stat_of(t + 1);
     }
-    // ---- stage per-qrow LSE and D ----------------------------------------
-    if (tid < TILE) {
-      const int gq = qbase + tid;
-      if (gq < S) {
-        lse_s[tid] = lsep[((int64_t)b * Hq + h) * S + gq];
-        dvec_s[tid] = dvecp[((int64_t)b * Hq + h) * S + gq];
-      } else {
-        lse_s[tid] = INFINITY;
-        dvec_s[tid] = 0.0f;
-      }
-    }
-    __syncthreads();
+    const char *qt = smem + (t & 1) * 2 * TILE;
+    const float *st = reinterpret_cast<const float *>(stats +
+                                                      (t & 1) * STATS);
+#pragma unroll
+    for (int r0 = 0; r0 < ROWS; r0 += 32)
+      if (!decltype(masked)::value || t * ROWS + r0 + 31 >= wkey)
+        queries(qt, st, t * ROWS + r0, r0, masked);
+    if (t + 1 < n_tiles) keep(t + 1, next);
+  };
+  // tiles that some of the workgroup's keys do not see whole, then the others
+  const int diagonal = min(n_tiles, (at.tile * KT + KT + ROWS - 1) / ROWS);
+  int t = tile0;
+  for (; t < diagonal; ++t) step(t, std::true_type{});
+  for (; t < n_tiles; ++t) step(t, std::false_type{});
 
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-      // this 32-qrow subtile reaches the wave's keys?
-      if (qbase + it * 32 + 31 >= wave_kmin) {
-        // ---- S[qrow][key] and dP[qrow][key] ------------------------------
-        f32x16v s = (f32x16v)(0.0f);
-        f32x16v dp = (f32x16v)(0.0f);
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks) {
-          const bf16x8v qfr = *reinterpret_cast<const bf16x8v *>(
-              q_img + (it * 32 + col) * ROW_STRIDE + (ks * 16 + hi * 8) * 2);
-          const bf16x8v dfr = *reinterpret_cast<const bf16x8v *>(
-              do_img + (it * 32 + col) * ROW_STRIDE + (ks * 16 + hi * 8) * 2);
-          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qfr, kf[ks], s, 0, 0, 0);
-          dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dfr, vf[ks], dp,
-                                                       0, 0, 0);
-        }
-
-        // ---- P and dS (both in C layout over qrow regs) ------------------
-        float pv[16], ds[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int qr = it * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
-          const int gq = qbase + qr;
-          const float p = (gq >= key) ? __expf(s[r] - lse_s[qr]) : 0.0f;
-          pv[r] = p;
-          ds[r] = p * (dp[r] - dvec_s[qr]) * scale;
-        }
-
-        // ---- dV += P^T dO; dK += dS^T Q ----------------------------------
-#pragma unroll
-        for (int kslot = 0; kslot < 2; ++kslot) {
-          const bf16x8v pf = repack_c_to_b(pv, kslot);
-          const bf16x8v dsf = repack_c_to_b(ds, kslot);
-          const int qoff = (it * 32 + kslot * 16 + hi * 8) * 2;
-#pragma unroll
-          for (int dt = 0; dt < DTILES; ++dt) {
-            const bf16x8v dotf = *reinterpret_cast<const bf16x8v *>(
-                dot_img + (dt * 32 + col) * TR_STRIDE + qoff);
-            const bf16x8v qtf = *reinterpret_cast<const bf16x8v *>(
-                qt_img + (dt * 32 + col) * TR_STRIDE + qoff);
-            acc_dv[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                dotf, pf, acc_dv[dt], 0, 0, 0);
-            acc_dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                qtf, dsf, acc_dk[dt], 0, 0, 0);
-          }
-        }
-      }
-    }
-    __syncthreads();
-  }
-
-  // ---- epilogue: dK, dV -> [b, key, h, :] ---------------------------------
   if (k_valid) {
-    const int64_t base = ((int64_t)(b * S + key) * Hq + h) * DH;
-#pragma unroll
-    for (int dt = 0; dt < DTILES; ++dt) {
-#pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        const int d0 = dt * 32 + 8 * rq + 4 * hi;
-        uint16_t wk[4], wv[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          wk[e] = rb::f32_to_bf16(acc_dk[dt][rq * 4 + e]);
-          wv[e] = rb::f32_to_bf16(acc_dv[dt][rq * 4 + e]);
-        }
-        *reinterpret_cast<uint2 *>(dkp + base + d0) =
-            *reinterpret_cast<const uint2 *>(wk);
-        *reinterpret_cast<uint2 *>(dvp + base + d0) =
-            *reinterpret_cast<const uint2 *>(wv);
-      }
-    }
+    const int64_t row0 =
+        (((int64_t)at.batch * S + key) * a.Hq + at.head) * DH;
+    store_row<DH>(a.dk + row0, acc_dk, a.scale, hi);
+    store_row<DH>(a.dv + row0, acc_dv, 1.0f, hi);
   }
+}
+
+template <int DH, int NW> void launch_bwd(const Args &a, hipStream_t stream) {
+  constexpr size_t sh_dq = 4 * tile_bytes<DH>();
+  constexpr size_t sh_dkdv = sh_dq + 2 * ROWS * 4 * 2;
+  static const bool once =
+      hipFuncSetAttribute(
+          reinterpret_cast<const void *>(&fa_bwd_dq_kernel<DH, NW>),
+          hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh_dq) ==
+          hipSuccess &&
+      hipFuncSetAttribute(
+          reinterpret_cast<const void *>(&fa_bwd_dkdv_kernel<DH, NW>),
+          hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh_dkdv) ==
+          hipSuccess;
+  TORCH_CHECK(once, "fa_bwd: LDS size");
+  const int64_t grid =
+      (int64_t)((a.S + NW * 32 - 1) / (NW * 32)) * a.Hq * a.B;
+  TORCH_CHECK(grid < (int64_t)1 << 31, "fa_bwd: grid");
+  hipLaunchKernelGGL((fa_bwd_dq_kernel<DH, NW>), dim3((unsigned)grid),
+                     dim3(NW * 64), sh_dq, stream, a);
+  hipLaunchKernelGGL((fa_bwd_dkdv_kernel<DH, NW>), dim3((unsigned)grid),
+                     dim3(NW * 64), sh_dkdv, stream, a);
 }
 
 }  // namespace
@@ -515,7 +382,20 @@ std::vector<at::Tensor> fa_bwd(at::Tensor dout, at::Tensor q, at::Tensor k,
             DH = (int)q.size(3);
   const int Hkv = (int)k.size(2);
   TORCH_CHECK(DH == 64 || DH == 128, "fa_bwd: DH must be 64 or 128");
-  TORCH_CHECK(lse.scalar_type() == at::kFloat && lse.is_contiguous());
+  TORCH_CHECK(lse.scalar_type() == at::kFloat && lse.is_contiguous() &&
+              lse.numel() == (int64_t)B * Hq * S, "fa_bwd: lse [B, Hq, S]");
+  TORCH_CHECK(Hkv > 0 && Hq % Hkv == 0 &&
+              k.sizes() == at::IntArrayRef({B, S, Hkv, DH}) &&
+              v.sizes() == k.sizes() && dout.sizes() == q.sizes() &&
+              out.sizes() == q.sizes() && k.scalar_type() == at::kBFloat16 &&
+              v.scalar_type() == at::kBFloat16 &&
+              dout.scalar_type() == at::kBFloat16 &&
+              out.scalar_type() == at::kBFloat16, "fa_bwd: shapes, types");
+  q = aligned16(q);
+  k = aligned16(k);
+  v = aligned16(v);
+  dout = aligned16(dout);
+  out = aligned16(out);
 
   auto dq = at::empty_like(q);
   // per-q-head dk/dv; group-summed by the caller when Hkv < Hq
@@ -523,51 +403,29 @@ std::vector<at::Tensor> fa_bwd(at::Tensor dout, at::Tensor q, at::Tensor k,
   auto dv = at::empty({B, S, Hq, DH}, q.options());
   auto dvec = at::empty({B, Hq, S}, q.options().dtype(at::kFloat));
 
+  if (dq.numel() == 0) return {dq, dk, dv};
+  Args a{};
+  a.q = (const uint16_t *)q.data_ptr();
+  a.k = (const uint16_t *)k.data_ptr();
+  a.v = (const uint16_t *)v.data_ptr();
+  a.dout = (const uint16_t *)dout.data_ptr();
+  a.out = (const uint16_t *)out.data_ptr();
+  a.lse = lse.data_ptr<float>();
+  a.dvec = dvec.data_ptr<float>();
+  a.dq = (uint16_t *)dq.data_ptr();
+  a.dk = (uint16_t *)dk.data_ptr();
+  a.dv = (uint16_t *)dv.data_ptr();
+  a.B = B; a.S = S; a.Hq = Hq; a.Hkv = Hkv;
+  a.scale = (float)scale;
   auto stream = at::hip::getCurrentHIPStream();
-  {
-    const int64_t rows = (int64_t)B * S * Hq;
-    const dim3 grid((unsigned)((rows + 63) / 64));
-    if (DH == 128)
-      hipLaunchKernelGGL((fa_bwd_preprocess_kernel<128>), grid, dim3(256), 0,
-                         stream, (const uint16_t *)dout.data_ptr(),
-                         (const uint16_t *)out.data_ptr(),
-                         dvec.data_ptr<float>(), B, S, Hq);
-    else
-      hipLaunchKernelGGL((fa_bwd_preprocess_kernel<64>), grid, dim3(256), 0,
-                         stream, (const uint16_t *)dout.data_ptr(),
-                         (const uint16_t *)out.data_ptr(),
-                         dvec.data_ptr<float>(), B, S, Hq);
-  }
-
-  const dim3 grid((S + 127) / 128, Hq, B);
-#define RB_LAUNCH_BWD(DHV)                                                    \
-  do {                                                                        \
-    constexpr int ROW_STRIDE = DHV * 2 + 16;                                  \
-    constexpr int TR_STRIDE = TILE * 2 + 16;                                  \
-    constexpr size_t sh_dq =                                                  \
-        2 * TILE * ROW_STRIDE + DHV * TR_STRIDE;                              \
-    constexpr size_t sh_dkdv = 2 * TILE * ROW_STRIDE +                        \
-        2 * DHV * TR_STRIDE + 2 * TILE * sizeof(float);                       \
-    hipLaunchKernelGGL((fa_bwd_dq_kernel<DHV>), grid, dim3(BLOCK), sh_dq,     \
-                       stream, (const uint16_t *)q.data_ptr(),                \
-                       (const uint16_t *)k.data_ptr(),                        \
-                       (const uint16_t *)v.data_ptr(),                        \
-                       (const uint16_t *)dout.data_ptr(),                     \
-                       lse.data_ptr<float>(), dvec.data_ptr<float>(),         \
-                       (uint16_t *)dq.data_ptr(), B, S, Hq, Hkv,              \
-                       (float)scale);                                         \
-    hipLaunchKernelGGL((fa_bwd_dkdv_kernel<DHV>), grid, dim3(BLOCK), sh_dkdv, \
-                       stream, (const uint16_t *)q.data_ptr(),                \
-                       (const uint16_t *)k.data_ptr(),                        \
-                       (const uint16_t *)v.data_ptr(),                        \
-                       (const uint16_t *)dout.data_ptr(),                     \
-                       lse.data_ptr<float>(), dvec.data_ptr<float>(),         \
-                       (uint16_t *)dk.data_ptr(), (uint16_t *)dv.data_ptr(),  \
-                       B, S, Hq, Hkv, (float)scale);                          \
-  } while (0)
-
-  if (DH == 128) RB_LAUNCH_BWD(128);
-  else RB_LAUNCH_BWD(64);
-#undef RB_LAUNCH_BWD
+  // Workgroups of two waves while there are too few tiles of 32 rows for four
+  // waves on every CU (us for 2 and 4 waves: 200 tokens, 12 heads of 64, 84
+  // tiles, 17 and 19; 512 tokens, 32 heads of 128, 512 tiles, 48 and 50; four
+  // times those 81 and 79).
+  const bool few = (int64_t)(S + 31) / 32 * Hq * B <= 512;
+  if (DH == 128)
+    few ? launch_bwd<128, 2>(a, stream) : launch_bwd<128, 4>(a, stream);
+  else
+    few ? launch_bwd<64, 2>(a, stream) : launch_bwd<64, 4>(a, stream);
   return {dq, dk, dv};
 }

@@ -318,11 +318,6 @@ void launch_prefill(const at::Tensor &q, const at::Tensor &k,
 
 }  // namespace
 
-// Contiguous values may start anywhere; the kernels load 16 bytes at a time.
-static at::Tensor aligned16(const at::Tensor &t) {
-  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 ? t.clone() : t;
-}
-
 static at::Tensor flash_fwd_impl(at::Tensor q, at::Tensor k, at::Tensor v,
                                  double scale, float *lsep) {
   TORCH_CHECK(q.is_cuda() && q.is_contiguous() && k.is_contiguous() &&
@@ -339,9 +334,9 @@ static at::Tensor flash_fwd_impl(at::Tensor q, at::Tensor k, at::Tensor v,
               v.scalar_type() == at::kBFloat16, "flash_prefill: k, v");
   auto out = at::empty_like(q);
   if (out.numel() == 0) return out;
-  q = aligned16(q);
-  k = aligned16(k);
-  v = aligned16(v);
+  q = flash::aligned16(q);
+  k = flash::aligned16(k);
+  v = flash::aligned16(v);
   if (DH == 128) launch_prefill<128>(q, k, v, out, lsep, (float)scale);
   else if (DH == 64) launch_prefill<64>(q, k, v, out, lsep, (float)scale);
   else if (DH == 256) launch_prefill<256>(q, k, v, out, lsep, (float)scale);

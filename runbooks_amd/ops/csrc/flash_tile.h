@@ -10,9 +10,16 @@
 // chunks, which a column read takes, fall on all 64 banks once.
 #pragma once
 
+#include <torch/extension.h>
+
 #include "common.h"
 
 namespace flash {
+
+// Contiguous values may start anywhere; the kernels load 16 bytes at a time.
+static inline at::Tensor aligned16(const at::Tensor &t) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 ? t.clone() : t;
+}
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8v;
 typedef __attribute__((ext_vector_type(16))) float f32x16v;

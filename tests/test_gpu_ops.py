@@ -411,6 +411,43 @@ def test_flash_prefill_tiles(B, S, Hq, Hkv, dh, scale):
             assert (lse[b, h] - s.logsumexp(-1)).abs().max() < 1e-5
 
 
+@pytest.mark.parametrize("B,S,Hq,Hkv,dh,scale", [
+    # up to 512 tiles of 32 rows, workgroups of 64 rows
+    (1, 2, 2, 1, 64, None), (2, 33, 3, 3, 128, -0.1), (1, 65, 2, 1, 128, 0.0),
+    (1, 97, 12, 12, 64, None),
+    # of 128 rows
+    (1, 545, 32, 8, 64, None), (2, 257, 40, 8, 128, None),
+    (3, 1001, 8, 8, 128, -0.05)])
+def test_flash_attention_bwd_tiles(B, S, Hq, Hkv, dh, scale):
+    """Gradients at remainders of the tiles, inputs off a 16-byte boundary,
+    from the result that the forward rounded. At most two roundings to bf16
+    (2^-9 relative) lie on the way to one; differences of dO V^T and D may be
+    half of their terms."""
+    _assert_hip()
+    g = torch.Generator(device=DEV).manual_seed(S)
+
+    def rows(h):
+        n = B * S * h * dh
+        return torch.randn(n + 1, generator=g, device=DEV).bfloat16()[1:] \
+            .view(B, S, h, dh)
+
+    q, k, v, dout = rows(Hq), rows(Hkv), rows(Hkv), rows(Hq)
+    scale = dh ** -0.5 if scale is None else scale
+    out, lse = ops.ext().flash_fwd_train(q, k, v, scale)
+    got = ops.ext().fa_bwd(dout, q, k, v, out, lse, scale)
+    hidden = torch.ones(S, S, dtype=torch.bool, device=DEV).triu(1)
+    for h in {0, Hq // 2, Hq - 1}:
+        at = h // (Hq // Hkv)
+        for b in range(B):
+            qs, ks, vs, do, o = (x[b, :, i].double() for x, i in (
+                (q, h), (k, at), (v, at), (dout, h), (out, h)))
+            p = (qs @ ks.t() * scale).masked_fill(
+                hidden, float("-inf")).softmax(-1)
+            ds = p * (do @ vs.t() - (do * o).sum(-1, keepdim=True)) * scale
+            for x, ref in zip(got, (ds @ ks, ds.t() @ qs, p.t() @ do)):
+                assert (x[b, :, h] - ref).norm() <= 2 ** -7 * ref.norm()
+
+
 @pytest.mark.parametrize("B,S,Hq,Hkv,dh", [
     (1, 64, 4, 4, 128),      # tiny, single WG tile
     (2, 333, 8, 2, 128),     # ragged S, GQA (group-summed dk/dv)

@@ -20,6 +20,8 @@ at::Tensor decode_gemm_raw(at::Tensor xs, at::Tensor ws, int64_t M, int64_t N, i
 at::Tensor decode_gemm(at::Tensor xs, at::Tensor ws, int64_t M, int64_t N, int64_t K, int64_t force_split);
 at::Tensor decode_swizzle_w(at::Tensor w);
 at::Tensor decode_swizzle_x(at::Tensor x);
+at::Tensor decode_swizzle_w8(at::Tensor w8);
+at::Tensor decode_gemm_fp8(at::Tensor xs, at::Tensor w8s, at::Tensor scale, int64_t M, int64_t N, int64_t K, bool raw);
 int64_t decode_gemm_split(int64_t N, int64_t K);
 bool decode_gemm_supported(int64_t M, int64_t N, int64_t K);
 at::Tensor sample_tokens(at::Tensor logits, double temperature, int64_t seed);
@@ -61,6 +63,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "one-time [N,K] -> fragment-lane-major weight layout");
   m.def("decode_swizzle_x", &decode_swizzle_x,
         "per-call x -> B-fragment lane order (zero-padded to M=32)");
+  m.def("decode_swizzle_w8", &decode_swizzle_w8,
+        "one-time weight layout swizzle for decode_gemm_fp8");
+  m.def("decode_gemm_fp8", &decode_gemm_fp8,
+        "decode GEMM with e4m3 weights and a scale per row",
+        py::arg("xs"), py::arg("w8s"), py::arg("scale"), py::arg("M"),
+        py::arg("N"), py::arg("K"), py::arg("raw") = false);
   m.def("decode_gemm_split", &decode_gemm_split);
   m.def("decode_gemm_supported", &decode_gemm_supported);
   m.def("sample_tokens", &sample_tokens, "greedy / Gumbel-max sampling");

@@ -19,9 +19,8 @@
 //    padding for m >= M; after that every wave reads the same contiguous
 //    L2-resident stream.
 //  * One wave owns 32 W rows x a DEEP contiguous k-range (K/(4*SPLIT)),
-//    no LDS and no barrier in the main loop (hipcc pipelines the 2x8
-//    ping-pong register ring freely; ~16 KB in flight per wave vs the
-//    ~9 KB/CU Little's-law requirement at 24.6 GB/s/CU).
+//    no LDS and no barrier in the main loop: a ring of two chunks in
+//    registers.
 //  * 4 waves per WG take adjacent k-quarters; one 16 KB LDS reduction
 //    combines them. SPLIT (1 for N>=16k, 2-4 for N=4096 shapes) adds
 //    fp32 slabs [SPLIT,M,N] reduced by a combine kernel (~1 MB next to
@@ -35,8 +34,6 @@
 // Reference parity: replaces hipBLASLt for the decode hot loop the way
 // the reference's external server image leans on cuBLAS
 // (substratusai/runbooks docs/container-contract.md serving contract).
-
-#include <stdlib.h>
 
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -52,87 +49,21 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8v;
 typedef __attribute__((ext_vector_type(16))) float f32x16v;
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4v;
 
-__device__ __forceinline__ bf16x8v nt_load8v(const uint16_t *p) {
-  union { u32x4v u; bf16x8v v; } c;
-  c.u = __builtin_nontemporal_load(reinterpret_cast<const u32x4v *>(p));
-  return c.v;
-}
-
 __device__ __forceinline__ bf16x8v load8v(const uint16_t *p) {
   union { u32x4v u; bf16x8v v; } c;
   c.u = *reinterpret_cast<const u32x4v *>(p);
   return c.v;
 }
 
-// One chunk of U k-steps. W nontemporal (streamed once, must not evict
-// L2); x plain (re-read by every n-block: L2 is exactly where it wants
-// to live). Both streams are lane*16B contiguous per instruction.
-#define RB_LOAD_CHUNK(WB, XB, SBASE)                                   \
-  _Pragma("unroll") for (int u = 0; u < U; ++u) {                      \
-    WB[u] = nt_load8v(wseg + (int64_t)((SBASE) + u) * 512 + lane8);    \
-    XB[u] = load8v(xs + (int64_t)((SBASE) + u) * 512 + lane8);         \
-  }
-
-#define RB_MFMA_CHUNK(WB, XB)                                          \
-  _Pragma("unroll") for (int u = 0; u < U; ++u) {                      \
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(WB[u], XB[u], acc,   \
-                                                  0, 0, 0);            \
-  }
-
-// STORE_BF16: write y bf16 directly (SPLIT == 1). Otherwise store an
-// fp32 slab slice at slabs + kslice*M*N for decode_gemm_combine.
-// U = k-steps (of 16) per unrolled chunk: 8 keeps 3 waves/SIMD, 12
-// trades occupancy (2/SIMD) for a deeper in-flight ring (RB_DG_U=12).
-template <bool STORE_BF16, int U = 8>
-__global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
-    const uint16_t *__restrict__ xs, const uint16_t *__restrict__ ws,
-    uint16_t *__restrict__ yp, float *__restrict__ slabs,
-    int M, int N, int K) {
-  const int tid = threadIdx.x;
-  const int wid = tid >> 6;
-  const int lane = tid & 63;
-  const int hi = lane >> 5;
-  const int col = lane & 31;
-  const int lane8 = lane * 8;
-
-  const int nblk = blockIdx.x;           // 32 W rows per WG
-  const int kslice = blockIdx.y;
-  const int split = gridDim.y;
-
-  // k-step range (steps of 16) for this (kslice, wave) group; contiguous
-  // per group so the W stream is one long sequential burst.
-  const int steps_total = K / 16;
-  const int ngroups = split * 4;
-  const int spg = (steps_total + ngroups - 1) / ngroups;
-  const int g = kslice * 4 + wid;
-  const int s0 = g * spg;
-  const int s1 = min(steps_total, s0 + spg);
-
-  const uint16_t *wseg = ws + (int64_t)nblk * steps_total * 512;
-
-  f32x16v acc = (f32x16v)(0.0f);
-
-  bf16x8v wA[U], xA[U], wB[U], xB[U];
-  int s = s0;
-  const int nmain = ((s1 - s0) / (2 * U)) * (2 * U);
-  if (nmain > 0) {
-    RB_LOAD_CHUNK(wA, xA, s);
-    const int smain = s0 + nmain;
-    for (; s + 2 * U <= smain; s += 2 * U) {
-      if (s + U < smain) { RB_LOAD_CHUNK(wB, xB, s + U); }
-      RB_MFMA_CHUNK(wA, xA);
-      if (s + 2 * U < smain) { RB_LOAD_CHUNK(wA, xA, s + 2 * U); }
-      if (s + U < smain) { RB_MFMA_CHUNK(wB, xB); }
-    }
-  }
-  // tail: single k-steps, no prefetch (<= 2U-1 iterations)
-  for (; s < s1; ++s) {
-    bf16x8v w1 = nt_load8v(wseg + (int64_t)s * 512 + lane8);
-    bf16x8v x1 = load8v(xs + (int64_t)s * 512 + lane8);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w1, x1, acc, 0, 0, 0);
-  }
-
-  // ---- cross-wave reduction in LDS -------------------------------------
+// Sums the four waves' accumulators of 32 rows of W and stores them, times the
+// rows' scales where there are any: y, or a slice of the slabs.
+template <bool STORE_BF16>
+__device__ __forceinline__ void finish(const f32x16v &acc, const float *scale,
+                                       uint16_t *yp, float *slabs, int M,
+                                       int N) {
+  const int tid = threadIdx.x, wid = tid >> 6;
+  const int hi = (tid & 63) >> 5, col = tid & 31;
+  const int nblk = blockIdx.x, kslice = blockIdx.y;
   __shared__ __attribute__((aligned(16))) float red[4][32][MMAX];
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
@@ -150,6 +81,7 @@ __global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
     for (int j = 0; j < 4; ++j) {
       sum[j] = red[0][en + j][em] + red[1][en + j][em] +
                red[2][en + j][em] + red[3][en + j][em];
+      if (scale != nullptr) sum[j] *= scale[nblk * 32 + en + j];
     }
     if (STORE_BF16) {
       union { uint16_t u[4]; uint64_t q; } o;
@@ -163,6 +95,113 @@ __global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
           make_float4(sum[0], sum[1], sum[2], sum[3]);
     }
   }
+}
+
+// Two words of e4m3 -> 8 bf16 (exact).
+__device__ __forceinline__ bf16x8v fp8_to_bf16(unsigned lo, unsigned up) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2v;
+  union { bf16x2v h[4]; bf16x8v v; } c;
+  c.h[0] = __builtin_convertvector(
+      __builtin_amdgcn_cvt_pk_f32_fp8(lo, false), bf16x2v);
+  c.h[1] = __builtin_convertvector(
+      __builtin_amdgcn_cvt_pk_f32_fp8(lo, true), bf16x2v);
+  c.h[2] = __builtin_convertvector(
+      __builtin_amdgcn_cvt_pk_f32_fp8(up, false), bf16x2v);
+  c.h[3] = __builtin_convertvector(
+      __builtin_amdgcn_cvt_pk_f32_fp8(up, true), bf16x2v);
+  return c.v;
+}
+
+// What a lane holds of a kilobyte of W: operands of 32 rows x 16 columns, or of
+// 32 rows x 32 columns in e4m3 (decode_swizzle_w, decode_swizzle_w8).
+template <bool FP8> struct Step {
+  static constexpr int X = FP8 ? 2 : 1;  // operands of x that go with it
+  u32x4v w;
+  bf16x8v x[X];
+};
+
+// STORE_BF16: write y bf16 directly (SPLIT == 1). Otherwise store an
+// fp32 slab slice at slabs + kslice*M*N for decode_gemm_combine.
+//
+// W nontemporal (streamed once, must not evict L2); x plain (re-read by every
+// n-block: L2 is exactly where it wants to live). Columns past M read the last
+// row again: their results are not stored, and x stays as short as it is.
+// Loads run a chunk of U kilobytes ahead, without a branch among them (one
+// makes the compiler wait for all of them); past a wave's range they read its
+// last kilobyte again.
+//
+// Bound by the weight stream, and with 32 rows by x (as long as W, or twice as
+// long as e4m3). us before -> now, weights out of cache, for N x K of
+// 12288 x 4096, 22016 x 4096, 4096 x 4096 and 4096 x 11008:
+//   bf16  1 row    23.1 -> 20.0  36.9 -> 32.3  8.9 -> 8.2  21.3 -> 17.3
+//         16 rows  24.3 -> 22.5  37.5 -> 33.1  9.1 -> 8.6  21.6 -> 17.7
+//         32 rows  23.5 -> 23.6  37.5 -> 38.3  9.3 -> 9.3  21.9 -> 20.2
+//   e4m3 (before: tiles through LDS, a slab slice per 256 columns)
+//         1 row    31.9 -> 13.8  47.3 -> 20.1  17.7 -> 6.3  39.5 -> 12.4
+//         16 rows  32.5 -> 14.1  49.3 -> 20.8  17.7 -> 6.5  37.7 -> 12.8
+//         32 rows  34.7 -> 17.7  56.5 -> 26.4  18.1 -> 7.7  38.1 -> 16.0
+template <bool FP8, bool STORE_BF16>
+__global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
+    const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws,
+    const float *__restrict__ scale, uint16_t *__restrict__ yp,
+    float *__restrict__ slabs, int M, int N, int K) {
+  constexpr int X = Step<FP8>::X, U = FP8 ? 4 : 8;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int hi = lane >> 5, col = lane & 31;
+  const int steps = K / (16 * X), groups = gridDim.y * 4;
+  const int g = blockIdx.y * 4 + wid;
+  const int s0 = (int)((int64_t)steps * g / groups);
+  const int s1 = (int)((int64_t)steps * (g + 1) / groups);
+  const uint8_t *wseg = ws + (int64_t)blockIdx.x * steps * 1024;
+  const unsigned wlane = lane * 16;
+  const unsigned xlane = (hi * 32 + min(col, M - 1)) * 8;
+
+  f32x16v acc = (f32x16v)(0.0f);
+  Step<FP8> a[U], b[U];
+  auto load = [&](Step<FP8> (&c)[U], int s) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t at = min(s + u, s1 - 1);
+      c[u].w = __builtin_nontemporal_load(
+          reinterpret_cast<const u32x4v *>(wseg + at * 1024 + wlane));
+#pragma unroll
+      for (int i = 0; i < X; ++i)
+        c[u].x[i] = load8v(xs + (at * X + i) * 512 + xlane);
+    }
+  };
+  auto multiply = [&](const Step<FP8> &c) {
+    if constexpr (FP8) {
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          fp8_to_bf16(c.w[0], c.w[1]), c.x[0], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          fp8_to_bf16(c.w[2], c.w[3]), c.x[1], acc, 0, 0, 0);
+    } else {
+      union { u32x4v u; bf16x8v v; } w;
+      w.u = c.w;
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w.v, c.x[0], acc, 0, 0, 0);
+    }
+  };
+  if (s0 < s1) {
+    int s = s0;
+    load(a, s);
+    for (; s + 2 * U < s1; s += 2 * U) {
+      load(b, s + U);
+#pragma unroll
+      for (int u = 0; u < U; ++u) multiply(a[u]);
+      load(a, s + 2 * U);
+#pragma unroll
+      for (int u = 0; u < U; ++u) multiply(b[u]);
+    }
+    load(b, s + U);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (s + u < s1) multiply(a[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (s + U + u < s1) multiply(b[u]);
+  }
+  finish<STORE_BF16>(acc, scale, yp, slabs, M, N);
 }
 
 // slabs [SPLIT, M, N] f32 -> y [M, N] bf16
@@ -263,16 +302,46 @@ at::Tensor decode_swizzle_x(at::Tensor x) {
   return xs;
 }
 
+// e4m3 bytes [N,K] -> [N/32][K/32][2][32][2][8]: a lane's 16 bytes are its
+// operands of two steps of 16 columns.
+at::Tensor decode_swizzle_w8(at::Tensor w8) {
+  TORCH_CHECK(w8.dim() == 2 && w8.scalar_type() == at::kByte &&
+              w8.is_contiguous(), "decode_swizzle_w8: contiguous bytes [N,K]");
+  const int64_t N = w8.size(0), K = w8.size(1);
+  TORCH_CHECK(N % 32 == 0 && K % 32 == 0, "decode_swizzle_w8: shape");
+  return w8.view({N / 32, 32, K / 32, 2, 2, 8})
+      .permute({0, 2, 4, 1, 3, 5}).contiguous();
+}
+
 // Raw variant for fused consumers: split == 1 returns y bf16 [M, N] (with
 // f32 a slab of one slice); split > 1 returns the fp32 slab [split, M, N]
 // UNCOMBINED — the consumer kernel (rmsnorm_res_slab_fwd_dec) folds the
 // slices while it reads, saving the combine launch inside the decode graph.
-static int dg_u() {
-  static int u = [] {
-    const char *e = getenv("RB_DG_U");
-    return (e != nullptr && atoi(e) == 12) ? 12 : 8;
-  }();
-  return u;
+template <bool FP8>
+static void launch(const at::Tensor &xs, const at::Tensor &ws,
+                   const float *scale, at::Tensor *y, at::Tensor *slabs,
+                   int split, int64_t M, int64_t N, int64_t K) {
+  const dim3 grid((unsigned)(N / 32), (unsigned)split);
+  auto stream = at::cuda::getCurrentHIPStream();
+  if (slabs == nullptr)
+    hipLaunchKernelGGL((decode_gemm_kernel<FP8, true>), grid, dim3(BLOCK), 0,
+                       stream, (const uint16_t *)xs.data_ptr(),
+                       (const uint8_t *)ws.data_ptr(), scale,
+                       (uint16_t *)y->data_ptr(), nullptr, (int)M, (int)N,
+                       (int)K);
+  else
+    hipLaunchKernelGGL((decode_gemm_kernel<FP8, false>), grid, dim3(BLOCK), 0,
+                       stream, (const uint16_t *)xs.data_ptr(),
+                       (const uint8_t *)ws.data_ptr(), scale, nullptr,
+                       slabs->data_ptr<float>(), (int)M, (int)N, (int)K);
+}
+
+static void combine(const at::Tensor &slabs, at::Tensor &y) {
+  hipLaunchKernelGGL(decode_gemm_combine_kernel,
+                     dim3(rb::rb_grid_1d(y.numel() / 4, 256)), dim3(256), 0,
+                     at::cuda::getCurrentHIPStream(),
+                     slabs.data_ptr<float>(), (uint16_t *)y.data_ptr(),
+                     (int)slabs.size(0), y.numel());
 }
 
 at::Tensor decode_gemm_raw(at::Tensor xs, at::Tensor ws, int64_t M,
@@ -282,39 +351,14 @@ at::Tensor decode_gemm_raw(at::Tensor xs, at::Tensor ws, int64_t M,
               ws.scalar_type() == at::kBFloat16, "decode_gemm_raw: inputs");
   TORCH_CHECK(xs.numel() == (K / 16) * 512 && ws.numel() == N * K &&
               decode_gemm_supported(M, N, K), "decode_gemm_raw: shape");
-  auto stream = at::cuda::getCurrentHIPStream();
   const int split = (int)decode_gemm_split(N, K);
   if (split == 1 && !f32) {
     auto y = at::empty({M, N}, xs.options());
-    if (dg_u() == 12)
-      hipLaunchKernelGGL((decode_gemm_kernel<true, 12>), dim3(N / 32, 1),
-                         dim3(BLOCK), 0, stream,
-                         (const uint16_t *)xs.data_ptr(),
-                         (const uint16_t *)ws.data_ptr(),
-                         (uint16_t *)y.data_ptr(), nullptr,
-                         (int)M, (int)N, (int)K);
-    else
-      hipLaunchKernelGGL((decode_gemm_kernel<true, 8>), dim3(N / 32, 1),
-                         dim3(BLOCK), 0, stream,
-                         (const uint16_t *)xs.data_ptr(),
-                         (const uint16_t *)ws.data_ptr(),
-                         (uint16_t *)y.data_ptr(), nullptr,
-                         (int)M, (int)N, (int)K);
+    launch<false>(xs, ws, nullptr, &y, nullptr, 1, M, N, K);
     return y;
   }
   auto slabs = at::empty({split, M, N}, xs.options().dtype(at::kFloat));
-  if (dg_u() == 12)
-    hipLaunchKernelGGL((decode_gemm_kernel<false, 12>), dim3(N / 32, split),
-                       dim3(BLOCK), 0, stream,
-                       (const uint16_t *)xs.data_ptr(),
-                       (const uint16_t *)ws.data_ptr(), nullptr,
-                       (float *)slabs.data_ptr(), (int)M, (int)N, (int)K);
-  else
-    hipLaunchKernelGGL((decode_gemm_kernel<false, 8>), dim3(N / 32, split),
-                       dim3(BLOCK), 0, stream,
-                       (const uint16_t *)xs.data_ptr(),
-                       (const uint16_t *)ws.data_ptr(), nullptr,
-                       (float *)slabs.data_ptr(), (int)M, (int)N, (int)K);
+  launch<false>(xs, ws, nullptr, nullptr, &slabs, split, M, N, K);
   return slabs;
 }
 
@@ -331,29 +375,43 @@ at::Tensor decode_gemm(at::Tensor xs, at::Tensor ws, int64_t M, int64_t N,
   TORCH_CHECK(decode_gemm_supported(M, N, K),
               "decode_gemm: unsupported shape ", M, "x", N, "x", K);
 
-  auto stream = at::cuda::getCurrentHIPStream();
   auto y = at::empty({M, N}, xs.options());
   const int split = force_split > 0 ? (int)force_split
                                     : (int)decode_gemm_split(N, K);
   if (split == 1) {
-    hipLaunchKernelGGL((decode_gemm_kernel<true>), dim3(N / 32, 1),
-                       dim3(BLOCK), 0, stream,
-                       (const uint16_t *)xs.data_ptr(),
-                       (const uint16_t *)ws.data_ptr(),
-                       (uint16_t *)y.data_ptr(), nullptr,
-                       (int)M, (int)N, (int)K);
-  } else {
-    auto slabs = at::empty({split, M, N}, xs.options().dtype(at::kFloat));
-    hipLaunchKernelGGL((decode_gemm_kernel<false>), dim3(N / 32, split),
-                       dim3(BLOCK), 0, stream,
-                       (const uint16_t *)xs.data_ptr(),
-                       (const uint16_t *)ws.data_ptr(), nullptr,
-                       (float *)slabs.data_ptr(), (int)M, (int)N, (int)K);
-    const int64_t mn = M * N;
-    const int grid = rb::rb_grid_1d(mn / 4, 256);
-    hipLaunchKernelGGL(decode_gemm_combine_kernel, dim3(grid), dim3(256),
-                       0, stream, (const float *)slabs.data_ptr(),
-                       (uint16_t *)y.data_ptr(), split, mn);
+    launch<false>(xs, ws, nullptr, &y, nullptr, 1, M, N, K);
+    return y;
   }
+  auto slabs = at::empty({split, M, N}, xs.options().dtype(at::kFloat));
+  launch<false>(xs, ws, nullptr, nullptr, &slabs, split, M, N, K);
+  combine(slabs, y);
+  return y;
+}
+
+// The product with e4m3 weights (decode_swizzle_w8) and a scale per row:
+// y [M, N] bf16, or with raw=true, where it is split, the uncombined fp32
+// slabs [split, M, N].
+at::Tensor decode_gemm_fp8(at::Tensor xs, at::Tensor w8s, at::Tensor scale,
+                           int64_t M, int64_t N, int64_t K, bool raw) {
+  TORCH_CHECK(xs.is_cuda() && w8s.is_cuda() && scale.is_cuda() &&
+              xs.is_contiguous() && w8s.is_contiguous() &&
+              scale.is_contiguous() && xs.scalar_type() == at::kBFloat16 &&
+              w8s.scalar_type() == at::kByte &&
+              scale.scalar_type() == at::kFloat, "decode_gemm_fp8: inputs");
+  TORCH_CHECK(M >= 1 && M <= MMAX && N % 32 == 0 && K % 32 == 0 && K > 0 &&
+              xs.numel() == (K / 16) * 512 && w8s.numel() == N * K &&
+              scale.numel() == N, "decode_gemm_fp8: shape");
+  const int split = (int)decode_gemm_split(N, K);
+  auto y = split > 1 && raw ? at::Tensor() : at::empty({M, N}, xs.options());
+  if (split == 1) {
+    if (N > 0)
+      launch<true>(xs, w8s, scale.data_ptr<float>(), &y, nullptr, 1, M, N, K);
+    return y;
+  }
+  auto slabs = at::empty({split, M, N}, xs.options().dtype(at::kFloat));
+  launch<true>(xs, w8s, scale.data_ptr<float>(), nullptr, &slabs, split, M, N,
+               K);
+  if (raw) return slabs;
+  combine(slabs, y);
   return y;
 }

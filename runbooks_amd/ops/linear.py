@@ -22,9 +22,9 @@ _USE_SKINNY = os.environ.get("RB_SKINNY_GEMM", "0") == "1"
 _USE_DECODE_GEMM = os.environ.get("RB_DECODE_GEMM", "1") == "1"
 
 
-# data_ptr(weight) -> (w8 uint8 view, f32 per-channel scale). Populated by
-# quantize_fp8 (serving with MODEL_LOAD_IN_8BIT); looked up on the decode
-# fast path.
+# data_ptr(weight) -> (e4m3 bytes in the decode GEMM's order, f32 per-channel
+# scale, weakref to the weight). Populated by quantize_fp8 (serving with
+# MODEL_LOAD_IN_8BIT); looked up on the decode fast path.
 _FP8_REGISTRY: dict[int, tuple[torch.Tensor, torch.Tensor]] = {}
 
 # data_ptr(weight) -> fragment-lane-major copy ([N/32][K/16][lane][8])
@@ -60,6 +60,11 @@ def register_decode_weight(weight: torch.Tensor) -> None:
 E4M3_MAX = 448.0
 
 
+def _fp8_served(n: int, k: int) -> bool:
+    """Sizes of a weight that the fp8 decode GEMM takes."""
+    return n % 64 == 0 and k % 256 == 0
+
+
 @torch.no_grad()
 def quantize_fp8(weight: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """Row-wise (per-output-channel) OCP e4m3 quantization; registers the
@@ -69,7 +74,9 @@ def quantize_fp8(weight: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     scale = weight.float().abs().amax(dim=1).clamp(min=1e-8) / E4M3_MAX
     w8 = (weight.float() / scale[:, None]).to(torch.float8_e4m3fn)
     w8_bytes = w8.view(torch.uint8).contiguous()
-    _FP8_REGISTRY[weight.data_ptr()] = (w8_bytes, scale.contiguous(),
+    served = (_backend.ext().decode_swizzle_w8(w8_bytes)
+              if weight.is_cuda and _fp8_served(*weight.shape) else w8_bytes)
+    _FP8_REGISTRY[weight.data_ptr()] = (served, scale.contiguous(),
                                         weakref.ref(weight))
     return w8_bytes, scale
 
@@ -78,6 +85,14 @@ def dequantize_fp8(w8_bytes: torch.Tensor, scale: torch.Tensor,
                    dtype=torch.bfloat16) -> torch.Tensor:
     return (w8_bytes.view(torch.float8_e4m3fn).float() *
             scale[:, None]).to(dtype)
+
+
+def _swizzled(x: torch.Tensor, m: int, k: int) -> torch.Tensor:
+    """x as the decode GEMM's operand: producers (rmsnorm_fwd_dec,
+    *_packed_dec) attach it; otherwise one tiny kernel builds it here."""
+    xs = getattr(x, "_rb_swz", None)
+    return xs if xs is not None else _backend.ext().decode_swizzle_x(
+        x.reshape(m, k).contiguous())
 
 
 def fast_linear(x: torch.Tensor, weight: torch.Tensor,
@@ -89,23 +104,17 @@ def fast_linear(x: torch.Tensor, weight: torch.Tensor,
         m = x.numel() // k
         n = weight.shape[0]
         if m <= 32:
-            if n % 64 == 0 and k % 256 == 0:
+            if _fp8_served(n, k):
                 q = _registry_get(_FP8_REGISTRY, weight)
                 if q is not None:
-                    y = _backend.ext().skinny_gemm_fp8(
-                        x.reshape(m, k).contiguous(), q[0], q[1])
+                    y = _backend.ext().decode_gemm_fp8(
+                        _swizzled(x, m, k), q[0], q[1], m, n, k)
                     return y.view(*x.shape[:-1], n)
             if _USE_DECODE_GEMM:
                 dw = _registry_get(_DECODE_W_REGISTRY, weight)
                 if dw is not None:
-                    # producers (rmsnorm_fwd_dec, *_packed_dec) attach the
-                    # pre-swizzled operand; otherwise one tiny swizzle
-                    # kernel builds it here
-                    xs = getattr(x, "_rb_swz", None)
-                    if xs is None:
-                        xs = _backend.ext().decode_swizzle_x(
-                            x.reshape(m, k).contiguous())
-                    y = _backend.ext().decode_gemm(xs, dw[0], m, n, k)
+                    y = _backend.ext().decode_gemm(_swizzled(x, m, k), dw[0],
+                                                   m, n, k)
                     return y.view(*x.shape[:-1], n)
             if _USE_SKINNY and n % 64 == 0 and k % 256 == 0:
                 y = _backend.ext().skinny_gemm(x.reshape(m, k).contiguous(),
@@ -120,16 +129,20 @@ def decode_linear_raw(x, weight, f32: bool = False):
     or a plain bf16 [M, N]; with f32=True always the slab (of one slice
     where the product is not split). Falls back to fast_linear when the
     weight has no registered decode layout. Returns (out, is_slab)."""
+    k = x.shape[-1]
+    m = x.numel() // k
+    n = weight.shape[0]
+    q = None if f32 or not _fp8_served(n, k) else \
+        _registry_get(_FP8_REGISTRY, weight)
+    if q is not None and m <= 32 and x.dtype == torch.bfloat16:
+        out = _backend.ext().decode_gemm_fp8(_swizzled(x, m, k), q[0], q[1],
+                                             m, n, k, True)
+        return out, out.dtype == torch.float32
     dw = _registry_get(_DECODE_W_REGISTRY, weight)
     if dw is None or not _USE_DECODE_GEMM:
         with torch.no_grad():
             return fast_linear(x, weight), False
-    k = x.shape[-1]
-    m = x.numel() // k
-    n = weight.shape[0]
-    xs = getattr(x, "_rb_swz", None)
-    if xs is None:
-        xs = _backend.ext().decode_swizzle_x(x.reshape(m, k).contiguous())
+    xs = _swizzled(x, m, k)
     out = _backend.ext().decode_gemm_raw(xs, dw[0], m, n, k, f32)
     return out, out.dtype == torch.float32
 

@@ -523,6 +523,29 @@ def test_cross_entropy_fwd_bwd(V):
                           rtol=2e-2), (logits.grad.cpu().float() - lc.grad).abs().max()
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1, 64, 256), (2, 96, 32), (7, 4096, 11008), (16, 12288, 4096),
+    (31, 4096, 4096), (32, 22016, 2080)])
+def test_decode_gemm_fp8(M, N, K):
+    """Both outputs against the product with the dequantized weights: exact
+    products, fp32 sums (their order: 1e-5), y rounded to bf16."""
+    _assert_hip()
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w8 = torch.randn(N, K, generator=g, device=DEV).to(torch.float8_e4m3fn)
+    scale = torch.rand(N, generator=g, device=DEV) + 0.5
+    ref = x.double() @ (w8.double() * scale.double()[:, None]).t()
+    e = ops.ext()
+    args = (e.decode_swizzle_x(x), e.decode_swizzle_w8(w8.view(torch.uint8)),
+            scale, M, N, K)
+    assert (e.decode_gemm_fp8(*args) - ref).norm() < 2 ** -8 * ref.norm()
+    raw = e.decode_gemm_fp8(*args, raw=True)
+    split = e.decode_gemm_split(N, K)
+    assert raw.dtype == (torch.float32 if split > 1 else torch.bfloat16)
+    if split > 1:
+        assert (raw.double().sum(0) - ref).norm() < 1e-5 * ref.norm()
+
+
 def test_skinny_gemm_fp8():
     """fp8 weight-only decode GEMM vs matmul on the dequantized weights
     (exact dequant path) and vs the original bf16 weights (e4m3 bound)."""

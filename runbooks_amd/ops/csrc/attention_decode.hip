@@ -31,14 +31,13 @@ constexpr int NW = 4;
 
 typedef __attribute__((ext_vector_type(8))) __bf16 rb_bf16x8v;
 typedef __attribute__((ext_vector_type(2))) __bf16 rb_bf16x2v;
-typedef __attribute__((ext_vector_type(16))) float rb_f32x16v;
 typedef __attribute__((ext_vector_type(4))) float rb_f32x4v;
 
 RB_DEV unsigned rb_pack_bf16(float lo, float hi) {
-  union { __bf16 b; unsigned short u; } a, b;
-  a.b = (__bf16)lo;
-  b.b = (__bf16)hi;
-  return ((unsigned)b.u << 16) | a.u;
+  typedef __attribute__((ext_vector_type(2))) float f32x2v;
+  union { rb_bf16x2v v; unsigned u; } c;
+  c.v = __builtin_convertvector((f32x2v){lo, hi}, rb_bf16x2v);
+  return c.u;
 }
 
 // one v_dot2_f32_bf16: c += a_pair . b_pair (packed bf16 pairs)
@@ -47,6 +46,16 @@ RB_DEV float rb_dot2(unsigned a, unsigned b, float c) {
   x.u = a;
   y.u = b;
   return __builtin_amdgcn_fdot2_f32_bf16(x.v, y.v, c, false);
+}
+
+// The sequence of a workgroup. Workgroups 256 apart in launch order share a CU;
+// in plain order those would be heads of one sequence wherever the batch divides
+// 256, and the CUs of the longest ones would run long after the others. The
+// sequences are shifted with head and split, once around over the whole grid:
+// a CU gets sequences spread evenly over the batch.
+RB_DEV int sequence_of() {
+  const unsigned y = blockIdx.y + gridDim.y * blockIdx.z;
+  return (blockIdx.x + y * gridDim.x / (gridDim.y * gridDim.z)) % gridDim.x;
 }
 
 // FP8: caches are e4m3 rows of fp8_row_bytes(DH) = DH bytes + f32
@@ -82,7 +91,7 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
   // iteration, and removes the cross-wave LDS merge entirely.
   constexpr bool HS = (G >= NW);
   constexpr int GW = HS ? G / NW : G;
-  const int b = blockIdx.x;
+  const int b = sequence_of();
   const int h_kv = blockIdx.y;
   const int split = SPLIT ? blockIdx.z : 0;
   const int hq0 = h_kv * G;
@@ -109,11 +118,9 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
   const int gl = lane % GL;                // lane within group
   const int d0 = gl * VE;                  // this lane's Dh slice
 
-  // Q for this wave's GW heads, pre-scaled (softmax scale folded in).
-  // bf16 caches keep Q as PACKED bf16 pairs too: the K dot then runs on
-  // v_dot2_f32_bf16 straight from the raw K words — no per-element
-  // convert+FMA chain (the kernel is VALU-saturated at occupancy 8;
-  // the same q*scale->bf16 rounding the MFMA kernel already makes).
+  // Q for this wave's GW heads. bf16 caches keep Q as PACKED bf16 pairs: the
+  // K dot then runs on v_dot2_f32_bf16 straight from the raw K words — no
+  // per-element convert+FMA chain — and is scaled in fp32.
   const int hq_base = hq0 + (HS ? wid * GW : 0);
   float qreg[GW][VE];
   unsigned qpk[GW][VE / 2];
@@ -139,8 +146,7 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
       } else {
 #pragma unroll
         for (int e2 = 0; e2 < VE / 2; ++e2)
-          qpk[g][e2] = rb_pack_bf16(tmp[2 * e2] * scale,
-                                    tmp[2 * e2 + 1] * scale);
+          qpk[g][e2] = rb_pack_bf16(tmp[2 * e2], tmp[2 * e2 + 1]);
       }
     }
   }
@@ -170,49 +176,58 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
   }
   __syncthreads();
 
-  // Software-pipelined KV stream: iteration i+1's K/V rows are issued
-  // as RAW bytes while i is computed. (Converting at load time puts an
-  // s_waitcnt vmcnt(0) between every row and its dot product — the
-  // unpipelined loop measured ~3.9 TB/s effective in-situ vs ~6 TB/s
-  // streaming.) Tail iterations clamp to the last row; the duplicate
-  // rows are masked out of the softmax with s = -inf, so the trip
-  // count is wave-uniform and the prefetch is branch-free inside.
+  // Software-pipelined KV stream: the K/V rows of later steps are issued as
+  // RAW bytes while one is computed. (Converting at load time puts an
+  // s_waitcnt vmcnt(0) between every row and its dot product.) Tail steps clamp
+  // to the last row; the duplicate rows are masked out of the softmax with
+  // s = -inf, so the trip count is wave-uniform and the prefetch is
+  // branch-free inside.
+  //
+  // A step is TPS tokens of every lane group, TPS * TPW consecutive ones of a
+  // wave. With few query heads the chain dot -> reduce -> exp -> accumulate is
+  // what a step takes, and two tokens share it; the longest sequence of a batch
+  // is one workgroup's chain.
+  // us, 32 heads of 128, before (plain order of the sequences, one token a
+  // step) and now: 32 sequences of 129 to 2015 tokens 141 -> 119 (4.7 TB/s),
+  // of 1072 each 102 -> 106 (5.3); one of 701 in one split 35 -> 23, with 16
+  // splits and their merge 13.2 -> 11.2; 16 of 800 to 3900 from an e4m3 cache
+  // 93 -> 79.
   constexpr int KBPL = FP8 ? VE : VE * 2;  // K/V bytes per lane
   constexpr int RW = KBPL / 4;             // u32 words of that
-  // Ring depth: the G>=4 instantiations are VGPR-capped at 2 waves/SIMD
-  // (qreg+acc alone are 2*G*VE floats), so two waves must hide the full
-  // HBM latency — a 4-deep ring keeps 3 iterations of K/V in flight for
-  // only +4*RW VGPRs. G<=2 runs 5-8 waves/SIMD where depth 2 suffices
-  // (deeper costs occupancy: 62->78 VGPRs drops the MHA kernel 8->6).
+  constexpr int TPS = GW == 1 || (GW == 2 && !FP8) ? 2 : 1;
   constexpr int DEPTH = (G >= 4) ? 4 : 2;
-  const int stride = HS ? TPW : NW * TPW;
-  const int tw0 = t_begin + (HS ? 0 : wid * TPW);  // wave's first token
+  const int stride = (HS ? 1 : NW) * TPW * TPS;    // tokens of a step
+  const int tw0 = t_begin + (HS ? 0 : wid * TPW * TPS);  // wave's first token
   const int t_base = tw0 + grp;            // this lane group's first
   const int niter = (t_end > tw0) ? (t_end - tw0 + stride - 1) / stride : 0;
 
-  uint32_t kraw[DEPTH][RW], vraw[DEPTH][RW];
-  float kscale[DEPTH], vscale[DEPTH];
+  uint32_t kraw[DEPTH][TPS][RW], vraw[DEPTH][TPS][RW];
+  float kscale[DEPTH][TPS], vscale[DEPTH][TPS];
 
   auto fetch = [&](int i, int slot) {
-    const int tt = min(t_base + i * stride, t_end - 1);
-    const int bi = tt / bs - blk0;
-    const int blk = (bi < BT_LDS) ? bt_lds[bi] : bt[tt / bs];
-    if (FP8) {
-      constexpr int RB8 = DH + 16;
-      const uint8_t *k8 = reinterpret_cast<const uint8_t *>(k_cache);
-      const uint8_t *v8 = reinterpret_cast<const uint8_t *>(v_cache);
-      const int64_t row = (((int64_t)blk * hkv + h_kv) * bs + (tt % bs)) * RB8;
-      rb::ld_words<RW>(kraw[slot], k8 + row + d0);
-      rb::ld_words<RW>(vraw[slot], v8 + row + d0);
-      kscale[slot] = *reinterpret_cast<const float *>(k8 + row + DH);
-      vscale[slot] = *reinterpret_cast<const float *>(v8 + row + DH);
-    } else {
-      const int64_t base =
-          (((int64_t)blk * hkv + h_kv) * bs + (tt % bs)) * DH + d0;
-      rb::ld_words<RW>(kraw[slot],
-                       reinterpret_cast<const uint8_t *>(k_cache + base));
-      rb::ld_words<RW>(vraw[slot],
-                       reinterpret_cast<const uint8_t *>(v_cache + base));
+#pragma unroll
+    for (int u = 0; u < TPS; ++u) {
+      const int tt = min(t_base + i * stride + u * TPW, t_end - 1);
+      const int bi = tt / bs - blk0;
+      const int blk = (bi < BT_LDS) ? bt_lds[bi] : bt[tt / bs];
+      if (FP8) {
+        constexpr int RB8 = DH + 16;
+        const uint8_t *k8 = reinterpret_cast<const uint8_t *>(k_cache);
+        const uint8_t *v8 = reinterpret_cast<const uint8_t *>(v_cache);
+        const int64_t row =
+            (((int64_t)blk * hkv + h_kv) * bs + (tt % bs)) * RB8;
+        rb::ld_words<RW>(kraw[slot][u], k8 + row + d0);
+        rb::ld_words<RW>(vraw[slot][u], v8 + row + d0);
+        kscale[slot][u] = *reinterpret_cast<const float *>(k8 + row + DH);
+        vscale[slot][u] = *reinterpret_cast<const float *>(v8 + row + DH);
+      } else {
+        const int64_t base =
+            (((int64_t)blk * hkv + h_kv) * bs + (tt % bs)) * DH + d0;
+        rb::ld_words<RW>(kraw[slot][u],
+                         reinterpret_cast<const uint8_t *>(k_cache + base));
+        rb::ld_words<RW>(vraw[slot][u],
+                         reinterpret_cast<const uint8_t *>(v_cache + base));
+      }
     }
   };
 
@@ -220,50 +235,64 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
   // ring buffer stays in registers (no dynamic indexing).
   auto step = [&](int i, int cur) {
     if (i + DEPTH - 1 < niter) fetch(i + DEPTH - 1, (cur + DEPTH - 1) % DEPTH);
-    const bool valid = t_base + i * stride < t_end;
-
-    float kf[VE], vf[VE];
-    if (FP8) {
-#pragma unroll
-      for (int w = 0; w < RW; ++w) {
-        rb::fp8w_to_f32(kraw[cur][w], kf + w * 4);
-        rb::fp8w_to_f32(vraw[cur][w], vf + w * 4);
-      }
-      const float ks = kscale[cur], vs = vscale[cur];
-#pragma unroll
-      for (int e = 0; e < VE; ++e) { kf[e] *= ks; vf[e] *= vs; }
-    } else {
-      // only V needs f32 elements (the p*v accumulate); the K dot runs
-      // packed below, straight from the raw words
-      const uint16_t *vr = reinterpret_cast<const uint16_t *>(vraw[cur]);
-#pragma unroll
-      for (int e = 0; e < VE; ++e) vf[e] = rb::bf16_to_f32(vr[e]);
-    }
-
 #pragma unroll
     for (int g = 0; g < GW; ++g) {
-      float s = 0.f;
-      if (FP8) {
+      float sc[TPS], mn = m[g];
 #pragma unroll
-        for (int e = 0; e < VE; ++e) s += qreg[g][e] * kf[e];
-      } else {
+      for (int u = 0; u < TPS; ++u) {
+        float x = 0.f;
+        if (FP8) {
+          float kf[VE];
 #pragma unroll
-        for (int e2 = 0; e2 < VE / 2; ++e2)
-          s = rb_dot2(kraw[cur][e2], qpk[g][e2], s);
+          for (int w = 0; w < RW; ++w)
+            rb::fp8w_to_f32(kraw[cur][u][w], kf + w * 4);
+#pragma unroll
+          for (int e = 0; e < VE; ++e) x += qreg[g][e] * kf[e];
+          x *= kscale[cur][u];
+        } else {
+          // the K dot runs packed, straight from the raw words
+#pragma unroll
+          for (int e2 = 0; e2 < VE / 2; ++e2)
+            x = rb_dot2(kraw[cur][u][e2], qpk[g][e2], x);
+          x *= scale;
+        }
+        sc[u] = x;
       }
       // reduce across the lane group
 #pragma unroll
       for (int off = GL / 2; off > 0; off >>= 1)
-        s += __shfl_xor(s, off, 64);
-      if (!valid) s = -INFINITY;
-      const float mn = fmaxf(m[g], s);
+#pragma unroll
+        for (int u = 0; u < TPS; ++u) sc[u] += __shfl_xor(sc[u], off, 64);
+#pragma unroll
+      for (int u = 0; u < TPS; ++u) {
+        if (t_base + i * stride + u * TPW >= t_end) sc[u] = -INFINITY;
+        mn = fmaxf(mn, sc[u]);
+      }
       if (mn != -INFINITY) {
         const float alpha = __expf(m[g] - mn);
-        const float p = __expf(s - mn);
-        l[g] = l[g] * alpha + p;
-#pragma unroll
-        for (int e = 0; e < VE; ++e) acc[g][e] = acc[g][e] * alpha + p * vf[e];
         m[g] = mn;
+        l[g] *= alpha;
+#pragma unroll
+        for (int e = 0; e < VE; ++e) acc[g][e] *= alpha;
+#pragma unroll
+        for (int u = 0; u < TPS; ++u) {
+          float p = __expf(sc[u] - mn);
+          l[g] += p;
+          float vf[VE];
+          if (FP8) {
+#pragma unroll
+            for (int w = 0; w < RW; ++w)
+              rb::fp8w_to_f32(vraw[cur][u][w], vf + w * 4);
+            p *= vscale[cur][u];
+          } else {
+            const uint16_t *vr =
+                reinterpret_cast<const uint16_t *>(vraw[cur][u]);
+#pragma unroll
+            for (int e = 0; e < VE; ++e) vf[e] = rb::bf16_to_f32(vr[e]);
+          }
+#pragma unroll
+          for (int e = 0; e < VE; ++e) acc[g][e] += p * vf[e];
+        }
       }
     }
   };
@@ -272,10 +301,9 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
   for (int d = 0; d < DEPTH - 1; ++d)
     if (d < niter) fetch(d, d);
   for (int i = 0; i < niter; i += DEPTH) {
-    step(i, 0);
-    if (i + 1 < niter) step(i + 1, 1 % DEPTH);
-    if (DEPTH > 2 && i + 2 < niter) step(i + 2, 2 % DEPTH);
-    if (DEPTH > 2 && i + 3 < niter) step(i + 3, 3 % DEPTH);
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+      if (i + d < niter) step(i + d, d);
   }
 
   // Merge the TPW groups inside each wave: lanes l^GL ... l^32 hold the
@@ -395,33 +423,53 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
   }
 }
 
-// Second pass for SPLIT mode: merge nsplit partials per (b, hq) row.
-__global__ void decode_combine_kernel(const float *__restrict__ partial,
-                                      uint16_t *__restrict__ out,
-                                      uint16_t *__restrict__ out_swz,
-                                      int Hq, int nsplit,
-                                      int dh) {
-  const int64_t row = blockIdx.x;          // b * Hq + hq
-  const float *p = partial + row * (int64_t)nsplit * (dh + 2);
+// Second pass for SPLIT mode: a wave merges the nsplit partials of one (b, hq)
+// row. The maxima and sums are one load of the wave, the rows (VE = dh / 64
+// values a lane) are loaded eight at a time: two round trips to memory where
+// loops over the splits made three per split (both kernels, one sequence of 4000
+// tokens, 8 kv heads, 16 splits: 23.1 -> 14.4 us with this change alone).
+template <int VE>
+__global__ __launch_bounds__(256) void decode_combine_kernel(
+    const float *__restrict__ partial, uint16_t *__restrict__ out,
+    uint16_t *__restrict__ out_swz, int rows, int Hq, int nsplit) {
+  constexpr int DH = VE * 64;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);  // b * Hq + hq
+  if (row >= rows) return;
+  const int lane = threadIdx.x & 63, d0 = lane * VE;
+  const float *p = partial + (int64_t)row * nsplit * (DH + 2);
   float mm = -INFINITY;
-  for (int s = 0; s < nsplit; ++s) mm = fmaxf(mm, p[s * (dh + 2) + dh]);
-  float ll = 0.f;
-  for (int s = 0; s < nsplit; ++s)
-    if (p[s * (dh + 2) + dh] != -INFINITY)
-      ll += p[s * (dh + 2) + dh + 1] * __expf(p[s * (dh + 2) + dh] - mm);
-  const float inv_l = (ll > 0.f) ? 1.0f / ll : 0.f;
-  const int b = (int)(row / Hq);
-  const int h = (int)(row % Hq);
-  for (int d = threadIdx.x; d < dh; d += blockDim.x) {
-    float o = 0.f;
-    for (int s = 0; s < nsplit; ++s) {
-      const float ms = p[s * (dh + 2) + dh];
-      if (ms != -INFINITY) o += p[s * (dh + 2) + d] * __expf(ms - mm);
+  for (int s = lane; s < nsplit; s += 64)
+    mm = fmaxf(mm, p[s * (DH + 2) + DH]);
+  mm = rb::wave_reduce_max(mm);
+  float ll = 0.f, o[VE];
+#pragma unroll
+  for (int e = 0; e < VE; ++e) o[e] = 0.f;
+  for (int s0 = 0; s0 < nsplit; s0 += 8) {
+    float w[8], x[8][VE];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float *r = p + min(s0 + i, nsplit - 1) * (DH + 2);
+      const float m = r[DH], l = r[DH + 1];
+#pragma unroll
+      for (int e = 0; e < VE; ++e) x[i][e] = r[d0 + e];
+      // partials of no keys have a maximum of minus infinity
+      w[i] = s0 + i < nsplit && m != -INFINITY ? __expf(m - mm) : 0.f;
+      ll += l * w[i];
     }
-    const uint16_t ob = rb::f32_to_bf16(o * inv_l);
-    out[row * dh + d] = ob;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int e = 0; e < VE; ++e)
+        if (w[i] != 0.f) o[e] += x[i][e] * w[i];
+  }
+  const float inv_l = (ll > 0.f) ? 1.0f / ll : 0.f;
+  const int b = row / Hq, h = row % Hq;
+#pragma unroll
+  for (int e = 0; e < VE; ++e) {
+    const uint16_t ob = rb::f32_to_bf16(o[e] * inv_l);
+    out[(int64_t)row * DH + d0 + e] = ob;
     if (out_swz != nullptr) {
-      const int kk = h * dh + d;
+      const int kk = h * DH + d0 + e;
       out_swz[(kk >> 4) * 512 + ((kk >> 3) & 1) * 256 + b * 8 +
               (kk & 7)] = ob;
     }
@@ -435,15 +483,22 @@ __global__ void decode_combine_kernel(const float *__restrict__ partial,
 // dot -> shfl-reduce -> exp -> acc; at G >= 4 that serial chain is the
 // bind (PMC: 57% WAIT_ANY / 28% VALU at 2 waves/SIMD pre-head-split,
 // and the head-split variant re-reads K/V NW times through L2). Here
-// the score block S[16 tok][G] is ONE mfma_f32_16x16x32_bf16 chain over
-// DH, and O^T accumulates via mfma_f32_32x32x16_bf16 — each K/V row is
+// scores and O^T are mfma_f32_16x16x32_bf16 chains — each K/V row is
 // read once, and per-block VALU drops ~60x.
 //
-//  * wave owns whole 16-token cache blocks (bi = blk_lo + wid, step NW).
+//  * a wave takes pairs of 16-token cache blocks, a step each: the chain scores
+//    -> maximum -> exp -> product, which is what a step takes, is shared by 32
+//    tokens. us, 32 query and 8 kv heads of 128, before (a block a step, P
+//    through shuffles, 32-column products of G columns) and now: 64 sequences
+//    of 1000 to 4003 tokens 139 -> 126 (5.2 TB/s), of 2500 each 122 -> 121;
+//    8 of them with 8 splits 29 -> 23, one of 4000 with 16 splits 23 -> 12.
+//    Two waves per SIMD: with one (280 registers) the first takes 137.
+//  * two score tiles S[16][G], whose rows are tokens in an order of our own
+//    choice: tile T's row 4 h + r is token 8 (h % 2) + 4 T + r of block h / 2.
+//    A lane's scores of both tiles are then 8 consecutive tokens of one block,
+//    and, rounded, the operand P[32 tok][G] as they are.
 //  * K is read DIRECTLY in A-fragment order from the [BS, Dh] block
-//    layout: lane l reads K[token l&15][dh (l>>4)*8 + 32*ks] — 16 B per
-//    lane from 16 adjacent 256 B rows inside one contiguous 4 KB block
-//    (64 B segments, L2-friendly), no staging.
+//    layout: 16 B per lane, 64 B segments, no staging.
 //  * V comes from the TRANSPOSED cache layout ([Dh, BS] per block,
 //    alloc_kv_cache v_transposed — the framework owns the layout, so
 //    the PV A-fragment is a direct 16 B/lane read too. The first cut
@@ -452,7 +507,6 @@ __global__ void decode_combine_kernel(const float *__restrict__ partial,
 //    lane stride lands on 2 of 64 banks at any 16-aligned row pitch).
 //  * fragment maps (guide + mfma_probe_16x16x32 GPU test):
 //      16x16x32: A[i=l&15][k=(l>>4)*8+e]; B[k][j=l&15]; C[j=l&15][i=(l>>4)*4+r]
-//      32x32x16: A[i=l&31][k=(l>>5)*8+e]; C[j=l&31][i=(r&3)+8*(r>>2)+4*(l>>5)]
 // ---------------------------------------------------------------------------
 // FP8 mode: K rows stay the scalar-path e4m3 layout ([BS][DH bytes +
 // f32 scale + pad], fp8_row_bytes); V blocks are TRANSPOSED e4m3
@@ -461,7 +515,7 @@ __global__ void decode_combine_kernel(const float *__restrict__ partial,
 // per-token K scale folds into the S rows after the score MFMA and the
 // V scale into P before the PV MFMA (softmax l/m stay on unscaled P).
 template <int DH, int G, bool SPLIT, bool FP8 = false>
-__global__ __launch_bounds__(BLOCK) void paged_decode_mfma_kernel(
+__global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k_cache,
     const uint16_t *__restrict__ v_cache,
     const int32_t *__restrict__ block_tables,
@@ -471,10 +525,10 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_mfma_kernel(
     int max_blocks, int nsplit, float scale) {
   constexpr int BS = 16;                  // cache block = one S tile
   constexpr int KS32 = DH / 32;           // QK^T contraction steps
-  constexpr int DT = DH / 32;             // O^T 32-row d-tiles
+  constexpr int DT = DH / 16;             // O^T 16-row d-tiles
   constexpr int FRW = FP8 ? 2 : 4;        // u32 words per raw fragment
 
-  const int b = blockIdx.x;
+  const int b = sequence_of();
   const int h_kv = blockIdx.y;
   const int split = SPLIT ? blockIdx.z : 0;
   const int hq0 = h_kv * G;
@@ -495,8 +549,6 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_mfma_kernel(
   const int wid = tid >> 6;
   const int i16 = lane & 15;
   const int h16 = lane >> 4;              // 0..3
-  const int h32 = lane >> 5;              // 0..1
-  const int c32 = lane & 31;
 
   const int32_t *bt = block_tables + (int64_t)b * max_blocks;
 
@@ -512,73 +564,81 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_mfma_kernel(
   __shared__ float mlds[NW][G][DH + 2];
   __syncthreads();
 
-  // Q fragments (B of the swapped QK^T), pre-scaled; head = i16.
+  // Q fragments (B of the swapped QK^T); head = i16.
   rb_bf16x8v qf[KS32];
   {
     const bool hv = i16 < G;
     const uint16_t *qp =
-        q + ((int64_t)b * Hq + hq0 + (hv ? i16 : 0)) * DH;
+        q + ((int64_t)b * Hq + hq0 + (hv ? i16 : 0)) * DH + h16 * 8;
 #pragma unroll
-    for (int ks = 0; ks < KS32; ++ks) {
-      float f[8];
-      rb::VIO<uint16_t>::load(qp + ks * 32 + h16 * 8, f);
-      union { unsigned short u[8]; rb_bf16x8v v; } c;
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        c.u[e] = rb::f32_to_bf16(hv ? f[e] * scale : 0.0f);
-      qf[ks] = c.v;
-    }
+    for (int ks = 0; ks < KS32; ++ks)
+      qf[ks] = hv ? *reinterpret_cast<const rb_bf16x8v *>(qp + ks * 32)
+                  : (rb_bf16x8v)(__bf16)0.0f;
   }
 
-  rb_f32x16v acc_o[DT];
+  rb_f32x4v acc_o[DT];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) acc_o[dt] = (rb_f32x16v)(0.0f);
-  float m_run = -INFINITY, l_run = 0.0f;
+  for (int dt = 0; dt < DT; ++dt) acc_o[dt] = (rb_f32x4v)(0.0f);
+  float m_run = -INFINITY, l_run = 0.0f;  // l_run: of this lane's tokens
 
   const int blk_lo = t_begin / BS;
   const int blk_hi = (t_end > t_begin) ? (t_end - 1) / BS : blk_lo - 1;
+  // this lane's tokens within a pair of blocks, as scores and as V columns
+  const int half = h16 >> 1, tok0 = (h16 & 1) * 8;
+  // the K row that this lane loads for tile 0 (tile 1: four rows on)
+  const int khalf = i16 >> 3, krow = (i16 >> 2 & 1) * 8 + (i16 & 3);
 
-  // 2-deep block ring: iteration i+1's K/V raw fragments are issued
-  // while i computes (PMC post-VT-layout: 74% WAIT_ANY at occupancy 2 —
-  // two waves/SIMD cannot hide HBM latency without in-flight depth).
-  // +(KS32+DT)*FRW words per slot keeps occupancy at 2.
-  uint32_t kfr[2][KS32][FRW], vfr[2][DT][FRW];
-  float ksc[2][4], vsc[2][4];            // fp8 per-token scales
+  // two pairs' raw fragments: the next one's are issued while one is computed
+  uint32_t kfr[2][2][KS32][FRW], vfr[2][DT][FRW];
+  float ksc[2][8], vsc[2][8];            // fp8 per-token scales
 
-  auto fetch = [&](int bi, int slot) {
+  auto block_of = [&](int bi) {          // the last one again past the end
+    bi = min(bi, blk_hi);
     const int bi_l = bi - blk0;
-    const int blk = (bi_l < BT_LDS) ? bt_lds[bi_l] : bt[bi];
+    return (bi_l < BT_LDS) ? bt_lds[bi_l] : bt[bi];
+  };
+  auto fetch = [&](int bi, int slot) {
+    const int blk_a = block_of(bi), blk_b = block_of(bi + 1);
+    const int64_t kblk = (int64_t)(khalf ? blk_b : blk_a) * hkv + h_kv;
+    const int64_t vblk = (int64_t)(half ? blk_b : blk_a) * hkv + h_kv;
     if (FP8) {
       constexpr int RB8 = DH + 16;       // fp8 K row bytes
-      const uint8_t *kb = reinterpret_cast<const uint8_t *>(k_cache) +
-          ((int64_t)blk * hkv + h_kv) * BS * RB8;
-      const uint8_t *vb = reinterpret_cast<const uint8_t *>(v_cache) +
-          ((int64_t)blk * hkv + h_kv) * (DH + 4) * BS;
+      const uint8_t *k8 = reinterpret_cast<const uint8_t *>(k_cache);
+      const uint8_t *kb = k8 + kblk * BS * RB8;
+      const uint8_t *vb =
+          reinterpret_cast<const uint8_t *>(v_cache) + vblk * (DH + 4) * BS;
 #pragma unroll
-      for (int ks = 0; ks < KS32; ++ks)
-        rb::ld_words<2>(kfr[slot][ks], kb + i16 * RB8 + ks * 32 + h16 * 8);
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int ks = 0; ks < KS32; ++ks)
+          rb::ld_words<2>(kfr[slot][t][ks],
+                          kb + (krow + 4 * t) * RB8 + ks * 32 + h16 * 8);
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
-        rb::ld_words<2>(vfr[slot][dt], vb + (dt * 32 + c32) * BS + h32 * 8);
+        rb::ld_words<2>(vfr[slot][dt], vb + (dt * 16 + i16) * BS + tok0);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int tok = h16 * 4 + r;
-        ksc[slot][r] = *reinterpret_cast<const float *>(kb + tok * RB8 + DH);
-        vsc[slot][r] = *reinterpret_cast<const float *>(
-            vb + DH * BS + tok * 4);
+      for (int e = 0; e < 8; ++e) {
+        ksc[slot][e] = *reinterpret_cast<const float *>(
+            k8 + (vblk * BS + tok0 + e) * RB8 + DH);
+        vsc[slot][e] = *reinterpret_cast<const float *>(
+            vb + DH * BS + (tok0 + e) * 4);
       }
     } else {
-      const uint16_t *kb = k_cache + ((int64_t)blk * hkv + h_kv) * BS * DH;
+      const uint8_t *kb = reinterpret_cast<const uint8_t *>(
+          k_cache + kblk * BS * DH);
       // v block is [DH][BS] (transposed layout)
-      const uint16_t *vb = v_cache + ((int64_t)blk * hkv + h_kv) * DH * BS;
+      const uint8_t *vb = reinterpret_cast<const uint8_t *>(
+          v_cache + vblk * DH * BS);
 #pragma unroll
-      for (int ks = 0; ks < KS32; ++ks)
-        rb::ld_words<4>(kfr[slot][ks], reinterpret_cast<const uint8_t *>(
-            kb + i16 * DH + ks * 32 + h16 * 8));
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int ks = 0; ks < KS32; ++ks)
+          rb::ld_words<4>(kfr[slot][t][ks],
+                          kb + ((krow + 4 * t) * DH + ks * 32 + h16 * 8) * 2);
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
-        rb::ld_words<4>(vfr[slot][dt], reinterpret_cast<const uint8_t *>(
-            vb + (dt * 32 + c32) * BS + h32 * 8));
+        rb::ld_words<4>(vfr[slot][dt],
+                        vb + ((dt * 16 + i16) * BS + tok0) * 2);
     }
   };
 
@@ -599,98 +659,85 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_mfma_kernel(
     return c.v;
   };
 
+  constexpr int PAIR = 2 * NW;            // blocks of a step
   auto step = [&](int bi, int cur) {
-    if (bi + NW <= blk_hi) fetch(bi + NW, cur ^ 1);
+    if (bi + PAIR <= blk_hi) fetch(bi + PAIR, cur ^ 1);
 
-    // ---- S[16 tok][16 heads] = K_blk @ Q^T ----------------------------
-    rb_f32x4v s4 = (rb_f32x4v)(0.0f);
+    // ---- scores of two tiles: element 4 T + r is token tok0 + 4 T + r ----
+    float p[8];
 #pragma unroll
-    for (int ks = 0; ks < KS32; ++ks) {
-      s4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(kfr[cur][ks]),
-                                                   qf[ks], s4, 0, 0, 0);
+    for (int t = 0; t < 2; ++t) {
+      rb_f32x4v s4 = (rb_f32x4v)(0.0f);
+#pragma unroll
+      for (int ks = 0; ks < KS32; ++ks)
+        s4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(kfr[cur][t][ks]),
+                                                     qf[ks], s4, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) p[t * 4 + r] = s4[r] * scale;
     }
     if (FP8) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) s4[r] *= ksc[cur][r];
+      for (int e = 0; e < 8; ++e) p[e] *= ksc[cur][e];
     }
 
     // ---- mask + online softmax (state per head = per col = per lane) --
-    float p4[4];
+    const int t0 = (bi + half) * BS + tok0;
     float mx = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int t = bi * BS + h16 * 4 + r;
-      p4[r] = (t >= t_begin && t < t_end) ? s4[r] : -INFINITY;
-      mx = fmaxf(mx, p4[r]);
+    for (int e = 0; e < 8; ++e) {
+      if (t0 + e < t_begin || t0 + e >= t_end) p[e] = -INFINITY;
+      mx = fmaxf(mx, p[e]);
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mn = fmaxf(m_run, mx);
-    if (mn != -INFINITY) {
-      const float alpha = (m_run == -INFINITY) ? 0.0f : __expf(m_run - mn);
-      float psum = 0.0f;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        p4[r] = (p4[r] == -INFINITY) ? 0.0f : __expf(p4[r] - mn);
-        psum += p4[r];
-      }
-      psum += __shfl_xor(psum, 16, 64);
-      psum += __shfl_xor(psum, 32, 64);
-      l_run = l_run * alpha + psum;
+    if (__any(mx > m_run)) {
+      const float mn = fmaxf(m_run, mx);
+      const float alpha = mn == -INFINITY ? 1.0f : __expf(m_run - mn);
+      l_run *= alpha;
       m_run = mn;
-      if (alpha != 1.0f) {
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc_o[dt][r] *= alpha;
-      }
-
-      // ---- P[tok][head] -> B fragment of PV (k = tok, col = head) ----
-      // source lane s = head + 16*(tok>>2) holds tokens 4*(s>>4)+r.
-      // target lane l needs tokens (l>>5)*8..+8 of head l&31 (<16).
-      // fp8: the per-token V scale rides on P here (l/m and psum above
-      // stay on the unscaled softmax numerators).
-      float pv0 = p4[0], pv1 = p4[1], pv2 = p4[2], pv3 = p4[3];
-      if (FP8) {
-        pv0 *= vsc[cur][0]; pv1 *= vsc[cur][1];
-        pv2 *= vsc[cur][2]; pv3 *= vsc[cur][3];
-      }
-      const unsigned w01 = rb_pack_bf16(pv0, pv1);
-      const unsigned w23 = rb_pack_bf16(pv2, pv3);
-      const int sh = c32 & 15;            // source head (cols 16+ unused)
-      const int s1 = sh + 16 * (h32 * 2);
-      const int s2 = s1 + 16;
-      union { unsigned u[4]; rb_bf16x8v v; } pf;
-      pf.u[0] = __shfl(w01, s1, 64);
-      pf.u[1] = __shfl(w23, s1, 64);
-      pf.u[2] = __shfl(w01, s2, 64);
-      pf.u[3] = __shfl(w23, s2, 64);
-
-      // ---- O^T[d][head] += V^T_blk @ P --------------------------------
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            frag(vfr[cur][dt]), pf.v, acc_o[dt], 0, 0, 0);
-      }
+        for (int r = 0; r < 4; ++r) acc_o[dt][r] *= alpha;
     }
+    // heads that have seen no finite score keep a finite reference
+    const float ref = m_run == -INFINITY ? 0.0f : m_run;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      p[e] = __expf(p[e] - ref);
+      l_run += p[e];
+      // fp8: the per-token V scale rides on P here (l stays on the unscaled
+      // softmax numerators)
+      if (FP8) p[e] *= vsc[cur][e];
+    }
+    union { unsigned u[4]; rb_bf16x8v v; } pf;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) pf.u[e] = rb_pack_bf16(p[2 * e], p[2 * e + 1]);
+
+    // ---- O^T[d][head] += V^T @ P ----------------------------------------
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+      acc_o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          frag(vfr[cur][dt]), pf.v, acc_o[dt], 0, 0, 0);
   };
 
-  const int bi0 = blk_lo + wid;
+  const int bi0 = blk_lo + 2 * wid;
   if (bi0 <= blk_hi) fetch(bi0, 0);
-  for (int bi = bi0; bi <= blk_hi; bi += 2 * NW) {
+  for (int bi = bi0; bi <= blk_hi; bi += 2 * PAIR) {
     step(bi, 0);
-    if (bi + NW <= blk_hi) step(bi + NW, 1);
+    if (bi + PAIR <= blk_hi) step(bi + PAIR, 1);
   }
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
 
   // ---- cross-wave merge via LDS (same scheme as the scalar kernel) ----
-  // acc_o lane map: head = c32, d = dt*32 + (r&3)+8*(r>>2)+4*h32.
-  if (c32 < G) {
+  // acc_o lane map: head = i16, d = dt*16 + 4*h16 + r.
+  if (i16 < G) {
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        mlds[wid][c32][dt * 32 + (r & 3) + 8 * (r >> 2) + 4 * h32] =
-            acc_o[dt][r];
+      for (int r = 0; r < 4; ++r)
+        mlds[wid][i16][dt * 16 + 4 * h16 + r] = acc_o[dt][r];
   }
   if (lane < 16 && i16 < G) {
     mlds[wid][i16][DH] = m_run;
@@ -793,9 +840,11 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                            seq_lens.data_ptr<int32_t>(), starts,
                            nullptr, nullptr, partial.data_ptr<float>(), hkv,
                            max_blocks, nsplit, scale);
-        hipLaunchKernelGGL(decode_combine_kernel, dim3(B * Hq), dim3(256), 0,
-                           stream, partial.data_ptr<float>(),
-                           (uint16_t *)out.data_ptr(), swz, Hq, nsplit, DH);
+        hipLaunchKernelGGL((decode_combine_kernel<DH / 64>),
+                           dim3((B * Hq + 3) / 4), dim3(256), 0, stream,
+                           partial.data_ptr<float>(),
+                           (uint16_t *)out.data_ptr(), swz, B * Hq, Hq,
+                           nsplit);
       }
       return;
     }
@@ -825,9 +874,11 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                        starts,
                        nullptr, nullptr, partial.data_ptr<float>(), hkv, bs,
                        max_blocks, nsplit, scale);
-    hipLaunchKernelGGL(decode_combine_kernel, dim3(B * Hq), dim3(256), 0, stream,
-                       partial.data_ptr<float>(), (uint16_t *)out.data_ptr(),
-                       swz, Hq, nsplit, DH);
+    hipLaunchKernelGGL((decode_combine_kernel<DH / 64>),
+                           dim3((B * Hq + 3) / 4), dim3(256), 0, stream,
+                           partial.data_ptr<float>(),
+                           (uint16_t *)out.data_ptr(), swz, B * Hq, Hq,
+                           nsplit);
   }
 }
 

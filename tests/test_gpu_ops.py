@@ -617,6 +617,41 @@ def test_geglu_packed():
     assert torch.allclose(got.float(), ref, atol=3e-2, rtol=3e-2)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hq,hkv,dh,vt", [
+    (4, 4, 128, False), (4, 2, 64, False), (2, 2, 256, False),
+    (8, 2, 128, True), (16, 1, 64, True), (8, 1, 128, True),
+    (8, 2, 128, False)])
+def test_paged_decode_steps(hq, hkv, dh, vt, fp8):
+    """Lengths around the tokens of a step (8 and 32 of a wave, four waves),
+    splits that leave parts empty, starts inside a block."""
+    _assert_hip()
+    from runbooks_amd.ops.kvcache import alloc_kv_cache
+    g = torch.Generator().manual_seed(dh + hq)
+    lens = [1, 7, 8, 9, 31, 32, 33, 63, 64, 65, 127, 129, 200]
+    B, wide = len(lens), 14
+    n = B * wide
+    kc, vc = alloc_kv_cache(n, hkv, dh, "cpu", fp8=fp8, v_transposed=vt)
+    k, v = (torch.randn(n * 16, hkv, dh, generator=g).bfloat16()
+            for _ in range(2))
+    ops.kv_append_ref(k, v, kc, vc, torch.arange(n * 16))
+    bt = torch.randperm(n, generator=g).view(B, wide).int()
+    sl = torch.tensor(lens, dtype=torch.int32)
+    starts = torch.tensor([x // 3 for x in lens], dtype=torch.int32)
+    q = torch.randn(B, hq, dh, generator=g).bfloat16()
+    for st in (None, starts):
+        ref = ops.paged_decode_ref(q.float(), kc if fp8 else kc.float(),
+                                   vc if fp8 else vc.float(), bt, sl,
+                                   dh ** -0.5, seq_starts=st)
+        for nsplit in (1, 2, 16):
+            got = ops.paged_decode(
+                q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), sl.to(DEV),
+                nsplit=nsplit,
+                seq_starts=None if st is None else st.to(DEV))
+            # weights (MFMA path) and result rounded to bf16, values up to 5
+            assert (got.cpu().float() - ref).abs().max() < 3e-2
+
+
 @pytest.mark.gpu
 @pytest.mark.skipif(not _EXPERIMENTAL, reason="RB_EXPERIMENTAL=1 only "
                     "(Dh=256 decode instantiation awaits GPU validation)")

@@ -120,7 +120,24 @@ class Attention(nn.Module):
         o = ops.causal_attention(q, k, v, scale=self.scale)
         return self.o_proj(o.reshape(B * S, self.hq * self.dh))
 
+    def _fused_append(self, x, kc) -> bool:
+        """One product for q, k and v, and one kernel for their rotation and
+        the cache (csrc/qkv_fused.hip)."""
+        return (getattr(self, "_qkv_w", None) is not None and
+                not torch.is_grad_enabled() and
+                self.cfg.pos == "rope" and ops.use_hip(x) and
+                self.dh in (64, 128, 256) and x.dtype == torch.bfloat16 and
+                kc.dtype in (torch.bfloat16, torch.uint8))
+
     def forward_prefill(self, x, cos, sin, positions, kc, vc, slot_mapping, B, S):
+        if self._fused_append(x, kc):
+            y = ops.fast_linear(x, self._qkv_w)
+            ops.ext().qkv_rope_append_(y, cos, sin, positions.to(torch.int32),
+                                       kc, vc, slot_mapping.to(torch.int32),
+                                       self.hq)
+            o = ops.ext().flash_prefill_qkv(y, B, S, self.hq, self.hkv,
+                                            self.dh, self.scale)
+            return self.o_proj(o.view(B * S, self.hq * self.dh))
         q, k, v = self._qkv(x, cos, sin, positions)
         ops.kv_append(k, v, kc, vc, slot_mapping)
         q = q.view(B, S, self.hq, self.dh)
@@ -132,14 +149,9 @@ class Attention(nn.Module):
                        block_tables, seq_lens, nsplit=None, slab_ok=False,
                        seq_starts=None):
         B = x.shape[0]
-        if getattr(self, "_qkv_w", None) is not None and \
-                self.cfg.pos == "rope" and ops.use_hip(x) and \
-                x.dtype == torch.bfloat16 and kc.dtype == torch.bfloat16:
+        if self._fused_append(x, kc):
             # fused decode hot path: one wide GEMM, then one kernel doing
-            # rope(q), rope(k)->cache, v->cache (csrc/qkv_fused.hip).
-            # fp8 caches take the generic path below (rope + fp8-quant
-            # kv_append): that mode targets long-context KV-bound decode
-            # where the attention read, not the epilogue, dominates.
+            # rope(q), rope(k)->cache, v->cache, quantized where the cache is
             y = ops.fast_linear(x, self._qkv_w)
             q = ops.ext().qkv_rope_append(y, cos, sin, positions, kc, vc,
                                           slot_mapping, self.hq)
@@ -251,6 +263,23 @@ class Block(nn.Module):
             return x + attn_fn(self.norm1(x)) + self.mlp(self.norm2(x))
         x = x + attn_fn(self.norm1(x))
         return x + self.mlp(self.norm2(x))
+
+    def fuses_residual(self) -> bool:
+        """The sums of the residual may go into the norms that follow them."""
+        return (isinstance(self.norm1, ops.RMSNorm) and
+                not self.cfg.parallel_residual and not self.cfg.single_norm)
+
+    def forward_pending(self, x, delta, attn_fn):
+        """forward() of a residual whose last term is still to be added:
+        x + delta -> (x, delta)."""
+        if delta is None:
+            h = self.norm1(x)
+        else:
+            x, h = ops.rmsnorm_res(x, delta, self.norm1.weight,
+                                   self.norm1.eps)
+        x, h = ops.rmsnorm_res(x, attn_fn(h), self.norm2.weight,
+                               self.norm2.eps)
+        return x, self.mlp(h)
 
     def forward_decode_fused(self, x_base, delta, attn_fn):
         """Decode hot path (sequential-residual RMSNorm models): the
@@ -392,23 +421,43 @@ class Transformer(nn.Module):
         x = self._embed(tokens, positions)
         ckpt = getattr(self, "grad_checkpointing", False) and \
             torch.is_grad_enabled()
-        for blk in self.blocks:
-            fn = lambda h, b=blk: b.attn.forward_train(  # noqa: E731
-                h, self.rope_cos, self.rope_sin, positions, B, S)
+
+        def run(blk, *args):
             if ckpt:
                 # recompute this block's activations in backward: peak
                 # activation memory drops from O(layers) to O(1) blocks
                 # (full fine-tunes of 70B-class models at long seq; LoRA
                 # at default shapes fits 288 GB without it)
-                x = torch.utils.checkpoint.checkpoint(
-                    blk, x, fn, use_reentrant=False)
-            else:
-                x = blk(x, fn)
-        x = self.norm_f(x)
+                return torch.utils.checkpoint.checkpoint(
+                    blk, *args, use_reentrant=False)
+            return blk(*args)
+
+        def attention(blk):
+            return lambda h: blk.attn.forward_train(
+                h, self.rope_cos, self.rope_sin, positions, B, S)
+
+        x = self._last_norm(*self._blocks(x, attention, run))
         logits = self.lm_head(x)
         if self._lm_vocab_parallel:
             logits = gather_from_tp(logits)
         return logits.view(B, S, -1)
+
+    def _blocks(self, x, attention, run=lambda blk, *args: blk(*args)):
+        """All blocks; attention(block) is its attn_fn. Returns the residual
+        and what is still to be added to it (None: nothing)."""
+        delta = None
+        for blk in self.blocks:
+            if blk.fuses_residual():
+                x, delta = run(blk.forward_pending, x, delta, attention(blk))
+            else:
+                x = run(blk, x, attention(blk))
+        return x, delta
+
+    def _last_norm(self, x, delta):
+        if delta is None:
+            return self.norm_f(x)
+        return ops.rmsnorm_res(x, delta, self.norm_f.weight,
+                               self.norm_f.eps)[1]
 
     def enable_grad_checkpointing(self, enabled: bool = True) -> None:
         self.grad_checkpointing = enabled
@@ -422,11 +471,16 @@ class Transformer(nn.Module):
             raise NotImplementedError("prefill through forward_ragged")
         B, S = tokens.shape
         x = self._embed(tokens, positions)
-        for blk, (kc, vc) in zip(self.blocks, caches):
-            fn = lambda h, b=blk, kc=kc, vc=vc: b.attn.forward_prefill(  # noqa: E731
-                h, self.rope_cos, self.rope_sin, positions, kc, vc, slot_mapping, B, S)
-            x = blk(x, fn)
-        x = self.norm_f(x.view(B, S, -1)[:, -1])
+        cache_of = dict(zip(self.blocks, caches))
+
+        def attention(blk):
+            kc, vc = cache_of[blk]
+            return lambda h: blk.attn.forward_prefill(
+                h, self.rope_cos, self.rope_sin, positions, kc, vc,
+                slot_mapping, B, S)
+
+        x = self._last_norm(*(None if r is None else r.view(B, S, -1)[:, -1]
+                              for r in self._blocks(x, attention)))
         logits = self.lm_head(x)
         return gather_from_tp(logits) if self._lm_vocab_parallel else logits
 
@@ -473,12 +527,16 @@ class Transformer(nn.Module):
             logits = self.lm_head(y)
             return (gather_from_tp(logits) if self._lm_vocab_parallel
                     else logits)
-        for blk, (kc, vc) in zip(self.blocks, caches):
-            fn = lambda h, b=blk, kc=kc, vc=vc: b.attn.forward_decode(  # noqa: E731
-                h, self.rope_cos, self.rope_sin, positions, kc, vc, slot_mapping,
-                block_tables, seq_lens, nsplit=nsplit, seq_starts=seq_starts)
-            x = blk(x, fn)
-        x = self.norm_f(x)
+        cache_of = dict(zip(self.blocks, caches))
+
+        def attention(blk):
+            kc, vc = cache_of[blk]
+            return lambda h: blk.attn.forward_decode(
+                h, self.rope_cos, self.rope_sin, positions, kc, vc,
+                slot_mapping, block_tables, seq_lens, nsplit=nsplit,
+                seq_starts=seq_starts)
+
+        x = self._last_norm(*self._blocks(x, attention))
         logits = self.lm_head(x)
         return gather_from_tp(logits) if self._lm_vocab_parallel else logits
 

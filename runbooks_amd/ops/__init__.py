@@ -16,7 +16,7 @@ from .linear import (Linear, decode_linear_raw, decode_operand,  # noqa: F401
                      decode_ready, fast_linear, linear_f32,
                      linear_f32_parts)
 from .norm import (RMSNorm, join_res32, layernorm_res32, norm_res32,  # noqa: F401
-                   rmsnorm, rmsnorm_ref, rmsnorm_res32)
+                   rmsnorm, rmsnorm_ref, rmsnorm_res, rmsnorm_res32)
 from .rope import rope, rope_frequencies, rope_ref, rope_tables  # noqa: F401
 from .sampling import sample_tokens  # noqa: F401
 from .shared_kv import alloc_shared_kv_cache  # noqa: F401

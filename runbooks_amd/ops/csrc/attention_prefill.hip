@@ -26,7 +26,8 @@
 //   A[i][k]: i = lane&31, k = (lane>>5)*8 + e (e = 0..7)
 //   C[i][j]: j = lane&31, i = (reg&3) + 8*(reg>>2) + 4*(lane>>5)
 //
-// q,k,v,out: [B, S, H, DH] bf16 token-major. DH in {64, 128, 256}.
+// q,k,v,out: [B, S, H, DH] bf16 token-major (tokens of q, and of k and v, at a
+// stride of their own). DH in {64, 128, 256}.
 
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -50,7 +51,8 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
     const uint16_t *__restrict__ qp, const uint16_t *__restrict__ kp,
     const uint16_t *__restrict__ vp, uint16_t *__restrict__ op,
     float *__restrict__ lsep,  // [B, Hq, S] log-sum-exp for training bwd
-    int B, int S, int Hq, int Hkv, float scale) {
+    int B, int S, int Hq, int Hkv, int64_t q_stride, int64_t kv_stride,
+    float scale) {
   constexpr int KSTEPS = DH / 16;       // QK^T contraction steps
   constexpr int DTILES = DH / 32;       // O column tiles
   constexpr int QT = NW / SPLIT * 32;
@@ -72,9 +74,8 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
   const int qrow = wrow + col;              // this lane's query row
   const bool q_valid = qrow < S;
 
-  const int64_t kv_stride = (int64_t)Hkv * DH;
-  const uint16_t *kb = kp + ((int64_t)b * S * Hkv + h_kv) * DH;
-  const uint16_t *vb = vp + ((int64_t)b * S * Hkv + h_kv) * DH;
+  const uint16_t *kb = kp + (int64_t)b * S * kv_stride + h_kv * DH;
+  const uint16_t *vb = vp + (int64_t)b * S * kv_stride + h_kv * DH;
   const TileLoad<DH, NW> load(wid, lane);
   const int kv_end = min(S, q0 + QT);       // causal upper bound for this WG
   const int n_tiles = (kv_end + ROWS - 1) / ROWS;
@@ -86,8 +87,9 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
   // of zero clears them, so that hidden scores stay at minus infinity --------
   bf16x8v qf[KSTEPS];
   {
-    const uint16_t *src = qp + ((int64_t)(b * S + (q_valid ? qrow : 0)) * Hq +
-                                h) * DH + hi * 8;
+    const uint16_t *src =
+        qp + ((int64_t)b * S + (q_valid ? qrow : 0)) * q_stride + h * DH +
+        hi * 8;
     const unsigned flip = scale < 0.0f ? 0x80008000u : 0u;
     const unsigned keep = scale == 0.0f ? 0u : ~0u;
 #pragma unroll
@@ -265,11 +267,15 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
   }
 }
 
-template <int DH, int NW, int SPLIT>
-void launch_prefill(const at::Tensor &q, const at::Tensor &k,
-                    const at::Tensor &v, at::Tensor &out, float *lsep,
-                    float scale) {
-  const int B = (int)q.size(0), S = (int)q.size(1), Hq = (int)q.size(2);
+struct Problem {
+  const uint16_t *q, *k, *v;
+  uint16_t *out;
+  float *lse;
+  int64_t B, S, Hq, Hkv, q_stride, kv_stride;
+  float scale;
+};
+
+template <int DH, int NW, int SPLIT> void launch_prefill(const Problem &p) {
   constexpr size_t merge =
       SPLIT == 1 ? 0 : (size_t)NW / SPLIT * (DH / 8 + 1) * 1024;
   constexpr size_t shmem = std::max((size_t)4 * tile_bytes<DH>(), merge);
@@ -278,20 +284,16 @@ void launch_prefill(const at::Tensor &q, const at::Tensor &k,
       hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) == hipSuccess;
   TORCH_CHECK(once, "flash_prefill: LDS size");
   constexpr int QT = NW / SPLIT * 32;
-  const int64_t grid = (int64_t)((S + QT - 1) / QT) * Hq * B;
+  const int64_t grid = (p.S + QT - 1) / QT * p.Hq * p.B;
   TORCH_CHECK(grid < (int64_t)1 << 31, "flash_prefill: grid");
-  hipLaunchKernelGGL((flash_prefill_kernel<DH, NW, SPLIT>), dim3((unsigned)grid),
-                     dim3(NW * 64), shmem, at::hip::getCurrentHIPStream(),
-                     (const uint16_t *)q.data_ptr(),
-                     (const uint16_t *)k.data_ptr(),
-                     (const uint16_t *)v.data_ptr(), (uint16_t *)out.data_ptr(),
-                     lsep, B, S, Hq, (int)k.size(2), scale);
+  hipLaunchKernelGGL((flash_prefill_kernel<DH, NW, SPLIT>),
+                     dim3((unsigned)grid), dim3(NW * 64), shmem,
+                     at::hip::getCurrentHIPStream(), p.q, p.k, p.v, p.out,
+                     p.lse, (int)p.B, (int)p.S, (int)p.Hq, (int)p.Hkv,
+                     p.q_stride, p.kv_stride, p.scale);
 }
 
-template <int DH>
-void launch_prefill(const at::Tensor &q, const at::Tensor &k,
-                    const at::Tensor &v, at::Tensor &out, float *lsep,
-                    float scale) {
+template <int DH> void launch_prefill(const Problem &p) {
   // Tiles of 32 query rows in all heads: one or two waves each, on 1024 SIMDs.
   // As long as there are fewer of them than SIMDs, the chain of a tile's keys
   // is what takes the time, and two waves halve it; small workgroups then use
@@ -304,16 +306,23 @@ void launch_prefill(const at::Tensor &q, const at::Tensor &k,
   // 256 columns take a SIMD's registers for one wave, so four waves fill a CU
   // (3000 tokens, 16 heads, 1504 tiles: <4,2> 151, <4,1> 141; with eight, which
   // spill, 281).
-  const int64_t tiles = (q.size(1) + 31) / 32 * q.size(2) * q.size(0);
+  const int64_t tiles = (p.S + 31) / 32 * p.Hq * p.B;
   if constexpr (DH == 256) {
-    if (tiles <= 1280) launch_prefill<DH, 4, 2>(q, k, v, out, lsep, scale);
-    else launch_prefill<DH, 4, 1>(q, k, v, out, lsep, scale);
+    if (tiles <= 1280) launch_prefill<DH, 4, 2>(p);
+    else launch_prefill<DH, 4, 1>(p);
   } else {
-    if (tiles <= 512) launch_prefill<DH, 2, 2>(q, k, v, out, lsep, scale);
-    else if (tiles <= 1536) launch_prefill<DH, 4, 2>(q, k, v, out, lsep, scale);
-    else if (tiles < 6144) launch_prefill<DH, 4, 1>(q, k, v, out, lsep, scale);
-    else launch_prefill<DH, 8, 1>(q, k, v, out, lsep, scale);
+    if (tiles <= 512) launch_prefill<DH, 2, 2>(p);
+    else if (tiles <= 1536) launch_prefill<DH, 4, 2>(p);
+    else if (tiles < 6144) launch_prefill<DH, 4, 1>(p);
+    else launch_prefill<DH, 8, 1>(p);
   }
+}
+
+void launch_prefill(int64_t DH, const Problem &p) {
+  if (DH == 128) launch_prefill<128>(p);
+  else if (DH == 64) launch_prefill<64>(p);
+  else if (DH == 256) launch_prefill<256>(p);
+  else TORCH_CHECK(false, "flash_prefill: DH must be 64, 128 or 256, got ", DH);
 }
 
 }  // namespace
@@ -337,10 +346,29 @@ static at::Tensor flash_fwd_impl(at::Tensor q, at::Tensor k, at::Tensor v,
   q = flash::aligned16(q);
   k = flash::aligned16(k);
   v = flash::aligned16(v);
-  if (DH == 128) launch_prefill<128>(q, k, v, out, lsep, (float)scale);
-  else if (DH == 64) launch_prefill<64>(q, k, v, out, lsep, (float)scale);
-  else if (DH == 256) launch_prefill<256>(q, k, v, out, lsep, (float)scale);
-  else TORCH_CHECK(false, "flash_prefill: DH must be 64, 128 or 256, got ", DH);
+  launch_prefill(DH, {(const uint16_t *)q.data_ptr(),
+                      (const uint16_t *)k.data_ptr(),
+                      (const uint16_t *)v.data_ptr(),
+                      (uint16_t *)out.data_ptr(), lsep, B, S, Hq, Hkv,
+                      (int64_t)Hq * DH, (int64_t)Hkv * DH, (float)scale});
+  return out;
+}
+
+// q, k and v side by side in the rows of y [B * S, (Hq + 2 Hkv) * DH].
+at::Tensor flash_prefill_qkv(at::Tensor y, int64_t B, int64_t S, int64_t Hq,
+                             int64_t Hkv, int64_t DH, double scale) {
+  const int64_t width = (Hq + 2 * Hkv) * DH;
+  TORCH_CHECK(y.is_cuda() && y.is_contiguous() && y.dim() == 2 &&
+              y.scalar_type() == at::kBFloat16 && y.size(0) == B * S &&
+              y.size(1) == width && Hkv > 0 && Hq % Hkv == 0 &&
+              reinterpret_cast<uintptr_t>(y.data_ptr()) % 16 == 0,
+              "flash_prefill_qkv: y");
+  auto out = at::empty({B, S, Hq, DH}, y.options());
+  if (out.numel() == 0) return out;
+  const uint16_t *p = (const uint16_t *)y.data_ptr();
+  launch_prefill(DH, {p, p + Hq * DH, p + (Hq + Hkv) * DH,
+                      (uint16_t *)out.data_ptr(), nullptr, B, S, Hq, Hkv,
+                      width, width, (float)scale});
   return out;
 }
 

@@ -27,6 +27,12 @@ std::vector<at::Tensor> paged_decode_swz(at::Tensor q, at::Tensor k_cache,
                                          at::Tensor seq_lens, int64_t nsplit,
                                          double scale,
                                          c10::optional<at::Tensor> seq_starts);
+at::Tensor flash_prefill_qkv(at::Tensor y, int64_t B, int64_t S, int64_t Hq,
+                             int64_t Hkv, int64_t DH, double scale);
+void qkv_rope_append_(at::Tensor y, at::Tensor cos, at::Tensor sin,
+                      at::Tensor positions, at::Tensor k_cache,
+                      at::Tensor v_cache, at::Tensor slot_mapping,
+                      int64_t hq);
 at::Tensor flash_prefill(at::Tensor q, at::Tensor k, at::Tensor v, double scale);
 std::vector<at::Tensor> flash_fwd_train(at::Tensor q, at::Tensor k, at::Tensor v,
                                         double scale);
@@ -74,6 +80,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("block_tables"), py::arg("seq_lens"), py::arg("nsplit"),
         py::arg("scale"), py::arg("seq_starts") = py::none());
   m.def("flash_prefill", &flash_prefill, "MFMA flash-attention prefill (causal)");
+  m.def("flash_prefill_qkv", &flash_prefill_qkv,
+        "flash_prefill of q, k and v side by side in one tensor");
+  m.def("qkv_rope_append_", &qkv_rope_append_,
+        "packed qkv: q and k rotated in place, k and v appended to the cache");
   m.def("flash_fwd_train", &flash_fwd_train,
         "MFMA flash-attention forward + log-sum-exp (training)");
   m.def("fa_bwd", &fa_bwd,

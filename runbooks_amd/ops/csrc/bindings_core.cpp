@@ -9,7 +9,10 @@ std::vector<at::Tensor> rmsnorm_res_fwd_dec(at::Tensor x, at::Tensor res, at::Te
 std::vector<at::Tensor> rmsnorm_res_slab_fwd_dec(at::Tensor x, at::Tensor slabs, at::Tensor w, double eps);
 std::vector<at::Tensor> rmsnorm_res32(at::Tensor x, c10::optional<at::Tensor> delta, at::Tensor w, double eps, bool want_swz, double offset);
 std::vector<at::Tensor> rmsnorm_bwd(at::Tensor x, at::Tensor w, at::Tensor dy,
-                                    at::Tensor inv_rms);
+                                    at::Tensor inv_rms, bool need_dw,
+                                    c10::optional<at::Tensor> add);
+std::vector<at::Tensor> rmsnorm_res_fwd(at::Tensor x, at::Tensor res,
+                                        at::Tensor w, double eps);
 std::vector<at::Tensor> layernorm_res32(at::Tensor x, c10::optional<at::Tensor> delta, at::Tensor w, at::Tensor b, double eps, bool want_swz);
 std::vector<at::Tensor> join_res32(at::Tensor x, c10::optional<at::Tensor> delta, at::Tensor other, bool want_swz);
 at::Tensor swiglu_packed(at::Tensor y);
@@ -37,7 +40,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "split-K slab combine + residual + RMSNorm + swizzle in one pass");
   m.def("rmsnorm_res32", &rmsnorm_res32,
         "fp32 residual += delta (or split-K slab), then RMSNorm");
-  m.def("rmsnorm_bwd", &rmsnorm_bwd, "fused RMSNorm backward");
+  m.def("rmsnorm_bwd", &rmsnorm_bwd, "fused RMSNorm backward", py::arg("x"),
+        py::arg("w"), py::arg("dy"), py::arg("inv_rms"),
+        py::arg("need_dw") = true, py::arg("add") = py::none());
+  m.def("rmsnorm_res_fwd", &rmsnorm_res_fwd,
+        "residual sum + RMSNorm forward -> {sum, y, inv_rms}");
   m.def("layernorm_res32", &layernorm_res32,
         "fp32 residual += delta (or split-K slab), then LayerNorm");
   m.def("join_res32", &join_res32,

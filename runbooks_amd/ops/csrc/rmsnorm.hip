@@ -12,6 +12,9 @@
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -29,6 +32,7 @@ constexpr int BLOCK = 256;
 // res32/rsplit (optional, bf16 path): the residual arrives as the
 // UNCOMBINED fp32 split-K slab [rsplit, n_rows, D] straight from
 // decode_gemm_raw — folding the slices here saves the combine launch.
+// One workgroup per row, any width (rows beyond the next kernel's).
 template <typename T>
 __global__ void rmsnorm_fwd_kernel(const T *__restrict__ x,
                                    const T *__restrict__ res,
@@ -113,88 +117,204 @@ __global__ void rmsnorm_fwd_kernel(const T *__restrict__ x,
   }
 }
 
-// Backward: one workgroup per row (grid sized to give every row its own
-// WG), dx in one pass. dw: each thread's column set is FIXED across its
-// rows (i strides by BLOCK), so the per-thread dw partials live in
-// REGISTERS (<= RB_RN_MAXV vectors = 32 floats at D=8192) and hit
-// global memory once via atomicAdd at the end. The round-1 version
-// accumulated dw element-wise in LDS — 16 scalar ds ops per 16 B of
-// input made LDS the bottleneck (65 us on [2048,4096] vs ~14 ideal).
-// D > 8*BLOCK*RB_RN_MAXV falls back to the LDS path.
-// Register-dw variant, D == NV * BLOCK * W exactly (llama 4096 -> NV=2
-// bf16). NV is a template int so every load is UNGUARDED — a runtime
-// `if (i < nvec)` around unrolled loads makes hipcc branch per element
-// and drain vmcnt(0) each time (cdna_hip_programming.md §5 trap (c));
-// the first cut of this kernel did exactly that and ran 7x slower than
-// the LDS version it meant to replace (r11: 472 us vs 65).
+// The same for rows of up to NV * BLOCK vectors: a thread's NV vectors stay in
+// registers between the two passes, so x, the residual and its slices are read
+// once. Vectors past the row's end read its last one again (a branch around a
+// load would make the compiler wait for each) and count nothing.
 template <typename T, int NV>
-__global__ void rmsnorm_bwd_reg_kernel(const T *__restrict__ x,
-                                       const T *__restrict__ w,
-                                       const T *__restrict__ dy,
-                                       const float *__restrict__ inv_rms,
-                                       T *__restrict__ dx,
-                                       float *__restrict__ dw,
-                                       int64_t n_rows, int D) {
+__global__ __launch_bounds__(BLOCK) void rmsnorm_fwd_reg_kernel(
+    const T *__restrict__ x, const T *__restrict__ res,
+    const float *__restrict__ res32, int rsplit, T *__restrict__ sum_out,
+    const T *__restrict__ w, T *__restrict__ y, float *__restrict__ inv_rms,
+    uint16_t *__restrict__ swz, int64_t n_rows, int D, float eps) {
   constexpr int W = rb::VIO<T>::W;
   __shared__ float red[BLOCK / RB_WAVE];
-
-  float dwacc[NV][W];
+  const int nvec = D / W;
+  int at[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v)
-#pragma unroll
-    for (int k = 0; k < W; ++k) dwacc[v][k] = 0.0f;
-
-  float wf[NV][W];
-#pragma unroll
-  for (int v = 0; v < NV; ++v)
-    rb::VIO<T>::load(w + (v * BLOCK + threadIdx.x) * W, wf[v]);
+    at[v] = min(v * BLOCK + (int)threadIdx.x, nvec - 1) * W;
 
   for (int64_t row = blockIdx.x; row < n_rows; row += gridDim.x) {
-    const T *xr = x + row * D;
-    const T *dyr = dy + row * D;
-    T *dxr = dx + row * D;
-    const float ir = inv_rms[row];
+    float f[NV][W], g[NV][W];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) rb::VIO<T>::load(x + row * D + at[v], f[v]);
+    if (res != nullptr) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v)
+        rb::VIO<T>::load(res + row * D + at[v], g[v]);
+#pragma unroll
+      for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int k = 0; k < W; ++k) f[v][k] += g[v][k];
+    } else if (res32 != nullptr) {
+      for (int sl = 0; sl < rsplit; ++sl) {
+        const float *rp = res32 + ((int64_t)sl * n_rows + row) * D;
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+#pragma unroll
+          for (int k = 0; k < W; k += 4)
+            rb::VIO<float>::load(rp + at[v] + k, g[v] + k);
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+#pragma unroll
+          for (int k = 0; k < W; ++k) f[v][k] += g[v][k];
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) rb::VIO<T>::load(w + at[v], g[v]);
+    float ss = 0.0f;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      if (v * BLOCK + (int)threadIdx.x >= nvec) continue;
+      if (sum_out != nullptr)
+        rb::VIO<T>::store(sum_out + row * D + at[v], f[v]);
+#pragma unroll
+      for (int k = 0; k < W; ++k) ss += f[v][k] * f[v][k];
+    }
+    ss = rb::block_reduce_sum(ss, red);
+    const float ir = rsqrtf(ss / (float)D + eps);
+    if (threadIdx.x == 0 && inv_rms != nullptr) inv_rms[row] = ir;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      if (v * BLOCK + (int)threadIdx.x >= nvec) continue;
+#pragma unroll
+      for (int k = 0; k < W; ++k) f[v][k] = f[v][k] * ir * g[v][k];
+      rb::VIO<T>::store(y + row * D + at[v], f[v]);
+      if constexpr (sizeof(T) == 2) {
+        if (swz != nullptr)
+          rb::VIO<T>::store(reinterpret_cast<T *>(swz) + (at[v] >> 4) * 512 +
+                            ((at[v] >> 3) & 1) * 256 + row * 8, f[v]);
+      }
+    }
+  }
+}
 
-    float xf[NV][W], df[NV][W];
+template <typename T>
+void launch_fwd(const T *x, const T *res, const float *res32, int rsplit,
+                T *sum_out, const T *w, T *y, float *inv_rms, uint16_t *swz,
+                int64_t n_rows, int D, float eps) {
+  if (n_rows == 0) return;
+  const int nv = (D / rb::VIO<T>::W + BLOCK - 1) / BLOCK;
+  auto stream = at::hip::getCurrentHIPStream();
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(std::min<int64_t>(n_rows, 2048)),
+                       dim3(BLOCK), 0, stream, x, res, res32, rsplit, sum_out,
+                       w, y, inv_rms, swz, n_rows, D, eps);
+  };
+  if (nv <= 1) go(rmsnorm_fwd_reg_kernel<T, 1>);
+  else if (nv == 2) go(rmsnorm_fwd_reg_kernel<T, 2>);
+  else if (nv <= 4) go(rmsnorm_fwd_reg_kernel<T, 4>);
+  else go(rmsnorm_fwd_kernel<T>);
+}
+
+// Backward: dx in one pass, rows of up to NV * BLOCK vectors in registers. With
+// `add`, dx also takes the gradient that reaches the normed sum by other ways.
+// DW: each thread's column set is FIXED across its rows, so its dw partials
+// live in registers until the workgroup's row of `dw` [workgroups, D] is
+// written, which rmsnorm_dw_kernel sums. Atomics of a row or a few per
+// workgroup instead are what such a kernel then takes. us on [2048, 4096]: 66
+// with them, 11 without dw, 14 with `add`, 25 with dw.
+template <typename T, int NV, bool DW>
+__global__ __launch_bounds__(BLOCK) void rmsnorm_bwd_reg_kernel(
+    const T *__restrict__ x, const T *__restrict__ w,
+    const T *__restrict__ dy, const float *__restrict__ inv_rms,
+    const T *__restrict__ add, T *__restrict__ dx, float *__restrict__ dw,
+    int64_t n_rows, int D) {
+  constexpr int W = rb::VIO<T>::W;
+  __shared__ float red[BLOCK / RB_WAVE];
+  const int nvec = D / W;
+  int at[NV];
+  float wf[NV][W], acc[DW ? NV : 1][W];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    at[v] = min(v * BLOCK + (int)threadIdx.x, nvec - 1) * W;
+    rb::VIO<T>::load(w + at[v], wf[v]);
+    if constexpr (DW) {
+#pragma unroll
+      for (int k = 0; k < W; ++k) acc[v][k] = 0.0f;
+    }
+  }
+  for (int64_t row = blockIdx.x; row < n_rows; row += gridDim.x) {
+    float xf[NV][W], df[NV][W], af[NV][W];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      rb::VIO<T>::load(x + row * D + at[v], xf[v]);
+      rb::VIO<T>::load(dy + row * D + at[v], df[v]);
+    }
+    if (add != nullptr) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v)
+        rb::VIO<T>::load(add + row * D + at[v], af[v]);
+    } else {
+#pragma unroll
+      for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int k = 0; k < W; ++k) af[v][k] = 0.0f;
+    }
+    const float ir = inv_rms[row];
     float s = 0.0f;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      const int i = v * BLOCK + threadIdx.x;
-      rb::VIO<T>::load(xr + i * W, xf[v]);
-      rb::VIO<T>::load(dyr + i * W, df[v]);
+      if (v * BLOCK + (int)threadIdx.x >= nvec) continue;
 #pragma unroll
       for (int k = 0; k < W; ++k) s += df[v][k] * wf[v][k] * xf[v][k];
     }
     s = rb::block_reduce_sum(s, red);
     const float c = ir * ir * ir * s / (float)D;
-
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      const int i = v * BLOCK + threadIdx.x;
+      if (v * BLOCK + (int)threadIdx.x >= nvec) continue;
       float o[W];
 #pragma unroll
       for (int k = 0; k < W; ++k) {
-        o[k] = ir * wf[v][k] * df[v][k] - c * xf[v][k];
-        dwacc[v][k] += df[v][k] * xf[v][k] * ir;
+        o[k] = af[v][k] + ir * wf[v][k] * df[v][k] - c * xf[v][k];
+        if constexpr (DW) acc[v][k] += df[v][k] * xf[v][k] * ir;
       }
-      rb::VIO<T>::store(dxr + i * W, o);
+      rb::VIO<T>::store(dx + row * D + at[v], o);
     }
   }
-
+  if constexpr (DW) {
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const int i = v * BLOCK + threadIdx.x;
+    for (int v = 0; v < NV; ++v) {
+      if (v * BLOCK + (int)threadIdx.x >= nvec) continue;
 #pragma unroll
-    for (int k = 0; k < W; ++k)
-      if (dwacc[v][k] != 0.0f) atomicAdd(dw + i * W + k, dwacc[v][k]);
+      for (int k = 0; k < W; k += 4)
+        rb::VIO<float>::store(dw + (int64_t)blockIdx.x * D + at[v] + k,
+                              acc[v] + k);
+    }
   }
 }
 
+// Column sums of part [n, D]: 64 columns a workgroup, 16 rows at a time.
+__global__ __launch_bounds__(BLOCK) void rmsnorm_dw_kernel(
+    const float *__restrict__ part, float *__restrict__ dw, int n, int D) {
+  __shared__ float4 red[BLOCK];
+  const int c = blockIdx.x * 64 + (threadIdx.x & 15) * 4;
+  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (c < D)
+    for (int r = threadIdx.x >> 4; r < n; r += 16) {
+      const float4 x = *reinterpret_cast<const float4 *>(
+          part + (int64_t)r * D + c);
+      sum.x += x.x; sum.y += x.y; sum.z += x.z; sum.w += x.w;
+    }
+  red[threadIdx.x] = sum;
+  __syncthreads();
+  if (threadIdx.x >= 16 || c >= D) return;
+  for (int r = 1; r < 16; ++r) {
+    const float4 x = red[r * 16 + threadIdx.x];
+    sum.x += x.x; sum.y += x.y; sum.z += x.z; sum.w += x.w;
+  }
+  *reinterpret_cast<float4 *>(dw + c) = sum;
+}
+
+// Wider rows: dw in LDS.
 template <typename T>
 __global__ void rmsnorm_bwd_kernel(const T *__restrict__ x,
                                            const T *__restrict__ w,
                                            const T *__restrict__ dy,
                                            const float *__restrict__ inv_rms,
+                                           const T *__restrict__ add,
                                            T *__restrict__ dx,
                                            float *__restrict__ dw,
                                            int64_t n_rows, int D) {
@@ -235,6 +355,11 @@ __global__ void rmsnorm_bwd_kernel(const T *__restrict__ x,
         o[k] = ir * wf[k] * df[k] - c * xf[k];
         dw_loc[i * W + k] += df[k] * xf[k] * ir;
       }
+      if (add != nullptr) {
+        rb::VIO<T>::load(add + row * D + i * W, xf);
+#pragma unroll
+        for (int k = 0; k < W; ++k) o[k] += xf[k];
+      }
       rb::VIO<T>::store(dxr + i * W, o);
     }
     __syncthreads();
@@ -254,13 +379,10 @@ std::vector<at::Tensor> rmsnorm_fwd(at::Tensor x, at::Tensor w, double eps) {
   const int64_t n_rows = x.numel() / D;
   auto y = at::empty_like(x);
   auto inv_rms = at::empty({n_rows}, x.options().dtype(at::kFloat));
-  auto stream = at::hip::getCurrentHIPStream();
 
   if (x.scalar_type() == at::kBFloat16) {
     TORCH_CHECK(D % 8 == 0, "rmsnorm bf16: D must be a multiple of 8");
-    hipLaunchKernelGGL(rmsnorm_fwd_kernel<uint16_t>, dim3(std::min<int64_t>(n_rows, 2048)),
-                       dim3(BLOCK), 0, stream,
-                       (const uint16_t *)x.data_ptr(),
+    launch_fwd<uint16_t>((const uint16_t *)x.data_ptr(),
                        (const uint16_t *)nullptr, (const float *)nullptr, 0,
                        (uint16_t *)nullptr,
                        (const uint16_t *)w.data_ptr(),
@@ -268,9 +390,7 @@ std::vector<at::Tensor> rmsnorm_fwd(at::Tensor x, at::Tensor w, double eps) {
                        (uint16_t *)nullptr, n_rows, D, (float)eps);
   } else if (x.scalar_type() == at::kFloat) {
     TORCH_CHECK(D % 4 == 0, "rmsnorm f32: D must be a multiple of 4");
-    hipLaunchKernelGGL(rmsnorm_fwd_kernel<float>, dim3(std::min<int64_t>(n_rows, 2048)),
-                       dim3(BLOCK), 0, stream,
-                       x.data_ptr<float>(), (const float *)nullptr,
+    launch_fwd<float>(x.data_ptr<float>(), (const float *)nullptr,
                        (const float *)nullptr, 0,
                        (float *)nullptr, w.data_ptr<float>(),
                        y.data_ptr<float>(),
@@ -295,15 +415,11 @@ std::vector<at::Tensor> rmsnorm_fwd_dec(at::Tensor x, at::Tensor w,
   TORCH_CHECK(n_rows <= 32 && D % 16 == 0, "rmsnorm_fwd_dec: shape");
   auto y = at::empty_like(x);
   auto swz = at::empty({(int64_t)(D / 16) * 512}, x.options());
-  auto stream = at::cuda::getCurrentHIPStream();
-  auto inv_rms = at::empty({n_rows}, x.options().dtype(at::kFloat));
-  hipLaunchKernelGGL(rmsnorm_fwd_kernel<uint16_t>, dim3(n_rows),
-                     dim3(BLOCK), 0, stream,
-                     (const uint16_t *)x.data_ptr(),
+  launch_fwd<uint16_t>((const uint16_t *)x.data_ptr(),
                      (const uint16_t *)nullptr, (const float *)nullptr, 0,
                      (uint16_t *)nullptr,
                      (const uint16_t *)w.data_ptr(),
-                     (uint16_t *)y.data_ptr(), inv_rms.data_ptr<float>(),
+                     (uint16_t *)y.data_ptr(), (float *)nullptr,
                      (uint16_t *)swz.data_ptr(), n_rows, D, (float)eps);
   return {y, swz};
 }
@@ -324,10 +440,7 @@ std::vector<at::Tensor> rmsnorm_res_fwd_dec(at::Tensor x, at::Tensor res,
   auto sum = at::empty_like(x);
   auto y = at::empty_like(x);
   auto swz = at::empty({(int64_t)(D / 16) * 512}, x.options());
-  auto stream = at::cuda::getCurrentHIPStream();
-  hipLaunchKernelGGL(rmsnorm_fwd_kernel<uint16_t>, dim3(n_rows),
-                     dim3(BLOCK), 0, stream,
-                     (const uint16_t *)x.data_ptr(),
+  launch_fwd<uint16_t>((const uint16_t *)x.data_ptr(),
                      (const uint16_t *)res.data_ptr(),
                      (const float *)nullptr, 0,
                      (uint16_t *)sum.data_ptr(),
@@ -335,6 +448,36 @@ std::vector<at::Tensor> rmsnorm_res_fwd_dec(at::Tensor x, at::Tensor res,
                      (uint16_t *)y.data_ptr(), (float *)nullptr,
                      (uint16_t *)swz.data_ptr(), n_rows, D, (float)eps);
   return {sum, y, swz};
+}
+
+// Residual + norm of any number of rows: {sum = x + res, y, inv_rms}.
+std::vector<at::Tensor> rmsnorm_res_fwd(at::Tensor x, at::Tensor res,
+                                        at::Tensor w, double eps) {
+  TORCH_CHECK(x.is_cuda() && x.is_contiguous() && res.is_contiguous() &&
+              w.is_contiguous() && x.sizes() == res.sizes() && x.dim() >= 1 &&
+              w.numel() == x.size(-1), "rmsnorm_res_fwd: shapes");
+  const int D = (int)x.size(-1);
+  const int64_t n_rows = D ? x.numel() / D : 0;
+  const bool bf16 = x.scalar_type() == at::kBFloat16;
+  TORCH_CHECK((bf16 || x.scalar_type() == at::kFloat) &&
+              res.scalar_type() == x.scalar_type() &&
+              w.scalar_type() == x.scalar_type() && D % (bf16 ? 8 : 4) == 0,
+              "rmsnorm_res_fwd: bf16 or f32, whole vectors");
+  auto sum = at::empty_like(x), y = at::empty_like(x);
+  auto inv_rms = at::empty({n_rows}, x.options().dtype(at::kFloat));
+  if (bf16)
+    launch_fwd<uint16_t>((const uint16_t *)x.data_ptr(),
+                         (const uint16_t *)res.data_ptr(), nullptr, 0,
+                         (uint16_t *)sum.data_ptr(),
+                         (const uint16_t *)w.data_ptr(),
+                         (uint16_t *)y.data_ptr(), inv_rms.data_ptr<float>(),
+                         nullptr, n_rows, D, (float)eps);
+  else
+    launch_fwd<float>(x.data_ptr<float>(), res.data_ptr<float>(), nullptr, 0,
+                      sum.data_ptr<float>(), w.data_ptr<float>(),
+                      y.data_ptr<float>(), inv_rms.data_ptr<float>(), nullptr,
+                      n_rows, D, (float)eps);
+  return {sum, y, inv_rms};
 }
 
 // Same, with the residual as an UNCOMBINED fp32 split-K slab
@@ -354,10 +497,7 @@ std::vector<at::Tensor> rmsnorm_res_slab_fwd_dec(at::Tensor x,
   auto sum = at::empty_like(x);
   auto y = at::empty_like(x);
   auto swz = at::empty({(int64_t)(D / 16) * 512}, x.options());
-  auto stream = at::cuda::getCurrentHIPStream();
-  hipLaunchKernelGGL(rmsnorm_fwd_kernel<uint16_t>, dim3(n_rows),
-                     dim3(BLOCK), 0, stream,
-                     (const uint16_t *)x.data_ptr(),
+  launch_fwd<uint16_t>((const uint16_t *)x.data_ptr(),
                      (const uint16_t *)nullptr,
                      (const float *)slabs.data_ptr(), (int)slabs.size(0),
                      (uint16_t *)sum.data_ptr(),
@@ -493,63 +633,75 @@ std::vector<at::Tensor> rmsnorm_res32(at::Tensor x,
   return {y, swz};
 }
 
-std::vector<at::Tensor> rmsnorm_bwd(at::Tensor x, at::Tensor w, at::Tensor dy,
-                                    at::Tensor inv_rms) {
-  TORCH_CHECK(x.is_cuda() && dy.is_contiguous() && x.is_contiguous(), "rmsnorm_bwd: bad args");
-  const int D = (int)x.size(-1);
-  const int64_t n_rows = x.numel() / D;
-  auto dx = at::empty_like(x);
-  auto dw = at::zeros({D}, x.options().dtype(at::kFloat));
+namespace {
+template <typename T>
+void launch_bwd(const at::Tensor &x, const at::Tensor &w, const at::Tensor &dy,
+                const at::Tensor &inv_rms, const at::Tensor *add,
+                at::Tensor &dx, float *dw, int64_t n_rows, int D) {
   auto stream = at::hip::getCurrentHIPStream();
-  const int nwg = (int)std::min<int64_t>(n_rows, 4096);
-  const size_t shmem = (size_t)D * sizeof(float) + (BLOCK / RB_WAVE) * sizeof(float);
-  TORCH_CHECK(shmem <= 160 * 1024, "rmsnorm_bwd: D too large for LDS accumulation");
-
-  // The register-dw variant measured 7x SLOWER than this LDS path on
-  // [2048,4096] (472 vs 65 us, r11/r13) despite clean ISA (no spills,
-  // 95 VGPR, 5 waves/SIMD) — root cause unidentified; the LDS
-  // accumulate stays the shipped path.
-  const int nv = 0;
-  if (x.scalar_type() == at::kBFloat16) {
-    auto a = (const uint16_t *)x.data_ptr();
-    auto b = (const uint16_t *)w.data_ptr();
-    auto c = (const uint16_t *)dy.data_ptr();
-    auto irp = inv_rms.data_ptr<float>();
-    auto dxp = (uint16_t *)dx.data_ptr();
-    auto dwp = dw.data_ptr<float>();
-    if (nv == 1)
-      hipLaunchKernelGGL((rmsnorm_bwd_reg_kernel<uint16_t, 1>), dim3(nwg),
-                         dim3(BLOCK), 0, stream, a, b, c, irp, dxp, dwp, n_rows, D);
-    else if (nv == 2)
-      hipLaunchKernelGGL((rmsnorm_bwd_reg_kernel<uint16_t, 2>), dim3(nwg),
-                         dim3(BLOCK), 0, stream, a, b, c, irp, dxp, dwp, n_rows, D);
-    else if (nv == 4)
-      hipLaunchKernelGGL((rmsnorm_bwd_reg_kernel<uint16_t, 4>), dim3(nwg),
-                         dim3(BLOCK), 0, stream, a, b, c, irp, dxp, dwp, n_rows, D);
-    else
-      hipLaunchKernelGGL(rmsnorm_bwd_kernel<uint16_t>, dim3(nwg), dim3(BLOCK),
-                         shmem, stream, a, b, c, irp, dxp, dwp, n_rows, D);
-  } else if (x.scalar_type() == at::kFloat) {
-    auto a = x.data_ptr<float>();
-    auto b = w.data_ptr<float>();
-    auto c = dy.data_ptr<float>();
-    auto irp = inv_rms.data_ptr<float>();
-    auto dxp = dx.data_ptr<float>();
-    auto dwp = dw.data_ptr<float>();
-    if (nv == 1)
-      hipLaunchKernelGGL((rmsnorm_bwd_reg_kernel<float, 1>), dim3(nwg),
-                         dim3(BLOCK), 0, stream, a, b, c, irp, dxp, dwp, n_rows, D);
-    else if (nv == 2)
-      hipLaunchKernelGGL((rmsnorm_bwd_reg_kernel<float, 2>), dim3(nwg),
-                         dim3(BLOCK), 0, stream, a, b, c, irp, dxp, dwp, n_rows, D);
-    else if (nv == 4)
-      hipLaunchKernelGGL((rmsnorm_bwd_reg_kernel<float, 4>), dim3(nwg),
-                         dim3(BLOCK), 0, stream, a, b, c, irp, dxp, dwp, n_rows, D);
-    else
-      hipLaunchKernelGGL(rmsnorm_bwd_kernel<float>, dim3(nwg), dim3(BLOCK),
-                         shmem, stream, a, b, c, irp, dxp, dwp, n_rows, D);
+  const T *ap = add == nullptr ? nullptr : (const T *)add->data_ptr();
+  const int nv = (D / rb::VIO<T>::W + BLOCK - 1) / BLOCK;
+  auto go = [&](auto kernel, size_t shmem, int64_t most, float *out) {
+    hipLaunchKernelGGL(kernel, dim3(std::min<int64_t>(n_rows, most)),
+                       dim3(BLOCK), shmem, stream, (const T *)x.data_ptr(),
+                       (const T *)w.data_ptr(), (const T *)dy.data_ptr(),
+                       inv_rms.data_ptr<float>(), ap, (T *)dx.data_ptr(), out,
+                       n_rows, D);
+  };
+  auto pick = [&](auto with_dw) {
+    constexpr bool DW = decltype(with_dw)::value;
+    const int64_t most = DW ? 512 : 2048;
+    const int n = (int)std::min(n_rows, most);
+    at::Tensor part;
+    if (DW) part = at::empty({n, D}, x.options().dtype(at::kFloat));
+    float *out = DW ? part.data_ptr<float>() : nullptr;
+    if (nv <= 1) go(rmsnorm_bwd_reg_kernel<T, 1, DW>, 0, most, out);
+    else if (nv == 2) go(rmsnorm_bwd_reg_kernel<T, 2, DW>, 0, most, out);
+    else go(rmsnorm_bwd_reg_kernel<T, 4, DW>, 0, most, out);
+    if (DW)
+      hipLaunchKernelGGL(rmsnorm_dw_kernel, dim3((D + 63) / 64), dim3(BLOCK),
+                         0, stream, out, dw, n, D);
+  };
+  if (nv > 4) {
+    const size_t shmem = ((size_t)D + BLOCK / RB_WAVE) * sizeof(float);
+    TORCH_CHECK(shmem <= 160 * 1024,
+                "rmsnorm_bwd: D too large for LDS accumulation");
+    go(rmsnorm_bwd_kernel<T>, shmem, 512, dw);
+  } else if (dw != nullptr) {
+    pick(std::true_type{});
   } else {
-    TORCH_CHECK(false, "rmsnorm_bwd: unsupported dtype");
+    pick(std::false_type{});
   }
+}
+}  // namespace
+
+// {dx (+ add), dw fp32, undefined without need_dw}
+std::vector<at::Tensor> rmsnorm_bwd(at::Tensor x, at::Tensor w, at::Tensor dy,
+                                    at::Tensor inv_rms, bool need_dw,
+                                    c10::optional<at::Tensor> add) {
+  TORCH_CHECK(x.is_cuda() && dy.is_contiguous() && x.is_contiguous() &&
+              dy.sizes() == x.sizes() && w.is_contiguous() &&
+              dy.scalar_type() == x.scalar_type() &&
+              w.scalar_type() == x.scalar_type(), "rmsnorm_bwd: bad args");
+  TORCH_CHECK(!add.has_value() ||
+              (add->is_contiguous() && add->sizes() == x.sizes() &&
+               add->scalar_type() == x.scalar_type()), "rmsnorm_bwd: add");
+  const int D = (int)x.size(-1);
+  const int64_t n_rows = D ? x.numel() / D : 0;
+  auto dx = at::empty_like(x);
+  at::Tensor dw;
+  // rows wider than the register kernels' always make dw
+  const int wide = 4 * BLOCK * (x.scalar_type() == at::kBFloat16 ? 8 : 4);
+  if (need_dw || D > wide)
+    dw = at::zeros({D}, x.options().dtype(at::kFloat));
+  float *dwp = dw.defined() ? dw.data_ptr<float>() : nullptr;
+  const at::Tensor *ap = add.has_value() ? &*add : nullptr;
+  if (n_rows == 0) return {dx, dw};
+  if (x.scalar_type() == at::kBFloat16)
+    launch_bwd<uint16_t>(x, w, dy, inv_rms, ap, dx, dwp, n_rows, D);
+  else if (x.scalar_type() == at::kFloat)
+    launch_bwd<float>(x, w, dy, inv_rms, ap, dx, dwp, n_rows, D);
+  else
+    TORCH_CHECK(false, "rmsnorm_bwd: unsupported dtype");
   return {dx, dw};
 }

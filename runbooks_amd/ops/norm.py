@@ -25,8 +25,35 @@ class _RMSNormFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, weight, inv_rms = ctx.saved_tensors
-        dx, dw = _backend.ext().rmsnorm_bwd(x, weight, dy.contiguous(), inv_rms)
-        return dx, dw.to(weight.dtype), None
+        dx, dw = _backend.ext().rmsnorm_bwd(x, weight, dy.contiguous(),
+                                            inv_rms, ctx.needs_input_grad[1])
+        return dx, _as_weight(dw, weight, ctx.needs_input_grad[1]), None
+
+
+def _as_weight(dw, weight, needed):
+    return dw.to(weight.dtype) if needed else None
+
+
+class _ResNormFn(torch.autograd.Function):
+    """(x + delta, rmsnorm(x + delta) * weight): the sum's gradient joins the
+    norm's in its backward kernel."""
+
+    @staticmethod
+    def forward(ctx, x, delta, weight, eps):
+        s, y, inv_rms = _backend.ext().rmsnorm_res_fwd(x, delta, weight, eps)
+        ctx.save_for_backward(s, weight, inv_rms)
+        ctx.set_materialize_grads(False)
+        return s, y
+
+    @staticmethod
+    def backward(ctx, ds, dy):
+        if dy is None:
+            return ds, ds, None, None
+        s, weight, inv_rms = ctx.saved_tensors
+        dx, dw = _backend.ext().rmsnorm_bwd(
+            s, weight, dy.contiguous(), inv_rms, ctx.needs_input_grad[2],
+            None if ds is None else ds.contiguous())
+        return dx, dx, _as_weight(dw, weight, ctx.needs_input_grad[2]), None
 
 
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.Tensor:
@@ -43,6 +70,22 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.T
             return y
         return _RMSNormFn.apply(x.contiguous(), weight.contiguous(), eps)
     return rmsnorm_ref(x, weight, eps)
+
+
+def rmsnorm_res(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor,
+                eps: float) -> tuple[torch.Tensor, torch.Tensor]:
+    """x + delta and its norm, differentiable."""
+    if not _backend.use_hip(x):
+        x = x + delta
+        return x, rmsnorm_ref(x, weight, eps)
+    if (not torch.is_grad_enabled() and x.dtype == torch.bfloat16
+            and x.numel() // x.shape[-1] <= 32 and x.shape[-1] % 16 == 0):
+        x, y, swz = _backend.ext().rmsnorm_res_fwd_dec(
+            x.contiguous(), delta.contiguous(), weight.contiguous(), eps)
+        y._rb_swz = swz
+        return x, y
+    return _ResNormFn.apply(x.contiguous(), delta.contiguous(),
+                            weight.contiguous(), eps)
 
 
 def rmsnorm_res32(x: torch.Tensor, delta: torch.Tensor | None,

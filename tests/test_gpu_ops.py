@@ -618,6 +618,98 @@ def test_geglu_packed():
 
 
 @pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("T,hq,hkv,dh,vt", [
+    (1, 4, 4, 128, False), (33, 2, 1, 256, False), (63, 8, 2, 64, True),
+    (64, 8, 2, 128, True), (65, 4, 1, 64, True), (200, 16, 4, 128, True)])
+def test_qkv_rope_append_layouts(T, hq, hkv, dh, vt, fp8):
+    """Rotation in place and to a tensor, into every cache layout; tokens that
+    fill cache blocks in order, out of order and not at all."""
+    _assert_hip()
+    from runbooks_amd.ops.kvcache import alloc_kv_cache, fp8_dequant_cache_ref
+    g = torch.Generator().manual_seed(T + dh)
+    y = torch.randn(T, (hq + 2 * hkv) * dh, generator=g).bfloat16()
+    cos, sin = ops.rope_tables(dh, 512)
+    pos = torch.randint(0, 512, (T,), generator=g, dtype=torch.int32)
+    n = T // 16 + 3
+    slots = torch.cat([16 * b + torch.arange(16) for b in
+                       torch.randperm(n, generator=g).tolist()])[:T].int()
+    if T > 40:
+        slots[17:30] = slots[17:30].flip(0)
+    if T > 1:
+        slots[T // 2] = -1
+    q, k, v = (x.view(T, -1, dh) for x in
+               y.split([hq * dh, hkv * dh, hkv * dh], -1))
+    q, k = (ops.rope_ref(x, cos, sin, pos) for x in (q, k))
+    kc, vc = alloc_kv_cache(n, hkv, dh, "cpu", fp8=fp8, v_transposed=vt)
+    got = [c.to(DEV) for c in (kc, vc)]
+    ops.kv_append_ref(k, v, kc, vc, slots)
+    args = (cos.to(DEV), sin.to(DEV), pos.to(DEV), *got, slots.to(DEV), hq)
+    qd = ops.ext().qkv_rope_append(y.to(DEV), *args)
+    # one rounding apart where the fused multiply-adds differ
+    assert (qd.cpu().float() - q.float()).abs().max() <= 2 ** -6
+
+    def check():
+        for c, ref in zip(got, (kc, vc)):
+            if fp8:
+                a, b = (fp8_dequant_cache_ref(x) for x in (c.cpu(), ref))
+                # a rounding to e4m3 (2^-3 of the value) may fall otherwise
+                assert ((a - b).abs() <= b.abs() / 8 + 1e-2).all()
+                assert (a - b).norm() <= 0.01 * b.norm()
+            else:
+                assert (c.cpu().float() - ref.float()).abs().max() <= 2 ** -6
+
+    check()
+    for c in got:
+        c.zero_()
+    yd = y.to(DEV)
+    ops.ext().qkv_rope_append_(yd, *args)
+    check()
+    want = torch.cat([x.reshape(T, -1) for x in (q, k, v)], -1)
+    assert (yd.cpu().float() - want.float()).abs().max() <= 2 ** -6
+
+
+def test_flash_prefill_qkv():
+    """q, k and v read side by side are read as if apart."""
+    _assert_hip()
+    y = torch.randn(2 * 77, (8 + 2 * 2) * 64, device=DEV).bfloat16()
+    q, k, v = (x.reshape(2, 77, -1, 64) for x in y.split([512, 128, 128], -1))
+    assert torch.equal(ops.ext().flash_prefill_qkv(y, 2, 77, 8, 2, 64, 0.125),
+                       ops.flash_prefill(q, k, v, 0.125))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,D", [
+    (1, 8), (3, 2048), (5, 2056), (700, 768), (2, 4544), (33, 8192),
+    (2, 8200)])
+def test_rmsnorm_residual(rows, D, dtype):
+    """Sum and norm forward and backward, a row in 1, 2 and 4 vectors a thread
+    and wider; weights with and without gradient."""
+    _assert_hip()
+    g = torch.Generator(device=DEV).manual_seed(D)
+    x, d, ds, dy = (torch.randn(rows, D, generator=g, device=DEV).to(dtype)
+                    for _ in range(4))
+    w = (1 + 0.1 * torch.randn(D, generator=g, device=DEV)).to(dtype)
+    tol = 1e-5 if dtype == torch.float32 else 2 ** -7
+    ref = [t.double().requires_grad_() for t in (x, d, w)]
+    s = ref[0] + ref[1]
+    y = s * (s.square().mean(-1, keepdim=True) + 1e-5).rsqrt() * ref[2]
+    torch.autograd.backward([s, y], [ds.double(), dy.double()])
+    for trains in (True, False):
+        leaves = [t.clone().requires_grad_() for t in (x, d)]
+        wt = w.clone().requires_grad_(trains)
+        got = ops.rmsnorm_res(*leaves, wt, 1e-5)
+        torch.autograd.backward(got, [ds, dy])
+        pairs = list(zip(got, (s, y))) + list(zip(
+            [t.grad for t in leaves], [t.grad for t in ref]))
+        if trains:
+            pairs.append((wt.grad, ref[2].grad))
+        else:
+            assert wt.grad is None
+        for a, b in pairs:
+            assert (a.double() - b).norm() <= tol * b.norm()
+
+
+@pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("hq,hkv,dh,vt", [
     (4, 4, 128, False), (4, 2, 64, False), (2, 2, 256, False),
     (8, 2, 128, True), (16, 1, 64, True), (8, 1, 128, True),

@@ -113,6 +113,16 @@ class Attention(nn.Module):
         return q, k, v
 
     def forward_train(self, x, cos, sin, positions, B, S):
+        group = getattr(self.q_proj, "_group", None)
+        if group is not None and self.cfg.pos == "rope" and \
+                self.dh in (64, 128) and cos.dtype == torch.float32 and \
+                (torch.is_grad_enabled() or
+                 getattr(self, "_qkv_w", None) is None):
+            y = group.packed(x)     # sibling adapters, q, k and v side by side
+            if y is not None:
+                o = ops.packed_attention(y, cos, sin, positions, B, S, self.hq,
+                                         self.hkv, self.scale)
+                return self.o_proj(o.view(B * S, self.hq * self.dh))
         q, k, v = self._qkv(x, cos, sin, positions)
         q = q.view(B, S, self.hq, self.dh)
         k = k.view(B, S, self.hkv, self.dh)
@@ -206,6 +216,10 @@ class MLP(nn.Module):
                 half = y.shape[-1] // 2
                 return self.down_proj(ops.swiglu(
                     y[:, :half].contiguous(), y[:, half:].contiguous()))
+            group = getattr(self.gate_proj, "_group", None)
+            y = group.packed(x) if group is not None else None
+            if y is not None:
+                return self.down_proj(ops.swiglu_packed(y))
             return self.down_proj(ops.swiglu(self.gate_proj(x), self.up_proj(x)))
         if self.act == "gelu_glu":
             # gemma GeGLU (tanh approximation); fused gate/up GEMM +

@@ -5,10 +5,12 @@ plain-PyTorch fp32 references (the numerics oracles). A GPU tensor with no
 built extension raises — there is no silent eager fallback on the GPU.
 """
 from ._backend import ext, has_hip, use_hip  # noqa: F401
-from .activations import cross_entropy, geglu, softcap, swiglu  # noqa: F401
+from .activations import (cross_entropy, geglu, softcap, swiglu,  # noqa: F401
+                          swiglu_packed)
 from .adamw import FusedAdamW  # noqa: F401
-from .attention import (causal_attention, flash_prefill, paged_decode,  # noqa: F401
-                        paged_decode_ref, paged_decode_with_operand)
+from .attention import (causal_attention, flash_prefill, packed_attention,  # noqa: F401
+                        paged_decode, paged_decode_ref,
+                        paged_decode_with_operand)
 from .kvcache import BLOCK_SIZE, alloc_kv_cache, kv_append, kv_append_ref  # noqa: F401
 from .latent import alloc_latent_cache, pad_to  # noqa: F401
 from .lightning import alloc_lightning_state  # noqa: F401

@@ -26,6 +26,24 @@ def swiglu(g: torch.Tensor, u: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.silu(g) * u
 
 
+class _SwiGLUPackedFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, y):
+        ctx.save_for_backward(y)
+        return _backend.ext().swiglu_packed(y)
+
+    @staticmethod
+    def backward(ctx, dh):
+        return _backend.ext().swiglu_packed_bwd(dh.contiguous(),
+                                                *ctx.saved_tensors)
+
+
+def swiglu_packed(y: torch.Tensor) -> torch.Tensor:
+    """silu(g) * u of g and u side by side in the rows of y [T, 2 I],
+    differentiable (GPU, bf16)."""
+    return _SwiGLUPackedFn.apply(y)
+
+
 def geglu(y: torch.Tensor, operand: bool = False) -> torch.Tensor:
     """gelu_tanh(y[:, :I]) * y[:, I:] of a fused gate/up product (serving;
     I % 8 == 0). operand=True also attaches the decode GEMM's operand

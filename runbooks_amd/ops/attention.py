@@ -50,6 +50,37 @@ class _FlashAttnTrain(torch.autograd.Function):
         return dq, dk, dv, None
 
 
+class _PackedAttnTrain(torch.autograd.Function):
+    """Rotation and causal attention of q, k and v side by side in the rows of
+    y [B * S, (hq + 2 hkv) * dh], of which it takes possession: q and k are
+    rotated in place. The gradient comes back side by side too."""
+
+    @staticmethod
+    def forward(ctx, y, cos, sin, positions, B, S, hq, hkv, scale):
+        ext, dh = _backend.ext(), y.shape[1] // (hq + 2 * hkv)
+        ext.rope_qkv_(y, cos, sin, positions, hq, hkv, dh)
+        out, lse = ext.flash_fwd_train_qkv(y, B, S, hq, hkv, dh, scale)
+        ctx.save_for_backward(y, cos, sin, positions, out, lse)
+        ctx.sizes = (B, S, hq, hkv, dh, scale)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        y, cos, sin, positions, out, lse = ctx.saved_tensors
+        _, _, hq, hkv, dh, _ = ctx.sizes
+        dy, dk, dv = _backend.ext().fa_bwd_qkv(dout.contiguous(), y, out, lse,
+                                               *ctx.sizes)
+        _backend.ext().rope_qkv_(dy, cos, sin, positions, hq, hkv, dh, True,
+                                 dk, dv)
+        return (dy,) + (None,) * 8
+
+
+def packed_attention(y, cos, sin, positions, B, S, hq, hkv, scale):
+    """Differentiable; GPU, bf16, head sizes 64 and 128. y is consumed."""
+    return _PackedAttnTrain.apply(y, cos, sin, positions, B, S, hq, hkv,
+                                  float(scale))
+
+
 def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                      scale: float | None = None, q_block: int = 256) -> torch.Tensor:
     """q [B, S, Hq, Dh]; k, v [B, S, Hkv, Dh] -> [B, S, Hq, Dh].

@@ -52,8 +52,10 @@ struct Args {
   const uint16_t *q, *k, *v, *dout, *out;
   const float *lse;                     // [B, Hq, S]
   float *dvec;                          // [B, Hq, S]
-  uint16_t *dq, *dk, *dv;               // [B, S, Hq, DH]
+  uint16_t *dq, *dk, *dv;               // per q-head
   int B, S, Hq, Hkv;
+  // elements between the tokens of q, of k and v, of dq, of dk and dv
+  int64_t q_stride, kv_stride, dq_stride, dkv_stride;
   float scale;
 };
 
@@ -115,19 +117,19 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
   const int qrow = wrow + col;
   const bool q_valid = qrow < S;
 
-  const int64_t kv_stride = (int64_t)a.Hkv * DH;
-  const int64_t kv0 = ((int64_t)at.batch * S * a.Hkv + h_kv) * DH;
+  const int64_t kv_stride = a.kv_stride;
+  const int64_t kv0 = (int64_t)at.batch * S * kv_stride + h_kv * DH;
   const uint16_t *kb = a.k + kv0, *vb = a.v + kv0;
   const TileLoad<DH, NW> load(wid, lane);
   const int n_tiles = (min(S, at.tile * QT + QT) + ROWS - 1) / ROWS;
   load(kb, kv_stride, 0, S, smem, wid);
   load(vb, kv_stride, 0, S, smem + TILE, wid);
 
-  const int64_t row0 =
-      (((int64_t)at.batch * S + (q_valid ? qrow : 0)) * a.Hq + at.head) * DH;
+  const int64_t token = (int64_t)at.batch * S + (q_valid ? qrow : 0);
+  const int64_t row0 = (token * a.Hq + at.head) * DH;    // of dout, out
   const int64_t stat = ((int64_t)at.batch * a.Hq + at.head) * S + qrow;
   bf16x8v qf[KSTEPS], dof[KSTEPS];
-  load_row<DH>(qf, a.q + row0, hi);
+  load_row<DH>(qf, a.q + token * a.q_stride + at.head * DH, hi);
   clear_if<DH>(a.scale == 0.0f, qf);
   load_row<DH>(dof, a.dout + row0, hi);
   float dvec = 0.0f;
@@ -200,7 +202,8 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
       if (t * ROWS + r0 <= wrow + 31)
         keys(kt, kt + TILE, t * ROWS + r0, r0, std::true_type{});
   }
-  if (q_valid) store_row<DH>(a.dq + row0, acc, a.scale, hi);
+  if (q_valid)
+    store_row<DH>(a.dq + token * a.dq_stride + at.head * DH, acc, a.scale, hi);
 }
 
 template <int DH, int NW>
@@ -222,9 +225,10 @@ void fa_bwd_dkdv_kernel(Args a) {
   const int key = wkey + col;
   const bool k_valid = key < S;
 
-  const int64_t q_stride = (int64_t)a.Hq * DH;
-  const int64_t q00 = ((int64_t)at.batch * S * a.Hq + at.head) * DH;
-  const uint16_t *qb = a.q + q00, *ob = a.dout + q00;
+  const int64_t o_stride = (int64_t)a.Hq * DH;
+  const int64_t token0 = (int64_t)at.batch * S;
+  const uint16_t *qb = a.q + token0 * a.q_stride + at.head * DH;
+  const uint16_t *ob = a.dout + token0 * o_stride + at.head * DH;
   const int64_t stat = ((int64_t)at.batch * a.Hq + at.head) * S;
   const float by = unit(a.scale), to2 = by * LOG2E;
   const TileLoad<DH, NW> load(wid, lane);
@@ -233,8 +237,8 @@ void fa_bwd_dkdv_kernel(Args a) {
   // tile t's rows and statistics; the latter through registers, stored when
   // the tile before it has been worked on
   auto send = [&](int t, char *tile) {
-    load(qb, q_stride, t * ROWS, S, tile, wid);
-    load(ob, q_stride, t * ROWS, S, tile + TILE, wid);
+    load(qb, a.q_stride, t * ROWS, S, tile, wid);
+    load(ob, o_stride, t * ROWS, S, tile + TILE, wid);
   };
   char *stats = smem + 4 * TILE;        // two buffers, like the tiles
   auto stat_of = [&](int t) {
@@ -255,7 +259,7 @@ void fa_bwd_dkdv_kernel(Args a) {
   bf16x8v kf[KSTEPS], vf[KSTEPS];
   {
     const int64_t row0 =
-        (((int64_t)at.batch * S + (k_valid ? key : 0)) * a.Hkv + h_kv) * DH;
+        (token0 + (k_valid ? key : 0)) * a.kv_stride + h_kv * DH;
     load_row<DH>(kf, a.k + row0, hi);
     clear_if<DH>(a.scale == 0.0f, kf);
     load_row<DH>(vf, a.v + row0, hi);
@@ -336,8 +340,7 @@ void fa_bwd_dkdv_kernel(Args a) {
   for (; t < n_tiles; ++t) step(t, std::false_type{});
 
   if (k_valid) {
-    const int64_t row0 =
-        (((int64_t)at.batch * S + key) * a.Hq + at.head) * DH;
+    const int64_t row0 = (token0 + key) * a.dkv_stride + at.head * DH;
     store_row<DH>(a.dk + row0, acc_dk, a.scale, hi);
     store_row<DH>(a.dv + row0, acc_dv, 1.0f, hi);
   }
@@ -363,6 +366,19 @@ template <int DH, int NW> void launch_bwd(const Args &a, hipStream_t stream) {
                      dim3(NW * 64), sh_dq, stream, a);
   hipLaunchKernelGGL((fa_bwd_dkdv_kernel<DH, NW>), dim3((unsigned)grid),
                      dim3(NW * 64), sh_dkdv, stream, a);
+}
+
+void launch_bwd(int64_t DH, const Args &a) {
+  auto stream = at::hip::getCurrentHIPStream();
+  // Workgroups of two waves while there are too few tiles of 32 rows for four
+  // waves on every CU (us for 2 and 4 waves: 200 tokens, 12 heads of 64, 84
+  // tiles, 17 and 19; 512 tokens, 32 heads of 128, 512 tiles, 48 and 50; four
+  // times those 81 and 79).
+  const bool few = (int64_t)(a.S + 31) / 32 * a.Hq * a.B <= 512;
+  if (DH == 128)
+    few ? launch_bwd<128, 2>(a, stream) : launch_bwd<128, 4>(a, stream);
+  else
+    few ? launch_bwd<64, 2>(a, stream) : launch_bwd<64, 4>(a, stream);
 }
 
 }  // namespace
@@ -417,15 +433,56 @@ std::vector<at::Tensor> fa_bwd(at::Tensor dout, at::Tensor q, at::Tensor k,
   a.dv = (uint16_t *)dv.data_ptr();
   a.B = B; a.S = S; a.Hq = Hq; a.Hkv = Hkv;
   a.scale = (float)scale;
-  auto stream = at::hip::getCurrentHIPStream();
-  // Workgroups of two waves while there are too few tiles of 32 rows for four
-  // waves on every CU (us for 2 and 4 waves: 200 tokens, 12 heads of 64, 84
-  // tiles, 17 and 19; 512 tokens, 32 heads of 128, 512 tiles, 48 and 50; four
-  // times those 81 and 79).
-  const bool few = (int64_t)(S + 31) / 32 * Hq * B <= 512;
-  if (DH == 128)
-    few ? launch_bwd<128, 2>(a, stream) : launch_bwd<128, 4>(a, stream);
-  else
-    few ? launch_bwd<64, 2>(a, stream) : launch_bwd<64, 4>(a, stream);
+  a.q_stride = a.dq_stride = a.dkv_stride = (int64_t)Hq * DH;
+  a.kv_stride = (int64_t)Hkv * DH;
+  launch_bwd(DH, a);
   return {dq, dk, dv};
+}
+
+// The same for q, k and v side by side in the rows of y
+// [B * S, (Hq + 2 Hkv) * DH]: {dy, dk, dv}. With fewer kv heads than query heads
+// dk and dv are per query head ([B * S, Hq, DH]) and their columns of dy are
+// not written; else dk and dv are empty.
+std::vector<at::Tensor> fa_bwd_qkv(at::Tensor dout, at::Tensor y,
+                                   at::Tensor out, at::Tensor lse, int64_t B,
+                                   int64_t S, int64_t Hq, int64_t Hkv,
+                                   int64_t DH, double scale) {
+  const int64_t width = (Hq + 2 * Hkv) * DH;
+  TORCH_CHECK(y.is_cuda() && y.is_contiguous() && y.dim() == 2 &&
+              y.scalar_type() == at::kBFloat16 && y.size(0) == B * S &&
+              y.size(1) == width && Hkv > 0 && Hq % Hkv == 0 &&
+              (DH == 64 || DH == 128) &&
+              reinterpret_cast<uintptr_t>(y.data_ptr()) % 16 == 0,
+              "fa_bwd_qkv: y");
+  TORCH_CHECK(dout.is_contiguous() && out.is_contiguous() &&
+              dout.numel() == B * S * Hq * DH && out.numel() == dout.numel() &&
+              dout.scalar_type() == at::kBFloat16 &&
+              out.scalar_type() == at::kBFloat16 && lse.is_contiguous() &&
+              lse.scalar_type() == at::kFloat && lse.numel() == B * Hq * S,
+              "fa_bwd_qkv: dout, out, lse");
+  dout = aligned16(dout);
+  out = aligned16(out);
+  auto dy = at::empty_like(y);
+  const bool grouped = Hq != Hkv;
+  auto dk = at::empty({grouped ? B * S : 0, Hq, DH}, y.options());
+  auto dv = at::empty_like(dk);
+  auto dvec = at::empty({B, Hq, S}, y.options().dtype(at::kFloat));
+  if (dy.numel() == 0) return {dy, dk, dv};
+  Args a{};
+  a.q = (const uint16_t *)y.data_ptr();
+  a.k = a.q + Hq * DH;
+  a.v = a.k + Hkv * DH;
+  a.dout = (const uint16_t *)dout.data_ptr();
+  a.out = (const uint16_t *)out.data_ptr();
+  a.lse = lse.data_ptr<float>();
+  a.dvec = dvec.data_ptr<float>();
+  a.dq = (uint16_t *)dy.data_ptr();
+  a.dk = grouped ? (uint16_t *)dk.data_ptr() : a.dq + Hq * DH;
+  a.dv = grouped ? (uint16_t *)dv.data_ptr() : a.dq + (Hq + Hkv) * DH;
+  a.B = (int)B; a.S = (int)S; a.Hq = (int)Hq; a.Hkv = (int)Hkv;
+  a.q_stride = a.kv_stride = a.dq_stride = width;
+  a.dkv_stride = grouped ? Hq * DH : width;
+  a.scale = (float)scale;
+  launch_bwd(DH, a);
+  return {dy, dk, dv};
 }

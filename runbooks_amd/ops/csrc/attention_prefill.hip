@@ -355,8 +355,9 @@ static at::Tensor flash_fwd_impl(at::Tensor q, at::Tensor k, at::Tensor v,
 }
 
 // q, k and v side by side in the rows of y [B * S, (Hq + 2 Hkv) * DH].
-at::Tensor flash_prefill_qkv(at::Tensor y, int64_t B, int64_t S, int64_t Hq,
-                             int64_t Hkv, int64_t DH, double scale) {
+static at::Tensor flash_qkv_impl(const at::Tensor &y, int64_t B, int64_t S,
+                                 int64_t Hq, int64_t Hkv, int64_t DH,
+                                 double scale, float *lse) {
   const int64_t width = (Hq + 2 * Hkv) * DH;
   TORCH_CHECK(y.is_cuda() && y.is_contiguous() && y.dim() == 2 &&
               y.scalar_type() == at::kBFloat16 && y.size(0) == B * S &&
@@ -367,9 +368,23 @@ at::Tensor flash_prefill_qkv(at::Tensor y, int64_t B, int64_t S, int64_t Hq,
   if (out.numel() == 0) return out;
   const uint16_t *p = (const uint16_t *)y.data_ptr();
   launch_prefill(DH, {p, p + Hq * DH, p + (Hq + Hkv) * DH,
-                      (uint16_t *)out.data_ptr(), nullptr, B, S, Hq, Hkv,
-                      width, width, (float)scale});
+                      (uint16_t *)out.data_ptr(), lse, B, S, Hq, Hkv, width,
+                      width, (float)scale});
   return out;
+}
+
+at::Tensor flash_prefill_qkv(at::Tensor y, int64_t B, int64_t S, int64_t Hq,
+                             int64_t Hkv, int64_t DH, double scale) {
+  return flash_qkv_impl(y, B, S, Hq, Hkv, DH, scale, nullptr);
+}
+
+std::vector<at::Tensor> flash_fwd_train_qkv(at::Tensor y, int64_t B, int64_t S,
+                                            int64_t Hq, int64_t Hkv,
+                                            int64_t DH, double scale) {
+  auto lse = at::empty({B, Hq, S}, y.options().dtype(at::kFloat));
+  auto out = flash_qkv_impl(y, B, S, Hq, Hkv, DH, scale,
+                            lse.data_ptr<float>());
+  return {out, lse};
 }
 
 at::Tensor flash_prefill(at::Tensor q, at::Tensor k, at::Tensor v,

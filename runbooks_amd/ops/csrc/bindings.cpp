@@ -27,6 +27,25 @@ std::vector<at::Tensor> paged_decode_swz(at::Tensor q, at::Tensor k_cache,
                                          at::Tensor seq_lens, int64_t nsplit,
                                          double scale,
                                          c10::optional<at::Tensor> seq_starts);
+std::vector<at::Tensor> flash_fwd_train_qkv(at::Tensor y, int64_t B, int64_t S,
+                                            int64_t Hq, int64_t Hkv,
+                                            int64_t DH, double scale);
+std::vector<at::Tensor> fa_bwd_qkv(at::Tensor dout, at::Tensor y,
+                                   at::Tensor out, at::Tensor lse, int64_t B,
+                                   int64_t S, int64_t Hq, int64_t Hkv,
+                                   int64_t DH, double scale);
+void rope_qkv_(at::Tensor y, at::Tensor cos, at::Tensor sin,
+               at::Tensor positions, int64_t hq, int64_t hkv, int64_t dh,
+               bool inverse, c10::optional<at::Tensor> dk,
+               c10::optional<at::Tensor> dv);
+at::Tensor swiglu_packed_bwd(at::Tensor dh, at::Tensor y);
+at::Tensor lora_down(at::Tensor x, std::vector<at::Tensor> as);
+at::Tensor lora_down_columns(at::Tensor dy, std::vector<at::Tensor> bs,
+                             double scale);
+void lora_add_(at::Tensor y, at::Tensor t, std::vector<at::Tensor> ms,
+               double scale, bool sum);
+at::Tensor lora_grad(at::Tensor x, at::Tensor t, std::vector<int64_t> widths,
+                     double scale, bool transposed);
 at::Tensor flash_prefill_qkv(at::Tensor y, int64_t B, int64_t S, int64_t Hq,
                              int64_t Hkv, int64_t DH, double scale);
 void qkv_rope_append_(at::Tensor y, at::Tensor cos, at::Tensor sin,
@@ -80,6 +99,22 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("block_tables"), py::arg("seq_lens"), py::arg("nsplit"),
         py::arg("scale"), py::arg("seq_starts") = py::none());
   m.def("flash_prefill", &flash_prefill, "MFMA flash-attention prefill (causal)");
+  m.def("flash_fwd_train_qkv", &flash_fwd_train_qkv,
+        "flash_fwd_train of q, k and v side by side in one tensor");
+  m.def("fa_bwd_qkv", &fa_bwd_qkv,
+        "fa_bwd of q, k and v side by side -> (dy, dk_perq, dv_perq)");
+  m.def("rope_qkv_", &rope_qkv_, "RoPE of q and k within packed rows",
+        py::arg("y"), py::arg("cos"), py::arg("sin"), py::arg("positions"),
+        py::arg("hq"), py::arg("hkv"), py::arg("dh"),
+        py::arg("inverse") = false, py::arg("dk") = py::none(),
+        py::arg("dv") = py::none());
+  m.def("swiglu_packed_bwd", &swiglu_packed_bwd,
+        "SwiGLU backward of g and u side by side");
+  m.def("lora_down", &lora_down, "t_i = x A_i^T of sibling adapters");
+  m.def("lora_down_columns", &lora_down_columns, "dt_i = scale dy_i B_i");
+  m.def("lora_add_", &lora_add_,
+        "y_i += scale t_i B_i^T, or y += scale sum t_i A_i");
+  m.def("lora_grad", &lora_grad, "scale x_i^T t_i, or scale t_i^T x");
   m.def("flash_prefill_qkv", &flash_prefill_qkv,
         "flash_prefill of q, k and v side by side in one tensor");
   m.def("qkv_rope_append_", &qkv_rope_append_,

@@ -55,7 +55,49 @@ __global__ void swiglu_bwd_kernel(const T *__restrict__ dy, const T *__restrict_
   }
 }
 
+// g and u side by side in the rows of y [T, 2 I], and so are their gradients.
+__global__ void swiglu_packed_bwd_kernel(const uint16_t *__restrict__ dh,
+                                         const uint16_t *__restrict__ y,
+                                         uint16_t *__restrict__ dy, int64_t T,
+                                         int I) {
+  const int nvec = I / 8;
+  const int64_t total = T * nvec, stride = (int64_t)gridDim.x * BLOCK;
+  for (int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x; i < total;
+       i += stride) {
+    const int64_t at = i / nvec * 2 * I + i % nvec * 8;
+    float d[8], g[8], u[8];
+    rb::VIO<uint16_t>::load(dh + i * 8, d);
+    rb::VIO<uint16_t>::load(y + at, g);
+    rb::VIO<uint16_t>::load(y + at + I, u);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float s = sigmoidf(g[e]), silu = g[e] * s;
+      g[e] = d[e] * u[e] * (s * (1.0f + g[e] * (1.0f - s)));
+      u[e] = d[e] * silu;
+    }
+    rb::VIO<uint16_t>::store(dy + at, g);
+    rb::VIO<uint16_t>::store(dy + at + I, u);
+  }
+}
+
 }  // namespace
+
+at::Tensor swiglu_packed_bwd(at::Tensor dh, at::Tensor y) {
+  TORCH_CHECK(dh.is_cuda() && dh.is_contiguous() && y.is_contiguous() &&
+              y.dim() == 2 && dh.dim() == 2 && dh.size(0) == y.size(0) &&
+              y.size(1) == 2 * dh.size(1) && dh.size(1) % 8 == 0 &&
+              dh.scalar_type() == at::kBFloat16 &&
+              y.scalar_type() == at::kBFloat16, "swiglu_packed_bwd: bf16");
+  auto dy = at::empty_like(y);
+  if (dh.numel() == 0) return dy;
+  const int grid = rb::rb_grid_1d(dh.numel() / 8, BLOCK);
+  hipLaunchKernelGGL(swiglu_packed_bwd_kernel, dim3(grid), dim3(BLOCK), 0,
+                     at::hip::getCurrentHIPStream(),
+                     (const uint16_t *)dh.data_ptr(),
+                     (const uint16_t *)y.data_ptr(), (uint16_t *)dy.data_ptr(),
+                     dh.size(0), (int)dh.size(1));
+  return dy;
+}
 
 at::Tensor swiglu_fwd(at::Tensor g, at::Tensor u) {
   TORCH_CHECK(g.is_cuda() && g.is_contiguous() && u.is_contiguous(), "swiglu: args");

@@ -17,6 +17,7 @@ import os
 import torch
 from torch import nn
 
+from ..ops import _backend
 from ..parallel.tp import ColumnParallelLinear, RowParallelLinear
 
 
@@ -125,6 +126,14 @@ class _LoRAGroup:
         self._t = None
         self._left = 0
 
+    def packed(self, x):
+        """All members' results on x side by side, or None where the members
+        have to be called one by one."""
+        if any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+               or m._backward_pre_hooks for m in self.members):
+            return None
+        return _packed(self.members, x) if _packs(self.members, x) else None
+
     def t_for(self, member, x):
         if self._x_id != id(x) or self._left <= 0:
             self._t = _LoRAGroupPrep.apply(
@@ -208,6 +217,95 @@ class _LoRAFused(torch.autograd.Function):
         return dx, None, da, db, None
 
 
+class _LoRAPacked(torch.autograd.Function):
+    """y = x W^T + s (x A_i^T) B_i^T for siblings side by side (W and y by
+    columns), or for one adapter: one product with the frozen weights each way,
+    and the adapters' products on kernels that read x, y and dy once for all of
+    them (csrc/lora_group.hip)."""
+
+    @staticmethod
+    def forward(ctx, x, w, scale, n, *ab):
+        ext = _backend.ext()
+        t = ext.lora_down(x, list(ab[:n]))
+        y = x @ w.t()
+        ext.lora_add_(y, t, list(ab[n:]), scale, False)
+        ctx.save_for_backward(x, w, t, *ab)
+        ctx.scale, ctx.n = scale, n
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        ext, n = _backend.ext(), ctx.n
+        x, w, t, *ab = ctx.saved_tensors
+        As, Bs = list(ab[:n]), list(ab[n:])
+        dy = dy.contiguous()
+        widths = [b.shape[0] for b in Bs]
+        dt = ext.lora_down_columns(dy, Bs, ctx.scale)
+        db = ext.lora_grad(dy, t, widths, ctx.scale, False).split(widths)
+        da = ext.lora_grad(x, dt, [], 1.0, True).chunk(n)
+        dx = None
+        if ctx.needs_input_grad[0]:
+            dx = dy @ w
+            ext.lora_add_(dx, dt, As, 1.0, True)
+        return (dx, None, None, None, *da, *db)
+
+
+def _packs(members, x) -> bool:
+    """True when _LoRAPacked's kernels take these adapters on x, of which the
+    weights have to be side by side in memory (_lay_side_by_side)."""
+    if not x.is_cuda or x.dtype != torch.bfloat16 or x.dim() != 2 or \
+            not x.is_contiguous() or x.data_ptr() % 16 or \
+            not 0 < x.shape[0] <= 1 << 22 or _USE_CUSTOM_GEMM or \
+            len(members) > 3 or os.environ.get("RB_LORA_MFMA", "1") != "1":
+        return False
+    for m in members:
+        w = m.base.weight
+        if (m.r != 16 or m.scale != members[0].scale or
+                (m.dropout is not None and m.training) or
+                not (isinstance(m.base, nn.Linear) or
+                     getattr(m.base, "tp", 1) == 1) or
+                getattr(m.base, "bias", None) is not None or
+                w.requires_grad or w.dtype != torch.bfloat16 or
+                not w.is_contiguous() or w.shape[0] % 64 or w.shape[1] % 64 or
+                w.shape[1] != x.shape[1]):
+            return False
+        for p in (m.lora_a, m.lora_b):
+            if p.dtype != torch.bfloat16 or not p.is_contiguous() or \
+                    p.data_ptr() % 16:
+                return False
+    return _side_by_side(members) and _backend.use_hip(x)
+
+
+def _side_by_side(members) -> bool:
+    ws = [m.base.weight for m in members]
+    return all(a.untyped_storage().data_ptr() == b.untyped_storage().data_ptr()
+               and a.data_ptr() + a.numel() * a.element_size() == b.data_ptr()
+               for a, b in zip(ws, ws[1:]))
+
+
+@torch.no_grad()
+def _lay_side_by_side(members) -> None:
+    """Makes the members' frozen weights slices of one matrix."""
+    ws = [m.base.weight for m in members]
+    if not all(w.is_cuda and w.dim() == 2 and w.shape[1] == ws[0].shape[1] and
+               w.dtype == ws[0].dtype and w.device == ws[0].device and
+               w.untyped_storage().nbytes() == w.numel() * w.element_size()
+               for w in ws):
+        return
+    whole = torch.cat([w.detach() for w in ws])
+    for w, part in zip(ws, whole.split([w.shape[0] for w in ws])):
+        w.data = part
+
+
+def _packed(members, x):
+    ws = [m.base.weight for m in members]
+    rows, cols = sum(w.shape[0] for w in ws), ws[0].shape[1]
+    w = ws[0].detach().as_strided((rows, cols), (cols, 1))
+    return _LoRAPacked.apply(x, w, members[0].scale,
+                             len(members), *(m.lora_a for m in members),
+                             *(m.lora_b for m in members))
+
+
 class LoRALinear(nn.Module):
     """Wraps a (possibly TP-sharded) linear: y = base(x) + scale * B(A(x)).
 
@@ -234,6 +332,8 @@ class LoRALinear(nn.Module):
 
     def forward(self, x):
         base = self.base
+        if _packs([self], x):
+            return _packed([self], x)
         if self.dropout is not None and self.training:
             # dropout on the adapter input (PEFT semantics) breaks the
             # single-addmm fusion; let autograd handle the composite
@@ -297,6 +397,7 @@ def apply_lora(model: nn.Module, r: int = 16, alpha: int = 32,
                        (isinstance(m.base, nn.Linear)
                         or getattr(m.base, "tp", 1) == 1) and
                        getattr(m.base, "bias", None) is None for m in ms):
+                    _lay_side_by_side(ms)
                     g = _LoRAGroup(ms)
                     for m in ms:
                         m._group = g

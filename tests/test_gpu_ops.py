@@ -1072,3 +1072,89 @@ def test_fp8_vt_append_matches_plain_layout():
     d1 = kc.fp8_dequant_cache_ref(v1.cpu())           # [nb,hkv,bs,dh]
     d2 = kc.fp8_dequant_cache_ref(v2.cpu())           # [nb,hkv,dh,bs]
     assert torch.allclose(d1, d2.permute(0, 1, 3, 2), atol=1e-6)
+
+
+@pytest.mark.parametrize("T", [1, 15, 33, 129, 300])
+@pytest.mark.parametrize("K,widths", [(64, (64,)), (192, (128, 64)),
+                                      (704, (256, 64, 64))])
+def test_lora_siblings(T, K, widths):
+    """Products of rank-16 adapters side by side vs fp64: sums in fp32, one
+    rounding to bf16 (2^-9 of a value, half of that over many)."""
+    _assert_hip()
+    ext = ops.ext()
+    torch.manual_seed(T + K)
+    x, *A = (torch.randn(n, K, device=DEV).bfloat16()
+             for n in (T, *[16] * len(widths)))
+    B = [torch.randn(n, 16, device=DEV).bfloat16() for n in widths]
+    y = torch.randn(T, sum(widths), device=DEV).bfloat16()
+
+    def close(got, ref):
+        assert (got.double() - ref).norm() < 2 ** -8 * ref.norm()
+
+    xd, ys = x.double(), y.double().split(widths, 1)
+    Ad, Bd = [a.double() for a in A], [b.double() for b in B]
+    t, dt = ext.lora_down(x, A), ext.lora_down_columns(y, B, 2.0)
+    close(t, torch.stack([xd @ a.t() for a in Ad]))
+    close(dt, torch.stack([2 * v @ b for v, b in zip(ys, Bd)]))
+    td, dtd = t.double(), dt.double()
+    y2, x2 = y.clone(), x.clone()
+    ext.lora_add_(y2, t, B, 2.0, False)
+    ext.lora_add_(x2, dt, A, 1.0, True)
+    close(y2, y.double() + 2 * torch.cat([v @ b.t() for v, b in
+                                          zip(td, Bd)], 1))
+    close(x2, xd + sum(d @ a for d, a in zip(dtd, Ad)))
+    close(ext.lora_grad(y, t, list(widths), 2.0, False),
+          torch.cat([2 * v.t() @ u for v, u in zip(ys, td)]))
+    close(ext.lora_grad(x, dt, [], 1.0, True),
+          torch.cat([d.t() @ xd for d in dtd]))
+
+
+@pytest.mark.parametrize("heads,kv,dh,B,S", [(4, 4, 64, 2, 33),
+                                             (4, 1, 128, 1, 100),
+                                             (6, 2, 64, 3, 1)])
+def test_lora_siblings_train(heads, kv, dh, B, S, monkeypatch):
+    """Loss and gradients with the siblings' results side by side: no further
+    from fp32 than with every adapter by itself, up to the chance of rounding."""
+    _assert_hip()
+    from runbooks_amd.models.config import ModelConfig
+    from runbooks_amd.models.transformer import Transformer
+    from runbooks_amd.train.lora import apply_lora
+
+    cfg = ModelConfig("siblings", 256, heads * dh, 2, heads, kv, 320,
+                      max_seq_len=128, head_dim=dh)
+    tokens = torch.randint(0, 256, (B, S + 1),
+                           generator=torch.Generator().manual_seed(S))
+
+    def run(dtype, device, one_by_one=False):
+        monkeypatch.setenv("RB_LORA_MFMA", "0" if one_by_one else "1")
+        torch.manual_seed(3)
+        m = Transformer(cfg, dtype=torch.bfloat16).to(device)
+        for p in m.parameters():
+            p.data = p.data.to(dtype)
+        for p in m.parameters():
+            if p.dim() == 2:        # the same everywhere, exact in bf16
+                p.data = (p.data.float() * 4).bfloat16().to(p)
+        apply_lora(m, r=16, alpha=32)
+        g = torch.Generator().manual_seed(4)
+        for n, p in m.named_parameters():
+            if "lora" in n:
+                p.data = (torch.randn(p.shape, generator=g) * 0.05) \
+                    .bfloat16().to(p)
+        logits = m(tokens[:, :-1].to(device))
+        loss = torch.nn.functional.cross_entropy(
+            logits.float().view(-1, 256), tokens[:, 1:].reshape(-1).to(device))
+        loss.backward()
+        return [loss.detach().float().cpu().view(1)] + [
+            p.grad.float().cpu() for n, p in m.named_parameters()
+            if "lora" in n]
+
+    ref = run(torch.float32, "cpu")
+    new = run(torch.bfloat16, DEV)
+    old = run(torch.bfloat16, DEV, one_by_one=True)
+
+    def far(got):
+        return sum(((g - r).norm() / (r.norm() + 1e-6)) ** 2
+                   for g, r in zip(got[1:], ref[1:])).sqrt()
+
+    assert abs(new[0] - ref[0]) < 2e-2 * ref[0]
+    assert far(new) < 1.25 * far(old) + 1e-3

@@ -141,7 +141,7 @@ class Attention(nn.Module):
 
     def forward_prefill(self, x, cos, sin, positions, kc, vc, slot_mapping, B, S):
         if self._fused_append(x, kc):
-            y = ops.fast_linear(x, self._qkv_w)
+            y = ops.wide_linear(x, self._qkv_w)
             ops.ext().qkv_rope_append_(y, cos, sin, positions.to(torch.int32),
                                        kc, vc, slot_mapping.to(torch.int32),
                                        self.hq)
@@ -200,7 +200,7 @@ class MLP(nn.Module):
         if self.act == "silu_glu":
             if getattr(self, "_gateup_w", None) is not None and \
                     not torch.is_grad_enabled():
-                y = ops.fast_linear(x, self._gateup_w)
+                y = ops.wide_linear(x, self._gateup_w)
                 if ops.use_hip(y):
                     I = y.shape[-1] // 2
                     if (y.dtype == torch.bfloat16 and I % 16 == 0 and
@@ -226,7 +226,7 @@ class MLP(nn.Module):
             # csrc geglu_packed epilogue.
             if getattr(self, "_gateup_w", None) is not None and \
                     not torch.is_grad_enabled():
-                y = ops.fast_linear(x, self._gateup_w)
+                y = ops.wide_linear(x, self._gateup_w)
                 if ops.use_hip(y):
                     I = y.shape[-1] // 2
                     if (y.dtype == torch.bfloat16 and I % 16 == 0 and

@@ -123,6 +123,73 @@ def fast_linear(x: torch.Tensor, weight: torch.Tensor,
     return F.linear(x, weight, bias)
 
 
+def _whole_rounds(rows: int, cols: int) -> int:
+    """Columns of a library product to be computed in a call of their own, a
+    whole number of rounds of 256 x 256 tiles over the 256 CUs; the rest in a
+    second one. `cols` where one call does for all.
+
+    In one call the library leaves CUs idle in the last round, or takes a slower
+    tile; the second call has a tile for what is left. us in one call and in
+    two, inputs of 4096: 2048 rows x 22016 402 and 268, 4096 x 22016 636 and 506,
+    2816 x 6144 216 and 111, 3001 x 28672 530 and 499, 8192 x 11008 643 and 503;
+    3584 x 12288 256 and 257, 6000 x 4096 155 and 160. Up to 1280 rows it gives
+    nothing on the whole (1024 x 22016 155 and 159, 1280 x 28672 239 and 230,
+    1024 x 28672 183 and 189), nor where all tiles are whole rounds by
+    themselves (6 x 128 tiles, 155 and 164)."""
+    down, across = -(-rows // 256), -(-cols // 256)
+    if down <= 5 or down > 256 or down * across % 256 == 0:
+        return cols
+    step = 256 // down
+    return min(across // step * step * 256 or cols, cols)
+
+
+def wide_product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """x @ weight^T on the GPU for a result that is not differentiated, in
+    whole rounds of tiles."""
+    rows, cols = x.shape[0], weight.shape[0]
+    main = _whole_rounds(rows, cols)
+    if main >= cols:
+        return x @ weight.t()
+    y = x.new_empty(rows, cols)
+    torch.mm(x, weight[:main].t(), out=y[:, :main])
+    torch.mm(x, weight[main:].t(), out=y[:, main:])
+    return y
+
+
+def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """fast_linear for a result that is not differentiated; of many rows a
+    wide_product."""
+    if x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and \
+            x.shape[0] > 1280:
+        return wide_product(x, weight)
+    return fast_linear(x, weight)
+
+
+def wide_product_grad(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """dy @ weight on the GPU, weight [N, K].
+
+    Wide results in whole rounds of tiles, like wide_product's (2048 rows of
+    4096 to 11008 columns: 284 and 171 us; to 4096 and 6144 columns 3 to 14%
+    slower in two calls). Long sums with few tiles in two halves: there the
+    library keeps tiles of 256 x 256, of which there are not enough (us in one
+    sum and in two, to 4096 columns: 2048 rows of 22016 456 and 335, 512 231 and
+    196, 1024 rows of 28672 344 and 296, 2048 380 and 441; with more tiles, 2560
+    rows of 22016, 372 and 390; of 12288 and 2048 rows 195 and 213)."""
+    rows, (n, k) = dy.shape[0], weight.shape
+    if k >= 8192:
+        main = _whole_rounds(rows, k)
+        if main < k:
+            dx = dy.new_empty(rows, k)
+            torch.mm(dy, weight[:, :main], out=dx[:, :main])
+            torch.mm(dy, weight[:, main:], out=dx[:, main:])
+            return dx
+    if n > 16384 and -(-rows // 256) * -(-k // 256) <= 144:
+        half = n // 128 * 64
+        return (dy[:, :half] @ weight[:half]).addmm_(dy[:, half:],
+                                                     weight[half:])
+    return dy @ weight
+
+
 def decode_linear_raw(x, weight, f32: bool = False):
     """Decode GEMM that may return an UNCOMBINED fp32 split-K slab
     [split, M, N] (consumer kernels fold it — rmsnorm_res_slab_fwd_dec),

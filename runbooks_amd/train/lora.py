@@ -18,6 +18,7 @@ import torch
 from torch import nn
 
 from ..ops import _backend
+from ..ops.linear import wide_product, wide_product_grad
 from ..parallel.tp import ColumnParallelLinear, RowParallelLinear
 
 
@@ -227,7 +228,7 @@ class _LoRAPacked(torch.autograd.Function):
     def forward(ctx, x, w, scale, n, *ab):
         ext = _backend.ext()
         t = ext.lora_down(x, list(ab[:n]))
-        y = x @ w.t()
+        y = wide_product(x, w)
         ext.lora_add_(y, t, list(ab[n:]), scale, False)
         ctx.save_for_backward(x, w, t, *ab)
         ctx.scale, ctx.n = scale, n
@@ -245,7 +246,7 @@ class _LoRAPacked(torch.autograd.Function):
         da = ext.lora_grad(x, dt, [], 1.0, True).chunk(n)
         dx = None
         if ctx.needs_input_grad[0]:
-            dx = dy @ w
+            dx = wide_product_grad(dy, w)
             ext.lora_add_(dx, dt, As, 1.0, True)
         return (dx, None, None, None, *da, *db)
 

@@ -1158,3 +1158,21 @@ def test_lora_siblings_train(heads, kv, dh, B, S, monkeypatch):
 
     assert abs(new[0] - ref[0]) < 2e-2 * ref[0]
     assert far(new) < 1.25 * far(old) + 1e-3
+
+
+@pytest.mark.parametrize("rows,n,k", [(1281, 2816, 64), (2048, 11008, 64),
+                                      (1536, 10816, 192), (300, 192, 8192),
+                                      (129, 16448, 64), (257, 16512, 4096)])
+def test_wide_products(rows, n, k):
+    """Products in one or two calls, [rows, k] by [n, k] and back, vs fp64."""
+    from runbooks_amd.ops.linear import wide_product, wide_product_grad
+    torch.manual_seed(rows)
+    x = torch.randn(rows, k, device=DEV).bfloat16()
+    w = torch.randn(n, k, device=DEV).bfloat16()
+    y = torch.randn(rows, n, device=DEV).bfloat16()
+    for got, ref in ((wide_product(x, w), x.double() @ w.double().t()),
+                     (wide_product_grad(x, w.t().contiguous()),
+                      x.double() @ w.double().t()),
+                     (wide_product_grad(y, w), y.double() @ w.double())):
+        # one rounding of the result, or two where a sum is in halves
+        assert (got.double() - ref).norm() < 2 ** -7.5 * ref.norm()

@@ -162,7 +162,7 @@ class Attention(nn.Module):
         if self._fused_append(x, kc):
             # fused decode hot path: one wide GEMM, then one kernel doing
             # rope(q), rope(k)->cache, v->cache, quantized where the cache is
-            y = ops.fast_linear(x, self._qkv_w)
+            y = ops.wide_linear(x, self._qkv_w)
             q = ops.ext().qkv_rope_append(y, cos, sin, positions, kc, vc,
                                           slot_mapping, self.hq)
         else:

@@ -1,5 +1,6 @@
 // Decode GEMM v2 for CDNA4 (gfx950): y[M,N] = x[M,K] @ W[N,K]^T,
-// M <= 32 (decode batch), bf16 in / bf16 out, fp32 accumulate.
+// M <= 32 (decode batch; to 128 rows: decode_gemm_rows_kernel), bf16 in / bf16
+// out, fp32 accumulate.
 //
 // The M<=32 decode GEMM is >99% W traffic, so the ONLY thing that
 // matters is shaping the weight read as perfectly coalesced nontemporal
@@ -37,6 +38,8 @@
 
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -202,6 +205,167 @@ __global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
       if (s + U + u < s1) multiply(b[u]);
   }
   finish<STORE_BF16>(acc, scale, yp, slabs, M, N);
+}
+
+// 33 to 128 rows (RB blocks of 32): x is longer than W's share of a workgroup, so
+// NWN waves with blocks of 32 rows of W of their own share its tiles, in LDS, as
+// they are in memory; 4 / NWN such groups take parts of the sums. A chunk is CH
+// steps of 16 columns: W's next chunk and x's are on their way, in registers,
+// during the products of this one. Pieces of 16 bytes of a tile's row r lie
+// at their index ^ r, so that a column of 32 rows spreads over the banks.
+// Rows past M, steps past the range: the last ones again; the former are not
+// stored, the latter not multiplied.
+//
+// Bound by the weight stream (22016 x 4096 at 5 TB/s with 64 rows), with 128
+// rows by the tiles of x (3.8 TB/s). W two chunks ahead and a chunk's operands
+// of x read at once: 22016 x 4096 of 45 rows 40.6 -> 34.0 us, 4096 x 4096 15.0 ->
+// 13.5 (library 43 and 23).
+template <int RB, int NWN, int CH, bool STORE_BF16>
+__global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
+    const uint16_t *__restrict__ x, const uint8_t *__restrict__ ws,
+    uint16_t *__restrict__ yp, float *__restrict__ slabs, int M, int N, int K) {
+  constexpr int KG = 4 / NWN, P = 2 * CH;          // pieces of a row
+  constexpr int XL = RB * CH / NWN;                // of x, a lane and chunk
+  constexpr int TILE = RB * 32 * P * 16;
+  static_assert(XL * NWN == RB * CH && (KG == 1 || 2 * KG * TILE >= NWN * RB * 4096),
+                "tiles");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, hi = lane >> 5, col = lane & 31;
+  const int wn = wid % NWN, kg = wid / NWN;
+  const int blocks = N / 32, nblk = blockIdx.x * NWN + wn;
+  const int steps = K / 16, groups = gridDim.y * KG;
+  const int g = blockIdx.y * KG + kg;
+  const int s0 = (int)((int64_t)steps * g / groups);
+  const int s1 = (int)((int64_t)steps * (g + 1) / groups);
+  const int full = steps / groups / CH;            // chunks of every group
+  const int chunks = ((steps + groups - 1) / groups + CH - 1) / CH;
+  const uint8_t *wseg =
+      ws + (int64_t)min(nblk, blocks - 1) * steps * 1024 + lane * 16;
+  char *mine = smem + kg * TILE;                   // buffers KG * TILE apart
+
+  struct X { u32x4v v[XL]; };
+  struct W { u32x4v v[CH]; };
+  int64_t xrow[XL];                                // where a lane's pieces begin
+  int xstep[XL], xput[XL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int p = (i * NWN + wn) * 64 + lane, row = p / P, c = p % P;
+    xrow[i] = (int64_t)min(row, M - 1) * K + (c & 1) * 8;
+    xstep[i] = c / 2;
+    xput[i] = (row * P + (c ^ (row & (P - 1)))) * 16;
+  }
+  auto load_x = [&](X &d, int s) {
+#pragma unroll
+    for (int i = 0; i < XL; ++i)
+      d.v[i] = *reinterpret_cast<const u32x4v *>(
+          x + xrow[i] + min(s + xstep[i], s1 - 1) * 16);
+  };
+  auto load_w = [&](W &d, int s) {
+#pragma unroll
+    for (int u = 0; u < CH; ++u)
+      d.v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4v *>(
+          wseg + (int64_t)min(s + u, s1 - 1) * 1024));
+  };
+  auto put_x = [&](const X &d, char *tile) {
+#pragma unroll
+    for (int i = 0; i < XL; ++i)
+      *reinterpret_cast<u32x4v *>(tile + xput[i]) = d.v[i];
+  };
+  auto meet = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+  f32x16v acc[RB];
+#pragma unroll
+  for (int b = 0; b < RB; ++b) acc[b] = (f32x16v)(0.0f);
+  auto read = [&](bf16x8v (&xv)[RB], const char *tile, int u) {
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+      const int row = b * 32 + col, c = u * 2 + hi;
+      xv[b] = *reinterpret_cast<const bf16x8v *>(
+          tile + (row * P + (c ^ (row & (P - 1)))) * 16);
+    }
+  };
+  X xr;
+  W w0, w1;
+  load_x(xr, s0);
+  load_w(w0, s0);
+  put_x(xr, mine);
+  load_x(xr, s0 + CH);
+  load_w(w1, s0 + CH);
+  meet();
+  // chunk c, of which `w` holds W and then W of chunk c + 2
+  auto step = [&](W &w, int c, auto whole) {
+    const int s = s0 + c * CH;
+    put_x(xr, mine + (~c & 1) * KG * TILE);
+    load_x(xr, s + 2 * CH);
+    const char *tile = mine + (c & 1) * KG * TILE;
+    bf16x8v xv[CH][RB];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) read(xv[u], tile, u);
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      union { u32x4v u; bf16x8v v; } a;
+      a.u = w.v[u];
+      if (whole || s + u < s1) {
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+          acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, xv[u][b],
+                                                           acc[b], 0, 0, 0);
+      }
+      w.v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4v *>(
+          wseg + (int64_t)min(s + 2 * CH + u, s1 - 1) * 1024));
+    }
+    meet();
+  };
+  int c = 0;
+  for (; c + 2 <= full; c += 2) {
+    step(w0, c, std::true_type{});
+    step(w1, c + 1, std::true_type{});
+  }
+  for (; c < chunks; c += 2) {
+    step(w0, c, std::false_type{});
+    step(w1, c + 1, std::false_type{});
+  }
+  // sum of the groups
+  if constexpr (KG == 2) {
+    float *red = reinterpret_cast<float *>(smem) + wn * RB * 1024 + lane;
+    if (kg == 1) {
+#pragma unroll
+      for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[(b * 16 + r) * 64] = acc[b][r];
+    }
+    __syncthreads();
+    if (kg == 1) return;
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[b][r] += red[(b * 16 + r) * 64];
+  }
+  if (nblk >= blocks) return;
+#pragma unroll
+  for (int b = 0; b < RB; ++b) {
+    const int m = b * 32 + col;
+    if (m >= M) continue;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int n = nblk * 32 + 8 * q + 4 * hi;
+      if (STORE_BF16) {
+        union { uint16_t u[4]; uint64_t q; } o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o.u[j] = rb::f32_to_bf16(acc[b][4 * q + j]);
+        *reinterpret_cast<uint64_t *>(yp + (int64_t)m * N + n) = o.q;
+      } else {
+        *reinterpret_cast<float4 *>(
+            slabs + ((int64_t)blockIdx.y * M + m) * N + n) =
+            make_float4(acc[b][4 * q], acc[b][4 * q + 1], acc[b][4 * q + 2],
+                        acc[b][4 * q + 3]);
+      }
+    }
+  }
 }
 
 // slabs [SPLIT, M, N] f32 -> y [M, N] bf16
@@ -413,5 +577,65 @@ at::Tensor decode_gemm_fp8(at::Tensor xs, at::Tensor w8s, at::Tensor scale,
                K);
   if (raw) return slabs;
   combine(slabs, y);
+  return y;
+}
+
+template <int RB, int NWN, int CH>
+static void launch_rows(const at::Tensor &x, const at::Tensor &ws, at::Tensor &y,
+                        int split) {
+  const int64_t M = x.size(0), K = x.size(1), N = y.size(1);
+  constexpr int lds = 2 * (4 / NWN) * RB * 32 * CH * 32;
+  static_assert(lds <= 64 * 1024, "tiles");
+  TORCH_CHECK(split >= 1 && split * (4 / NWN) <= K / 16, "decode_gemm_rows");
+  const dim3 grid((unsigned)((N / 32 + NWN - 1) / NWN), (unsigned)split);
+  auto go = [&](auto kernel, float *slabs) {
+    hipLaunchKernelGGL(kernel, grid, dim3(BLOCK), lds,
+                       at::cuda::getCurrentHIPStream(),
+                       (const uint16_t *)x.data_ptr(),
+                       (const uint8_t *)ws.data_ptr(),
+                       (uint16_t *)y.data_ptr(), slabs, (int)M, (int)N, (int)K);
+  };
+  if (split == 1) {
+    go(decode_gemm_rows_kernel<RB, NWN, CH, true>, nullptr);
+    return;
+  }
+  auto slabs = at::empty({split, M, N}, x.options().dtype(at::kFloat));
+  go(decode_gemm_rows_kernel<RB, NWN, CH, false>, slabs.data_ptr<float>());
+  combine(slabs, y);
+}
+
+// y [M, N] = x [M, K] W^T of 1 to 128 rows; ws from decode_swizzle_w.
+//
+// One workgroup for every CU where it can be had, as a second on some of them
+// has the others wait: four blocks of W for wide weights, unsplit; else two, or
+// four for long rows, of which splits to fill the CUs cost less (us with two
+// and four at their best split: 4096 x 11008 of 64 rows 25 and 26, of 100 rows
+// 32 and 30; 3072 x 24576 38 and 34, 50 and 41; 4096 x 4096 14 and 16, 17 and
+// 20; 22016 x 4096 of 64 rows 45 and 36, 12288 x 4096 25 and 26).
+at::Tensor decode_gemm_rows(at::Tensor x, at::Tensor ws, int64_t N) {
+  TORCH_CHECK(x.is_cuda() && ws.is_cuda() && x.dim() == 2 &&
+              x.is_contiguous() && ws.is_contiguous() &&
+              x.scalar_type() == at::kBFloat16 &&
+              ws.scalar_type() == at::kBFloat16 &&
+              reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
+              "decode_gemm_rows: inputs");
+  const int64_t M = x.size(0), K = x.size(1);
+  TORCH_CHECK(M >= 1 && M <= 128 && N > 0 && N % 32 == 0 && K % 16 == 0 &&
+              K >= 1024 && K < (1 << 24) && ws.numel() == N * K,
+              "decode_gemm_rows: shape");
+  auto y = at::empty({M, N}, x.options());
+  const bool four = N >= 20480 || K >= (M <= 64 ? 20480 : 8192);
+  const int64_t wgs = (N / 32 + (four ? 3 : 1)) / (four ? 4 : 2);
+  int split = 1;
+  while (split < 8 && wgs * split * 2 <= 256 && K / (split * 2) >= 256)
+    split *= 2;
+  auto go = [&](auto rb) {
+    constexpr int RB = decltype(rb)::value;
+    if (four) launch_rows<RB, 4, RB == 4 ? 4 : 8>(x, ws, y, split);
+    else launch_rows<RB, 2, 4>(x, ws, y, split);
+  };
+  if (M <= 32) go(std::integral_constant<int, 1>{});
+  else if (M <= 64) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 4>{});
   return y;
 }

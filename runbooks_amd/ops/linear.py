@@ -1,7 +1,7 @@
 """Linear dispatch: route decode-shaped matmuls to the skinny GEMM.
 
-Batch-<=32 single-token decode GEMMs are weight-bandwidth bound;
-csrc/skinny_gemm.hip streams W at HBM rate where hipBLASLt's tiles
+Decode GEMMs and others of up to 128 rows are weight-bandwidth bound;
+csrc/decode_gemm.hip streams W at HBM rate where hipBLASLt's tiles
 measured 25-45% (profiles/). Everything else (prefill, training) stays
 on hipBLASLt via F.linear — the library is the right tool for big GEMMs.
 """
@@ -31,7 +31,8 @@ _FP8_REGISTRY: dict[int, tuple[torch.Tensor, torch.Tensor]] = {}
 # consumed by csrc/decode_gemm.hip. A second full-precision weight copy:
 # 288 GB HBM3E per GPU makes layout-specialized decode weights the right
 # trade on MI355X (prefill/training keep the original [N,K] tensor).
-# value: (swizzled copy, (N, K), weakref to the registered tensor).
+# value: (swizzled copy, (N, K), the weight's version, weakref to the registered
+# tensor).
 # data_ptr alone is NOT a safe key — a freed weight's address gets
 # recycled by later allocations, so every lookup verifies tensor
 # identity through the weakref (stale entries are dropped lazily).
@@ -48,13 +49,17 @@ def _registry_get(reg: dict, weight: torch.Tensor):
     return entry
 
 
+def _version(weight: torch.Tensor):
+    return None if weight.is_inference() else weight._version
+
+
 def register_decode_weight(weight: torch.Tensor) -> None:
     """Build + register the decode-GEMM weight layout for `weight`."""
     for ptr in [p for p, e in _DECODE_W_REGISTRY.items() if e[-1]() is None]:
         del _DECODE_W_REGISTRY[ptr]          # purge dead entries
     ws = _backend.ext().decode_swizzle_w(weight.data)
     _DECODE_W_REGISTRY[weight.data_ptr()] = (
-        ws, (int(weight.shape[0]), int(weight.shape[1])),
+        ws, (int(weight.shape[0]), int(weight.shape[1])), _version(weight),
         weakref.ref(weight))
 
 E4M3_MAX = 448.0
@@ -120,7 +125,29 @@ def fast_linear(x: torch.Tensor, weight: torch.Tensor,
                 y = _backend.ext().skinny_gemm(x.reshape(m, k).contiguous(),
                                                weight)
                 return y.view(*x.shape[:-1], n)
+        elif m <= 128:
+            y = _rows_linear(x, weight, m, n, k)
+            if y is not None:
+                return y
     return F.linear(x, weight, bias)
+
+
+def _rows_linear(x: torch.Tensor, weight: torch.Tensor, m: int, n: int,
+                 k: int) -> torch.Tensor | None:
+    """x @ weight^T of up to 128 rows on the decode GEMM that reads x as it is,
+    or None where the weight has no decode layout (or has changed since).
+
+    us on the library and there: 64 rows, 22016 x 4096 44.4 and 35.8, 4096 x
+    4096 23.0 and 14.1, 4096 x 14336 40.4 and 27.3, 3072 x 24576 102 and 34; 128
+    rows, 46.5 and 46.9, 26.9 and 17.6, 76.9 and 32.5, 133 and 43."""
+    if not _USE_DECODE_GEMM or n % 32 or k % 16 or k < 1024 or \
+            not x.is_contiguous() or x.data_ptr() % 16:
+        return None
+    dw = _registry_get(_DECODE_W_REGISTRY, weight)
+    if dw is None or dw[2] != _version(weight):
+        return None
+    y = _backend.ext().decode_gemm_rows(x.view(m, k), dw[0], n)
+    return y.view(*x.shape[:-1], n)
 
 
 def _whole_rounds(rows: int, cols: int) -> int:
@@ -157,11 +184,22 @@ def wide_product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 
 def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """fast_linear for a result that is not differentiated; of many rows a
-    wide_product."""
-    if x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and \
-            x.shape[0] > 1280:
-        return wide_product(x, weight)
+    """fast_linear for a result that is not differentiated, of rows x that are
+    there also where they have a decode operand; of many rows a wide_product.
+
+    From 17 to 32 rows the kernel that shares x is the faster one where it has
+    about one workgroup for every CU (us without and with it, 32 rows: 22016 x
+    4096 34.9 and 31.2, 12288 x 4096 23.2 and 21.7; 49152 x 3072 52.7 and 53.0,
+    6144 x 4096 15.9 and 15.4, of 24 rows 47.9 and 52.6, 14.7 and 15.0)."""
+    if x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2:
+        (m, k), n = x.shape, weight.shape[0]
+        if m > 1280:
+            return wide_product(x, weight)
+        if 16 < m <= 32 and 10240 <= n <= 32768 and \
+                _registry_get(_FP8_REGISTRY, weight) is None:
+            y = _rows_linear(x, weight, m, n, k)
+            if y is not None:
+                return y
     return fast_linear(x, weight)
 
 

@@ -1176,3 +1176,31 @@ def test_wide_products(rows, n, k):
                      (wide_product_grad(y, w), y.double() @ w.double())):
         # one rounding of the result, or two where a sum is in halves
         assert (got.double() - ref).norm() < 2 ** -7.5 * ref.norm()
+
+
+@pytest.mark.parametrize("M", [1, 32, 33, 64, 65, 128])
+@pytest.mark.parametrize("N,K", [(32, 1024), (96, 1040), (20512, 1024),
+                                 (160, 8208), (4096, 4096)])
+def test_decode_gemm_rows(M, N, K):
+    """Rows as they are by a weight in the decode layout vs fp64: one rounding
+    of the result."""
+    _assert_hip()
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device=DEV).bfloat16()
+    w = torch.randn(N, K, device=DEV).bfloat16()
+    y = ops.ext().decode_gemm_rows(x, ops.ext().decode_swizzle_w(w), N)
+    ref = x.double() @ w.double().t()
+    assert (y.double() - ref).norm() < 2 ** -8 * ref.norm()
+
+
+def test_decode_gemm_rows_of_changed_weight():
+    """Products of 33 to 128 rows follow a weight that changes in place."""
+    from runbooks_amd.ops.linear import fast_linear, register_decode_weight
+    w = torch.randn(64, 1024, device=DEV).bfloat16()
+    x = torch.randn(40, 1024, device=DEV).bfloat16()
+    register_decode_weight(w)
+    with torch.no_grad():
+        before = fast_linear(x, w)
+        w.mul_(2)
+        after = fast_linear(x, w)
+    assert (after - 2 * before).norm() < 2 ** -7 * after.norm()

@@ -508,6 +508,19 @@ static void combine(const at::Tensor &slabs, at::Tensor &y) {
                      (int)slabs.size(0), y.numel());
 }
 
+// Sum of fp32 parts [P, M, N], rounded to bf16.
+at::Tensor sum_parts(at::Tensor parts) {
+  TORCH_CHECK(parts.is_cuda() && parts.dim() == 3 && parts.is_contiguous() &&
+              parts.scalar_type() == at::kFloat && parts.size(2) % 4 == 0 &&
+              parts.size(0) > 0 &&
+              reinterpret_cast<uintptr_t>(parts.data_ptr()) % 16 == 0,
+              "sum_parts: fp32 [P, M, 4 n]");
+  auto y = at::empty({parts.size(1), parts.size(2)},
+                     parts.options().dtype(at::kBFloat16));
+  if (y.numel() > 0) combine(parts, y);
+  return y;
+}
+
 at::Tensor decode_gemm_raw(at::Tensor xs, at::Tensor ws, int64_t M,
                            int64_t N, int64_t K, bool f32) {
   TORCH_CHECK(xs.is_cuda() && ws.is_cuda() && xs.is_contiguous() &&

@@ -129,6 +129,13 @@ def fast_linear(x: torch.Tensor, weight: torch.Tensor,
             y = _rows_linear(x, weight, m, n, k)
             if y is not None:
                 return y
+        if (m > 32 and k > _LONG_ROW and n % 4 == 0 and x.dim() == 2 and
+                -(-m // 256) * -(-n // 256) <= 144):
+            # with few tiles the library is slow at such sums, as in
+            # linear_f32_parts (us in one and in two, 3072 x 24576: 512 rows
+            # 274 and 155, 1021 274 and 210, 3001 666 and 405; 5000 rows, 240
+            # tiles, 541 in one)
+            return _backend.ext().sum_parts(linear_f32_parts(x, weight))
     return F.linear(x, weight, bias)
 
 

@@ -1204,3 +1204,16 @@ def test_decode_gemm_rows_of_changed_weight():
         w.mul_(2)
         after = fast_linear(x, w)
     assert (after - 2 * before).norm() < 2 ** -7 * after.norm()
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 64, 16448), (700, 260, 24576)])
+def test_long_rows(m, n, k):
+    """Sums in two fp32 parts: one rounding of the result, as in one."""
+    from runbooks_amd.ops.linear import fast_linear
+    torch.manual_seed(m)
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    w = torch.randn(n, k, device=DEV).bfloat16()
+    with torch.no_grad():
+        y = fast_linear(x, w)
+    ref = x.double() @ w.double().t()
+    assert (y.double() - ref).norm() < 2 ** -8 * ref.norm()

@@ -18,7 +18,7 @@
 //   lora_add (columns) 26, 18      53, 42
 //   lora_down_columns  70, 13      57, 26
 //   dB                 76, 15      51, 27
-//   dA                 20, 20      20, 18
+//   dA                 20, 14      20, 13
 //   lora_add (sum)     18, 8       18, 8
 // and no additions of dx, copies of t or transposes of A around them.
 //
@@ -488,10 +488,12 @@ at::Tensor lora_grad(at::Tensor x, at::Tensor t, std::vector<int64_t> widths,
   }
   const int64_t wide = transposed ? a.n * R : R;
   const int64_t tiles = C / 64;
-  // shares of the rows until there are four workgroups for every CU, of at
-  // least 128 rows each
+  // shares of the rows, of at least 128 each, until there are as many workgroups
+  // as the CUs' LDS holds (dA of 2048 x 4096, three siblings: 20 us with twice
+  // as many, 14 so)
+  const int64_t want = transposed ? 512 : 1024;
   const int64_t shares = std::max<int64_t>(
-      1, std::min<int64_t>((T + 127) / 128, (1024 + tiles - 1) / tiles));
+      1, std::min<int64_t>((T + 127) / 128, (want + tiles - 1) / tiles));
   auto parts = at::empty({shares, C * wide}, x.options().dtype(at::kFloat));
   auto out = transposed ? at::empty({wide, C}, x.options())
                         : at::empty({C, wide}, x.options());

@@ -6,10 +6,10 @@ GPU), so a ring all-reduce is bound by ONE link. Buckets default to 64 MiB
 buckets are in flight while backward is still producing grads, keeping
 all 7 links busy via RCCL's fully-connected topology.
 
-Mechanics: a post-accumulate-grad hook moves each finished ``.grad``
-into its slot of a pre-allocated flat bucket buffer (autograd would
-replace a pre-seeded grad view out-of-place, so the copy is explicit);
-the moment a bucket is complete its async all-reduce launches (RCCL's
+Mechanics: a post-accumulate-grad hook takes each finished ``.grad``, and
+several together are added into their slots of a pre-allocated flat bucket
+buffer (autograd would replace a pre-seeded grad view out-of-place, so the
+copy is explicit); the moment a bucket is complete its async all-reduce launches (RCCL's
 internal stream) while backward keeps producing the next bucket.
 ``finish_backward()`` waits, averages, and points every ``.grad`` at its
 reduced bucket slice for the optimizer.
@@ -36,6 +36,25 @@ class _Bucket:
             off += p.numel()
         self.pending = 0
         self.work = None
+        self.arrived = []           # (slot, gradient) not yet in the buffer
+        self.arrived_on = None      # the stream that they arrived on
+        self.arrived_bytes = 0
+
+    def flush(self):
+        """Accumulates what has arrived into the flat buffer, on the stream that
+        it arrived on; the current one waits for that."""
+        if not self.arrived:
+            return
+        slots, grads = zip(*self.arrived)
+        self.arrived, self.arrived_bytes = [], 0
+        views = [self.views[i] for i in slots]
+        there = self.arrived_on
+        if there is None or there == torch.cuda.current_stream(there.device):
+            torch._foreach_add_(views, list(grads))
+            return
+        with torch.cuda.stream(there):
+            torch._foreach_add_(views, list(grads))
+        torch.cuda.current_stream(there.device).wait_stream(there)
 
 
 class DataParallel(nn.Module):
@@ -96,13 +115,25 @@ class DataParallel(nn.Module):
             b.work = None
 
     # -- backward-side hooks ---------------------------------------------------
+    # Gradients of a bucket go into the buffer together, in one launch: the 448
+    # adapters of a 7B model took as many of 4 us each, 1.8 ms of a step of 71.
+    # As many bytes are held up at most.
+    _HELD = 8 << 20
+
     def _on_grad(self, p: torch.nn.Parameter):
         b, i = self._param_bucket[id(p)]
         # accumulate into the flat buffer and release the autograd tensor;
         # micro-batch accumulation keeps adding into the same slot.
-        b.views[i].add_(p.grad)
+        stream = torch.cuda.current_stream(p.device) if p.is_cuda else None
+        if stream != b.arrived_on or any(i == j for j, _ in b.arrived):
+            b.flush()
+            b.arrived_on = stream
+        b.arrived.append((i, p.grad))
+        b.arrived_bytes += p.grad.numel() * p.grad.element_size()
         p.grad = None
         b.pending -= 1
+        if b.pending == 0 or b.arrived_bytes >= self._HELD:
+            b.flush()
         if b.pending == 0 and comm.is_dist() and self.sync:
             b.work = dist.all_reduce(b.buffer, op=dist.ReduceOp.SUM, async_op=True)
 
@@ -111,6 +142,8 @@ class DataParallel(nn.Module):
         into the flat buckets without reducing (grad-accumulation
         micro-batches); the last micro-batch passes sync=True."""
         self.sync = sync
+        for b in self._buckets:
+            b.flush()
         self._reset_pending()
 
     def finish_backward(self):
@@ -118,6 +151,7 @@ class DataParallel(nn.Module):
         Call after backward()."""
         ws = comm.world_size()
         for b in self._buckets:
+            b.flush()
             if b.work is not None:
                 b.work.wait()
             if ws > 1:
@@ -127,10 +161,13 @@ class DataParallel(nn.Module):
         self._reset_pending()
 
     def grad_buffers(self):
+        for b in self._buckets:
+            b.flush()
         return [b.buffer for b in self._buckets]
 
     def zero_grad(self, set_to_none: bool = False):  # noqa: ARG002
         for b in self._buckets:
+            b.arrived, b.arrived_bytes = [], 0
             b.buffer.zero_()
             for p in b.params:
                 p.grad = None   # next backward must produce a fresh tensor

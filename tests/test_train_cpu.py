@@ -353,3 +353,35 @@ def test_grad_checkpointing_with_lora_groups():
     assert g0.keys() == g1.keys() and len(g0) > 0
     for n in g0:
         assert torch.equal(g0[n], g1[n]), n
+
+
+def test_gradients_arrive_together(monkeypatch):
+    """Flat buckets hold the plain gradients whether they are flushed one by
+    one, in groups or at the end (a parameter without a gradient keeps its
+    bucket open), over accumulated micro-batches."""
+    from runbooks_amd.parallel import DataParallel
+
+    for held in (1, 200, 1 << 20):
+        monkeypatch.setattr(DataParallel, "_HELD", held)
+        torch.manual_seed(0)
+        net = torch.nn.Sequential(*(torch.nn.Linear(4, 4) for _ in range(5)))
+        net.unused = torch.nn.Parameter(torch.ones(3))
+        ddp = DataParallel(net)
+        xs = torch.randn(2, 6, 4)
+        ref = torch.autograd.grad(
+            sum(torch.nn.Sequential(*list(net.children()))(x).pow(2).sum()
+                for x in xs), [p for p in net.children() for p in
+                               p.parameters()])
+        for i, x in enumerate(xs):
+            ddp.start_microbatch(sync=i == 1)
+            y = x
+            for layer in net.children():
+                y = layer(y)
+            y.pow(2).sum().backward()
+        ddp.finish_backward()
+        for p, r in zip((p for m in net.children() for p in m.parameters()),
+                        ref):
+            assert torch.allclose(p.grad, r, rtol=1e-5, atol=1e-6)
+        assert torch.equal(net.unused.grad, torch.zeros(3))
+        ddp.zero_grad()
+        assert all(not b.any() for b in ddp.grad_buffers())

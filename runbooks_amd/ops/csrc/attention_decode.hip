@@ -48,6 +48,22 @@ RB_DEV float rb_dot2(unsigned a, unsigned b, float c) {
   return __builtin_amdgcn_fdot2_f32_bf16(x.v, y.v, c, false);
 }
 
+// VE outputs of sequence b from column kk0 of a row (a multiple of VE, as VE is
+// of 4) in the decode GEMM's operand layout, [K/16][2][32][8].
+template <int VE>
+RB_DEV void store_operand(uint16_t *swz, int kk0, int b, const float (&v)[VE],
+                          float scale) {
+  constexpr int W = VE < 8 ? VE : 8;
+#pragma unroll
+  for (int e0 = 0; e0 < VE; e0 += W) {
+    const int kk = kk0 + e0;
+    uint16_t *p =
+        swz + (kk >> 4) * 512 + ((kk >> 3) & 1) * 256 + b * 8 + (kk & 7);
+#pragma unroll
+    for (int e = 0; e < W; ++e) p[e] = rb::f32_to_bf16(v[e0 + e] * scale);
+  }
+}
+
 // The sequence of a workgroup. Workgroups 256 apart in launch order share a CU;
 // in plain order those would be heads of one sequence wherever the batch divides
 // 256, and the CUs of the longest ones would run long after the others. The
@@ -347,17 +363,8 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
 #pragma unroll
           for (int e = 0; e < VE; ++e)
             op[e] = rb::f32_to_bf16(acc[g][e] * inv_l);
-          if (VE >= 8 && out_swz != nullptr) {
-#pragma unroll
-            for (int e8 = 0; e8 < VE; e8 += 8) {
-              const int kk = h * DH + d0 + e8;
-              uint16_t *sp = out_swz + (kk >> 4) * 512 +
-                             ((kk >> 3) & 1) * 256 + b * 8;
-#pragma unroll
-              for (int e = 0; e < 8 && e < VE; ++e)
-                sp[e] = rb::f32_to_bf16(acc[g][e8 + e] * inv_l);
-            }
-          }
+          if (out_swz != nullptr)
+            store_operand<VE>(out_swz, h * DH + d0, b, acc[g], inv_l);
         }
       }
     }
@@ -405,20 +412,8 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
       uint16_t *op = out + ((int64_t)b * Hq + hq0 + g) * DH + d0;
 #pragma unroll
       for (int e = 0; e < VE; ++e) op[e] = rb::f32_to_bf16(av[e] * inv_l);
-      if (out_swz != nullptr) {
-        // also emit the decode-GEMM operand layout for o_proj
-        // ([K/16][2][32][8] over K = Hq*DH, m = b): saves the standalone
-        // decode_swizzle_x launch per layer. VE >= 8, d0 8-aligned.
-#pragma unroll
-        for (int e8 = 0; e8 < VE; e8 += 8) {
-          const int kk = (hq0 + g) * DH + d0 + e8;
-          uint16_t *sp = out_swz + (kk >> 4) * 512 + ((kk >> 3) & 1) * 256 +
-                         b * 8;
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            sp[e] = rb::f32_to_bf16(av[e8 + e] * inv_l);
-        }
-      }
+      if (out_swz != nullptr)
+        store_operand<VE>(out_swz, (hq0 + g) * DH + d0, b, av, inv_l);
     }
   }
 }
@@ -776,17 +771,8 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
       uint16_t *op = out + ((int64_t)b * Hq + hq0 + g) * DH + d0;
 #pragma unroll
       for (int e = 0; e < VE; ++e) op[e] = rb::f32_to_bf16(av[e] * inv_l);
-      if (VE >= 8 && out_swz != nullptr) {
-#pragma unroll
-        for (int e8 = 0; e8 < VE; e8 += 8) {
-          const int kk = (hq0 + g) * DH + d0 + e8;
-          uint16_t *sp = out_swz + (kk >> 4) * 512 + ((kk >> 3) & 1) * 256 +
-                         b * 8;
-#pragma unroll
-          for (int e = 0; e < 8 && e < VE; ++e)
-            sp[e] = rb::f32_to_bf16(av[e8 + e] * inv_l);
-        }
-      }
+      if (out_swz != nullptr)
+        store_operand<VE>(out_swz, (hq0 + g) * DH + d0, b, av, inv_l);
     }
   }
 }

@@ -1217,3 +1217,26 @@ def test_long_rows(m, n, k):
         y = fast_linear(x, w)
     ref = x.double() @ w.double().t()
     assert (y.double() - ref).norm() < 2 ** -8 * ref.norm()
+
+
+
+@pytest.mark.parametrize("hq,hkv,dh,vt", [(3, 3, 64, False), (16, 4, 64, False),
+                                          (16, 1, 64, False), (8, 2, 128, False),
+                                          (8, 2, 64, True), (4, 4, 256, False)])
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_paged_decode_operand(hq, hkv, dh, vt, nsplit):
+    """The operand that goes with the result holds the same values, whatever a
+    lane's share of a head."""
+    _assert_hip()
+    from runbooks_amd.ops import kvcache as kc
+    torch.manual_seed(hq + dh)
+    B = 5
+    k, v = kc.alloc_kv_cache(B * 4, hkv, dh, DEV, v_transposed=vt)
+    k.normal_()
+    v.normal_()
+    q = torch.randn(B, hq, dh, dtype=torch.bfloat16, device=DEV)
+    bt = torch.arange(B * 4, dtype=torch.int32, device=DEV).view(B, 4)
+    sl = torch.tensor([64, 1, 17, 33, 50], dtype=torch.int32, device=DEV)
+    out, swz = ops.paged_decode_with_operand(q, k, v, bt, sl, nsplit=nsplit)
+    rows = swz.view(-1, 2, 32, 8)[:, :, :B].permute(2, 0, 1, 3)
+    assert torch.equal(rows.reshape(B, hq * dh), out.view(B, hq * dh))

@@ -541,6 +541,12 @@ class Transformer(nn.Module):
             logits = self.lm_head(y)
             return (gather_from_tp(logits) if self._lm_vocab_parallel
                     else logits)
+        if ops.use_hip(x) and B <= 32 and self._affine_ready():
+            x = self._decode_affine(x, caches, slot_mapping, block_tables,
+                                    seq_lens, nsplit, seq_starts)
+            logits = self.lm_head(x)
+            return (gather_from_tp(logits) if self._lm_vocab_parallel
+                    else logits)
         cache_of = dict(zip(self.blocks, caches))
 
         def attention(blk):
@@ -553,6 +559,35 @@ class Transformer(nn.Module):
         x = self._last_norm(*self._blocks(x, attention))
         logits = self.lm_head(x)
         return gather_from_tp(logits) if self._lm_vocab_parallel else logits
+
+    def _affine_ready(self) -> bool:
+        """Every block has its products for _decode_affine, of weights that have
+        not changed since."""
+        return (os.environ.get("RB_FUSED_RESID", "1") == "1" and
+                all(getattr(blk, "_affine", None) is not None and
+                    blk._affine.current() for blk in self.blocks))
+
+    def _decode_affine(self, x, caches, slot_mapping, block_tables, seq_lens,
+                       nsplit, seq_starts):
+        """Decode of layer-norm models with biases (opt, gpt2): nine launches a
+        layer, the residual in fp32. Returns the last norm's result."""
+        res, delta = x.float(), None
+        for blk, (kc, vc) in zip(self.blocks, caches):
+            h = ops.norm_res32(blk.norm1, res, delta, x.dtype, operand=True)
+            q, k, v = blk._affine.qkv(h._rb_swz, h.shape[0])
+            attn = blk.attn
+            q = q.view(-1, attn.hq, attn.dh)
+            ops.kv_append(k.view(-1, attn.hkv, attn.dh),
+                          v.view(-1, attn.hkv, attn.dh), kc, vc, slot_mapping)
+            o, swz = ops.paged_decode_with_operand(
+                q, kc, vc, block_tables, seq_lens, scale=attn.scale,
+                nsplit=nsplit, seq_starts=seq_starts)
+            delta = blk._affine.o(swz, h.shape[0])
+            h = ops.norm_res32(blk.norm2, res, delta, x.dtype, operand=True)
+            delta = blk._affine.mlp(h._rb_swz, h.shape[0])
+        return ops.norm_res32(
+            self.norm_f, res, delta, x.dtype,
+            operand=ops.decode_ready(self.lm_head.weight, res.shape[0]))
 
     @torch.no_grad()
     def forward_ragged(self, batch: RaggedBatch, caches):
@@ -699,6 +734,65 @@ class Transformer(nn.Module):
                 for _ in range(self.cfg.num_layers)]
 
 
+class _AffineBlock:
+    """A block's products with their biases and activation in the decode GEMM's
+    layout (csrc/decode_gemm.hip, decode_affine)."""
+
+    ACTS = {"relu": 1, "gelu": 2, "gelu_tanh": 3}
+
+    @staticmethod
+    def serves(model, blk) -> bool:
+        cfg, a, m = model.cfg, blk.attn, blk.mlp
+        return (cfg.norm == "layernorm" and cfg.pos == "learned" and
+                cfg.act in _AffineBlock.ACTS and not cfg.parallel_residual and
+                not cfg.single_norm and model.tp == 1 and
+                cfg.hidden_size % 32 == 0 and cfg.hidden_size <= 16384 and
+                m.fc1.weight.shape[0] % 32 == 0 and
+                a.hq * a.dh % 32 == 0 and a.hkv * a.dh % 32 == 0 and
+                all(n.weight is not None and n.bias is not None
+                    for n in (blk.norm1, blk.norm2, model.norm_f)))
+
+    def __init__(self, blk, act: str):
+        a, m = blk.attn, blk.mlp
+        qkv = (a.q_proj, a.k_proj, a.v_proj)
+        self.act = self.ACTS[act]
+        self.widths = [p.weight.shape[0] for p in qkv]
+        self.sources = [t for p in (*qkv, a.o_proj, m.fc1, m.down_proj)
+                        for t in (p.weight, p.bias) if t is not None]
+        self.versions = self._versions()
+        swizzle = ops.ext().decode_swizzle_w
+        bias = [p.bias for p in qkv]
+        self.qkv_w = swizzle(torch.cat([p.weight.data for p in qkv]))
+        self.qkv_b = None if bias[0] is None else torch.cat(
+            [b.data for b in bias])
+        self.rest = [(swizzle(p.weight.data), p.weight.shape[0],
+                      p.weight.shape[1], p.bias)
+                     for p in (a.o_proj, m.fc1, m.down_proj)]
+        self.k = a.q_proj.weight.shape[1]
+
+    def _versions(self):
+        return [(t.data_ptr(), None if t.is_inference() else t._version)
+                for t in self.sources]
+
+    def current(self) -> bool:
+        return self._versions() == self.versions
+
+    def qkv(self, swz, rows: int):
+        return ops.ext().decode_affine(swz, self.qkv_w, self.qkv_b, rows,
+                                       self.k, self.widths)
+
+    def _one(self, i: int, swz, rows: int, act: int = 0, operand=False):
+        w, n, k, b = self.rest[i]
+        return ops.ext().decode_affine(swz, w, b, rows, k, [n], act,
+                                       operand)[0]
+
+    def o(self, swz, rows: int):
+        return self._one(0, swz, rows)
+
+    def mlp(self, swz, rows: int):
+        return self._one(2, self._one(1, swz, rows, self.act, True), rows)
+
+
 def _fuse_projections(model: "Transformer") -> list[torch.Tensor]:
     """Fused qkv and gate/up weights; returns every layer's serving
     weights."""
@@ -775,10 +869,16 @@ def fuse_for_inference(model: "Transformer",
                                           model.lm_head.weight.shape[1]):
             cands.append(model.lm_head.weight)
         need = sum(2 * w.numel() for w in cands)
+        affine = [] if model.ragged else [
+            blk for blk in model.blocks if model.lm_head.weight.is_cuda and
+            _AffineBlock.serves(model, blk)]
+        need += sum(2 * p.numel() for blk in affine for p in blk.parameters())
         free, total = torch.cuda.mem_get_info()
         if free - need >= int(0.35 * total):
             for w in cands:
                 register_decode_weight(w)
+            for blk in affine:
+                blk._affine = _AffineBlock(blk, model.cfg.act)
 
     if load_in_8bit and torch.cuda.is_available():
         # MODEL_LOAD_IN_8BIT: decode weights additionally stored as OCP

@@ -143,11 +143,10 @@ template <bool FP8> struct Step {
 //         1 row    31.9 -> 13.8  47.3 -> 20.1  17.7 -> 6.3  39.5 -> 12.4
 //         16 rows  32.5 -> 14.1  49.3 -> 20.8  17.7 -> 6.5  37.7 -> 12.8
 //         32 rows  34.7 -> 17.7  56.5 -> 26.4  18.1 -> 7.7  38.1 -> 16.0
-template <bool FP8, bool STORE_BF16>
-__global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
-    const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws,
-    const float *__restrict__ scale, uint16_t *__restrict__ yp,
-    float *__restrict__ slabs, int M, int N, int K) {
+template <bool FP8>
+__device__ __forceinline__ f32x16v weight_stream(
+    const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws, int M,
+    int K) {
   constexpr int X = Step<FP8>::X, U = FP8 ? 4 : 8;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -204,7 +203,71 @@ __global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
     for (int u = 0; u < U; ++u)
       if (s + U + u < s1) multiply(b[u]);
   }
+  return acc;
+}
+
+template <bool FP8, bool STORE_BF16>
+__global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
+    const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws,
+    const float *__restrict__ scale, uint16_t *__restrict__ yp,
+    float *__restrict__ slabs, int M, int N, int K) {
+  const f32x16v acc = weight_stream<FP8>(xs, ws, M, K);
   finish<STORE_BF16>(acc, scale, yp, slabs, M, N);
+}
+
+// act(x W^T + bias) of small models, whose decode is bound by its launches: the
+// columns go to up to three matrices (q, k, v), or to the operand of the next
+// product. us for 1 row, in launches of their own and here: q, k, v of 768 x
+// 768 27 and 5, 3072 x 768 with its activation 13 and 5, 768 x 3072 18 and 7.
+struct Affine {
+  const uint16_t *bias;                 // or null
+  uint16_t *out[3];
+  int end[3];                           // columns before the next matrix
+  int act;                              // 0 none, 1 relu, 2 gelu, 3 gelu_tanh
+  bool operand;                         // out[0] as [N/16][2][32][8]
+};
+
+__device__ __forceinline__ float activate(float x, int act) {
+  if (act == 1) return x < 0.0f ? 0.0f : x;
+  if (act == 2) return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f));
+  if (act == 3)
+    return 0.5f * x * (1.0f + tanhf(0.79788456080286536f *
+                                    (x + 0.044715f * x * x * x)));
+  return x;
+}
+
+__global__ __launch_bounds__(BLOCK, 1) void decode_affine_kernel(
+    const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws, Affine a,
+    int M, int K) {
+  const f32x16v acc = weight_stream<false>(xs, ws, M, K);
+  const int tid = threadIdx.x, wid = tid >> 6;
+  const int hi = (tid & 63) >> 5, col = tid & 31;
+  __shared__ __attribute__((aligned(16))) float red[4][32][MMAX];
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    red[wid][(r & 3) + 8 * (r >> 2) + 4 * hi][col] = acc[r];
+  __syncthreads();
+  const int m = tid >> 3, en = (tid & 7) * 4;
+  if (m >= M) return;
+  const int n = blockIdx.x * 32 + en;
+  union { uint16_t u[4]; uint64_t q; } o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float f = red[0][en + j][m] + red[1][en + j][m] + red[2][en + j][m] +
+              red[3][en + j][m];
+    if (a.bias != nullptr) f += rb::bf16_to_f32(a.bias[n + j]);
+    o.u[j] = rb::f32_to_bf16(activate(f, a.act));
+  }
+  uint16_t *dst;
+  if (a.operand) {
+    dst = a.out[0] + (n >> 4) * 512 + (n >> 3 & 1) * 256 + m * 8 + (n & 7);
+  } else {
+    // ends are multiples of 32, like a workgroup's columns
+    const int i = n < a.end[0] ? 0 : n < a.end[1] ? 1 : 2;
+    const int first = i == 0 ? 0 : a.end[i - 1];
+    dst = a.out[i] + (int64_t)m * (a.end[i] - first) + n - first;
+  }
+  *reinterpret_cast<uint64_t *>(dst) = o.q;
 }
 
 // 33 to 128 rows (RB blocks of 32): x is longer than W's share of a workgroup, so
@@ -506,6 +569,47 @@ static void combine(const at::Tensor &slabs, at::Tensor &y) {
                      at::cuda::getCurrentHIPStream(),
                      slabs.data_ptr<float>(), (uint16_t *)y.data_ptr(),
                      (int)slabs.size(0), y.numel());
+}
+
+// act(x W^T + bias), xs and ws as in decode_gemm, columns to matrices of
+// `widths` (multiples of 32, up to three), or as the operand of the next product.
+std::vector<at::Tensor> decode_affine(at::Tensor xs, at::Tensor ws,
+                                      c10::optional<at::Tensor> bias,
+                                      int64_t M, int64_t K,
+                                      std::vector<int64_t> widths, int64_t act,
+                                      bool operand) {
+  Affine a{};
+  int64_t N = 0;
+  TORCH_CHECK(!widths.empty() && widths.size() <= 3 &&
+              (!operand || widths.size() == 1), "decode_affine: widths");
+  TORCH_CHECK(M >= 1 && M <= MMAX && K > 0 && K % 16 == 0 && act >= 0 &&
+              act <= 3, "decode_affine: rows, act");
+  std::vector<at::Tensor> out;
+  for (size_t i = 0; i < widths.size(); ++i) {
+    TORCH_CHECK(widths[i] > 0 && widths[i] % 32 == 0, "decode_affine: widths");
+    out.push_back(operand
+                      ? at::empty({widths[i] / 16 * 512}, xs.options())
+                      : at::empty({M, widths[i]}, xs.options()));
+    a.out[i] = (uint16_t *)out[i].data_ptr();
+    N += widths[i];
+    a.end[i] = (int)N;
+  }
+  TORCH_CHECK(xs.is_cuda() && ws.is_cuda() && xs.is_contiguous() &&
+              ws.is_contiguous() && xs.scalar_type() == at::kBFloat16 &&
+              ws.scalar_type() == at::kBFloat16 &&
+              xs.numel() == (K / 16) * 512 && ws.numel() == N * K,
+              "decode_affine: inputs");
+  TORCH_CHECK(!bias.has_value() ||
+              (bias->is_cuda() && bias->is_contiguous() && bias->numel() == N &&
+               bias->scalar_type() == at::kBFloat16), "decode_affine: bias");
+  a.bias = bias.has_value() ? (const uint16_t *)bias->data_ptr() : nullptr;
+  a.act = (int)act;
+  a.operand = operand;
+  hipLaunchKernelGGL(decode_affine_kernel, dim3((unsigned)(N / 32)),
+                     dim3(BLOCK), 0, at::cuda::getCurrentHIPStream(),
+                     (const uint16_t *)xs.data_ptr(),
+                     (const uint8_t *)ws.data_ptr(), a, (int)M, (int)K);
+  return out;
 }
 
 // Sum of fp32 parts [P, M, N], rounded to bf16.

@@ -1240,3 +1240,62 @@ def test_paged_decode_operand(hq, hkv, dh, vt, nsplit):
     out, swz = ops.paged_decode_with_operand(q, k, v, bt, sl, nsplit=nsplit)
     rows = swz.view(-1, 2, 32, 8)[:, :, :B].permute(2, 0, 1, 3)
     assert torch.equal(rows.reshape(B, hq * dh), out.view(B, hq * dh))
+
+
+@pytest.mark.parametrize("B", [1, 7, 32])
+@pytest.mark.parametrize("act,bias,ff", [("relu", True, 352),
+                                         ("gelu_tanh", True, 1056),
+                                         ("gelu", False, 64)])
+def test_decode_affine(B, act, bias, ff, monkeypatch):
+    """Decode of layer-norm models in nine launches a layer: no further from
+    fp32 than in launches of their own."""
+    _assert_hip()
+    from runbooks_amd.models.config import ModelConfig
+    from runbooks_amd.models.transformer import Transformer, fuse_for_inference
+    cfg = ModelConfig("affine", 256, 192, 2, 3, 3, ff, max_seq_len=128,
+                      head_dim=64, norm="layernorm", act=act, pos="learned",
+                      attn_bias=bias, mlp_bias=bias)
+    g = torch.Generator().manual_seed(B)
+    lens = torch.randint(1, 60, (B,), generator=g)
+    tokens = torch.randint(0, 256, (B,), generator=g)
+    tables = torch.arange(B * 4).view(B, 4)
+    kv = [torch.randn(B * 4, 3, 16, 64, generator=g).bfloat16()
+          for _ in range(4)]
+    slots = torch.tensor([int(tables[i, (n - 1) // 16]) * 16 + (n - 1) % 16
+                          for i, n in enumerate(lens.tolist())])
+
+    def run(dtype, device):
+        torch.manual_seed(1)
+        m = Transformer(cfg, dtype=torch.bfloat16).to(device)
+        with torch.no_grad():
+            for p in m.parameters():
+                p.data = p.data.to(dtype)
+                if p.dim() == 1:
+                    p += torch.linspace(-0.5, 0.5, p.numel(),
+                                        device=device).bfloat16().to(dtype)
+        if device != "cpu":
+            fuse_for_inference(m.eval())
+        caches = [tuple(c.to(device, dtype, copy=True) for c in kv[i:i + 2])
+                  for i in (0, 2)]
+        i32 = dict(device=device, dtype=torch.int32)
+        out = m.decode(tokens.to(device), (lens - 1).to(**i32), caches,
+                       slots.to(**i32), tables.to(**i32), lens.to(**i32),
+                       nsplit=1)
+        return m, out.float().cpu(), [c.float().cpu() for kc in caches
+                                      for c in kc]
+
+    _, ref, ref_kv = run(torch.float32, "cpu")
+    m, new, new_kv = run(torch.bfloat16, DEV)
+    assert m._affine_ready()
+    monkeypatch.setenv("RB_FUSED_RESID", "0")
+    _, old, old_kv = run(torch.bfloat16, DEV)
+
+    def far(got, want):
+        return ((got - want).norm() / want.norm()).item()
+
+    assert far(new, ref) < 1.1 * far(old, ref) + 1e-3
+    for n, o, r in zip(new_kv, old_kv, ref_kv):
+        assert far(n, r) < 1.1 * far(o, r) + 1e-4
+    with torch.no_grad():       # weights that change leave the path
+        m.blocks[0].mlp.fc1.weight.mul_(2)
+    assert not m._affine_ready()

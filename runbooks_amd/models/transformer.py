@@ -460,6 +460,14 @@ class Transformer(nn.Module):
         """All blocks; attention(block) is its attn_fn. Returns the residual
         and what is still to be added to it (None: nothing)."""
         delta = None
+        if self._sums_in_layer_norms(x):
+            dtype, x = x.dtype, x.float()
+            for blk in self.blocks:
+                h = ops.norm_res32(blk.norm1, x, delta, dtype)
+                delta = attention(blk)(h)
+                h = ops.norm_res32(blk.norm2, x, delta, dtype)
+                delta = blk.mlp(h)
+            return x, delta
         for blk in self.blocks:
             if blk.fuses_residual():
                 x, delta = run(blk.forward_pending, x, delta, attention(blk))
@@ -467,9 +475,23 @@ class Transformer(nn.Module):
                 x = run(blk, x, attention(blk))
         return x, delta
 
+    def _sums_in_layer_norms(self, x) -> bool:
+        """The residual may be kept in fp32 and added to in the kernels of the
+        layer norms (results that are not differentiated)."""
+        return (x.is_cuda and x.dtype == torch.bfloat16 and
+                not torch.is_grad_enabled() and self.cfg.norm == "layernorm" and
+                not self.cfg.parallel_residual and not self.cfg.single_norm and
+                x.dim() == 2 and
+                all(n.weight is not None and n.bias is not None and
+                    n.weight.dtype == x.dtype
+                    for blk in self.blocks for n in (blk.norm1, blk.norm2)))
+
     def _last_norm(self, x, delta):
         if delta is None:
             return self.norm_f(x)
+        if x.dtype == torch.float32 and delta.dtype != x.dtype:
+            return ops.norm_res32(self.norm_f, x.contiguous(), delta,
+                                  delta.dtype)
         return ops.rmsnorm_res(x, delta, self.norm_f.weight,
                                self.norm_f.eps)[1]
 

@@ -1299,3 +1299,32 @@ def test_decode_affine(B, act, bias, ff, monkeypatch):
     with torch.no_grad():       # weights that change leave the path
         m.blocks[0].mlp.fc1.weight.mul_(2)
     assert not m._affine_ready()
+
+
+@pytest.mark.parametrize("B,S", [(1, 1), (2, 63), (3, 65)])
+def test_layer_norm_sums(B, S):
+    """Logits of a layer-norm model with the residual's sums in the norms and
+    biases in the products: no further from fp32 than without."""
+    _assert_hip()
+    from runbooks_amd.models.config import ModelConfig
+    from runbooks_amd.models.transformer import Transformer
+    cfg = ModelConfig("sums", 256, 192, 2, 3, 3, 352, max_seq_len=128,
+                      head_dim=64, norm="layernorm", act="relu", pos="learned",
+                      attn_bias=True, mlp_bias=True)
+    tokens = torch.randint(0, 256, (B, S),
+                           generator=torch.Generator().manual_seed(S))
+
+    def run(dtype, device, grad):
+        torch.manual_seed(1)
+        m = Transformer(cfg, dtype=torch.bfloat16).to(device)
+        for p in m.parameters():
+            p.data = p.data.to(dtype)
+            if p.dim() == 1:
+                p.data += torch.linspace(-0.5, 0.5, p.numel(),
+                                         device=device).bfloat16().to(dtype)
+        with torch.set_grad_enabled(grad):
+            return m(tokens.to(device)).detach().float().cpu()
+
+    ref = run(torch.float32, "cpu", False)
+    new, old = run(torch.bfloat16, DEV, False), run(torch.bfloat16, DEV, True)
+    assert (new - ref).norm() < 1.1 * (old - ref).norm() + 1e-3 * ref.norm()

@@ -122,8 +122,8 @@ class GraphedDecoder:
                          seq_starts or [0] * n, state_slots)
 
         # one copy, and one launch within the graph: as seven tensors, each
-        # converted on the way, they were 13 launches, 50 us of a small model's
-        # 530 us step
+        # converted on the way, they were 13 launches (a step of opt-125m 533
+        # and 511 us)
         size = 6 * b + bt.numel()
         self.arrived[:size].copy_(self.h_staging[:size], non_blocking=True)
         g.replay()

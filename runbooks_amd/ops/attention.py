@@ -29,9 +29,10 @@ class _FlashAttnTrain(torch.autograd.Function):
     """
 
     @staticmethod
-    def forward(ctx, q, k, v, scale):
+    def forward(ctx, q, k, v, scale, ordered):
         qc, kc, vc = q.contiguous(), k.contiguous(), v.contiguous()
-        out, lse = _backend.ext().flash_fwd_train(qc, kc, vc, float(scale))
+        out, lse = _backend.ext().flash_fwd_train(qc, kc, vc, float(scale),
+                                                  ordered)
         ctx.save_for_backward(qc, kc, vc, out, lse)
         ctx.scale = float(scale)
         return out
@@ -47,7 +48,7 @@ class _FlashAttnTrain(torch.autograd.Function):
             b, s = dk.shape[0], dk.shape[1]
             dk = dk.view(b, s, hkv, g, -1).sum(dim=3)
             dv = dv.view(b, s, hkv, g, -1).sum(dim=3)
-        return dq, dk, dv, None
+        return dq, dk, dv, None, None
 
 
 class _PackedAttnTrain(torch.autograd.Function):
@@ -82,8 +83,11 @@ def packed_attention(y, cos, sin, positions, B, S, hq, hkv, scale):
 
 
 def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
-                     scale: float | None = None, q_block: int = 256) -> torch.Tensor:
-    """q [B, S, Hq, Dh]; k, v [B, S, Hkv, Dh] -> [B, S, Hq, Dh].
+                     scale: float | None = None, q_block: int = 256,
+                     ordered: bool = False) -> torch.Tensor:
+    """q [B, S, Hq, Dh]; k, v [B, S, Hkv, Dh] -> [B, S, Hq, Dh]. ``ordered``:
+    heads of 64 add and round in the one order that models keep whose
+    gradients jump with the forward's roundings (ReLU).
 
     Differentiable. GPU bf16 (Dh 64/128) runs the MFMA flash kernels;
     otherwise the chunked fp32 reference below (also the numerics oracle
@@ -95,7 +99,8 @@ def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             and q.dtype == torch.bfloat16:
         if scale is None:
             scale = 1.0 / math.sqrt(q.shape[-1])
-        return _FlashAttnTrain.apply(q, k, v, scale)
+        return _FlashAttnTrain.apply(q, k, v, scale,
+                                     ordered and q.shape[-1] == 64)
     return causal_attention_ref(q, k, v, scale=scale, q_block=q_block)
 
 

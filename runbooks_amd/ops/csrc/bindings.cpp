@@ -54,7 +54,7 @@ void qkv_rope_append_(at::Tensor y, at::Tensor cos, at::Tensor sin,
                       int64_t hq);
 at::Tensor flash_prefill(at::Tensor q, at::Tensor k, at::Tensor v, double scale);
 std::vector<at::Tensor> flash_fwd_train(at::Tensor q, at::Tensor k, at::Tensor v,
-                                        double scale);
+                                        double scale, bool ordered);
 std::vector<at::Tensor> fa_bwd(at::Tensor dout, at::Tensor q, at::Tensor k,
                                at::Tensor v, at::Tensor out, at::Tensor lse,
                                double scale);
@@ -120,7 +120,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("qkv_rope_append_", &qkv_rope_append_,
         "packed qkv: q and k rotated in place, k and v appended to the cache");
   m.def("flash_fwd_train", &flash_fwd_train,
-        "MFMA flash-attention forward + log-sum-exp (training)");
+        "MFMA flash-attention forward + log-sum-exp (training)", py::arg("q"),
+        py::arg("k"), py::arg("v"), py::arg("scale"),
+        py::arg("ordered") = false);
   m.def("fa_bwd", &fa_bwd,
         "MFMA flash-attention backward -> (dq, dk_perq, dv_perq)");
   m.def("swiglu_fwd", &swiglu_fwd, "fused silu(g)*u");

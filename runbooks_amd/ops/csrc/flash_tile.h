@@ -84,16 +84,17 @@ RB_DEV bf16x8v row_frag(const char *tile, int r0, int ks, int col, int hi) {
 
 // Operand of columns 32 dt .. 32 dt + 31 along rows r0 .. r0 + 15, in the order
 // of a score tile's registers: element e of lane (hi, col) is column
-// 32 dt + col, row r0 + 8 (e / 4) + 4 hi + e % 4. r0 % 16 == 0.
-template <int DH>
+// 32 dt + col, row r0 + 8 (e / 4) + 4 hi + e % 4; PLAIN: row r0 + 8 hi + e.
+// r0 % 16 == 0.
+template <int DH, bool PLAIN = false>
 RB_DEV bf16x8v column_frag(const char *tile, int r0, int dt, int lane) {
   const int i = lane & 15, hi = lane >> 5;
-  const int r = 4 * hi + (i >> 2);
+  const int r = (PLAIN ? 8 : 4) * hi + (i >> 2), r2 = r + (PLAIN ? 4 : 8);
   const int chunk = dt * 4 + (lane >> 4 & 1) * 2 + (i >> 1 & 1);
   const char *lo = tile + (r0 + r) * (DH * 2) +
                    (chunk ^ mix<DH>(r)) * 16 + (i & 1) * 8;
-  const char *up = tile + (r0 + r + 8) * (DH * 2) +
-                   (chunk ^ mix<DH>(r + 8)) * 16 + (i & 1) * 8;
+  const char *up = tile + (r0 + r2) * (DH * 2) +
+                   (chunk ^ mix<DH>(r2)) * 16 + (i & 1) * 8;
   return rb::lds_column8(lo, up);
 }
 

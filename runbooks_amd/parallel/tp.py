@@ -126,8 +126,10 @@ class RowParallelLinear(nn.Module):
 
     def forward(self, x):
         if self.tp == 1 and self.bias is not None and \
-                x.numel() > 128 * x.shape[-1]:
-            # with its bias in one launch; few rows have products of their own
+                not torch.is_grad_enabled() and x.numel() > 128 * x.shape[-1]:
+            # with its bias in one launch; few rows have products of their
+            # own, and training rounds the product first (as with ordered
+            # attention, gradients of ReLU models follow the roundings)
             return fast_linear(x, self.weight, self.bias)
         y = fast_linear(x, self.weight)
         if self.tp > 1:

@@ -1,6 +1,7 @@
 """GPU kernel numerics: every gfx950 HIP kernel vs its plain-PyTorch fp32
 CPU reference. Run on an MI355X box with `pytest -m gpu`."""
 import math
+import zlib
 
 import pytest
 import torch
@@ -409,6 +410,55 @@ def test_flash_prefill_tiles(B, S, Hq, Hkv, dh, scale):
             ref = s.softmax(-1) @ v[b, :, at].double()
             assert (out[b, :, h] - ref).norm() < 2 ** -8 * ref.norm()
             assert (lse[b, h] - s.logsumexp(-1)).abs().max() < 1e-5
+
+
+def _hashed(n, salt):
+    """Values in [-2, 2) that are the same everywhere."""
+    i = torch.arange(n, dtype=torch.int64) + salt * 7919
+    h = (i * 2654435761) & 0xffffffff
+    h = ((h >> 15) ^ h) * 2246822519 & 0xffffffff
+    h = (h >> 13) ^ h
+    return ((h & 0xffff).float() / 65536 - 0.5) * 4
+
+
+@pytest.mark.parametrize("B,S,Hq,Hkv,bits", [
+    (1, 1, 1, 1, (4093165637, 932004135)),
+    (2, 31, 3, 3, (2980831709, 3346004597)),
+    (1, 64, 4, 2, (3987702248, 4086934317)),
+    (1, 65, 12, 12, (329763779, 1455785953)),
+    (2, 257, 12, 12, (1483102084, 2568763203)),
+    (1, 300, 4, 1, (2206580616, 3272915928)),
+    (1, 1021, 12, 12, (277277627, 2214567642))])
+def test_flash_ordered_bits(B, S, Hq, Hkv, bits):
+    """The training forward of ReLU models does not change a bit of its
+    results (CRCs of them and of the log-sum-exp): their gradients would."""
+    _assert_hip()
+    q, k, v = (_hashed(B * S * h * 64, salt).view(B, S, h, 64).bfloat16()
+               .to(DEV) for salt, h in ((1, Hq), (2, Hkv), (3, Hkv)))
+    out, lse = ops.ext().flash_fwd_train(q, k, v, 0.125, ordered=True)
+    assert bits == tuple(zlib.crc32(x.cpu().numpy().tobytes())
+                         for x in (out.view(torch.int16), lse))
+    assert torch.equal(out, ops.causal_attention(q, k, v, ordered=True))
+
+
+@pytest.mark.parametrize("S,scale", [(97, None), (200, -0.1), (130, 0.0),
+                                     (33, 0.3)])
+def test_flash_ordered(S, scale):
+    """As test_flash_prefill_tiles, with any factor."""
+    _assert_hip()
+    g = torch.Generator(device=DEV).manual_seed(S)
+    q, k, v = (torch.randn(2, S, h, 64, generator=g, device=DEV).bfloat16()
+               for h in (6, 3, 3))
+    scale = 0.125 if scale is None else scale
+    out, lse = ops.ext().flash_fwd_train(q, k, v, scale, ordered=True)
+    ref = q.double().transpose(1, 2) @ k.double().repeat_interleave(
+        2, 2).permute(0, 2, 3, 1).contiguous() * scale
+    ref.masked_fill_(torch.ones(S, S, dtype=torch.bool, device=DEV).triu(1),
+                     float("-inf"))
+    assert (lse - ref.logsumexp(-1)).abs().max() < 1e-5
+    ref = ref.softmax(-1) @ v.double().repeat_interleave(2, 2).transpose(
+        1, 2).contiguous()
+    assert (out.transpose(1, 2) - ref).norm() < 2 ** -8 * ref.norm()
 
 
 @pytest.mark.parametrize("B,S,Hq,Hkv,dh,scale", [

@@ -1,6 +1,10 @@
 """Trainer loop + checkpoint/resume on CPU."""
+import pytest
 import torch
 
+from runbooks_amd import ops
+from runbooks_amd.models import build_model
+from runbooks_amd.parallel.tp import RowParallelLinear
 from runbooks_amd.train import (TrainConfig, Trainer, latest_checkpoint,
                                 load_checkpoint, save_checkpoint)
 
@@ -385,3 +389,31 @@ def test_gradients_arrive_together(monkeypatch):
         assert torch.equal(net.unused.grad, torch.zeros(3))
         ddp.zero_grad()
         assert all(not b.any() for b in ddp.grad_buffers())
+
+
+@pytest.mark.parametrize("model,ordered", [("tiny-opt", True),
+                                           ("tiny-gpt2", False),
+                                           ("tiny-llama", False)])
+def test_relu_models_train_on_ordered_attention(model, ordered, monkeypatch):
+    seen, plain = [], ops.causal_attention
+
+    def attention(*args, ordered=False, **kw):
+        seen.append(ordered)
+        return plain(*args, ordered=ordered, **kw)
+
+    monkeypatch.setattr(ops, "causal_attention", attention)
+    build_model(model, dtype=torch.float32, tp=1)(
+        torch.zeros(1, 5, dtype=torch.long))
+    assert seen and set(seen) == {ordered}
+
+
+def test_training_rounds_row_products_before_the_bias():
+    torch.manual_seed(0)
+    layer = RowParallelLinear(96, 64, bias=True, tp_size=1,
+                              dtype=torch.bfloat16)
+    with torch.no_grad():
+        layer.weight.normal_()
+        layer.bias.normal_()
+    x = torch.randn(300, 96).bfloat16()
+    assert torch.equal(layer(x), torch.nn.functional.linear(x, layer.weight) +
+                       layer.bias)

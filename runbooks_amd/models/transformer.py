@@ -127,8 +127,8 @@ class Attention(nn.Module):
         q = q.view(B, S, self.hq, self.dh)
         k = k.view(B, S, self.hkv, self.dh)
         v = v.view(B, S, self.hkv, self.dh)
-        o = ops.causal_attention(q, k, v, scale=self.scale,
-                                 ordered=self.cfg.act == "relu")
+        ordered = {"ordered": True} if self.cfg.act == "relu" else {}
+        o = ops.causal_attention(q, k, v, scale=self.scale, **ordered)
         return self.o_proj(o.reshape(B * S, self.hq * self.dh))
 
     def _fused_append(self, x, kc) -> bool:

@@ -40,6 +40,7 @@ from ..parallel import (
     comm,
     gather_from_tp,
 )
+from ..utils.modules import plain
 from .config import LatentAttentionSpec, ModelConfig
 from .dual import DualBlock
 from .hybrid import SequentialBlock
@@ -281,8 +282,10 @@ class Block(nn.Module):
 
     def fuses_residual(self) -> bool:
         """The sums of the residual may go into the norms that follow them."""
-        return (isinstance(self.norm1, ops.RMSNorm) and
-                not self.cfg.parallel_residual and not self.cfg.single_norm)
+        return (self.cfg.norm == "rmsnorm" and
+                not self.cfg.parallel_residual and not self.cfg.single_norm and
+                plain(Block, self) and
+                plain(ops.RMSNorm, self.norm1, self.norm2))
 
     def forward_pending(self, x, delta, attn_fn):
         """forward() of a residual whose last term is still to be added:
@@ -473,6 +476,8 @@ class Transformer(nn.Module):
             if blk.fuses_residual():
                 x, delta = run(blk.forward_pending, x, delta, attention(blk))
             else:
+                if delta is not None:
+                    x, delta = x + delta, None
                 x = run(blk, x, attention(blk))
         return x, delta
 
@@ -482,10 +487,15 @@ class Transformer(nn.Module):
         return (x.is_cuda and x.dtype == torch.bfloat16 and
                 not torch.is_grad_enabled() and self.cfg.norm == "layernorm" and
                 not self.cfg.parallel_residual and not self.cfg.single_norm and
-                x.dim() == 2 and
-                all(n.weight is not None and n.bias is not None and
-                    n.weight.dtype == x.dtype
-                    for blk in self.blocks for n in (blk.norm1, blk.norm2)))
+                x.dim() == 2 and len(self.blocks) > 0 and
+                plain(Block, *self.blocks) and
+                all(plain(nn.LayerNorm, n) and n.weight is not None and
+                    n.bias is not None and n.weight.dtype == x.dtype
+                    for n in self._layer_norms()))
+
+    def _layer_norms(self):
+        return [n for blk in self.blocks for n in (blk.norm1, blk.norm2)] + \
+            [self.norm_f]
 
     def _last_norm(self, x, delta):
         if delta is None:
@@ -493,6 +503,8 @@ class Transformer(nn.Module):
         if x.dtype == torch.float32 and delta.dtype != x.dtype:
             return ops.norm_res32(self.norm_f, x.contiguous(), delta,
                                   delta.dtype)
+        if not plain(ops.RMSNorm, self.norm_f):
+            return self.norm_f(x + delta)
         return ops.rmsnorm_res(x, delta, self.norm_f.weight,
                                self.norm_f.eps)[1]
 
@@ -585,10 +597,13 @@ class Transformer(nn.Module):
 
     def _affine_ready(self) -> bool:
         """Every block has its products for _decode_affine, of weights that have
-        not changed since."""
+        not changed since, and no module that they do the work of would do
+        more."""
         return (os.environ.get("RB_FUSED_RESID", "1") == "1" and
                 all(getattr(blk, "_affine", None) is not None and
-                    blk._affine.current() for blk in self.blocks))
+                    _AffineBlock.plain(blk) and
+                    blk._affine.current() for blk in self.blocks) and
+                plain(nn.LayerNorm, *self._layer_norms()))
 
     def _decode_affine(self, x, caches, slot_mapping, block_tables, seq_lens,
                        nsplit, seq_starts):
@@ -774,6 +789,14 @@ class _AffineBlock:
                 a.hq * a.dh % 32 == 0 and a.hkv * a.dh % 32 == 0 and
                 all(n.weight is not None and n.bias is not None
                     for n in (blk.norm1, blk.norm2, model.norm_f)))
+
+    @staticmethod
+    def plain(blk) -> bool:
+        a, m = blk.attn, blk.mlp
+        return (plain(Block, blk) and plain(MLP, m) and
+                plain(ColumnParallelLinear, a.q_proj, a.k_proj, a.v_proj,
+                      m.fc1) and
+                plain(RowParallelLinear, a.o_proj, m.down_proj))
 
     def __init__(self, blk, act: str):
         a, m = blk.attn, blk.mlp

@@ -20,6 +20,7 @@ from torch import nn
 from ..ops import _backend
 from ..ops.linear import wide_product, wide_product_grad
 from ..parallel.tp import ColumnParallelLinear, RowParallelLinear
+from ..utils.modules import plain
 
 
 def _delta_add_(y, t, w, scale, w_transposed=True):
@@ -130,10 +131,9 @@ class _LoRAGroup:
     def packed(self, x):
         """All members' results on x side by side, or None where the members
         have to be called one by one."""
-        if any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-               or m._backward_pre_hooks for m in self.members):
-            return None
-        return _packed(self.members, x) if _packs(self.members, x) else None
+        if plain(LoRALinear, *self.members) and _packs(self.members, x):
+            return _packed(self.members, x)
+        return None
 
     def t_for(self, member, x):
         if self._x_id != id(x) or self._left <= 0:

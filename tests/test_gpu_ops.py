@@ -1378,3 +1378,53 @@ def test_layer_norm_sums(B, S):
     ref = run(torch.float32, "cpu", False)
     new, old = run(torch.bfloat16, DEV, False), run(torch.bfloat16, DEV, True)
     assert (new - ref).norm() < 1.1 * (old - ref).norm() + 1e-3 * ref.norm()
+
+
+@pytest.mark.parametrize("where", ["block", "norm1", "fc1", "adapters"])
+def test_decode_affine_leaves_modules_that_do_more(where):
+    """A hook, or an adapter put in later, takes decoding off the path that
+    does the work of its module."""
+    _assert_hip()
+    from runbooks_amd.models import build_model
+    from runbooks_amd.models.transformer import fuse_for_inference
+    from runbooks_amd.train import apply_lora
+    m = fuse_for_inference(build_model("opt-125m", dtype=torch.bfloat16, tp=1,
+                                       device=DEV).eval())
+    caches = m.alloc_caches(2, DEV)
+    i32 = dict(device=DEV, dtype=torch.int32)
+
+    def decode():
+        return m.decode(torch.tensor([5], device=DEV),
+                        torch.tensor([0], **i32), caches,
+                        torch.tensor([0], **i32), torch.tensor([[0]], **i32),
+                        torch.tensor([1], **i32), nsplit=1)
+
+    first = decode()
+    assert m._affine_ready()
+    blk, fired = m.blocks[1], []
+    if where == "adapters":
+        apply_lora(m, r=8)
+        with torch.no_grad():
+            blk.mlp.fc1.lora_b.normal_()
+        assert not torch.allclose(decode(), first, atol=1e-2)
+        return
+    {"block": blk, "norm1": blk.norm1, "fc1": blk.mlp.fc1}[
+        where].register_forward_hook(lambda *a: fired.append(1))
+    again = decode()
+    assert fired == [1]
+    assert (again - first).norm() < 0.03 * first.norm()
+
+
+@pytest.mark.parametrize("name", ["opt-125m", "smoke-llama"])
+def test_prefill_hooks_fire(name):
+    _assert_hip()
+    from runbooks_amd.models import build_model
+    m = build_model(name, dtype=torch.bfloat16, tp=1, device=DEV).eval()
+    tokens, fired = torch.arange(40, device=DEV).view(1, 40), []
+    with torch.no_grad():
+        want = m(tokens)
+        for mod in (m.blocks[0], m.blocks[1].norm2, m.norm_f):
+            mod.register_forward_hook(lambda *a: fired.append(1))
+        got = m(tokens)
+    assert len(fired) == 3
+    assert (got - want).norm() < 0.03 * want.norm()

@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from runbooks_amd import ops
 from runbooks_amd.models import build_model, get_config, list_configs
 from runbooks_amd.serve import Engine
 from runbooks_amd.train import apply_lora, lora_state_dict, merge_lora
@@ -746,3 +747,51 @@ def test_engine_fuzz_vt_gqa_bf16(seed):
     assert not eng.has_work()
     eng.flush_prefix_cache()
     assert len(eng.allocator.free) == eng.allocator.num_blocks
+
+
+@pytest.mark.parametrize("name", ["tiny-llama", "tiny-opt", "tiny-falcon"])
+@pytest.mark.parametrize("grad", [True, False])
+def test_module_hooks_fire(name, grad):
+    """Hooks of blocks and norms see every pass, and change nothing else."""
+    m = build_model(name, dtype=torch.float32, tp=1)
+    tokens = torch.randint(0, 256, (2, 16))
+    with torch.set_grad_enabled(grad):
+        want, fired = m(tokens), []
+        blk = m.blocks[0]
+        hooked = [blk, m.blocks[1].norm1, blk.norm2, m.norm_f]
+        for mod in hooked:
+            if mod is not None:
+                mod.register_forward_hook(
+                    lambda mod, args, out: fired.append(mod))
+        assert torch.allclose(m(tokens), want, atol=1e-5)
+    assert {id(x) for x in fired} == {id(x) for x in hooked if x is not None}
+    assert len(fired) == len([x for x in hooked if x is not None])
+
+
+def test_modules_of_other_kinds_run():
+    """A norm of a subclass, a forward of an object's own and a global hook
+    are not passed by."""
+    m = build_model("tiny-llama", dtype=torch.float32, tp=1)
+    tokens = torch.randint(0, 256, (1, 8))
+    calls = []
+
+    class Norm(ops.RMSNorm):
+        def forward(self, x):
+            calls.append("norm")
+            return super().forward(x)
+
+    m.blocks[1].norm2.__class__ = Norm
+    m(tokens)
+    assert calls == ["norm"]
+    m.norm_f.forward = lambda x: calls.append("own") or x
+    m(tokens)
+    assert calls == ["norm", "norm", "own"]
+    m = build_model("tiny-llama", dtype=torch.float32, tp=1)
+    seen = []
+    handle = torch.nn.modules.module.register_module_forward_hook(
+        lambda mod, args, out: seen.append(type(mod).__name__))
+    try:
+        m(tokens)
+    finally:
+        handle.remove()
+    assert seen.count("Block") == 2 and seen.count("RMSNorm") == 5

@@ -773,8 +773,9 @@ class Transformer(nn.Module):
 
 
 class _AffineBlock:
-    """A block's products with their biases and activation in the decode GEMM's
-    layout (csrc/decode_gemm.hip, decode_affine)."""
+    """A block's products with their biases and activation in a launch each
+    (csrc/decode_gemm.hip, decode_affine). They read the parameters, so a
+    captured step follows weights that change in place."""
 
     ACTS = {"relu": 1, "gelu": 2, "gelu_tanh": 3}
 
@@ -800,43 +801,38 @@ class _AffineBlock:
 
     def __init__(self, blk, act: str):
         a, m = blk.attn, blk.mlp
-        qkv = (a.q_proj, a.k_proj, a.v_proj)
         self.act = self.ACTS[act]
-        self.widths = [p.weight.shape[0] for p in qkv]
-        self.sources = [t for p in (*qkv, a.o_proj, m.fc1, m.down_proj)
+        self.qkv_proj = (a.q_proj, a.k_proj, a.v_proj)
+        self.o_proj, self.fc1, self.down_proj = a.o_proj, m.fc1, m.down_proj
+        self.sources = [t for p in (*self.qkv_proj, a.o_proj, m.fc1,
+                                    m.down_proj)
                         for t in (p.weight, p.bias) if t is not None]
         self.versions = self._versions()
-        swizzle = ops.ext().decode_swizzle_w
-        bias = [p.bias for p in qkv]
-        self.qkv_w = swizzle(torch.cat([p.weight.data for p in qkv]))
-        self.qkv_b = None if bias[0] is None else torch.cat(
-            [b.data for b in bias])
-        self.rest = [(swizzle(p.weight.data), p.weight.shape[0],
-                      p.weight.shape[1], p.bias)
-                     for p in (a.o_proj, m.fc1, m.down_proj)]
-        self.k = a.q_proj.weight.shape[1]
 
     def _versions(self):
-        return [(t.data_ptr(), None if t.is_inference() else t._version)
+        return [(t.data_ptr(), t.dtype,
+                 None if t.is_inference() else t._version)
                 for t in self.sources]
 
     def current(self) -> bool:
+        """The parameters are those of the time of fusing."""
         return self._versions() == self.versions
 
-    def qkv(self, swz, rows: int):
-        return ops.ext().decode_affine(swz, self.qkv_w, self.qkv_b, rows,
-                                       self.k, self.widths)
+    @staticmethod
+    def _products(projections, swz, rows: int, act: int = 0, operand=False):
+        return ops.ext().decode_affine(
+            swz, [p.weight for p in projections],
+            [p.bias for p in projections], rows, act, operand)
 
-    def _one(self, i: int, swz, rows: int, act: int = 0, operand=False):
-        w, n, k, b = self.rest[i]
-        return ops.ext().decode_affine(swz, w, b, rows, k, [n], act,
-                                       operand)[0]
+    def qkv(self, swz, rows: int):
+        return self._products(self.qkv_proj, swz, rows)
 
     def o(self, swz, rows: int):
-        return self._one(0, swz, rows)
+        return self._products((self.o_proj,), swz, rows)[0]
 
     def mlp(self, swz, rows: int):
-        return self._one(2, self._one(1, swz, rows, self.act, True), rows)
+        h = self._products((self.fc1,), swz, rows, self.act, True)[0]
+        return self._products((self.down_proj,), h, rows)[0]
 
 
 def _fuse_projections(model: "Transformer") -> list[torch.Tensor]:
@@ -915,15 +911,12 @@ def fuse_for_inference(model: "Transformer",
                                           model.lm_head.weight.shape[1]):
             cands.append(model.lm_head.weight)
         need = sum(2 * w.numel() for w in cands)
-        affine = [] if model.ragged else [
-            blk for blk in model.blocks if model.lm_head.weight.is_cuda and
-            _AffineBlock.serves(model, blk)]
-        need += sum(2 * p.numel() for blk in affine for p in blk.parameters())
         free, total = torch.cuda.mem_get_info()
         if free - need >= int(0.35 * total):
             for w in cands:
                 register_decode_weight(w)
-            for blk in affine:
+        for blk in () if model.ragged else model.blocks:
+            if model.lm_head.weight.is_cuda and _AffineBlock.serves(model, blk):
                 blk._affine = _AffineBlock(blk, model.cfg.act)
 
     if load_in_8bit and torch.cuda.is_available():

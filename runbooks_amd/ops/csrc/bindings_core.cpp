@@ -24,7 +24,7 @@ at::Tensor decode_gemm(at::Tensor xs, at::Tensor ws, int64_t M, int64_t N, int64
 at::Tensor decode_swizzle_w(at::Tensor w);
 at::Tensor decode_swizzle_x(at::Tensor x);
 at::Tensor decode_swizzle_w8(at::Tensor w8);
-std::vector<at::Tensor> decode_affine(at::Tensor xs, at::Tensor ws, c10::optional<at::Tensor> bias, int64_t M, int64_t K, std::vector<int64_t> widths, int64_t act, bool operand);
+std::vector<at::Tensor> decode_affine(at::Tensor xs, std::vector<at::Tensor> ws, std::vector<c10::optional<at::Tensor>> biases, int64_t M, int64_t act, bool operand);
 at::Tensor sum_parts(at::Tensor parts);
 at::Tensor decode_gemm_rows(at::Tensor x, at::Tensor ws, int64_t N);
 at::Tensor decode_gemm_fp8(at::Tensor xs, at::Tensor w8s, at::Tensor scale, int64_t M, int64_t N, int64_t K, bool raw);
@@ -77,9 +77,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "one-time weight layout swizzle for decode_gemm_fp8");
   m.def("decode_affine", &decode_affine,
         "act(x W^T + bias) to up to three matrices, or as an operand",
-        py::arg("xs"), py::arg("ws"), py::arg("bias"), py::arg("M"),
-        py::arg("K"), py::arg("widths"), py::arg("act") = 0,
-        py::arg("operand") = false);
+        py::arg("xs"), py::arg("ws"), py::arg("biases"), py::arg("M"),
+        py::arg("act") = 0, py::arg("operand") = false);
   m.def("sum_parts", &sum_parts, "fp32 [P, M, N] -> their sum [M, N] bf16");
   m.def("decode_gemm_rows", &decode_gemm_rows, "x [M <= 128, K] W^T");
   m.def("decode_gemm_fp8", &decode_gemm_fp8,

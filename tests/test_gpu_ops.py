@@ -1380,6 +1380,84 @@ def test_layer_norm_sums(B, S):
     assert (new - ref).norm() < 1.1 * (old - ref).norm() + 1e-3 * ref.norm()
 
 
+@pytest.mark.parametrize("M,widths,K", [
+    (1, [32], 32), (16, [32, 64, 32], 96), (17, [64, 32, 32], 288),
+    (31, [4096], 160), (32, [4128], 1056), (9, [4128, 32], 800)])
+@pytest.mark.parametrize("act,bias", [(0, True), (1, False), (2, True),
+                                      (3, True)])
+def test_decode_affine_products(M, widths, K, act, bias):
+    """Edges of the row blocks, of the waves' shares of K and of the matrices;
+    fp32 sums, one rounding (2^-9 relative, twice that for the sums' own and
+    the activation's)."""
+    _assert_hip()
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    ws = [torch.randn(n, K, generator=g, device=DEV).bfloat16()
+          for n in widths]
+    bs = [torch.randn(n, generator=g, device=DEV).bfloat16() if bias else None
+          for n in widths]
+    xs = ops.ext().decode_swizzle_x(x)
+    out = ops.ext().decode_affine(xs, ws, bs, M, act)
+    f = [lambda y: y, torch.relu, torch.nn.functional.gelu,
+         lambda y: torch.nn.functional.gelu(y, approximate="tanh")][act]
+    for y, w, b in zip(out, ws, bs):
+        ref = x.double() @ w.double().t()
+        ref = f(ref if b is None else ref + b.double())
+        assert y.shape == ref.shape
+        assert (y - ref).norm() <= 2 ** -8 * ref.norm()
+    h = ops.ext().decode_affine(xs, ws[:1], bs[:1], M, act, operand=True)[0]
+    assert torch.equal(h.view(-1, 2, 32, 8)[:, :, :M].permute(2, 0, 1, 3)
+                       .reshape(M, -1), out[0])
+
+
+@pytest.mark.parametrize("batch", [1, 20])
+@pytest.mark.parametrize("name", ["q_proj", "v_proj.bias", "fc1", "fc1.bias",
+                                  "o_proj", "down_proj.bias"])
+def test_captured_decode_follows_weights(name, batch):
+    """A captured step of a layer-norm model computes with weights that were
+    changed after the capture, as an eager one does: through the parameter, or
+    past its version through .data."""
+    _assert_hip()
+    from runbooks_amd.models.config import ModelConfig
+    from runbooks_amd.models.transformer import Transformer, fuse_for_inference
+    from runbooks_amd.serve.graph import GraphedDecoder
+    cfg = ModelConfig("follow", 256, 192, 2, 3, 3, 352, max_seq_len=64,
+                      head_dim=64, norm="layernorm", act="relu", pos="learned",
+                      attn_bias=True, mlp_bias=True)
+    torch.manual_seed(1)
+    m = fuse_for_inference(Transformer(cfg, dtype=torch.bfloat16, tp=1)
+                           .to(DEV).eval())
+    caches = m.alloc_caches(batch + 1, DEV)
+    for c in (c for kv in caches for c in kv):
+        c.normal_()
+    step = (list(range(batch)), [9] * batch,
+            [i * 16 + 9 for i in range(batch)], [[i] for i in range(batch)],
+            [10] * batch)
+    i32 = dict(device=DEV, dtype=torch.int32)
+
+    def eager():
+        return m.decode(torch.tensor(step[0], device=DEV),
+                        torch.tensor(step[1], **i32), caches,
+                        torch.tensor(step[2], **i32),
+                        torch.tensor(step[3], **i32),
+                        torch.tensor(step[4], **i32), nsplit=1)
+
+    with torch.no_grad():
+        graphed = GraphedDecoder(m, caches, batch, 1, batch, DEV)
+        layer, _, which = name.partition(".")
+        blk = m.blocks[1]
+        p = getattr(getattr(blk.attn, layer, None) or getattr(blk.mlp, layer),
+                    which or "weight")
+        before = graphed.decode(*step).clone()
+        assert m._affine_ready()
+        for change in (p, p.data):
+            change.add_(torch.randn_like(p))
+            got, want = graphed.decode(*step), eager()
+            assert (got - want).norm() < 0.02 * want.norm()
+            assert (got - before).norm() > 0.05 * before.norm()
+            before = got.clone()
+
+
 @pytest.mark.parametrize("where", ["block", "norm1", "fc1", "adapters"])
 def test_decode_affine_leaves_modules_that_do_more(where):
     """A hook, or an adapter put in later, takes decoding off the path that

@@ -23,9 +23,9 @@ _USE_DECODE_GEMM = os.environ.get("RB_DECODE_GEMM", "1") == "1"
 
 
 # data_ptr(weight) -> (e4m3 bytes in the decode GEMM's order, f32 per-channel
-# scale, weakref to the weight). Populated by quantize_fp8 (serving with
-# MODEL_LOAD_IN_8BIT); looked up on the decode fast path.
-_FP8_REGISTRY: dict[int, tuple[torch.Tensor, torch.Tensor]] = {}
+# scale, the weight's version, weakref to the weight). Populated by quantize_fp8
+# (serving with MODEL_LOAD_IN_8BIT); looked up on the decode fast path.
+_FP8_REGISTRY: dict[int, tuple] = {}
 
 # data_ptr(weight) -> fragment-lane-major copy ([N/32][K/16][lane][8])
 # consumed by csrc/decode_gemm.hip. A second full-precision weight copy:
@@ -39,18 +39,21 @@ _FP8_REGISTRY: dict[int, tuple[torch.Tensor, torch.Tensor]] = {}
 _DECODE_W_REGISTRY: dict[int, tuple] = {}
 
 
+def _version(weight: torch.Tensor):
+    return None if weight.is_inference() else weight._version
+
+
 def _registry_get(reg: dict, weight: torch.Tensor):
+    """A weight's entry, for all products alike: none once the weight has
+    changed in place (changes through .data leave no trace). The entry stays,
+    as a captured step may read its copy."""
     entry = reg.get(weight.data_ptr())
     if entry is None:
         return None
     if entry[-1]() is not weight:
         del reg[weight.data_ptr()]
         return None
-    return entry
-
-
-def _version(weight: torch.Tensor):
-    return None if weight.is_inference() else weight._version
+    return entry if entry[-2] == _version(weight) else None
 
 
 def register_decode_weight(weight: torch.Tensor) -> None:
@@ -82,7 +85,7 @@ def quantize_fp8(weight: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     served = (_backend.ext().decode_swizzle_w8(w8_bytes)
               if weight.is_cuda and _fp8_served(*weight.shape) else w8_bytes)
     _FP8_REGISTRY[weight.data_ptr()] = (served, scale.contiguous(),
-                                        weakref.ref(weight))
+                                        _version(weight), weakref.ref(weight))
     return w8_bytes, scale
 
 
@@ -142,7 +145,7 @@ def fast_linear(x: torch.Tensor, weight: torch.Tensor,
 def _rows_linear(x: torch.Tensor, weight: torch.Tensor, m: int, n: int,
                  k: int) -> torch.Tensor | None:
     """x @ weight^T of up to 128 rows on the decode GEMM that reads x as it is,
-    or None where the weight has no decode layout (or has changed since).
+    or None where the weight has no decode layout.
 
     us on the library and there: 64 rows, 22016 x 4096 44.4 and 35.8, 4096 x
     4096 23.0 and 14.1, 4096 x 14336 40.4 and 27.3, 3072 x 24576 102 and 34; 128
@@ -151,7 +154,7 @@ def _rows_linear(x: torch.Tensor, weight: torch.Tensor, m: int, n: int,
             not x.is_contiguous() or x.data_ptr() % 16:
         return None
     dw = _registry_get(_DECODE_W_REGISTRY, weight)
-    if dw is None or dw[2] != _version(weight):
+    if dw is None:
         return None
     y = _backend.ext().decode_gemm_rows(x.view(m, k), dw[0], n)
     return y.view(*x.shape[:-1], n)

@@ -1243,6 +1243,30 @@ def test_decode_gemm_rows(M, N, K):
     assert (y.double() - ref).norm() < 2 ** -8 * ref.norm()
 
 
+@pytest.mark.parametrize("m", [1, 16, 20, 32, 40])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_products_of_changed_weight(m, fp8):
+    """Products of any number of rows follow a weight that changes in place,
+    whichever of its layouts they would read."""
+    from runbooks_amd.ops.linear import (decode_linear_raw, fast_linear,
+                                         quantize_fp8, register_decode_weight,
+                                         wide_linear)
+    torch.manual_seed(m)
+    w = torch.randn(10240, 1024, device=DEV).bfloat16()
+    x = torch.randn(m, 1024, device=DEV).bfloat16()
+    (quantize_fp8 if fp8 else register_decode_weight)(w)
+    products = [fast_linear, wide_linear]
+    if m <= 32:
+        products.append(lambda x, w: decode_linear_raw(x, w)[0])
+    with torch.no_grad():
+        w.copy_(torch.randn(10240, 1024, device=DEV))
+        ref = x.double() @ w.double().t()
+        for product in products:
+            y = product(x, w).double()
+            y = y.sum(0) if y.dim() == 3 else y
+            assert (y - ref).norm() < 2 ** -8 * ref.norm()
+
+
 def test_decode_gemm_rows_of_changed_weight():
     """Products of 33 to 128 rows follow a weight that changes in place."""
     from runbooks_amd.ops.linear import fast_linear, register_decode_weight

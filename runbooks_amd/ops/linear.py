@@ -218,11 +218,12 @@ def wide_product_grad(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
     Wide results in whole rounds of tiles, like wide_product's (2048 rows of
     4096 to 11008 columns: 284 and 171 us; to 4096 and 6144 columns 3 to 14%
-    slower in two calls). Long sums with few tiles in two halves: there the
-    library keeps tiles of 256 x 256, of which there are not enough (us in one
-    sum and in two, to 4096 columns: 2048 rows of 22016 456 and 335, 512 231 and
-    196, 1024 rows of 28672 344 and 296, 2048 380 and 441; with more tiles, 2560
-    rows of 22016, 372 and 390; of 12288 and 2048 rows 195 and 213)."""
+    slower in two calls). Long sums with few tiles in two fp32 halves, rounded
+    once: there the library keeps tiles of 256 x 256, of which there are not
+    enough (us in one sum and in two, to 4096 columns: 2048 rows of 22016 453
+    and 372, 512 213 and 163, 1024 rows of 28672 359 and 307, 2048 401 and 463;
+    with more tiles, 2560 rows of 22016, 372 and 390; of 12288 and 2048 rows 195
+    and 213)."""
     rows, (n, k) = dy.shape[0], weight.shape
     if k >= 8192:
         main = _whole_rounds(rows, k)
@@ -231,10 +232,13 @@ def wide_product_grad(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
             torch.mm(dy, weight[:, :main], out=dx[:, :main])
             torch.mm(dy, weight[:, main:], out=dx[:, main:])
             return dx
-    if n > 16384 and -(-rows // 256) * -(-k // 256) <= 144:
+    if n > 16384 and k % 4 == 0 and \
+            -(-rows // 256) * -(-k // 256) <= 144:
         half = n // 128 * 64
-        return (dy[:, :half] @ weight[:half]).addmm_(dy[:, half:],
-                                                     weight[half:])
+        parts = torch.empty(2, rows, k, dtype=torch.float32, device=dy.device)
+        for part, at in zip(parts, (slice(0, half), slice(half, n))):
+            torch.mm(dy[:, at], weight[at], out_dtype=torch.float32, out=part)
+        return _backend.ext().sum_parts(parts)
     return dy @ weight
 
 

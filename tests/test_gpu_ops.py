@@ -1224,8 +1224,9 @@ def test_wide_products(rows, n, k):
                      (wide_product_grad(x, w.t().contiguous()),
                       x.double() @ w.double().t()),
                      (wide_product_grad(y, w), y.double() @ w.double())):
-        # one rounding of the result, or two where a sum is in halves
-        assert (got.double() - ref).norm() < 2 ** -7.5 * ref.norm()
+        # one rounding of the result (at most 2^-9 of each value; of two the
+        # norm is larger, 2^-8.9), fp32 sums
+        assert (got.double() - ref).norm() < (2 ** -9 + 1e-5) * ref.norm()
 
 
 @pytest.mark.parametrize("M", [1, 32, 33, 64, 65, 128])

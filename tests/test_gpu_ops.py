@@ -1212,7 +1212,8 @@ def test_lora_siblings_train(heads, kv, dh, B, S, monkeypatch):
 
 @pytest.mark.parametrize("rows,n,k", [(1281, 2816, 64), (2048, 11008, 64),
                                       (1536, 10816, 192), (300, 192, 8192),
-                                      (129, 16448, 64), (257, 16512, 4096)])
+                                      (129, 16448, 64), (257, 16512, 4096),
+                                      (65, 32768, 64), (65, 32832, 64)])
 def test_wide_products(rows, n, k):
     """Products in one or two calls, [rows, k] by [n, k] and back, vs fp64."""
     from runbooks_amd.ops.linear import wide_product, wide_product_grad

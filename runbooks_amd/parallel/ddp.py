@@ -36,7 +36,7 @@ class _Bucket:
             off += p.numel()
         self.pending = 0
         self.work = None
-        self.arrived = []           # (slot, gradient) not yet in the buffer
+        self.arrived = {}           # slot -> gradient not yet in the buffer
         self.arrived_on = None      # the stream that they arrived on
         self.arrived_bytes = 0
 
@@ -45,15 +45,15 @@ class _Bucket:
         it arrived on; the current one waits for that."""
         if not self.arrived:
             return
-        slots, grads = zip(*self.arrived)
-        self.arrived, self.arrived_bytes = [], 0
-        views = [self.views[i] for i in slots]
+        views = [self.views[i] for i in self.arrived]
+        grads = list(self.arrived.values())
+        self.arrived, self.arrived_bytes = {}, 0
         there = self.arrived_on
         if there is None or there == torch.cuda.current_stream(there.device):
-            torch._foreach_add_(views, list(grads))
+            torch._foreach_add_(views, grads)
             return
         with torch.cuda.stream(there):
-            torch._foreach_add_(views, list(grads))
+            torch._foreach_add_(views, grads)
         torch.cuda.current_stream(there.device).wait_stream(there)
 
 
@@ -125,10 +125,10 @@ class DataParallel(nn.Module):
         # accumulate into the flat buffer and release the autograd tensor;
         # micro-batch accumulation keeps adding into the same slot.
         stream = torch.cuda.current_stream(p.device) if p.is_cuda else None
-        if stream != b.arrived_on or any(i == j for j, _ in b.arrived):
+        if stream != b.arrived_on or i in b.arrived:
             b.flush()
             b.arrived_on = stream
-        b.arrived.append((i, p.grad))
+        b.arrived[i] = p.grad
         b.arrived_bytes += p.grad.numel() * p.grad.element_size()
         p.grad = None
         b.pending -= 1
@@ -167,7 +167,7 @@ class DataParallel(nn.Module):
 
     def zero_grad(self, set_to_none: bool = False):  # noqa: ARG002
         for b in self._buckets:
-            b.arrived, b.arrived_bytes = [], 0
+            b.arrived, b.arrived_bytes = {}, 0
             b.buffer.zero_()
             for p in b.params:
                 p.grad = None   # next backward must produce a fresh tensor

@@ -1,4 +1,6 @@
 """Trainer loop + checkpoint/resume on CPU."""
+import sys
+
 import pytest
 import torch
 
@@ -417,3 +419,25 @@ def test_training_rounds_row_products_before_the_bias():
     x = torch.randn(300, 96).bfloat16()
     assert torch.equal(layer(x), torch.nn.functional.linear(x, layer.weight) +
                        layer.bias)
+
+
+@pytest.mark.parametrize("n", [30, 300])
+def test_gradient_hook_takes_the_same_however_many_wait(n):
+    """Host work of a gradient's arrival, counted in calls: none of it grows
+    with the gradients that wait in its bucket."""
+    from runbooks_amd.parallel import DataParallel
+    net = torch.nn.ParameterList(torch.nn.Parameter(torch.ones(2))
+                                 for _ in range(n))
+    net.last = torch.nn.Parameter(torch.ones(2))    # keeps the bucket open
+    ddp, calls = DataParallel(net), []
+    ddp.start_microbatch(sync=False)
+    for p in net:
+        p.grad = torch.ones(2)
+    sys.setprofile(lambda frame, event, arg: calls.append(event))
+    try:
+        for p in net:
+            ddp._on_grad(p)
+    finally:
+        sys.setprofile(None)
+    assert len(calls) < 40 * n
+    assert sum(int(b.sum()) for b in ddp.grad_buffers()) == 2 * n

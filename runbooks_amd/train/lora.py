@@ -253,7 +253,12 @@ class _LoRAPacked(torch.autograd.Function):
 
 def _packs(members, x) -> bool:
     """True when _LoRAPacked's kernels take these adapters on x, of which the
-    weights have to be side by side in memory (_lay_side_by_side)."""
+    weights have to be side by side in memory (_lay_side_by_side). What never
+    changes comes first: a layer that is refused for its bias or its rank pays
+    for little else."""
+    for m in members:
+        if m.r != 16 or getattr(m.base, "bias", None) is not None:
+            return False
     if not x.is_cuda or x.dtype != torch.bfloat16 or x.dim() != 2 or \
             not x.is_contiguous() or x.data_ptr() % 16 or \
             not 0 < x.shape[0] <= 1 << 22 or _USE_CUSTOM_GEMM or \
@@ -261,11 +266,10 @@ def _packs(members, x) -> bool:
         return False
     for m in members:
         w = m.base.weight
-        if (m.r != 16 or m.scale != members[0].scale or
+        if (m.scale != members[0].scale or
                 (m.dropout is not None and m.training) or
                 not (isinstance(m.base, nn.Linear) or
                      getattr(m.base, "tp", 1) == 1) or
-                getattr(m.base, "bias", None) is not None or
                 w.requires_grad or w.dtype != torch.bfloat16 or
                 not w.is_contiguous() or w.shape[0] % 64 or w.shape[1] % 64 or
                 w.shape[1] != x.shape[1]):

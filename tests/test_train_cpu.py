@@ -441,3 +441,11 @@ def test_gradient_hook_takes_the_same_however_many_wait(n):
         sys.setprofile(None)
     assert len(calls) < 40 * n
     assert sum(int(b.sum()) for b in ddp.grad_buffers()) == 2 * n
+
+
+@pytest.mark.parametrize("bias,r", [(True, 16), (False, 8)])
+def test_adapters_that_never_pack_are_refused_at_once(bias, r):
+    """Without a look at the input, which here has nothing to look at."""
+    from runbooks_amd.train.lora import LoRALinear, _packs
+    layer = LoRALinear(torch.nn.Linear(64, 64, bias=bias), r=r)
+    assert not _packs([layer], None)

@@ -185,9 +185,9 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
       load(vb, kv_stride, (t + 1) * ROWS, S, next + TILE, wid);
     }
   };
-  const int full = wrow / ROWS;         // tiles that every row sees whole
+  const Walk mine = walk(wrow, S);
   int t = 0;
-  for (; t < full; ++t) {
+  for (; t < mine.full; ++t) {
     arrive(t);
     const char *kt = smem + (t & 1) * 2 * TILE;
 #pragma unroll
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
     const char *kt = smem + (t & 1) * 2 * TILE;
 #pragma unroll
     for (int r0 = 0; r0 < ROWS; r0 += 32)
-      if (t * ROWS + r0 <= wrow + 31)
+      if (t * ROWS + r0 <= mine.last)
         keys(kt, kt + TILE, t * ROWS + r0, r0, std::true_type{});
   }
   if (q_valid)

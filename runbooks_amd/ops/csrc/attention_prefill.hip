@@ -236,9 +236,9 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
   };
   // first all-visible tiles, then those on the diagonal, then those that only
   // other waves need
-  const int full = wrow / ROWS;
+  const Walk mine = walk(wrow, S);
   int t = 0;
-  for (; t < full; ++t) {
+  for (; t < mine.full; ++t) {
     arrive(t);
     const char *kt = smem + (t & 1) * 2 * TILE;
 #pragma unroll
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
 #pragma unroll
     for (int i = 0; i < ROWS; i += SUB * 32 * SPLIT) {
       const int r0 = i + part * 32, kbase = t * ROWS + r0;
-      if (kbase <= wrow + 31)
+      if (kbase <= mine.last)
         keys(kt, kt + TILE, kbase, r0, std::true_type{});
     }
   }
@@ -446,6 +446,19 @@ std::vector<at::Tensor> flash_fwd_train_qkv(at::Tensor y, int64_t B, int64_t S,
 at::Tensor flash_prefill(at::Tensor q, at::Tensor k, at::Tensor v,
                          double scale) {
   return flash_fwd_impl(q, k, v, scale, nullptr);
+}
+
+// The walks of the waves of every workgroup of `rows` query rows: {tiles of the
+// workgroup, full, last} each.
+std::vector<std::vector<int64_t>> flash_walks(int64_t S, int64_t rows) {
+  std::vector<std::vector<int64_t>> out;
+  for (int64_t q0 = 0; q0 < S; q0 += rows)
+    for (int64_t w = q0; w < q0 + rows; w += 32) {
+      const Walk k = walk((int)w, (int)S);
+      out.push_back({(std::min(S, q0 + rows) + ROWS - 1) / ROWS, k.full,
+                     k.last});
+    }
+  return out;
 }
 
 // Training forward: additionally returns the per-row log-sum-exp

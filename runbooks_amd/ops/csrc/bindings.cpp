@@ -52,6 +52,7 @@ void qkv_rope_append_(at::Tensor y, at::Tensor cos, at::Tensor sin,
                       at::Tensor positions, at::Tensor k_cache,
                       at::Tensor v_cache, at::Tensor slot_mapping,
                       int64_t hq);
+std::vector<std::vector<int64_t>> flash_walks(int64_t S, int64_t rows);
 at::Tensor flash_prefill(at::Tensor q, at::Tensor k, at::Tensor v, double scale);
 std::vector<at::Tensor> flash_fwd_train(at::Tensor q, at::Tensor k, at::Tensor v,
                                         double scale, bool ordered);
@@ -99,6 +100,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("block_tables"), py::arg("seq_lens"), py::arg("nsplit"),
         py::arg("scale"), py::arg("seq_starts") = py::none());
   m.def("flash_prefill", &flash_prefill, "MFMA flash-attention prefill (causal)");
+  m.def("flash_walks", &flash_walks,
+        "how the waves of the flash kernels walk the tiles (host only)");
   m.def("flash_fwd_train_qkv", &flash_fwd_train_qkv,
         "flash_fwd_train of q, k and v side by side in one tensor");
   m.def("fa_bwd_qkv", &fa_bwd_qkv,

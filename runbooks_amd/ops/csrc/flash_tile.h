@@ -74,6 +74,14 @@ template <int DH, int NW> struct TileLoad {
   }
 };
 
+// How a wave of 32 query rows from `wrow` on walks the tiles of its workgroup,
+// all of which it waits for with the others: `full` tiles that all its rows see
+// whole, then those up to key `last`. Rows past the end see none.
+struct Walk { int full, last; };
+__host__ __device__ constexpr Walk walk(int wrow, int rows) {
+  return wrow < rows ? Walk{wrow / ROWS, wrow + 31} : Walk{0, -1};
+}
+
 // Operand of rows r0 .. r0 + 31 along columns 16 ks .. 16 ks + 15: element e
 // of lane (hi, col) is row r0 + col, column 16 ks + 8 hi + e. r0 % 16 == 0.
 template <int DH>

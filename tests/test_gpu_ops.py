@@ -385,7 +385,9 @@ def test_flash_prefill(B, S, Hq, Hkv, dh):
     (1, 1601, 32, 8, 128, None), (2, 737, 32, 32, 64, None),
     (1, 1313, 32, 32, 256, None),
     # eight waves
-    (1, 1537, 128, 8, 64, None), (3, 1025, 64, 2, 128, None)])
+    (1, 1537, 128, 8, 64, None), (3, 1025, 64, 2, 128, None),
+    (1, 6209, 32, 8, 128, None), (6, 320, 128, 64, 64, None),
+    (6, 288, 128, 64, 128, 0.0)])
 def test_flash_prefill_tiles(B, S, Hq, Hkv, dh, scale):
     """Every split of the rows over waves, at remainders of its tiles, with
     inputs that start off a 16-byte boundary. Weights and result are rounded to

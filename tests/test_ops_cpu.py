@@ -278,3 +278,22 @@ def test_fp8_vt_reference_roundtrip():
     # quantization error itself is bounded (e4m3 rows)
     live = d1.permute(0, 2, 1, 3).reshape(-1, hkv, dh)[:T]
     assert torch.allclose(live, v, atol=0.1, rtol=0.1)
+
+
+@pytest.mark.parametrize("rows", [32, 64, 128, 256])
+def test_flash_waves_wait_for_the_same_tiles(rows):
+    """Every wave of a workgroup of the flash kernels meets the others at each
+    of its tiles and no more: as many barriers, whatever is left of the rows.
+    What it takes as seen whole is, and rows past the end see nothing."""
+    ext = pytest.importorskip("runbooks_amd.ops._hip")
+    for S in range(1, 1100):
+        walks = ext.flash_walks(S, rows)
+        assert len(walks) == -(-S // rows) * rows // 32
+        for i, (tiles, full, last) in enumerate(walks):
+            row = i * 32
+            assert full <= tiles == -(-min(S, row // rows * rows + rows) // 64)
+            if row >= S:
+                assert (full, last) == (0, -1)
+            else:
+                assert full == row // 64 and last == row + 31
+                assert -(-min(S, row + 32) // 64) <= tiles

@@ -165,6 +165,9 @@ class Attention(nn.Module):
             # fused decode hot path: one wide GEMM, then one kernel doing
             # rope(q), rope(k)->cache, v->cache, quantized where the cache is
             y = ops.wide_linear(x, self._qkv_w)
+            if kc.dtype == torch.uint8:     # whole numbers of any type
+                positions = positions.to(torch.int32)
+                slot_mapping = slot_mapping.to(torch.int32)
             q = ops.ext().qkv_rope_append(y, cos, sin, positions, kc, vc,
                                           slot_mapping, self.hq)
         else:

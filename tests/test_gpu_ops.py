@@ -1534,3 +1534,25 @@ def test_prefill_hooks_fire(name):
         got = m(tokens)
     assert len(fired) == 3
     assert (got - want).norm() < 0.03 * want.norm()
+
+
+def test_fp8_decode_takes_positions_of_64_bits():
+    """As rotation and append in launches of their own did."""
+    _assert_hip()
+    from runbooks_amd.models import build_model
+    from runbooks_amd.models.transformer import fuse_for_inference
+    m = fuse_for_inference(build_model("smoke-llama", dtype=torch.bfloat16,
+                                       tp=1, device=DEV).eval())
+    caches = m.alloc_caches(4, DEV, fp8=True)
+    for c in (c for kv in caches for c in kv):
+        c.zero_()
+    i32 = dict(device=DEV, dtype=torch.int32)
+
+    def decode(dtype):
+        return m.decode(torch.tensor([3, 5], device=DEV),
+                        torch.tensor([0, 0], device=DEV, dtype=dtype), caches,
+                        torch.tensor([0, 16], device=DEV, dtype=dtype),
+                        torch.tensor([[0], [1]], **i32),
+                        torch.tensor([1, 1], **i32), nsplit=1)
+
+    assert torch.equal(decode(torch.int64), decode(torch.int32))

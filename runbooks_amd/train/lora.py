@@ -118,13 +118,13 @@ class _LoRAGroupPrep(torch.autograd.Function):
 
 
 class _LoRAGroup:
-    """Shared-input sibling adapters + the per-forward tcat cache (keyed
-    on activation identity; dropped after every member consumed it so no
+    """Shared-input sibling adapters + the per-forward tcat cache (of the
+    input that it holds; dropped after every member consumed it so no
     autograd graph outlives the step)."""
 
     def __init__(self, members):
         self.members = members
-        self._x_id = None
+        self._x = None
         self._t = None
         self._left = 0
 
@@ -136,10 +136,10 @@ class _LoRAGroup:
         return None
 
     def t_for(self, member, x):
-        if self._x_id != id(x) or self._left <= 0:
+        if self._x is not x or self._left <= 0:
             self._t = _LoRAGroupPrep.apply(
                 x, *[m.lora_a for m in self.members])
-            self._x_id = id(x)
+            self._x = x
             self._left = len(self.members)
         i = self.members.index(member)
         off = sum(m.r for m in self.members[:i])
@@ -147,7 +147,7 @@ class _LoRAGroup:
         self._left -= 1
         if self._left == 0:
             self._t = None
-            self._x_id = None
+            self._x = None
         return t
 
 
@@ -337,7 +337,9 @@ class LoRALinear(nn.Module):
 
     def forward(self, x):
         base = self.base
-        if _packs([self], x):
+        group = getattr(self, "_group", None)
+        # siblings run one way: t_for counts on a call of each
+        if all(_packs([m], x) for m in (group.members if group else (self,))):
             return _packed([self], x)
         if self.dropout is not None and self.training:
             # dropout on the adapter input (PEFT semantics) breaks the
@@ -351,7 +353,6 @@ class LoRALinear(nn.Module):
         if (isinstance(base, nn.Linear) or
                 (getattr(base, "tp", 1) == 1 and base.bias is None)) and \
                 x.dim() == 2 and getattr(base, "bias", None) is None:
-            group = getattr(self, "_group", None)
             if group is not None:
                 # shared-input siblings (q/k/v, gate/up): the A-GEMM,
                 # its dA and the t-path dx merge run ONCE per group

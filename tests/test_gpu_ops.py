@@ -1556,3 +1556,30 @@ def test_fp8_decode_takes_positions_of_64_bits():
                         torch.tensor([1, 1], **i32), nsplit=1)
 
     assert torch.equal(decode(torch.int64), decode(torch.int32))
+
+
+@pytest.mark.parametrize("narrow", [32, 64])
+def test_lora_siblings_of_other_widths(narrow):
+    """Sibling adapters of which some could run on the packed kernels and
+    others not: every pass uses its own input, and nothing of it stays."""
+    _assert_hip()
+    from runbooks_amd.train.lora import apply_lora
+    torch.manual_seed(0)
+    net = torch.nn.Module()
+    for name, n in (("q_proj", 64), ("k_proj", narrow), ("v_proj", narrow)):
+        setattr(net, name, torch.nn.Linear(64, n, bias=False))
+    net = net.to(DEV, torch.bfloat16)
+    apply_lora(net, r=16)
+    members = [net.q_proj, net.k_proj, net.v_proj]
+    with torch.no_grad():
+        for m in members:
+            m.lora_b.normal_()
+    for _ in range(4):
+        x = torch.randn(40, 64, device=DEV).bfloat16()
+        for m in members:
+            ref = x.double() @ (m.weight.double().t() + m.scale *
+                                m.lora_a.double().t() @ m.lora_b.double().t())
+            # t and the result are rounded, the latter twice at most
+            assert (m(x) - ref).norm() < 2 ** -7 * ref.norm()
+        assert m._group._t is None
+        del x

@@ -240,6 +240,8 @@ class _LoRAPacked(torch.autograd.Function):
         x, w, t, *ab = ctx.saved_tensors
         As, Bs = list(ab[:n]), list(ab[n:])
         dy = dy.contiguous()
+        if dy.data_ptr() % 16:      # a caller's own gradient may start anywhere
+            dy = dy.clone()
         widths = [b.shape[0] for b in Bs]
         dt = ext.lora_down_columns(dy, Bs, ctx.scale)
         db = ext.lora_grad(dy, t, widths, ctx.scale, False).split(widths)

@@ -1583,3 +1583,19 @@ def test_lora_siblings_of_other_widths(narrow):
             assert (m(x) - ref).norm() < 2 ** -7 * ref.norm()
         assert m._group._t is None
         del x
+
+
+def test_lora_packed_takes_any_gradient():
+    """A gradient that starts off a 16-byte boundary."""
+    _assert_hip()
+    from runbooks_amd.train.lora import LoRALinear
+    torch.manual_seed(0)
+    layer = LoRALinear(torch.nn.Linear(64, 128, bias=False).to(
+        DEV, torch.bfloat16), r=16)
+    with torch.no_grad():
+        layer.lora_b.normal_()
+    x = torch.randn(40, 64, device=DEV).bfloat16().requires_grad_()
+    dy = torch.randn(40 * 128 + 1, device=DEV).bfloat16()[1:].view(40, 128)
+    grads = [torch.autograd.grad(layer(x), (x, layer.lora_a, layer.lora_b), g)
+             for g in (dy, dy.clone())]
+    assert all(torch.equal(a, b) for a, b in zip(*grads))

@@ -287,6 +287,14 @@ __global__ __launch_bounds__(256) void lora_grad_kernel(
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     char *buf = smem + ((b - b0) & 1) * BUF;
+    if ((b + 1) * 128 > T) {
+      // rows past the end, which m's zeros would not hide if the last row,
+      // which they repeat, is not finite
+      for (int at = (int)(T - b * 128) * 128 + tid * 16; at < 2 * TILE;
+           at += 256 * 16)
+        *reinterpret_cast<uint4 *>(buf + at) = make_uint4(0, 0, 0, 0);
+      __syncthreads();
+    }
     if (b + 1 < b1) send(b + 1, smem + ((b - b0 + 1) & 1) * BUF);
     const char *tile = buf + (wid >> 1) * TILE;
 #pragma unroll

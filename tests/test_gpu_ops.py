@@ -1599,3 +1599,25 @@ def test_lora_packed_takes_any_gradient():
     grads = [torch.autograd.grad(layer(x), (x, layer.lora_a, layer.lora_b), g)
              for g in (dy, dy.clone())]
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+@pytest.mark.parametrize("T", [1, 63, 130, 256])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_lora_grad_of_infinite_rows(T, transposed):
+    """An infinite value in the last row is infinite in its column's sums, and
+    in no other's."""
+    _assert_hip()
+    torch.manual_seed(T)
+    x = torch.randn(T, 128, device=DEV).bfloat16()
+    x[-1, 70] = float("inf")
+    t = torch.randn(2, T, 16, device=DEV).bfloat16()
+    got = ops.ext().lora_grad(x, t, [64, 64], 1.0, transposed).double()
+    if transposed:
+        ref = torch.cat([m.double().t() @ x.double() for m in t])
+    else:
+        ref = torch.cat([x[:, i * 64:i * 64 + 64].double().t() @ t[i].double()
+                         for i in range(2)])
+    assert torch.equal(got.isinf(), ref.isinf()) and not got.isnan().any()
+    assert torch.equal(got.sign()[got.isinf()], ref.sign()[ref.isinf()])
+    assert ((got - ref)[ref.isfinite()].norm() <
+            2 ** -8 * ref[ref.isfinite()].norm())

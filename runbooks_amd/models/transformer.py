@@ -487,18 +487,23 @@ class Transformer(nn.Module):
     def _sums_in_layer_norms(self, x) -> bool:
         """The residual may be kept in fp32 and added to in the kernels of the
         layer norms (results that are not differentiated)."""
-        return (x.is_cuda and x.dtype == torch.bfloat16 and
+        if not (x.is_cuda and x.dtype == torch.bfloat16 and
                 not torch.is_grad_enabled() and self.cfg.norm == "layernorm" and
                 not self.cfg.parallel_residual and not self.cfg.single_norm and
-                x.dim() == 2 and len(self.blocks) > 0 and
-                plain(Block, *self.blocks) and
-                all(plain(nn.LayerNorm, n) and n.weight is not None and
-                    n.bias is not None and n.weight.dtype == x.dtype
-                    for n in self._layer_norms()))
+                x.dim() == 2 and len(self.blocks) > 0):
+            return False
+        norms = self._layer_norms()
+        return (plain(Block, *self.blocks) and plain(nn.LayerNorm, *norms) and
+                all(p["weight"] is not None and p["bias"] is not None and
+                    p["weight"].dtype == x.dtype
+                    for p in (n._parameters for n in norms)))
 
     def _layer_norms(self):
-        return [n for blk in self.blocks for n in (blk.norm1, blk.norm2)] + \
-            [self.norm_f]
+        # of every pass: without nn.Module's search for attributes
+        norms = [m[name] for m in (blk._modules for blk in self.blocks)
+                 for name in ("norm1", "norm2")]
+        norms.append(self.norm_f)
+        return norms
 
     def _last_norm(self, x, delta):
         if delta is None:

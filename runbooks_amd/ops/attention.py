@@ -34,14 +34,14 @@ class _FlashAttnTrain(torch.autograd.Function):
         out, lse = _backend.ext().flash_fwd_train(qc, kc, vc, float(scale),
                                                   ordered)
         ctx.save_for_backward(qc, kc, vc, out, lse)
-        ctx.scale = float(scale)
+        ctx.scale, ctx.ordered = float(scale), ordered
         return out
 
     @staticmethod
     def backward(ctx, dout):
         q, k, v, out, lse = ctx.saved_tensors
         dq, dk, dv = _backend.ext().fa_bwd(dout.contiguous(), q, k, v, out,
-                                           lse, ctx.scale)
+                                           lse, ctx.scale, ctx.ordered)
         hq, hkv = q.shape[2], k.shape[2]
         if hkv != hq:  # sum the q-head group (GQA/MQA)
             g = hq // hkv
@@ -86,8 +86,8 @@ def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                      scale: float | None = None, q_block: int = 256,
                      ordered: bool = False) -> torch.Tensor:
     """q [B, S, Hq, Dh]; k, v [B, S, Hkv, Dh] -> [B, S, Hq, Dh]. ``ordered``:
-    heads of 64 add and round in the one order that models keep whose
-    gradients jump with the forward's roundings (ReLU).
+    heads of 64 add and round in the one order, forward and backward, that
+    models keep whose gradients jump with the roundings (ReLU).
 
     Differentiable. GPU bf16 (Dh 64/128) runs the MFMA flash kernels;
     otherwise the chunked fp32 reference below (also the numerics oracle

@@ -59,15 +59,6 @@ struct Args {
   float scale;
 };
 
-// Eight values of two score tiles' registers -> a B operand.
-RB_DEV bf16x8v operand(const f32x16v &p, int ks) {
-  union { unsigned u[4]; bf16x8v v; } c;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    c.u[i] = pack2(p[ks * 8 + 2 * i], p[ks * 8 + 2 * i + 1]);
-  return c.v;
-}
-
 // A row's operands along DH, from memory.
 template <int DH>
 RB_DEV void load_row(bf16x8v *f, const uint16_t *row, int hi) {
@@ -101,7 +92,12 @@ RB_DEV void clear_if(bool yes, bf16x8v *f) {
   for (int ks = 0; ks < DH / 16; ++ks) f[ks] = (bf16x8v)(__bf16)0.0f;
 }
 
-template <int DH, int NW>
+// ORDERED: the counterpart of the ordered forward (attention_prefill.hip), with
+// one order of its roundings too, as gradients make the next step's weights:
+// rows in their own order, natural exponentials of scores less LSE, dP less D,
+// each dS times the factor, D summed by quarters of a row. us, both kernels, 12
+// heads of 64, 4 x 512 and 2047 tokens: 32 and 91, otherwise 28 and 77.
+template <int DH, int NW, bool ORDERED>
 __global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
   constexpr int KSTEPS = DH / 16, DTILES = DH / 32;
   constexpr int QT = NW * 32, TILE = tile_bytes<DH>();
@@ -133,17 +129,36 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
   clear_if<DH>(a.scale == 0.0f, qf);
   load_row<DH>(dof, a.dout + row0, hi);
   float dvec = 0.0f;
+  if constexpr (ORDERED) {
+    float part[4];
 #pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) {
-    const bf16x8v o = *reinterpret_cast<const bf16x8v *>(
-        a.out + row0 + ks * 16 + hi * 8);
+    for (int c = 0; c < 4; ++c) {
+      part[c] = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) dvec += (float)o[e] * (float)dof[ks][e];
+      for (int v = 0; v < DH / 32; ++v) {
+        float o[8], d[8];
+        rb::VIO<uint16_t>::load(a.out + row0 + c * (DH / 4) + v * 8, o);
+        rb::VIO<uint16_t>::load(a.dout + row0 + c * (DH / 4) + v * 8, d);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part[c] += o[e] * d[e];
+      }
+    }
+    dvec = (part[0] + part[1]) + (part[2] + part[3]);
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+      const bf16x8v o = *reinterpret_cast<const bf16x8v *>(
+          a.out + row0 + ks * 16 + hi * 8);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dvec += (float)o[e] * (float)dof[ks][e];
+    }
+    dvec += __shfl_xor(dvec, 32, 64);
   }
-  dvec += __shfl_xor(dvec, 32, 64);
   if (q_valid && hi == 0) a.dvec[stat] = dvec;
   const float by = unit(a.scale), to2 = by * LOG2E;
-  const float s0 = q_valid ? -a.lse[stat] / by : 0.0f;
+  const float lse = q_valid ? a.lse[stat] : 0.0f;
+  const float s0 = ORDERED ? 0.0f : -lse / by;
+  const float d0 = ORDERED ? 0.0f : -dvec;
 
   f32x16v acc[DTILES];
 #pragma unroll
@@ -151,7 +166,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
 
   auto keys = [&](const char *kt, const char *vt, int kbase, int r0,
                   auto masked) {
-    f32x16v s = (f32x16v)(s0), dp = (f32x16v)(-dvec);
+    f32x16v s = (f32x16v)(s0), dp = (f32x16v)(d0);
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
       s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
@@ -161,18 +176,20 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      float p = __builtin_amdgcn_exp2f(s[r] * to2);
+      float p = ORDERED ? __expf(s[r] * by - lse)
+                        : __builtin_amdgcn_exp2f(s[r] * to2);
       if constexpr (decltype(masked)::value)
         if (kbase + (r & 3) + 8 * (r >> 2) + 4 * hi > qrow) p = 0.0f;
-      s[r] = p * dp[r];
+      s[r] = ORDERED ? p * (dp[r] - dvec) * a.scale : p * dp[r];
     }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      const bf16x8v ds = operand(s, ks);
+      const bf16x8v ds = score_frag<ORDERED>(s, ks);
 #pragma unroll
       for (int dt = 0; dt < DTILES; ++dt)
         acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            column_frag<DH>(kt, r0 + ks * 16, dt, lane), ds, acc[dt], 0, 0, 0);
+            column_frag<DH, ORDERED>(kt, r0 + ks * 16, dt, lane), ds, acc[dt],
+            0, 0, 0);
     }
   };
   // waits for tile t and sends for the next one
@@ -203,10 +220,11 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
         keys(kt, kt + TILE, t * ROWS + r0, r0, std::true_type{});
   }
   if (q_valid)
-    store_row<DH>(a.dq + token * a.dq_stride + at.head * DH, acc, a.scale, hi);
+    store_row<DH>(a.dq + token * a.dq_stride + at.head * DH, acc,
+                  ORDERED ? 1.0f : a.scale, hi);
 }
 
-template <int DH, int NW>
+template <int DH, int NW, bool ORDERED>
 __global__ __launch_bounds__(NW * 64, DH == 128 ? 1 : 2)
 void fa_bwd_dkdv_kernel(Args a) {
   constexpr int KSTEPS = DH / 16, DTILES = DH / 32;
@@ -244,8 +262,12 @@ void fa_bwd_dkdv_kernel(Args a) {
   auto stat_of = [&](int t) {
     const int row = t * ROWS + (tid & 63);
     if (tid >= 2 * ROWS) return 0.0f;
-    if (tid >= ROWS) return row < S ? -a.dvec[stat + row] : 0.0f;
     // rows past the end: weights of zero
+    if constexpr (ORDERED) {
+      if (tid >= ROWS) return row < S ? a.dvec[stat + row] : 0.0f;
+      return row < S ? a.lse[stat + row] : INFINITY;
+    }
+    if (tid >= ROWS) return row < S ? -a.dvec[stat + row] : 0.0f;
     return row < S ? -a.lse[stat + row] / by : by < 0.0f ? INFINITY
                                                          : -INFINITY;
   };
@@ -275,17 +297,21 @@ void fa_bwd_dkdv_kernel(Args a) {
   auto queries = [&](const char *qt, const float *st, int qbase, int r0,
                      auto masked) {
     const char *ot = qt + TILE;
-    f32x16v s, dp;
+    f32x16v s = (f32x16v)(0.0f), dp = (f32x16v)(0.0f), lse, dvec;
 #pragma unroll
     for (int rq = 0; rq < 4; ++rq) {
       const float4 l = *reinterpret_cast<const float4 *>(
           st + r0 + 8 * rq + 4 * hi);
       const float4 d = *reinterpret_cast<const float4 *>(
           st + ROWS + r0 + 8 * rq + 4 * hi);
-      s[rq * 4] = l.x; s[rq * 4 + 1] = l.y;
-      s[rq * 4 + 2] = l.z; s[rq * 4 + 3] = l.w;
-      dp[rq * 4] = d.x; dp[rq * 4 + 1] = d.y;
-      dp[rq * 4 + 2] = d.z; dp[rq * 4 + 3] = d.w;
+      lse[rq * 4] = l.x; lse[rq * 4 + 1] = l.y;
+      lse[rq * 4 + 2] = l.z; lse[rq * 4 + 3] = l.w;
+      dvec[rq * 4] = d.x; dvec[rq * 4 + 1] = d.y;
+      dvec[rq * 4 + 2] = d.z; dvec[rq * 4 + 3] = d.w;
+    }
+    if constexpr (!ORDERED) {
+      s = lse;
+      dp = dvec;
     }
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
@@ -296,23 +322,25 @@ void fa_bwd_dkdv_kernel(Args a) {
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      float p = __builtin_amdgcn_exp2f(s[r] * to2);
+      float p = ORDERED ? __expf(s[r] * by - lse[r])
+                        : __builtin_amdgcn_exp2f(s[r] * to2);
       if constexpr (decltype(masked)::value)
         if (qbase + (r & 3) + 8 * (r >> 2) + 4 * hi < key) p = 0.0f;
       s[r] = p;
-      dp[r] *= p;
+      dp[r] = ORDERED ? p * (dp[r] - dvec[r]) * a.scale : dp[r] * p;
     }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      const bf16x8v pf = operand(s, ks), dsf = operand(dp, ks);
+      const bf16x8v pf = score_frag<ORDERED>(s, ks);
+      const bf16x8v dsf = score_frag<ORDERED>(dp, ks);
 #pragma unroll
       for (int dt = 0; dt < DTILES; ++dt) {
         acc_dv[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            column_frag<DH>(ot, r0 + ks * 16, dt, lane), pf, acc_dv[dt],
-            0, 0, 0);
+            column_frag<DH, ORDERED>(ot, r0 + ks * 16, dt, lane), pf,
+            acc_dv[dt], 0, 0, 0);
         acc_dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            column_frag<DH>(qt, r0 + ks * 16, dt, lane), dsf, acc_dk[dt],
-            0, 0, 0);
+            column_frag<DH, ORDERED>(qt, r0 + ks * 16, dt, lane), dsf,
+            acc_dk[dt], 0, 0, 0);
       }
     }
   };
@@ -341,41 +369,45 @@ void fa_bwd_dkdv_kernel(Args a) {
 
   if (k_valid) {
     const int64_t row0 = (token0 + key) * a.dkv_stride + at.head * DH;
-    store_row<DH>(a.dk + row0, acc_dk, a.scale, hi);
+    store_row<DH>(a.dk + row0, acc_dk, ORDERED ? 1.0f : a.scale, hi);
     store_row<DH>(a.dv + row0, acc_dv, 1.0f, hi);
   }
 }
 
-template <int DH, int NW> void launch_bwd(const Args &a, hipStream_t stream) {
+template <int DH, int NW, bool ORDERED = false>
+void launch_bwd(const Args &a, hipStream_t stream) {
   constexpr size_t sh_dq = 4 * tile_bytes<DH>();
   constexpr size_t sh_dkdv = sh_dq + 2 * ROWS * 4 * 2;
   static const bool once =
       hipFuncSetAttribute(
-          reinterpret_cast<const void *>(&fa_bwd_dq_kernel<DH, NW>),
+          reinterpret_cast<const void *>(&fa_bwd_dq_kernel<DH, NW, ORDERED>),
           hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh_dq) ==
           hipSuccess &&
       hipFuncSetAttribute(
-          reinterpret_cast<const void *>(&fa_bwd_dkdv_kernel<DH, NW>),
+          reinterpret_cast<const void *>(&fa_bwd_dkdv_kernel<DH, NW, ORDERED>),
           hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh_dkdv) ==
           hipSuccess;
   TORCH_CHECK(once, "fa_bwd: LDS size");
   const int64_t grid =
       (int64_t)((a.S + NW * 32 - 1) / (NW * 32)) * a.Hq * a.B;
   TORCH_CHECK(grid < (int64_t)1 << 31, "fa_bwd: grid");
-  hipLaunchKernelGGL((fa_bwd_dq_kernel<DH, NW>), dim3((unsigned)grid),
+  hipLaunchKernelGGL((fa_bwd_dq_kernel<DH, NW, ORDERED>), dim3((unsigned)grid),
                      dim3(NW * 64), sh_dq, stream, a);
-  hipLaunchKernelGGL((fa_bwd_dkdv_kernel<DH, NW>), dim3((unsigned)grid),
+  hipLaunchKernelGGL((fa_bwd_dkdv_kernel<DH, NW, ORDERED>), dim3((unsigned)grid),
                      dim3(NW * 64), sh_dkdv, stream, a);
 }
 
-void launch_bwd(int64_t DH, const Args &a) {
+void launch_bwd(int64_t DH, const Args &a, bool ordered = false) {
   auto stream = at::hip::getCurrentHIPStream();
   // Workgroups of two waves while there are too few tiles of 32 rows for four
   // waves on every CU (us for 2 and 4 waves: 200 tokens, 12 heads of 64, 84
   // tiles, 17 and 19; 512 tokens, 32 heads of 128, 512 tiles, 48 and 50; four
   // times those 81 and 79).
   const bool few = (int64_t)(a.S + 31) / 32 * a.Hq * a.B <= 512;
-  if (DH == 128)
+  if (ordered)
+    few ? launch_bwd<64, 2, true>(a, stream)
+        : launch_bwd<64, 4, true>(a, stream);
+  else if (DH == 128)
     few ? launch_bwd<128, 2>(a, stream) : launch_bwd<128, 4>(a, stream);
   else
     few ? launch_bwd<64, 2>(a, stream) : launch_bwd<64, 4>(a, stream);
@@ -389,7 +421,7 @@ void launch_bwd(int64_t DH, const Args &a) {
 
 std::vector<at::Tensor> fa_bwd(at::Tensor dout, at::Tensor q, at::Tensor k,
                                at::Tensor v, at::Tensor out, at::Tensor lse,
-                               double scale) {
+                               double scale, bool ordered) {
   TORCH_CHECK(q.is_cuda() && q.is_contiguous() && k.is_contiguous() &&
               v.is_contiguous() && dout.is_contiguous() && out.is_contiguous(),
               "fa_bwd: contiguous GPU tensors");
@@ -397,7 +429,8 @@ std::vector<at::Tensor> fa_bwd(at::Tensor dout, at::Tensor q, at::Tensor k,
   const int B = (int)q.size(0), S = (int)q.size(1), Hq = (int)q.size(2),
             DH = (int)q.size(3);
   const int Hkv = (int)k.size(2);
-  TORCH_CHECK(DH == 64 || DH == 128, "fa_bwd: DH must be 64 or 128");
+  TORCH_CHECK(DH == 64 || (DH == 128 && !ordered),
+              "fa_bwd: DH must be 64 or 128, ordered 64");
   TORCH_CHECK(lse.scalar_type() == at::kFloat && lse.is_contiguous() &&
               lse.numel() == (int64_t)B * Hq * S, "fa_bwd: lse [B, Hq, S]");
   TORCH_CHECK(Hkv > 0 && Hq % Hkv == 0 &&
@@ -435,7 +468,7 @@ std::vector<at::Tensor> fa_bwd(at::Tensor dout, at::Tensor q, at::Tensor k,
   a.scale = (float)scale;
   a.q_stride = a.dq_stride = a.dkv_stride = (int64_t)Hq * DH;
   a.kv_stride = (int64_t)Hkv * DH;
-  launch_bwd(DH, a);
+  launch_bwd(DH, a, ordered);
   return {dq, dk, dv};
 }
 

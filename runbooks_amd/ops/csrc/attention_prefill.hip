@@ -171,19 +171,11 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
       }
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        // the halves of the wave exchange the middle keys of 16
-        unsigned w[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          w[i] = pack2(s[0][ks * 8 + 2 * i], s[0][ks * 8 + 2 * i + 1]);
-        auto w02 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
-        auto w13 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
-        union { unsigned u[4]; bf16x8v v; } pf;
-        pf.u[0] = w02[0]; pf.u[1] = w13[0]; pf.u[2] = w02[1]; pf.u[3] = w13[1];
+        const bf16x8v pf = score_frag<true>(s[0], ks);
 #pragma unroll
         for (int dt = 0; dt < DTILES; ++dt)
           acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              column_frag<DH, true>(vt, r0 + ks * 16, dt, lane), pf.v,
+              column_frag<DH, true>(vt, r0 + ks * 16, dt, lane), pf,
               acc_o[dt], 0, 0, 0);
       }
       return;
@@ -211,14 +203,11 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
       }
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        union { unsigned u[4]; bf16x8v v; } pf;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          pf.u[i] = pack2(s[u][ks * 8 + 2 * i], s[u][ks * 8 + 2 * i + 1]);
+        const bf16x8v pf = score_frag(s[u], ks);
 #pragma unroll
         for (int dt = 0; dt < DTILES; ++dt)
           acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              column_frag<DH>(vt, r0 + u * 32 + ks * 16, dt, lane), pf.v,
+              column_frag<DH>(vt, r0 + u * 32 + ks * 16, dt, lane), pf,
               acc_o[dt], 0, 0, 0);
       }
     }

@@ -58,7 +58,7 @@ std::vector<at::Tensor> flash_fwd_train(at::Tensor q, at::Tensor k, at::Tensor v
                                         double scale, bool ordered);
 std::vector<at::Tensor> fa_bwd(at::Tensor dout, at::Tensor q, at::Tensor k,
                                at::Tensor v, at::Tensor out, at::Tensor lse,
-                               double scale);
+                               double scale, bool ordered);
 at::Tensor swiglu_fwd(at::Tensor g, at::Tensor u);
 std::vector<at::Tensor> swiglu_bwd(at::Tensor dy, at::Tensor g, at::Tensor u);
 std::vector<at::Tensor> cross_entropy_fwd(at::Tensor logits, at::Tensor targets,
@@ -127,7 +127,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("k"), py::arg("v"), py::arg("scale"),
         py::arg("ordered") = false);
   m.def("fa_bwd", &fa_bwd,
-        "MFMA flash-attention backward -> (dq, dk_perq, dv_perq)");
+        "MFMA flash-attention backward -> (dq, dk_perq, dv_perq)", py::arg("dout"),
+        py::arg("q"), py::arg("k"), py::arg("v"), py::arg("out"),
+        py::arg("lse"), py::arg("scale"), py::arg("ordered") = false);
   m.def("swiglu_fwd", &swiglu_fwd, "fused silu(g)*u");
   m.def("swiglu_bwd", &swiglu_bwd, "fused SwiGLU backward");
   m.def("cross_entropy_fwd", &cross_entropy_fwd, "fused CE: per-row loss + lse");

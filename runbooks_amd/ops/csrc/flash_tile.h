@@ -106,6 +106,25 @@ RB_DEV bf16x8v column_frag(const char *tile, int r0, int dt, int lane) {
   return rb::lds_column8(lo, up);
 }
 
+// Eight values of a score tile's registers -> the other operand: rows in the order
+// of the registers, as column_frag takes them; PLAIN: in their own, for which
+// the halves of the wave exchange the middle ones of 16.
+template <bool PLAIN = false>
+RB_DEV bf16x8v score_frag(const f32x16v &p, int ks) {
+  union { unsigned u[4]; bf16x8v v; } c;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    c.u[i] = pack2(p[ks * 8 + 2 * i], p[ks * 8 + 2 * i + 1]);
+  if constexpr (PLAIN) {
+    const auto a = __builtin_amdgcn_permlane32_swap(c.u[0], c.u[2], false,
+                                                    false);
+    const auto b = __builtin_amdgcn_permlane32_swap(c.u[1], c.u[3], false,
+                                                    false);
+    c.u[0] = a[0]; c.u[1] = b[0]; c.u[2] = a[1]; c.u[3] = b[1];
+  }
+  return c.v;
+}
+
 // Workgroup -> (tile, head, batch). Tiles of a causal triangle differ in
 // length: the longest come first. The heads of one key/value head stay on one
 // XCD, whose L2 then holds their keys, when those heads divide by the XCDs.

@@ -424,33 +424,47 @@ def _hashed(n, salt):
 
 
 @pytest.mark.parametrize("B,S,Hq,Hkv,bits", [
-    (1, 1, 1, 1, (4093165637, 932004135)),
-    (2, 31, 3, 3, (2980831709, 3346004597)),
-    (1, 64, 4, 2, (3987702248, 4086934317)),
-    (1, 65, 12, 12, (329763779, 1455785953)),
-    (2, 257, 12, 12, (1483102084, 2568763203)),
-    (1, 300, 4, 1, (2206580616, 3272915928)),
-    (1, 1021, 12, 12, (277277627, 2214567642))])
+    (1, 1, 1, 1, (4093165637, 932004135, 3265854109, 3265854109, 34914089)),
+    (2, 31, 3, 3, (2980831709, 3346004597, 2951792153, 627292471,
+                   1842450457)),
+    (1, 64, 4, 2, (3987702248, 4086934317, 3359148874, 2069512852,
+                   558976727)),
+    (1, 65, 12, 12, (329763779, 1455785953, 2509830808, 4046418718,
+                     123667421)),
+    (2, 257, 12, 12, (1483102084, 2568763203, 2368670429, 1348113486,
+                      3775892656)),
+    (1, 300, 4, 1, (2206580616, 3272915928, 1571533394, 3616146700,
+                    1162676308)),
+    (1, 1021, 12, 12, (277277627, 2214567642, 3491892497, 2225167499,
+                       4002099437))])
 def test_flash_ordered_bits(B, S, Hq, Hkv, bits):
-    """The training forward of ReLU models does not change a bit of its
-    results (CRCs of them and of the log-sum-exp): their gradients would."""
+    """The attention that ReLU models train on does not change a bit of its
+    result, log-sum-exp and gradients (their CRCs), as the model's gradients
+    and the weights of later steps would follow."""
     _assert_hip()
-    q, k, v = (_hashed(B * S * h * 64, salt).view(B, S, h, 64).bfloat16()
-               .to(DEV) for salt, h in ((1, Hq), (2, Hkv), (3, Hkv)))
+    q, k, v, dout = (_hashed(B * S * h * 64, salt).view(B, S, h, 64)
+                     .bfloat16().to(DEV).requires_grad_()
+                     for salt, h in ((1, Hq), (2, Hkv), (3, Hkv), (4, Hq)))
     out, lse = ops.ext().flash_fwd_train(q, k, v, 0.125, ordered=True)
-    assert bits == tuple(zlib.crc32(x.cpu().numpy().tobytes())
-                         for x in (out.view(torch.int16), lse))
-    assert torch.equal(out, ops.causal_attention(q, k, v, ordered=True))
+    grads = ops.ext().fa_bwd(dout, q, k, v, out, lse, 0.125, ordered=True)
+    crc = [zlib.crc32(x.detach().cpu().numpy().tobytes()) for x in
+           (out.view(torch.int16), lse, *(g.view(torch.int16)
+                                          for g in grads))]
+    assert tuple(crc) == bits
+    y = ops.causal_attention(q, k, v, ordered=True)
+    y.backward(dout.detach())
+    assert torch.equal(y, out) and torch.equal(q.grad, grads[0])
 
 
 @pytest.mark.parametrize("S,scale", [(97, None), (200, -0.1), (130, 0.0),
                                      (33, 0.3)])
 def test_flash_ordered(S, scale):
-    """As test_flash_prefill_tiles, with any factor."""
+    """As test_flash_prefill_tiles and test_flash_attention_bwd_tiles, with any
+    factor."""
     _assert_hip()
     g = torch.Generator(device=DEV).manual_seed(S)
-    q, k, v = (torch.randn(2, S, h, 64, generator=g, device=DEV).bfloat16()
-               for h in (6, 3, 3))
+    q, k, v, dout = (torch.randn(2, S, h, 64, generator=g, device=DEV)
+                     .bfloat16() for h in (6, 3, 3, 6))
     scale = 0.125 if scale is None else scale
     out, lse = ops.ext().flash_fwd_train(q, k, v, scale, ordered=True)
     ref = q.double().transpose(1, 2) @ k.double().repeat_interleave(
@@ -458,9 +472,20 @@ def test_flash_ordered(S, scale):
     ref.masked_fill_(torch.ones(S, S, dtype=torch.bool, device=DEV).triu(1),
                      float("-inf"))
     assert (lse - ref.logsumexp(-1)).abs().max() < 1e-5
-    ref = ref.softmax(-1) @ v.double().repeat_interleave(2, 2).transpose(
+    p, vs = ref.softmax(-1), v.double().repeat_interleave(2, 2).transpose(
         1, 2).contiguous()
+    ref = p @ vs
     assert (out.transpose(1, 2) - ref).norm() < 2 ** -8 * ref.norm()
+    got = ops.ext().fa_bwd(dout, q, k, v, out, lse, scale, ordered=True)
+    for b in range(2):
+        for h in range(6):
+            qs, ks, do, o = (x[b, :, i].double() for x, i in (
+                (q, h), (k, h // 2), (dout, h), (out, h)))
+            w = p[b, h]
+            ds = w * (do @ vs[b, h].t() -
+                      (do * o).sum(-1, keepdim=True)) * scale
+            for x, r in zip(got, (ds @ ks, ds.t() @ qs, w.t() @ do)):
+                assert (x[b, :, h] - r).norm() <= 2 ** -7 * r.norm()
 
 
 @pytest.mark.parametrize("B,S,Hq,Hkv,dh,scale", [

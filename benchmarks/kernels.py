@@ -200,16 +200,18 @@ def main():
 
     # fp8 decode GEMM
     from runbooks_amd.ops.linear import quantize_fp8
-    xs = torch.randn(32, 4096, dtype=bf16, device=dev)
+    xs = ops.ext().decode_swizzle_x(
+        torch.randn(32, 4096, dtype=bf16, device=dev))
     qs = [quantize_fp8(torch.randn(12288, 4096, dtype=bf16, device=dev))
           for _ in range(10)]
+    qs = [(ops.ext().decode_swizzle_w8(w8), scale) for w8, scale in qs]
     i = [0]
 
     def fp8():
         i[0] = (i[0] + 1) % 10
-        return ops.ext().skinny_gemm_fp8(xs, *qs[i[0]])
+        return ops.ext().decode_gemm_fp8(xs, *qs[i[0]], 32, 12288, 4096)
     us = timeit(fp8)
-    out.append(row("skinny_fp8_decode", "32x12288x4096", us, 12288 * 4096,
+    out.append(row("decode_gemm_fp8", "32x12288x4096", us, 12288 * 4096,
                    flops=2 * 32 * 12288 * 4096))
 
     # train GEMM shapes (hipBLASLt, fresh weights)

@@ -930,9 +930,9 @@ def fuse_for_inference(model: "Transformer",
     if load_in_8bit and torch.cuda.is_available():
         # MODEL_LOAD_IN_8BIT: decode weights additionally stored as OCP
         # e4m3 + per-channel scales — the decode GEMM streams half the
-        # bytes (ops/csrc/skinny_gemm.hip fp8 path). bf16 masters stay for
-        # prefill/big-M GEMMs: 288 GB HBM3E makes both-copies the right
-        # trade on MI355X.
+        # bytes (ops/csrc/decode_gemm.hip, decode_gemm_fp8). bf16 masters
+        # stay for prefill/big-M GEMMs: 288 GB HBM3E makes both-copies the
+        # right trade on MI355X.
         from ..ops.linear import quantize_fp8
         for w in weights:
             if w.shape[0] % 64 == 0 and w.shape[1] % 256 == 0:

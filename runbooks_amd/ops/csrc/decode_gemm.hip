@@ -349,7 +349,7 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_affine_kernel(
     *reinterpret_cast<uint64_t *>(dst) = *reinterpret_cast<uint64_t *>(o);
 }
 
-// 33 to 128 rows (RB blocks of 32): x is longer than W's share of a workgroup, so
+// 17 to 128 rows (RB blocks of 32): x is longer than W's share of a workgroup, so
 // NWN waves with blocks of 32 rows of W of their own share its tiles, in LDS, as
 // they are in memory; 4 / NWN such groups take parts of the sums. A chunk is CH
 // steps of 16 columns: W's next chunk and x's are on their way, in registers,

@@ -1,4 +1,4 @@
-"""Linear dispatch: route decode-shaped matmuls to the skinny GEMM.
+"""Linear dispatch: route decode-shaped matmuls to the decode GEMM.
 
 Decode GEMMs and others of up to 128 rows are weight-bandwidth bound;
 csrc/decode_gemm.hip streams W at HBM rate where hipBLASLt's tiles

@@ -1,13 +1,18 @@
 """LoRA adapters (Hu et al. 2021) over the transformer's linear layers.
 
 The reference platform's fine-tune path is LoRA via the external HF
-trainer image (reference examples/llama2-7b/finetuned-model.yaml,
-SURVEY.md §2b "trainer image"); here it is native: frozen base weights,
-trainable low-rank A/B pairs on the attention + MLP projections. The
-fused fwd+bwd path (_LoRAFused) keeps every product a single hipBLASLt
-call and rides both gradient merges on addmm epilogues — no separate
-mul/add kernels (the eager formulation measured ~450 extra elementwise
-launches per llama2-7b step; profiles/).
+trainer image (reference examples/llama2-7b/finetuned-model.yaml); here it
+is native: frozen base weights, trainable low-rank A/B pairs on the
+attention + MLP projections. Three ways, by what a layer is:
+
+* rank 16, bf16, no bias, on the GPU (_LoRAPacked): siblings that share
+  their input side by side, one library product with the frozen weights
+  each way, the adapters' products on kernels of csrc/lora_group.hip that
+  read x, y and dy once for all of them;
+* other layers without bias (_LoRAFused, _LoRAFusedT): library products,
+  both gradient merges in place (the eager formulation measured ~450 extra
+  elementwise launches per llama2-7b step);
+* the rest (bias, dropout, sharded): the composite, by autograd.
 """
 from __future__ import annotations
 

@@ -644,6 +644,25 @@ def test_skinny_gemm_fp8():
     _FP8_REGISTRY.clear()
 
 
+@pytest.mark.parametrize("m", [1, 16, 32])
+def test_fp8_weights_as_served(m):
+    """The e4m3 weights that models run on, through the dispatch: one rounding
+    of the product with the dequantized ones."""
+    _assert_hip()
+    from runbooks_amd.ops.linear import (decode_linear_raw, dequantize_fp8,
+                                         quantize_fp8)
+    torch.manual_seed(m)
+    x = torch.randn(m, 1024, device=DEV).bfloat16()
+    w = torch.randn(4096, 1024, device=DEV).bfloat16()
+    deq = dequantize_fp8(*quantize_fp8(w), dtype=torch.float32)
+    ref = x.double() @ deq.double().t()
+    with torch.no_grad():
+        raw = decode_linear_raw(x, w)[0].double()
+        for y in (ops.fast_linear(x, w), raw.sum(0) if raw.dim() == 3
+                  else raw):
+            assert (y - ref).norm() < 2 ** -8 * ref.norm()
+
+
 _EXPERIMENTAL = __import__("os").environ.get("RB_EXPERIMENTAL") == "1"
 
 

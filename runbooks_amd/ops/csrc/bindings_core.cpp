@@ -32,7 +32,28 @@ int64_t decode_gemm_split(int64_t N, int64_t K);
 bool decode_gemm_supported(int64_t M, int64_t N, int64_t K);
 at::Tensor sample_tokens(at::Tensor logits, double temperature, int64_t seed);
 
+// Whether tensors have been written to (their version counters), asked for
+// before every replay of a captured step: 0.8 us for 129 weights, 12 in Python.
+class Versions {
+ public:
+  explicit Versions(std::vector<at::Tensor> tensors)
+      : tensors_(std::move(tensors)), sum_(sum()) {}
+  bool current() const { return sum() == sum_; }
+
+ private:
+  int64_t sum() const {                 // counters only rise
+    int64_t s = 0;
+    for (const at::Tensor &t : tensors_) s += t._version();
+    return s;
+  }
+  std::vector<at::Tensor> tensors_;
+  int64_t sum_;
+};
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  py::class_<Versions>(m, "Versions")
+      .def(py::init<std::vector<at::Tensor>>())
+      .def("current", &Versions::current);
   m.doc() = "runbooks_amd gfx950 HIP kernels: core serving ops";
   m.def("rmsnorm_fwd", &rmsnorm_fwd, "fused RMSNorm forward (bf16/f32)");
   m.def("rmsnorm_fwd_dec", &rmsnorm_fwd_dec,

@@ -7,7 +7,9 @@ on hipBLASLt via F.linear — the library is the right tool for big GEMMs.
 """
 from __future__ import annotations
 
+import contextlib
 import os
+import threading
 import weakref
 
 import torch
@@ -53,7 +55,29 @@ def _registry_get(reg: dict, weight: torch.Tensor):
     if entry[-1]() is not weight:
         del reg[weight.data_ptr()]
         return None
-    return entry if entry[-2] == _version(weight) else None
+    if entry[-2] != _version(weight):
+        return None
+    served = getattr(_RECORD, "weights", None)
+    if served is not None:
+        served[id(weight)] = weight
+    return entry
+
+
+_RECORD = threading.local()
+
+
+@contextlib.contextmanager
+def copies_read():
+    """Within it, the weights of which this thread looked a copy up are
+    gathered; afterwards the list holds a Versions of them."""
+    _RECORD.weights, result = {}, []
+    try:
+        yield result
+    finally:
+        weights = list(_RECORD.weights.values())
+        _RECORD.weights = None
+    result.append(_backend.ext().Versions(
+        [w for w in weights if not w.is_inference()]))
 
 
 def register_decode_weight(weight: torch.Tensor) -> None:

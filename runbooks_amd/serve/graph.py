@@ -15,6 +15,8 @@ from __future__ import annotations
 
 import torch
 
+from ..ops.linear import copies_read
+
 
 def fixed_nsplit(batch: int, hkv: int, mfma: bool = False) -> int:
     """Work-split for the paged-decode kernel, chosen per bucket at capture
@@ -63,7 +65,9 @@ class GraphedDecoder:
                                    device=dev)
         self.inputs = torch.zeros(self.h_staging.shape, dtype=torch.int32,
                                   device=dev)
-        self.graphs = {}     # bucket -> (CUDAGraph, logits_out)
+        # bucket -> (CUDAGraph, logits_out, versions of the weights whose
+        # copies it reads)
+        self.graphs = {}
         self._pool = None
 
     # -- capture -----------------------------------------------------------
@@ -99,14 +103,15 @@ class GraphedDecoder:
         torch.cuda.current_stream().wait_stream(s)
 
         g = torch.cuda.CUDAGraph()
-        if self._pool is None:
-            with torch.cuda.graph(g):
-                out = step()
-            self._pool = g.pool()
-        else:
-            with torch.cuda.graph(g, pool=self._pool):
-                out = step()
-        self.graphs[b] = (g, out)
+        with copies_read() as versions:
+            if self._pool is None:
+                with torch.cuda.graph(g):
+                    out = step()
+                self._pool = g.pool()
+            else:
+                with torch.cuda.graph(g, pool=self._pool):
+                    out = step()
+        self.graphs[b] = (g, out, *versions)
 
     # -- replay ------------------------------------------------------------
     def decode(self, tokens, positions, slots, block_rows, seq_lens,
@@ -115,9 +120,11 @@ class GraphedDecoder:
         Returns logits [len(tokens), V] (a view into the static output)."""
         n = len(tokens)
         b = next(x for x in self.buckets if x >= n)
-        if b not in self.graphs:
+        if b not in self.graphs or not self.graphs[b][2].current():
+            # not yet, or weights have changed since: their products then run
+            # without a copy
             self._capture(b)
-        g, out = self.graphs[b]
+        g, out, _ = self.graphs[b]
         bt = self._stage(b, tokens, positions, slots, block_rows, seq_lens,
                          seq_starts or [0] * n, state_slots)
 

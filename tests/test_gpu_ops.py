@@ -1530,6 +1530,47 @@ def test_captured_decode_follows_weights(name, batch):
             before = got.clone()
 
 
+@pytest.mark.parametrize("batch", [1, 20, 40])
+@pytest.mark.parametrize("eight_bit", [False, True])
+def test_captured_decode_follows_weights_with_copies(batch, eight_bit):
+    """A captured step whose products read copies of the weights is captured
+    again once a weight has been written to."""
+    _assert_hip()
+    from runbooks_amd.models.config import ModelConfig
+    from runbooks_amd.models.transformer import Transformer, fuse_for_inference
+    from runbooks_amd.serve.graph import GraphedDecoder
+    cfg = ModelConfig("copies", 256, 1024, 2, 8, 8, 1024, max_seq_len=64,
+                      head_dim=128)
+    torch.manual_seed(1)
+    m = fuse_for_inference(Transformer(cfg, dtype=torch.bfloat16, tp=1)
+                           .to(DEV).eval(), load_in_8bit=eight_bit)
+    caches = m.alloc_caches(batch + 1, DEV)
+    for c in (c for kv in caches for c in kv):
+        c.normal_()
+    step = (list(range(batch)), [9] * batch,
+            [i * 16 + 9 for i in range(batch)], [[i] for i in range(batch)],
+            [10] * batch)
+    i32 = dict(device=DEV, dtype=torch.int32)
+    with torch.no_grad():
+        graphed = GraphedDecoder(m, caches, batch, 1, batch, DEV)
+        before = graphed.decode(*step).clone()
+        first = graphed.graphs[batch][0]
+        for p in (m.blocks[1].attn.v_proj.weight, m.blocks[0].mlp.up_proj.weight,
+                  m.blocks[1].mlp.down_proj.weight, m.lm_head.weight):
+            graphed.decode(*step)
+            assert graphed.graphs[batch][0] is first
+            p.copy_(torch.randn_like(p) * 0.05)
+            got = graphed.decode(*step).clone()
+            want = m.decode(torch.tensor(step[0], device=DEV),
+                            torch.tensor(step[1], **i32), caches,
+                            torch.tensor(step[2], **i32),
+                            torch.tensor(step[3], **i32),
+                            torch.tensor(step[4], **i32), nsplit=1)
+            assert (got - want).norm() < 0.02 * want.norm()
+            assert (got - before).norm() > 0.05 * before.norm()
+            before, first = got, graphed.graphs[batch][0]
+
+
 @pytest.mark.parametrize("where", ["block", "norm1", "fc1", "adapters"])
 def test_decode_affine_leaves_modules_that_do_more(where):
     """A hook, or an adapter put in later, takes decoding off the path that

@@ -297,3 +297,15 @@ def test_flash_waves_wait_for_the_same_tiles(rows):
             else:
                 assert full == row // 64 and last == row + 31
                 assert -(-min(S, row + 32) // 64) <= tiles
+
+
+def test_versions_of_weights():
+    """Any write through a tensor or a view of it shows, nothing else does."""
+    core = pytest.importorskip("runbooks_amd.ops._hip_core")
+    ws = [torch.zeros(4, 4) for _ in range(3)]
+    versions = core.Versions(ws)
+    ws[1].sum(), ws[2].clone().add_(1)
+    assert versions.current()
+    ws[2][1:3].add_(1)
+    assert not versions.current()
+    assert core.Versions(ws).current() and core.Versions([]).current()

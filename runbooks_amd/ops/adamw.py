@@ -86,6 +86,10 @@ class FusedAdamW(torch.optim.Optimizer):
 
             if step_num is None:
                 continue
+            # the kernels write past autograd: readers of a weight's version
+            # (its copies for decoding among them) learn of it here
+            torch.autograd.graph.increment_version(
+                [p for p in group["params"] if p.grad is not None])
 
             if uniform_step and group["params"][0].is_cuda:
                 sig = [(p.data_ptr(), p.grad.data_ptr())

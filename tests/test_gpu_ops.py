@@ -1315,6 +1315,29 @@ def test_products_of_changed_weight(m, fp8):
             assert (y - ref).norm() < 2 ** -8 * ref.norm()
 
 
+@pytest.mark.parametrize("m", [1, 40])
+@pytest.mark.parametrize("uniform", [True, False])
+def test_products_of_trained_weight(m, uniform):
+    """A step of the optimizer, whose kernels write past autograd, is followed
+    by the products of a weight that has a decode layout."""
+    from runbooks_amd.ops.linear import fast_linear, register_decode_weight
+    torch.manual_seed(m)
+    w = torch.nn.Parameter(torch.randn(64, 1024, device=DEV).bfloat16())
+    other = torch.nn.Parameter(torch.ones(8, device=DEV).bfloat16())
+    register_decode_weight(w)
+    opt = ops.FusedAdamW([w, other], lr=0.1)
+    if not uniform:             # a step for each parameter
+        other.grad = torch.ones_like(other)
+        opt.step()
+    other.grad, w.grad = torch.ones_like(other), torch.randn_like(w)
+    opt.step()
+    x = torch.randn(m, 1024, device=DEV).bfloat16()
+    with torch.no_grad():
+        y = fast_linear(x, w)
+    ref = x.double() @ w.double().t()
+    assert (y - ref).norm() < 2 ** -8 * ref.norm()
+
+
 def test_decode_gemm_rows_of_changed_weight():
     """Products of 33 to 128 rows follow a weight that changes in place."""
     from runbooks_amd.ops.linear import fast_linear, register_decode_weight

@@ -449,3 +449,10 @@ def test_adapters_that_never_pack_are_refused_at_once(bias, r):
     from runbooks_amd.train.lora import LoRALinear, _packs
     layer = LoRALinear(torch.nn.Linear(64, 64, bias=bias), r=r)
     assert not _packs([layer], None)
+
+
+def test_optimizer_steps_show_in_versions():
+    ps = [torch.nn.Parameter(torch.ones(4)) for _ in range(2)]
+    ps[0].grad = torch.ones(4)
+    ops.FusedAdamW(ps, lr=0.1).step()
+    assert ps[0]._version > 0 and ps[1]._version == 0

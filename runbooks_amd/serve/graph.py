@@ -17,6 +17,8 @@ import torch
 
 from ..ops.linear import copies_read
 
+RING = 8        # staging buffers
+
 
 def fixed_nsplit(batch: int, hkv: int, mfma: bool = False) -> int:
     """Work-split for the paged-decode kernel, chosen per bucket at capture
@@ -58,7 +60,14 @@ class GraphedDecoder:
         dev = device
         pin = dict(dtype=torch.int64,
                    pin_memory=torch.cuda.is_available())
-        self.h_staging = torch.zeros(B * 6 + B * max_blocks, **pin)
+        # a step's inputs leave their buffer when the GPU comes to its copy, so
+        # steps that are called without waiting need one each: two halves of a
+        # ring, an event behind the copies of each (one for every step took 4
+        # us of 503)
+        self._ring = list(torch.zeros(RING, B * 6 + B * max_blocks, **pin))
+        self._sent = [None, None]
+        self._turn = -1
+        self.h_staging = self._ring[0]
         self._np = self.h_staging.numpy()
         # the same on the device, as it arrives and as the kernels take it
         self.arrived = torch.zeros(self.h_staging.shape, dtype=torch.int64,
@@ -125,6 +134,7 @@ class GraphedDecoder:
             # without a copy
             self._capture(b)
         g, out, _ = self.graphs[b]
+        half, place = self._next_buffer()
         bt = self._stage(b, tokens, positions, slots, block_rows, seq_lens,
                          seq_starts or [0] * n, state_slots)
 
@@ -133,8 +143,22 @@ class GraphedDecoder:
         # and 511 us)
         size = 6 * b + bt.numel()
         self.arrived[:size].copy_(self.h_staging[:size], non_blocking=True)
+        if place == RING // 2 - 1:
+            self._sent[half] = torch.cuda.Event()
+            self._sent[half].record()
         g.replay()
         return out[:n]
+
+    def _next_buffer(self) -> tuple[int, int]:
+        """Turns to the next staging buffer once its last inputs have left;
+        which half of the ring it is in, and its place there."""
+        self._turn = (self._turn + 1) % RING
+        half, place = divmod(self._turn, RING // 2)
+        if place == 0 and self._sent[half] is not None:
+            self._sent[half].synchronize()
+        self.h_staging = self._ring[self._turn]
+        self._np = self.h_staging.numpy()
+        return half, place
 
     def _stage(self, b, tokens, positions, slots, block_rows, seq_lens,
                seq_starts, state_slots=None):

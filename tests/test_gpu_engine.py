@@ -227,3 +227,26 @@ def test_qwen2_style_gqa_bias_vt_decode():
         scale = ref.abs().max().item()
         assert (got - ref).abs().max().item() / scale < 3e-2, \
             (got[:, :8], ref[:, :8])
+
+
+def test_graphed_decode_without_waiting():
+    """Steps that are called one after the other while the GPU is busy each
+    run on their own inputs."""
+    assert ops.has_hip()
+    from runbooks_amd.models.transformer import fuse_for_inference
+    from runbooks_amd.serve.graph import GraphedDecoder
+    m = fuse_for_inference(build_model("smoke-llama", dtype=torch.bfloat16,
+                                       tp=1, device=DEV).eval())
+    caches = m.alloc_caches(20, DEV)
+    steps = [([3 + i], [0], [i * 16], [[i]], [1]) for i in range(19)]
+    with torch.no_grad():
+        graphed = GraphedDecoder(m, caches, 1, 1, 19, DEV)
+        want = []
+        for step in steps:
+            want.append(graphed.decode(*step).clone())
+            torch.cuda.synchronize()
+        torch.cuda._sleep(int(2e8))
+        got = [graphed.decode(*step).clone() for step in steps]
+    for g, w in zip(got, want):
+        assert torch.equal(g, w)
+    assert not torch.equal(want[0], want[1])

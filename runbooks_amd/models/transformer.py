@@ -797,7 +797,12 @@ class _AffineBlock:
                 m.fc1.weight.shape[0] % 32 == 0 and
                 a.hq * a.dh % 32 == 0 and a.hkv * a.dh % 32 == 0 and
                 all(n.weight is not None and n.bias is not None
-                    for n in (blk.norm1, blk.norm2, model.norm_f)))
+                    for n in (blk.norm1, blk.norm2, model.norm_f)) and
+                all(t.dtype == torch.bfloat16 and t.is_contiguous() and
+                    t.data_ptr() % 16 == 0
+                    for p in (a.q_proj, a.k_proj, a.v_proj, a.o_proj, m.fc1,
+                              m.down_proj)
+                    for t in (p.weight, p.bias) if t is not None))
 
     @staticmethod
     def plain(blk) -> bool:

@@ -4,6 +4,7 @@ import torch
 
 from runbooks_amd import ops
 from runbooks_amd.models import build_model, get_config, list_configs
+from runbooks_amd.models.transformer import _AffineBlock
 from runbooks_amd.serve import Engine
 from runbooks_amd.train import apply_lora, lora_state_dict, merge_lora
 
@@ -795,3 +796,19 @@ def test_modules_of_other_kinds_run():
     finally:
         handle.remove()
     assert seen.count("Block") == 2 and seen.count("RMSNorm") == 5
+
+
+@pytest.mark.parametrize("lies", ["as made", "transposed", "off alignment"])
+def test_weights_as_decode_reads_them(lies):
+    """Decode of layer-norm models reads the parameters as they lie: those that
+    lie otherwise stay with the products that take any."""
+    m = build_model("tiny-opt", dtype=torch.bfloat16, tp=1)
+    blk = m.blocks[0]
+    w = blk.mlp.fc1.weight
+    if lies == "transposed":
+        w.data = w.data.t().contiguous().t()
+    elif lies == "off alignment":
+        flat = torch.empty(w.numel() + 8, dtype=w.dtype)
+        at = 1 if flat.data_ptr() % 16 == 0 else 0
+        w.data = flat[at:at + w.numel()].view(w.shape).copy_(w.data)
+    assert _AffineBlock.serves(m, blk) == (lies == "as made")

@@ -912,7 +912,7 @@ def fuse_for_inference(model: "Transformer",
             model.dtype == torch.bfloat16:
         # Register fragment-lane-major weight copies for the v2 decode
         # GEMM (csrc/decode_gemm.hip): doubles decode-weight memory, which
-        # 288 GB HBM3E affords for every BASELINE config at TP=1 except
+        # 288 GB HBM3E affords for every served model at TP=1 except
         # llama2-70b (which serves via MODEL_LOAD_IN_8BIT / TP>1). Budget
         # guard: keep at least ~35% of the GPU free for KV cache.
         from ..ops.linear import register_decode_weight

@@ -7,7 +7,7 @@
 //    4 contiguous KV rows per iteration at 16/8 B per lane.
 //  * GQA/MQA-native: a workgroup handles one (seq, kv_head); its G query
 //    heads share each K/V read (falcon-40b MQA G=16, llama2-70b G=8,
-//    llama2-7b MHA G=1 — SURVEY.md §2b "server image").
+//    llama2-7b MHA G=1).
 //  * flash-style online softmax entirely in registers; group partials
 //    merged via shfl_xor(16/32), wave partials via LDS.
 //  * kv-split ("flash-decoding") for long sequences / small batch: grid z
@@ -77,7 +77,7 @@ RB_DEV int sequence_of() {
 // FP8: caches are e4m3 rows of fp8_row_bytes(DH) = DH bytes + f32
 // scale (+pad): decode attention is KV-bandwidth bound at long context,
 // so halving cache bytes halves the dominant stream AND doubles KV
-// capacity within 288 GB (BASELINE config #5). Dequant rides
+// capacity within 288 GB. Dequant rides
 // v_cvt_pk_f32_fp8 in the inner loop.
 template <int DH, int G, bool SPLIT, bool FP8 = false>
 __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
@@ -950,8 +950,7 @@ std::vector<at::Tensor> paged_decode_swz(at::Tensor q, at::Tensor k_cache,
       default: TORCH_CHECK(false, "paged_decode: unsupported G=", G);
     }
   } else if (dh == 256) {
-    // gemma-7b (wide heads, MHA). VE=16 -> ~70 VGPRs at G=1; first GPU
-    // validation is the RB_EXPERIMENTAL test (round 2).
+    // gemma-7b (wide heads, MHA). VE=16 -> ~70 VGPRs at G=1.
     switch (G) {
       case 1: RB_DEC(256, 1); break;
       case 2: RB_DEC(256, 2); break;

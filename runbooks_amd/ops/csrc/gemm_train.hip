@@ -4,14 +4,10 @@
 // dim — the nn.Linear forward shape). Target: the training-step
 // projection GEMMs (M=2048), where hipBLASLt measured 860-1140 TF/s
 // in-situ (profiles/train_*.csv) while this template's verified ceiling
-// is ~1320-1340 TF/s on random operands
-// (cdna_hip_programming.md §5 "The 256^2 8-phase template").
+// is ~1320-1340 TF/s on random operands.
 //
-// Status: drafted offline at the end of round 1 (no GPU budget left to
-// validate); NOT wired into any model path. Gated behind
-// RB_EXPERIMENTAL: tests skip unless it is set. Round 2: run
-// `RB_EXPERIMENTAL=1 pytest tests/test_gpu_ops.py -k train_gemm` first,
-// then benchmarks/kernels.py.
+// Status: NOT wired into any model path by default (RB_EXPERIMENTAL_GEMM=1
+// does). Its tests run with RB_EXPERIMENTAL=1; benchmarks/kernels.py times it.
 //
 // Grid fill: when (M/256)*(N/256) < 256 the host splits K (fp32 slabs
 // + a combine kernel, the skinny_gemm.hip pattern) — M=2048 N=4096 runs

@@ -4,7 +4,7 @@
 // HBM-bound pass per direction. Reference semantics match the plain
 // PyTorch fp32 RMSNorm used by the test-suite reference models
 // (llama-family norm; the reference platform delegates this to external
-// HuggingFace trainer images — see SURVEY.md §2b).
+// HuggingFace trainer images).
 //
 // Layout: x [N, D] row-major. One workgroup (256 threads) per row,
 // grid-strided. All math in fp32; bf16 IO vectorized 8-wide (16 B/lane).

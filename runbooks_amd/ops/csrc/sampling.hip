@@ -2,7 +2,7 @@
 //
 // greedy_sample: per-row argmax over the vocab (the serving engine's
 // greedy decode — reference behavior: the external basaran server image's
-// sampling loop, SURVEY.md §2b "server image").
+// sampling loop).
 //
 // gumbel_sample: temperature sampling via the Gumbel-max trick:
 // argmax(logits/T + G) with G ~ Gumbel(0,1) samples exactly from

@@ -143,7 +143,7 @@ class Engine:
         self.seed = seed
         # fp8-e4m3 KV cache (RB_KV_FP8=1 or kv_fp8=True): halves the
         # decode-attention read stream and doubles KV capacity — the
-        # long-context lever for the 288 GB/GPU KV story (BASELINE #5).
+        # long-context lever for the 288 GB/GPU KV story.
         import os as _os0
         self.kv_fp8 = (kv_fp8 if kv_fp8 is not None
                        else _os0.environ.get("RB_KV_FP8", "0") == "1")

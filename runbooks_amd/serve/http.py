@@ -24,7 +24,7 @@ from pydantic import BaseModel
 from .engine import Engine
 from .tokenizer import load_tokenizer
 
-# per-request latency logging (SURVEY.md §5 tracing: the reference has
+# per-request latency logging (the reference has
 # none; the serving runtime logs one structured line per request)
 logger = logging.getLogger("runbooks_amd.serve")
 
@@ -209,7 +209,7 @@ def build_app(engine: Engine, tokenizer=None,
 
     # Prometheus metrics (the reference exposes controller metrics behind
     # kube-rbac-proxy; the serving runtime gets request/token counters and
-    # latency histograms — SURVEY.md §5 observability)
+    # latency histograms)
     m_reqs, m_tokens, m_lat = M_REQS, M_TOKENS, M_LAT
     if M_REQS is not None:
         @app.get("/metrics")

@@ -1,5 +1,5 @@
 """Training data: jsonl instruction datasets (the reference's dataset
-artifact format — SURVEY.md §2b "dataset-loader image") and synthetic
+artifact format) and synthetic
 token streams for benchmarking (no network in bench environments)."""
 from __future__ import annotations
 

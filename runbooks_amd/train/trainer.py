@@ -1,7 +1,7 @@
 """The fine-tune loop: LoRA (or full) training with DP over RCCL.
 
-Native replacement for the reference's external HF trainer image
-(SURVEY.md §2b "trainer image"): params arrive via PARAM_* env /
+Native replacement for the reference's external HF trainer
+image: params arrive via PARAM_* env /
 params.json (utils.params), data from /content/data, checkpoints to
 /content/artifacts.
 """
@@ -197,7 +197,7 @@ class Trainer:
         """Resume model weights, optimizer moments, and the step counter
         from the latest checkpoint in output_dir (the bucket-mounted
         /content/artifacts in-cluster — artifacts survive cluster
-        re-creation via the deterministic bucket path, SURVEY.md §5)."""
+        re-creation via the deterministic bucket path)."""
         latest = ckpt_mod.latest_checkpoint(self.cfg.output_dir)
         if latest is None:
             return False

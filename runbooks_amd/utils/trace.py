@@ -1,6 +1,6 @@
 """Lightweight span tracing -> chrome://tracing JSON.
 
-SURVEY.md §5 "Tracing / profiling": the reference has none; the rebuild
+The reference has no tracing; this framework
 gets rocprofv3 for kernels (profiles/) and this host-side tracer for
 scheduler/step spans. Enable with RB_TRACE=/path/out.json (the engine
 wraps its step phases) or use Tracer directly; open the dump in

@@ -1,7 +1,7 @@
 """In-pod workload entrypoints (the images' mains).
 
 These are the native replacements for the reference's external workload
-images (SURVEY.md §2b): model-loader, dataset-loader, trainer, server,
+images: model-loader, dataset-loader, trainer, server,
 plus the entrypoint shim that turns /content/params.json into PARAM_*
 env vars (documented in the reference container contract,
 reference docs/container-contract.md:34-48, implemented only in its

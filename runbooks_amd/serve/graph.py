@@ -134,7 +134,7 @@ class GraphedDecoder:
             # without a copy
             self._capture(b)
         g, out, _ = self.graphs[b]
-        half, place = self._next_buffer()
+        self._next_buffer()
         bt = self._stage(b, tokens, positions, slots, block_rows, seq_lens,
                          seq_starts or [0] * n, state_slots)
 
@@ -143,22 +143,22 @@ class GraphedDecoder:
         # and 511 us)
         size = 6 * b + bt.numel()
         self.arrived[:size].copy_(self.h_staging[:size], non_blocking=True)
-        if place == RING // 2 - 1:
-            self._sent[half] = torch.cuda.Event()
-            self._sent[half].record()
         g.replay()
         return out[:n]
 
-    def _next_buffer(self) -> tuple[int, int]:
-        """Turns to the next staging buffer once its last inputs have left;
-        which half of the ring it is in, and its place there."""
+    def _next_buffer(self) -> None:
+        """Turns to the next staging buffer once its last inputs have left."""
         self._turn = (self._turn + 1) % RING
         half, place = divmod(self._turn, RING // 2)
-        if place == 0 and self._sent[half] is not None:
-            self._sent[half].synchronize()
+        if place == 0:
+            # every copy of the other half is on its way, also where a step
+            # ended early
+            self._sent[1 - half] = torch.cuda.Event()
+            self._sent[1 - half].record()
+            if self._sent[half] is not None:
+                self._sent[half].synchronize()
         self.h_staging = self._ring[self._turn]
         self._np = self.h_staging.numpy()
-        return half, place
 
     def _stage(self, b, tokens, positions, slots, block_rows, seq_lens,
                seq_starts, state_slots=None):

@@ -229,9 +229,10 @@ def test_qwen2_style_gqa_bias_vt_decode():
             (got[:, :8], ref[:, :8])
 
 
-def test_graphed_decode_without_waiting():
+@pytest.mark.parametrize("refused", [False, True])
+def test_graphed_decode_without_waiting(refused):
     """Steps that are called one after the other while the GPU is busy each
-    run on their own inputs."""
+    run on their own inputs, also among calls that are refused."""
     assert ops.has_hip()
     from runbooks_amd.models.transformer import fuse_for_inference
     from runbooks_amd.serve.graph import GraphedDecoder
@@ -246,7 +247,12 @@ def test_graphed_decode_without_waiting():
             want.append(graphed.decode(*step).clone())
             torch.cuda.synchronize()
         torch.cuda._sleep(int(2e8))
-        got = [graphed.decode(*step).clone() for step in steps]
+        got = []
+        for step in steps:
+            if refused and graphed._turn % 4 == 2:
+                with pytest.raises(ValueError):
+                    graphed.decode([1], ["no number"], *step[2:])
+            got.append(graphed.decode(*step).clone())
     for g, w in zip(got, want):
         assert torch.equal(g, w)
     assert not torch.equal(want[0], want[1])

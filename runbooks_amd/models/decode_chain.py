@@ -1,0 +1,153 @@
+"""Decode of RMSNorm models of up to 32 sequences, a layer in six launches
+(csrc/decode_ends.h, csrc/decode_res.hip):
+
+  * q, k and v, rotated and cached;
+  * attention, and the sum of its parts where sequences are split;
+  * the output projection with the residual and the next norm's sums;
+  * gate and up projection with the gated unit;
+  * the down projection with the residual and the next norm's sums.
+
+A norm's 1 / rms is left to the product that reads its result. Where a step has
+no kernel of this kind (8-bit caches, wide residuals, long sums of many rows) it
+is the launches of Block.forward_decode_fused.
+"""
+from __future__ import annotations
+
+import torch
+
+from .. import ops
+from ..parallel import ColumnParallelLinear, RowParallelLinear
+from ..utils.modules import plain
+
+
+class _Layer:
+    """Copies that a block's products read."""
+
+    def __init__(self, blk):
+        a, m = blk.attn, blk.mlp
+        self.blk, self.attn = blk, a
+        self.gelu = m.act == "gelu_glu"
+        self.qkv, self.o = ops.Copy(a._qkv_w), ops.Copy(a.o_proj.weight)
+        self.gate_up = ops.Copy(m._gateup_w)
+        self.down = ops.Copy(m.down_proj.weight)
+
+    def served(self) -> bool:
+        return (all(c.ws is not None for c in (self.qkv, self.o, self.gate_up,
+                                               self.down)) and
+                self.qkv.half * 2 == self.attn.dh and
+                self.gate_up.half * 2 == self.gate_up.n)
+
+
+def layers_of(model, block_type, attention_type, mlp_type):
+    """A _Layer for every block, or None where one is not served or a module
+    would do more than its kernels."""
+    cfg = model.cfg
+    if not (cfg.pos == "rope" and cfg.act in ("silu_glu", "gelu_glu") and
+            model.tp == 1 and model.rope_cos.dtype == torch.float32):
+        return None
+    blocks = list(model.blocks)
+    mlps, attns = [b.mlp for b in blocks], [b.attn for b in blocks]
+    if not (blocks and plain(block_type, *blocks) and plain(mlp_type, *mlps) and
+            plain(attention_type, *attns) and
+            plain(ops.RMSNorm, *(n for b in blocks
+                                 for n in (b.norm1, b.norm2))) and
+            plain(RowParallelLinear, *(m.down_proj for m in mlps),
+                  *(a.o_proj for a in attns)) and
+            plain(ColumnParallelLinear, *(m.gate_proj for m in mlps),
+                  *(m.up_proj for m in mlps), *(a.q_proj for a in attns))):
+        return None
+    for b in blocks:
+        if (getattr(b.attn, "_qkv_w", None) is None or
+                getattr(b.mlp, "_gateup_w", None) is None or
+                b.attn.o_proj.bias is not None or
+                b.mlp.down_proj.bias is not None or
+                any(n.weight.dtype != torch.bfloat16 or
+                    not n.weight.is_contiguous()
+                    for n in (b.norm1, b.norm2))):
+            return None
+    layers = [_Layer(b) for b in blocks]
+    return layers if all(layer.served() for layer in layers) else None
+
+
+class _Normed:
+    """A norm's result for the products that read it: an operand, rows, or both,
+    without its 1 / rms where there are squares."""
+
+    def __init__(self, swz=None, rows=None, squares=None, eps=0.0):
+        self.swz, self.rows = swz, rows
+        self.squares, self.eps = squares, eps
+
+
+def _shares_x(copy, m: int) -> bool:
+    """From 17 rows the kernel that shares x between workgroups' waves wins
+    where it has about one workgroup for every CU (ops.wide_linear)."""
+    return 16 < m <= 32 and not copy.fp8 and 10240 <= copy.n <= 32768
+
+
+def _heads(layer, y, m, cos, sin, positions, kc, vc, slots):
+    ext, c, hq = ops.ext(), layer.qkv, layer.attn.hq
+    if kc.dtype != torch.bfloat16:          # rows of it share a scale
+        if y.squares is not None:
+            out = ext.decode_normed(y.swz, c.ws, c.scale, m, c.n, c.k,
+                                    y.squares, y.eps, c.half)
+        else:
+            out = ops.wide_linear(y.rows, layer.attn._qkv_w)
+        return ext.qkv_rope_append(out, cos, sin, positions.to(torch.int32),
+                                   kc, vc, slots.to(torch.int32), hq)
+    if y.squares is None and _shares_x(c, m):
+        return ext.rows_heads(y.rows, c.ws, c.n, cos, sin, positions, kc, vc,
+                              slots, hq)
+    return ext.decode_heads(y.swz, c.ws, c.scale, m, c.n, c.k, y.squares, y.eps,
+                            cos, sin, positions, kc, vc, slots, hq)
+
+
+def _gated(layer, y, m):
+    ext, c = ops.ext(), layer.gate_up
+    if y.rows is not None and _shares_x(c, m):
+        return ext.rows_glu(y.rows, c.ws, c.n, layer.gelu, True, y.squares,
+                            y.eps)
+    return ext.decode_glu(y.swz, c.ws, c.scale, m, c.n, c.k, layer.gelu,
+                          y.squares, y.eps)
+
+
+def _add(x, operand, copy, norm, rows: bool):
+    """x + operand W^T and its norm, as rows where those will do."""
+    ext, m = ops.ext(), x.shape[0]
+    # the kernel whose workgroups have whole sums reads x once for 16 columns,
+    # which is what it takes with many long rows (us in parts and whole, with
+    # the norm: 32 rows, 4096 x 4096 13.8 and 10.1, 4096 x 11008 23.8 and 24.0,
+    # 4096 x 14336 27.1 and 29.6, 3072 x 24576 39.7 and 45.7; 16 rows 13.2 and
+    # 8.4, 22.0 and 20.5, 25.4 and 24.2, 34.2 and 33.7)
+    if (m <= 16 or copy.k <= 8192) and \
+            ext.decode_res_supported(m, copy.n, copy.k, copy.fp8):
+        x, y, squares = ext.decode_res(operand, copy.ws, copy.scale, x,
+                                       norm.weight, rows)
+        return x, _Normed(None if rows else y, y if rows else None, squares,
+                          norm.eps)
+    delta = copy.product(operand, m)
+    add = (ext.rmsnorm_res_slab_fwd_dec if delta.dtype == torch.float32 else
+           ext.rmsnorm_res_fwd_dec)
+    x, rows_, swz = add(x, delta, norm.weight, norm.eps)
+    return x, _Normed(swz, rows_)
+
+
+def run(model, layers, x, positions, caches, slots, tables, seq_lens, nsplit,
+        seq_starts):
+    """x [m, hidden], embedded tokens -> (residual, what the last block has
+    still to add to it: bf16 [m, hidden] or fp32 parts of it)."""
+    ext, m = ops.ext(), x.shape[0]
+    cos, sin = model.rope_cos, model.rope_sin
+    norm = layers[0].blk.norm1
+    rows, swz = ext.rmsnorm_fwd_dec(x, norm.weight, norm.eps)
+    y = _Normed(swz, rows)
+    for i, (layer, (kc, vc)) in enumerate(zip(layers, caches)):
+        blk, attn = layer.blk, layer.attn
+        q = _heads(layer, y, m, cos, sin, positions, kc, vc, slots)
+        _, o = ops.paged_decode_with_operand(
+            q, kc, vc, tables, seq_lens, scale=attn.scale, nsplit=nsplit,
+            seq_starts=seq_starts)
+        x, y = _add(x, o, layer.o, blk.norm2, _shares_x(layer.gate_up, m))
+        h = _gated(layer, y, m)
+        if i + 1 < len(layers):
+            x, y = _add(x, h, layer.down, layers[i + 1].blk.norm1, False)
+    return x, layers[-1].down.product(h, m)

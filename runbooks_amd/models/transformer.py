@@ -41,6 +41,7 @@ from ..parallel import (
     gather_from_tp,
 )
 from ..utils.modules import plain
+from . import decode_chain
 from .config import LatentAttentionSpec, ModelConfig
 from .dual import DualBlock
 from .hybrid import SequentialBlock
@@ -568,12 +569,18 @@ class Transformer(nn.Module):
                 os.environ.get("RB_FUSED_RESID", "1") == "1"):
             # fused residual chain: zero standalone adds in the hot loop
             delta = None
-            for blk, (kc, vc) in zip(self.blocks, caches):
-                fn = lambda h, b=blk, kc=kc, vc=vc: b.attn.forward_decode(  # noqa: E731
-                    h, self.rope_cos, self.rope_sin, positions, kc, vc,
-                    slot_mapping, block_tables, seq_lens, nsplit=nsplit,
-                    slab_ok=True, seq_starts=seq_starts)
-                x, delta = blk.forward_decode_fused(x, delta, fn)
+            layers = decode_chain.layers_of(self, Block, Attention, MLP)
+            if layers is not None:
+                x, delta = decode_chain.run(
+                    self, layers, x, positions, caches, slot_mapping,
+                    block_tables, seq_lens, nsplit, seq_starts)
+            else:
+                for blk, (kc, vc) in zip(self.blocks, caches):
+                    fn = lambda h, b=blk, kc=kc, vc=vc: b.attn.forward_decode(  # noqa: E731
+                        h, self.rope_cos, self.rope_sin, positions, kc, vc,
+                        slot_mapping, block_tables, seq_lens, nsplit=nsplit,
+                        slab_ok=True, seq_starts=seq_starts)
+                    x, delta = blk.forward_decode_fused(x, delta, fn)
             if delta.dtype == torch.float32:
                 _, y, swz = ops.ext().rmsnorm_res_slab_fwd_dec(
                     x, delta, self.norm_f.weight, self.norm_f.eps)
@@ -848,9 +855,9 @@ class _AffineBlock:
         return self._products((self.down_proj,), h, rows)[0]
 
 
-def _fuse_projections(model: "Transformer") -> list[torch.Tensor]:
-    """Fused qkv and gate/up weights; returns every layer's serving
-    weights."""
+def _fuse_projections(model: "Transformer") -> dict[torch.Tensor, int]:
+    """Fused qkv and gate/up weights; returns every layer's serving weights
+    with the distance of the rows that their copies pair (0: none)."""
     for blk in model.blocks:
         attn = blk.attn
         if (attn.q_proj.bias is None and
@@ -883,11 +890,25 @@ def _fuse_projections(model: "Transformer") -> list[torch.Tensor]:
                                                 requires_grad=False)
             mlp.up_proj.weight = nn.Parameter(fused[half:],
                                               requires_grad=False)
-    return [w for blk in model.blocks
+    # the copies of weights whose rows meet in what follows the product are
+    # paired: a rotation's halves, gate and unit
+    def half_of(w, half):
+        return half if half % 16 == 0 and w is not None and \
+            w.shape[0] % (2 * half) == 0 else 0
+
+    halves = {}
+    for blk in model.blocks:
+        qkv = getattr(blk.attn, "_qkv_w", None)
+        if qkv is not None and model.cfg.pos == "rope":
+            halves[qkv] = half_of(qkv, blk.attn.dh // 2)
+        gateup = getattr(blk.mlp, "_gateup_w", None)
+        if gateup is not None:
+            halves[gateup] = half_of(gateup, gateup.shape[0] // 2)
+    return {w: halves.get(w, 0) for blk in model.blocks
             for w in (getattr(blk.attn, "_qkv_w", None),
                       getattr(blk.mlp, "_gateup_w", None),
                       blk.attn.o_proj.weight, blk.mlp.down_proj.weight)
-            if w is not None]
+            if w is not None}
 
 
 def fuse_for_inference(model: "Transformer",
@@ -900,9 +921,9 @@ def fuse_for_inference(model: "Transformer",
     the separate-projection training path keeps working.
     """
     if model.ragged:
-        weights = [w for blk in model.blocks for w in blk.fuse()]
+        weights = {w: 0 for blk in model.blocks for w in blk.fuse()}
         if model.cfg.loop is not None:
-            weights.append(model.loop_in.weight)
+            weights[model.loop_in.weight] = 0
         if model.cfg.streams is not None:
             model.fuse_streams()
     else:
@@ -927,7 +948,7 @@ def fuse_for_inference(model: "Transformer",
         free, total = torch.cuda.mem_get_info()
         if free - need >= int(0.35 * total):
             for w in cands:
-                register_decode_weight(w)
+                register_decode_weight(w, weights.get(w, 0))
         for blk in () if model.ragged else model.blocks:
             if model.lm_head.weight.is_cuda and _AffineBlock.serves(model, blk):
                 blk._affine = _AffineBlock(blk, model.cfg.act)
@@ -939,9 +960,9 @@ def fuse_for_inference(model: "Transformer",
         # stay for prefill/big-M GEMMs: 288 GB HBM3E makes both-copies the
         # right trade on MI355X.
         from ..ops.linear import quantize_fp8
-        for w in weights:
+        for w, half in weights.items():
             if w.shape[0] % 64 == 0 and w.shape[1] % 256 == 0:
-                quantize_fp8(w)
+                quantize_fp8(w, half)
         if model.lm_head.weight.shape[0] % 64 == 0 and \
                 model.lm_head.weight.shape[1] % 256 == 0:
             quantize_fp8(model.lm_head.weight)

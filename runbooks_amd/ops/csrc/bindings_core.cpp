@@ -19,15 +19,24 @@ at::Tensor swiglu_packed(at::Tensor y);
 at::Tensor geglu_packed(at::Tensor y);
 std::vector<at::Tensor> swiglu_packed_dec(at::Tensor y);
 std::vector<at::Tensor> geglu_packed_dec(at::Tensor y);
-at::Tensor decode_gemm_raw(at::Tensor xs, at::Tensor ws, int64_t M, int64_t N, int64_t K, bool f32);
-at::Tensor decode_gemm(at::Tensor xs, at::Tensor ws, int64_t M, int64_t N, int64_t K, int64_t force_split);
-at::Tensor decode_swizzle_w(at::Tensor w);
+at::Tensor decode_gemm_raw(at::Tensor xs, at::Tensor ws, int64_t M, int64_t N, int64_t K, bool f32, int64_t half);
+at::Tensor decode_gemm(at::Tensor xs, at::Tensor ws, int64_t M, int64_t N, int64_t K, int64_t force_split, int64_t half);
+at::Tensor decode_glu(at::Tensor xs, at::Tensor ws, c10::optional<at::Tensor> scale, int64_t M, int64_t N, int64_t K, bool gelu, c10::optional<at::Tensor> squares, double eps);
+at::Tensor decode_heads(at::Tensor xs, at::Tensor ws, c10::optional<at::Tensor> scale, int64_t M, int64_t N, int64_t K, c10::optional<at::Tensor> squares, double eps, at::Tensor cos, at::Tensor sin, at::Tensor positions, at::Tensor k_cache, at::Tensor v_cache, at::Tensor slots, int64_t hq);
+at::Tensor decode_normed(at::Tensor xs, at::Tensor ws, c10::optional<at::Tensor> scale, int64_t M, int64_t N, int64_t K, at::Tensor squares, double eps, int64_t half);
+bool rows_ends_pay(int64_t M, int64_t N, int64_t K);
+bool decode_res_supported(int64_t M, int64_t N, int64_t K, bool fp8);
+std::vector<at::Tensor> decode_res(at::Tensor xs, at::Tensor ws, c10::optional<at::Tensor> scale, at::Tensor res, at::Tensor norm, bool rows);
+std::vector<at::Tensor> rmsnorm_res_slab_fwd(at::Tensor x, at::Tensor slabs, at::Tensor w, double eps);
+at::Tensor rows_glu(at::Tensor x, at::Tensor ws, int64_t N, bool gelu, bool operand, c10::optional<at::Tensor> squares, double eps);
+at::Tensor rows_heads(at::Tensor x, at::Tensor ws, int64_t N, at::Tensor cos, at::Tensor sin, at::Tensor positions, at::Tensor k_cache, at::Tensor v_cache, at::Tensor slots, int64_t hq, bool rows);
+at::Tensor decode_swizzle_w(at::Tensor w, int64_t half);
 at::Tensor decode_swizzle_x(at::Tensor x);
-at::Tensor decode_swizzle_w8(at::Tensor w8);
+at::Tensor decode_swizzle_w8(at::Tensor w8, int64_t half);
 std::vector<at::Tensor> decode_affine(at::Tensor xs, std::vector<at::Tensor> ws, std::vector<c10::optional<at::Tensor>> biases, int64_t M, int64_t act, bool operand);
 at::Tensor sum_parts(at::Tensor parts);
-at::Tensor decode_gemm_rows(at::Tensor x, at::Tensor ws, int64_t N);
-at::Tensor decode_gemm_fp8(at::Tensor xs, at::Tensor w8s, at::Tensor scale, int64_t M, int64_t N, int64_t K, bool raw);
+at::Tensor decode_gemm_rows(at::Tensor x, at::Tensor ws, int64_t N, int64_t half, bool raw);
+at::Tensor decode_gemm_fp8(at::Tensor xs, at::Tensor w8s, at::Tensor scale, int64_t M, int64_t N, int64_t K, bool raw, int64_t half);
 int64_t decode_gemm_split(int64_t N, int64_t K);
 bool decode_gemm_supported(int64_t M, int64_t N, int64_t K);
 at::Tensor sample_tokens(at::Tensor logits, double temperature, int64_t seed);
@@ -84,28 +93,67 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_gemm_raw", &decode_gemm_raw,
         "decode GEMM returning the uncombined fp32 slab at split>1 (or always)",
         py::arg("xs"), py::arg("ws"), py::arg("M"), py::arg("N"),
-        py::arg("K"), py::arg("f32") = false);
+        py::arg("K"), py::arg("f32") = false, py::arg("half") = 0);
   m.def("decode_gemm", &decode_gemm,
         "v2 weight-stream decode GEMM over pre-swizzled operands: "
         "y[M<=32,N] = x @ W^T (bf16), 1KiB coalesced nt weight bursts",
         py::arg("xs"), py::arg("ws"), py::arg("M"), py::arg("N"),
-        py::arg("K"), py::arg("force_split") = -1);
+        py::arg("K"), py::arg("force_split") = -1, py::arg("half") = 0);
+  m.def("decode_glu", &decode_glu,
+        "gated unit of a decode product, as the next one's operand",
+        py::arg("xs"), py::arg("ws"), py::arg("scale"), py::arg("M"),
+        py::arg("N"), py::arg("K"), py::arg("gelu"),
+        py::arg("squares") = py::none(), py::arg("eps") = 0.0);
+  m.def("decode_heads", &decode_heads,
+        "decode product of q, k and v -> rotated q, keys and values cached",
+        py::arg("xs"), py::arg("ws"), py::arg("scale"), py::arg("M"),
+        py::arg("N"), py::arg("K"), py::arg("squares"), py::arg("eps"),
+        py::arg("cos"), py::arg("sin"), py::arg("positions"),
+        py::arg("k_cache"), py::arg("v_cache"), py::arg("slots"),
+        py::arg("hq"));
+  m.def("decode_normed", &decode_normed,
+        "decode product of an input without its norm's 1 / rms",
+        py::arg("xs"), py::arg("ws"), py::arg("scale"), py::arg("M"),
+        py::arg("N"), py::arg("K"), py::arg("squares"), py::arg("eps"),
+        py::arg("half") = 0);
+  m.def("rows_ends_pay", &rows_ends_pay);
+  m.def("decode_res_supported", &decode_res_supported);
+  m.def("decode_res", &decode_res,
+        "residual + decode product -> {sum, normed without 1 / rms, squares}",
+        py::arg("xs"), py::arg("ws"), py::arg("scale"), py::arg("res"),
+        py::arg("norm"), py::arg("rows") = false);
+  m.def("rmsnorm_res_slab_fwd", &rmsnorm_res_slab_fwd,
+        "residual + parts of a product, then RMSNorm -> {sum, y}");
+  m.def("rows_glu", &rows_glu, "decode_glu of up to 128 rows as they lie",
+        py::arg("x"), py::arg("ws"), py::arg("N"), py::arg("gelu"),
+        py::arg("operand") = false, py::arg("squares") = py::none(),
+        py::arg("eps") = 0.0);
+  m.def("rows_heads", &rows_heads,
+        "decode_heads of up to 128 rows as they lie", py::arg("x"),
+        py::arg("ws"), py::arg("N"), py::arg("cos"), py::arg("sin"),
+        py::arg("positions"), py::arg("k_cache"), py::arg("v_cache"),
+        py::arg("slots"), py::arg("hq"), py::arg("rows") = false);
   m.def("decode_swizzle_w", &decode_swizzle_w,
-        "one-time [N,K] -> fragment-lane-major weight layout");
+        "one-time [N,K] -> fragment-lane-major weight layout", py::arg("w"),
+        py::arg("half") = 0);
   m.def("decode_swizzle_x", &decode_swizzle_x,
         "per-call x -> B-fragment lane order (zero-padded to M=32)");
   m.def("decode_swizzle_w8", &decode_swizzle_w8,
-        "one-time weight layout swizzle for decode_gemm_fp8");
+        "one-time weight layout swizzle for decode_gemm_fp8", py::arg("w8"),
+        py::arg("half") = 0);
   m.def("decode_affine", &decode_affine,
         "act(x W^T + bias) to up to three matrices, or as an operand",
         py::arg("xs"), py::arg("ws"), py::arg("biases"), py::arg("M"),
         py::arg("act") = 0, py::arg("operand") = false);
   m.def("sum_parts", &sum_parts, "fp32 [P, M, N] -> their sum [M, N] bf16");
-  m.def("decode_gemm_rows", &decode_gemm_rows, "x [M <= 128, K] W^T");
+  m.def("decode_gemm_rows", &decode_gemm_rows, "x [M <= 128, K] W^T",
+        py::arg("x"), py::arg("ws"), py::arg("N"), py::arg("half") = 0,
+        py::arg("raw") = false);
   m.def("decode_gemm_fp8", &decode_gemm_fp8,
         "decode GEMM with e4m3 weights and a scale per row",
         py::arg("xs"), py::arg("w8s"), py::arg("scale"), py::arg("M"),
-        py::arg("N"), py::arg("K"), py::arg("raw") = false);
+        py::arg("N"), py::arg("K"), py::arg("raw") = false,
+        py::arg("half") = 0);
   m.def("decode_gemm_split", &decode_gemm_split);
   m.def("decode_gemm_supported", &decode_gemm_supported);
   m.def("sample_tokens", &sample_tokens, "greedy / Gumbel-max sampling");

@@ -42,32 +42,68 @@
 #include <type_traits>
 
 #include "common.h"
+#include "decode_ends.h"
 
 namespace {
 
 constexpr int BLOCK = 256;   // 4 waves
 constexpr int MMAX = 32;
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8v;
-typedef __attribute__((ext_vector_type(16))) float f32x16v;
-typedef __attribute__((ext_vector_type(4))) float f32x4v;
-typedef __attribute__((ext_vector_type(4))) unsigned int u32x4v;
+using ends::bf16x8v;
+using ends::Ends;
+using ends::f32x16v;
+using ends::f32x4v;
+using ends::fp8_to_bf16;
+using ends::Kind;
+using ends::load8v;
+using ends::u32x4v;
 
-__device__ __forceinline__ bf16x8v load8v(const uint16_t *p) {
-  union { u32x4v u; bf16x8v v; } c;
-  c.u = *reinterpret_cast<const u32x4v *>(p);
-  return c.v;
-}
+// What a thread needs for its ends besides the sums; issued before the stream
+// of W (begin) and behind its first loads (rest), so that their ways to memory
+// lie beside its own. A thread's row m is that of its place in finish().
+template <Kind KIND> struct Early {
+  static constexpr int PARTS = 8;       // of 4 squares, for up to 256 in all
+  float4 squares[PARTS];
+  float norm;
+  int position;
+  ends::Turn<2> turn;
+  RB_DEV void begin(const Ends &e, int M) {
+    const int m = min((int)threadIdx.x >> 3, M - 1), i = threadIdx.x & 7;
+    if constexpr (KIND == ends::QKV) position = e.pos[m];
+    if (KIND != ends::SLAB && e.squares != nullptr) {
+#pragma unroll
+      for (int j = 0; j < PARTS; ++j)
+        squares[j] = *reinterpret_cast<const float4 *>(
+            e.squares + (int64_t)m * e.parts +
+            min((j * 8 + i) * 4, e.parts - 4));
+    }
+  }
+  RB_DEV void rest(const Ends &e, int M) {
+    const int m = min((int)threadIdx.x >> 3, M - 1), i = threadIdx.x & 7;
+    norm = 1.0f;
+    if (KIND != ends::SLAB && e.squares != nullptr) {
+      float ss = 0.0f;
+#pragma unroll
+      for (int j = 0; j < PARTS; ++j)
+        if ((j * 8 + i) * 4 < e.parts)
+          ss += (squares[j].x + squares[j].y) + (squares[j].z + squares[j].w);
+#pragma unroll
+      for (int off = 4; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+      norm = rsqrtf(ss * e.inv_d + e.eps);
+    }
+    if constexpr (KIND == ends::QKV)
+      turn.load(e, m, blockIdx.x * 16 + i * 2, position);
+  }
+};
 
-// Sums the four waves' accumulators of 32 rows of W and stores them, times the
-// rows' scales where there are any: y, or a slice of the slabs.
-template <bool STORE_BF16>
-__device__ __forceinline__ void finish(const f32x16v &acc, const float *scale,
-                                       uint16_t *yp, float *slabs, int M,
-                                       int N) {
+// Sums the four waves' accumulators of 32 rows of W, times the rows' scales
+// where there are any, and hands them on.
+template <Kind KIND>
+__device__ __forceinline__ void finish(const f32x16v &acc, const Ends &e,
+                                       const Early<KIND> &early, int M, int N) {
   const int tid = threadIdx.x, wid = tid >> 6;
   const int hi = (tid & 63) >> 5, col = tid & 31;
-  const int nblk = blockIdx.x, kslice = blockIdx.y;
+  const int nblk = blockIdx.x;
   __shared__ __attribute__((aligned(16))) float red[4][32][MMAX];
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
@@ -78,42 +114,31 @@ __device__ __forceinline__ void finish(const f32x16v &acc, const float *scale,
 
   // 1024 outputs, 4 per thread, n fastest so bf16 stores coalesce 8 B.
   const int em = tid >> 3;               // 0..31
-  const int en = (tid & 7) * 4;          // 0,4,..,28
-  if (em < M) {
-    float sum[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      sum[j] = red[0][en + j][em] + red[1][en + j][em] +
-               red[2][en + j][em] + red[3][en + j][em];
-      if (scale != nullptr) sum[j] *= scale[nblk * 32 + en + j];
-    }
-    if (STORE_BF16) {
-      union { uint16_t u[4]; uint64_t q; } o;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) o.u[j] = rb::f32_to_bf16(sum[j]);
-      *reinterpret_cast<uint64_t *>(
-          yp + (int64_t)em * N + nblk * 32 + en) = o.q;
+  if (em >= M) return;
+  auto sum = [&](int r) {
+    float x = red[0][r][em] + red[1][r][em] + red[2][r][em] + red[3][r][em];
+    if (KIND != ends::SLAB) x *= early.norm;
+    if (e.scale != nullptr) x *= e.scale[ends::column(e.half, nblk, r)];
+    return x;
+  };
+  if constexpr (KIND == ends::GLU || KIND == ends::QKV) {
+    const int c = (tid & 7) * 2;
+    float a[2] = {sum(c), sum(c + 1)}, b[2] = {sum(16 + c), sum(17 + c)};
+    if constexpr (KIND == ends::GLU)
+      ends::put_gated<2>(e, em, nblk * 16 + c, N, a, b);
+    else
+      ends::put_heads<2>(e, early.turn, em, nblk * 16 + c, N, a, b);
+  } else {
+    const int en = (tid & 7) * 4;        // 0,4,..,28
+    const int n = ends::column(e.half, nblk, en);
+    const float f[4] = {sum(en), sum(en + 1), sum(en + 2), sum(en + 3)};
+    if constexpr (KIND == ends::PLAIN) {
+      ends::put<4>(e.y + (int64_t)em * N + n, f);
     } else {
-      float *slab = slabs + ((int64_t)kslice * M + em) * N + nblk * 32 + en;
-      *reinterpret_cast<float4 *>(slab) =
-          make_float4(sum[0], sum[1], sum[2], sum[3]);
+      float *slab = e.slabs + ((int64_t)blockIdx.y * M + em) * N + n;
+      *reinterpret_cast<float4 *>(slab) = make_float4(f[0], f[1], f[2], f[3]);
     }
   }
-}
-
-// Two words of e4m3 -> 8 bf16 (exact).
-__device__ __forceinline__ bf16x8v fp8_to_bf16(unsigned lo, unsigned up) {
-  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2v;
-  union { bf16x2v h[4]; bf16x8v v; } c;
-  c.h[0] = __builtin_convertvector(
-      __builtin_amdgcn_cvt_pk_f32_fp8(lo, false), bf16x2v);
-  c.h[1] = __builtin_convertvector(
-      __builtin_amdgcn_cvt_pk_f32_fp8(lo, true), bf16x2v);
-  c.h[2] = __builtin_convertvector(
-      __builtin_amdgcn_cvt_pk_f32_fp8(up, false), bf16x2v);
-  c.h[3] = __builtin_convertvector(
-      __builtin_amdgcn_cvt_pk_f32_fp8(up, true), bf16x2v);
-  return c.v;
 }
 
 // What a lane holds of a kilobyte of W: operands of 32 rows x 16 columns, or of
@@ -124,9 +149,6 @@ template <bool FP8> struct Step {
   bf16x8v x[X];
 };
 
-// STORE_BF16: write y bf16 directly (SPLIT == 1). Otherwise store an
-// fp32 slab slice at slabs + kslice*M*N for decode_gemm_combine.
-//
 // W nontemporal (streamed once, must not evict L2); x plain (re-read by every
 // n-block: L2 is exactly where it wants to live). Columns past M read the last
 // row again: their results are not stored, and x stays as short as it is.
@@ -144,10 +166,10 @@ template <bool FP8> struct Step {
 //         1 row    31.9 -> 13.8  47.3 -> 20.1  17.7 -> 6.3  39.5 -> 12.4
 //         16 rows  32.5 -> 14.1  49.3 -> 20.8  17.7 -> 6.5  37.7 -> 12.8
 //         32 rows  34.7 -> 17.7  56.5 -> 26.4  18.1 -> 7.7  38.1 -> 16.0
-template <bool FP8>
+template <bool FP8, typename Meanwhile>
 __device__ __forceinline__ f32x16v weight_stream(
     const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws, int M,
-    int K) {
+    int K, Meanwhile meanwhile) {
   constexpr int X = Step<FP8>::X, U = FP8 ? 4 : 8;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -185,9 +207,10 @@ __device__ __forceinline__ f32x16v weight_stream(
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w.v, c.x[0], acc, 0, 0, 0);
     }
   };
+  if (s0 < s1) load(a, s0);
+  meanwhile();
   if (s0 < s1) {
     int s = s0;
-    load(a, s);
     for (; s + 2 * U < s1; s += 2 * U) {
       load(b, s + U);
 #pragma unroll
@@ -207,13 +230,15 @@ __device__ __forceinline__ f32x16v weight_stream(
   return acc;
 }
 
-template <bool FP8, bool STORE_BF16>
+template <bool FP8, Kind KIND>
 __global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
-    const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws,
-    const float *__restrict__ scale, uint16_t *__restrict__ yp,
-    float *__restrict__ slabs, int M, int N, int K) {
-  const f32x16v acc = weight_stream<FP8>(xs, ws, M, K);
-  finish<STORE_BF16>(acc, scale, yp, slabs, M, N);
+    const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws, Ends e,
+    int M, int N, int K) {
+  Early<KIND> early;
+  early.begin(e, M);
+  const f32x16v acc =
+      weight_stream<FP8>(xs, ws, M, K, [&] { early.rest(e, M); });
+  finish<KIND>(acc, e, early, M, N);
 }
 
 // act(x W^T + bias) of models whose decode is bound by its launches: the columns
@@ -362,15 +387,15 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_affine_kernel(
 // rows by the tiles of x (3.8 TB/s). W two chunks ahead and a chunk's operands
 // of x read at once: 22016 x 4096 of 45 rows 40.6 -> 34.0 us, 4096 x 4096 15.0 ->
 // 13.5 (library 43 and 23).
-template <int RB, int NWN, int CH, bool STORE_BF16>
+template <int RB, int NWN, int CH, Kind KIND>
 __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
-    const uint16_t *__restrict__ x, const uint8_t *__restrict__ ws,
-    uint16_t *__restrict__ yp, float *__restrict__ slabs, int M, int N, int K) {
+    const uint16_t *__restrict__ x, const uint8_t *__restrict__ ws, Ends e,
+    int M, int N, int K) {
   constexpr int KG = 4 / NWN, P = 2 * CH;          // pieces of a row
   constexpr int XL = RB * CH / NWN;                // of x, a lane and chunk
   constexpr int TILE = RB * 32 * P * 16;
-  static_assert(XL * NWN == RB * CH && (KG == 1 || 2 * KG * TILE >= NWN * RB * 4096),
-                "tiles");
+  static_assert(XL * NWN == RB * CH &&
+                2 * KG * TILE >= (KG - 1) * NWN * RB * 4096, "tiles");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, hi = lane >> 5, col = lane & 31;
@@ -385,6 +410,10 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
   const uint8_t *wseg =
       ws + (int64_t)min(nblk, blocks - 1) * steps * 1024 + lane * 16;
   char *mine = smem + kg * TILE;                   // buffers KG * TILE apart
+  constexpr bool NORM = RB == 1 && KIND != ends::SLAB;
+  __shared__ float norms[NORM ? MMAX : 1];
+  Early<ends::PLAIN> early;
+  if constexpr (NORM) early.begin(e, M);
 
   struct X { u32x4v v[XL]; };
   struct W { u32x4v v[CH]; };
@@ -437,6 +466,10 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
   put_x(xr, mine);
   load_x(xr, s0 + CH);
   load_w(w1, s0 + CH);
+  if constexpr (NORM) {
+    early.rest(e, M);
+    if (threadIdx.x % 8 == 0) norms[threadIdx.x / 8] = early.norm;
+  }
   meet();
   // chunk c, of which `w` holds W and then W of chunk c + 2
   auto step = [&](W &w, int c, auto whole) {
@@ -472,40 +505,77 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
     step(w1, c + 1, std::false_type{});
   }
   // sum of the groups
-  if constexpr (KG == 2) {
+  if constexpr (KG > 1) {
     float *red = reinterpret_cast<float *>(smem) + wn * RB * 1024 + lane;
-    if (kg == 1) {
+    if (kg > 0) {
 #pragma unroll
       for (int b = 0; b < RB; ++b)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) red[(b * 16 + r) * 64] = acc[b][r];
+        for (int r = 0; r < 16; ++r)
+          red[((kg - 1) * NWN * RB + b) * 1024 + r * 64] = acc[b][r];
     }
     __syncthreads();
-    if (kg == 1) return;
+    if (kg > 0) return;
 #pragma unroll
-    for (int b = 0; b < RB; ++b)
+    for (int g = 0; g < KG - 1; ++g)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[b][r] += red[(b * 16 + r) * 64];
+      for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          acc[b][r] += red[(g * NWN * RB + b) * 1024 + r * 64];
   }
   if (nblk >= blocks) return;
+  if constexpr (NORM) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][r] *= norms[col];
+  }
+  if constexpr (KIND == ends::GLU || KIND == ends::QKV) {
+    // registers r and r + 8 of a lane are a pair, 4 neighbours at a time
+    constexpr bool HEADS = KIND == ends::QKV;
+    ends::Turn<4> turn[HEADS ? RB : 1][2];
+    if constexpr (HEADS) {
+#pragma unroll
+      for (int b = 0; b < RB; ++b) {
+        const int m = min(b * 32 + col, M - 1), position = e.pos[m];
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          turn[b][q].load(e, m, nblk * 16 + 8 * q + 4 * hi, position);
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+      const int m = b * 32 + col;
+      if (m >= M) continue;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int p = nblk * 16 + 8 * q + 4 * hi;
+        float f[4], g[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          f[j] = acc[b][4 * q + j];
+          g[j] = acc[b][8 + 4 * q + j];
+        }
+        if constexpr (HEADS) ends::put_heads<4>(e, turn[b][q], m, p, N, f, g);
+        else ends::put_gated<4>(e, m, p, N, f, g);
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int b = 0; b < RB; ++b) {
     const int m = b * 32 + col;
     if (m >= M) continue;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int n = nblk * 32 + 8 * q + 4 * hi;
-      if (STORE_BF16) {
-        union { uint16_t u[4]; uint64_t q; } o;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o.u[j] = rb::f32_to_bf16(acc[b][4 * q + j]);
-        *reinterpret_cast<uint64_t *>(yp + (int64_t)m * N + n) = o.q;
-      } else {
+      const int n = ends::column(e.half, nblk, 8 * q + 4 * hi);
+      const float f[4] = {acc[b][4 * q], acc[b][4 * q + 1], acc[b][4 * q + 2],
+                          acc[b][4 * q + 3]};
+      if constexpr (KIND == ends::PLAIN)
+        ends::put<4>(e.y + (int64_t)m * N + n, f);
+      else
         *reinterpret_cast<float4 *>(
-            slabs + ((int64_t)blockIdx.y * M + m) * N + n) =
-            make_float4(acc[b][4 * q], acc[b][4 * q + 1], acc[b][4 * q + 2],
-                        acc[b][4 * q + 3]);
-      }
+            e.slabs + ((int64_t)blockIdx.y * M + m) * N + n) =
+            make_float4(f[0], f[1], f[2], f[3]);
     }
   }
 }
@@ -583,14 +653,24 @@ bool decode_gemm_supported(int64_t M, int64_t N, int64_t K) {
   return M >= 1 && M <= MMAX && N % 32 == 0 && K % 16 == 0 && K >= 1024;
 }
 
+static at::Tensor in_pairs(const at::Tensor &w, int64_t half) {
+  if (half == 0) return w;
+  const int64_t N = w.size(0), K = w.size(1);
+  TORCH_CHECK(half > 0 && half % 16 == 0 && N % (2 * half) == 0,
+              "decode_swizzle_w: pairs");
+  return w.view({N / (2 * half), 2, half / 16, 16, K}).transpose(1, 2)
+      .reshape({N, K});
+}
+
 // One-time weight swizzle (host-side tensor ops): [N,K] ->
 // [N/32][K/16][2][32][8] = fragment-lane-major chunks of 1 KiB.
-at::Tensor decode_swizzle_w(at::Tensor w) {
+// With `half` its rows go in pairs (decode_ends.h).
+at::Tensor decode_swizzle_w(at::Tensor w, int64_t half) {
   TORCH_CHECK(w.dim() == 2 && w.scalar_type() == at::kBFloat16 &&
               w.is_contiguous(), "decode_swizzle_w: contiguous bf16 [N,K]");
   const int64_t N = w.size(0), K = w.size(1);
   TORCH_CHECK(N % 32 == 0 && K % 16 == 0, "decode_swizzle_w: shape");
-  return w.view({N / 32, 32, K / 16, 2, 8})
+  return in_pairs(w, half).view({N / 32, 32, K / 16, 2, 8})
       .permute({0, 2, 3, 1, 4}).contiguous();
 }
 
@@ -610,36 +690,48 @@ at::Tensor decode_swizzle_x(at::Tensor x) {
 
 // e4m3 bytes [N,K] -> [N/32][K/32][2][32][2][8]: a lane's 16 bytes are its
 // operands of two steps of 16 columns.
-at::Tensor decode_swizzle_w8(at::Tensor w8) {
+at::Tensor decode_swizzle_w8(at::Tensor w8, int64_t half) {
   TORCH_CHECK(w8.dim() == 2 && w8.scalar_type() == at::kByte &&
               w8.is_contiguous(), "decode_swizzle_w8: contiguous bytes [N,K]");
   const int64_t N = w8.size(0), K = w8.size(1);
   TORCH_CHECK(N % 32 == 0 && K % 32 == 0, "decode_swizzle_w8: shape");
-  return w8.view({N / 32, 32, K / 32, 2, 2, 8})
+  return in_pairs(w8, half).view({N / 32, 32, K / 32, 2, 2, 8})
       .permute({0, 2, 4, 1, 3, 5}).contiguous();
 }
 
-// Raw variant for fused consumers: split == 1 returns y bf16 [M, N] (with
-// f32 a slab of one slice); split > 1 returns the fp32 slab [split, M, N]
-// UNCOMBINED — the consumer kernel (rmsnorm_res_slab_fwd_dec) folds the
-// slices while it reads, saving the combine launch inside the decode graph.
 template <bool FP8>
-static void launch(const at::Tensor &xs, const at::Tensor &ws,
-                   const float *scale, at::Tensor *y, at::Tensor *slabs,
-                   int split, int64_t M, int64_t N, int64_t K) {
-  const dim3 grid((unsigned)(N / 32), (unsigned)split);
-  auto stream = at::cuda::getCurrentHIPStream();
-  if (slabs == nullptr)
-    hipLaunchKernelGGL((decode_gemm_kernel<FP8, true>), grid, dim3(BLOCK), 0,
-                       stream, (const uint16_t *)xs.data_ptr(),
-                       (const uint8_t *)ws.data_ptr(), scale,
-                       (uint16_t *)y->data_ptr(), nullptr, (int)M, (int)N,
+static void launch(Kind kind, const at::Tensor &xs, const at::Tensor &ws,
+                   const Ends &e, int split, int64_t M, int64_t N, int64_t K) {
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(N / 32), (unsigned)split),
+                       dim3(BLOCK), 0, at::cuda::getCurrentHIPStream(),
+                       (const uint16_t *)xs.data_ptr(),
+                       (const uint8_t *)ws.data_ptr(), e, (int)M, (int)N,
                        (int)K);
-  else
-    hipLaunchKernelGGL((decode_gemm_kernel<FP8, false>), grid, dim3(BLOCK), 0,
-                       stream, (const uint16_t *)xs.data_ptr(),
-                       (const uint8_t *)ws.data_ptr(), scale, nullptr,
-                       slabs->data_ptr<float>(), (int)M, (int)N, (int)K);
+  };
+  switch (kind) {
+    case ends::SLAB: return go(decode_gemm_kernel<FP8, ends::SLAB>);
+    case ends::PLAIN: return go(decode_gemm_kernel<FP8, ends::PLAIN>);
+    case ends::GLU: return go(decode_gemm_kernel<FP8, ends::GLU>);
+    case ends::QKV: return go(decode_gemm_kernel<FP8, ends::QKV>);
+  }
+}
+
+// The sums of a product as slabs [split, M, N], or, unsplit, y [M, N] bf16.
+template <bool FP8>
+static at::Tensor sums(const at::Tensor &xs, const at::Tensor &ws, Ends e,
+                       int split, bool slab, int64_t M, int64_t N, int64_t K) {
+  at::Tensor out;
+  if (slab) {
+    out = at::empty({split, M, N}, xs.options().dtype(at::kFloat));
+    e.slabs = out.data_ptr<float>();
+  } else {
+    out = at::empty({M, N}, xs.options());
+    e.y = (uint16_t *)out.data_ptr();
+  }
+  if (N > 0)
+    launch<FP8>(slab ? ends::SLAB : ends::PLAIN, xs, ws, e, split, M, N, K);
+  return out;
 }
 
 static void combine(const at::Tensor &slabs, at::Tensor &y) {
@@ -714,47 +806,122 @@ at::Tensor sum_parts(at::Tensor parts) {
   return y;
 }
 
+// An operand [K/16][2][32][8] and W [N, K] as decode_swizzle_w or
+// decode_swizzle_w8 (with the scales of its rows) lays it.
+static bool check_product(const at::Tensor &xs, const at::Tensor &ws,
+                          const c10::optional<at::Tensor> &scale, int64_t M,
+                          int64_t N, int64_t K, int64_t half) {
+  const bool fp8 = ws.scalar_type() == at::kByte;
+  TORCH_CHECK(xs.is_cuda() && ws.device() == xs.device() &&
+              xs.is_contiguous() && ws.is_contiguous() &&
+              xs.scalar_type() == at::kBFloat16 &&
+              (fp8 || ws.scalar_type() == at::kBFloat16), "decode_gemm: inputs");
+  TORCH_CHECK(M >= 1 && M <= MMAX && N >= 0 && N % 32 == 0 && K > 0 &&
+              K % (fp8 ? 32 : 16) == 0 && xs.numel() == (K / 16) * 512 &&
+              ws.numel() == N * K &&
+              (fp8 || decode_gemm_supported(M, N, K)), "decode_gemm: shape ",
+              M, "x", N, "x", K);
+  TORCH_CHECK(half == 0 ||
+              (half > 0 && half % 16 == 0 && N % (2 * half) == 0),
+              "decode_gemm: pairs");
+  TORCH_CHECK(fp8 == scale.has_value() &&
+              (!fp8 || (scale->device() == xs.device() &&
+                        scale->is_contiguous() &&
+                        scale->scalar_type() == at::kFloat &&
+                        scale->numel() == N)), "decode_gemm: scales");
+  return fp8;
+}
+
+// The input came without its norm's 1 / rms: `squares` [M, parts] are parts of
+// the sums of squares of its rows of d.
+static void set_squares(Ends &e, const c10::optional<at::Tensor> &squares,
+                        int64_t M, int64_t d, double eps) {
+  if (!squares.has_value()) return;
+  TORCH_CHECK(squares->is_cuda() && squares->is_contiguous() &&
+              squares->dim() == 2 && squares->size(0) == M &&
+              squares->size(1) % 4 == 0 && squares->size(1) > 0 &&
+              squares->size(1) <= 256 &&
+              squares->scalar_type() == at::kFloat &&
+              reinterpret_cast<uintptr_t>(squares->data_ptr()) % 16 == 0,
+              "decode_gemm: squares [M, 4 n <= 256]");
+  e.squares = squares->data_ptr<float>();
+  e.parts = (int)squares->size(1);
+  e.inv_d = 1.0f / (float)d;
+  e.eps = (float)eps;
+}
+
+// Where queries, keys and values [M, N] of heads go.
+static void set_heads(Ends &e, int64_t M, int64_t N, const at::Tensor &cos,
+                      const at::Tensor &sin, const at::Tensor &positions,
+                      const at::Tensor &k_cache, const at::Tensor &v_cache,
+                      const at::Tensor &slots, int64_t hq) {
+  TORCH_CHECK(k_cache.is_cuda() && k_cache.dim() == 4 && v_cache.dim() == 4 &&
+              k_cache.scalar_type() == at::kBFloat16 &&
+              v_cache.scalar_type() == at::kBFloat16 &&
+              k_cache.is_contiguous() && v_cache.is_contiguous() &&
+              reinterpret_cast<uintptr_t>(k_cache.data_ptr()) % 8 == 0 &&
+              reinterpret_cast<uintptr_t>(v_cache.data_ptr()) % 8 == 0,
+              "decode_heads: caches");
+  e.hq = (int)hq;
+  e.hkv = (int)k_cache.size(1);
+  e.bs = (int)k_cache.size(2);
+  e.dh = (int)k_cache.size(3);
+  const int64_t dh = e.dh;
+  TORCH_CHECK(dh % 32 == 0 && dh > 0 && e.bs > 0 && hq > 0 && e.hkv > 0 &&
+              (hq + 2 * e.hkv) * dh == N &&
+              v_cache.numel() == k_cache.numel() &&
+              v_cache.size(1) == k_cache.size(1), "decode_heads: widths");
+  e.vt = v_cache.size(3) == e.bs && v_cache.size(2) == dh && dh != e.bs;
+  TORCH_CHECK(positions.is_cuda() && slots.is_cuda() &&
+              positions.scalar_type() == at::kInt &&
+              slots.scalar_type() == at::kInt && positions.is_contiguous() &&
+              slots.is_contiguous() && positions.numel() >= M &&
+              slots.numel() >= M, "decode_heads: positions, slots");
+  TORCH_CHECK(cos.is_cuda() && sin.is_cuda() &&
+              cos.scalar_type() == at::kFloat &&
+              sin.scalar_type() == at::kFloat && cos.is_contiguous() &&
+              sin.is_contiguous() && cos.size(-1) == dh / 2 &&
+              sin.sizes() == cos.sizes() &&
+              reinterpret_cast<uintptr_t>(cos.data_ptr()) % 8 == 0 &&
+              reinterpret_cast<uintptr_t>(sin.data_ptr()) % 8 == 0,
+              "decode_heads: tables");
+  e.half = (int)(dh / 2);
+  e.cs = cos.data_ptr<float>();
+  e.sn = sin.data_ptr<float>();
+  e.pos = positions.data_ptr<int32_t>();
+  e.slots = slots.data_ptr<int32_t>();
+  e.k_cache = (uint16_t *)k_cache.data_ptr();
+  e.v_cache = (uint16_t *)v_cache.data_ptr();
+}
+
+// Raw variant for fused consumers: split == 1 returns y bf16 [M, N] (with
+// f32 a slab of one slice); split > 1 returns the fp32 slab [split, M, N]
+// UNCOMBINED — the consumer kernel (rmsnorm_res_slab_fwd) folds the
+// slices while it reads, saving the combine launch inside the decode graph.
 at::Tensor decode_gemm_raw(at::Tensor xs, at::Tensor ws, int64_t M,
-                           int64_t N, int64_t K, bool f32) {
-  TORCH_CHECK(xs.is_cuda() && ws.is_cuda() && xs.is_contiguous() &&
-              ws.is_contiguous() && xs.scalar_type() == at::kBFloat16 &&
-              ws.scalar_type() == at::kBFloat16, "decode_gemm_raw: inputs");
-  TORCH_CHECK(xs.numel() == (K / 16) * 512 && ws.numel() == N * K &&
-              decode_gemm_supported(M, N, K), "decode_gemm_raw: shape");
+                           int64_t N, int64_t K, bool f32, int64_t half) {
+  TORCH_CHECK(!check_product(xs, ws, c10::nullopt, M, N, K, half),
+              "decode_gemm_raw: bf16");
+  Ends e{};
+  e.half = (int)half;
   const int split = (int)decode_gemm_split(N, K);
-  if (split == 1 && !f32) {
-    auto y = at::empty({M, N}, xs.options());
-    launch<false>(xs, ws, nullptr, &y, nullptr, 1, M, N, K);
-    return y;
-  }
-  auto slabs = at::empty({split, M, N}, xs.options().dtype(at::kFloat));
-  launch<false>(xs, ws, nullptr, nullptr, &slabs, split, M, N, K);
-  return slabs;
+  return sums<false>(xs, ws, e, split, split > 1 || f32, M, N, K);
 }
 
 // xs from decode_swizzle_x, ws from decode_swizzle_w; M/N/K of the
 // ORIGINAL y[M,N] = x[M,K] @ W[N,K]^T problem.
 at::Tensor decode_gemm(at::Tensor xs, at::Tensor ws, int64_t M, int64_t N,
-                       int64_t K, int64_t force_split) {
-  TORCH_CHECK(xs.is_cuda() && ws.is_cuda() && xs.is_contiguous() &&
-              ws.is_contiguous(), "decode_gemm: contiguous GPU tensors");
-  TORCH_CHECK(xs.scalar_type() == at::kBFloat16 &&
-              ws.scalar_type() == at::kBFloat16, "decode_gemm: bf16 only");
-  TORCH_CHECK(xs.numel() == (K / 16) * 512, "decode_gemm: xs size");
-  TORCH_CHECK(ws.numel() == N * K, "decode_gemm: ws size");
-  TORCH_CHECK(decode_gemm_supported(M, N, K),
-              "decode_gemm: unsupported shape ", M, "x", N, "x", K);
-
-  auto y = at::empty({M, N}, xs.options());
+                       int64_t K, int64_t force_split, int64_t half) {
+  TORCH_CHECK(!check_product(xs, ws, c10::nullopt, M, N, K, half),
+              "decode_gemm: bf16 only");
+  Ends e{};
+  e.half = (int)half;
   const int split = force_split > 0 ? (int)force_split
                                     : (int)decode_gemm_split(N, K);
-  if (split == 1) {
-    launch<false>(xs, ws, nullptr, &y, nullptr, 1, M, N, K);
-    return y;
-  }
-  auto slabs = at::empty({split, M, N}, xs.options().dtype(at::kFloat));
-  launch<false>(xs, ws, nullptr, nullptr, &slabs, split, M, N, K);
-  combine(slabs, y);
+  auto out = sums<false>(xs, ws, e, split, split > 1, M, N, K);
+  if (split == 1) return out;
+  auto y = at::empty({M, N}, xs.options());
+  combine(out, y);
   return y;
 }
 
@@ -762,55 +929,112 @@ at::Tensor decode_gemm(at::Tensor xs, at::Tensor ws, int64_t M, int64_t N,
 // y [M, N] bf16, or with raw=true, where it is split, the uncombined fp32
 // slabs [split, M, N].
 at::Tensor decode_gemm_fp8(at::Tensor xs, at::Tensor w8s, at::Tensor scale,
-                           int64_t M, int64_t N, int64_t K, bool raw) {
-  TORCH_CHECK(xs.is_cuda() && w8s.is_cuda() && scale.is_cuda() &&
-              xs.is_contiguous() && w8s.is_contiguous() &&
-              scale.is_contiguous() && xs.scalar_type() == at::kBFloat16 &&
-              w8s.scalar_type() == at::kByte &&
-              scale.scalar_type() == at::kFloat, "decode_gemm_fp8: inputs");
-  TORCH_CHECK(M >= 1 && M <= MMAX && N % 32 == 0 && K % 32 == 0 && K > 0 &&
-              xs.numel() == (K / 16) * 512 && w8s.numel() == N * K &&
-              scale.numel() == N, "decode_gemm_fp8: shape");
+                           int64_t M, int64_t N, int64_t K, bool raw,
+                           int64_t half) {
+  TORCH_CHECK(check_product(xs, w8s, scale, M, N, K, half),
+              "decode_gemm_fp8: inputs");
+  Ends e{};
+  e.half = (int)half;
+  e.scale = scale.data_ptr<float>();
   const int split = (int)decode_gemm_split(N, K);
-  auto y = split > 1 && raw ? at::Tensor() : at::empty({M, N}, xs.options());
-  if (split == 1) {
-    if (N > 0)
-      launch<true>(xs, w8s, scale.data_ptr<float>(), &y, nullptr, 1, M, N, K);
-    return y;
+  auto out = sums<true>(xs, w8s, e, split, split > 1, M, N, K);
+  if (split == 1 || raw) return out;
+  auto y = at::empty({M, N}, xs.options());
+  combine(out, y);
+  return y;
+}
+
+static void launch_ends(Kind kind, const at::Tensor &xs, const at::Tensor &ws,
+                        const c10::optional<at::Tensor> &scale, Ends &e,
+                        int64_t M, int64_t N, int64_t K) {
+  if (scale.has_value()) {
+    e.scale = scale->data_ptr<float>();
+    launch<true>(kind, xs, ws, e, 1, M, N, K);
+  } else {
+    launch<false>(kind, xs, ws, e, 1, M, N, K);
   }
-  auto slabs = at::empty({split, M, N}, xs.options().dtype(at::kFloat));
-  launch<true>(xs, w8s, scale.data_ptr<float>(), nullptr, &slabs, split, M, N,
-               K);
-  if (raw) return slabs;
-  combine(slabs, y);
+}
+
+// Gate and unit of a gated unit in one product: act(x G^T) * (x U^T) as the
+// operand of the next one. W = [G ; U], its copy paired by half its rows;
+// squares: set_squares.
+at::Tensor decode_glu(at::Tensor xs, at::Tensor ws,
+                      c10::optional<at::Tensor> scale, int64_t M, int64_t N,
+                      int64_t K, bool gelu, c10::optional<at::Tensor> squares,
+                      double eps) {
+  check_product(xs, ws, scale, M, N, K, N / 2);
+  TORCH_CHECK(N > 0, "decode_glu: rows");
+  Ends e{};
+  e.half = (int)(N / 2);
+  e.gelu = gelu;
+  set_squares(e, squares, M, K, eps);
+  auto out = at::empty({N / 32 * 512}, xs.options());
+  e.operand = (uint16_t *)out.data_ptr();
+  launch_ends(ends::GLU, xs, ws, scale, e, M, N, K);
+  return out;
+}
+
+// Rotated q [M, hq, dh] of one product; its rotated keys and its values go to
+// the bf16 cache. W's copy is paired by half a head.
+at::Tensor decode_heads(at::Tensor xs, at::Tensor ws,
+                        c10::optional<at::Tensor> scale, int64_t M, int64_t N,
+                        int64_t K, c10::optional<at::Tensor> squares,
+                        double eps, at::Tensor cos, at::Tensor sin,
+                        at::Tensor positions, at::Tensor k_cache,
+                        at::Tensor v_cache, at::Tensor slots, int64_t hq) {
+  Ends e{};
+  set_heads(e, M, N, cos, sin, positions, k_cache, v_cache, slots, hq);
+  check_product(xs, ws, scale, M, N, K, e.half);
+  set_squares(e, squares, M, K, eps);
+  auto q = at::empty({M, hq, e.dh}, xs.options());
+  e.q = (uint16_t *)q.data_ptr();
+  launch_ends(ends::QKV, xs, ws, scale, e, M, N, K);
+  return q;
+}
+
+// The product with the input's norm left out of it (squares: set_squares).
+at::Tensor decode_normed(at::Tensor xs, at::Tensor ws,
+                         c10::optional<at::Tensor> scale, int64_t M, int64_t N,
+                         int64_t K, at::Tensor squares, double eps,
+                         int64_t half) {
+  check_product(xs, ws, scale, M, N, K, half);
+  TORCH_CHECK(N > 0, "decode_normed: rows");
+  Ends e{};
+  e.half = (int)half;
+  set_squares(e, squares, M, K, eps);
+  auto y = at::empty({M, N}, xs.options());
+  e.y = (uint16_t *)y.data_ptr();
+  launch_ends(ends::PLAIN, xs, ws, scale, e, M, N, K);
   return y;
 }
 
 template <int RB, int NWN, int CH>
-static void launch_rows(const at::Tensor &x, const at::Tensor &ws, at::Tensor &y,
-                        int split) {
-  const int64_t M = x.size(0), K = x.size(1), N = y.size(1);
+static void launch_rows(Kind kind, const at::Tensor &x, const at::Tensor &ws,
+                        const Ends &e, int64_t N, int split) {
+  const int64_t M = x.size(0), K = x.size(1);
   constexpr int lds = 2 * (4 / NWN) * RB * 32 * CH * 32;
   static_assert(lds <= 64 * 1024, "tiles");
   TORCH_CHECK(split >= 1 && split * (4 / NWN) <= K / 16, "decode_gemm_rows");
-  const dim3 grid((unsigned)((N / 32 + NWN - 1) / NWN), (unsigned)split);
-  auto go = [&](auto kernel, float *slabs) {
-    hipLaunchKernelGGL(kernel, grid, dim3(BLOCK), lds,
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel,
+                       dim3((unsigned)((N / 32 + NWN - 1) / NWN),
+                            (unsigned)split), dim3(BLOCK), lds,
                        at::cuda::getCurrentHIPStream(),
                        (const uint16_t *)x.data_ptr(),
-                       (const uint8_t *)ws.data_ptr(),
-                       (uint16_t *)y.data_ptr(), slabs, (int)M, (int)N, (int)K);
+                       (const uint8_t *)ws.data_ptr(), e, (int)M, (int)N,
+                       (int)K);
   };
-  if (split == 1) {
-    go(decode_gemm_rows_kernel<RB, NWN, CH, true>, nullptr);
-    return;
+  if (kind == ends::GLU)
+    return go(decode_gemm_rows_kernel<RB, NWN, CH, ends::GLU>);
+  if (kind == ends::QKV)
+    return go(decode_gemm_rows_kernel<RB, NWN, CH, ends::QKV>);
+  if constexpr (NWN > 1) {
+    kind == ends::SLAB ? go(decode_gemm_rows_kernel<RB, NWN, CH, ends::SLAB>)
+                       : go(decode_gemm_rows_kernel<RB, NWN, CH, ends::PLAIN>);
   }
-  auto slabs = at::empty({split, M, N}, x.options().dtype(at::kFloat));
-  go(decode_gemm_rows_kernel<RB, NWN, CH, false>, slabs.data_ptr<float>());
-  combine(slabs, y);
 }
 
-// y [M, N] = x [M, K] W^T of 1 to 128 rows; ws from decode_swizzle_w.
+// How a product of 1 to 128 rows is cut.
 //
 // One workgroup for every CU where it can be had, as a second on some of them
 // has the others wait: four blocks of W for wide weights, unsplit; else two, or
@@ -818,8 +1042,50 @@ static void launch_rows(const at::Tensor &x, const at::Tensor &ws, at::Tensor &y
 // and four at their best split: 4096 x 11008 of 64 rows 25 and 26, of 100 rows
 // 32 and 30; 3072 x 24576 38 and 34, 50 and 41; 4096 x 4096 14 and 16, 17 and
 // 20; 22016 x 4096 of 64 rows 45 and 36, 12288 x 4096 25 and 26).
-at::Tensor decode_gemm_rows(at::Tensor x, at::Tensor ws, int64_t N) {
-  TORCH_CHECK(x.is_cuda() && ws.is_cuda() && x.dim() == 2 &&
+struct Cut { int blocks, split; };
+static Cut cut_of(int64_t M, int64_t N, int64_t K) {
+  Cut c{N >= 20480 || K >= (M <= 64 ? 20480 : 8192) ? 4 : 2, 1};
+  const int64_t wgs = (N / 32 + c.blocks - 1) / c.blocks;
+  while (c.split < 8 && wgs * c.split * 2 <= 256 && K / (c.split * 2) >= 256)
+    c.split *= 2;
+  return c;
+}
+
+// The same for products with ends, which need whole sums: one block of W for a
+// workgroup where two are too few workgroups (6144 x 4096 of 64 rows and its
+// rotation: 25.6 us in two parts and three launches, 23.8 with two blocks whole).
+static Cut whole_cut_of(int64_t M, int64_t N, int64_t K) {
+  Cut c = cut_of(M, N, K);
+  if (c.blocks == 2 && c.split > 1 && M <= 64) c.blocks = 1;
+  c.split = 1;
+  return c;
+}
+
+// Whether such a product is the faster way: of more than 64 rows, workgroups
+// of one block find no registers, and parts win (6144 x 4096 of 128 rows 32.1
+// and 34.7 us).
+bool rows_ends_pay(int64_t M, int64_t N, int64_t K) {
+  return whole_cut_of(M, N, K).blocks == 1 || cut_of(M, N, K).split == 1;
+}
+
+static void run_rows(Kind kind, const at::Tensor &x, const at::Tensor &ws,
+                     const Ends &e, int64_t N, Cut c) {
+  auto go = [&](auto rb) {
+    constexpr int RB = decltype(rb)::value;
+    if constexpr (RB < 4)
+      if (c.blocks == 1) return launch_rows<RB, 1, 4>(kind, x, ws, e, N, 1);
+    if (c.blocks == 2) launch_rows<RB, 2, 4>(kind, x, ws, e, N, c.split);
+    else launch_rows<RB, 4, RB == 4 ? 4 : 8>(kind, x, ws, e, N, c.split);
+  };
+  const int64_t M = x.size(0);
+  if (M <= 32) go(std::integral_constant<int, 1>{});
+  else if (M <= 64) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 4>{});
+}
+
+static void check_rows(const at::Tensor &x, const at::Tensor &ws, int64_t N,
+                       int64_t half) {
+  TORCH_CHECK(x.is_cuda() && ws.device() == x.device() && x.dim() == 2 &&
               x.is_contiguous() && ws.is_contiguous() &&
               x.scalar_type() == at::kBFloat16 &&
               ws.scalar_type() == at::kBFloat16 &&
@@ -829,19 +1095,68 @@ at::Tensor decode_gemm_rows(at::Tensor x, at::Tensor ws, int64_t N) {
   TORCH_CHECK(M >= 1 && M <= 128 && N > 0 && N % 32 == 0 && K % 16 == 0 &&
               K >= 1024 && K < (1 << 24) && ws.numel() == N * K,
               "decode_gemm_rows: shape");
-  auto y = at::empty({M, N}, x.options());
-  const bool four = N >= 20480 || K >= (M <= 64 ? 20480 : 8192);
-  const int64_t wgs = (N / 32 + (four ? 3 : 1)) / (four ? 4 : 2);
-  int split = 1;
-  while (split < 8 && wgs * split * 2 <= 256 && K / (split * 2) >= 256)
-    split *= 2;
-  auto go = [&](auto rb) {
-    constexpr int RB = decltype(rb)::value;
-    if (four) launch_rows<RB, 4, RB == 4 ? 4 : 8>(x, ws, y, split);
-    else launch_rows<RB, 2, 4>(x, ws, y, split);
-  };
-  if (M <= 32) go(std::integral_constant<int, 1>{});
-  else if (M <= 64) go(std::integral_constant<int, 2>{});
-  else go(std::integral_constant<int, 4>{});
+  TORCH_CHECK(half == 0 ||
+              (half > 0 && half % 16 == 0 && N % (2 * half) == 0),
+              "decode_gemm_rows: pairs");
+}
+
+// y [M, N] = x [M, K] W^T of 1 to 128 rows; ws from decode_swizzle_w. raw:
+// where it is split, the fp32 parts [split, M, N].
+at::Tensor decode_gemm_rows(at::Tensor x, at::Tensor ws, int64_t N,
+                            int64_t half, bool raw) {
+  check_rows(x, ws, N, half);
+  const int64_t M = x.size(0), K = x.size(1);
+  const Cut c = cut_of(M, N, K);
+  Ends e{};
+  e.half = (int)half;
+  at::Tensor y, slabs;
+  if (c.split > 1) {
+    slabs = at::empty({c.split, M, N}, x.options().dtype(at::kFloat));
+    e.slabs = slabs.data_ptr<float>();
+  }
+  if (c.split == 1 || !raw) {
+    y = at::empty({M, N}, x.options());
+    e.y = (uint16_t *)y.data_ptr();
+  }
+  run_rows(c.split > 1 ? ends::SLAB : ends::PLAIN, x, ws, e, N, c);
+  if (c.split > 1 && raw) return slabs;
+  if (c.split > 1) combine(slabs, y);
   return y;
+}
+
+// decode_glu of 1 to 128 rows x as they lie: the gated rows [M, N / 2], or,
+// of up to 32 rows (which may come without their 1 / rms), an operand.
+at::Tensor rows_glu(at::Tensor x, at::Tensor ws, int64_t N, bool gelu,
+                    bool operand, c10::optional<at::Tensor> squares,
+                    double eps) {
+  check_rows(x, ws, N, N / 2);
+  const int64_t M = x.size(0), K = x.size(1);
+  TORCH_CHECK(M <= MMAX || !(operand || squares.has_value()),
+              "rows_glu: operand, squares");
+  Ends e{};
+  e.half = (int)(N / 2);
+  e.gelu = gelu;
+  set_squares(e, squares, M, K, eps);
+  auto out = operand ? at::empty({N / 32 * 512}, x.options())
+                     : at::empty({M, N / 2}, x.options());
+  (operand ? e.operand : e.y) = (uint16_t *)out.data_ptr();
+  run_rows(ends::GLU, x, ws, e, N, whole_cut_of(M, N, K));
+  return out;
+}
+
+// decode_heads of 1 to 128 rows x as they lie: rotated q [M, hq, dh], or, in
+// rows, q and k rotated and v side by side [M, N].
+at::Tensor rows_heads(at::Tensor x, at::Tensor ws, int64_t N, at::Tensor cos,
+                      at::Tensor sin, at::Tensor positions, at::Tensor k_cache,
+                      at::Tensor v_cache, at::Tensor slots, int64_t hq,
+                      bool rows) {
+  Ends e{};
+  const int64_t M = x.size(0), K = x.size(1);
+  set_heads(e, M, N, cos, sin, positions, k_cache, v_cache, slots, hq);
+  check_rows(x, ws, N, e.half);
+  auto out = rows ? at::empty({M, N}, x.options())
+                  : at::empty({M, hq, (int64_t)e.dh}, x.options());
+  (rows ? e.y : e.q) = (uint16_t *)out.data_ptr();
+  run_rows(ends::QKV, x, ws, e, N, whole_cut_of(M, N, K));
+  return out;
 }

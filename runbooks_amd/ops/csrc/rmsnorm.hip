@@ -507,6 +507,27 @@ std::vector<at::Tensor> rmsnorm_res_slab_fwd_dec(at::Tensor x,
   return {sum, y, swz};
 }
 
+// The same of any number of rows, without the operand: {sum, y}.
+std::vector<at::Tensor> rmsnorm_res_slab_fwd(at::Tensor x, at::Tensor slabs,
+                                             at::Tensor w, double eps) {
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous() &&
+              slabs.is_contiguous() && w.is_contiguous() &&
+              x.scalar_type() == at::kBFloat16 &&
+              w.scalar_type() == at::kBFloat16 &&
+              slabs.scalar_type() == at::kFloat && slabs.dim() == 3 &&
+              slabs.size(1) == x.size(0) && slabs.size(2) == x.size(1) &&
+              w.numel() == x.size(1) && x.size(1) % 8 == 0,
+              "rmsnorm_res_slab_fwd: x [T, 8 n] bf16, slabs [P, T, 8 n]");
+  auto sum = at::empty_like(x), y = at::empty_like(x);
+  launch_fwd<uint16_t>((const uint16_t *)x.data_ptr(), nullptr,
+                       slabs.data_ptr<float>(), (int)slabs.size(0),
+                       (uint16_t *)sum.data_ptr(),
+                       (const uint16_t *)w.data_ptr(),
+                       (uint16_t *)y.data_ptr(), nullptr, nullptr, x.size(0),
+                       (int)x.size(1), (float)eps);
+  return {sum, y};
+}
+
 // Norm of a 32-bit residual: x += delta in place, y = rmsnorm(x) * (offset + w)
 // in w's dtype. `nd` delta terms of type DT (0: none; > 1: the uncombined split-K
 // slab of decode_gemm_raw) lie n_rows * D apart. swz as above (bf16 only).

@@ -25,16 +25,18 @@ _USE_DECODE_GEMM = os.environ.get("RB_DECODE_GEMM", "1") == "1"
 
 
 # data_ptr(weight) -> (e4m3 bytes in the decode GEMM's order, f32 per-channel
-# scale, the weight's version, weakref to the weight). Populated by quantize_fp8
-# (serving with MODEL_LOAD_IN_8BIT); looked up on the decode fast path.
+# scale, distance of rows in pairs (below), the weight's version, weakref to the
+# weight). Populated by quantize_fp8 (serving with MODEL_LOAD_IN_8BIT); looked up
+# on the decode fast path.
 _FP8_REGISTRY: dict[int, tuple] = {}
 
 # data_ptr(weight) -> fragment-lane-major copy ([N/32][K/16][lane][8])
 # consumed by csrc/decode_gemm.hip. A second full-precision weight copy:
 # 288 GB HBM3E per GPU makes layout-specialized decode weights the right
 # trade on MI355X (prefill/training keep the original [N,K] tensor).
-# value: (swizzled copy, (N, K), the weight's version, weakref to the registered
-# tensor).
+# value: (swizzled copy, (N, K), distance of rows in pairs, the weight's version,
+# weakref to the registered tensor). Pairs (csrc/decode_ends.h; 0: rows in order)
+# let a product end in what follows it, a gated unit or a rotation.
 # data_ptr alone is NOT a safe key — a freed weight's address gets
 # recycled by later allocations, so every lookup verifies tensor
 # identity through the weakref (stale entries are dropped lazily).
@@ -80,14 +82,16 @@ def copies_read():
         [w for w in weights if not w.is_inference()]))
 
 
-def register_decode_weight(weight: torch.Tensor) -> None:
-    """Build + register the decode-GEMM weight layout for `weight`."""
+def register_decode_weight(weight: torch.Tensor, half: int = 0) -> None:
+    """Build + register the decode-GEMM weight layout for `weight`; with `half`
+    its rows go in pairs that far apart."""
     for ptr in [p for p, e in _DECODE_W_REGISTRY.items() if e[-1]() is None]:
         del _DECODE_W_REGISTRY[ptr]          # purge dead entries
-    ws = _backend.ext().decode_swizzle_w(weight.data)
+    ws = _backend.ext().decode_swizzle_w(weight.data, half)
     _DECODE_W_REGISTRY[weight.data_ptr()] = (
-        ws, (int(weight.shape[0]), int(weight.shape[1])), _version(weight),
-        weakref.ref(weight))
+        ws, (int(weight.shape[0]), int(weight.shape[1])), half,
+        _version(weight), weakref.ref(weight))
+
 
 E4M3_MAX = 448.0
 
@@ -98,17 +102,19 @@ def _fp8_served(n: int, k: int) -> bool:
 
 
 @torch.no_grad()
-def quantize_fp8(weight: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+def quantize_fp8(weight: torch.Tensor, half: int = 0
+                 ) -> tuple[torch.Tensor, torch.Tensor]:
     """Row-wise (per-output-channel) OCP e4m3 quantization; registers the
-    pair so fast_linear dispatches to the fp8 decode GEMM. Pass the
+    pair so fast_linear dispatches to the fp8 decode GEMM (`half`: as in
+    register_decode_weight, of the copy that it reads). Pass the
     PERSISTENT tensor object (Parameter / fused buffer), not .data —
     lookups verify identity via weakref."""
     scale = weight.float().abs().amax(dim=1).clamp(min=1e-8) / E4M3_MAX
     w8 = (weight.float() / scale[:, None]).to(torch.float8_e4m3fn)
     w8_bytes = w8.view(torch.uint8).contiguous()
-    served = (_backend.ext().decode_swizzle_w8(w8_bytes)
+    served = (_backend.ext().decode_swizzle_w8(w8_bytes, half)
               if weight.is_cuda and _fp8_served(*weight.shape) else w8_bytes)
-    _FP8_REGISTRY[weight.data_ptr()] = (served, scale.contiguous(),
+    _FP8_REGISTRY[weight.data_ptr()] = (served, scale.contiguous(), half,
                                         _version(weight), weakref.ref(weight))
     return w8_bytes, scale
 
@@ -140,13 +146,13 @@ def fast_linear(x: torch.Tensor, weight: torch.Tensor,
                 q = _registry_get(_FP8_REGISTRY, weight)
                 if q is not None:
                     y = _backend.ext().decode_gemm_fp8(
-                        _swizzled(x, m, k), q[0], q[1], m, n, k)
+                        _swizzled(x, m, k), q[0], q[1], m, n, k, half=q[2])
                     return y.view(*x.shape[:-1], n)
             if _USE_DECODE_GEMM:
                 dw = _registry_get(_DECODE_W_REGISTRY, weight)
                 if dw is not None:
                     y = _backend.ext().decode_gemm(_swizzled(x, m, k), dw[0],
-                                                   m, n, k)
+                                                   m, n, k, half=dw[2])
                     return y.view(*x.shape[:-1], n)
             if _USE_SKINNY and n % 64 == 0 and k % 256 == 0:
                 y = _backend.ext().skinny_gemm(x.reshape(m, k).contiguous(),
@@ -166,6 +172,14 @@ def fast_linear(x: torch.Tensor, weight: torch.Tensor,
     return F.linear(x, weight, bias)
 
 
+def _rows_copy(x: torch.Tensor, weight: torch.Tensor, m: int, n: int, k: int):
+    """The registered copy of `weight` where decode_gemm_rows takes x and it."""
+    if not _USE_DECODE_GEMM or n % 32 or k % 16 or k < 1024 or \
+            not x.is_contiguous() or x.data_ptr() % 16:
+        return None
+    return _registry_get(_DECODE_W_REGISTRY, weight)
+
+
 def _rows_linear(x: torch.Tensor, weight: torch.Tensor, m: int, n: int,
                  k: int) -> torch.Tensor | None:
     """x @ weight^T of up to 128 rows on the decode GEMM that reads x as it is,
@@ -174,14 +188,58 @@ def _rows_linear(x: torch.Tensor, weight: torch.Tensor, m: int, n: int,
     us on the library and there: 64 rows, 22016 x 4096 44.4 and 35.8, 4096 x
     4096 23.0 and 14.1, 4096 x 14336 40.4 and 27.3, 3072 x 24576 102 and 34; 128
     rows, 46.5 and 46.9, 26.9 and 17.6, 76.9 and 32.5, 133 and 43."""
-    if not _USE_DECODE_GEMM or n % 32 or k % 16 or k < 1024 or \
-            not x.is_contiguous() or x.data_ptr() % 16:
-        return None
-    dw = _registry_get(_DECODE_W_REGISTRY, weight)
+    dw = _rows_copy(x, weight, m, n, k)
     if dw is None:
         return None
-    y = _backend.ext().decode_gemm_rows(x.view(m, k), dw[0], n)
+    y = _backend.ext().decode_gemm_rows(x.view(m, k), dw[0], n, dw[2])
     return y.view(*x.shape[:-1], n)
+
+
+def _rows_served(x: torch.Tensor, weight: torch.Tensor):
+    """_rows_copy for results that are not differentiated, of 33 to 128 rows."""
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and
+            32 < x.shape[0] <= 128 and not torch.is_grad_enabled() and
+            weight.is_contiguous()):
+        return None
+    return _rows_copy(x, weight, x.shape[0], weight.shape[0], x.shape[1])
+
+
+def rows_glu(x: torch.Tensor, weight: torch.Tensor, gelu: bool
+             ) -> torch.Tensor | None:
+    """act(x G^T) * (x U^T) of weight = [G ; U] and 33 to 128 rows in one
+    launch, or None where no paired copy serves it (us with the product and the
+    gated unit apart and here, 64 rows: 22016 x 4096 40.2 and 37.6, 49152 x 3072
+    64.5 and 59.1)."""
+    dw, n = _rows_served(x, weight), weight.shape[0]
+    if dw is None or dw[2] * 2 != n or \
+            not _backend.ext().rows_ends_pay(x.shape[0], n, x.shape[1]):
+        return None
+    return _backend.ext().rows_glu(x, dw[0], n, gelu)
+
+
+def rows_heads(x: torch.Tensor, weight: torch.Tensor, cos, sin, positions, kc,
+               vc, slots, hq: int, rows: bool) -> torch.Tensor | None:
+    """The product of 33 to 128 rows with joint weights of q, k and v whose
+    rotation and cache write it does too: q [T, hq, dh], or, in rows, q, k and v
+    side by side; None where no paired copy serves it."""
+    dw, n = _rows_served(x, weight), weight.shape[0]
+    if dw is None or kc.dtype != torch.bfloat16 or \
+            dw[2] * 2 != kc.shape[3] or \
+            not _backend.ext().rows_ends_pay(x.shape[0], n, x.shape[1]):
+        return None
+    return _backend.ext().rows_heads(x, dw[0], n, cos, sin, positions, kc, vc,
+                                     slots, hq, rows)
+
+
+def rows_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
+    """x @ weight^T of 33 to 128 rows for a norm that adds up parts of it
+    (ops.rmsnorm_res): fp32 [P, T, N], or [T, N] where the kernel splits
+    nothing; None where no copy serves it. us with the sum in a launch of its
+    own and in the norm, 64 rows: 4096 x 4096 17.8 and 16.4, 4096 x 11008 29.3
+    and 27.6."""
+    dw = _rows_served(x, weight)
+    return None if dw is None else _backend.ext().decode_gemm_rows(
+        x, dw[0], weight.shape[0], dw[2], True)
 
 
 def _whole_rounds(rows: int, cols: int) -> int:
@@ -281,15 +339,39 @@ def decode_linear_raw(x, weight, f32: bool = False):
         _registry_get(_FP8_REGISTRY, weight)
     if q is not None and m <= 32 and x.dtype == torch.bfloat16:
         out = _backend.ext().decode_gemm_fp8(_swizzled(x, m, k), q[0], q[1],
-                                             m, n, k, True)
+                                             m, n, k, True, q[2])
         return out, out.dtype == torch.float32
     dw = _registry_get(_DECODE_W_REGISTRY, weight)
     if dw is None or not _USE_DECODE_GEMM:
         with torch.no_grad():
             return fast_linear(x, weight), False
     xs = _swizzled(x, m, k)
-    out = _backend.ext().decode_gemm_raw(xs, dw[0], m, n, k, f32)
+    out = _backend.ext().decode_gemm_raw(xs, dw[0], m, n, k, f32, dw[2])
     return out, out.dtype == torch.float32
+
+
+class Copy:
+    """What the decode products of up to 32 rows read of a weight [n, k]."""
+
+    def __init__(self, weight: torch.Tensor):
+        self.n, self.k = weight.shape
+        q = _registry_get(_FP8_REGISTRY, weight) \
+            if _fp8_served(self.n, self.k) else None
+        dw = _registry_get(_DECODE_W_REGISTRY, weight) \
+            if q is None and _USE_DECODE_GEMM else None
+        self.fp8 = q is not None
+        self.ws, self.scale, self.half = \
+            (q[0], q[1], q[2]) if self.fp8 else \
+            (dw[0], None, dw[2]) if dw is not None else (None, None, 0)
+
+    def product(self, xs, m: int):
+        """Of an operand: bf16 [m, n], or fp32 parts [P, m, n] of it."""
+        ext = _backend.ext()
+        if self.fp8:
+            return ext.decode_gemm_fp8(xs, self.ws, self.scale, m, self.n,
+                                       self.k, True, self.half)
+        return ext.decode_gemm_raw(xs, self.ws, m, self.n, self.k,
+                                   half=self.half)
 
 
 def decode_ready(weight: torch.Tensor, m: int) -> bool:

@@ -74,7 +74,12 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.T
 
 def rmsnorm_res(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor,
                 eps: float) -> tuple[torch.Tensor, torch.Tensor]:
-    """x + delta and its norm, differentiable."""
+    """x + delta and its norm, differentiable. delta may come as fp32 parts
+    [P, T, D] of it (ops.rows_parts); their sum is not differentiated."""
+    if delta.dim() == 3 and x.dim() == 2:
+        x, y = _backend.ext().rmsnorm_res_slab_fwd(
+            x.contiguous(), delta, weight.contiguous(), eps)
+        return x, y
     if not _backend.use_hip(x):
         x = x + delta
         return x, rmsnorm_ref(x, weight, eps)

@@ -1,0 +1,260 @@
+"""Decode products with what follows them in the same kernel (csrc/decode_ends.h,
+csrc/decode_res.hip), and the steps of a model that run on them."""
+import dataclasses
+
+import pytest
+import torch
+
+from runbooks_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+# one rounding to bf16 (half a unit of 8 bits), fp32 sums and exponentials
+BF16 = 2 ** -8 + 1e-4
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+def _rows(operand, cols, m):
+    return operand.view(cols // 16, 2, 32, 8).permute(2, 0, 1, 3) \
+        .reshape(32, cols)[:m]
+
+
+def _weight(n, k, half, fp8):
+    """The copy that kernels read, its scales, and its values."""
+    w = torch.randn(n, k, device=DEV).bfloat16()
+    if not fp8:
+        return ops.ext().decode_swizzle_w(w, half), None, w.double()
+    w8 = w.to(torch.float8_e4m3fn)
+    scale = torch.rand(n, device=DEV) + 0.5
+    return (ops.ext().decode_swizzle_w8(w8.view(torch.uint8), half), scale,
+            w8.double() * scale.double()[:, None])
+
+
+def _squares(x, parts):
+    """Sums of squares of x's rows in `parts` uneven parts."""
+    share = torch.rand(x.shape[0], parts, device=DEV)
+    share /= share.sum(1, keepdim=True)
+    return share * x.float().square().sum(1, keepdim=True)
+
+
+def _inverse_rms(x):
+    return (x.double().square().mean(1, keepdim=True) + 1e-5).rsqrt()
+
+
+def _act(g, gelu):
+    return torch.nn.functional.gelu(g, approximate="tanh") if gelu else \
+        torch.nn.functional.silu(g)
+
+
+@pytest.mark.parametrize("m", [1, 5, 16, 17, 32])
+@pytest.mark.parametrize("inter,k,parts", [(16, 1024, None), (48, 1056, 4),
+                                           (5504, 4096, 256)])
+@pytest.mark.parametrize("fp8,gelu", [(False, False), (False, True),
+                                      (True, False)])
+def test_gated_unit(m, inter, k, parts, fp8, gelu):
+    torch.manual_seed(m + inter)
+    ws, scale, w = _weight(2 * inter, k, inter, fp8)
+    x = (torch.randn(m, k, device=DEV) / k ** 0.5).bfloat16()
+    squares = None if parts is None else _squares(x, parts)
+    f = 1.0 if parts is None else _inverse_rms(x)
+    y = f * (x.double() @ w.t())
+    ref = _act(y[:, :inter], gelu) * y[:, inter:]
+    e = ops.ext()
+    h = e.decode_glu(e.decode_swizzle_x(x), ws, scale, m, 2 * inter, k, gelu,
+                     squares, 1e-5)
+    assert _rel(_rows(h, inter, m), ref) < BF16
+    if not fp8:
+        h = e.rows_glu(x, ws, 2 * inter, gelu, True, squares, 1e-5)
+        assert _rel(_rows(h, inter, m), ref) < BF16
+
+
+@pytest.mark.parametrize("m", [1, 33, 64, 65, 128])
+@pytest.mark.parametrize("inter,k", [(16, 1024), (10256, 1040)])
+def test_gated_unit_of_rows(m, inter, k):
+    torch.manual_seed(m + inter)
+    ws, _, w = _weight(2 * inter, k, inter, False)
+    x = (torch.randn(m, k, device=DEV) / k ** 0.5).bfloat16()
+    y = x.double() @ w.t()
+    ref = _act(y[:, :inter], False) * y[:, inter:]
+    assert _rel(ops.ext().rows_glu(x, ws, 2 * inter, False), ref) < BF16
+
+
+def _heads_case(m, hq, hkv, dh, vt):
+    n, k = (hq + 2 * hkv) * dh, 1056
+    cos, sin = ops.rope_tables(dh, 50, device=DEV)
+    pos = torch.randint(0, 50, (m,), dtype=torch.int32, device=DEV)
+    slots = torch.randperm(16 * 10, device=DEV)[:m].to(torch.int32)
+    if m > 2:
+        slots[1] = -1               # written nowhere
+    kc = torch.zeros(10, hkv, 16, dh, device=DEV, dtype=torch.bfloat16)
+    vc = torch.zeros(10, hkv, *((dh, 16) if vt else (16, dh)), device=DEV,
+                     dtype=torch.bfloat16)
+    return n, k, cos, sin, pos, slots, kc, vc
+
+
+def _heads_ref(y, cos, sin, pos, slots, kc, hq, hkv, dh):
+    m = y.shape[0]
+    y = y.view(m, hq + 2 * hkv, dh)
+    c, s = (t.double()[pos.long()][:, None] for t in (cos, sin))
+    a, b = y[:, :hq + hkv].split(dh // 2, -1)
+    turned = torch.cat([a * c - b * s, b * c + a * s], -1)
+    kr, vr = (torch.zeros(kc.shape, dtype=torch.float64, device=DEV)
+              for _ in range(2))
+    for i, t in enumerate(slots.tolist()):
+        if t >= 0:
+            kr[t // 16, :, t % 16] = turned[i, hq:]
+            vr[t // 16, :, t % 16] = y[i, hq + hkv:]
+    return turned[:, :hq], kr, vr, torch.cat([turned, y[:, hq + hkv:]], 1)
+
+
+@pytest.mark.parametrize("m", [1, 16, 32, 33, 64, 65, 128])
+@pytest.mark.parametrize("hq,hkv,dh,vt", [(1, 1, 64, False), (4, 1, 128, True),
+                                          (3, 3, 256, False),
+                                          (48, 24, 128, False)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_heads(m, hq, hkv, dh, vt, fp8):
+    if fp8 and m > 32:
+        pytest.skip("8-bit weights are read by up to 32 rows")
+    torch.manual_seed(m + dh)
+    n, k, cos, sin, pos, slots, kc, vc = _heads_case(m, hq, hkv, dh, vt)
+    ws, scale, w = _weight(n, k, dh // 2, fp8)
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    e, y = ops.ext(), x.double() @ w.t()
+    at = (cos, sin, pos, kc, vc, slots, hq)
+    calls = []
+    if m <= 32:
+        xs, squares = e.decode_swizzle_x(x), _squares(x, 12)
+        calls += [(1.0, lambda: e.decode_heads(xs, ws, scale, m, n, k, None,
+                                               0.0, *at)),
+                  (_inverse_rms(x), lambda: e.decode_heads(
+                      xs, ws, scale, m, n, k, squares, 1e-5, *at))]
+    if not fp8:
+        calls += [(1.0, lambda: e.rows_heads(x, ws, n, *at)),
+                  (1.0, lambda: e.rows_heads(x, ws, n, *at, rows=True))]
+    for f, call in calls:
+        kc.zero_(), vc.zero_()
+        q, kr, vr, rows = _heads_ref(f * y, cos, sin, pos, slots, kc, hq, hkv,
+                                     dh)
+        got = call()
+        assert _rel(got, q if got.dim() == 3 else rows.view(m, n)) < BF16
+        assert _rel(kc, kr) < BF16
+        assert _rel(vc.transpose(-1, -2) if vt else vc, vr) < BF16
+
+
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32])
+@pytest.mark.parametrize("n,k", [(64, 64), (64, 2080), (4096, 4096),
+                                 (3072, 11008)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_residual_sum(m, n, k, fp8):
+    e = ops.ext()
+    if not e.decode_res_supported(m, n, k, fp8):
+        assert fp8 and k % 64
+        return
+    torch.manual_seed(m + n)
+    ws, scale, w = _weight(n, k, 0, fp8)
+    x = (torch.randn(m, k, device=DEV) / k ** 0.5).bfloat16()
+    res = torch.randn(m, n, device=DEV).bfloat16()
+    g = torch.randn(n, device=DEV).bfloat16()
+    ref = res.double() + x.double() @ w.t()
+    for rows in (False, True):
+        s, y, squares = e.decode_res(e.decode_swizzle_x(x), ws, scale, res, g,
+                                     rows)
+        assert _rel(s, ref) < BF16
+        assert _rel(y if rows else _rows(y, n, m), ref * g.double()) < BF16
+        assert squares.shape == (m, n // 16)
+        assert _rel(squares.sum(1), ref.square().sum(1)) < 1e-4
+
+
+@pytest.mark.parametrize("m", [1, 20, 32, 50, 128])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_products_of_paired_copies(m, fp8):
+    """A product that ends in nothing else gives its columns in their own
+    order, whatever the order of the copy, and the same bits."""
+    from runbooks_amd.ops.linear import (decode_linear_raw, fast_linear,
+                                         quantize_fp8, register_decode_weight,
+                                         rows_parts, wide_linear)
+    torch.manual_seed(m)
+    # sizes of each kernel: split or not, in rows or as an operand
+    for n in (1536, 10752):
+        w = torch.randn(n, 2048, device=DEV).bfloat16()
+        x = torch.randn(m, 2048, device=DEV).bfloat16()
+        products = [fast_linear, wide_linear]
+        if m <= 32:
+            products.append(lambda x, w: decode_linear_raw(x, w)[0])
+        elif not fp8:
+            products.append(rows_parts)
+        got = []
+        with torch.no_grad():
+            for half in (0, 64, n // 2):
+                (quantize_fp8 if fp8 else register_decode_weight)(w, half)
+                got.append([p(x, w) for p in products])
+        for paired in got[1:]:
+            for a, b in zip(paired, got[0]):
+                assert torch.equal(a, b)
+
+
+def _model(kv, inter, hidden=1024, eight_bit=False):
+    from runbooks_amd.models import build_model, get_config
+    from runbooks_amd.models.config import register
+    from runbooks_amd.models.transformer import fuse_for_inference
+    cfg = dataclasses.replace(
+        get_config("smoke-llama"), name=f"ends-{kv}-{inter}-{hidden}",
+        hidden_size=hidden, num_heads=8, num_kv_heads=kv, head_dim=128,
+        intermediate_size=inter, num_layers=2)
+    register(cfg)
+    m = build_model(cfg.name, dtype=torch.bfloat16, tp=1, device=DEV, seed=3)
+    return fuse_for_inference(m.eval(), load_in_8bit=eight_bit)
+
+
+def _step(m, batch, fp8):
+    """Arguments of a decode step behind caches of random contents."""
+    g = torch.Generator(device=DEV).manual_seed(batch)
+    caches = m.alloc_caches(batch * 2 + 1, DEV, fp8=fp8)
+    for layer in caches:
+        hkv = layer[0].shape[1]
+        k, v = (torch.randn(batch * 32, hkv, 128, device=DEV,
+                            generator=g).bfloat16() for _ in range(2))
+        ops.kv_append(k, v, *layer, torch.arange(batch * 32, device=DEV,
+                                                 dtype=torch.int32))
+    i32 = dict(dtype=torch.int32, device=DEV)
+    lens = torch.arange(batch, **i32) % 31 + 1
+    return (torch.arange(batch, device=DEV) % 50, lens - 1, caches,
+            torch.arange(batch, **i32) * 32 + lens - 1,
+            torch.arange(2 * batch, **i32).view(batch, 2), lens)
+
+
+@pytest.mark.parametrize("batch", [1, 16, 17, 32])
+@pytest.mark.parametrize("kv,inter,hidden,eight_bit", [
+    (8, 2048, 1024, False), (2, 1040, 1024, False), (8, 6144, 1024, False),
+    (8, 2048, 1024, True), (8, 2048, 4160, False)])
+def test_decode_step(monkeypatch, batch, kv, inter, hidden, eight_bit):
+    """A whole step on these kernels and on the modules: some twenty roundings
+    of 2^-9 a layer, two layers, not in the same places."""
+    from runbooks_amd.models import decode_chain
+    from runbooks_amd.models.transformer import MLP, Attention, Block
+    m = _model(kv, inter, hidden, eight_bit)
+    args = _step(m, batch, eight_bit)
+    with torch.no_grad():
+        assert decode_chain.layers_of(m, Block, Attention, MLP) is not None
+        got = m.decode(*args)
+        monkeypatch.setattr(decode_chain, "layers_of", lambda *a: None)
+        ref = m.decode(*args)
+    assert _rel(got, ref.double()) < 2e-2
+
+
+def test_hooked_modules_are_called():
+    m = _model(8, 2048)
+    args = _step(m, 3, False)
+    seen = []
+    with torch.no_grad():
+        want = m.decode(*args)
+        hook = m.blocks[1].mlp.register_forward_hook(
+            lambda mod, x, y: seen.append(y))
+        got = m.decode(*args)
+        hook.remove()
+    assert len(seen) == 1
+    assert _rel(got, want.double()) < 2e-2

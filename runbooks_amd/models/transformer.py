@@ -142,15 +142,29 @@ class Attention(nn.Module):
                 self.dh in (64, 128, 256) and x.dtype == torch.bfloat16 and
                 kc.dtype in (torch.bfloat16, torch.uint8))
 
-    def forward_prefill(self, x, cos, sin, positions, kc, vc, slot_mapping, B, S):
+    def _out(self, o, parts: bool):
+        """The output projection; with `parts`, possibly as parts of its sums
+        (ops.rows_parts)."""
+        if parts and self.o_proj.bias is None:
+            y = ops.rows_parts(o, self.o_proj.weight)
+            if y is not None:
+                return y
+        return self.o_proj(o)
+
+    def forward_prefill(self, x, cos, sin, positions, kc, vc, slot_mapping, B,
+                        S, parts=False):
         if self._fused_append(x, kc):
-            y = ops.wide_linear(x, self._qkv_w)
-            ops.ext().qkv_rope_append_(y, cos, sin, positions.to(torch.int32),
-                                       kc, vc, slot_mapping.to(torch.int32),
-                                       self.hq)
+            positions = positions.to(torch.int32)
+            slot_mapping = slot_mapping.to(torch.int32)
+            y = ops.rows_heads(x, self._qkv_w, cos, sin, positions, kc, vc,
+                               slot_mapping, self.hq, rows=True)
+            if y is None:
+                y = ops.wide_linear(x, self._qkv_w)
+                ops.ext().qkv_rope_append_(y, cos, sin, positions, kc, vc,
+                                           slot_mapping, self.hq)
             o = ops.ext().flash_prefill_qkv(y, B, S, self.hq, self.hkv,
                                             self.dh, self.scale)
-            return self.o_proj(o.view(B * S, self.hq * self.dh))
+            return self._out(o.view(B * S, self.hq * self.dh), parts)
         q, k, v = self._qkv(x, cos, sin, positions)
         ops.kv_append(k, v, kc, vc, slot_mapping)
         q = q.view(B, S, self.hq, self.dh)
@@ -160,17 +174,21 @@ class Attention(nn.Module):
 
     def forward_decode(self, x, cos, sin, positions, kc, vc, slot_mapping,
                        block_tables, seq_lens, nsplit=None, slab_ok=False,
-                       seq_starts=None):
+                       seq_starts=None, parts=False):
         B = x.shape[0]
         if self._fused_append(x, kc):
             # fused decode hot path: one wide GEMM, then one kernel doing
-            # rope(q), rope(k)->cache, v->cache, quantized where the cache is
-            y = ops.wide_linear(x, self._qkv_w)
+            # rope(q), rope(k)->cache, v->cache, quantized where the cache is;
+            # or one kernel for all of it
             if kc.dtype == torch.uint8:     # whole numbers of any type
                 positions = positions.to(torch.int32)
                 slot_mapping = slot_mapping.to(torch.int32)
-            q = ops.ext().qkv_rope_append(y, cos, sin, positions, kc, vc,
-                                          slot_mapping, self.hq)
+            q = ops.rows_heads(x, self._qkv_w, cos, sin, positions, kc, vc,
+                               slot_mapping, self.hq, rows=False)
+            if q is None:
+                y = ops.wide_linear(x, self._qkv_w)
+                q = ops.ext().qkv_rope_append(y, cos, sin, positions, kc, vc,
+                                              slot_mapping, self.hq)
         else:
             q, k, v = self._qkv(x, cos, sin, positions)
             ops.kv_append(k, v, kc, vc, slot_mapping)
@@ -183,7 +201,7 @@ class Attention(nn.Module):
         if slab_ok and self.tp == 1 and self.o_proj.bias is None:
             out, _ = ops.decode_linear_raw(o2, self.o_proj.weight)
             return out
-        return self.o_proj(o2)
+        return self._out(o2, parts)
 
 
 class MLP(nn.Module):
@@ -202,7 +220,14 @@ class MLP(nn.Module):
         self.down_proj = RowParallelLinear(cfg.intermediate_size, cfg.hidden_size,
                                            bias=cfg.mlp_bias, tp_size=tp, dtype=dtype)
 
-    def forward(self, x, slab_ok=False):
+    def forward(self, x, slab_ok=False, parts=False):
+        if self.act in ("silu_glu", "gelu_glu") and \
+                getattr(self, "_gateup_w", None) is not None:
+            h = ops.rows_glu(x, self._gateup_w, self.act == "gelu_glu")
+            if h is not None:
+                y = ops.rows_parts(h, self.down_proj.weight) \
+                    if parts and self.down_proj.bias is None else None
+                return self.down_proj(h) if y is None else y
         if self.act == "silu_glu":
             if getattr(self, "_gateup_w", None) is not None and \
                     not torch.is_grad_enabled():
@@ -291,9 +316,17 @@ class Block(nn.Module):
                 plain(Block, self) and
                 plain(ops.RMSNorm, self.norm1, self.norm2))
 
-    def forward_pending(self, x, delta, attn_fn):
+    def adds_parts(self) -> bool:
+        """fuses_residual(), and what its sublayers return goes there straight
+        from their last product, so that it may come as parts of its sums."""
+        return (self.attn.tp == 1 and not torch.is_grad_enabled() and
+                self.fuses_residual() and plain(MLP, self.mlp) and
+                plain(RowParallelLinear, self.attn.o_proj, self.mlp.down_proj))
+
+    def forward_pending(self, x, delta, attn_fn, parts=False):
         """forward() of a residual whose last term is still to be added:
-        x + delta -> (x, delta)."""
+        x + delta -> (x, delta). With `parts`, the new delta may be parts of
+        it (ops.rows_parts)."""
         if delta is None:
             h = self.norm1(x)
         else:
@@ -301,7 +334,7 @@ class Block(nn.Module):
                                    self.norm1.eps)
         x, h = ops.rmsnorm_res(x, attn_fn(h), self.norm2.weight,
                                self.norm2.eps)
-        return x, self.mlp(h)
+        return x, self.mlp(h, parts=True) if parts else self.mlp(h)
 
     def forward_decode_fused(self, x_base, delta, attn_fn):
         """Decode hot path (sequential-residual RMSNorm models): the
@@ -476,9 +509,14 @@ class Transformer(nn.Module):
                 h = ops.norm_res32(blk.norm2, x, delta, dtype)
                 delta = blk.mlp(h)
             return x, delta
-        for blk in self.blocks:
+        blocks = list(self.blocks)
+        for blk, after in zip(blocks, blocks[1:] + [None]):
             if blk.fuses_residual():
-                x, delta = run(blk.forward_pending, x, delta, attention(blk))
+                # the norm after the last block may see a part of the rows
+                parts = after is not None and blk.adds_parts() and \
+                    after.fuses_residual()
+                x, delta = run(blk.forward_pending, x, delta, attention(blk),
+                               parts)
             else:
                 if delta is not None:
                     x, delta = x + delta, None
@@ -535,7 +573,7 @@ class Transformer(nn.Module):
             kc, vc = cache_of[blk]
             return lambda h: blk.attn.forward_prefill(
                 h, self.rope_cos, self.rope_sin, positions, kc, vc,
-                slot_mapping, B, S)
+                slot_mapping, B, S, parts=blk.adds_parts())
 
         x = self._last_norm(*(None if r is None else r.view(B, S, -1)[:, -1]
                               for r in self._blocks(x, attention)))
@@ -604,7 +642,7 @@ class Transformer(nn.Module):
             return lambda h: blk.attn.forward_decode(
                 h, self.rope_cos, self.rope_sin, positions, kc, vc,
                 slot_mapping, block_tables, seq_lens, nsplit=nsplit,
-                seq_starts=seq_starts)
+                seq_starts=seq_starts, parts=blk.adds_parts())
 
         x = self._last_norm(*self._blocks(x, attention))
         logits = self.lm_head(x)

@@ -653,13 +653,10 @@ bool decode_gemm_supported(int64_t M, int64_t N, int64_t K) {
   return M >= 1 && M <= MMAX && N % 32 == 0 && K % 16 == 0 && K >= 1024;
 }
 
-static at::Tensor in_pairs(const at::Tensor &w, int64_t half) {
-  if (half == 0) return w;
-  const int64_t N = w.size(0), K = w.size(1);
-  TORCH_CHECK(half > 0 && half % 16 == 0 && N % (2 * half) == 0,
-              "decode_swizzle_w: pairs");
-  return w.view({N / (2 * half), 2, half / 16, 16, K}).transpose(1, 2)
-      .reshape({N, K});
+static void check_pairs(int64_t N, int64_t half) {
+  TORCH_CHECK(half == 0 ||
+              (half > 0 && half % 16 == 0 && N % (2 * half) == 0),
+              "decode_gemm: pairs");
 }
 
 // One-time weight swizzle (host-side tensor ops): [N,K] ->
@@ -670,8 +667,12 @@ at::Tensor decode_swizzle_w(at::Tensor w, int64_t half) {
               w.is_contiguous(), "decode_swizzle_w: contiguous bf16 [N,K]");
   const int64_t N = w.size(0), K = w.size(1);
   TORCH_CHECK(N % 32 == 0 && K % 16 == 0, "decode_swizzle_w: shape");
-  return in_pairs(w, half).view({N / 32, 32, K / 16, 2, 8})
-      .permute({0, 2, 3, 1, 4}).contiguous();
+  check_pairs(N, half);
+  if (half == 0)
+    return w.view({N / 32, 32, K / 16, 2, 8})
+        .permute({0, 2, 3, 1, 4}).contiguous();
+  return w.view({N / (2 * half), 2, half / 16, 16, K / 16, 2, 8})
+      .permute({0, 2, 4, 5, 1, 3, 6}).contiguous();
 }
 
 at::Tensor decode_swizzle_x(at::Tensor x) {
@@ -695,8 +696,12 @@ at::Tensor decode_swizzle_w8(at::Tensor w8, int64_t half) {
               w8.is_contiguous(), "decode_swizzle_w8: contiguous bytes [N,K]");
   const int64_t N = w8.size(0), K = w8.size(1);
   TORCH_CHECK(N % 32 == 0 && K % 32 == 0, "decode_swizzle_w8: shape");
-  return in_pairs(w8, half).view({N / 32, 32, K / 32, 2, 2, 8})
-      .permute({0, 2, 4, 1, 3, 5}).contiguous();
+  check_pairs(N, half);
+  if (half == 0)
+    return w8.view({N / 32, 32, K / 32, 2, 2, 8})
+        .permute({0, 2, 4, 1, 3, 5}).contiguous();
+  return w8.view({N / (2 * half), 2, half / 16, 16, K / 32, 2, 2, 8})
+      .permute({0, 2, 4, 6, 1, 3, 5, 7}).contiguous();
 }
 
 template <bool FP8>
@@ -821,9 +826,7 @@ static bool check_product(const at::Tensor &xs, const at::Tensor &ws,
               ws.numel() == N * K &&
               (fp8 || decode_gemm_supported(M, N, K)), "decode_gemm: shape ",
               M, "x", N, "x", K);
-  TORCH_CHECK(half == 0 ||
-              (half > 0 && half % 16 == 0 && N % (2 * half) == 0),
-              "decode_gemm: pairs");
+  check_pairs(N, half);
   TORCH_CHECK(fp8 == scale.has_value() &&
               (!fp8 || (scale->device() == xs.device() &&
                         scale->is_contiguous() &&
@@ -1095,9 +1098,7 @@ static void check_rows(const at::Tensor &x, const at::Tensor &ws, int64_t N,
   TORCH_CHECK(M >= 1 && M <= 128 && N > 0 && N % 32 == 0 && K % 16 == 0 &&
               K >= 1024 && K < (1 << 24) && ws.numel() == N * K,
               "decode_gemm_rows: shape");
-  TORCH_CHECK(half == 0 ||
-              (half > 0 && half % 16 == 0 && N % (2 * half) == 0),
-              "decode_gemm_rows: pairs");
+  check_pairs(N, half);
 }
 
 // y [M, N] = x [M, K] W^T of 1 to 128 rows; ws from decode_swizzle_w. raw:

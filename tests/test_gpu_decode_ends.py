@@ -258,3 +258,40 @@ def test_hooked_modules_are_called():
         hook.remove()
     assert len(seen) == 1
     assert _rel(got, want.double()) < 2e-2
+
+
+@pytest.mark.parametrize("batch", [33, 64, 65, 128])
+@pytest.mark.parametrize("kv,inter", [(8, 2048), (2, 1040), (2, 12288)])
+def test_wide_decode_step(monkeypatch, batch, kv, inter):
+    """As test_decode_step, of more rows."""
+    m = _model(kv, inter)
+    args = _step(m, batch, False)
+    with torch.no_grad():
+        got = m.decode(*args)
+        for name in ("rows_heads", "rows_glu", "rows_parts"):
+            monkeypatch.setattr(ops, name, lambda *a, **k: None)
+        ref = m.decode(*args)
+    assert _rel(got, ref.double()) < 2e-2
+
+
+@pytest.mark.parametrize("tokens", [31, 33, 128, 129])
+@pytest.mark.parametrize("kv", [2, 8])
+def test_short_prompt(monkeypatch, tokens, kv):
+    """Logits and cached keys and values of a prompt on these kernels and on the
+    modules; the bound as in test_decode_step."""
+    m = _model(kv, 2048)
+    i32 = dict(dtype=torch.int32, device=DEV)
+
+    def prompt():
+        caches = m.alloc_caches(16, DEV)
+        with torch.no_grad():
+            logits = m.prefill(torch.arange(tokens, device=DEV)[None] % 50,
+                               torch.arange(tokens, **i32), caches,
+                               torch.arange(tokens, **i32) + 5)
+        return [logits] + [c for layer in caches for c in layer]
+
+    got = prompt()
+    for name in ("rows_heads", "rows_glu", "rows_parts"):
+        monkeypatch.setattr(ops, name, lambda *a, **k: None)
+    for a, b in zip(got, prompt()):
+        assert _rel(a, b.double()) < 2e-2

@@ -599,6 +599,12 @@ class Transformer(nn.Module):
                 seq_of=self._decode_cu[B][:B], rows=None,
                 n_seqs=B, n_short=B, t_short=B, max_q=1, max_keys=None),
                 caches)
+        if self._affine_chain_ready(tokens, positions, caches, slot_mapping):
+            logits = self.lm_head(self._decode_affine_chain(
+                tokens, positions, caches, slot_mapping, block_tables,
+                seq_lens, nsplit, seq_starts))
+            return (gather_from_tp(logits) if self._lm_vocab_parallel
+                    else logits)
         x = self._embed(tokens.view(B, 1), positions)
         if (ops.use_hip(x) and x.dtype == torch.bfloat16 and B <= 32 and
                 self.cfg.norm == "rmsnorm" and
@@ -657,6 +663,59 @@ class Transformer(nn.Module):
                     _AffineBlock.plain(blk) and
                     blk._affine.current() for blk in self.blocks) and
                 plain(nn.LayerNorm, *self._layer_norms()))
+
+    def _affine_chain_ready(self, tokens, positions, caches, slots) -> bool:
+        """_affine_ready, and every workgroup of a product can norm the rows
+        for itself, and what it reads lies as its kernel takes it (up to 4 rows
+        of up to 4096 columns)."""
+        B = tokens.shape[0]
+        tables = (self.embed, getattr(self, "embed_pos", None))
+        return (tokens.is_cuda and tables[1] is not None and
+                self.cfg.embed_scale == 1.0 and
+                (B > 4 or max(self.cfg.intermediate_size, self.cfg.num_heads *
+                              self.cfg.head_dim) <= 4096) and
+                getattr(self.blocks[0], "_affine", None) is not None and
+                ops.ext().normed_affine_supported(B, self.cfg.hidden_size) and
+                tokens.dim() == 1 and tokens.is_contiguous() and
+                tokens.dtype == torch.int64 and
+                positions.dtype == slots.dtype == torch.int32 and
+                positions.is_contiguous() and slots.is_contiguous() and
+                positions.numel() == B and
+                all(kc.dtype == torch.bfloat16 and kc.is_contiguous() and
+                    vc.is_contiguous() for kc, vc in caches) and
+                plain(nn.Embedding, *tables) and
+                all(t.max_norm is None for t in tables) and
+                self._affine_ready() and
+                all(p.dtype == torch.bfloat16 and p.is_contiguous() and
+                    p.data_ptr() % 16 == 0
+                    for p in (*(t.weight for t in tables),
+                              *(p for n in self._layer_norms()
+                                for p in (n.weight, n.bias)))))
+
+    def _decode_affine_chain(self, tokens, positions, caches, slots,
+                             block_tables, seq_lens, nsplit, seq_starts):
+        """Decode of layer-norm models with biases (opt, gpt2), of few rows and
+        columns: a launch for a product, the norm before it in it
+        (csrc/decode_affine.hip), and for attention. Returns the last norm's
+        result."""
+        ext = ops.ext()
+        res = ext.embed_res32(tokens, positions, self.embed.weight,
+                              self.embed_pos.weight)
+        rows = ext.affine_in_rows(res.shape[0])
+        for blk, (kc, vc) in zip(self.blocks, caches):
+            attn, products = blk.attn, blk._affine
+            q = products.normed(blk.norm1, res, products.qkv_proj,
+                                caches=(kc, vc, slots))
+            o, swz = ops.paged_decode_with_operand(
+                q.view(-1, attn.hq, attn.dh), kc, vc, block_tables, seq_lens,
+                scale=attn.scale, nsplit=nsplit, seq_starts=seq_starts)
+            products.add(res, o.flatten(1) if rows else swz, products.o_proj)
+            h = products.normed(blk.norm2, res, (products.fc1,), products.act,
+                                operand=not rows)
+            products.add(res, h, products.down_proj)
+        return ops.norm_res32(
+            self.norm_f, res, None, self.embed.weight.dtype,
+            operand=ops.decode_ready(self.lm_head.weight, res.shape[0]))
 
     def _decode_affine(self, x, caches, slot_mapping, block_tables, seq_lens,
                        nsplit, seq_starts):
@@ -881,6 +940,21 @@ class _AffineBlock:
         return ops.ext().decode_affine(
             swz, [p.weight for p in projections],
             [p.bias for p in projections], rows, act, operand)
+
+    @staticmethod
+    def normed(norm, res, projections, act: int = 0, operand=False,
+               caches=(None, None, None)):
+        """The first product of the norm of a residual; with caches the others
+        go there."""
+        return ops.ext().normed_affine(
+            res, norm.weight, norm.bias, norm.eps,
+            [p.weight for p in projections], [p.bias for p in projections],
+            act, operand, *caches)[0]
+
+    @staticmethod
+    def add(res, x, projection):
+        """res += the product."""
+        ops.ext().affine_add_(x, projection.weight, projection.bias, res)
 
     def qkv(self, swz, rows: int):
         return self._products(self.qkv_proj, swz, rows)

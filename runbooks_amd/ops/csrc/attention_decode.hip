@@ -9,7 +9,7 @@
 //    heads share each K/V read (falcon-40b MQA G=16, llama2-70b G=8,
 //    llama2-7b MHA G=1).
 //  * flash-style online softmax entirely in registers; group partials
-//    merged via shfl_xor(16/32), wave partials via LDS.
+//    merged by lane permutations, wave partials via LDS.
 //  * kv-split ("flash-decoding") for long sequences / small batch: grid z
 //    = nsplit partitions, fp32 partials (m, l, acc) merged by a tiny
 //    second kernel — sized so batch*Hkv*nsplit >> 256 CUs.
@@ -21,6 +21,8 @@
 
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
+
+#include <algorithm>
 
 #include "common.h"
 
@@ -79,8 +81,8 @@ RB_DEV int sequence_of() {
 // so halving cache bytes halves the dominant stream AND doubles KV
 // capacity within 288 GB. Dequant rides
 // v_cvt_pk_f32_fp8 in the inner loop.
-template <int DH, int G, bool SPLIT, bool FP8 = false>
-__global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
+template <int DH, int G, bool SPLIT, bool FP8 = false, int WAVES = NW>
+__global__ __launch_bounds__(WAVES * 64) void paged_decode_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k_cache,
     const uint16_t *__restrict__ v_cache, const int32_t *__restrict__ block_tables,
     const int32_t *__restrict__ seq_lens,
@@ -95,7 +97,7 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
   // first fp8 cut used 16-lane groups and showed ZERO long-context win).
   // (G > 4 keeps 16-lane groups even for fp8: qreg[G][VE]+acc[G][VE]
   // at VE=16 would spill past 256 VGPRs)
-  constexpr int GL = (FP8 && G <= 4) ? 8 : 16;
+  constexpr int GL = (FP8 && G <= 4) || (DH == 64 && G < NW) ? 8 : 16;
   constexpr int VE = DH / GL;              // elems per lane
   constexpr int TPW = 64 / GL;             // tokens per wave pass
   // Head-split mode (G >= NW): each wave owns GW = G/NW query heads
@@ -185,9 +187,13 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
   constexpr int BT_LDS = 512;
   __shared__ int32_t bt_lds[BT_LDS];
   const int blk0 = t_begin / bs;
-  if (t_begin < t_end) {
+  if (!SPLIT && seq_starts == nullptr) {
+    // without waiting for the length
+    for (int i = (int)threadIdx.x; i < min(max_blocks, BT_LDS); i += WAVES * 64)
+      bt_lds[i] = bt[i];
+  } else if (t_begin < t_end) {
     const int nbt = min((t_end - 1) / bs - blk0 + 1, BT_LDS);
-    for (int i = (int)threadIdx.x; i < nbt; i += BLOCK)
+    for (int i = (int)threadIdx.x; i < nbt; i += WAVES * 64)
       bt_lds[i] = bt[blk0 + i];
   }
   __syncthreads();
@@ -212,7 +218,7 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
   constexpr int RW = KBPL / 4;             // u32 words of that
   constexpr int TPS = GW == 1 || (GW == 2 && !FP8) ? 2 : 1;
   constexpr int DEPTH = (G >= 4) ? 4 : 2;
-  const int stride = (HS ? 1 : NW) * TPW * TPS;    // tokens of a step
+  const int stride = (HS ? 1 : WAVES) * TPW * TPS;    // tokens of a step
   const int tw0 = t_begin + (HS ? 0 : wid * TPW * TPS);  // wave's first token
   const int t_base = tw0 + grp;            // this lane group's first
   const int niter = (t_end > tw0) ? (t_end - tw0 + stride - 1) / stride : 0;
@@ -275,10 +281,7 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
         sc[u] = x;
       }
       // reduce across the lane group
-#pragma unroll
-      for (int off = GL / 2; off > 0; off >>= 1)
-#pragma unroll
-        for (int u = 0; u < TPS; ++u) sc[u] += __shfl_xor(sc[u], off, 64);
+      rb::lane_sums<GL>(sc);
 #pragma unroll
       for (int u = 0; u < TPS; ++u) {
         if (t_base + i * stride + u * TPW >= t_end) sc[u] = -INFINITY;
@@ -323,26 +326,28 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
   }
 
   // Merge the TPW groups inside each wave: lanes l^GL ... l^32 hold the
-  // same d0 slice, so shfl_xor merges matching elements.
-#pragma unroll
-  for (int off = GL; off <= 32; off <<= 1) {
+  // same d0 slice, so lanes apart by a bit merge matching
+  // elements.
+  auto merge = [&](auto bit) {
+    constexpr int OFF = decltype(bit)::value;
 #pragma unroll
     for (int g = 0; g < GW; ++g) {
-      const float mo = __shfl_xor(m[g], off, 64);
-      const float lo = __shfl_xor(l[g], off, 64);
+      const float mo = rb::lane_xor<OFF>(m[g]);
+      const float lo = rb::lane_xor<OFF>(l[g]);
       const float mn = fmaxf(m[g], mo);
-      if (mn == -INFINITY) continue;
-      const float a1 = __expf(m[g] - mn);
-      const float a2 = __expf(mo - mn);
+      // lanes without a key yet keep their zeros
+      const float a1 = mn == -INFINITY ? 1.0f : __expf(m[g] - mn);
+      const float a2 = mn == -INFINITY ? 0.0f : __expf(mo - mn);
 #pragma unroll
-      for (int e = 0; e < VE; ++e) {
-        const float ao = __shfl_xor(acc[g][e], off, 64);
-        acc[g][e] = acc[g][e] * a1 + ao * a2;
-      }
+      for (int e = 0; e < VE; ++e)
+        acc[g][e] = acc[g][e] * a1 + rb::lane_xor<OFF>(acc[g][e]) * a2;
       l[g] = l[g] * a1 + lo * a2;
       m[g] = mn;
     }
-  }
+  };
+  if constexpr (GL == 8) merge(std::integral_constant<int, 8>{});
+  merge(std::integral_constant<int, 16>{});
+  merge(std::integral_constant<int, 32>{});
 
   if constexpr (HS) {
     // Head-split: each wave owns its GW heads outright — write out
@@ -371,9 +376,9 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
     return;
   }
 
-  // Merge across the 4 waves via LDS. Layout per (wave, head):
+  // Merge across the waves via LDS. Layout per (wave, head):
   // [DH acc][m][l] floats.
-  __shared__ float lds[HS ? 1 : NW][HS ? 1 : G][DH + 2];
+  __shared__ float lds[HS ? 1 : WAVES][HS ? 1 : G][DH + 2];
   if (grp == 0) {   // lanes 0..GL-1 of each wave hold the wave's merged state
 #pragma unroll
     for (int g = 0; g < GW; ++g) {
@@ -384,18 +389,18 @@ __global__ __launch_bounds__(BLOCK) void paged_decode_kernel(
   }
   __syncthreads();
 
-  // Wave `wid` finalizes heads g = wid, wid+NW, ... (lanes 0..15 active).
-  for (int g = wid; g < G; g += NW) {
+  // Wave `wid` finalizes heads g = wid, wid+WAVES, ... (lanes 0..15 active).
+  for (int g = wid; g < G; g += WAVES) {
     if (grp != 0) continue;
     float mm = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) mm = fmaxf(mm, lds[w][g][DH]);
+    for (int w = 0; w < WAVES; ++w) mm = fmaxf(mm, lds[w][g][DH]);
     float ll = 0.f, av[VE];
 #pragma unroll
     for (int e = 0; e < VE; ++e) av[e] = 0.f;
     if (mm != -INFINITY) {
 #pragma unroll
-      for (int w = 0; w < NW; ++w) {
+      for (int w = 0; w < WAVES; ++w) {
         const float a = __expf(lds[w][g][DH] - mm);
         ll += lds[w][g][DH + 1] * a;
 #pragma unroll
@@ -683,8 +688,8 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
       if (t0 + e < t_begin || t0 + e >= t_end) p[e] = -INFINITY;
       mx = fmaxf(mx, p[e]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = fmaxf(mx, rb::lane_xor<16>(mx));
+    mx = fmaxf(mx, rb::lane_xor<32>(mx));
     if (__any(mx > m_run)) {
       const float mn = fmaxf(m_run, mx);
       const float alpha = mn == -INFINITY ? 1.0f : __expf(m_run - mn);
@@ -722,8 +727,8 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
     step(bi, 0);
     if (bi + PAIR <= blk_hi) step(bi + PAIR, 1);
   }
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run += rb::lane_xor<16>(l_run);
+  l_run += rb::lane_xor<32>(l_run);
 
   // ---- cross-wave merge via LDS (same scheme as the scalar kernel) ----
   // acc_o lane map: head = i16, d = dt*16 + 4*h16 + r.
@@ -777,6 +782,25 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
   }
 }
 
+// Whether a workgroup of 8 or 16 waves takes a whole sequence of a kv head, rather
+// than several of 4 waves parts of it: where that is a workgroup for every CU, or
+// tables (the only bound on lengths that is known here) so short that a CU's share
+// of them costs less than the sum of the parts in a launch of its own. More waves
+// also shorten the time that a batch's longest sequences run after the others.
+//
+// us in parts, by 4 waves, and here: 32 heads of 128, sequences of 129 to 2015
+// tokens, 32 of them 114.5 and 107.5 (unsplit before, too), 8 34.4 and 33.1; 64 of
+// 100 to 1000 116 and 103; 4 of 200 9.7 and 7.4, of 1000 19.6 and 17.9; one of 200
+// 8.4 and 6.3, of 500 9.6 and 9.4, of 1000 11.1 and 13.8; 12 heads of 64, 64
+// sequences of 37 to 1400 47.8 and 36 to 39; 16 heads of 256, 32 sequences 101 and
+// 99 (8 waves; 107 with 16), 4 of 500 14.6 and 14.4; e4m3, 16 sequences of 800 to
+// 3900 75.8 and 73.3 (78.8 with 16 waves).
+template <int DH> bool whole_sequences(int64_t B, int64_t hkv, int64_t longest) {
+  const int64_t base = B * hkv;
+  return base >= 256 ||
+         longest <= (DH > 128 ? 4 : 8) * std::max<int64_t>(32, base);
+}
+
 template <int DH, int G, bool FP8>
 void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                    const at::Tensor &v_cache, const at::Tensor &block_tables,
@@ -793,6 +817,10 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
   const int max_blocks = (int)block_tables.size(1);
   uint16_t *swz = out_swz.has_value() ? (uint16_t *)out_swz->data_ptr()
                                       : nullptr;
+  // parts of fewer tokens cost more than they save (one sequence of 37 tokens, 32
+  // heads of 128: 16 parts 8.2 us, one 4.1; matrix instructions, 32 query heads,
+  // one of 500: 16 parts 7.5, 10 7.9)
+  const int64_t longest = (int64_t)max_blocks * bs;
   // MFMA route: keyed on the TRANSPOSED V layout (bf16 [Dh, BS] /
   // fp8 [Dh+4, BS] blocks) the allocator chooses for MFMA-eligible
   // models (G >= 4, DH <= 128, 16-token blocks — RB_DECODE_MFMA=0 at
@@ -801,6 +829,8 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
   // versa.
   const bool vt = v_cache.size(3) == bs &&
       v_cache.size(2) == (int64_t)(FP8 ? DH + 4 : DH);
+  nsplit = (int)std::min<int64_t>(nsplit,
+                                  (longest + 63) / (vt ? 32 : 64));
   if constexpr (G >= 4 && DH <= 128) {
     if (vt && bs == 16) {
       if (nsplit <= 1) {
@@ -837,35 +867,33 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
   }
   TORCH_CHECK(!vt, "paged_decode: transposed V cache requires the MFMA "
               "path (bf16, G>=4, Dh<=128, bs==16); got G=", G, " Dh=", DH);
-  if (nsplit <= 1) {
-    hipLaunchKernelGGL((paged_decode_kernel<DH, G, false, FP8>),
-                       dim3(B, hkv, 1),
-                       dim3(BLOCK), 0, stream, (const uint16_t *)q.data_ptr(),
+  const int Hq = hkv * G;
+  auto go = [&](auto kernel, int waves, int splits, float *partial) {
+    hipLaunchKernelGGL(kernel, dim3(B, hkv, splits), dim3(waves * 64), 0,
+                       stream, (const uint16_t *)q.data_ptr(),
                        (const uint16_t *)k_cache.data_ptr(),
                        (const uint16_t *)v_cache.data_ptr(),
-                       block_tables.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(),
-                       starts,
-                       (uint16_t *)out.data_ptr(), swz, nullptr, hkv, bs,
-                       max_blocks, 1, scale);
-  } else {
-    const int Hq = hkv * G;
-    auto partial = at::empty({B, Hq, nsplit, DH + 2},
-                             q.options().dtype(at::kFloat));
-    hipLaunchKernelGGL((paged_decode_kernel<DH, G, true, FP8>),
-                       dim3(B, hkv, nsplit),
-                       dim3(BLOCK), 0, stream, (const uint16_t *)q.data_ptr(),
-                       (const uint16_t *)k_cache.data_ptr(),
-                       (const uint16_t *)v_cache.data_ptr(),
-                       block_tables.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(),
-                       starts,
-                       nullptr, nullptr, partial.data_ptr<float>(), hkv, bs,
-                       max_blocks, nsplit, scale);
-    hipLaunchKernelGGL((decode_combine_kernel<DH / 64>),
-                           dim3((B * Hq + 3) / 4), dim3(256), 0, stream,
-                           partial.data_ptr<float>(),
-                           (uint16_t *)out.data_ptr(), swz, B * Hq, Hq,
-                           nsplit);
+                       block_tables.data_ptr<int32_t>(),
+                       seq_lens.data_ptr<int32_t>(), starts,
+                       splits > 1 ? nullptr : (uint16_t *)out.data_ptr(),
+                       splits > 1 ? nullptr : swz, partial, hkv, bs, max_blocks,
+                       splits, scale);
+  };
+  if constexpr (G < NW) {
+    constexpr int MORE = FP8 || DH > 128 ? 8 : 16;
+    if (longest > 64 && whole_sequences<DH>(B, hkv, longest))
+      return go(paged_decode_kernel<DH, G, false, FP8, MORE>, MORE, 1, nullptr);
   }
+  if (nsplit <= 1)
+    return go(paged_decode_kernel<DH, G, false, FP8>, NW, 1, nullptr);
+  auto partial = at::empty({B, Hq, nsplit, DH + 2},
+                           q.options().dtype(at::kFloat));
+  go(paged_decode_kernel<DH, G, true, FP8>, NW, nsplit,
+     partial.data_ptr<float>());
+  hipLaunchKernelGGL((decode_combine_kernel<DH / 64>),
+                     dim3((B * Hq + 3) / 4), dim3(256), 0, stream,
+                     partial.data_ptr<float>(), (uint16_t *)out.data_ptr(), swz,
+                     B * Hq, Hq, nsplit);
 }
 
 }  // namespace

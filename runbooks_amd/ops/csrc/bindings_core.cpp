@@ -34,6 +34,11 @@ at::Tensor decode_swizzle_w(at::Tensor w, int64_t half);
 at::Tensor decode_swizzle_x(at::Tensor x);
 at::Tensor decode_swizzle_w8(at::Tensor w8, int64_t half);
 std::vector<at::Tensor> decode_affine(at::Tensor xs, std::vector<at::Tensor> ws, std::vector<c10::optional<at::Tensor>> biases, int64_t M, int64_t act, bool operand);
+bool normed_affine_supported(int64_t M, int64_t K);
+bool affine_in_rows(int64_t M);
+std::vector<at::Tensor> normed_affine(at::Tensor res, at::Tensor gain, at::Tensor shift, double eps, std::vector<at::Tensor> ws, std::vector<c10::optional<at::Tensor>> biases, int64_t act, bool operand, c10::optional<at::Tensor> k_cache, c10::optional<at::Tensor> v_cache, c10::optional<at::Tensor> slots);
+void affine_add_(at::Tensor x, at::Tensor w, c10::optional<at::Tensor> bias, at::Tensor res);
+at::Tensor embed_res32(at::Tensor tokens, at::Tensor positions, at::Tensor table, at::Tensor places);
 at::Tensor sum_parts(at::Tensor parts);
 at::Tensor decode_gemm_rows(at::Tensor x, at::Tensor ws, int64_t N, int64_t half, bool raw);
 at::Tensor decode_gemm_fp8(at::Tensor xs, at::Tensor w8s, at::Tensor scale, int64_t M, int64_t N, int64_t K, bool raw, int64_t half);
@@ -145,6 +150,17 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "act(x W^T + bias) to up to three matrices, or as an operand",
         py::arg("xs"), py::arg("ws"), py::arg("biases"), py::arg("M"),
         py::arg("act") = 0, py::arg("operand") = false);
+  m.def("normed_affine_supported", &normed_affine_supported);
+  m.def("affine_in_rows", &affine_in_rows);
+  m.def("normed_affine", &normed_affine,
+        "decode_affine of a residual's layer norm; k and v to the cache",
+        py::arg("res"), py::arg("gain"), py::arg("shift"), py::arg("eps"),
+        py::arg("ws"), py::arg("biases"), py::arg("act") = 0,
+        py::arg("operand") = false, py::arg("k_cache") = py::none(),
+        py::arg("v_cache") = py::none(), py::arg("slots") = py::none());
+  m.def("affine_add_", &affine_add_, "residual += x W^T + bias");
+  m.def("embed_res32", &embed_res32,
+        "embeddings of tokens and positions, added up in fp32");
   m.def("sum_parts", &sum_parts, "fp32 [P, M, N] -> their sum [M, N] bf16");
   m.def("decode_gemm_rows", &decode_gemm_rows, "x [M <= 128, K] W^T",
         py::arg("x"), py::arg("ws"), py::arg("N"), py::arg("half") = 0,

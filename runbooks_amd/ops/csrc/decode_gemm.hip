@@ -52,7 +52,6 @@ constexpr int MMAX = 32;
 using ends::bf16x8v;
 using ends::Ends;
 using ends::f32x16v;
-using ends::f32x4v;
 using ends::fp8_to_bf16;
 using ends::Kind;
 using ends::load8v;
@@ -239,139 +238,6 @@ __global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
   const f32x16v acc =
       weight_stream<FP8>(xs, ws, M, K, [&] { early.rest(e, M); });
   finish<KIND>(acc, e, early, M, N);
-}
-
-// act(x W^T + bias) of models whose decode is bound by its launches: the columns
-// go to up to three matrices (q, k, v), or to the operand of the next product.
-// W and bias are the parameters themselves, so that captured steps follow them
-// too: a workgroup takes 16 rows of W as they lie, its waves parts of the sums,
-// 64 bytes of each row an instruction (16x16x32 products: A[i=l&15][k=(l>>4)*8+e],
-// B[k][j=l&15], C[j=l&15][i=(l>>4)*4+r]).
-//
-// us in a graph, weights out of cache, on the library without the activation, in
-// the layout of decode_gemm (32 rows a workgroup) and here, of 1 and 32 rows:
-//   q, k, v 768 x 768   21  4.3  3.6   20  5.1  4.0
-//   768 x 768            6.8 4.1 3.5    6.6 4.8 3.9
-//   3072 x 768           8  4.3  3.9    9  4.9  4.7
-//   768 x 3072          13  7.2  6.4    9  9.2  8.5
-//   q, k, v 1600 x 1600 38  6.8  8.5   35  7.4  9.1
-//   16384 x 4096        35 24   29     31 27   35 (5.5 and 4.7 TB/s of 1 row)
-// so wide weights would gain by the layout's copies, which follow nothing.
-struct Affine {
-  const uint16_t *w[3], *bias[3];       // [rows, K] each; bias may be null
-  uint16_t *out[3];
-  int end[3];                           // columns before the next matrix
-  int act;                              // 0 none, 1 relu, 2 gelu, 3 gelu_tanh
-  bool operand;                         // out[0] as [N/16][2][32][8]
-};
-
-__device__ __forceinline__ float activate(float x, int act) {
-  if (act == 1) return x < 0.0f ? 0.0f : x;
-  if (act == 2) return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f));
-  if (act == 3)
-    return 0.5f * x * (1.0f + tanhf(0.79788456080286536f *
-                                    (x + 0.044715f * x * x * x)));
-  return x;
-}
-
-// R blocks of 16 rows of W by B of x: R = 1, which is the most workgroups, while
-// they are no more than the CUs or x is no longer than their part of W.
-template <int R, int B>
-__global__ __launch_bounds__(BLOCK, 2) void decode_affine_kernel(
-    const uint16_t *__restrict__ xs, Affine a, int M, int K) {
-  constexpr int U = R == 1 ? 8 : 4;
-  const int tid = threadIdx.x;
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63, i16 = lane & 15, grp = lane >> 4;
-  // ends are multiples of 32: a workgroup's rows are of one matrix
-  const int n0 = blockIdx.x * 16 * R;
-  const int of = n0 < a.end[0] ? 0 : n0 < a.end[1] ? 1 : 2;
-  const int first = of == 0 ? 0 : a.end[of - 1];
-  const uint16_t *w = a.w[of] + (int64_t)(n0 - first + i16) * K + grp * 8;
-  const uint16_t *x = xs + (grp >> 1) * 512 + (grp & 1) * 256;
-  int xrow[B];                          // rows past M: the last one again
-#pragma unroll
-  for (int b = 0; b < B; ++b) xrow[b] = min(b * 16 + i16, M - 1) * 8;
-  const int steps = K / 32, s0 = steps * wid / 4, s1 = steps * (wid + 1) / 4;
-
-  f32x4v acc[R][B];
-#pragma unroll
-  for (int i = 0; i < R; ++i)
-#pragma unroll
-    for (int b = 0; b < B; ++b) acc[i][b] = (f32x4v)(0.0f);
-  struct Chunk { bf16x8v w[U][R], x[U][B]; };
-  Chunk c0, c1;
-  auto load = [&](Chunk &c, int s) {    // past the end: the last one again
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int at = min(s + u, s1 - 1);
-#pragma unroll
-      for (int i = 0; i < R; ++i)
-        c.w[u][i] = load8v(w + (int64_t)i * 16 * K + at * 32);
-#pragma unroll
-      for (int b = 0; b < B; ++b)
-        c.x[u][b] = load8v(x + (int64_t)at * 1024 + xrow[b]);
-    }
-  };
-  auto multiply = [&](const Chunk &c, int s) {
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (s + u < s1) {
-#pragma unroll
-        for (int i = 0; i < R; ++i)
-#pragma unroll
-          for (int b = 0; b < B; ++b)
-            acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                c.w[u][i], c.x[u][b], acc[i][b], 0, 0, 0);
-      }
-  };
-  if (s0 < s1) {
-    int s = s0;
-    load(c0, s);
-    for (; s + 2 * U < s1; s += 2 * U) {
-      load(c1, s + U);
-      multiply(c0, s);
-      load(c0, s + 2 * U);
-      multiply(c1, s + U);
-    }
-    if (s + U < s1) {
-      load(c1, s + U);
-      multiply(c0, s);
-      multiply(c1, s + U);
-    } else {
-      multiply(c0, s);
-    }
-  }
-  __shared__ float red[4][16 * R][16 * B + 1];
-#pragma unroll
-  for (int i = 0; i < R; ++i)
-#pragma unroll
-    for (int b = 0; b < B; ++b)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        red[wid][i * 16 + grp * 4 + r][b * 16 + i16] = acc[i][b][r];
-  __syncthreads();
-  constexpr int V = 2 * R;              // columns of a thread
-  const int m = tid >> 3, en = (tid & 7) * V;
-  if (m >= min(M, 16 * B)) return;
-  const int n = n0 + en;
-  __attribute__((aligned(8))) uint16_t o[V];
-#pragma unroll
-  for (int j = 0; j < V; ++j) {
-    float f = red[0][en + j][m] + red[1][en + j][m] + red[2][en + j][m] +
-              red[3][en + j][m];
-    if (a.bias[of] != nullptr)
-      f += rb::bf16_to_f32(a.bias[of][n - first + j]);
-    o[j] = rb::f32_to_bf16(activate(f, a.act));
-  }
-  uint16_t *dst =
-      a.operand ? a.out[0] + (n >> 4) * 512 + (n >> 3 & 1) * 256 + m * 8 +
-                      (n & 7)
-                : a.out[of] + (int64_t)m * (a.end[of] - first) + n - first;
-  if constexpr (R == 1)
-    *reinterpret_cast<uint32_t *>(dst) = *reinterpret_cast<uint32_t *>(o);
-  else
-    *reinterpret_cast<uint64_t *>(dst) = *reinterpret_cast<uint64_t *>(o);
 }
 
 // 17 to 128 rows (RB blocks of 32): x is longer than W's share of a workgroup, so
@@ -668,11 +534,13 @@ at::Tensor decode_swizzle_w(at::Tensor w, int64_t half) {
   const int64_t N = w.size(0), K = w.size(1);
   TORCH_CHECK(N % 32 == 0 && K % 16 == 0, "decode_swizzle_w: shape");
   check_pairs(N, half);
-  if (half == 0)
-    return w.view({N / 32, 32, K / 16, 2, 8})
-        .permute({0, 2, 3, 1, 4}).contiguous();
-  return w.view({N / (2 * half), 2, half / 16, 16, K / 16, 2, 8})
-      .permute({0, 2, 4, 5, 1, 3, 6}).contiguous();
+  // moved by words of 8 bytes
+  const auto q = (w.storage_offset() % 4 ? w.clone() : w).view(at::kLong);
+  const auto laid =
+      half == 0 ? q.view({N / 32, 32, K / 16, 2, 2}).permute({0, 2, 3, 1, 4})
+                : q.view({N / (2 * half), 2, half / 16, 16, K / 16, 2, 2})
+                      .permute({0, 2, 4, 5, 1, 3, 6});
+  return laid.contiguous().view(at::kBFloat16).view({N / 32, K / 16, 2, 32, 8});
 }
 
 at::Tensor decode_swizzle_x(at::Tensor x) {
@@ -697,11 +565,12 @@ at::Tensor decode_swizzle_w8(at::Tensor w8, int64_t half) {
   const int64_t N = w8.size(0), K = w8.size(1);
   TORCH_CHECK(N % 32 == 0 && K % 32 == 0, "decode_swizzle_w8: shape");
   check_pairs(N, half);
-  if (half == 0)
-    return w8.view({N / 32, 32, K / 32, 2, 2, 8})
-        .permute({0, 2, 4, 1, 3, 5}).contiguous();
-  return w8.view({N / (2 * half), 2, half / 16, 16, K / 32, 2, 2, 8})
-      .permute({0, 2, 4, 6, 1, 3, 5, 7}).contiguous();
+  const auto q = (w8.storage_offset() % 8 ? w8.clone() : w8).view(at::kLong);
+  const auto laid =
+      half == 0 ? q.view({N / 32, 32, K / 32, 2, 2}).permute({0, 2, 4, 1, 3})
+                : q.view({N / (2 * half), 2, half / 16, 16, K / 32, 2, 2})
+                      .permute({0, 2, 4, 6, 1, 3, 5});
+  return laid.contiguous().view(at::kByte).view({N / 32, K / 32, 2, 32, 2, 8});
 }
 
 template <bool FP8>
@@ -745,57 +614,6 @@ static void combine(const at::Tensor &slabs, at::Tensor &y) {
                      at::cuda::getCurrentHIPStream(),
                      slabs.data_ptr<float>(), (uint16_t *)y.data_ptr(),
                      (int)slabs.size(0), y.numel());
-}
-
-// act(x W^T + bias) with up to three parameters W [N_i, K] and their biases, to a
-// matrix each, or as the operand of the next product; xs as in decode_gemm.
-std::vector<at::Tensor> decode_affine(
-    at::Tensor xs, std::vector<at::Tensor> ws,
-    std::vector<c10::optional<at::Tensor>> biases, int64_t M, int64_t act,
-    bool operand) {
-  TORCH_CHECK(!ws.empty() && ws.size() <= 3 && biases.size() == ws.size() &&
-              (!operand || ws.size() == 1), "decode_affine: matrices");
-  TORCH_CHECK(M >= 1 && M <= MMAX && act >= 0 && act <= 3,
-              "decode_affine: rows, act");
-  const int64_t K = ws[0].dim() == 2 ? ws[0].size(1) : 0;
-  TORCH_CHECK(K > 0 && K % 32 == 0 && K < (1 << 24) && xs.is_cuda() &&
-              xs.is_contiguous() && xs.scalar_type() == at::kBFloat16 &&
-              xs.numel() == (K / 16) * 512, "decode_affine: operand");
-  Affine a{};
-  int64_t N = 0;
-  std::vector<at::Tensor> out;
-  for (size_t i = 0; i < ws.size(); ++i) {
-    const at::Tensor &w = ws[i];
-    TORCH_CHECK(w.device() == xs.device() && w.dim() == 2 && w.size(1) == K &&
-                w.size(0) > 0 && w.size(0) % 32 == 0 && w.is_contiguous() &&
-                w.scalar_type() == at::kBFloat16 &&
-                reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
-                "decode_affine: weights [32 n, 32 k] bf16");
-    const auto &b = biases[i];
-    TORCH_CHECK(!b.has_value() ||
-                (b->device() == xs.device() && b->is_contiguous() &&
-                 b->numel() == w.size(0) &&
-                 b->scalar_type() == at::kBFloat16), "decode_affine: bias");
-    out.push_back(operand ? at::empty({w.size(0) / 16 * 512}, xs.options())
-                          : at::empty({M, w.size(0)}, xs.options()));
-    a.w[i] = (const uint16_t *)w.data_ptr();
-    a.bias[i] = b.has_value() ? (const uint16_t *)b->data_ptr() : nullptr;
-    a.out[i] = (uint16_t *)out[i].data_ptr();
-    N += w.size(0);
-    TORCH_CHECK(N < (int64_t)1 << 31, "decode_affine: columns");
-    a.end[i] = (int)N;
-  }
-  a.act = (int)act;
-  a.operand = operand;
-  auto go = [&](auto kernel, int rows) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(N / rows)), dim3(BLOCK), 0,
-                       at::cuda::getCurrentHIPStream(),
-                       (const uint16_t *)xs.data_ptr(), a, (int)M, (int)K);
-  };
-  if (M <= 16) go(decode_affine_kernel<1, 1>, 16);
-  else if (N <= 16 * 256) go(decode_affine_kernel<1, 2>, 16);
-  else go(decode_affine_kernel<2, 2>, 32);
-  return out;
 }
 
 // Sum of fp32 parts [P, M, N], rounded to bf16.

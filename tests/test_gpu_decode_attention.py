@@ -1,0 +1,55 @@
+"""Decode attention by workgroups of whole sequences (csrc/attention_decode.hip)."""
+import pytest
+import torch
+
+from runbooks_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+# one rounding to bf16 (half a unit of 8 bits) beside fp32 sums
+BF16 = 2 ** -8 + 1e-4
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("batch,hq,hkv,dh,blocks,nsplit", [
+    (3, 12, 12, 64, 16, 16), (22, 12, 12, 64, 40, 3), (2, 8, 4, 64, 16, 16),
+    (4, 32, 32, 128, 30, 8), (16, 32, 16, 128, 40, 2), (8, 32, 32, 128, 130, 4),
+    (4, 16, 16, 256, 15, 16), (16, 16, 16, 256, 40, 4), (2, 4, 4, 128, 4, 16),
+    (1, 4, 4, 128, 129, 16)])
+def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
+    """By 4, 8 or 16 waves or in parts, with and without a window's start, and
+    with sequences as short and as long as the table: the plain result but for
+    roundings of the probabilities' sums and of the output."""
+    torch.manual_seed(batch + dh)
+    tokens = blocks * 16
+    lens = torch.randint(1, tokens + 1, (batch,))
+    lens[0], lens[-1] = 1, tokens
+    kc, vc = ops.alloc_kv_cache(batch * blocks, hkv, dh, DEV,
+                                dtype=torch.bfloat16, fp8=fp8)
+    k, v = (torch.randn(batch * tokens, hkv, dh, device=DEV).bfloat16()
+            for _ in "kv")
+    ops.kv_append(k, v, kc, vc, torch.arange(batch * tokens, device=DEV,
+                                             dtype=torch.int32))
+    q = torch.randn(batch, hq, dh, device=DEV).bfloat16()
+    i32 = dict(dtype=torch.int32, device=DEV)
+    tables = torch.randperm(batch * blocks, device=DEV).to(torch.int32) \
+        .view(batch, blocks)
+    for starts in (None, torch.clamp(lens - 40, min=0)):
+        args = [lens.to(**i32), dh ** -0.5]
+        s = None if starts is None else starts.to(**i32)
+        got = ops.ext().paged_decode_swz(q, kc, vc, tables, args[0], nsplit,
+                                         args[1], s)
+        pick = sorted({0, batch // 2, batch - 1})
+        ref = ops.paged_decode_ref(
+            q[pick].cpu(), kc.cpu(), vc.cpu(), tables[pick].cpu(), lens[pick],
+            args[1], None if starts is None else starts[pick])
+        assert _rel(got[0][pick].cpu(), ref.double()) < 2 * BF16
+        if batch <= 32:
+            operand = ops.ext().decode_swizzle_x(got[0].view(batch, -1))
+            assert torch.equal(got[1].view(-1, 32, 8)[:, :batch],
+                               operand.view(-1, 32, 8)[:, :batch])

@@ -40,6 +40,9 @@ std::vector<at::Tensor> normed_affine(at::Tensor res, at::Tensor gain, at::Tenso
 void affine_add_(at::Tensor x, at::Tensor w, c10::optional<at::Tensor> bias, at::Tensor res);
 at::Tensor embed_res32(at::Tensor tokens, at::Tensor positions, at::Tensor table, at::Tensor places);
 at::Tensor sum_parts(at::Tensor parts);
+bool tile_gemm_takes(at::Tensor x, at::Tensor w, bool glu);
+int64_t tile_gemm_parts(int64_t M, int64_t N, int64_t K);
+at::Tensor tile_gemm(at::Tensor x, at::Tensor w, int64_t max_parts, int64_t glu, int64_t tile, int64_t parts);
 at::Tensor decode_gemm_rows(at::Tensor x, at::Tensor ws, int64_t N, int64_t half, bool raw);
 at::Tensor decode_gemm_fp8(at::Tensor xs, at::Tensor w8s, at::Tensor scale, int64_t M, int64_t N, int64_t K, bool raw, int64_t half);
 int64_t decode_gemm_split(int64_t N, int64_t K);
@@ -162,6 +165,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("embed_res32", &embed_res32,
         "embeddings of tokens and positions, added up in fp32");
   m.def("sum_parts", &sum_parts, "fp32 [P, M, N] -> their sum [M, N] bf16");
+  m.def("tile_gemm_takes", &tile_gemm_takes, py::arg("x"), py::arg("w"),
+        py::arg("glu") = false, "whether tile_gemm takes x and W");
+  m.def("tile_gemm_parts", &tile_gemm_parts,
+        "parts that tile_gemm makes of sums where it may");
+  m.def("tile_gemm", &tile_gemm, py::arg("x"), py::arg("w"),
+        py::arg("max_parts") = 1, py::arg("glu") = 0, py::arg("tile") = -1,
+        py::arg("parts") = 0,
+        "x @ W^T of many rows (gemm_tiles.hip): bf16 [M, N], or, where max_parts "
+        "allows, fp32 parts [P, M, N]; glu 1 / 2: SiLU / GELU units of [G ; U]");
   m.def("decode_gemm_rows", &decode_gemm_rows, "x [M <= 128, K] W^T",
         py::arg("x"), py::arg("ws"), py::arg("N"), py::arg("half") = 0,
         py::arg("raw") = false);

@@ -1,0 +1,423 @@
+// Products of many rows, x [M, K] times W [N, K] transposed, bf16 with fp32 sums,
+// in tiles that suit their sizes, and ended by what follows them: parts of sums
+// for the norm that adds them up, or a gated unit.
+//
+// Bound by L2, which feeds LDS at 16 TB/s (62 GB/s a CU: what is left of a
+// product of 8192 x 8192 x 4096 without its matrix instructions takes 269 us in
+// tiles of 256 x 256 and 554 in those of 128 x 128), and by the matrix cores
+// (without loads 312 us, 1760 TFLOP/s; both together 401). So tiles are as large
+// as their number allows; where it does not, for prompts of some hundred rows,
+// workgroups share the sums.
+//
+// us in the library and here, weights out of cache: 256 x 4096 x 11008 51 and 36
+// (4 parts), 512 x 4096 x 11008 75 and 47 (4), 1021 x 4096 x 11008 105 and 80 (2),
+// 512 x 3072 x 24576 267 and 82 (4), 512 x 22016 x 4096 80 and 77, 1021 x 49152 x
+// 3072 240 and 235, 2048 x 4096 x 14336 205 and 180, 7931 x 28672 x 4096 1300 and
+// 1340 (1420 and 1340 with the gated unit).
+
+#include <torch/extension.h>
+#include <ATen/hip/HIPContext.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "common.h"
+#include "decode_ends.h"
+
+namespace tiles {
+
+using ends::bf16x8v;
+using ends::f32x4v;
+using ends::u32x4v;
+
+__device__ __forceinline__ void put(uint16_t *p, const float (&f)[4]) {
+  typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4v;
+  *reinterpret_cast<bf16x4v *>(p) =
+      __builtin_convertvector((f32x4v){f[0], f[1], f[2], f[3]}, bf16x4v);
+}
+
+// 16 bytes a lane to LDS at lds + lane * 16, past the registers. As text, for
+// the compiler waits for all such loads before it reads LDS again.
+__device__ __forceinline__ void dma(u32x4v rsrc, unsigned voff, unsigned soff,
+                                    unsigned lds) {
+  asm volatile(
+      "s_mov_b32 m0, %3\n\ts_nop 0\n\t"
+      "buffer_load_dwordx4 %0, %1, %2 offen lds"
+      :: "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory", "m0");
+}
+
+// As text, for the compiler copies sums between the register files otherwise.
+__device__ __forceinline__ void mma(f32x4v &c, bf16x8v a, bf16x8v b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+               : "+a"(c) : "v"(a), "v"(b));
+}
+
+enum Kind {
+  PLAIN,        // y [M, N] bf16
+  PARTS,        // fp32 [P, M, N], K-tiles kt * p .. of every part
+  SILU, GELU,   // act(x G^T) * (x U^T) of W = [G ; U], y [M, N / 2]
+};
+
+// Waits until the last products are in their registers, if `left` is 0. The
+// compiler does not know what mma() takes, and may move sums about right behind
+// the loop; this stands in it, and with a branch of its own, for otherwise the
+// compiler makes a copy of the loop's body for its last round.
+__device__ __forceinline__ void settle(int left) {
+  asm volatile(
+      "s_cmp_lg_u32 %0, 0\n\ts_cbranch_scc1 .Lsettled%=\n\t"
+      "s_nop 15\n\ts_nop 15\n.Lsettled%=:" :: "s"(left) : "scc");
+}
+
+// A sum's way out of the matrix registers: as text, it stays where its use is.
+__device__ __forceinline__ void take(float (&f)[4], const f32x4v &c) {
+  asm volatile(
+      "v_accvgpr_read_b32 %0, %4\n\tv_accvgpr_read_b32 %1, %5\n\t"
+      "v_accvgpr_read_b32 %2, %6\n\tv_accvgpr_read_b32 %3, %7"
+      : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3])
+      : "a"(c[0]), "a"(c[1]), "a"(c[2]), "a"(c[3]));
+}
+
+// Four waves, each a quarter of a tile of BM rows of x and BN rows of W: one wave
+// a SIMD, whose 512 registers hold the sums and two sets of operands. K goes by
+// 64 columns (a K-tile), through SX buffers of x and SW of W in LDS, straight
+// from memory. A row of a buffer has 128 bytes; its pieces of 16 lie at their
+// index ^ (row / 2) % 8, so that the operands of 16 rows spread over the banks.
+//
+// A K-tile is 2 F slots of a matrix instruction and what is issued beside it,
+// so that no unit gets a burst (loads all at once, in half of the slots, took
+// 103 us where these take 79, of 512 x 22016 x 4096): in the first half the
+// operands of the second are read; from slot B1, when all waves have read theirs
+// and the buffer is free, it is filled for the K-tile SX (SW) on; from slot B2,
+// when the next K-tile is there, that one's first operands are read.
+//
+// Workgroups stay for all of their tiles, and the buffers are filled for the
+// next one during the end of the one before. Tiles go to XCDs in runs, down
+// bands of 8, so that those that run together share rows in its L2 (7931 x 28672
+// x 4096: 1432 us down all rows and one tile a workgroup, 1330 now).
+template <int BM, int BN, int WR, int WC, int SX, int SW, Kind KIND>
+__global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
+    const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
+    void *__restrict__ y, int M, int N, int K, int tm, int tn, int kt) {
+  constexpr bool GLU = KIND == SILU || KIND == GELU;
+  constexpr int WAVES = WR * WC, FM = BM / WR / 16, FN = BN / WC / 16;
+  constexpr int LOADS = (BM + BN) / 8 / WAVES;      // of a wave and K-tile
+  constexpr int XL = BM / 8 / WAVES, WL = LOADS - XL;
+  constexpr int XS = BM * 128, WS = BN * 128;       // bytes of a buffer
+  static_assert(SW == SX || SW == SX + 1, "buffers");
+  static_assert(!GLU || FN % 2 == 0, "pairs");
+  static_assert(BN % (8 * WAVES) == 0 && BM % (8 * WAVES) == 0, "loads");
+  extern __shared__ __attribute__((aligned(128))) char smem[];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wid / WC, wn = wid % WC;
+
+  // this workgroup's tiles: every per-th of its XCD's
+  const int nwg = tm * tn, xcd = blockIdx.x % 8;
+  const int q8 = nwg / 8, r8 = nwg % 8;
+  const int begin = xcd * q8 + min(xcd, r8);
+  const int end = begin + q8 + (xcd < r8);
+  const int per = (gridDim.x + 7 - xcd) / 8;
+  int at = begin + blockIdx.x / 8;
+  if (at >= end) return;
+  const int kb = blockIdx.y * kt, kn = min(kt, K / 64 - kb);
+
+  struct Place { int m0, n0; u32x4v rx, rw; };
+  auto place = [&](int at) {
+    Place p;
+    const int band = at / (8 * tn), in = at % (8 * tn);
+    const int rows = min(8, tm - band * 8);
+    p.m0 = (band * 8 + in % rows) * BM;
+    p.n0 = in / rows * BN;
+    auto rsrc = [&](const uint16_t *base, int row, int rows) {
+      const uint64_t a = (uint64_t)(base + (int64_t)row * K);
+      u32x4v v;
+      v[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
+      v[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffff);
+      v[2] = __builtin_amdgcn_readfirstlane(
+          (uint32_t)rows * (uint32_t)K * 2);
+      v[3] = 0x00020000;
+      return v;
+    };
+    p.rx = rsrc(x, p.m0, min(M - p.m0, BM));
+    p.rw = GLU ? rsrc(w, p.n0 / 2, N - p.n0 / 2)
+               : rsrc(w, p.n0, min(N - p.n0, BN));
+    return p;
+  };
+  Place here = place(at);
+
+  unsigned voff[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int row = (i * WAVES + wid) * 8 + (lane >> 3);
+    const int c = (lane & 7) ^ ((row >> 1) & 7);
+    int from = i < XL ? row : row - BM;
+    if (GLU && i >= XL) {               // a wave's gates, then its units
+      const int in = from % (FN * 16);
+      from = from / (FN * 16) * (FN * 8) + in % (FN * 8) +
+             (in < FN * 8 ? 0 : N / 2);
+    }
+    voff[i] = (unsigned)from * (unsigned)(K * 2) + c * 16;
+  }
+  auto load = [&](const Place &p, int t, int b, int i) {
+    const unsigned at = (i * WAVES + wid) * 1024;
+    dma(i < XL ? p.rx : p.rw, voff[i], (unsigned)(kb + t) * 128,
+        i < XL ? b * XS + at : SX * XS + b * WS + at - XS);
+  };
+  f32x4v acc[FM][FN];
+  auto clear = [&] {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = (f32x4v)(0.0f);
+  };
+  clear();
+
+  const int fr = lane & 15, fk = lane >> 4, sw = (fr >> 1) & 7;
+  const int xa = (wm * FM * 16 + fr) * 128;
+  const int wa = SX * XS + (wn * FN * 16 + fr) * 128;
+  const int c0 = (fk ^ sw) * 16, c1 = ((fk + 4) ^ sw) * 16;
+  bf16x8v fx[2][FM], fw[2][FN];
+  auto frag = [&](int set, int bx, int bw, int i) {
+    const char *b = smem + (set ? c1 : c0);
+    if (i < FN)
+      fw[set][i] =
+          *reinterpret_cast<const bf16x8v *>(b + bw * WS + wa + i * 2048);
+    else
+      fx[set][i - FN] = *reinterpret_cast<const bf16x8v *>(
+          b + bx * XS + xa + (i - FN) * 2048);
+  };
+  auto wait = [](auto n) {
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(decltype(n)::value)
+                 : "memory");
+  };
+#pragma unroll
+  for (int u = -SW; u < 0; ++u)
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      if (i >= XL) load(here, u + SW, u + SW, i);
+      else if (u + SX >= 0) load(here, u + SX, u + SX, i);
+  constexpr int AHEAD = (SX - 2) * LOADS + (SW > SX ? WL : 0);
+  wait(std::integral_constant<int, AHEAD + LOADS>());
+#pragma unroll
+  for (int i = 0; i < FM + FN; ++i) frag(0, 0, 0, i);
+
+  constexpr int F = FM * FN, R = FM + FN;
+  constexpr int B1 = F / 2 > R + 1 ? F / 2 : (R + 2 < F ? R + 2 : F - 1);
+  constexpr int B2 = F + (F - 2 - F * 6 / 16 >= R ? F * 6 / 16
+                          : F - R > 2 ? (F - R) / 2 : 1);
+  constexpr int R1 = (B1 - 2) / R > 0 ? (B1 - 2) / R : 1;
+  constexpr int R2 = (2 * F - B2 - 1) / R > 0 ? (2 * F - B2 - 1) / R : 1;
+  constexpr int D = (2 * F - B1) / LOADS;
+  constexpr int BEFORE =
+      (B2 - B1 + D - 1) / D < LOADS ? (B2 - B1 + D - 1) / D : LOADS;
+  static_assert(D > 0 && (R - 1) * R1 < B1 && B2 + 1 + (R - 1) * R2 < 2 * F,
+                "slots");
+  int bx = 0, bw = 0;
+  while (true) {
+    const int then = at + per;
+    const bool more = then < end;
+    const Place next = more ? place(then) : here;
+    for (int t = 0; t < kn; ++t) {
+      const int nx = bx + 1 == SX ? 0 : bx + 1, nw = bw + 1 == SW ? 0 : bw + 1;
+      Place p;                        // of the K-tiles that are fetched now
+      p.rx = t + SX < kn ? here.rx : next.rx;
+      p.rw = t + SW < kn ? here.rw : next.rw;
+      const int tx = t + SX < kn ? t + SX : t + SX - kn;
+      const int tw = t + SW < kn ? t + SW : t + SW - kn;
+#pragma unroll
+      for (int set = 0; set < 2; ++set)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) {
+            const int q = (set * FM + i) * FN + j;
+            if (q == B1)
+              asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (q == B2) wait(std::integral_constant<int, AHEAD + BEFORE>());
+            mma(acc[i][j], fw[set][j], fx[set][i]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (q % R1 == 0 && q / R1 < R) frag(1, bx, bw, q / R1);
+            if (q > B2 && (q - B2 - 1) % R2 == 0 && (q - B2 - 1) / R2 < R)
+              frag(0, nx, nw, (q - B2 - 1) / R2);
+            if (q >= B1 && (q - B1) % D == 0 && (q - B1) / D < LOADS) {
+              const int l = (q - B1) / D;
+              load(p, l < XL ? tx : tw, l < XL ? bx : bw, l);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+      bx = nx;
+      bw = nw;
+      settle(kn - 1 - t);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      const int m = here.m0 + (wm * FM + i) * 16 + fr;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (GLU) {
+#pragma unroll
+        for (int j = 0; j < FN / 2; ++j) {
+          const int n = here.n0 / 2 + (wn * FN / 2 + j) * 16 + fk * 4;
+          if (m >= M || n >= N / 2) continue;
+          float g[4], u[4];
+          take(g, acc[i][j]);
+          take(u, acc[i][j + FN / 2]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            g[e] = ends::gate(g[e], u[e], KIND == GELU);
+          put((uint16_t *)y + (int64_t)m * (N / 2) + n, g);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          const int n = here.n0 + (wn * FN + j) * 16 + fk * 4;
+          if (m >= M || n >= N) continue;
+          float f[4];
+          take(f, acc[i][j]);
+          if constexpr (KIND == PARTS) {
+            *reinterpret_cast<f32x4v *>(
+                (float *)y + ((int64_t)blockIdx.y * M + m) * N + n) =
+                (f32x4v){f[0], f[1], f[2], f[3]};
+          } else {
+            put((uint16_t *)y + (int64_t)m * N + n, f);
+          }
+        }
+      }
+    }
+    if (!more) break;
+    clear();
+    asm volatile("s_nop 7" ::: "memory");
+    at = then;
+    here = next;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+}  // namespace tiles
+
+namespace {
+
+using tiles::Kind;
+
+// What a tile takes in us, fitted to products of 129 to 8192 rows: a K-tile, and
+// begin and end. Small ones are bound by L2, at 32 and 40 kB a K-tile.
+struct Tile {
+  int bm, bn;
+  double step, rest;
+};
+
+constexpr Tile TILES[] = {{256, 256, 1.40, 7.0}, {192, 256, 1.04, 6.5},
+                          {256, 192, 1.13, 6.5}, {256, 128, 0.78, 6.0},
+                          {128, 256, 0.80, 6.0}, {128, 192, 0.74, 5.0},
+                          {128, 128, 0.54, 5.0}};
+constexpr int N_TILES = sizeof(TILES) / sizeof(TILES[0]), MAX_PARTS = 4;
+
+struct Choice { int tile = -1, parts = 1; double us = 1e30; };
+
+// Whether each of `parts` has K-tiles enough for the buffers.
+bool divides(int64_t K, int parts) {
+  const int64_t all = K / 64, each = (all + parts - 1) / parts;
+  return all - (parts - 1) * each >= 4;
+}
+
+// The fastest by these times: rounds of 256 workgroups, and fp32 parts written
+// and read at 5 TB/s.
+Choice choose(int64_t M, int64_t N, int64_t K, int max_parts, int only) {
+  Choice best;
+  for (int v = 0; v < N_TILES; ++v) {
+    if (only >= 0 && v != only) continue;
+    const Tile &t = TILES[v];
+    const int64_t n = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn);
+    for (int p = 1; p <= max_parts; ++p) {
+      if (!divides(K, p)) continue;
+      const int64_t rounds = (n * p + 255) / 256;
+      const double steps = (double)((K / 64 + p - 1) / p);
+      double us = rounds * steps * t.step + t.rest * (1 + 0.3 * (rounds - 1));
+      if (p > 1) us += p * M * N * 8 / 5e6;
+      if (us < best.us) best = {v, p, us};
+    }
+  }
+  return best;
+}
+
+template <int BM, int BN, int SX, int SW, Kind KIND>
+void launch(const at::Tensor &x, const at::Tensor &w, at::Tensor &y, int parts) {
+  auto kernel = tiles::gemm_tiles_kernel<BM, BN, 2, 2, SX, SW, KIND>;
+  constexpr int lds = (SX * BM + SW * BN) * 128;
+  static const bool once =
+      hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, lds) ==
+      hipSuccess;
+  TORCH_CHECK(once, "tile_gemm: LDS size");
+  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
+  const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
+  const int kt = (K / 64 + parts - 1) / parts;
+  hipLaunchKernelGGL(kernel, dim3(std::min(tm * tn, 256), parts), dim3(256),
+                     lds, at::cuda::getCurrentHIPStream(),
+                     (const uint16_t *)x.data_ptr(),
+                     (const uint16_t *)w.data_ptr(), y.data_ptr(), M, N, K, tm,
+                     tn, kt);
+  C10_CUDA_KERNEL_LAUNCH_CHECK();
+}
+
+template <Kind KIND>
+void run(int tile, const at::Tensor &x, const at::Tensor &w, at::Tensor &y,
+         int parts) {
+  switch (tile) {
+    case 0: return launch<256, 256, 2, 2, KIND>(x, w, y, parts);
+    case 1: return launch<192, 256, 2, 2, KIND>(x, w, y, parts);
+    case 2: return launch<256, 192, 2, 2, KIND>(x, w, y, parts);
+    case 3: return launch<256, 128, 3, 3, KIND>(x, w, y, parts);
+    case 4: return launch<128, 256, 2, 3, KIND>(x, w, y, parts);
+    case 5: return launch<128, 192, 3, 4, KIND>(x, w, y, parts);
+    default: return launch<128, 128, 3, 4, KIND>(x, w, y, parts);
+  }
+}
+
+bool fits(const at::Tensor &t) {
+  return t.is_cuda() && t.dim() == 2 && t.is_contiguous() &&
+         t.scalar_type() == at::kBFloat16 && t.size(0) > 0 &&
+         t.size(0) < (1 << 24) &&
+         reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+
+}  // namespace
+
+// Whether tile_gemm takes x and W (with `glu`, W = [G ; U]).
+bool tile_gemm_takes(at::Tensor x, at::Tensor w, bool glu) {
+  return fits(x) && fits(w) && x.size(1) == w.size(1) &&
+         x.device() == w.device() && x.size(1) % 64 == 0 &&
+         x.size(1) >= 256 && x.size(1) <= (1 << 20) &&
+         w.size(0) % (glu ? 8 : 4) == 0 &&
+         (!glu || w.size(0) * w.size(1) * 2 < ((int64_t)1 << 32));
+}
+
+// Parts that tile_gemm makes of sums where it may.
+int64_t tile_gemm_parts(int64_t M, int64_t N, int64_t K) {
+  return choose(M, N, K, MAX_PARTS, -1).parts;
+}
+
+// x W^T: bf16 [M, N]; where max_parts > 1, possibly fp32 parts [P, M, N] of the
+// sums. glu 1 (SiLU) or 2 (tanh-GELU): act(x G^T) * (x U^T) of W = [G ; U]. tile
+// and parts: the choice of a test.
+at::Tensor tile_gemm(at::Tensor x, at::Tensor w, int64_t max_parts, int64_t glu,
+                     int64_t tile, int64_t parts) {
+  TORCH_CHECK(tile_gemm_takes(x, w, glu != 0) && glu >= 0 && glu <= 2 &&
+              (glu == 0 || (max_parts <= 1 && parts <= 1)) &&
+              tile < N_TILES && max_parts <= MAX_PARTS && parts <= MAX_PARTS,
+              "tile_gemm: x ", x.sizes(), ", W ", w.sizes());
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  Choice c = choose(M, N, K, (int)max_parts, (int)tile);
+  if (parts > 0) c.parts = (int)parts;
+  TORCH_CHECK(divides(K, c.parts), "tile_gemm: parts");
+  if (c.parts > 1) {
+    auto y = at::empty({c.parts, M, N}, x.options().dtype(at::kFloat));
+    run<tiles::PARTS>(c.tile, x, w, y, c.parts);
+    return y;
+  }
+  auto y = at::empty({M, glu ? N / 2 : N}, x.options());
+  if (glu == 1) run<tiles::SILU>(c.tile, x, w, y, 1);
+  else if (glu == 2) run<tiles::GELU>(c.tile, x, w, y, 1);
+  else run<tiles::PLAIN>(c.tile, x, w, y, 1);
+  return y;
+}

@@ -195,6 +195,15 @@ def _rows_linear(x: torch.Tensor, weight: torch.Tensor, m: int, n: int,
     return y.view(*x.shape[:-1], n)
 
 
+def _tiles_serve(x: torch.Tensor, weight: torch.Tensor, glu: bool = False
+                 ) -> bool:
+    """The tiles of csrc/gemm_tiles.hip take x, of more than 128 rows, for a
+    result that is not differentiated."""
+    return (x.is_cuda and x.dim() == 2 and x.shape[0] > 128 and
+            x.dtype == torch.bfloat16 and not torch.is_grad_enabled() and
+            _backend.ext().tile_gemm_takes(x, weight, glu))
+
+
 def _rows_served(x: torch.Tensor, weight: torch.Tensor):
     """_rows_copy for results that are not differentiated, of 33 to 128 rows."""
     if not (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and
@@ -206,10 +215,15 @@ def _rows_served(x: torch.Tensor, weight: torch.Tensor):
 
 def rows_glu(x: torch.Tensor, weight: torch.Tensor, gelu: bool
              ) -> torch.Tensor | None:
-    """act(x G^T) * (x U^T) of weight = [G ; U] and 33 to 128 rows in one
-    launch, or None where no paired copy serves it (us with the product and the
-    gated unit apart and here, 64 rows: 22016 x 4096 40.2 and 37.6, 49152 x 3072
-    64.5 and 59.1)."""
+    """act(x G^T) * (x U^T) of weight = [G ; U] and more than 32 rows in one
+    launch, or None where nothing serves it: up to 128 rows a paired copy (us
+    with the product and the gated unit apart and here, 64 rows: 22016 x 4096
+    40.2 and 37.6, 49152 x 3072 64.5 and 59.1), above that tiles (22016 x 4096: 129
+    rows 55 and 49, 512 91 and 77, 2048 298 and 297, 5000 720 and 663; 28672 x
+    4096: 600 143 and 147, 1021 203 and 188, 7931 1425 and 1340; 49152 x 3072:
+    256 98 and 78, 1021 269 and 236, 3001 744 and 706)."""
+    if _tiles_serve(x, weight, True):
+        return _backend.ext().tile_gemm(x, weight, glu=2 if gelu else 1)
     dw, n = _rows_served(x, weight), weight.shape[0]
     if dw is None or dw[2] * 2 != n or \
             not _backend.ext().rows_ends_pay(x.shape[0], n, x.shape[1]):
@@ -232,14 +246,40 @@ def rows_heads(x: torch.Tensor, weight: torch.Tensor, cos, sin, positions, kc,
 
 
 def rows_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
-    """x @ weight^T of 33 to 128 rows for a norm that adds up parts of it
+    """x @ weight^T of more than 32 rows for a norm that adds up parts of it
     (ops.rmsnorm_res): fp32 [P, T, N], or [T, N] where the kernel splits
-    nothing; None where no copy serves it. us with the sum in a launch of its
+    nothing; None where nothing serves it. us with the sum in a launch of its
     own and in the norm, 64 rows: 4096 x 4096 17.8 and 16.4, 4096 x 11008 29.3
-    and 27.6."""
+    and 27.6.
+
+    Above 128 rows in tiles, where these are few and so share the sums, or one
+    round of them does (us with the norm, library and here: 4096 x 4096 129 rows
+    31 and 19, 300 32 and 27, 512 34 and 31; 4096 x 14336 129 58 and 39, 512 97
+    and 65, 1021 141 and 109, 2048 220 and 206; 3072 x 24576 512 151 and 90,
+    1021 209 and 136, 2048 328 and 252; 8192 x 8192 512 87 and 74). Otherwise
+    the library is as fast or faster (4096 x 4096 768 39 and 45, 8192 x 8192
+    1280 147 and 157)."""
+    if _tiles_serve(x, weight):
+        (m, k), n = x.shape, weight.shape[0]
+        if _backend.ext().tile_gemm_parts(m, n, k) > 1:
+            return _backend.ext().tile_gemm(x, weight, max_parts=4)
+        return _one_round(x, weight)
     dw = _rows_served(x, weight)
     return None if dw is None else _backend.ext().decode_gemm_rows(
         x, dw[0], weight.shape[0], dw[2], True)
+
+
+def _one_round(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
+    """x @ weight^T of long rows in one round of tiles of 256 x 128, or None
+    where the library is as good: it takes 192 or 256 columns, too few tiles for
+    256 CUs (us there and here, to 4096 columns: 2048 rows of 11008 160 and 145,
+    of 14336 205 and 180; 2048 of 4096 58 and 58; 1280 of 11008 119 and 130)."""
+    (m, k), n = x.shape, weight.shape[0]
+    tiles = -(-m // 256) * -(-n // 128)
+    if k > 8192 and 224 <= tiles <= 256 and m <= 2048 and \
+            _backend.ext().tile_gemm_takes(x, weight):
+        return _backend.ext().tile_gemm(x, weight)
+    return None
 
 
 def _whole_rounds(rows: int, cols: int) -> int:
@@ -265,6 +305,9 @@ def _whole_rounds(rows: int, cols: int) -> int:
 def wide_product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """x @ weight^T on the GPU for a result that is not differentiated, in
     whole rounds of tiles."""
+    y = _one_round(x, weight)
+    if y is not None:
+        return y
     rows, cols = x.shape[0], weight.shape[0]
     main = _whole_rounds(rows, cols)
     if main >= cols:
@@ -285,6 +328,10 @@ def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     6144 x 4096 15.9 and 15.4, of 24 rows 47.9 and 52.6, 14.7 and 15.0)."""
     if x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2:
         (m, k), n = x.shape, weight.shape[0]
+        if m <= 320 and n >= 12288 and _tiles_serve(x, weight):
+            # us in the library and in tiles, 12288 x 4096: 129 rows 39 and 35,
+            # 300 52 and 46, 384 51 and 53; 6144 x 4096 200 25 and 34
+            return _backend.ext().tile_gemm(x, weight)
         if m > 1280:
             return wide_product(x, weight)
         if 16 < m <= 32 and 10240 <= n <= 32768 and \

@@ -25,7 +25,7 @@ CSRC = ROOT / "runbooks_amd" / "ops" / "csrc"
 # streams, `dual` those with norms and input convolutions side by side, `main`
 # the rest.
 GROUPS = {"core": ("rmsnorm", "layernorm", "glu", "decode_gemm", "decode_res",
-                    "decode_affine", "sampling"),
+                    "decode_affine", "gemm_tiles", "sampling"),
           "streams": ("streams", "qkv_prep", "min_gru", "moe"),
           "delta": ("delta", "delta_out", "general_delta"),
           "dual": ("canon", "qkv_conv", "poly_norm")}

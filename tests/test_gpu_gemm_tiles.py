@@ -1,0 +1,106 @@
+"""Products in tiles (csrc/gemm_tiles.hip) at the edges of their tiles, with
+their sums in parts and ended by a gated unit, against fp32."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TILES = range(7)        # 256x256 192x256 256x192 256x128 128x256 128x192 128x128
+
+
+def _inputs(m, n, k, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed + m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(n, k, device="cuda", generator=g) * k ** -0.5).bfloat16()
+    return x, w
+
+
+def _check(got, x, w, rounding):
+    """Sums of k products in fp32, in any order: off by at most k eps times the
+    sum of their absolute values; and their rounding."""
+    ref = x.float() @ w.float().t()
+    size = x.float().abs() @ w.float().abs().t()
+    bound = rounding * ref.abs() + 2 * x.shape[1] * 2.0 ** -24 * size
+    assert bool(((got.float() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("m,n,k", [
+    (1, 4, 256),            # less than a fragment, the fewest columns of K
+    (129, 260, 320),        # remainders of every tile, odd K-tiles
+    (256, 512, 512),        # whole tiles
+    (513, 1028, 448),
+    (4100, 4360, 256),      # several tiles for a workgroup
+])
+def test_product(tile, m, n, k):
+    from runbooks_amd import ops
+    x, w = _inputs(m, n, k)
+    _check(ops.ext().tile_gemm(x, w, tile=tile), x, w, 2.0 ** -8)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("m,n,k,parts", [
+    (129, 260, 1088, 4),    # 5, 5, 5 and 2 K-tiles are not enough: refused
+    (130, 516, 1024, 4),
+    (300, 260, 576, 2),     # 5 and 4
+    (257, 4100, 1472, 3),
+])
+def test_parts(tile, m, n, k, parts):
+    from runbooks_amd import ops
+    x, w = _inputs(m, n, k)
+    run = lambda: ops.ext().tile_gemm(x, w, parts, tile=tile, parts=parts)  # noqa: E731
+    if -(-(k // 64) // parts) * (parts - 1) + 4 > k // 64:
+        with pytest.raises(RuntimeError):
+            run()
+        return
+    y = run()
+    assert y.shape == (parts, m, n) and y.dtype == torch.float32
+    _check(y.sum(0), x, w, 2.0 ** -22)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("glu", [1, 2])
+@pytest.mark.parametrize("m,n,k", [(1, 8, 256), (200, 520, 320),
+                                   (4100, 4360, 256)])
+def test_gated_unit(tile, glu, m, n, k):
+    from runbooks_amd import ops
+    x, w = _inputs(m, n, k)
+    got = ops.ext().tile_gemm(x, w, glu=glu, tile=tile).float()
+    g, u = (x.float() @ w.float().t()).chunk(2, 1)
+    act = torch.nn.functional.silu(g) if glu == 1 else \
+        torch.nn.functional.gelu(g, approximate="tanh")
+    ref = act * u
+    # the product's errors (of values around 1, 1e-5) through gate and unit,
+    # and one rounding
+    assert bool(((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(129, 4096, 4096), (512, 4096, 11008),
+                                   (300, 3072, 24576), (768, 4096, 4096)])
+def test_sums_for_the_norm(m, n, k):
+    """rows_parts of more than 128 rows: parts, or what the library is left
+    with; refused are rows and parameters that do not lie as the kernel reads
+    them."""
+    from runbooks_amd import ops
+    x, w = _inputs(m, n, k)
+    with torch.no_grad():
+        y = ops.rows_parts(x, w)
+        if y is not None:
+            _check(y.sum(0) if y.dim() == 3 else y, x, w, 2.0 ** -8)
+        wide = torch.zeros(m, 2 * k, device="cuda", dtype=torch.bfloat16)
+        assert ops.rows_parts(wide[:, :k], w) is None
+        assert ops.rows_glu(x.float(), w.float(), False) is None
+    assert ops.rows_parts(x, w) is None         # would be differentiated
+
+
+def test_one_row_does_not_reach_others():
+    """An infinite and a NaN row stay to themselves."""
+    from runbooks_amd import ops
+    x, w = _inputs(300, 520, 512)
+    clean = ops.ext().tile_gemm(x, w)
+    x[7] = float("inf")
+    x[299, 3] = float("nan")
+    got = ops.ext().tile_gemm(x, w)
+    keep = [i for i in range(300) if i not in (7, 299)]
+    assert torch.equal(got[keep], clean[keep])
+    assert bool(got[299].isnan().all()) and not bool(got[7].isfinite().any())

@@ -97,7 +97,7 @@ __device__ __forceinline__ void take(float (&f)[4], const f32x4v &c) {
 template <int BM, int BN, int WR, int WC, int SX, int SW, Kind KIND>
 __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
-    void *__restrict__ y, int M, int N, int K, int tm, int tn, int kt) {
+    void *__restrict__ y, int M, int N, int K, int tm, int tn, int kt, int first) {
   constexpr bool GLU = KIND == SILU || KIND == GELU;
   constexpr int WAVES = WR * WC, FM = BM / WR / 16, FN = BN / WC / 16;
   constexpr int LOADS = (BM + BN) / 8 / WAVES;      // of a wave and K-tile
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
     const int band = at / (8 * tn), in = at % (8 * tn);
     const int rows = min(8, tm - band * 8);
     p.m0 = (band * 8 + in % rows) * BM;
-    p.n0 = in / rows * BN;
+    p.n0 = first + in / rows * BN;
     auto rsrc = [&](const uint16_t *base, int row, int rows) {
       const uint64_t a = (uint64_t)(base + (int64_t)row * K);
       u32x4v v;
@@ -306,13 +306,19 @@ struct Tile {
   double step, rest;
 };
 
-constexpr Tile TILES[] = {{256, 256, 1.40, 7.0}, {192, 256, 1.04, 6.5},
+constexpr Tile TILES[] = {{256, 256, 1.40, 7.0}, {192, 256, 1.12, 6.5},
                           {256, 192, 1.13, 6.5}, {256, 128, 0.78, 6.0},
                           {128, 256, 0.80, 6.0}, {128, 192, 0.74, 5.0},
                           {128, 128, 0.54, 5.0}};
 constexpr int N_TILES = sizeof(TILES) / sizeof(TILES[0]), MAX_PARTS = 4;
 
-struct Choice { int tile = -1, parts = 1; double us = 1e30; };
+// Columns (of W's rows) up to `split` in tiles of `tile`, the others in `rest`;
+// split 0: all in `tile`.
+struct Choice {
+  int tile = -1, parts = 1, rest = -1;
+  int64_t split = 0;
+  double us = 1e30;
+};
 
 // Whether each of `parts` has K-tiles enough for the buffers.
 bool divides(int64_t K, int parts) {
@@ -334,14 +340,35 @@ Choice choose(int64_t M, int64_t N, int64_t K, int max_parts, int only) {
       const double steps = (double)((K / 64 + p - 1) / p);
       double us = rounds * steps * t.step + t.rest * (1 + 0.3 * (rounds - 1));
       if (p > 1) us += p * M * N * 8 / 5e6;
-      if (us < best.us) best = {v, p, us};
+      if (us < best.us) best = {v, p, -1, 0, us};
     }
   }
   return best;
 }
 
+// choose(), or whole rounds of a tile and the rest in a launch of its own, where
+// a round that is nearly empty would follow (us with the gated unit, in one, in
+// two, and the library's product and the unit: 700 x 22016 x 4096 134, 125 and
+// 151, 2200 x 22016 x 4096 362, 309 and 330, 1800 x 28672 x 4096 387, 337 and 354,
+// 6500 x 28672 x 4096 1127, 1093 and 1283).
+Choice choose_two(int64_t M, int64_t N, int64_t K) {
+  Choice best = choose(M, N, K, 1, -1);
+  for (int v = 0; v < N_TILES; ++v) {
+    const Tile &t = TILES[v];
+    const int64_t tm = (M + t.bm - 1) / t.bm, tn = (N + t.bn - 1) / t.bn;
+    const int64_t rounds = tm * tn / 256, cols = rounds * 256 / tm;
+    if (rounds == 0 || cols >= tn) continue;
+    const Choice rest = choose(M, N - cols * t.bn, K, 1, -1);
+    const double us = rounds * (K / 64) * t.step +
+                      t.rest * (1 + 0.3 * (rounds - 1)) + rest.us;
+    if (us + 3 < best.us) best = {v, 1, rest.tile, cols * t.bn, us + 3};
+  }
+  return best;
+}
+
 template <int BM, int BN, int SX, int SW, Kind KIND>
-void launch(const at::Tensor &x, const at::Tensor &w, at::Tensor &y, int parts) {
+void launch(const at::Tensor &x, const at::Tensor &w, at::Tensor &y, int parts,
+            int64_t first, int64_t last) {
   auto kernel = tiles::gemm_tiles_kernel<BM, BN, 2, 2, SX, SW, KIND>;
   constexpr int lds = (SX * BM + SW * BN) * 128;
   static const bool once =
@@ -350,27 +377,27 @@ void launch(const at::Tensor &x, const at::Tensor &w, at::Tensor &y, int parts) 
       hipSuccess;
   TORCH_CHECK(once, "tile_gemm: LDS size");
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
-  const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
+  const int tm = (M + BM - 1) / BM, tn = (int)((last - first + BN - 1) / BN);
   const int kt = (K / 64 + parts - 1) / parts;
   hipLaunchKernelGGL(kernel, dim3(std::min(tm * tn, 256), parts), dim3(256),
                      lds, at::cuda::getCurrentHIPStream(),
                      (const uint16_t *)x.data_ptr(),
                      (const uint16_t *)w.data_ptr(), y.data_ptr(), M, N, K, tm,
-                     tn, kt);
+                     tn, kt, (int)first);
   C10_CUDA_KERNEL_LAUNCH_CHECK();
 }
 
 template <Kind KIND>
 void run(int tile, const at::Tensor &x, const at::Tensor &w, at::Tensor &y,
-         int parts) {
+         int parts, int64_t first, int64_t last) {
   switch (tile) {
-    case 0: return launch<256, 256, 2, 2, KIND>(x, w, y, parts);
-    case 1: return launch<192, 256, 2, 2, KIND>(x, w, y, parts);
-    case 2: return launch<256, 192, 2, 2, KIND>(x, w, y, parts);
-    case 3: return launch<256, 128, 3, 3, KIND>(x, w, y, parts);
-    case 4: return launch<128, 256, 2, 3, KIND>(x, w, y, parts);
-    case 5: return launch<128, 192, 3, 4, KIND>(x, w, y, parts);
-    default: return launch<128, 128, 3, 4, KIND>(x, w, y, parts);
+    case 0: return launch<256, 256, 2, 2, KIND>(x, w, y, parts, first, last);
+    case 1: return launch<192, 256, 2, 2, KIND>(x, w, y, parts, first, last);
+    case 2: return launch<256, 192, 2, 2, KIND>(x, w, y, parts, first, last);
+    case 3: return launch<256, 128, 3, 3, KIND>(x, w, y, parts, first, last);
+    case 4: return launch<128, 256, 2, 3, KIND>(x, w, y, parts, first, last);
+    case 5: return launch<128, 192, 3, 4, KIND>(x, w, y, parts, first, last);
+    default: return launch<128, 128, 3, 4, KIND>(x, w, y, parts, first, last);
   }
 }
 
@@ -407,17 +434,27 @@ at::Tensor tile_gemm(at::Tensor x, at::Tensor w, int64_t max_parts, int64_t glu,
               tile < N_TILES && max_parts <= MAX_PARTS && parts <= MAX_PARTS,
               "tile_gemm: x ", x.sizes(), ", W ", w.sizes());
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  Choice c = choose(M, N, K, (int)max_parts, (int)tile);
+  Choice c = max_parts > 1 || tile >= 0 ? choose(M, N, K, (int)max_parts,
+                                                 (int)tile)
+                                        : choose_two(M, N, K);
   if (parts > 0) c.parts = (int)parts;
   TORCH_CHECK(divides(K, c.parts), "tile_gemm: parts");
   if (c.parts > 1) {
     auto y = at::empty({c.parts, M, N}, x.options().dtype(at::kFloat));
-    run<tiles::PARTS>(c.tile, x, w, y, c.parts);
+    run<tiles::PARTS>(c.tile, x, w, y, c.parts, 0, N);
     return y;
   }
   auto y = at::empty({M, glu ? N / 2 : N}, x.options());
-  if (glu == 1) run<tiles::SILU>(c.tile, x, w, y, 1);
-  else if (glu == 2) run<tiles::GELU>(c.tile, x, w, y, 1);
-  else run<tiles::PLAIN>(c.tile, x, w, y, 1);
+  auto go = [&](int t, int64_t first, int64_t last) {
+    if (glu == 1) run<tiles::SILU>(t, x, w, y, 1, first, last);
+    else if (glu == 2) run<tiles::GELU>(t, x, w, y, 1, first, last);
+    else run<tiles::PLAIN>(t, x, w, y, 1, first, last);
+  };
+  if (c.split > 0) {
+    go(c.tile, 0, c.split);
+    go(c.rest, c.split, N);
+  } else {
+    go(c.tile, 0, N);
+  }
   return y;
 }

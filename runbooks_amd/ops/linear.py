@@ -219,9 +219,9 @@ def rows_glu(x: torch.Tensor, weight: torch.Tensor, gelu: bool
     launch, or None where nothing serves it: up to 128 rows a paired copy (us
     with the product and the gated unit apart and here, 64 rows: 22016 x 4096
     40.2 and 37.6, 49152 x 3072 64.5 and 59.1), above that tiles (22016 x 4096: 129
-    rows 55 and 49, 512 91 and 77, 2048 298 and 297, 5000 720 and 663; 28672 x
-    4096: 600 143 and 147, 1021 203 and 188, 7931 1425 and 1340; 49152 x 3072:
-    256 98 and 78, 1021 269 and 236, 3001 744 and 706)."""
+    rows 55 and 48, 512 91 and 77, 1537 247 and 233, 2048 298 and 270, 4500 623
+    and 586; 28672 x 4096: 1400 277 and 283, 1800 354 and 337, 6500 1283 and
+    1093; 49152 x 3072: 256 98 and 76, 1021 267 and 228, 3200 821 and 713)."""
     if _tiles_serve(x, weight, True):
         return _backend.ext().tile_gemm(x, weight, glu=2 if gelu else 1)
     dw, n = _rows_served(x, weight), weight.shape[0]

@@ -75,6 +75,19 @@ def test_gated_unit(tile, glu, m, n, k):
     assert bool(((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(700, 22016, 512), (2200, 22016, 1024),
+                                   (1800, 28680, 1024)])
+def test_two_launches(m, n, k):
+    """Sizes of more tiles than whole rounds: columns in tiles of two sizes."""
+    from runbooks_amd import ops
+    x, w = _inputs(m, n, k)
+    _check(ops.ext().tile_gemm(x, w), x, w, 2.0 ** -8)
+    g, u = (x.float() @ w.float().t()).chunk(2, 1)
+    ref = torch.nn.functional.silu(g) * u
+    got = ops.ext().tile_gemm(x, w, glu=1).float()
+    assert bool(((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(129, 4096, 4096), (512, 4096, 11008),
                                    (300, 3072, 24576), (768, 4096, 4096)])
 def test_sums_for_the_norm(m, n, k):

@@ -41,6 +41,7 @@ void affine_add_(at::Tensor x, at::Tensor w, c10::optional<at::Tensor> bias, at:
 at::Tensor embed_res32(at::Tensor tokens, at::Tensor positions, at::Tensor table, at::Tensor places);
 at::Tensor sum_parts(at::Tensor parts);
 bool tile_gemm_takes(at::Tensor x, at::Tensor w, bool glu);
+at::Tensor tile_lora(at::Tensor x, at::Tensor w, at::Tensor t, std::vector<at::Tensor> bs, double scale, int64_t tile);
 int64_t tile_gemm_parts(int64_t M, int64_t N, int64_t K);
 at::Tensor tile_gemm(at::Tensor x, at::Tensor w, int64_t max_parts, int64_t glu, int64_t tile, int64_t parts);
 at::Tensor decode_gemm_rows(at::Tensor x, at::Tensor ws, int64_t N, int64_t half, bool raw);
@@ -167,6 +168,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sum_parts", &sum_parts, "fp32 [P, M, N] -> their sum [M, N] bf16");
   m.def("tile_gemm_takes", &tile_gemm_takes, py::arg("x"), py::arg("w"),
         py::arg("glu") = false, "whether tile_gemm takes x and W");
+  m.def("tile_lora", &tile_lora, py::arg("x"), py::arg("w"), py::arg("t"),
+        py::arg("bs"), py::arg("scale"), py::arg("tile") = -1,
+        "x @ W^T + scale t_i @ B_i^T of siblings side by side");
   m.def("tile_gemm_parts", &tile_gemm_parts,
         "parts that tile_gemm makes of sums where it may");
   m.def("tile_gemm", &tile_gemm, py::arg("x"), py::arg("w"),

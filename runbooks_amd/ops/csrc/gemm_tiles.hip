@@ -52,10 +52,28 @@ __device__ __forceinline__ void mma(f32x4v &c, bf16x8v a, bf16x8v b) {
                : "+a"(c) : "v"(a), "v"(b));
 }
 
+// A product by itself, outside of the matrix registers, which the sums fill.
+__device__ __forceinline__ f32x4v product(bf16x8v a, bf16x8v b) {
+  f32x4v c;
+  asm volatile(
+      "s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, 0\n\ts_nop 15"
+      : "=&v"(c) : "v"(a), "v"(b));
+  return c;
+}
+
 enum Kind {
   PLAIN,        // y [M, N] bf16
   PARTS,        // fp32 [P, M, N], K-tiles kt * p .. of every part
   SILU, GELU,   // act(x G^T) * (x U^T) of W = [G ; U], y [M, N / 2]
+  LORA,         // y_i + scale t_i B_i^T of siblings side by side
+};
+
+// Adapters of rank 16: t [n, M, 16] and B_i [columns of i, 16], the first columns
+// of the siblings multiples of 16.
+struct Adapters {
+  const uint16_t *t, *b[3];
+  int start[4], n;
+  float scale;
 };
 
 // Waits until the last products are in their registers, if `left` is 0. The
@@ -75,6 +93,65 @@ __device__ __forceinline__ void take(float (&f)[4], const f32x4v &c) {
       "v_accvgpr_read_b32 %2, %6\n\tv_accvgpr_read_b32 %3, %7"
       : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3])
       : "a"(c[0]), "a"(c[1]), "a"(c[2]), "a"(c[3]));
+}
+
+// The end of LORA, in fp32 and rounded once: a product more, of 16 columns (and
+// 16 absent ones), for each of 16 x 16 sums, from rows m0 and columns n0 on. In a
+// pass of its own over y it took 42 us of 2048 x 22016 (lora_group.hip).
+template <int FM, int FN>
+__device__ __forceinline__ void end_lora(const Adapters &a,
+                                         const f32x4v (&acc)[FM][FN],
+                                         uint16_t *y, int m0, int n0, int fr,
+                                         int fk, int M, int N) {
+  const bf16x8v none = (bf16x8v)(__bf16)0.0f;
+  auto sibling = [&](int n) {
+    return (a.n > 1 && n >= a.start[1]) + (a.n > 2 && n >= a.start[2]);
+  };
+  auto start = [&](int s) {
+    return s == 0 ? 0 : s == 1 ? a.start[1] : a.start[2];
+  };
+  const int at = (fk & 1) * 8;
+  bf16x8v bw[FN], tx[FM];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int n = __builtin_amdgcn_readfirstlane(min(n0 + j * 16, N - 16));
+    const int s = sibling(n);
+    const uint16_t *b = s == 0 ? a.b[0] : s == 1 ? a.b[1] : a.b[2];
+    const bf16x8v v = ends::load8v(
+        b + (int64_t)(n - start(s) + fr) * 16 + at);
+    bw[j] = fk < 2 ? v : none;
+  }
+  // of these and those below, where the compiler sees it: otherwise it waits
+  // for all loads in the loop over K that follows
+  constexpr int loaded = 0x0f70;        // vmcnt(0)
+  __builtin_amdgcn_s_waitcnt(loaded);
+  int now = -1;
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int n = __builtin_amdgcn_readfirstlane(n0 + j * 16);
+    if (n >= N) continue;
+    const int s = sibling(n);
+    if (s != now) {
+      now = s;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const bf16x8v v = ends::load8v(
+            a.t + ((int64_t)s * M + min(m0 + i * 16 + fr, M - 1)) * 16 + at);
+        tx[i] = fk < 2 ? v : none;
+      }
+      __builtin_amdgcn_s_waitcnt(loaded);
+    }
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      const int m = m0 + i * 16 + fr;
+      const f32x4v d = product(bw[j], tx[i]);
+      float f[4];
+      take(f, acc[i][j]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[e] += a.scale * d[e];
+      if (m < M) put(y + (int64_t)m * N + n + fk * 4, f);
+    }
+  }
 }
 
 // Four waves, each a quarter of a tile of BM rows of x and BN rows of W: one wave
@@ -97,7 +174,8 @@ __device__ __forceinline__ void take(float (&f)[4], const f32x4v &c) {
 template <int BM, int BN, int WR, int WC, int SX, int SW, Kind KIND>
 __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
-    void *__restrict__ y, int M, int N, int K, int tm, int tn, int kt, int first) {
+    void *__restrict__ y, int M, int N, int K, int tm, int tn, int kt, int first,
+    Adapters lora) {
   constexpr bool GLU = KIND == SILU || KIND == GELU;
   constexpr int WAVES = WR * WC, FM = BM / WR / 16, FN = BN / WC / 16;
   constexpr int LOADS = (BM + BN) / 8 / WAVES;      // of a wave and K-tile
@@ -250,6 +328,10 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
       settle(kn - 1 - t);
     }
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (KIND == LORA)
+      end_lora<FM, FN>(lora, acc, (uint16_t *)y, here.m0 + wm * FM * 16,
+                       here.n0 + wn * FN * 16, fr, fk, M, N);
+    else
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
       const int m = here.m0 + (wm * FM + i) * 16 + fr;
@@ -368,7 +450,7 @@ Choice choose_two(int64_t M, int64_t N, int64_t K) {
 
 template <int BM, int BN, int SX, int SW, Kind KIND>
 void launch(const at::Tensor &x, const at::Tensor &w, at::Tensor &y, int parts,
-            int64_t first, int64_t last) {
+            int64_t first, int64_t last, const tiles::Adapters &lora) {
   auto kernel = tiles::gemm_tiles_kernel<BM, BN, 2, 2, SX, SW, KIND>;
   constexpr int lds = (SX * BM + SW * BN) * 128;
   static const bool once =
@@ -383,21 +465,22 @@ void launch(const at::Tensor &x, const at::Tensor &w, at::Tensor &y, int parts,
                      lds, at::cuda::getCurrentHIPStream(),
                      (const uint16_t *)x.data_ptr(),
                      (const uint16_t *)w.data_ptr(), y.data_ptr(), M, N, K, tm,
-                     tn, kt, (int)first);
+                     tn, kt, (int)first, lora);
   C10_CUDA_KERNEL_LAUNCH_CHECK();
 }
 
 template <Kind KIND>
 void run(int tile, const at::Tensor &x, const at::Tensor &w, at::Tensor &y,
-         int parts, int64_t first, int64_t last) {
+         int parts, int64_t first, int64_t last,
+         const tiles::Adapters &lora = {}) {
   switch (tile) {
-    case 0: return launch<256, 256, 2, 2, KIND>(x, w, y, parts, first, last);
-    case 1: return launch<192, 256, 2, 2, KIND>(x, w, y, parts, first, last);
-    case 2: return launch<256, 192, 2, 2, KIND>(x, w, y, parts, first, last);
-    case 3: return launch<256, 128, 3, 3, KIND>(x, w, y, parts, first, last);
-    case 4: return launch<128, 256, 2, 3, KIND>(x, w, y, parts, first, last);
-    case 5: return launch<128, 192, 3, 4, KIND>(x, w, y, parts, first, last);
-    default: return launch<128, 128, 3, 4, KIND>(x, w, y, parts, first, last);
+    case 0: return launch<256, 256, 2, 2, KIND>(x, w, y, parts, first, last, lora);
+    case 1: return launch<192, 256, 2, 2, KIND>(x, w, y, parts, first, last, lora);
+    case 2: return launch<256, 192, 2, 2, KIND>(x, w, y, parts, first, last, lora);
+    case 3: return launch<256, 128, 3, 3, KIND>(x, w, y, parts, first, last, lora);
+    case 4: return launch<128, 256, 2, 3, KIND>(x, w, y, parts, first, last, lora);
+    case 5: return launch<128, 192, 3, 4, KIND>(x, w, y, parts, first, last, lora);
+    default: return launch<128, 128, 3, 4, KIND>(x, w, y, parts, first, last, lora);
   }
 }
 
@@ -455,6 +538,47 @@ at::Tensor tile_gemm(at::Tensor x, at::Tensor w, int64_t max_parts, int64_t glu,
     go(c.rest, c.split, N);
   } else {
     go(c.tile, 0, N);
+  }
+  return y;
+}
+
+// x W^T + scale t_i B_i^T of one to three siblings side by side: t [n, M, 16], B_i
+// [columns of i, 16].
+at::Tensor tile_lora(at::Tensor x, at::Tensor w, at::Tensor t,
+                     std::vector<at::Tensor> bs, double scale, int64_t tile) {
+  const int64_t M = x.size(0), N = w.size(0);
+  tiles::Adapters a{};
+  a.n = (int)bs.size();
+  TORCH_CHECK(tile_gemm_takes(x, w, false) && tile < N_TILES && a.n >= 1 &&
+              a.n <= 3, "tile_lora: x ", x.sizes(), ", W ", w.sizes());
+  auto adapter = [&](const at::Tensor &m) {
+    TORCH_CHECK(m.is_contiguous() && m.device() == x.device() &&
+                m.scalar_type() == at::kBFloat16 && m.size(-1) == 16 &&
+                reinterpret_cast<uintptr_t>(m.data_ptr()) % 16 == 0,
+                "tile_lora: adapters of rank 16, bf16");
+    return (const uint16_t *)m.data_ptr();
+  };
+  TORCH_CHECK(t.dim() == 3 && t.size(0) == a.n && t.size(1) == M,
+              "tile_lora: t [n, M, 16]");
+  a.t = adapter(t);
+  int64_t at = 0;
+  for (int i = 0; i < a.n; ++i) {
+    TORCH_CHECK(bs[i].dim() == 2 && bs[i].size(0) % 16 == 0 &&
+                bs[i].size(0) > 0, "tile_lora: columns");
+    a.b[i] = adapter(bs[i]);
+    a.start[i] = (int)at;
+    at += bs[i].size(0);
+  }
+  TORCH_CHECK(at == N, "tile_lora: columns of the siblings");
+  a.scale = (float)scale;
+  const Choice c = tile >= 0 ? choose(M, N, x.size(1), 1, (int)tile)
+                             : choose_two(M, N, x.size(1));
+  auto y = at::empty({M, N}, x.options());
+  if (c.split > 0) {
+    run<tiles::LORA>(c.tile, x, w, y, 1, 0, c.split, a);
+    run<tiles::LORA>(c.rest, x, w, y, 1, c.split, N, a);
+  } else {
+    run<tiles::LORA>(c.tile, x, w, y, 1, 0, N, a);
   }
   return y;
 }

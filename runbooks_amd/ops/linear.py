@@ -342,6 +342,24 @@ def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return fast_linear(x, weight)
 
 
+def wide_product_lora(x: torch.Tensor, weight: torch.Tensor, t: torch.Tensor,
+                      bs: list, scale: float) -> torch.Tensor:
+    """wide_product(x, weight) + scale t_i B_i^T of adapters side by side
+    (csrc/lora_group.hip), in tiles that end with the adapters' part, or in the
+    library and a pass over its result (us there and in tiles: 12288 x 4096 129
+    rows 42 and 36, 512 60 and 56, 2048 174 and 170, 3001 263 and 254; 6144 x
+    4096 2048 92 and 84; 22016 x 4096 700 153 and 128, 2600 396 and 386, 3001 433
+    and 454; 28672 x 4096 2600 506 and 499, 3001 561 and 564; 4096 x 4096 512 32
+    and 36, 2048 68 and 60; 4096 x 11008 700 84 and 91, 2048 152 and 147)."""
+    ext, m, n = _backend.ext(), x.shape[0], weight.shape[0]
+    if (m >= 1024 or (m > 128 and n >= 6144)) and m * n <= 60_000_000 and \
+            ext.tile_gemm_takes(x, weight):
+        return ext.tile_lora(x, weight, t, bs, scale)
+    y = wide_product(x, weight)
+    ext.lora_add_(y, t, bs, scale, False)
+    return y
+
+
 def wide_product_grad(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """dy @ weight on the GPU, weight [N, K].
 

@@ -23,7 +23,7 @@ import torch
 from torch import nn
 
 from ..ops import _backend
-from ..ops.linear import wide_product, wide_product_grad
+from ..ops.linear import wide_product_grad, wide_product_lora
 from ..parallel.tp import ColumnParallelLinear, RowParallelLinear
 from ..utils.modules import plain
 
@@ -233,8 +233,7 @@ class _LoRAPacked(torch.autograd.Function):
     def forward(ctx, x, w, scale, n, *ab):
         ext = _backend.ext()
         t = ext.lora_down(x, list(ab[:n]))
-        y = wide_product(x, w)
-        ext.lora_add_(y, t, list(ab[n:]), scale, False)
+        y = wide_product_lora(x, w, t, list(ab[n:]), scale)
         ctx.save_for_backward(x, w, t, *ab)
         ctx.scale, ctx.n = scale, n
         return y

@@ -75,6 +75,23 @@ def test_gated_unit(tile, glu, m, n, k):
     assert bool(((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4).all())
 
 
+@pytest.mark.parametrize("tile", [-1, *TILES])
+@pytest.mark.parametrize("m,widths,k", [
+    (1, [16], 256), (300, [208, 16, 64], 320),  # siblings within a tile
+    (513, [512, 576], 448), (4100, [2048, 1152, 1152], 256)])
+def test_adapters(tile, m, widths, k):
+    from runbooks_amd import ops
+    x, w = _inputs(m, sum(widths), k)
+    t = torch.randn(len(widths), m, 16, device="cuda").bfloat16()
+    bs = [torch.randn(n, 16, device="cuda").bfloat16() for n in widths]
+    got = ops.ext().tile_lora(x, w, t, bs, 0.3, tile=tile)
+    more = torch.cat([ti.float() @ b.float().t() for ti, b in zip(t, bs)], 1)
+    ref = x.float() @ w.float().t() + 0.3 * more
+    # sums of k products of size 1 / sqrt(k) and of 16 of size 1
+    bound = 2.0 ** -8 * ref.abs() + 2.0 ** -24 * (2 * k ** 1.5 + 2 * 16 * 16)
+    assert bool(((got.float() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(700, 22016, 512), (2200, 22016, 1024),
                                    (1800, 28680, 1024)])
 def test_two_launches(m, n, k):

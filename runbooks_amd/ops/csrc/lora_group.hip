@@ -1,7 +1,9 @@
 // Products of LoRA adapters of rank 16 that share their input, for CDNA4
 // (gfx950): n <= 3 siblings side by side (q, k, v; gate, up; or one alone).
 //
-//   y [T, N]  = x [T, K] W^T            (a library product of all siblings)
+//   y [T, N]  = x [T, K] W^T            (a product of all siblings; where it runs
+//                                       in tiles, gemm_tiles.hip, it ends with
+//                                       the next but one)
 //   t_i       = x A_i^T                                  lora_down
 //   y_i      += s t_i B_i^T             (columns of i)   lora_add
 //   dt_i      = s dy_i B_i                               lora_down (columns)

@@ -1,9 +1,10 @@
-"""Linear dispatch: route decode-shaped matmuls to the decode GEMM.
+"""Linear dispatch: which product runs on which kernel.
 
-Decode GEMMs and others of up to 128 rows are weight-bandwidth bound;
-csrc/decode_gemm.hip streams W at HBM rate where hipBLASLt's tiles
-measured 25-45% (profiles/). Everything else (prefill, training) stays
-on hipBLASLt via F.linear — the library is the right tool for big GEMMs.
+Products of up to 128 rows are bound by the weights; csrc/decode_gemm.hip streams
+W at HBM rate where hipBLASLt's tiles measured 25-45% (profiles/). Above that
+prompts and fine-tunes run on csrc/gemm_tiles.hip where there are too few tiles
+for the library's, or where what follows the product can end it, and otherwise on
+hipBLASLt via F.linear.
 """
 from __future__ import annotations
 

@@ -584,8 +584,10 @@ class Transformer(nn.Module):
     def decode(self, tokens, positions, caches, slot_mapping, block_tables,
                seq_lens, nsplit=None, seq_starts=None, state_slots=None):
         """tokens [B] (one new token per sequence) -> logits [B, V].
-        ``nsplit`` fixes the paged-decode work split (required under
-        hipGraph capture, serve/graph.py); ``state_slots`` [B] names the
+        ``nsplit`` is the most parts that decode attention takes a
+        sequence in (required under hipGraph capture, serve/graph.py; fewer
+        where they would not pay, csrc/attention_decode.hip);
+        ``state_slots`` [B] names the
         sequences' state slots (models with recurrent layers)."""
         B = tokens.shape[0]
         if self.ragged:

@@ -199,7 +199,9 @@ def _is_vt(k_cache, v_cache) -> bool:
 
 
 def _auto_nsplit(B, hkv, seq_lens, mfma=False):
-    """Work-split (measured sweeps: profiles/decode_attn_pipeline.md).
+    """The most parts of a sequence (measured sweeps:
+    profiles/decode_attn_pipeline.md); the kernels' launch takes fewer where
+    they would not pay (paged_decode_parts).
     The MFMA path is block-granular and latency-light: ~512 WGs is the
     knee. The scalar kernels want ~1024 (4 WGs/CU). Chunks should still
     cover >= ~64 tokens each."""

@@ -26,6 +26,9 @@
 
 #include "common.h"
 
+int64_t paged_decode_parts(int64_t nsplit, int64_t longest, int64_t dh,
+                           int64_t group, bool fp8, bool transposed);
+
 namespace {
 
 constexpr int BLOCK = 256;    // 4 waves
@@ -187,11 +190,7 @@ __global__ __launch_bounds__(WAVES * 64) void paged_decode_kernel(
   constexpr int BT_LDS = 512;
   __shared__ int32_t bt_lds[BT_LDS];
   const int blk0 = t_begin / bs;
-  if (!SPLIT && seq_starts == nullptr) {
-    // without waiting for the length
-    for (int i = (int)threadIdx.x; i < min(max_blocks, BT_LDS); i += WAVES * 64)
-      bt_lds[i] = bt[i];
-  } else if (t_begin < t_end) {
+  if (t_begin < t_end) {
     const int nbt = min((t_end - 1) / bs - blk0 + 1, BT_LDS);
     for (int i = (int)threadIdx.x; i < nbt; i += WAVES * 64)
       bt_lds[i] = bt[blk0 + i];
@@ -782,23 +781,9 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
   }
 }
 
-// Whether a workgroup of 8 or 16 waves takes a whole sequence of a kv head, rather
-// than several of 4 waves parts of it: where that is a workgroup for every CU, or
-// tables (the only bound on lengths that is known here) so short that a CU's share
-// of them costs less than the sum of the parts in a launch of its own. More waves
-// also shorten the time that a batch's longest sequences run after the others.
-//
-// us in parts, by 4 waves, and here: 32 heads of 128, sequences of 129 to 2015
-// tokens, 32 of them 114.5 and 107.5 (unsplit before, too), 8 34.4 and 33.1; 64 of
-// 100 to 1000 116 and 103; 4 of 200 9.7 and 7.4, of 1000 19.6 and 17.9; one of 200
-// 8.4 and 6.3, of 500 9.6 and 9.4, of 1000 11.1 and 13.8; 12 heads of 64, 64
-// sequences of 37 to 1400 47.8 and 36 to 39; 16 heads of 256, 32 sequences 101 and
-// 99 (8 waves; 107 with 16), 4 of 500 14.6 and 14.4; e4m3, 16 sequences of 800 to
-// 3900 75.8 and 73.3 (78.8 with 16 waves).
-template <int DH> bool whole_sequences(int64_t B, int64_t hkv, int64_t longest) {
-  const int64_t base = B * hkv;
-  return base >= 256 ||
-         longest <= (DH > 128 ? 4 : 8) * std::max<int64_t>(32, base);
+// Waves of a workgroup that has a whole sequence of a kv head to itself.
+constexpr int whole_waves(int64_t dh, bool fp8) {
+  return fp8 || dh > 128 ? 8 : 16;
 }
 
 template <int DH, int G, bool FP8>
@@ -817,9 +802,6 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
   const int max_blocks = (int)block_tables.size(1);
   uint16_t *swz = out_swz.has_value() ? (uint16_t *)out_swz->data_ptr()
                                       : nullptr;
-  // parts of fewer tokens cost more than they save (one sequence of 37 tokens, 32
-  // heads of 128: 16 parts 8.2 us, one 4.1; matrix instructions, 32 query heads,
-  // one of 500: 16 parts 7.5, 10 7.9)
   const int64_t longest = (int64_t)max_blocks * bs;
   // MFMA route: keyed on the TRANSPOSED V layout (bf16 [Dh, BS] /
   // fp8 [Dh+4, BS] blocks) the allocator chooses for MFMA-eligible
@@ -829,8 +811,7 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
   // versa.
   const bool vt = v_cache.size(3) == bs &&
       v_cache.size(2) == (int64_t)(FP8 ? DH + 4 : DH);
-  nsplit = (int)std::min<int64_t>(nsplit,
-                                  (longest + 63) / (vt ? 32 : 64));
+  nsplit = (int)paged_decode_parts(nsplit, longest, DH, G, FP8, vt);
   if constexpr (G >= 4 && DH <= 128) {
     if (vt && bs == 16) {
       if (nsplit <= 1) {
@@ -880,8 +861,8 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                        splits, scale);
   };
   if constexpr (G < NW) {
-    constexpr int MORE = FP8 || DH > 128 ? 8 : 16;
-    if (longest > 64 && whole_sequences<DH>(B, hkv, longest))
+    constexpr int MORE = whole_waves(DH, FP8);
+    if (nsplit <= 1 && longest > 64)
       return go(paged_decode_kernel<DH, G, false, FP8, MORE>, MORE, 1, nullptr);
   }
   if (nsplit <= 1)
@@ -897,6 +878,35 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
 }
 
 }  // namespace
+
+// Parts that a sequence of a kv head is taken in, of the nsplit that there are
+// workgroups of 4 waves for; `longest` is what a block table has room for, the only
+// bound on the lengths that is known here.
+//
+// Parts of fewer than 64 tokens cost more than they save (one sequence of 37
+// tokens, 32 heads of 128: 16 parts 8.2 us, one 4.1; matrix instructions take 32:
+// 32 query heads, one of 500, 16 parts 7.5, 10 7.9). One workgroup of 8 or 16 waves
+// takes all of a sequence where it has at least twice the waves of all parts, or
+// the table is short: then it is as fast for the longest sequence of an uneven
+// batch, too, and the launch that adds up the parts goes.
+//
+// us in parts and whole, 32 heads of 128 in bf16: one sequence of 200 tokens 9.1
+// and 7.1, of 512 9.8 and 9.5, of 1024 12.0 and 16.2; 4 of 512 13.8 and 12.2, one of
+// 512 and 3 of 50 10.1 and 10.5, one of 1024 and 3 of 50 12.7 and 16.6; 16 (two
+// parts) of 800 to 3900 122 and 123, 4000 and 15 of 100 63.7 and 54.3; 8 (four) of
+// 129 to 2015 34.5 and 34.4, of 2000 54.4 and 49.6, 5 of 2000 and 3 that pad the batch
+// 38.2 and 33.4, 4000 and 7 of 100 35.8 and 47.3. e4m3: 16 (two) of 800 to 3900 74.5
+// and 75.4, 4000 and 15 of 100 36.1 and 39.3; 8 (four), 4000 and 7 of 100 22.6 and
+// 37.5. 16 heads of 256: 4 of 256 12.9 and 10.7, one of 256 and 7 of 50 11.0 and 9.9,
+// one of 512 and 7 of 50 12.2 and 15.2; 16 (four), 4000 and 15 of 100 44 and 80.
+int64_t paged_decode_parts(int64_t nsplit, int64_t longest, int64_t dh,
+                           int64_t group, bool fp8, bool transposed) {
+  const int64_t parts =
+      std::min(nsplit, (longest + 63) / (transposed ? 32 : 64));
+  const bool whole = group < NW && (longest <= (dh > 128 ? 256 : 512) ||
+                                    parts * 2 * NW <= whole_waves(dh, fp8));
+  return whole ? 1 : std::max<int64_t>(parts, 1);
+}
 
 std::vector<at::Tensor> paged_decode_swz(at::Tensor q, at::Tensor k_cache,
                                          at::Tensor v_cache,

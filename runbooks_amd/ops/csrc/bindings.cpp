@@ -21,6 +21,8 @@ at::Tensor paged_decode(at::Tensor q, at::Tensor k_cache, at::Tensor v_cache,
                         at::Tensor block_tables, at::Tensor seq_lens,
                         int64_t nsplit, double scale,
                         c10::optional<at::Tensor> seq_starts);
+int64_t paged_decode_parts(int64_t nsplit, int64_t longest, int64_t dh,
+                           int64_t group, bool fp8, bool transposed);
 std::vector<at::Tensor> paged_decode_swz(at::Tensor q, at::Tensor k_cache,
                                          at::Tensor v_cache,
                                          at::Tensor block_tables,
@@ -94,6 +96,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
         py::arg("block_tables"), py::arg("seq_lens"), py::arg("nsplit"),
         py::arg("scale"), py::arg("seq_starts") = py::none());
+  m.def("paged_decode_parts", &paged_decode_parts,
+        "parts that a sequence is taken in", py::arg("nsplit"),
+        py::arg("longest"), py::arg("dh"), py::arg("group"), py::arg("fp8"),
+        py::arg("transposed"));
   m.def("paged_decode_swz", &paged_decode_swz,
         "paged decode also emitting the o_proj decode-GEMM operand",
         py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),

@@ -21,8 +21,10 @@ RING = 8        # staging buffers
 
 
 def fixed_nsplit(batch: int, hkv: int, mfma: bool = False) -> int:
-    """Work-split for the paged-decode kernel, chosen per bucket at capture
-    time (the eager heuristic in ops/attention.py reads seq_lens.max() —
+    """The most parts of a sequence for the paged-decode kernel, chosen per
+    bucket at capture time (paged_decode_parts in csrc/attention_decode.hip
+    takes fewer where they would not pay: short tables, or two parts of few
+    query heads; the eager heuristic in ops/attention.py reads seq_lens.max() —
     a host sync, impossible inside a graph). base = batch*hkv workgroups
     per split; split until ~4x256 CUs are covered — the head-split GQA
     kernels run 4-5 waves/SIMD, so ~4 WGs/CU (1024 WGs) fills the

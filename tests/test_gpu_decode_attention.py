@@ -20,7 +20,8 @@ def _rel(a, b):
     (3, 12, 12, 64, 16, 16), (22, 12, 12, 64, 40, 3), (2, 8, 4, 64, 16, 16),
     (4, 32, 32, 128, 30, 8), (16, 32, 16, 128, 40, 2), (8, 32, 32, 128, 130, 4),
     (4, 16, 16, 256, 15, 16), (16, 16, 16, 256, 40, 4), (2, 4, 4, 128, 4, 16),
-    (1, 4, 4, 128, 129, 16)])
+    (1, 4, 4, 128, 129, 16), (3, 12, 12, 64, 40, 1), (5, 32, 32, 128, 33, 2),
+    (2, 8, 4, 128, 40, 1), (3, 4, 4, 256, 17, 1), (2, 4, 4, 256, 16, 8)])
 def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
     """By 4, 8 or 16 waves or in parts, with and without a window's start, and
     with sequences as short and as long as the table: the plain result but for
@@ -53,3 +54,34 @@ def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
             operand = ops.ext().decode_swizzle_x(got[0].view(batch, -1))
             assert torch.equal(got[1].view(-1, 32, 8)[:, :batch],
                                operand.view(-1, 32, 8)[:, :batch])
+
+
+def test_uneven_captured_bucket():
+    """One long sequence among short ones and rows that pad the batch, by the
+    split of a captured step: each the plain result."""
+    from runbooks_amd.serve.graph import fixed_nsplit
+    torch.manual_seed(0)
+    lens = torch.tensor([4000, 100, 17, 100, 1, 1, 1, 1])
+    heads, dh, blocks = 32, 128, 257
+    nsplit = fixed_nsplit(len(lens), heads)
+    assert ops.ext().paged_decode_parts(nsplit, blocks * 16, dh, 1, False,
+                                        False) == nsplit
+    used = (lens + 15) // 16
+    kc, vc = ops.alloc_kv_cache(int(used.sum()) + 1, heads, dh, DEV,
+                                dtype=torch.bfloat16)
+    kc.normal_()
+    vc.normal_()
+    i32 = dict(dtype=torch.int32, device=DEV)
+    tables = torch.full((len(lens), blocks), int(used.sum()), **i32)
+    at = 0
+    for row, n in zip(tables, used.tolist()):
+        row[:n] = torch.arange(at, at + n, **i32)
+        at += n
+    q = torch.randn(len(lens), heads, dh, device=DEV).bfloat16()
+    starts = torch.zeros(len(lens), **i32)
+    got = ops.ext().paged_decode_swz(q, kc, vc, tables, lens.to(**i32), nsplit,
+                                     dh ** -0.5, starts)[0]
+    ref = ops.paged_decode_ref(q.cpu(), kc.cpu(), vc.cpu(), tables.cpu(), lens,
+                               dh ** -0.5)
+    for i in range(len(lens)):
+        assert _rel(got[i].cpu(), ref[i].double()) < 2 * BF16

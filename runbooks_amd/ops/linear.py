@@ -319,6 +319,19 @@ def wide_product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return y
 
 
+def _wide_in_tiles(m: int, n: int, k: int) -> bool:
+    """Whether wide weights' product of few rows runs in own tiles: one row of
+    tiles of 256, or a second one that is nearly as good (us in the library and
+    in tiles: 12288 x 4096 129 rows 38 and 36, 256 48 and 43, 320 51 and 47;
+    12288 x 3072 192 33 and 32, 320 42 and 40; 15360 x 5120 256 64 and 59, 320 60
+    and 64; 18432 x 3072 256 51 and 45; 12288 x 1024 256 17 and 16, 320 17 and 18).
+    Wider ones the library takes in whole rounds (24576 x 4096 192 58 and 60,
+    320 72 and 79; 32768 x 1024 320 26 and 31; 24576 x 8192 129 100 and 119), of
+    narrower ones there are too few tiles (6144 x 4096 200 25 and 34)."""
+    return 12288 <= n < 20480 and \
+        (m <= 256 or (m <= 320 and n < 15360 and 2048 <= k < 8192))
+
+
 def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """fast_linear for a result that is not differentiated, of rows x that are
     there also where they have a decode operand; of many rows a wide_product.
@@ -329,9 +342,7 @@ def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     6144 x 4096 15.9 and 15.4, of 24 rows 47.9 and 52.6, 14.7 and 15.0)."""
     if x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2:
         (m, k), n = x.shape, weight.shape[0]
-        if m <= 320 and n >= 12288 and _tiles_serve(x, weight):
-            # us in the library and in tiles, 12288 x 4096: 129 rows 39 and 35,
-            # 300 52 and 46, 384 51 and 53; 6144 x 4096 200 25 and 34
+        if _wide_in_tiles(m, n, k) and _tiles_serve(x, weight):
             return _backend.ext().tile_gemm(x, weight)
         if m > 1280:
             return wide_product(x, weight)

@@ -1,0 +1,17 @@
+"""Which products of prompts and fine-tunes run in own tiles (ops/linear.py): the
+sizes that were measured to be faster there, and those that were not."""
+import pytest
+
+from runbooks_amd.ops import linear
+
+
+@pytest.mark.parametrize("m,n,k,tiles", [
+    (129, 12288, 4096, True), (256, 12288, 3072, True),
+    (320, 12288, 4096, True), (256, 15360, 5120, True),
+    (192, 18432, 2048, True),
+    (320, 12288, 1024, False), (320, 15360, 5120, False),
+    (320, 24576, 1024, False), (129, 24576, 8192, False),
+    (257, 32768, 4096, False), (321, 12288, 4096, False),
+    (200, 6144, 4096, False)])
+def test_wide_products(m, n, k, tiles):
+    assert linear._wide_in_tiles(m, n, k) is tiles

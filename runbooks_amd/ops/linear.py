@@ -259,15 +259,22 @@ def rows_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
     and 65, 1021 141 and 109, 2048 220 and 206; 3072 x 24576 512 151 and 90,
     1021 209 and 136, 2048 328 and 252; 8192 x 8192 512 87 and 74). Otherwise
     the library is as fast or faster (4096 x 4096 768 39 and 45, 8192 x 8192
-    1280 147 and 157)."""
+    1280 147 and 157), as it is with short sums, where begin and end of a tile
+    count for more (2048 x 2048 129 13 and 15, 400 16 and 19; 1024 x 2816 129 12
+    and 15, 1021 19 and 21; but 3584 x 3584 300 29 and 23, 2048 x 5632 400 29 and 24).
+    """
     if _tiles_serve(x, weight):
         (m, k), n = x.shape, weight.shape[0]
-        if _backend.ext().tile_gemm_parts(m, n, k) > 1:
+        if _sums_in_parts(m, n, k):
             return _backend.ext().tile_gemm(x, weight, max_parts=4)
         return _one_round(x, weight)
     dw = _rows_served(x, weight)
     return None if dw is None else _backend.ext().decode_gemm_rows(
         x, dw[0], weight.shape[0], dw[2], True)
+
+
+def _sums_in_parts(m: int, n: int, k: int) -> bool:
+    return k >= 3072 and _backend.ext().tile_gemm_parts(m, n, k) > 1
 
 
 def _one_round(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:

@@ -15,3 +15,14 @@ from runbooks_amd.ops import linear
     (200, 6144, 4096, False)])
 def test_wide_products(m, n, k, tiles):
     assert linear._wide_in_tiles(m, n, k) is tiles
+
+
+@pytest.mark.parametrize("m,n,k,parts", [
+    (129, 4096, 4096, True), (512, 4096, 11008, True),
+    (300, 3584, 3584, True), (400, 2048, 5632, True),
+    (129, 2048, 2048, False), (400, 2048, 2048, False),
+    (1021, 1024, 1024, False), (129, 1024, 2816, False),
+    (768, 4096, 4096, False), (4096, 4096, 14336, False)])
+def test_sums_in_parts(m, n, k, parts):
+    pytest.importorskip("runbooks_amd.ops._hip_core")
+    assert linear._sums_in_parts(m, n, k) is parts

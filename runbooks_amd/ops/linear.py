@@ -361,18 +361,40 @@ def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return fast_linear(x, weight)
 
 
+def _lora_in_tiles(m: int, n: int, k: int) -> bool:
+    """Whether a product that adapters' parts are added to runs in tiles that end
+    with them, or in the library with a pass over its result.
+
+    Rows of up to 5120: where the result is wide or has more than 32 tiles of 256 x
+    256 (us in the library with the pass and in tiles: 12288 x 4096 129 rows 44 and
+    38, 2048 174 and 163, 3001 258 and 242; 6144 x 4096 129 44 and 34, 3001 143 and
+    135; 22016 x 4096 700 149 and 127, 2600 394 and 391; 28672 x 4096 2048 388 and
+    393; 27648 x 5120 1536 393 and 346; 4096 x 4096 900 42 and 36, 512 34 and 39;
+    2048 x 2048 1800 25 and 20), up to where the library has whole rounds of its
+    larger tiles (22016 x 4096 3001 436 and 478, 4096 588 and 614).
+
+    Longer rows: where one round of tiles does (4096 x 11008 1800 158 and 139, 2048
+    164 and 146, 3001 209 and 201; 4096 x 14336 2048 205 and 185; 5120 x 13824 1536
+    190 and 175; 8192 x 8192 1024 123 and 111). With fewer tiles CUs are idle for
+    long (4096 x 14336 512 94 and 136, 1280 152 and 166, 2048 x 5632 1024 42 and 57),
+    with more the library is as fast (4096 x 14336 4096 320 and 333, 8192 x 28672
+    700 288 and 348)."""
+    def tiles(rows, cols):
+        return -(-m // rows) * -(-n // cols)
+    if m <= 128 or n < 2048 or m * n > 60_000_000:
+        return False
+    if k <= 5120:
+        return n >= 6144 or tiles(256, 256) > 32
+    return k <= 16384 and n >= 4096 and \
+        any(224 <= t <= 256 for t in (tiles(256, 128), tiles(192, 256)))
+
+
 def wide_product_lora(x: torch.Tensor, weight: torch.Tensor, t: torch.Tensor,
                       bs: list, scale: float) -> torch.Tensor:
     """wide_product(x, weight) + scale t_i B_i^T of adapters side by side
-    (csrc/lora_group.hip), in tiles that end with the adapters' part, or in the
-    library and a pass over its result (us there and in tiles: 12288 x 4096 129
-    rows 42 and 36, 512 60 and 56, 2048 174 and 170, 3001 263 and 254; 6144 x
-    4096 2048 92 and 84; 22016 x 4096 700 153 and 128, 2600 396 and 386, 3001 433
-    and 454; 28672 x 4096 2600 506 and 499, 3001 561 and 564; 4096 x 4096 512 32
-    and 36, 2048 68 and 60; 4096 x 11008 700 84 and 91, 2048 152 and 147)."""
-    ext, m, n = _backend.ext(), x.shape[0], weight.shape[0]
-    if (m >= 1024 or (m > 128 and n >= 6144)) and m * n <= 60_000_000 and \
-            ext.tile_gemm_takes(x, weight):
+    (csrc/lora_group.hip)."""
+    ext, (n, k) = _backend.ext(), weight.shape
+    if _lora_in_tiles(x.shape[0], n, k) and ext.tile_gemm_takes(x, weight):
         return ext.tile_lora(x, weight, t, bs, scale)
     y = wide_product(x, weight)
     ext.lora_add_(y, t, bs, scale, False)

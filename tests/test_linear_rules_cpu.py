@@ -26,3 +26,17 @@ def test_wide_products(m, n, k, tiles):
 def test_sums_in_parts(m, n, k, parts):
     pytest.importorskip("runbooks_amd.ops._hip_core")
     assert linear._sums_in_parts(m, n, k) is parts
+
+
+@pytest.mark.parametrize("m,n,k,tiles", [
+    (129, 12288, 4096, True), (2048, 22016, 4096, True),
+    (256, 6144, 4096, True), (2048, 4096, 4096, True),
+    (1800, 2048, 2048, True), (2048, 4096, 11008, True),
+    (3001, 4096, 14336, True), (1024, 8192, 8192, True),
+    (3001, 28672, 4096, False), (512, 4096, 4096, False),
+    (1024, 2048, 5632, False), (1280, 4096, 11008, False),
+    (1536, 4096, 14336, False), (1800, 768, 3072, False),
+    (700, 8192, 28672, False), (2048, 8192, 8192, False),
+    (128, 22016, 4096, False)])
+def test_products_with_adapters(m, n, k, tiles):
+    assert linear._lora_in_tiles(m, n, k) is tiles

@@ -74,15 +74,16 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.T
 
 def rmsnorm_res(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor,
                 eps: float) -> tuple[torch.Tensor, torch.Tensor]:
-    """x + delta and its norm, differentiable. delta may come as fp32 parts
-    [P, T, D] of it (ops.rows_parts); their sum is not differentiated."""
-    if delta.dim() == 3 and x.dim() == 2:
-        x, y = _backend.ext().rmsnorm_res_slab_fwd(
-            x.contiguous(), delta, weight.contiguous(), eps)
-        return x, y
+    """x + delta and its norm, differentiable. On the GPU, where nothing is
+    differentiated, delta may come as fp32 parts [P, T, D] of it
+    (ops.rows_parts)."""
     if not _backend.use_hip(x):
         x = x + delta
         return x, rmsnorm_ref(x, weight, eps)
+    if delta.dim() == 3 and x.dim() == 2 and not torch.is_grad_enabled():
+        x, y = _backend.ext().rmsnorm_res_slab_fwd(
+            x.contiguous(), delta, weight.contiguous(), eps)
+        return x, y
     if (not torch.is_grad_enabled() and x.dtype == torch.bfloat16
             and x.numel() // x.shape[-1] <= 32 and x.shape[-1] % 16 == 0):
         x, y, swz = _backend.ext().rmsnorm_res_fwd_dec(

@@ -134,3 +134,17 @@ def test_one_row_does_not_reach_others():
     keep = [i for i in range(300) if i not in (7, 299)]
     assert torch.equal(got[keep], clean[keep])
     assert bool(got[299].isnan().all()) and not bool(got[7].isfinite().any())
+
+
+def test_parts_are_not_differentiated():
+    """A norm's sum of parts is refused where its gradient would be lost."""
+    from runbooks_amd import ops
+    x = torch.randn(200, 64, device="cuda").bfloat16()
+    parts = torch.randn(2, 200, 64, device="cuda")
+    w = torch.ones(64, device="cuda").bfloat16()
+    with pytest.raises(RuntimeError):
+        ops.rmsnorm_res(x, parts, w, 1e-5)
+    with torch.no_grad():
+        s, _ = ops.rmsnorm_res(x, parts, w, 1e-5)
+    ref = x.float() + parts.sum(0)
+    assert bool(((s.float() - ref).abs() <= 2.0 ** -8 * ref.abs()).all())

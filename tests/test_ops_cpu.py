@@ -328,3 +328,16 @@ def test_parts_of_a_sequence():
     assert parts(16, 512, group=4, vt=True) == 16
     assert parts(16, 64, group=8, vt=True) == 3
     assert parts(0, 4112) == 1 and parts(4, 0, group=4) == 1
+
+
+def test_residual_norm_of_a_batch_of_terms():
+    """x + delta broadcasts on the CPU, also where delta has the dimensions
+    that parts of a sum have on the GPU, and is differentiated."""
+    x = torch.randn(3, 8, requires_grad=True)
+    delta = torch.randn(2, 3, 8, requires_grad=True)
+    w = torch.rand(8)
+    s, y = ops.rmsnorm_res(x, delta, w, 1e-5)
+    assert torch.equal(s, x + delta)
+    assert torch.equal(y, ops.rmsnorm_ref(x + delta, w, 1e-5))
+    y.sum().backward()
+    assert x.grad is not None and delta.grad.shape == delta.shape

@@ -147,4 +147,5 @@ def test_parts_are_not_differentiated():
     with torch.no_grad():
         s, _ = ops.rmsnorm_res(x, parts, w, 1e-5)
     ref = x.float() + parts.sum(0)
-    assert bool(((s.float() - ref).abs() <= 2.0 ** -8 * ref.abs()).all())
+    # one rounding, and the order of three fp32 terms of up to 5
+    assert bool(((s.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2e-6).all())

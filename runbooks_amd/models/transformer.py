@@ -319,9 +319,13 @@ class Block(nn.Module):
     def adds_parts(self) -> bool:
         """fuses_residual(), and what its sublayers return goes there straight
         from their last product, so that it may come as parts of its sums."""
-        return (self.attn.tp == 1 and not torch.is_grad_enabled() and
+        attn = self.attn
+        return (type(attn) is Attention and attn.tp == 1 and
+                "forward_prefill" not in attn.__dict__ and
+                "forward_decode" not in attn.__dict__ and
+                not torch.is_grad_enabled() and
                 self.fuses_residual() and plain(MLP, self.mlp) and
-                plain(RowParallelLinear, self.attn.o_proj, self.mlp.down_proj))
+                plain(RowParallelLinear, attn.o_proj, self.mlp.down_proj))
 
     def forward_pending(self, x, delta, attn_fn, parts=False):
         """forward() of a residual whose last term is still to be added:
@@ -571,9 +575,10 @@ class Transformer(nn.Module):
 
         def attention(blk):
             kc, vc = cache_of[blk]
+            kw = {"parts": True} if blk.adds_parts() else {}
             return lambda h: blk.attn.forward_prefill(
                 h, self.rope_cos, self.rope_sin, positions, kc, vc,
-                slot_mapping, B, S, parts=blk.adds_parts())
+                slot_mapping, B, S, **kw)
 
         x = self._last_norm(*(None if r is None else r.view(B, S, -1)[:, -1]
                               for r in self._blocks(x, attention)))
@@ -647,10 +652,11 @@ class Transformer(nn.Module):
 
         def attention(blk):
             kc, vc = cache_of[blk]
+            kw = {"parts": True} if blk.adds_parts() else {}
             return lambda h: blk.attn.forward_decode(
                 h, self.rope_cos, self.rope_sin, positions, kc, vc,
                 slot_mapping, block_tables, seq_lens, nsplit=nsplit,
-                seq_starts=seq_starts, parts=blk.adds_parts())
+                seq_starts=seq_starts, **kw)
 
         x = self._last_norm(*self._blocks(x, attention))
         logits = self.lm_head(x)

@@ -812,3 +812,38 @@ def test_weights_as_decode_reads_them(lies):
         at = 1 if flat.data_ptr() % 16 == 0 else 0
         w.data = flat[at:at + w.numel()].view(w.shape).copy_(w.data)
     assert _AffineBlock.serves(m, blk) == (lies == "as made")
+
+
+@pytest.mark.parametrize("own", ["class", "object"])
+def test_attention_of_ones_own_is_called_as_ever(own):
+    """An attention with prefill and decode of its own, by its class or on the
+    object, is called with the arguments of before sums in parts."""
+    from runbooks_amd.models.transformer import Attention
+    calls = []
+
+    def prefill(self, x, cos, sin, positions, kc, vc, slot_mapping, B, S):
+        calls.append("prefill")
+        return Attention.forward_prefill(self, x, cos, sin, positions, kc, vc,
+                                         slot_mapping, B, S)
+
+    def decode(self, x, cos, sin, positions, kc, vc, slot_mapping,
+               block_tables, seq_lens, nsplit=None, slab_ok=False,
+               seq_starts=None):
+        calls.append("decode")
+        return Attention.forward_decode(self, x, cos, sin, positions, kc, vc,
+                                        slot_mapping, block_tables, seq_lens,
+                                        nsplit, slab_ok, seq_starts)
+
+    m = build_model("tiny-llama", dtype=torch.float32)
+    ref = Engine(m, device="cpu", dtype=torch.float32).generate(
+        [1, 2, 3], max_new_tokens=3)
+    attn = m.blocks[1].attn
+    if own == "class":
+        attn.__class__ = type("Own", (Attention,), {
+            "forward_prefill": prefill, "forward_decode": decode})
+    else:
+        attn.forward_prefill = prefill.__get__(attn)
+        attn.forward_decode = decode.__get__(attn)
+    got = Engine(m, device="cpu", dtype=torch.float32).generate(
+        [1, 2, 3], max_new_tokens=3)
+    assert got == ref and calls == ["prefill", "decode", "decode"]

@@ -17,7 +17,7 @@ import torch
 
 from .. import ops
 from ..parallel import ColumnParallelLinear, RowParallelLinear
-from ..utils.modules import plain
+from ..utils.modules import plain, untouched
 
 
 class _Layer:
@@ -49,6 +49,8 @@ def layers_of(model, block_type, attention_type, mlp_type):
     mlps, attns = [b.mlp for b in blocks], [b.attn for b in blocks]
     if not (blocks and plain(block_type, *blocks) and plain(mlp_type, *mlps) and
             plain(attention_type, *attns) and
+            untouched(("forward_decode", "forward_decode_fused"), *attns,
+                      *blocks) and
             plain(ops.RMSNorm, *(n for b in blocks
                                  for n in (b.norm1, b.norm2))) and
             plain(RowParallelLinear, *(m.down_proj for m in mlps),

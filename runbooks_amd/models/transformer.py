@@ -40,7 +40,7 @@ from ..parallel import (
     comm,
     gather_from_tp,
 )
-from ..utils.modules import plain
+from ..utils.modules import plain, untouched
 from . import decode_chain
 from .config import LatentAttentionSpec, ModelConfig
 from .dual import DualBlock
@@ -321,8 +321,7 @@ class Block(nn.Module):
         from their last product, so that it may come as parts of its sums."""
         attn = self.attn
         return (type(attn) is Attention and attn.tp == 1 and
-                "forward_prefill" not in attn.__dict__ and
-                "forward_decode" not in attn.__dict__ and
+                untouched(("forward_prefill", "forward_decode"), attn) and
                 not torch.is_grad_enabled() and
                 self.fuses_residual() and plain(MLP, self.mlp) and
                 plain(RowParallelLinear, attn.o_proj, self.mlp.down_proj))

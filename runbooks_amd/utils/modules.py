@@ -20,3 +20,9 @@ def plain(cls: type, *modules) -> bool:
                 d["_backward_hooks"] or d["_backward_pre_hooks"]):
             return False
     return True
+
+
+def untouched(names, *modules) -> bool:
+    """True where no object of `modules` has methods of its own of these
+    names: those that are called in place of forward()."""
+    return not any(name in m.__dict__ for m in modules for name in names)

@@ -260,6 +260,29 @@ def test_hooked_modules_are_called():
     assert _rel(got, want.double()) < 2e-2
 
 
+@pytest.mark.parametrize("which", ["attention", "block"])
+def test_methods_of_an_object_are_called(which):
+    """Decoding goes by the step of an attention or a block that has one of its
+    own."""
+    m = _model(8, 2048)
+    args = _step(m, 3, False)
+    seen = []
+    blk = m.blocks[1]
+    owner, name = (blk.attn, "forward_decode") if which == "attention" else \
+        (blk, "forward_decode_fused")
+    plain = getattr(owner, name)
+
+    def step(*a, **kw):
+        seen.append(1)
+        return plain(*a, **kw)
+    with torch.no_grad():
+        want = m.decode(*args)
+        setattr(owner, name, step)
+        got = m.decode(*args)
+    assert len(seen) == 1
+    assert _rel(got, want.double()) < 2e-2
+
+
 @pytest.mark.parametrize("batch", [33, 64, 65, 128])
 @pytest.mark.parametrize("kv,inter", [(8, 2048), (2, 1040), (2, 12288)])
 def test_wide_decode_step(monkeypatch, batch, kv, inter):

@@ -317,13 +317,13 @@ class Block(nn.Module):
                 plain(ops.RMSNorm, self.norm1, self.norm2))
 
     def adds_parts(self) -> bool:
-        """fuses_residual(), and what its sublayers return goes there straight
+        """Where fuses_residual(): what its sublayers return goes there straight
         from their last product, so that it may come as parts of its sums."""
         attn = self.attn
         return (type(attn) is Attention and attn.tp == 1 and
-                untouched(("forward_prefill", "forward_decode"), attn) and
-                not torch.is_grad_enabled() and
-                self.fuses_residual() and plain(MLP, self.mlp) and
+                untouched(("forward_prefill", "forward_decode",
+                           "forward_pending"), attn, self) and
+                plain(MLP, self.mlp) and
                 plain(RowParallelLinear, attn.o_proj, self.mlp.down_proj))
 
     def forward_pending(self, x, delta, attn_fn, parts=False):
@@ -490,7 +490,7 @@ class Transformer(nn.Module):
                     blk, *args, use_reentrant=False)
             return blk(*args)
 
-        def attention(blk):
+        def attention(blk, parts):
             return lambda h: blk.attn.forward_train(
                 h, self.rope_cos, self.rope_sin, positions, B, S)
 
@@ -501,29 +501,35 @@ class Transformer(nn.Module):
         return logits.view(B, S, -1)
 
     def _blocks(self, x, attention, run=lambda blk, *args: blk(*args)):
-        """All blocks; attention(block) is its attn_fn. Returns the residual
-        and what is still to be added to it (None: nothing)."""
+        """All blocks; attention(block, parts) is its attn_fn, which with `parts`
+        may return parts of its sums. Returns the residual and what is still to
+        be added to it (None: nothing)."""
         delta = None
         if self._sums_in_layer_norms(x):
             dtype, x = x.dtype, x.float()
             for blk in self.blocks:
                 h = ops.norm_res32(blk.norm1, x, delta, dtype)
-                delta = attention(blk)(h)
+                delta = attention(blk, False)(h)
                 h = ops.norm_res32(blk.norm2, x, delta, dtype)
                 delta = blk.mlp(h)
             return x, delta
         blocks = list(self.blocks)
-        for blk, after in zip(blocks, blocks[1:] + [None]):
-            if blk.fuses_residual():
-                # the norm after the last block may see a part of the rows
-                parts = after is not None and blk.adds_parts() and \
-                    after.fuses_residual()
-                x, delta = run(blk.forward_pending, x, delta, attention(blk),
-                               parts)
+        fuses = [blk.fuses_residual() for blk in blocks]
+        # sums of up to 32 rows come whole: without a look at the modules, which
+        # takes the host 10 us a block (a prompt of 20 tokens of llama2-7b is
+        # bound by the host: 3.5 ms, 0.4 less without)
+        many = x.is_cuda and x.shape[0] > 32 and not torch.is_grad_enabled()
+        # the norm after the last block may see a part of the rows
+        for blk, fused, then in zip(blocks, fuses, fuses[1:] + [False]):
+            if fused:
+                parts = many and blk.adds_parts()
+                x, delta = run(blk.forward_pending, x, delta,
+                               attention(blk, parts),
+                               *((True,) if parts and then else ()))
             else:
                 if delta is not None:
                     x, delta = x + delta, None
-                x = run(blk, x, attention(blk))
+                x = run(blk, x, attention(blk, False))
         return x, delta
 
     def _sums_in_layer_norms(self, x) -> bool:
@@ -572,9 +578,9 @@ class Transformer(nn.Module):
         x = self._embed(tokens, positions)
         cache_of = dict(zip(self.blocks, caches))
 
-        def attention(blk):
+        def attention(blk, parts):
             kc, vc = cache_of[blk]
-            kw = {"parts": True} if blk.adds_parts() else {}
+            kw = {"parts": True} if parts else {}
             return lambda h: blk.attn.forward_prefill(
                 h, self.rope_cos, self.rope_sin, positions, kc, vc,
                 slot_mapping, B, S, **kw)
@@ -649,9 +655,9 @@ class Transformer(nn.Module):
                     else logits)
         cache_of = dict(zip(self.blocks, caches))
 
-        def attention(blk):
+        def attention(blk, parts):
             kc, vc = cache_of[blk]
-            kw = {"parts": True} if blk.adds_parts() else {}
+            kw = {"parts": True} if parts else {}
             return lambda h: blk.attn.forward_decode(
                 h, self.rope_cos, self.rope_sin, positions, kc, vc,
                 slot_mapping, block_tables, seq_lens, nsplit=nsplit,

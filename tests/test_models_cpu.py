@@ -847,3 +847,23 @@ def test_attention_of_ones_own_is_called_as_ever(own):
     got = Engine(m, device="cpu", dtype=torch.float32).generate(
         [1, 2, 3], max_new_tokens=3)
     assert got == ref and calls == ["prefill", "decode", "decode"]
+
+
+def test_few_rows_cost_no_look_at_modules(monkeypatch):
+    """Whether sums may come in parts is asked of blocks only for rows of which
+    they do, and a block's own forward_pending is called as ever."""
+    from runbooks_amd.models.transformer import Block
+
+    def asked(self):
+        raise AssertionError("asked")
+    monkeypatch.setattr(Block, "adds_parts", asked)
+    m = build_model("tiny-llama", dtype=torch.float32)
+    calls = []
+
+    def pending(self, x, delta, attn_fn):
+        calls.append(1)
+        return Block.forward_pending(self, x, delta, attn_fn)
+    m.blocks[0].forward_pending = pending.__get__(m.blocks[0])
+    eng = Engine(m, device="cpu", dtype=torch.float32)
+    assert len(eng.generate([1, 2, 3], max_new_tokens=3)) == 3
+    assert len(calls) == 3

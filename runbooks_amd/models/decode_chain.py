@@ -80,12 +80,6 @@ class _Normed:
         self.squares, self.eps = squares, eps
 
 
-def _shares_x(copy, m: int) -> bool:
-    """From 17 rows the kernel that shares x between workgroups' waves wins
-    where it has about one workgroup for every CU (ops.wide_linear)."""
-    return 16 < m <= 32 and not copy.fp8 and 10240 <= copy.n <= 32768
-
-
 def _heads(layer, y, m, cos, sin, positions, kc, vc, slots):
     ext, c, hq = ops.ext(), layer.qkv, layer.attn.hq
     if kc.dtype != torch.bfloat16:          # rows of it share a scale
@@ -96,7 +90,7 @@ def _heads(layer, y, m, cos, sin, positions, kc, vc, slots):
             out = ops.wide_linear(y.rows, layer.attn._qkv_w)
         return ext.qkv_rope_append(out, cos, sin, positions.to(torch.int32),
                                    kc, vc, slots.to(torch.int32), hq)
-    if y.squares is None and _shares_x(c, m):
+    if y.squares is None and c.shares_x(m):
         return ext.rows_heads(y.rows, c.ws, c.n, cos, sin, positions, kc, vc,
                               slots, hq)
     return ext.decode_heads(y.swz, c.ws, c.scale, m, c.n, c.k, y.squares, y.eps,
@@ -105,7 +99,7 @@ def _heads(layer, y, m, cos, sin, positions, kc, vc, slots):
 
 def _gated(layer, y, m):
     ext, c = ops.ext(), layer.gate_up
-    if y.rows is not None and _shares_x(c, m):
+    if y.rows is not None and c.shares_x(m):
         return ext.rows_glu(y.rows, c.ws, c.n, layer.gelu, True, y.squares,
                             y.eps)
     return ext.decode_glu(y.swz, c.ws, c.scale, m, c.n, c.k, layer.gelu,
@@ -148,7 +142,7 @@ def run(model, layers, x, positions, caches, slots, tables, seq_lens, nsplit,
         _, o = ops.paged_decode_with_operand(
             q, kc, vc, tables, seq_lens, scale=attn.scale, nsplit=nsplit,
             seq_starts=seq_starts)
-        x, y = _add(x, o, layer.o, blk.norm2, _shares_x(layer.gate_up, m))
+        x, y = _add(x, o, layer.o, blk.norm2, layer.gate_up.shares_x(m))
         h = _gated(layer, y, m)
         if i + 1 < len(layers):
             x, y = _add(x, h, layer.down, layers[i + 1].blk.norm1, False)

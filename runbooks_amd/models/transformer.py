@@ -223,7 +223,14 @@ class MLP(nn.Module):
     def forward(self, x, slab_ok=False, parts=False):
         if self.act in ("silu_glu", "gelu_glu") and \
                 getattr(self, "_gateup_w", None) is not None:
-            h = ops.rows_glu(x, self._gateup_w, self.act == "gelu_glu")
+            gelu, down = self.act == "gelu_glu", self.down_proj
+            if x.dim() == 2 and x.shape[0] <= 32 and down.bias is None and \
+                    down.tp == 1 and plain(RowParallelLinear, down):
+                y = ops.few_rows_mlp(x, self._gateup_w, down.weight, gelu,
+                                     slab_ok)
+                if y is not None:
+                    return y
+            h = ops.rows_glu(x, self._gateup_w, gelu)
             if h is not None:
                 y = ops.rows_parts(h, self.down_proj.weight) \
                     if parts and self.down_proj.bias is None else None

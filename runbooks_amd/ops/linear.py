@@ -205,11 +205,14 @@ def _tiles_serve(x: torch.Tensor, weight: torch.Tensor, glu: bool = False
             _backend.ext().tile_gemm_takes(x, weight, glu))
 
 
-def _rows_served(x: torch.Tensor, weight: torch.Tensor):
-    """_rows_copy for results that are not differentiated, of 33 to 128 rows."""
+def _rows_served(x: torch.Tensor, weight: torch.Tensor, least: int = 33):
+    """_rows_copy for results that are not differentiated, of `least` to 128
+    rows; up to 32 only where no 8-bit weights serve them."""
     if not (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and
-            32 < x.shape[0] <= 128 and not torch.is_grad_enabled() and
+            least <= x.shape[0] <= 128 and not torch.is_grad_enabled() and
             weight.is_contiguous()):
+        return None
+    if x.shape[0] <= 32 and _registry_get(_FP8_REGISTRY, weight) is not None:
         return None
     return _rows_copy(x, weight, x.shape[0], weight.shape[0], x.shape[1])
 
@@ -236,8 +239,9 @@ def rows_heads(x: torch.Tensor, weight: torch.Tensor, cos, sin, positions, kc,
                vc, slots, hq: int, rows: bool) -> torch.Tensor | None:
     """The product of 33 to 128 rows with joint weights of q, k and v whose
     rotation and cache write it does too: q [T, hq, dh], or, in rows, q, k and v
-    side by side; None where no paired copy serves it."""
-    dw, n = _rows_served(x, weight), weight.shape[0]
+    side by side, also of fewer (a step of so few goes by decode_chain.py); None
+    where no paired copy serves it."""
+    dw, n = _rows_served(x, weight, 1 if rows else 33), weight.shape[0]
     if dw is None or kc.dtype != torch.bfloat16 or \
             dw[2] * 2 != kc.shape[3] or \
             not _backend.ext().rows_ends_pay(x.shape[0], n, x.shape[1]):
@@ -470,6 +474,11 @@ class Copy:
             (q[0], q[1], q[2]) if self.fp8 else \
             (dw[0], None, dw[2]) if dw is not None else (None, None, 0)
 
+    def shares_x(self, m: int) -> bool:
+        """From 17 rows the kernel that shares x between workgroups' waves wins
+        where it has about one workgroup for every CU (wide_linear)."""
+        return 16 < m <= 32 and not self.fp8 and 10240 <= self.n <= 32768
+
     def product(self, xs, m: int):
         """Of an operand: bf16 [m, n], or fp32 parts [P, m, n] of it."""
         ext = _backend.ext()
@@ -478,6 +487,33 @@ class Copy:
                                        self.k, True, self.half)
         return ext.decode_gemm_raw(xs, self.ws, m, self.n, self.k,
                                    half=self.half)
+
+
+def few_rows_mlp(x: torch.Tensor, weight: torch.Tensor, down: torch.Tensor,
+                 gelu: bool, raw: bool) -> torch.Tensor | None:
+    """act(x G^T) * (x U^T) D^T of weight = [G ; U] and up to 32 rows, the gated
+    unit as the end of the first product; with `raw` possibly fp32 parts of it;
+    None where there are no copies for it.
+
+    A product of a paired copy that ends in nothing is slower than one of a copy in
+    order, for its columns go to memory in pieces of 32 bytes (us of 16 and 32
+    rows: 49152 x 3072 48.3 and 58.4, 46.3 and 53.1 in order; 22016 x 4096 32.0 and
+    36.3, 32.8 and 35.4)."""
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and
+            1 <= x.shape[0] <= 32 and not torch.is_grad_enabled() and
+            weight.is_contiguous() and down.is_contiguous()):
+        return None
+    first, second = Copy(weight), Copy(down)
+    if first.ws is None or second.ws is None or first.half * 2 != first.n:
+        return None
+    ext, (m, k) = _backend.ext(), x.shape
+    if first.shares_x(m) and x.is_contiguous() and x.data_ptr() % 16 == 0:
+        h = ext.rows_glu(x, first.ws, first.n, gelu, True)
+    else:
+        h = ext.decode_glu(_swizzled(x, m, k), first.ws, first.scale, m,
+                           first.n, k, gelu)
+    y = second.product(h, m)
+    return y if raw or y.dtype != torch.float32 else ext.sum_parts(y)
 
 
 def decode_ready(weight: torch.Tensor, m: int) -> bool:

@@ -318,3 +318,37 @@ def test_short_prompt(monkeypatch, tokens, kv):
         monkeypatch.setattr(ops, name, lambda *a, **k: None)
     for a, b in zip(got, prompt()):
         assert _rel(a, b.double()) < 2e-2
+
+
+@pytest.mark.parametrize("tokens", [1, 9, 16, 17, 32])
+@pytest.mark.parametrize("kv,inter,eight_bit", [
+    (8, 2048, False), (2, 1040, False), (2, 6144, False), (8, 2048, True)])
+def test_shortest_prompts(monkeypatch, tokens, kv, inter, eight_bit):
+    """Prompts of up to 32 tokens, whose products end in the rotation and the
+    gated unit: as test_short_prompt, the products of modules called in their
+    place."""
+    m = _model(kv, inter, eight_bit=eight_bit)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    ended = []
+
+    def prompt():
+        caches = m.alloc_caches(16, DEV)
+        with torch.no_grad():
+            logits = m.prefill(torch.arange(tokens, device=DEV)[None] % 50,
+                               torch.arange(tokens, **i32), caches,
+                               torch.arange(tokens, **i32) + 5)
+        return [logits] + [c for layer in caches for c in layer]
+
+    for name in ("rows_heads", "few_rows_mlp"):
+        def seen(*a, f=getattr(ops, name), **k):
+            y = f(*a, **k)
+            ended.append(y is not None)
+            return y
+        monkeypatch.setattr(ops, name, seen)
+    got = prompt()
+    # 8-bit weights have their own product of q, k and v
+    assert ended == [not eight_bit, True] * 2
+    for name in ("rows_heads", "few_rows_mlp"):
+        monkeypatch.setattr(ops, name, lambda *a, **k: None)
+    for a, b in zip(got, prompt()):
+        assert _rel(a, b.double()) < 2e-2

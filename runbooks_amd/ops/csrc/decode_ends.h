@@ -60,10 +60,10 @@ enum Kind {
 
 struct Ends {
   uint16_t *y;            // PLAIN, GLU: rows; QKV: rows of all heads (or null)
-  uint16_t *operand;      // GLU: [N / 32][2][32][8] (or null)
   float *slabs;
   const float *scale;     // of W's rows, in their own order (or null)
   int half;               // distance of paired rows; 0: rows in order
+  uint16_t *operand;      // GLU: [N / 32][2][32][8] (or null)
   // input without its norm's 1 / rms: sums of squares of its rows [M, parts],
   // parts a multiple of 4 (or null)
   const float *squares;

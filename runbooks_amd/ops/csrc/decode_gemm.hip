@@ -231,8 +231,8 @@ __device__ __forceinline__ f32x16v weight_stream(
 
 template <bool FP8, Kind KIND>
 __global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
-    const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws, Ends e,
-    int M, int N, int K) {
+    const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws, int M,
+    int N, int K, Ends e) {
   Early<KIND> early;
   early.begin(e, M);
   const f32x16v acc =
@@ -255,8 +255,8 @@ __global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
 // 13.5 (library 43 and 23).
 template <int RB, int NWN, int CH, Kind KIND>
 __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
-    const uint16_t *__restrict__ x, const uint8_t *__restrict__ ws, Ends e,
-    int M, int N, int K) {
+    const uint16_t *__restrict__ x, const uint8_t *__restrict__ ws, int M,
+    int N, int K, Ends e) {
   constexpr int KG = 4 / NWN, P = 2 * CH;          // pieces of a row
   constexpr int XL = RB * CH / NWN;                // of x, a lane and chunk
   constexpr int TILE = RB * 32 * P * 16;
@@ -580,8 +580,8 @@ static void launch(Kind kind, const at::Tensor &xs, const at::Tensor &ws,
     hipLaunchKernelGGL(kernel, dim3((unsigned)(N / 32), (unsigned)split),
                        dim3(BLOCK), 0, at::cuda::getCurrentHIPStream(),
                        (const uint16_t *)xs.data_ptr(),
-                       (const uint8_t *)ws.data_ptr(), e, (int)M, (int)N,
-                       (int)K);
+                       (const uint8_t *)ws.data_ptr(), (int)M, (int)N, (int)K,
+                       e);
   };
   switch (kind) {
     case ends::SLAB: return go(decode_gemm_kernel<FP8, ends::SLAB>);
@@ -842,8 +842,8 @@ static void launch_rows(Kind kind, const at::Tensor &x, const at::Tensor &ws,
                             (unsigned)split), dim3(BLOCK), lds,
                        at::cuda::getCurrentHIPStream(),
                        (const uint16_t *)x.data_ptr(),
-                       (const uint8_t *)ws.data_ptr(), e, (int)M, (int)N,
-                       (int)K);
+                       (const uint8_t *)ws.data_ptr(), (int)M, (int)N, (int)K,
+                       e);
   };
   if (kind == ends::GLU)
     return go(decode_gemm_rows_kernel<RB, NWN, CH, ends::GLU>);

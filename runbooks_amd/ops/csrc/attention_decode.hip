@@ -27,7 +27,7 @@
 #include "common.h"
 
 int64_t paged_decode_parts(int64_t nsplit, int64_t longest, int64_t dh,
-                           int64_t group, bool fp8, bool transposed);
+                           int64_t group, bool transposed);
 
 namespace {
 
@@ -84,8 +84,9 @@ RB_DEV int sequence_of() {
 // so halving cache bytes halves the dominant stream AND doubles KV
 // capacity within 288 GB. Dequant rides
 // v_cvt_pk_f32_fp8 in the inner loop.
-template <int DH, int G, bool SPLIT, bool FP8 = false, int WAVES = NW>
-__global__ __launch_bounds__(WAVES * 64) void paged_decode_kernel(
+template <int DH, int G, bool SPLIT, bool FP8 = false, int WAVES = NW,
+          int PER_SIMD = 1>
+__global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k_cache,
     const uint16_t *__restrict__ v_cache, const int32_t *__restrict__ block_tables,
     const int32_t *__restrict__ seq_lens,
@@ -781,11 +782,6 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
   }
 }
 
-// Waves of a workgroup that has a whole sequence of a kv head to itself.
-constexpr int whole_waves(int64_t dh, bool fp8) {
-  return fp8 || dh > 128 ? 8 : 16;
-}
-
 template <int DH, int G, bool FP8>
 void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                    const at::Tensor &v_cache, const at::Tensor &block_tables,
@@ -811,7 +807,7 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
   // versa.
   const bool vt = v_cache.size(3) == bs &&
       v_cache.size(2) == (int64_t)(FP8 ? DH + 4 : DH);
-  nsplit = (int)paged_decode_parts(nsplit, longest, DH, G, FP8, vt);
+  nsplit = (int)paged_decode_parts(nsplit, longest, DH, G, vt);
   if constexpr (G >= 4 && DH <= 128) {
     if (vt && bs == 16) {
       if (nsplit <= 1) {
@@ -861,9 +857,31 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                        splits, scale);
   };
   if constexpr (G < NW) {
-    constexpr int MORE = whole_waves(DH, FP8);
-    if (nsplit <= 1 && longest > 64)
-      return go(paged_decode_kernel<DH, G, false, FP8, MORE>, MORE, 1, nullptr);
+    // Whole sequences by 8 waves: of a short one more have nothing to do, and a CU
+    // has room for more workgroups (which is why one query head a kv head keeps
+    // to 64 registers, of 68). By 16 where long tables and few workgroups leave
+    // the longest sequences to the end; by 4 where there are workgroups enough and
+    // 8 waves take too many registers (e4m3 107, two query heads 93).
+    // us by 4, 8 and 16 waves, 32 heads of 128 in bf16: 32 sequences of 100 tokens
+    // 14.0, 13.7 and 17.3, of 300 31.9, 31.8 and 33.2, of 129 to 2015 111, 107 and
+    // 111, 4000 and 31 of 100 115, 69 and 58; 16 of 100 9.0, 9.3 and 10.3, of 800 to
+    // 3900 135, 120 and 117, 4000 and 15 of 100 111, 65 and 50; one of 100 5.8, 5.3
+    // and 6.1, of 512 13.2, 9.6 and 9.5; 12 heads of 64, 64 of 37 to 1400 33, 32 and
+    // 34. By 4 and 8 waves, e4m3: 32 of 100 11.0 and 14.9, of 50 to 1000 32.0 and
+    // 35.7, 64 of 300 34.9 and 40.4, of 1000 104 and 103, 16 of 1000 27.0 and 28.2,
+    // 4000 and 15 of 100 55 and 39; 12 heads of 64, 64 of 50 to 1000 20.9 and 18.8,
+    // 128 of them 28.8 and 29.2. 32 kv heads with two queries each, 64 sequences of
+    // 100 27 and 33, of 50 to 1000 113 and 108. 16 heads of 256, 40 sequences of 100
+    // 17.6 and 18.7, of 50 to 1000 84 and 73.
+    constexpr int ROOM = !FP8 && G == 1 && DH <= 128 ? 8 : 1;
+    const int64_t base = (int64_t)B * hkv;
+    if constexpr (ROOM == 8 && DH == 128)
+      if (nsplit <= 1 && longest > 512 && base <= 512)
+        return go(paged_decode_kernel<DH, G, false, FP8, 16, ROOM>, 16, 1,
+                  nullptr);
+    const bool many = (FP8 || G > 1) && base > (DH == 64 ? 1023 : 512);
+    if (nsplit <= 1 && longest > 64 && !many)
+      return go(paged_decode_kernel<DH, G, false, FP8, 8, ROOM>, 8, 1, nullptr);
   }
   if (nsplit <= 1)
     return go(paged_decode_kernel<DH, G, false, FP8>, NW, 1, nullptr);
@@ -885,26 +903,29 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
 //
 // Parts of fewer than 64 tokens cost more than they save (one sequence of 37
 // tokens, 32 heads of 128: 16 parts 8.2 us, one 4.1; matrix instructions take 32:
-// 32 query heads, one of 500, 16 parts 7.5, 10 7.9). One workgroup of 8 or 16 waves
-// takes all of a sequence where it has at least twice the waves of all parts, or
-// the table is short: then it is as fast for the longest sequence of an uneven
-// batch, too, and the launch that adds up the parts goes.
+// 32 query heads, one of 500, 16 parts 7.5, 10 7.9). One workgroup of more waves
+// takes all of a sequence in place of two parts, or where the table is short: then
+// the launch that adds up the parts goes, and the longest sequence of an uneven
+// batch takes about as long. In place of more parts it does not, and an engine's
+// tables are wide whatever the lengths.
 //
 // us in parts and whole, 32 heads of 128 in bf16: one sequence of 200 tokens 9.1
 // and 7.1, of 512 9.8 and 9.5, of 1024 12.0 and 16.2; 4 of 512 13.8 and 12.2, one of
 // 512 and 3 of 50 10.1 and 10.5, one of 1024 and 3 of 50 12.7 and 16.6; 16 (two
 // parts) of 800 to 3900 122 and 123, 4000 and 15 of 100 63.7 and 54.3; 8 (four) of
-// 129 to 2015 34.5 and 34.4, of 2000 54.4 and 49.6, 5 of 2000 and 3 that pad the batch
-// 38.2 and 33.4, 4000 and 7 of 100 35.8 and 47.3. e4m3: 16 (two) of 800 to 3900 74.5
-// and 75.4, 4000 and 15 of 100 36.1 and 39.3; 8 (four), 4000 and 7 of 100 22.6 and
-// 37.5. 16 heads of 256: 4 of 256 12.9 and 10.7, one of 256 and 7 of 50 11.0 and 9.9,
-// one of 512 and 7 of 50 12.2 and 15.2; 16 (four), 4000 and 15 of 100 44 and 80.
+// 384 16.8 and 13.9, of 129 to 2015 34.5 and 34.4, 5 of 2000 and 3 that pad the batch
+// 38.2 and 33.4, 4000 and 7 of 100 35.8 and 47.3. e4m3: 16 (two) of 256 15.9 and 12.4,
+// of 800 to 3900 74.5 and 75.4, 4000 and 15 of 100 36.1 and 39.3; 8 (four) of 384 14.4
+// and 10.0, 4000 and 7 of 100 22.6 and 37.5. 16 heads of 256: 4 of 256 12.9 and 10.7,
+// one of 256 and 7 of 50 11.0 and 9.9, one of 512 and 7 of 50 12.2 and 15.2; 32 (two)
+// of 100 to 2000 110 and 108, 4000 and 31 of 100 79 and 84; 16 (four), 4000 and 15 of
+// 100 44 and 80.
 int64_t paged_decode_parts(int64_t nsplit, int64_t longest, int64_t dh,
-                           int64_t group, bool fp8, bool transposed) {
+                           int64_t group, bool transposed) {
   const int64_t parts =
       std::min(nsplit, (longest + 63) / (transposed ? 32 : 64));
-  const bool whole = group < NW && (longest <= (dh > 128 ? 256 : 512) ||
-                                    parts * 2 * NW <= whole_waves(dh, fp8));
+  const bool whole =
+      group < NW && (parts <= 2 || longest <= (dh > 128 ? 256 : 512));
   return whole ? 1 : std::max<int64_t>(parts, 1);
 }
 

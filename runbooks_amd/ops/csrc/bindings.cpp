@@ -22,7 +22,7 @@ at::Tensor paged_decode(at::Tensor q, at::Tensor k_cache, at::Tensor v_cache,
                         int64_t nsplit, double scale,
                         c10::optional<at::Tensor> seq_starts);
 int64_t paged_decode_parts(int64_t nsplit, int64_t longest, int64_t dh,
-                           int64_t group, bool fp8, bool transposed);
+                           int64_t group, bool transposed);
 std::vector<at::Tensor> paged_decode_swz(at::Tensor q, at::Tensor k_cache,
                                          at::Tensor v_cache,
                                          at::Tensor block_tables,
@@ -98,7 +98,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("scale"), py::arg("seq_starts") = py::none());
   m.def("paged_decode_parts", &paged_decode_parts,
         "parts that a sequence is taken in", py::arg("nsplit"),
-        py::arg("longest"), py::arg("dh"), py::arg("group"), py::arg("fp8"),
+        py::arg("longest"), py::arg("dh"), py::arg("group"),
         py::arg("transposed"));
   m.def("paged_decode_swz", &paged_decode_swz,
         "paged decode also emitting the o_proj decode-GEMM operand",

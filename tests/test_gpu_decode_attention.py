@@ -21,7 +21,10 @@ def _rel(a, b):
     (4, 32, 32, 128, 30, 8), (16, 32, 16, 128, 40, 2), (8, 32, 32, 128, 130, 4),
     (4, 16, 16, 256, 15, 16), (16, 16, 16, 256, 40, 4), (2, 4, 4, 128, 4, 16),
     (1, 4, 4, 128, 129, 16), (3, 12, 12, 64, 40, 1), (5, 32, 32, 128, 33, 2),
-    (2, 8, 4, 128, 40, 1), (3, 4, 4, 256, 17, 1), (2, 4, 4, 256, 16, 8)])
+    (2, 8, 4, 128, 40, 1), (3, 4, 4, 256, 17, 1), (2, 4, 4, 256, 16, 8),
+    # as many workgroups as change the number of waves, and one more sequence
+    (16, 32, 32, 128, 33, 1), (17, 32, 32, 128, 33, 1),
+    (43, 24, 24, 64, 5, 1), (17, 64, 32, 128, 5, 1)])
 def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
     """By 4, 8 or 16 waves or in parts, with and without a window's start, and
     with sequences as short and as long as the table: the plain result but for
@@ -64,7 +67,7 @@ def test_uneven_captured_bucket():
     lens = torch.tensor([4000, 100, 17, 100, 1, 1, 1, 1])
     heads, dh, blocks = 32, 128, 257
     nsplit = fixed_nsplit(len(lens), heads)
-    assert ops.ext().paged_decode_parts(nsplit, blocks * 16, dh, 1, False,
+    assert ops.ext().paged_decode_parts(nsplit, blocks * 16, dh, 1,
                                         False) == nsplit
     used = (lens + 15) // 16
     kc, vc = ops.alloc_kv_cache(int(used.sum()) + 1, heads, dh, DEV,

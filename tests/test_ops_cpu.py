@@ -313,15 +313,15 @@ def test_versions_of_weights():
 
 def test_parts_of_a_sequence():
     """Long tables keep the caller's split of 256 sequence-heads and more, so
-    that one long request is not left to one CU; short tables and two parts
-    (of four waves each, where one workgroup has sixteen) are not split."""
+    that one long request is not left to one CU; short tables are not split,
+    nor sequences of which there would be two parts."""
     ext = pytest.importorskip("runbooks_amd.ops._hip")
 
-    def parts(nsplit, longest, dh=128, group=1, fp8=False, vt=False):
-        return ext.paged_decode_parts(nsplit, longest, dh, group, fp8, vt)
+    def parts(nsplit, longest, dh=128, group=1, vt=False):
+        return ext.paged_decode_parts(nsplit, longest, dh, group, vt)
     assert parts(4, 4112) == 4 and parts(16, 4112) == 16
-    assert parts(2, 4112) == 1 and parts(2, 4112, fp8=True) == 2
-    assert parts(2, 8208, dh=256) == 2 and parts(1, 8208, dh=256) == 1
+    assert parts(2, 4112) == 1 and parts(3, 8208, dh=256) == 3
+    assert parts(2, 8208, group=4) == 2 and parts(1, 8208, dh=256) == 1
     assert parts(16, 512) == 1 and parts(16, 528) == 9
     assert parts(16, 256, dh=256) == 1 and parts(16, 272, dh=256) == 5
     assert parts(16, 512, group=4) == 8         # a share of the query heads

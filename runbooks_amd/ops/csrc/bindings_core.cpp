@@ -43,6 +43,7 @@ at::Tensor sum_parts(at::Tensor parts);
 bool tile_gemm_takes(at::Tensor x, at::Tensor w, bool glu);
 at::Tensor tile_lora(at::Tensor x, at::Tensor w, at::Tensor t, std::vector<at::Tensor> bs, double scale, int64_t tile);
 int64_t tile_gemm_parts(int64_t M, int64_t N, int64_t K);
+std::vector<int64_t> tile_gemm_choice(int64_t M, int64_t N, int64_t K, int64_t max_parts);
 at::Tensor tile_gemm(at::Tensor x, at::Tensor w, int64_t max_parts, int64_t glu, int64_t tile, int64_t parts);
 at::Tensor decode_gemm_rows(at::Tensor x, at::Tensor ws, int64_t N, int64_t half, bool raw);
 at::Tensor decode_gemm_fp8(at::Tensor xs, at::Tensor w8s, at::Tensor scale, int64_t M, int64_t N, int64_t K, bool raw, int64_t half);
@@ -173,6 +174,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "x @ W^T + scale t_i @ B_i^T of siblings side by side");
   m.def("tile_gemm_parts", &tile_gemm_parts,
         "parts that tile_gemm makes of sums where it may");
+  m.def("tile_gemm_choice", &tile_gemm_choice, py::arg("M"), py::arg("N"),
+        py::arg("K"), py::arg("max_parts") = 1,
+        "tile, parts, tile of the rest and its first column");
   m.def("tile_gemm", &tile_gemm, py::arg("x"), py::arg("w"),
         py::arg("max_parts") = 1, py::arg("glu") = 0, py::arg("tile") = -1,
         py::arg("parts") = 0,

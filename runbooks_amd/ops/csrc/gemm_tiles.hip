@@ -507,6 +507,15 @@ int64_t tile_gemm_parts(int64_t M, int64_t N, int64_t K) {
   return choose(M, N, K, MAX_PARTS, -1).parts;
 }
 
+// What tile_gemm and tile_lora run: tile, parts, the tile of the columns from
+// `split` on (-1: none) and split.
+std::vector<int64_t> tile_gemm_choice(int64_t M, int64_t N, int64_t K,
+                                      int64_t max_parts) {
+  const Choice c = max_parts > 1 ? choose(M, N, K, (int)max_parts, -1)
+                                 : choose_two(M, N, K);
+  return {c.tile, c.parts, c.rest, c.split};
+}
+
 // x W^T: bf16 [M, N]; where max_parts > 1, possibly fp32 parts [P, M, N] of the
 // sums. glu 1 (SiLU) or 2 (tanh-GELU): act(x G^T) * (x U^T) of W = [G ; U]. tile
 // and parts: the choice of a test.

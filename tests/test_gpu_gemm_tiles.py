@@ -92,11 +92,13 @@ def test_adapters(tile, m, widths, k):
     assert bool(((got.float() - ref).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("m,n,k", [(700, 22016, 512), (2200, 22016, 1024),
+@pytest.mark.parametrize("m,n,k", [(700, 22016, 4096), (2200, 22016, 1024),
                                    (1800, 28680, 1024)])
 def test_two_launches(m, n, k):
     """Sizes of more tiles than whole rounds: columns in tiles of two sizes."""
     from runbooks_amd import ops
+    _, parts, rest, split = ops.ext().tile_gemm_choice(m, n, k)
+    assert parts == 1 and rest >= 0 and 0 < split < n
     x, w = _inputs(m, n, k)
     _check(ops.ext().tile_gemm(x, w), x, w, 2.0 ** -8)
     g, u = (x.float() @ w.float().t()).chunk(2, 1)
@@ -105,16 +107,134 @@ def test_two_launches(m, n, k):
     assert bool(((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4).all())
 
 
-@pytest.mark.parametrize("m,n,k", [(129, 4096, 4096), (512, 4096, 11008),
-                                   (300, 3072, 24576), (768, 4096, 4096)])
-def test_sums_for_the_norm(m, n, k):
-    """rows_parts of more than 128 rows: parts, or what the library is left
-    with; refused are rows and parameters that do not lie as the kernel reads
-    them."""
+def _with_adapters(x, w, t, bs, scale):
+    more = torch.cat([ti.float() @ b.float().t() for ti, b in zip(t, bs)], 1)
+    return x.float() @ w.float().t() + scale * more
+
+
+@pytest.mark.parametrize("m,widths,k", [
+    (700, [11008, 11008], 4096),            # siblings meet in the first launch
+    (700, [18432, 2560, 1024], 4096),       # in the second one
+    (3001, [4096, 1024, 1024], 4096)])      # between them, and in the second
+def test_adapters_in_two_launches(m, widths, k):
+    from runbooks_amd import ops
+    n = sum(widths)
+    _, _, rest, split = ops.ext().tile_gemm_choice(m, n, k)
+    assert rest >= 0 and 0 < split < n
+    x, w = _inputs(m, n, k)
+    t = torch.randn(len(widths), m, 16, device="cuda").bfloat16()
+    bs = [torch.randn(c, 16, device="cuda").bfloat16() for c in widths]
+    got = ops.ext().tile_lora(x, w, t, bs, 0.3)
+    ref = _with_adapters(x, w, t, bs, 0.3)
+    bound = 2.0 ** -8 * ref.abs() + 2.0 ** -24 * (2 * k ** 1.5 + 2 * 16 * 16)
+    assert bool(((got.float() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m,widths,k,tiles", [
+    (1100, [2048], 256, True), (129, [4096, 1024, 1024], 320, True),
+    (1100, [4096], 8192, False), (512, [4096], 256, False)])
+def test_products_with_adapters(monkeypatch, m, widths, k, tiles):
+    """Both ways that wide_product_lora may take, by its own rule and against
+    it: the library's rounds the product and the sum."""
+    from runbooks_amd import ops
+    from runbooks_amd.ops import linear
+    n = sum(widths)
+    x, w = _inputs(m, n, k)
+    t = torch.randn(len(widths), m, 16, device="cuda").bfloat16()
+    bs = [torch.randn(c, 16, device="cuda").bfloat16() for c in widths]
+    ref = _with_adapters(x, w, t, bs, 0.3)
+    tile = ops.ext().tile_lora(x, w, t, bs, 0.3)
+    got = linear.wide_product_lora(x, w, t, bs, 0.3)
+    assert linear._lora_in_tiles(m, n, k) is tiles
+    assert torch.equal(got, tile) is tiles
+    monkeypatch.setattr(linear, "_lora_in_tiles", lambda *a: not tiles)
+    other = linear.wide_product_lora(x, w, t, bs, 0.3)
+    sums = 2.0 ** -24 * (2 * k ** 1.5 + 2 * 16 * 16)
+    product = (x.float() @ w.float().t()).abs()
+    for y in (got, other):
+        bound = 2.0 ** -8 * (ref.abs() + product * 1.01) + sums
+        assert bool(((y.float() - ref).abs() <= bound).all())
+
+
+def test_packed_adapter_in_tiles():
+    """A LoRA layer whose product ends with its adapter, forward and backward,
+    against fp32: results and gradients of one bf16 rounding and fp32 sums over
+    inputs of one rounding more (t, dt, the gradients' own)."""
+    from torch import nn
+
+    from runbooks_amd.ops import linear
+    from runbooks_amd.train.lora import LoRALinear
+    m, n, k = 1100, 2048, 512
+    assert linear._lora_in_tiles(m, n, k)
+    torch.manual_seed(0)
+    base = nn.Linear(k, n, bias=False, device="cuda", dtype=torch.bfloat16)
+    base.weight.requires_grad_(False)
+    layer = LoRALinear(base, r=16, alpha=32, dtype=torch.bfloat16).cuda()
+    with torch.no_grad():
+        layer.lora_a.normal_(0, k ** -0.5)
+        layer.lora_b.normal_(0, 0.25)
+    x = torch.randn(m, k, device="cuda").bfloat16().requires_grad_()
+    dy = torch.randn(m, n, device="cuda").bfloat16()
+    y = layer(x)
+    assert y.grad_fn.name() == "_LoRAPackedBackward"
+    y.backward(dy)
+    leaves = [v.detach().float().requires_grad_()
+              for v in (x, layer.lora_a, layer.lora_b)]
+    xf, a, b = leaves
+    ref = xf @ base.weight.float().t() + layer.scale * (xf @ a.t()) @ b.t()
+    ref.backward(dy.float())
+    for got, want in ((y, ref), (x.grad, xf.grad), (layer.lora_a.grad, a.grad),
+                      (layer.lora_b.grad, b.grad)):
+        assert float((got - want).detach().norm() / want.detach().norm()) < 2 * 2.0 ** -8
+
+
+@pytest.mark.parametrize("m,n,k,taken", [
+    (1000, 8192, 8256, True), (1793, 4096, 8256, True),
+    (1000, 8192, 8192, False), (1700, 3072, 8256, False)])
+def test_one_round_of_tiles(m, n, k, taken):
+    """Long rows that one round of tiles does, and their neighbours."""
+    from runbooks_amd import ops
+    from runbooks_amd.ops import linear
+    x, w = _inputs(m, n, k)
+    y = linear._one_round(x, w)
+    assert (y is not None) is taken
+    got = linear.wide_product(x, w)
+    _check(got, x, w, 2.0 ** -8)
+    if taken:
+        assert torch.equal(got, ops.ext().tile_gemm(x, w))
+
+
+@pytest.mark.parametrize("m,n,k,taken", [
+    (129, 12288, 256, True), (256, 18432, 320, True), (320, 12288, 2048, True),
+    (257, 12288, 1024, False), (256, 20480, 256, False)])
+def test_wide_products_of_few_rows(monkeypatch, m, n, k, taken):
+    from runbooks_amd import ops
+    from runbooks_amd.ops import linear
+    x, w = _inputs(m, n, k)
+    called = []
+    monkeypatch.setattr(linear, "fast_linear",
+                        lambda *a, f=linear.fast_linear: called.append(1) or
+                        f(*a))
+    with torch.no_grad():
+        got = ops.wide_linear(x, w)
+    _check(got, x, w, 2.0 ** -8)
+    assert (not called) is taken
+
+
+@pytest.mark.parametrize("m,n,k,parts", [
+    (129, 4096, 4096, 4), (512, 4096, 11008, 4), (300, 3072, 24576, 3),
+    (1793, 4096, 11008, 1),                     # whole, in one round
+    (768, 4096, 4096, None), (400, 2048, 2048, None)])
+def test_sums_for_the_norm(m, n, k, parts):
+    """rows_parts of more than 128 rows: parts, one round of tiles, or None
+    where the library is as fast; refused are rows and parameters that do not
+    lie as the kernel reads them."""
     from runbooks_amd import ops
     x, w = _inputs(m, n, k)
     with torch.no_grad():
         y = ops.rows_parts(x, w)
+        assert (None if y is None else
+                y.shape[0] if y.dim() == 3 else 1) == parts
         if y is not None:
             _check(y.sum(0) if y.dim() == 3 else y, x, w, 2.0 ** -8)
         wide = torch.zeros(m, 2 * k, device="cuda", dtype=torch.bfloat16)

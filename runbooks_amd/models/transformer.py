@@ -906,7 +906,7 @@ class Transformer(nn.Module):
 
 class _AffineBlock:
     """A block's products with their biases and activation in a launch each
-    (csrc/decode_gemm.hip, decode_affine). They read the parameters, so a
+    (csrc/decode_affine.hip). They read the parameters, so a
     captured step follows weights that change in place."""
 
     ACTS = {"relu": 1, "gelu": 2, "gelu_tanh": 3}

@@ -18,7 +18,8 @@
 //                         49152 x 3072       51.0 49.2  50.1 47.0  57.6 52.8
 // (6144 columns were split before, for their number of workgroups). The sums of
 // squares add 0.3 us. A step of llama2-7b, with the residual sums of
-// decode_res.hip: one sequence 3343 -> 2990, 32 6990 -> 6647.
+// decode_res.hip and attention by whole sequences: one sequence 3335 -> 2972, 32
+// 7026 -> 6534.
 #pragma once
 
 #include "common.h"

@@ -225,7 +225,10 @@ def rows_glu(x: torch.Tensor, weight: torch.Tensor, gelu: bool
     40.2 and 37.6, 49152 x 3072 64.5 and 59.1), above that tiles (22016 x 4096: 129
     rows 55 and 48, 512 91 and 77, 1537 247 and 233, 2048 298 and 270, 4500 623
     and 586; 28672 x 4096: 1400 277 and 283, 1800 354 and 337, 6500 1283 and
-    1093; 49152 x 3072: 256 98 and 76, 1021 267 and 228, 3200 821 and 713)."""
+    1093; 49152 x 3072: 256 98 and 76, 1021 267 and 228, 3200 821 and 713; 11264 x 2048:
+    900 55 and 40; 5632 x 1024: 129 15 and 12; 57344 x 8192: 256 243 and 244, 1536
+    1083 and 1051, 4096 2613 and 2633. Of 200 sizes two were slower by more than 2%,
+    1400 x 28672 x 4096 274 and 292 and 640 x 49152 x 3072 189 and 196)."""
     if _tiles_serve(x, weight, True):
         return _backend.ext().tile_gemm(x, weight, glu=2 if gelu else 1)
     dw, n = _rows_served(x, weight), weight.shape[0]
@@ -285,7 +288,10 @@ def _one_round(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
     """x @ weight^T of long rows in one round of tiles of 256 x 128, or None
     where the library is as good: it takes 192 or 256 columns, too few tiles for
     256 CUs (us there and here, to 4096 columns: 2048 rows of 11008 160 and 145,
-    of 14336 205 and 180; 2048 of 4096 58 and 58; 1280 of 11008 119 and 130)."""
+    of 14336 205 and 193, of 20480 323 and 265, of 28672 367 and 394; to 3584 2048 of
+    14336 190 and 175; to 5120 1536 of 13824 191 and 182; to 8192 1024 of 13824 194
+    and 186, of 28672 446 and 397; to 14336 512 of 11008 167 and 156, 257 of 13824 152
+    and 159. Outside: 2048 of 4096 58 and 58; 1280 of 11008 119 and 130)."""
     (m, k), n = x.shape, weight.shape[0]
     tiles = -(-m // 256) * -(-n // 128)
     if k > 8192 and 224 <= tiles <= 256 and m <= 2048 and \

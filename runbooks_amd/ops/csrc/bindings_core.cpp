@@ -42,6 +42,10 @@ at::Tensor embed_res32(at::Tensor tokens, at::Tensor positions, at::Tensor table
 at::Tensor sum_parts(at::Tensor parts);
 bool tile_gemm_takes(at::Tensor x, at::Tensor w, bool glu);
 at::Tensor tile_lora(at::Tensor x, at::Tensor w, at::Tensor t, std::vector<at::Tensor> bs, double scale, int64_t tile);
+bool tile_gemm_down_takes(at::Tensor x, at::Tensor w);
+bool tile_gemm_down_pays(int64_t M, int64_t N, int64_t K);
+std::vector<int64_t> tile_gemm_down_choice(int64_t M, int64_t N, int64_t K, int64_t max_parts);
+at::Tensor tile_gemm_down(at::Tensor x, at::Tensor w, at::Tensor t, std::vector<at::Tensor> as, int64_t max_parts, int64_t tile, int64_t parts);
 int64_t tile_gemm_parts(int64_t M, int64_t N, int64_t K);
 std::vector<int64_t> tile_gemm_choice(int64_t M, int64_t N, int64_t K, int64_t max_parts);
 at::Tensor tile_gemm(at::Tensor x, at::Tensor w, int64_t max_parts, int64_t glu, int64_t tile, int64_t parts);
@@ -172,6 +176,18 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_lora", &tile_lora, py::arg("x"), py::arg("w"), py::arg("t"),
         py::arg("bs"), py::arg("scale"), py::arg("tile") = -1,
         "x @ W^T + scale t_i @ B_i^T of siblings side by side");
+  m.def("tile_gemm_down_takes", &tile_gemm_down_takes, py::arg("x"),
+        py::arg("w"), "whether tile_gemm_down takes x and W");
+  m.def("tile_gemm_down_pays", &tile_gemm_down_pays, py::arg("M"),
+        py::arg("N"), py::arg("K"), "whether it is as good as the library");
+  m.def("tile_gemm_down_choice", &tile_gemm_down_choice, py::arg("M"),
+        py::arg("N"), py::arg("K"), py::arg("max_parts") = 1,
+        "tile, parts, tile of the rest and its first column");
+  m.def("tile_gemm_down", &tile_gemm_down, py::arg("x"), py::arg("w"),
+        py::arg("t"), py::arg("as_"), py::arg("max_parts") = 1,
+        py::arg("tile") = -1, py::arg("parts") = 0,
+        "x @ W + sum_i t_i A_i of many rows, W [K, N] (gemm_tiles.hip): bf16 "
+        "[M, N], or, where max_parts > 1, possibly fp32 parts [P, M, N]");
   m.def("tile_gemm_parts", &tile_gemm_parts,
         "parts that tile_gemm makes of sums where it may");
   m.def("tile_gemm_choice", &tile_gemm_choice, py::arg("M"), py::arg("N"),

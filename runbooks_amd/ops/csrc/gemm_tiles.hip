@@ -1,6 +1,7 @@
 // Products of many rows, x [M, K] times W [N, K] transposed, bf16 with fp32 sums,
 // in tiles that suit their sizes, and ended by what follows them: parts of sums
-// for the norm that adds them up, or a gated unit.
+// for the norm that adds them up, a gated unit, adapters; and x [M, K] times W [K,
+// N], gradients of inputs, with adapters.
 //
 // Bound by L2, which feeds LDS at 16 TB/s (62 GB/s a CU: what is left of a
 // product of 8192 x 8192 x 4096 without its matrix instructions takes 269 us in
@@ -69,12 +70,29 @@ enum Kind {
 };
 
 // Adapters of rank 16: t [n, M, 16] and B_i [columns of i, 16], the first columns
-// of the siblings multiples of 16.
+// of the siblings multiples of 16; DOWN: A_i [16, N], start[i] elements behind b[0].
 struct Adapters {
   const uint16_t *t, *b[3];
   int start[4], n;
   float scale;
 };
+
+// Of which columns of y adapters' part is: the sibling of column n.
+__device__ __forceinline__ int sibling(const Adapters &a, int n) {
+  return (a.n > 1 && n >= a.start[1]) + (a.n > 2 && n >= a.start[2]);
+}
+
+// `bytes` from p on, a buffer whose loads past the end give zeros.
+__device__ __forceinline__ u32x4v buffer(const uint16_t *p, uint32_t bytes) {
+  const uint64_t a = (uint64_t)p;
+  u32x4v v;
+  v[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
+  v[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffff);
+  v[2] = __builtin_amdgcn_readfirstlane(bytes);
+  v[3] = 0x00020000;
+  return v;
+}
+constexpr unsigned NOWHERE = 0x80000000;    // past the end of every such buffer
 
 // Waits until the last products are in their registers, if `left` is 0. The
 // compiler does not know what mma() takes, and may move sums about right behind
@@ -104,9 +122,6 @@ __device__ __forceinline__ void end_lora(const Adapters &a,
                                          uint16_t *y, int m0, int n0, int fr,
                                          int fk, int M, int N) {
   const bf16x8v none = (bf16x8v)(__bf16)0.0f;
-  auto sibling = [&](int n) {
-    return (a.n > 1 && n >= a.start[1]) + (a.n > 2 && n >= a.start[2]);
-  };
   auto start = [&](int s) {
     return s == 0 ? 0 : s == 1 ? a.start[1] : a.start[2];
   };
@@ -115,7 +130,7 @@ __device__ __forceinline__ void end_lora(const Adapters &a,
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
     const int n = __builtin_amdgcn_readfirstlane(min(n0 + j * 16, N - 16));
-    const int s = sibling(n);
+    const int s = sibling(a, n);
     const uint16_t *b = s == 0 ? a.b[0] : s == 1 ? a.b[1] : a.b[2];
     const bf16x8v v = ends::load8v(
         b + (int64_t)(n - start(s) + fr) * 16 + at);
@@ -130,7 +145,7 @@ __device__ __forceinline__ void end_lora(const Adapters &a,
   for (int j = 0; j < FN; ++j) {
     const int n = __builtin_amdgcn_readfirstlane(n0 + j * 16);
     if (n >= N) continue;
-    const int s = sibling(n);
+    const int s = sibling(a, n);
     if (s != now) {
       now = s;
 #pragma unroll
@@ -171,12 +186,27 @@ __device__ __forceinline__ void end_lora(const Adapters &a,
 // next one during the end of the one before. Tiles go to XCDs in runs, down
 // bands of 8, so that those that run together share rows in its L2 (7931 x 28672
 // x 4096: 1432 us down all rows and one tile a workgroup, 1330 now).
-template <int BM, int BN, int WR, int WC, int SX, int SW, Kind KIND>
+//
+// DOWN: W is [K, N] and lies in LDS as it does in memory, a row of BN columns for
+// each of a K-tile's 64; ds_read_b64_tr takes operands out of it, four of a column
+// each. Pieces of 32 bytes lie at their index ^ (row % 4 + row / 8 % 2 * 4), so that
+// the eight rows that half a wave reads spread over the banks.
+//
+// Its adapters are one K-tile more, the columns of t_i and the rows of A_i side by
+// side (and zeros): no pass over y, and sums that are rounded once. With the pass
+// (8 to 20 us), the library took 359 us for 2048 x 22016 to 4096 columns in its best
+// form, two fp32 halves and their sum, and this takes 297 (1245 TFLOP/s; two parts
+// of 256 x 256, bound by power: 1.7 GHz); a step of llama2-7b, 4 x 512 tokens, 67.0 ms
+// before and 63.3 now.
+template <int BM, int BN, int WR, int WC, int SX, int SW, Kind KIND, bool DOWN>
 __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
     void *__restrict__ y, int M, int N, int K, int tm, int tn, int kt, int first,
     Adapters lora) {
   constexpr bool GLU = KIND == SILU || KIND == GELU;
+  static_assert(!DOWN || KIND == PLAIN || KIND == PARTS, "ends");
+  static_assert(!DOWN || ((BN == 128 || BN == 256) && WR * WC == 4),
+                "siblings of a load");
   constexpr int WAVES = WR * WC, FM = BM / WR / 16, FN = BN / WC / 16;
   constexpr int LOADS = (BM + BN) / 8 / WAVES;      // of a wave and K-tile
   constexpr int XL = BM / 8 / WAVES, WL = LOADS - XL;
@@ -197,49 +227,114 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
   const int per = (gridDim.x + 7 - xcd) / 8;
   int at = begin + blockIdx.x / 8;
   if (at >= end) return;
-  const int kb = blockIdx.y * kt, kn = min(kt, K / 64 - kb);
+  // K-tiles of this part, and of them those of x and W
+  const int kb = blockIdx.y * kt, kw = min(kt, K / 64 - kb);
+  const int kn =
+      kw + (DOWN && lora.n > 0 && blockIdx.y + 1 == gridDim.y ? 1 : 0);
 
-  struct Place { int m0, n0; u32x4v rx, rw; };
+  struct Place { int m0, n0; u32x4v rx, rw; unsigned sx, sw; };
   auto place = [&](int at) {
     Place p;
     const int band = at / (8 * tn), in = at % (8 * tn);
     const int rows = min(8, tm - band * 8);
     p.m0 = (band * 8 + in % rows) * BM;
     p.n0 = first + in / rows * BN;
-    auto rsrc = [&](const uint16_t *base, int row, int rows) {
-      const uint64_t a = (uint64_t)(base + (int64_t)row * K);
-      u32x4v v;
-      v[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
-      v[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffff);
-      v[2] = __builtin_amdgcn_readfirstlane(
-          (uint32_t)rows * (uint32_t)K * 2);
-      v[3] = 0x00020000;
-      return v;
+    auto rows_of = [&](const uint16_t *base, int row, int rows) {
+      return buffer(base + (int64_t)row * K, (uint32_t)rows * (uint32_t)K * 2);
     };
-    p.rx = rsrc(x, p.m0, min(M - p.m0, BM));
-    p.rw = GLU ? rsrc(w, p.n0 / 2, N - p.n0 / 2)
-               : rsrc(w, p.n0, min(N - p.n0, BN));
+    p.rx = rows_of(x, p.m0, min(M - p.m0, BM));
+    if constexpr (!DOWN)
+      p.rw = GLU ? rows_of(w, p.n0 / 2, N - p.n0 / 2)
+                 : rows_of(w, p.n0, min(N - p.n0, BN));
     return p;
   };
   Place here = place(at);
 
   unsigned voff[LOADS];
+  auto row_of = [&](int i) { return (i * WAVES + wid) * 8 + (lane >> 3); };
+  auto offsets_x = [&] {
 #pragma unroll
-  for (int i = 0; i < LOADS; ++i) {
-    const int row = (i * WAVES + wid) * 8 + (lane >> 3);
-    const int c = (lane & 7) ^ ((row >> 1) & 7);
-    int from = i < XL ? row : row - BM;
-    if (GLU && i >= XL) {               // a wave's gates, then its units
-      const int in = from % (FN * 16);
-      from = from / (FN * 16) * (FN * 8) + in % (FN * 8) +
-             (in < FN * 8 ? 0 : N / 2);
+    for (int i = 0; i < XL; ++i)
+      voff[i] = (unsigned)row_of(i) * (unsigned)(K * 2) +
+                ((lane & 7) ^ ((row_of(i) >> 1) & 7)) * 16;
+  };
+  // DOWN: a wave's load is of 64 / PR rows of PR pieces
+  constexpr int PR = BN / 8;
+  auto down_row = [&](int i) {
+    return ((i - XL) * WAVES + wid) * (64 / PR) + lane / PR;
+  };
+  auto down_column = [&](int i) {
+    const int k = down_row(i);
+    return ((lane % PR) ^ ((k & 3) << 1 | (k >> 3 & 1) << 3)) * 8;
+  };
+  auto offsets_w = [&] {
+#pragma unroll
+    for (int i = XL; i < LOADS; ++i) {
+      if (DOWN) {
+        voff[i] = (unsigned)(down_row(i) * N + down_column(i)) * 2;
+        continue;
+      }
+      const int row = row_of(i), c = (lane & 7) ^ ((row >> 1) & 7);
+      int from = row - BM;
+      if (GLU) {                        // a wave's gates, then its units
+        const int in = from % (FN * 16);
+        from = from / (FN * 16) * (FN * 8) + in % (FN * 8) +
+               (in < FN * 8 ? 0 : N / 2);
+      }
+      voff[i] = (unsigned)from * (unsigned)(K * 2) + c * 16;
     }
-    voff[i] = (unsigned)from * (unsigned)(K * 2) + c * 16;
-  }
-  auto load = [&](const Place &p, int t, int b, int i) {
+  };
+  offsets_x();
+  offsets_w();
+  // What K-tile t of x and of W is loaded from: by its first column; W, DOWN, as a
+  // buffer of its rows, what is past them being past the buffer.
+  auto aim_x = [&](Place &p, int t) {
+    p.sx = (unsigned)(kb + t) * 128;
+    if constexpr (DOWN) {
+      if (t == kw) {
+        p.sx = 0;
+        p.rx = buffer(lora.t + (int64_t)p.m0 * 16,
+                      (uint32_t)(lora.n * M - p.m0) * 32);
+#pragma unroll
+        for (int i = 0; i < XL; ++i) {
+          const int row = row_of(i), c = (lane & 7) ^ ((row >> 1) & 7);
+          voff[i] = (c >> 1) < lora.n
+                        ? (unsigned)((c >> 1) * M + row) * 32 + (c & 1) * 16
+                        : NOWHERE;
+        }
+      } else if (t == 0) {
+        offsets_x();
+      }
+    }
+  };
+  auto aim_w = [&](Place &p, int t) {
+    p.sw = (unsigned)(kb + t) * 128;
+    if constexpr (DOWN) {
+      p.sw = 0;
+      p.rw = buffer(w + (int64_t)(kb + t) * 64 * N + p.n0,
+                    (uint32_t)(64 * N - p.n0) * 2);
+      if (t == kw) {
+        p.rw = buffer(lora.b[0], NOWHERE);
+#pragma unroll
+        for (int i = XL; i < LOADS; ++i) {
+          const int k = down_row(i), n = p.n0 + down_column(i), s = k >> 4;
+          // selects, no branches, which would cut the loop in pieces
+          const int from = ((s == 0) * lora.start[0] + (s == 1) * lora.start[1] +
+                            (s == 2) * lora.start[2] + (k & 15) * N + n) * 2;
+          const bool there = (s < lora.n) & (n < N);
+          voff[i] = there ? (unsigned)from : NOWHERE;
+        }
+      } else if (t == 0) {
+        offsets_w();
+      }
+    }
+  };
+  auto load = [&](const Place &p, int b, int i) {
     const unsigned at = (i * WAVES + wid) * 1024;
-    dma(i < XL ? p.rx : p.rw, voff[i], (unsigned)(kb + t) * 128,
-        i < XL ? b * XS + at : SX * XS + b * WS + at - XS);
+    if (i < XL)
+      dma(p.rx, voff[i], p.sx, b * XS + at);
+    else
+      dma(p.rw, voff[i], p.sw, SX * XS + b * WS + at - XS);
   };
   f32x4v acc[FM][FN];
   auto clear = [&] {
@@ -255,9 +350,18 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
   const int wa = SX * XS + (wn * FN * 16 + fr) * 128;
   const int c0 = (fk ^ sw) * 16, c1 = ((fk + 4) ^ sw) * 16;
   bf16x8v fx[2][FM], fw[2][FN];
+  // DOWN: this lane's 8 bytes of row 8 fk + fr / 4, by fragment
+  int dw[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j)
+    dw[j] = SX * XS + (fk * 8 + (fr >> 2)) * BN * 2 + (fr & 3) * 8 +
+            ((wn * FN + j) ^ (fr >> 2 | (fk & 1) << 2)) * 32;
   auto frag = [&](int set, int bx, int bw, int i) {
     const char *b = smem + (set ? c1 : c0);
-    if (i < FN)
+    if (DOWN && i < FN) {
+      const char *p = smem + (dw[i] + bw * WS) + set * 32 * BN * 2;
+      fw[set][i] = rb::lds_column8(p, p + 4 * BN * 2);
+    } else if (i < FN)
       fw[set][i] =
           *reinterpret_cast<const bf16x8v *>(b + bw * WS + wa + i * 2048);
     else
@@ -269,11 +373,15 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
                  : "memory");
   };
 #pragma unroll
-  for (int u = -SW; u < 0; ++u)
+  for (int u = -SW; u < 0; ++u) {
+    Place p = here;
+    aim_w(p, u + SW);
+    if (u + SX >= 0) aim_x(p, u + SX);
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
-      if (i >= XL) load(here, u + SW, u + SW, i);
-      else if (u + SX >= 0) load(here, u + SX, u + SX, i);
+      if (i >= XL) load(p, u + SW, i);
+      else if (u + SX >= 0) load(p, u + SX, i);
+  }
   constexpr int AHEAD = (SX - 2) * LOADS + (SW > SX ? WL : 0);
   wait(std::integral_constant<int, AHEAD + LOADS>());
 #pragma unroll
@@ -300,8 +408,12 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
       Place p;                        // of the K-tiles that are fetched now
       p.rx = t + SX < kn ? here.rx : next.rx;
       p.rw = t + SW < kn ? here.rw : next.rw;
+      p.m0 = t + SX < kn ? here.m0 : next.m0;
+      p.n0 = t + SW < kn ? here.n0 : next.n0;
       const int tx = t + SX < kn ? t + SX : t + SX - kn;
       const int tw = t + SW < kn ? t + SW : t + SW - kn;
+      aim_x(p, tx);
+      aim_w(p, tw);
 #pragma unroll
       for (int set = 0; set < 2; ++set)
 #pragma unroll
@@ -319,13 +431,13 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
               frag(0, nx, nw, (q - B2 - 1) / R2);
             if (q >= B1 && (q - B1) % D == 0 && (q - B1) / D < LOADS) {
               const int l = (q - B1) / D;
-              load(p, l < XL ? tx : tw, l < XL ? bx : bw, l);
+              load(p, l < XL ? bx : bw, l);
             }
             __builtin_amdgcn_sched_barrier(0);
           }
       bx = nx;
       bw = nw;
-      settle(kn - 1 - t);
+      settle(__builtin_amdgcn_readfirstlane(kn - 1 - t));
     }
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (KIND == LORA)
@@ -448,17 +560,66 @@ Choice choose_two(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
-template <int BM, int BN, int SX, int SW, Kind KIND>
+// The same for W [K, N], in a fine-tune's steps, whose products keep the chip so
+// busy that it lowers its clock (2.4 GHz to 1.7): a K-tile takes `few` us where up
+// to half of the CUs have a workgroup, `all` where each has one. Fitted to 64 to
+// 8192 rows. Parts are added up by a launch of their own.
+struct DownTile { double few, all; };
+constexpr DownTile DOWN_TILES[N_TILES] = {{1.29, 1.54}, {1.09, 1.24}, {}, {.79, .91},
+                                          {.83, .94}, {}, {.57, .585}};
+
+double down_us(int v, int64_t M, int64_t N, int64_t K, int p) {
+  const Tile &t = TILES[v];
+  const int64_t n = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn) * p;
+  const int64_t rounds = (n + 255) / 256;
+  const double fill = (double)n / (rounds * 256);
+  const DownTile &d = DOWN_TILES[v];
+  const double step = d.few + (d.all - d.few) * std::max(0.0, 2 * fill - 1);
+  const double us = rounds * (double)((K / 64 + p - 1) / p + 1) * step +
+                    t.rest * (1 + 0.3 * (rounds - 1));
+  return p == 1 ? us : us + M * N * (p * 8 + 2) / 5e6 + 5.0;
+}
+
+Choice choose_down(int64_t M, int64_t N, int64_t K, int max_parts, int only) {
+  Choice best;
+  auto all = [&](int64_t cols, int most, auto &&take) {
+    for (int v = 0; v < N_TILES; ++v) {
+      if (TILES[v].bn == 192 || (only >= 0 && v != only)) continue;
+      for (int p = 1; p <= most; ++p)
+        if (divides(K, p)) take(v, p, down_us(v, M, cols, K, p));
+    }
+  };
+  all(N, max_parts, [&](int v, int p, double us) {
+    if (us < best.us) best = {v, p, -1, 0, us};
+  });
+  if (only >= 0) return best;
+  // whole rounds of a tile, and the rest in a launch of its own
+  all(N, 1, [&](int v, int, double) {
+    const Tile &t = TILES[v];
+    const int64_t tm = (M + t.bm - 1) / t.bm, tn = (N + t.bn - 1) / t.bn;
+    const int64_t cols = tm * tn / 256 * 256 / tm;
+    if (cols == 0 || cols >= tn) return;
+    const double first = down_us(v, M, cols * t.bn, K, 1);
+    all(N - cols * t.bn, 1, [&](int r, int, double us) {
+      if (first + us + 3 < best.us)
+        best = {v, 1, r, cols * t.bn, first + us + 3};
+    });
+  });
+  return best;
+}
+
+template <int BM, int BN, int SX, int SW, Kind KIND, bool DOWN>
 void launch(const at::Tensor &x, const at::Tensor &w, at::Tensor &y, int parts,
             int64_t first, int64_t last, const tiles::Adapters &lora) {
-  auto kernel = tiles::gemm_tiles_kernel<BM, BN, 2, 2, SX, SW, KIND>;
+  auto kernel = tiles::gemm_tiles_kernel<BM, BN, 2, 2, SX, SW, KIND, DOWN>;
   constexpr int lds = (SX * BM + SW * BN) * 128;
   static const bool once =
       hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds) ==
       hipSuccess;
   TORCH_CHECK(once, "tile_gemm: LDS size");
-  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
+  const int M = (int)x.size(0), K = (int)x.size(1);
+  const int N = (int)w.size(DOWN ? 1 : 0);
   const int tm = (M + BM - 1) / BM, tn = (int)((last - first + BN - 1) / BN);
   const int kt = (K / 64 + parts - 1) / parts;
   hipLaunchKernelGGL(kernel, dim3(std::min(tm * tn, 256), parts), dim3(256),
@@ -469,19 +630,29 @@ void launch(const at::Tensor &x, const at::Tensor &w, at::Tensor &y, int parts,
   C10_CUDA_KERNEL_LAUNCH_CHECK();
 }
 
-template <Kind KIND>
+template <Kind KIND, bool DOWN = false>
 void run(int tile, const at::Tensor &x, const at::Tensor &w, at::Tensor &y,
          int parts, int64_t first, int64_t last,
          const tiles::Adapters &lora = {}) {
+  auto go = [&](auto bm, auto bn, auto sx, auto sw) {
+    if constexpr (!DOWN || bn() != 192)
+      launch<bm(), bn(), sx(), sw(), KIND, DOWN>(x, w, y, parts, first, last,
+                                                 lora);
+  };
+  using std::integral_constant;
+#define TILE(bm, bn, sx, sw)                                             \
+  return go(integral_constant<int, bm>(), integral_constant<int, bn>(), \
+            integral_constant<int, sx>(), integral_constant<int, sw>())
   switch (tile) {
-    case 0: return launch<256, 256, 2, 2, KIND>(x, w, y, parts, first, last, lora);
-    case 1: return launch<192, 256, 2, 2, KIND>(x, w, y, parts, first, last, lora);
-    case 2: return launch<256, 192, 2, 2, KIND>(x, w, y, parts, first, last, lora);
-    case 3: return launch<256, 128, 3, 3, KIND>(x, w, y, parts, first, last, lora);
-    case 4: return launch<128, 256, 2, 3, KIND>(x, w, y, parts, first, last, lora);
-    case 5: return launch<128, 192, 3, 4, KIND>(x, w, y, parts, first, last, lora);
-    default: return launch<128, 128, 3, 4, KIND>(x, w, y, parts, first, last, lora);
+    case 0: TILE(256, 256, 2, 2);
+    case 1: TILE(192, 256, 2, 2);
+    case 2: TILE(256, 192, 2, 2);
+    case 3: TILE(256, 128, 3, 3);
+    case 4: TILE(128, 256, 2, 3);
+    case 5: TILE(128, 192, 3, 4);
+    default: TILE(128, 128, 3, 4);
   }
+#undef TILE
 }
 
 bool fits(const at::Tensor &t) {
@@ -551,30 +722,46 @@ at::Tensor tile_gemm(at::Tensor x, at::Tensor w, int64_t max_parts, int64_t glu,
   return y;
 }
 
+// Adapters of rank 16 as the tiles read them: t [n, M, 16], and matrices whose
+// dimension `wide` is 16.
+static tiles::Adapters tile_adapters(const at::Tensor &x, const at::Tensor &t,
+                                     const std::vector<at::Tensor> &ms,
+                                     int wide) {
+  tiles::Adapters a{};
+  a.n = (int)ms.size();
+  a.scale = 1.0f;
+  TORCH_CHECK(a.n <= 3, "tiles: at most 3 adapters");
+  auto adapter = [&](const at::Tensor &m, int d) {
+    TORCH_CHECK(m.is_contiguous() && m.device() == x.device() &&
+                m.scalar_type() == at::kBFloat16 && m.size(d) == 16 &&
+                reinterpret_cast<uintptr_t>(m.data_ptr()) % 16 == 0,
+                "tiles: adapters of rank 16, bf16");
+    return (const uint16_t *)m.data_ptr();
+  };
+  if (a.n == 0) return a;
+  TORCH_CHECK(t.dim() == 3 && t.size(0) == a.n && t.size(1) == x.size(0) &&
+              a.n * t.size(1) * 32 < (int64_t)tiles::NOWHERE,
+              "tiles: t [n, M, 16]");
+  a.t = adapter(t, 2);
+  for (int i = 0; i < a.n; ++i) {
+    TORCH_CHECK(ms[i].dim() == 2, "tiles: adapters' matrices");
+    a.b[i] = adapter(ms[i], wide);
+  }
+  return a;
+}
+
 // x W^T + scale t_i B_i^T of one to three siblings side by side: t [n, M, 16], B_i
 // [columns of i, 16].
 at::Tensor tile_lora(at::Tensor x, at::Tensor w, at::Tensor t,
                      std::vector<at::Tensor> bs, double scale, int64_t tile) {
   const int64_t M = x.size(0), N = w.size(0);
-  tiles::Adapters a{};
-  a.n = (int)bs.size();
-  TORCH_CHECK(tile_gemm_takes(x, w, false) && tile < N_TILES && a.n >= 1 &&
-              a.n <= 3, "tile_lora: x ", x.sizes(), ", W ", w.sizes());
-  auto adapter = [&](const at::Tensor &m) {
-    TORCH_CHECK(m.is_contiguous() && m.device() == x.device() &&
-                m.scalar_type() == at::kBFloat16 && m.size(-1) == 16 &&
-                reinterpret_cast<uintptr_t>(m.data_ptr()) % 16 == 0,
-                "tile_lora: adapters of rank 16, bf16");
-    return (const uint16_t *)m.data_ptr();
-  };
-  TORCH_CHECK(t.dim() == 3 && t.size(0) == a.n && t.size(1) == M,
-              "tile_lora: t [n, M, 16]");
-  a.t = adapter(t);
+  TORCH_CHECK(tile_gemm_takes(x, w, false) && tile < N_TILES && !bs.empty(),
+              "tile_lora: x ", x.sizes(), ", W ", w.sizes());
+  tiles::Adapters a = tile_adapters(x, t, bs, 1);
   int64_t at = 0;
   for (int i = 0; i < a.n; ++i) {
-    TORCH_CHECK(bs[i].dim() == 2 && bs[i].size(0) % 16 == 0 &&
-                bs[i].size(0) > 0, "tile_lora: columns");
-    a.b[i] = adapter(bs[i]);
+    TORCH_CHECK(bs[i].size(0) % 16 == 0 && bs[i].size(0) > 0,
+                "tile_lora: columns");
     a.start[i] = (int)at;
     at += bs[i].size(0);
   }
@@ -588,6 +775,88 @@ at::Tensor tile_lora(at::Tensor x, at::Tensor w, at::Tensor t,
     run<tiles::LORA>(c.rest, x, w, y, 1, c.split, N, a);
   } else {
     run<tiles::LORA>(c.tile, x, w, y, 1, 0, N, a);
+  }
+  return y;
+}
+
+// Whether tile_gemm_down takes x [M, K] and W [K, N].
+bool tile_gemm_down_takes(at::Tensor x, at::Tensor w) {
+  return fits(x) && fits(w) && x.size(1) == w.size(0) &&
+         x.device() == w.device() && x.size(1) % 64 == 0 &&
+         x.size(1) >= 256 && x.size(1) <= (1 << 20) && w.size(1) % 8 == 0 &&
+         w.size(1) < (1 << 22);
+}
+
+// Whether tile_gemm_down, with the parts' sum, is as good as the library and a pass
+// for the adapters. It is not where one launch leaves CUs idle, of sums that are not
+// much longer than the result is wide: there the library splits them (us there and
+// here: 12288 to 4096 columns, 2500 rows 213 and 238; 4096 to 4096, 1100 rows 51 and
+// 56; 5632 to 2048, 2500 rows 68 and 75; 8192 to 8192, 1100 rows 139 and 148). Of 295
+// other sizes, 33 to 8192 rows of 2048 to 57344 columns, 14 are slower, by 3 to 6%
+// and one by 12 (300 rows, 4096 to 11008, 53 and 59), the mean is 0.78: 12288 to 4096,
+// 300 rows 118 and 56, 2048 198 and 172; 22016 to 4096, 512 rows 202 and 99, 2048 359
+// and 297, 3001 428 and 431; 4096 to 11008, 2048 rows 179 and 168; 4096 to 14336, 3001
+// rows 317 and 292.
+bool tile_gemm_down_pays(int64_t M, int64_t N, int64_t K) {
+  if (M <= 32) return false;            // a few rows were not measured
+  const Choice c = choose_down(M, N, K, MAX_PARTS, -1);
+  if (c.tile < 0) return false;
+  const Tile &t = TILES[c.tile];
+  const int64_t tiles = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn);
+  const int64_t rounds = (tiles + 255) / 256;
+  return !(M >= 1024 && c.parts == 1 && c.rest < 0 && tiles * 10 < rounds * 2304 &&
+           N <= K && (N <= 4096 || K < 2 * N));
+}
+
+std::vector<int64_t> tile_gemm_down_choice(int64_t M, int64_t N, int64_t K,
+                                           int64_t max_parts) {
+  const Choice c = choose_down(M, N, K, (int)max_parts, -1);
+  return {c.tile, c.parts, c.rest, c.split};
+}
+
+// x W + sum_i t_i A_i, W [K, N] and up to three adapters A_i [16, N], t [n, M, 16]:
+// bf16 [M, N], or, where max_parts > 1, possibly fp32 parts [P, M, N] of the sums.
+at::Tensor tile_gemm_down(at::Tensor x, at::Tensor w, at::Tensor t,
+                          std::vector<at::Tensor> as, int64_t max_parts,
+                          int64_t tile, int64_t parts) {
+  TORCH_CHECK(tile_gemm_down_takes(x, w) && tile < N_TILES &&
+              max_parts >= 1 && max_parts <= MAX_PARTS && parts <= MAX_PARTS &&
+              (tile < 0 || TILES[tile].bn != 192),
+              "tile_gemm_down: x ", x.sizes(), ", W ", w.sizes());
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(1);
+  tiles::Adapters a = tile_adapters(x, t, as, 0);
+  for (const auto &m : as)
+    TORCH_CHECK(m.size(1) == N, "tile_gemm_down: columns of A");
+  // the kernel reads all A_i from the first in memory on, within 2 GiB
+  at::Tensor near;
+  if (a.n > 1) {
+    int order[3] = {0, 1, 2};
+    std::sort(order, order + a.n,
+              [&](int i, int j) { return a.b[i] < a.b[j]; });
+    if (a.b[order[a.n - 1]] + 16 * N - a.b[order[0]] >= (1 << 30)) {
+      near = at::cat(as);
+      for (int i = 0; i < a.n; ++i)
+        a.b[i] = (const uint16_t *)near.data_ptr() + i * 16 * N;
+      order[0] = 0;
+    }
+    const uint16_t *base = a.b[order[0]];
+    for (int i = 0; i < a.n; ++i) a.start[i] = (int)(a.b[i] - base);
+    a.b[0] = base;
+  }
+  Choice c = choose_down(M, N, K, (int)max_parts, (int)tile);
+  if (parts > 0) c.parts = (int)parts;
+  TORCH_CHECK(divides(K, c.parts), "tile_gemm_down: parts");
+  if (c.parts > 1) {
+    auto y = at::empty({c.parts, M, N}, x.options().dtype(at::kFloat));
+    run<tiles::PARTS, true>(c.tile, x, w, y, c.parts, 0, N, a);
+    return y;
+  }
+  auto y = at::empty({M, N}, x.options());
+  if (c.split > 0) {
+    run<tiles::PLAIN, true>(c.tile, x, w, y, 1, 0, c.split, a);
+    run<tiles::PLAIN, true>(c.rest, x, w, y, 1, c.split, N, a);
+  } else {
+    run<tiles::PLAIN, true>(c.tile, x, w, y, 1, 0, N, a);
   }
   return y;
 }

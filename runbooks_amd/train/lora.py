@@ -6,9 +6,9 @@ is native: frozen base weights, trainable low-rank A/B pairs on the
 attention + MLP projections. Three ways, by what a layer is:
 
 * rank 16, bf16, no bias, on the GPU (_LoRAPacked): siblings that share
-  their input side by side, one library product with the frozen weights
-  each way, the adapters' products on kernels of csrc/lora_group.hip that
-  read x, y and dy once for all of them;
+  their input side by side, one product with the frozen weights each way
+  (csrc/gemm_tiles.hip), the adapters' other products on kernels of
+  csrc/lora_group.hip that read x, y and dy once for all of them;
 * other layers without bias (_LoRAFused, _LoRAFusedT): library products,
   both gradient merges in place (the eager formulation measured ~450 extra
   elementwise launches per llama2-7b step);
@@ -226,8 +226,8 @@ class _LoRAFused(torch.autograd.Function):
 class _LoRAPacked(torch.autograd.Function):
     """y = x W^T + s (x A_i^T) B_i^T for siblings side by side (W and y by
     columns), or for one adapter: one product with the frozen weights each way,
-    and the adapters' products on kernels that read x, y and dy once for all of
-    them (csrc/lora_group.hip)."""
+    which the adapters' end, and their other products on kernels that read x and dy
+    once for all of them (csrc/lora_group.hip)."""
 
     @staticmethod
     def forward(ctx, x, w, scale, n, *ab):
@@ -252,8 +252,7 @@ class _LoRAPacked(torch.autograd.Function):
         da = ext.lora_grad(x, dt, [], 1.0, True).chunk(n)
         dx = None
         if ctx.needs_input_grad[0]:
-            dx = wide_product_grad(dy, w)
-            ext.lora_add_(dx, dt, As, 1.0, True)
+            dx = wide_product_grad(dy, w, dt, As)
         return (dx, None, None, None, *da, *db)
 
 

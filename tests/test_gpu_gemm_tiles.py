@@ -243,6 +243,145 @@ def test_sums_for_the_norm(m, n, k, parts):
     assert ops.rows_parts(x, w) is None         # would be differentiated
 
 
+def _down_inputs(m, n, k, siblings, apart=False):
+    """x [m, k], W [k, n], t and A of siblings, one after the other in memory
+    or, `apart`, further from each other than 2 GiB."""
+    x, w = _inputs(m, n, k)
+    t = torch.randn(siblings, m, 16, device="cuda").bfloat16()
+    if apart:
+        room = torch.empty((1 << 30) + 4 * 16 * n, device="cuda",
+                           dtype=torch.bfloat16)
+        As = [room[-16 * n:].view(16, n), room[:16 * n].view(16, n)][:siblings]
+        for a in As:
+            a.normal_()
+    else:
+        As = [torch.randn(16, n, device="cuda").bfloat16()
+              for _ in range(siblings)]
+    return x, w.t().contiguous(), t, As
+
+
+def _check_down(got, x, w, t, As, rounding):
+    """fp32 sums of k + 16 n products in any order, and their rounding."""
+    ref = x.double() @ w.double()
+    size = x.abs().double() @ w.abs().double()
+    for ti, a in zip(t, As):
+        ref += ti.double() @ a.double()
+        size += ti.abs().double() @ a.abs().double()
+    bound = rounding * ref.abs() + \
+        2 * (x.shape[1] + 16 * len(As)) * 2.0 ** -24 * size
+    assert bool(((got.double() - ref).abs() <= bound).all())
+
+
+DOWN_TILES = [0, 1, 3, 4, 6]            # of 128 and 256 columns
+
+
+@pytest.mark.parametrize("tile", DOWN_TILES)
+@pytest.mark.parametrize("m,n,k,siblings", [
+    (1, 8, 256, 0),             # less than a fragment, the fewest rows of W
+    (129, 264, 320, 1),         # remainders of every tile, odd K-tiles
+    (256, 512, 512, 2),         # whole tiles
+    (513, 1032, 448, 3),
+    (4100, 4360, 256, 3)])      # several tiles for a workgroup
+def test_product_down_columns(tile, m, n, k, siblings):
+    from runbooks_amd import ops
+    args = _down_inputs(m, n, k, siblings)
+    _check_down(ops.ext().tile_gemm_down(*args, tile=tile), *args, 2.0 ** -8)
+
+
+@pytest.mark.parametrize("tile", DOWN_TILES)
+@pytest.mark.parametrize("m,n,k,siblings,parts", [
+    (130, 520, 1024, 1, 4), (300, 264, 576, 3, 2), (257, 4104, 1472, 0, 3)])
+def test_parts_down_columns(tile, m, n, k, siblings, parts):
+    """The adapters go with the last part, once."""
+    from runbooks_amd import ops
+    args = _down_inputs(m, n, k, siblings)
+    y = ops.ext().tile_gemm_down(*args, max_parts=parts, tile=tile, parts=parts)
+    assert y.shape == (parts, m, n) and y.dtype == torch.float32
+    _check_down(y.double().sum(0), *args, 2.0 ** -24)
+
+
+def test_adapters_apart_in_memory():
+    from runbooks_amd import ops
+    args = _down_inputs(200, 512, 256, 2, apart=True)
+    _check_down(ops.ext().tile_gemm_down(*args), *args, 2.0 ** -8)
+
+
+def test_two_launches_down_columns():
+    from runbooks_amd import ops
+    m, n, k = 3001, 14336, 4096
+    _, parts, rest, split = ops.ext().tile_gemm_down_choice(m, n, k, 4)
+    assert parts == 1 and rest >= 0 and 0 < split < n
+    args = _down_inputs(m, n, k, 1)
+    _check_down(ops.ext().tile_gemm_down(*args), *args, 2.0 ** -8)
+
+
+def test_infinite_values_stay_in_their_row_and_column():
+    """Absent siblings and columns past the end are zeros times zeros."""
+    from runbooks_amd import ops
+    x, w, t, As = _down_inputs(300, 520, 512, 1)
+    clean = ops.ext().tile_gemm_down(x, w, t, As)
+    t[0, 7, 3] = float("inf")
+    As[0][5, 11] = float("-inf")
+    w[:, 519] = float("nan")
+    got = ops.ext().tile_gemm_down(x, w, t, As)
+    rows = [i for i in range(300) if i != 7]
+    cols = [i for i in range(519) if i != 11]
+    assert torch.equal(got[rows][:, cols], clean[rows][:, cols])
+    assert not bool(got[:, 11].isfinite().any() | got[7, :519].isfinite().any())
+    assert bool(got[:, 519].isnan().all())
+
+
+@pytest.mark.parametrize("m,n,k,siblings,tiles", [
+    (2048, 4096, 1024, 1, True), (300, 4096, 6144, 3, True),
+    (1100, 4096, 4096, 1, False), (77, 64, 192, 2, False)])
+def test_gradients_of_inputs(monkeypatch, m, n, k, siblings, tiles):
+    """Both ways that wide_product_grad may take, by its own rule and, where
+    the tiles take it, against it: the library's rounds the product and the
+    sum."""
+    from runbooks_amd import ops
+    from runbooks_amd.ops import linear
+    x, w, t, As = _down_inputs(m, n, k, siblings)
+    ext = ops.ext()
+    taken = ext.tile_gemm_down_takes(x, w)
+    assert (taken and ext.tile_gemm_down_pays(m, n, k)) is tiles
+    called = []
+    monkeypatch.setattr(linear, "_library_grad",
+                        lambda *a, f=linear._library_grad: called.append(1) or
+                        f(*a))
+    got = linear.wide_product_grad(x, w, t, As)
+    assert (not called) is tiles
+    other = ext.tile_gemm_down(x, w, t, As) if taken and not tiles else \
+        linear._library_grad(x, w)
+    if tiles or not taken:
+        ext.lora_add_(other, t, As, 1.0, True)
+    product = 2.0 ** -8 * (x.double() @ w.double()).abs().max()
+    for y in (got, other):
+        ref = x.double() @ w.double() + sum(
+            ti.double() @ a.double() for ti, a in zip(t, As))
+        bound = 2.0 ** -8 * ref.abs() + product + 1e-4
+        assert bool(((y.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("change", ["rows", "columns", "aligned", "type", "rank"])
+def test_refused_down_columns(change):
+    from runbooks_amd import ops
+    x, w, t, As = _down_inputs(200, 512, 320, 1)
+    if change == "rows":
+        x, w = x[:, :300].contiguous(), w[:300]
+    elif change == "columns":
+        w = w[:, :508].contiguous()
+    elif change == "aligned":
+        x = torch.zeros(200 * 320 + 1, device="cuda",
+                        dtype=torch.bfloat16)[1:].view(200, 320)
+    elif change == "type":
+        x, w = x.float(), w.float()
+    else:
+        t = t[:, :, :8].contiguous()
+    assert ops.ext().tile_gemm_down_takes(x, w) is (change == "rank")
+    with pytest.raises(RuntimeError):
+        ops.ext().tile_gemm_down(x, w, t, As)
+
+
 def test_one_row_does_not_reach_others():
     """An infinite and a NaN row stay to themselves."""
     from runbooks_amd import ops

@@ -46,6 +46,9 @@ at::Tensor lora_down_columns(at::Tensor dy, std::vector<at::Tensor> bs,
                              double scale);
 void lora_add_(at::Tensor y, at::Tensor t, std::vector<at::Tensor> ms,
                double scale, bool sum);
+std::vector<at::Tensor> lora_grads(at::Tensor dy, at::Tensor t, at::Tensor x,
+                                   at::Tensor dt, std::vector<int64_t> widths,
+                                   double scale);
 at::Tensor lora_grad(at::Tensor x, at::Tensor t, std::vector<int64_t> widths,
                      double scale, bool transposed);
 at::Tensor flash_prefill_qkv(at::Tensor y, int64_t B, int64_t S, int64_t Hq,
@@ -124,6 +127,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("lora_add_", &lora_add_,
         "y_i += scale t_i B_i^T, or y += scale sum t_i A_i");
   m.def("lora_grad", &lora_grad, "scale x_i^T t_i, or scale t_i^T x");
+  m.def("lora_grads", &lora_grads, "scale dy_i^T t_i, and dt_i^T x");
   m.def("flash_prefill_qkv", &flash_prefill_qkv,
         "flash_prefill of q, k and v side by side in one tensor");
   m.def("qkv_rope_append_", &qkv_rope_append_,

@@ -292,6 +292,28 @@ RB_DEV __attribute__((ext_vector_type(8))) __bf16 lds_column8(const char *lo,
   return r.v;
 }
 
+typedef __attribute__((ext_vector_type(4))) unsigned int u32x4v;
+
+// `bytes` from p on, a buffer whose loads past the end give zeros.
+RB_DEV u32x4v buffer(const uint16_t *p, uint32_t bytes) {
+  const uint64_t a = (uint64_t)p;
+  u32x4v v;
+  v[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
+  v[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffff);
+  v[2] = __builtin_amdgcn_readfirstlane(bytes);
+  v[3] = 0x00020000;
+  return v;
+}
+
+// 16 bytes a lane from a buffer to LDS at lds + lane * 16, past the registers.
+// As text, for the compiler waits for all such loads before it reads LDS again.
+RB_DEV void lds_load(u32x4v from, unsigned voff, unsigned soff, unsigned lds) {
+  asm volatile(
+      "s_mov_b32 m0, %3\n\ts_nop 0\n\t"
+      "buffer_load_dwordx4 %0, %1, %2 offen lds"
+      :: "v"(voff), "s"(from), "s"(soff), "s"(lds) : "memory", "m0");
+}
+
 // two floats -> packed bf16 words (round to nearest even)
 RB_DEV uint32_t pack_bf16x2(float lo, float hi) {
   return f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);

@@ -29,22 +29,13 @@ namespace tiles {
 
 using ends::bf16x8v;
 using ends::f32x4v;
-using ends::u32x4v;
+using rb::buffer;
+using rb::u32x4v;
 
 __device__ __forceinline__ void put(uint16_t *p, const float (&f)[4]) {
   typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4v;
   *reinterpret_cast<bf16x4v *>(p) =
       __builtin_convertvector((f32x4v){f[0], f[1], f[2], f[3]}, bf16x4v);
-}
-
-// 16 bytes a lane to LDS at lds + lane * 16, past the registers. As text, for
-// the compiler waits for all such loads before it reads LDS again.
-__device__ __forceinline__ void dma(u32x4v rsrc, unsigned voff, unsigned soff,
-                                    unsigned lds) {
-  asm volatile(
-      "s_mov_b32 m0, %3\n\ts_nop 0\n\t"
-      "buffer_load_dwordx4 %0, %1, %2 offen lds"
-      :: "v"(voff), "s"(rsrc), "s"(soff), "s"(lds) : "memory", "m0");
 }
 
 // As text, for the compiler copies sums between the register files otherwise.
@@ -82,16 +73,6 @@ __device__ __forceinline__ int sibling(const Adapters &a, int n) {
   return (a.n > 1 && n >= a.start[1]) + (a.n > 2 && n >= a.start[2]);
 }
 
-// `bytes` from p on, a buffer whose loads past the end give zeros.
-__device__ __forceinline__ u32x4v buffer(const uint16_t *p, uint32_t bytes) {
-  const uint64_t a = (uint64_t)p;
-  u32x4v v;
-  v[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
-  v[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffff);
-  v[2] = __builtin_amdgcn_readfirstlane(bytes);
-  v[3] = 0x00020000;
-  return v;
-}
 constexpr unsigned NOWHERE = 0x80000000;    // past the end of every such buffer
 
 // Waits until the last products are in their registers, if `left` is 0. The
@@ -332,9 +313,9 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
   auto load = [&](const Place &p, int b, int i) {
     const unsigned at = (i * WAVES + wid) * 1024;
     if (i < XL)
-      dma(p.rx, voff[i], p.sx, b * XS + at);
+      rb::lds_load(p.rx, voff[i], p.sx, b * XS + at);
     else
-      dma(p.rw, voff[i], p.sw, SX * XS + b * WS + at - XS);
+      rb::lds_load(p.rw, voff[i], p.sw, SX * XS + b * WS + at - XS);
   };
   f32x4v acc[FM][FN];
   auto clear = [&] {

@@ -248,8 +248,8 @@ class _LoRAPacked(torch.autograd.Function):
             dy = dy.clone()
         widths = [b.shape[0] for b in Bs]
         dt = ext.lora_down_columns(dy, Bs, ctx.scale)
-        db = ext.lora_grad(dy, t, widths, ctx.scale, False).split(widths)
-        da = ext.lora_grad(x, dt, [], 1.0, True).chunk(n)
+        db, da = ext.lora_grads(dy, t, x, dt, widths, ctx.scale)
+        db, da = db.split(widths), da.chunk(n)
         dx = None
         if ctx.needs_input_grad[0]:
             dx = wide_product_grad(dy, w, dt, As)

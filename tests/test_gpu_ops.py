@@ -1205,6 +1205,33 @@ def test_lora_siblings(T, K, widths):
           torch.cat([d.t() @ xd for d in dtd]))
 
 
+@pytest.mark.parametrize("T", [1, 17, 130])
+@pytest.mark.parametrize("K,widths", [
+    (1088, (1088,)),            # a last chunk by itself, waves without one
+    (2048, (2112, 64)),         # as many chunks as are fetched ahead
+    (8256, (4160, 64, 1024))])  # many turns
+def test_lora_siblings_long(T, K, widths):
+    """Sums over more columns than all waves fetch at a time, and both gradients
+    in one launch, which are the same as each by itself."""
+    _assert_hip()
+    ext = ops.ext()
+    torch.manual_seed(T + K)
+    x, *A = (torch.randn(n, K, device=DEV).bfloat16()
+             for n in (T, *[16] * len(widths)))
+    B = [torch.randn(n, 16, device=DEV).bfloat16() for n in widths]
+    y = torch.randn(T, sum(widths), device=DEV).bfloat16()
+    t, dt = ext.lora_down(x, A), ext.lora_down_columns(y, B, 2.0)
+    # fp32 sums and one rounding
+    for got, ref in ((t, [x.double() @ a.double().t() for a in A]),
+                     (dt, [2 * v.double() @ b.double() for v, b in
+                           zip(y.split(widths, 1), B)])):
+        ref = torch.stack(ref)
+        assert (got.double() - ref).norm() < 2 ** -8 * ref.norm()
+    db, da = ext.lora_grads(y, t, x, dt, list(widths), 2.0)
+    assert torch.equal(db, ext.lora_grad(y, t, list(widths), 2.0, False))
+    assert torch.equal(da, ext.lora_grad(x, dt, [], 1.0, True))
+
+
 @pytest.mark.parametrize("heads,kv,dh,B,S", [(4, 4, 64, 2, 33),
                                              (4, 1, 128, 1, 100),
                                              (6, 2, 64, 3, 1)])

@@ -69,14 +69,57 @@ RB_DEV void store_operand(uint16_t *swz, int kk0, int b, const float (&v)[VE],
   }
 }
 
-// The sequence of a workgroup. Workgroups 256 apart in launch order share a CU;
-// in plain order those would be heads of one sequence wherever the batch divides
-// 256, and the CUs of the longest ones would run long after the others. The
-// sequences are shifted with head and split, once around over the whole grid:
+// What a workgroup of a grid (B, Hkv, splits) takes. Workgroups 256 apart in launch
+// order share a CU; in plain order those would be heads of one sequence wherever
+// the batch divides 256, and the CUs of the longest ones would run long after the
+// others.
+struct Place { int b, h, split; };
+
+// The sequences are shifted with head and split, once around over the whole grid:
 // a CU gets sequences spread evenly over the batch.
-RB_DEV int sequence_of() {
+RB_DEV Place shifted_place() {
   const unsigned y = blockIdx.y + gridDim.y * blockIdx.z;
-  return (blockIdx.x + y * gridDim.x / (gridDim.y * gridDim.z)) % gridDim.x;
+  const unsigned b =
+      (blockIdx.x + y * gridDim.x / (gridDim.y * gridDim.z)) % gridDim.x;
+  return {(int)b, (int)blockIdx.y, (int)blockIdx.z};
+}
+
+// The longest sequences first, so that none is begun late, and every other 256
+// workgroups the other way round, so that a CU that has a long one gets a short one
+// with it. Up to 64 sequences, whose lengths one wave compares for all (B steps of
+// three instructions; all waves of a CU together took 0.8 us).
+//
+// us by shifts and sorted, 32 heads of 128: 32 sequences of 129 to 2015 tokens 108
+// and 101 (5.6 TB/s), 16 of 800 to 3900 in e4m3 76 and 69, 64 of 100 to 1200 133 and
+// 124, 32 of 1072 each 104 and 104; 8 kv heads of 128 with four queries each: 64 of
+// 1000 to 4003 128 and 118 (5.7 TB/s), 32 of 100 to 4000 in two parts 61 and 55; 16
+// heads of 256: 7 of 90 to 1801 in parts 32.4 and 29.1, 16 of 100 to 2000 60 and 57.
+// Where nothing is uneven it costs 0.2 to 0.4 us (32 of 100 with a table of 4096
+// 14.0 and 14.2, 8 of 400 18.0 and 18.2), so tables of up to 512 tokens go by shifts.
+RB_DEV Place sorted_place(const int32_t *lens, const int32_t *starts) {
+  __shared__ int found;
+  const int B = gridDim.x, hkv = gridDim.y, of_each = hkv * gridDim.z;
+  const int all = B * of_each;
+  const int id = blockIdx.x + B * (blockIdx.y + hkv * blockIdx.z);
+  const int round = id & ~255;
+  const int at = id & 256 ? round + min(256, all - round) - 1 - (id & 255) : id;
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    int key = -1;                       // all of them different
+    if (lane < B)
+      key = max(0, lens[lane] - (starts ? starts[lane] : 0)) * 64 + lane;
+    int longer = 0;
+#pragma unroll
+    for (int i0 = 0; i0 < 64; i0 += 8)
+      if (i0 < B)
+#pragma unroll
+        for (int i = i0; i < i0 + 8; ++i)
+          longer += __builtin_amdgcn_readlane(key, i) > key;
+    if (lane < B && longer == at / of_each) found = lane;
+  }
+  __syncthreads();
+  const int rest = at % of_each;
+  return {found, rest % hkv, rest / hkv};
 }
 
 // FP8: caches are e4m3 rows of fp8_row_bytes(DH) = DH bytes + f32
@@ -93,7 +136,7 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
     const int32_t *__restrict__ seq_starts, uint16_t *__restrict__ out,
     uint16_t *__restrict__ out_swz,
     float *__restrict__ partial, int hkv, int bs, int max_blocks, int nsplit,
-    float scale) {
+    float scale, bool sorted) {
   // Lane-group geometry: GL lanes cover one token's Dh. bf16 reads 2 B
   // per element, so 16 lanes x VE=DH/16 elems = 16 B/lane; fp8 reads
   // 1 B per element, so 8-lane groups with VE=DH/8 keep the loads at
@@ -113,9 +156,9 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
   // iteration, and removes the cross-wave LDS merge entirely.
   constexpr bool HS = (G >= NW);
   constexpr int GW = HS ? G / NW : G;
-  const int b = sequence_of();
-  const int h_kv = blockIdx.y;
-  const int split = SPLIT ? blockIdx.z : 0;
+  const Place place =
+      sorted ? sorted_place(seq_lens, seq_starts) : shifted_place();
+  const int b = place.b, h_kv = place.h, split = place.split;
   const int hq0 = h_kv * G;
   const int Hq = hkv * G;
 
@@ -522,15 +565,15 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
     const int32_t *__restrict__ seq_lens,
     const int32_t *__restrict__ seq_starts, uint16_t *__restrict__ out,
     uint16_t *__restrict__ out_swz, float *__restrict__ partial, int hkv,
-    int max_blocks, int nsplit, float scale) {
+    int max_blocks, int nsplit, float scale, bool sorted) {
   constexpr int BS = 16;                  // cache block = one S tile
   constexpr int KS32 = DH / 32;           // QK^T contraction steps
   constexpr int DT = DH / 16;             // O^T 16-row d-tiles
   constexpr int FRW = FP8 ? 2 : 4;        // u32 words per raw fragment
 
-  const int b = sequence_of();
-  const int h_kv = blockIdx.y;
-  const int split = SPLIT ? blockIdx.z : 0;
+  const Place place =
+      sorted ? sorted_place(seq_lens, seq_starts) : shifted_place();
+  const int b = place.b, h_kv = place.h, split = place.split;
   const int hq0 = h_kv * G;
   const int Hq = hkv * G;
 
@@ -799,6 +842,7 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
   uint16_t *swz = out_swz.has_value() ? (uint16_t *)out_swz->data_ptr()
                                       : nullptr;
   const int64_t longest = (int64_t)max_blocks * bs;
+  const bool sorted = B > 1 && B <= 64 && longest > 512;
   // MFMA route: keyed on the TRANSPOSED V layout (bf16 [Dh, BS] /
   // fp8 [Dh+4, BS] blocks) the allocator chooses for MFMA-eligible
   // models (G >= 4, DH <= 128, 16-token blocks — RB_DECODE_MFMA=0 at
@@ -819,7 +863,7 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                            block_tables.data_ptr<int32_t>(),
                            seq_lens.data_ptr<int32_t>(), starts,
                            (uint16_t *)out.data_ptr(), swz, nullptr, hkv,
-                           max_blocks, 1, scale);
+                           max_blocks, 1, scale, sorted);
       } else {
         const int Hq = hkv * G;
         auto partial = at::empty({B, Hq, nsplit, DH + 2},
@@ -832,7 +876,7 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                            block_tables.data_ptr<int32_t>(),
                            seq_lens.data_ptr<int32_t>(), starts,
                            nullptr, nullptr, partial.data_ptr<float>(), hkv,
-                           max_blocks, nsplit, scale);
+                           max_blocks, nsplit, scale, sorted);
         hipLaunchKernelGGL((decode_combine_kernel<DH / 64>),
                            dim3((B * Hq + 3) / 4), dim3(256), 0, stream,
                            partial.data_ptr<float>(),
@@ -854,7 +898,7 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                        seq_lens.data_ptr<int32_t>(), starts,
                        splits > 1 ? nullptr : (uint16_t *)out.data_ptr(),
                        splits > 1 ? nullptr : swz, partial, hkv, bs, max_blocks,
-                       splits, scale);
+                       splits, scale, sorted);
   };
   if constexpr (G < NW) {
     // Whole sequences by 8 waves: of a short one more have nothing to do, and a CU

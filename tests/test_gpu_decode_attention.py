@@ -59,6 +59,41 @@ def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
                                operand.view(-1, 32, 8)[:, :batch])
 
 
+@pytest.mark.parametrize("hq,hkv,nsplit", [(3, 3, 1), (5, 5, 3), (8, 2, 1),
+                                           (8, 2, 2)])
+@pytest.mark.parametrize("batch", [2, 31, 64, 65])
+def test_sorted_sequences(batch, hq, hkv, nsplit):
+    """Every sequence and head is somebody's, whatever the lengths (of some the
+    same, of one none that its window sees), whole and in parts, in rounds of
+    256 workgroups that are full and not."""
+    torch.manual_seed(batch)
+    dh, blocks = 64, 33
+    lens = torch.randint(1, blocks * 16 + 1, (batch,))
+    lens[::3] = 77
+    starts = torch.clamp(lens - 60, min=0)
+    starts[1] = lens[1]
+    vt = hq // hkv >= 4
+    kc, vc = ops.alloc_kv_cache(batch * blocks, hkv, dh, DEV,
+                                dtype=torch.bfloat16, v_transposed=vt)
+    kc.normal_()
+    vc.normal_()
+    i32 = dict(dtype=torch.int32, device=DEV)
+    tables = torch.randperm(batch * blocks, device=DEV).to(torch.int32) \
+        .view(batch, blocks)
+    q = torch.randn(batch, hq, dh, device=DEV).bfloat16()
+    for s in (None, starts):
+        got = ops.ext().paged_decode_swz(
+            q, kc, vc, tables, lens.to(**i32), nsplit, dh ** -0.5,
+            None if s is None else s.to(**i32))[0].cpu()
+        ref = ops.paged_decode_ref(q.cpu(), kc.cpu(), vc.cpu(), tables.cpu(),
+                                   lens, dh ** -0.5, s)
+        for i in range(batch):
+            if s is not None and s[i] == lens[i]:
+                assert not bool(got[i].any())
+            else:   # 16-bit probabilities in matrix products
+                assert _rel(got[i], ref[i].double()) < (4 if vt else 2) * BF16
+
+
 def test_uneven_captured_bucket():
     """One long sequence among short ones and rows that pad the batch, by the
     split of a captured step: each the plain result."""

@@ -10,6 +10,9 @@
 A norm's 1 / rms is left to the product that reads its result. Where a step has
 no kernel of this kind (8-bit caches, wide residuals, long sums of many rows) it
 is the launches of Block.forward_decode_fused.
+
+33 to 64 rows, sequences or tokens of a prompt, go the same way with rows in place
+of operands (run_rows).
 """
 from __future__ import annotations
 
@@ -38,19 +41,19 @@ class _Layer:
                 self.gate_up.half * 2 == self.gate_up.n)
 
 
-def layers_of(model, block_type, attention_type, mlp_type):
-    """A _Layer for every block, or None where one is not served or a module
-    would do more than its kernels."""
+def _served(model) -> bool:
     cfg = model.cfg
-    if not (cfg.pos == "rope" and cfg.act in ("silu_glu", "gelu_glu") and
-            model.tp == 1 and model.rope_cos.dtype == torch.float32):
-        return None
-    blocks = list(model.blocks)
+    return (cfg.pos == "rope" and cfg.act in ("silu_glu", "gelu_glu") and
+            model.tp == 1 and model.rope_cos.dtype == torch.float32)
+
+
+def _layers(blocks, steps, block_type, attention_type, mlp_type):
+    """A _Layer for each of `blocks`, or None where one is not served or a module
+    would do more than its kernels (or has `steps` of its own)."""
     mlps, attns = [b.mlp for b in blocks], [b.attn for b in blocks]
     if not (blocks and plain(block_type, *blocks) and plain(mlp_type, *mlps) and
             plain(attention_type, *attns) and
-            untouched(("forward_decode", "forward_decode_fused"), *attns,
-                      *blocks) and
+            untouched(steps, *attns, *blocks) and
             plain(ops.RMSNorm, *(n for b in blocks
                                  for n in (b.norm1, b.norm2))) and
             plain(RowParallelLinear, *(m.down_proj for m in mlps),
@@ -69,6 +72,13 @@ def layers_of(model, block_type, attention_type, mlp_type):
             return None
     layers = [_Layer(b) for b in blocks]
     return layers if all(layer.served() for layer in layers) else None
+
+
+def layers_of(model, *types):
+    """A _Layer for every block of a step, or None."""
+    return _layers(list(model.blocks),
+                   ("forward_decode", "forward_decode_fused"), *types) \
+        if _served(model) else None
 
 
 class _Normed:
@@ -147,3 +157,77 @@ def run(model, layers, x, positions, caches, slots, tables, seq_lens, nsplit,
         if i + 1 < len(layers):
             x, y = _add(x, h, layer.down, layers[i + 1].blk.norm1, False)
     return x, layers[-1].down.product(h, m)
+
+
+def _rows_layer(blk, m: int, kc, types):
+    """blk's _Layer where its kernels serve m rows, else None."""
+    layers = _layers([blk], ("forward_prefill", "forward_decode",
+                             "forward_pending"), *types)
+    if layers is None or kc.dtype != torch.bfloat16:
+        return None
+    y, pays = layers[0], ops.ext().rows_ends_pay
+    return y if (not any(c.fp8 for c in (y.qkv, y.o, y.gate_up, y.down)) and
+                 min(y.qkv.k, y.o.k, y.down.k) >= 1024 and
+                 all(n.weight.data_ptr() % 16 == 0
+                     for n in (blk.norm1, blk.norm2)) and
+                 pays(m, y.qkv.n, y.qkv.k) and
+                 pays(m, y.gate_up.n, y.gate_up.k)) else None
+
+
+def _add_rows(x, rows, copy, norm):
+    """x + rows W^T and its norm: whole sums with the residual behind them, or, of
+    long rows, parts and a launch that adds them up (us of 45 and 64 rows, in parts
+    with the norm and whole: 4096 x 4096 15.8 and 12.2, 16.4 and 13.5; 2048 x 2048
+    11.2 and 7.6, 11.9 and 8.2; 4096 x 11008 26.6 and 28.6, 28.6 and 32.6; 4096 x
+    14336 28.8 and 37.6, 30.8 and 39.6). A prompt of 45 tokens of llama2-7b, all in
+    all, 3560 -> 3410 us."""
+    ext, m = ops.ext(), x.shape[0]
+    if copy.half == 0 and copy.k <= 8192 and \
+            ext.rows_res_supported(m, copy.n, copy.k):
+        x, y, squares = ext.rows_res(rows, copy.ws, x, norm.weight)
+        return x, _Normed(rows=y, squares=squares, eps=norm.eps)
+    delta = ext.decode_gemm_rows(rows, copy.ws, copy.n, copy.half, True)
+    if delta.dim() == 3:
+        x, y, squares = ext.parts_res(delta, x, norm.weight)
+        return x, _Normed(rows=y, squares=squares, eps=norm.eps)
+    x, y = ops.rmsnorm_res(x, delta, norm.weight, norm.eps)
+    return x, _Normed(rows=y)
+
+
+def run_rows(model, x, positions, caches, slots, attend, joint: bool, *types):
+    """x [m, hidden], 33 to 64 embedded tokens, through the blocks up to the first
+    that is not served -> (residual, what the last of them has still to add to it
+    or None, how many they are). attend(attention, q, keys, values) returns the
+    heads' results as rows; with `joint`, q is q, k and v side by side.
+
+    A block is looked at while the GPU is at the one before it: a look at all of
+    llama2-7b takes the host 0.55 ms, for which an idle GPU would wait (one prompt
+    of 45 tokens 4.17 ms, so 3.69)."""
+    cfg, ext, m = model.cfg, ops.ext(), x.shape[0]
+    if not (_served(model) and cfg.norm == "rmsnorm" and
+            not cfg.parallel_residual and not cfg.single_norm and
+            cfg.head_dim in (64, 128, 256) and
+            ext.parts_res_supported(cfg.hidden_size)):
+        return x, None, 0
+    blocks = list(model.blocks)
+    layer = _rows_layer(blocks[0], m, caches[0][0], types) if blocks else None
+    if layer is None:
+        return x, None, 0
+    cos, sin = model.rope_cos, model.rope_sin
+    positions = positions.to(torch.int32)
+    slots = slots.to(torch.int32)
+    norm = layer.blk.norm1
+    y = _Normed(rows=ops.rmsnorm(x, norm.weight, norm.eps))
+    for i, (kc, vc) in enumerate(caches, 1):
+        c = layer.qkv
+        q = ext.rows_heads(y.rows, c.ws, c.n, cos, sin, positions, kc, vc,
+                           slots, layer.attn.hq, joint, y.squares, y.eps)
+        x, y = _add_rows(x, attend(layer.attn, q, kc, vc), layer.o,
+                         layer.blk.norm2)
+        c, down = layer.gate_up, layer.down
+        h = ext.rows_glu(y.rows, c.ws, c.n, layer.gelu, False, y.squares, y.eps)
+        layer = _rows_layer(blocks[i], m, caches[i][0], types) \
+            if i < len(blocks) else None
+        if layer is None:
+            return x, ext.decode_gemm_rows(h, down.ws, down.n, down.half), i
+        x, y = _add_rows(x, h, down, layer.blk.norm1)

@@ -507,12 +507,12 @@ class Transformer(nn.Module):
             logits = gather_from_tp(logits)
         return logits.view(B, S, -1)
 
-    def _blocks(self, x, attention, run=lambda blk, *args: blk(*args)):
-        """All blocks; attention(block, parts) is its attn_fn, which with `parts`
-        may return parts of its sums. Returns the residual and what is still to
-        be added to it (None: nothing)."""
-        delta = None
-        if self._sums_in_layer_norms(x):
+    def _blocks(self, x, attention, run=lambda blk, *args: blk(*args),
+                delta=None, first=0):
+        """All blocks, or those from `first` on; attention(block, parts) is its
+        attn_fn, which with `parts` may return parts of its sums. x + delta ->
+        the residual and what is still to be added to it (None: nothing)."""
+        if delta is None and self._sums_in_layer_norms(x):
             dtype, x = x.dtype, x.float()
             for blk in self.blocks:
                 h = ops.norm_res32(blk.norm1, x, delta, dtype)
@@ -520,7 +520,7 @@ class Transformer(nn.Module):
                 h = ops.norm_res32(blk.norm2, x, delta, dtype)
                 delta = blk.mlp(h)
             return x, delta
-        blocks = list(self.blocks)
+        blocks = list(self.blocks)[first:]
         fuses = [blk.fuses_residual() for blk in blocks]
         # sums of up to 32 rows come whole: without a look at the modules, which
         # takes the host 10 us a block (a prompt of 20 tokens of llama2-7b is
@@ -592,8 +592,15 @@ class Transformer(nn.Module):
                 h, self.rope_cos, self.rope_sin, positions, kc, vc,
                 slot_mapping, B, S, **kw)
 
+        def attend(attn, y, kc, vc):
+            return ops.ext().flash_prefill_qkv(
+                y, B, S, attn.hq, attn.hkv, attn.dh, attn.scale).flatten(2) \
+                .flatten(0, 1)
+
+        sums = self._few_rows(x, positions, caches, slot_mapping, attend, True,
+                              attention)
         x = self._last_norm(*(None if r is None else r.view(B, S, -1)[:, -1]
-                              for r in self._blocks(x, attention)))
+                              for r in sums))
         logits = self.lm_head(x)
         return gather_from_tp(logits) if self._lm_vocab_parallel else logits
 
@@ -670,9 +677,27 @@ class Transformer(nn.Module):
                 slot_mapping, block_tables, seq_lens, nsplit=nsplit,
                 seq_starts=seq_starts, **kw)
 
-        x = self._last_norm(*self._blocks(x, attention))
+        def attend(attn, q, kc, vc):
+            return ops.paged_decode_with_operand(
+                q, kc, vc, block_tables, seq_lens, scale=attn.scale,
+                nsplit=nsplit, seq_starts=seq_starts)[0].flatten(1)
+
+        sums = self._few_rows(x, positions, caches, slot_mapping, attend, False,
+                              attention)
+        x = self._last_norm(*sums)
         logits = self.lm_head(x)
         return gather_from_tp(logits) if self._lm_vocab_parallel else logits
+
+    def _few_rows(self, x, positions, caches, slots, attend, joint, attention):
+        """_blocks(x, attention), as far as it goes by decode_chain.run_rows."""
+        delta, first = None, 0
+        if (32 < x.shape[0] <= 64 and ops.use_hip(x) and
+                x.dtype == torch.bfloat16 and not torch.is_grad_enabled() and
+                os.environ.get("RB_FUSED_RESID", "1") == "1"):
+            x, delta, first = decode_chain.run_rows(
+                self, x, positions, caches, slots, attend, joint, Block,
+                Attention, MLP)
+        return self._blocks(x, attention, delta=delta, first=first)
 
     def _affine_ready(self) -> bool:
         """Every block has its products for _decode_affine, of weights that have

@@ -29,7 +29,7 @@ bool decode_res_supported(int64_t M, int64_t N, int64_t K, bool fp8);
 std::vector<at::Tensor> decode_res(at::Tensor xs, at::Tensor ws, c10::optional<at::Tensor> scale, at::Tensor res, at::Tensor norm, bool rows);
 std::vector<at::Tensor> rmsnorm_res_slab_fwd(at::Tensor x, at::Tensor slabs, at::Tensor w, double eps);
 at::Tensor rows_glu(at::Tensor x, at::Tensor ws, int64_t N, bool gelu, bool operand, c10::optional<at::Tensor> squares, double eps);
-at::Tensor rows_heads(at::Tensor x, at::Tensor ws, int64_t N, at::Tensor cos, at::Tensor sin, at::Tensor positions, at::Tensor k_cache, at::Tensor v_cache, at::Tensor slots, int64_t hq, bool rows);
+at::Tensor rows_heads(at::Tensor x, at::Tensor ws, int64_t N, at::Tensor cos, at::Tensor sin, at::Tensor positions, at::Tensor k_cache, at::Tensor v_cache, at::Tensor slots, int64_t hq, bool rows, c10::optional<at::Tensor> squares, double eps);
 at::Tensor decode_swizzle_w(at::Tensor w, int64_t half);
 at::Tensor decode_swizzle_x(at::Tensor x);
 at::Tensor decode_swizzle_w8(at::Tensor w8, int64_t half);
@@ -41,6 +41,10 @@ void affine_add_(at::Tensor x, at::Tensor w, c10::optional<at::Tensor> bias, at:
 at::Tensor embed_res32(at::Tensor tokens, at::Tensor positions, at::Tensor table, at::Tensor places);
 at::Tensor sum_parts(at::Tensor parts);
 bool tile_gemm_takes(at::Tensor x, at::Tensor w, bool glu);
+bool rows_res_supported(int64_t M, int64_t N, int64_t K);
+bool parts_res_supported(int64_t N);
+std::vector<at::Tensor> parts_res(at::Tensor parts, at::Tensor res, at::Tensor norm);
+std::vector<at::Tensor> rows_res(at::Tensor x, at::Tensor ws, at::Tensor res, at::Tensor norm);
 at::Tensor tile_lora(at::Tensor x, at::Tensor w, at::Tensor t, std::vector<at::Tensor> bs, double scale, int64_t tile);
 bool tile_gemm_down_takes(at::Tensor x, at::Tensor w);
 bool tile_gemm_down_pays(int64_t M, int64_t N, int64_t K);
@@ -146,7 +150,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "decode_heads of up to 128 rows as they lie", py::arg("x"),
         py::arg("ws"), py::arg("N"), py::arg("cos"), py::arg("sin"),
         py::arg("positions"), py::arg("k_cache"), py::arg("v_cache"),
-        py::arg("slots"), py::arg("hq"), py::arg("rows") = false);
+        py::arg("slots"), py::arg("hq"), py::arg("rows") = false,
+        py::arg("squares") = py::none(), py::arg("eps") = 0.0);
   m.def("decode_swizzle_w", &decode_swizzle_w,
         "one-time [N,K] -> fragment-lane-major weight layout", py::arg("w"),
         py::arg("half") = 0);
@@ -173,6 +178,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sum_parts", &sum_parts, "fp32 [P, M, N] -> their sum [M, N] bf16");
   m.def("tile_gemm_takes", &tile_gemm_takes, py::arg("x"), py::arg("w"),
         py::arg("glu") = false, "whether tile_gemm takes x and W");
+  m.def("parts_res_supported", &parts_res_supported);
+  m.def("parts_res", &parts_res, "the same of fp32 parts of the product");
+  m.def("rows_res_supported", &rows_res_supported);
+  m.def("rows_res", &rows_res,
+        "x W^T + residual of 17 to 64 rows x, times the next norm's weight, and "
+        "parts of its squares");
   m.def("tile_lora", &tile_lora, py::arg("x"), py::arg("w"), py::arg("t"),
         py::arg("bs"), py::arg("scale"), py::arg("tile") = -1,
         "x @ W^T + scale t_i @ B_i^T of siblings side by side");

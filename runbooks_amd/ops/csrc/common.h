@@ -314,6 +314,15 @@ RB_DEV void lds_load(u32x4v from, unsigned voff, unsigned soff, unsigned lds) {
       :: "v"(voff), "s"(from), "s"(soff), "s"(lds) : "memory", "m0");
 }
 
+// The same of what is read once, and should not push other things out of L2.
+RB_DEV void lds_load_once(u32x4v from, unsigned voff, unsigned soff,
+                          unsigned lds) {
+  asm volatile(
+      "s_mov_b32 m0, %3\n\ts_nop 0\n\t"
+      "buffer_load_dwordx4 %0, %1, %2 offen nt lds"
+      :: "v"(voff), "s"(from), "s"(soff), "s"(lds) : "memory", "m0");
+}
+
 // two floats -> packed bf16 words (round to nearest even)
 RB_DEV uint32_t pack_bf16x2(float lo, float hi) {
   return f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);

@@ -66,8 +66,9 @@ template <Kind KIND> struct Early {
   float norm;
   int position;
   ends::Turn<2> turn;
-  RB_DEV void begin(const Ends &e, int M) {
-    const int m = min((int)threadIdx.x >> 3, M - 1), i = threadIdx.x & 7;
+  RB_DEV void begin(const Ends &e, int M, int base = 0) {
+    const int m = min(base + ((int)threadIdx.x >> 3), M - 1);
+    const int i = threadIdx.x & 7;
     if constexpr (KIND == ends::QKV) position = e.pos[m];
     if (KIND != ends::SLAB && e.squares != nullptr) {
 #pragma unroll
@@ -276,10 +277,12 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
   const uint8_t *wseg =
       ws + (int64_t)min(nblk, blocks - 1) * steps * 1024 + lane * 16;
   char *mine = smem + kg * TILE;                   // buffers KG * TILE apart
-  constexpr bool NORM = RB == 1 && KIND != ends::SLAB;
-  __shared__ float norms[NORM ? MMAX : 1];
-  Early<ends::PLAIN> early;
-  if constexpr (NORM) early.begin(e, M);
+  constexpr bool NORM = RB <= 2 && KIND != ends::SLAB;
+  __shared__ float norms[NORM ? RB * 32 : 1];
+  Early<ends::PLAIN> early[NORM ? RB : 1];
+  if constexpr (NORM)
+#pragma unroll
+    for (int b = 0; b < RB; ++b) early[b].begin(e, M, b * 32);
 
   struct X { u32x4v v[XL]; };
   struct W { u32x4v v[CH]; };
@@ -325,23 +328,36 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
           tile + (row * P + (c ^ (row & (P - 1)))) * 16);
     }
   };
-  X xr;
+  // of up to 64 rows x is two chunks ahead, too, which more have no registers for
+  // (us with x one and two ahead: 12288 x 4096 of 45 rows 24.8 and 24.1, of 32 23.5
+  // and 22.3; 5120 x 13824 35.2 and 33.4, 37.0 and 33.0)
+  constexpr int FAR = RB <= 2 ? 2 : 1;
+  X x0, x1;
   W w0, w1;
-  load_x(xr, s0);
+  load_x(x0, s0);
   load_w(w0, s0);
-  put_x(xr, mine);
-  load_x(xr, s0 + CH);
+  if constexpr (FAR == 2) load_x(x1, s0 + CH);
+  else put_x(x0, mine);
+  if constexpr (FAR == 1) load_x(x0, s0 + CH);
   load_w(w1, s0 + CH);
+  if constexpr (FAR == 2) {
+    put_x(x0, mine);
+    load_x(x0, s0 + 2 * CH);
+  }
   if constexpr (NORM) {
-    early.rest(e, M);
-    if (threadIdx.x % 8 == 0) norms[threadIdx.x / 8] = early.norm;
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+      early[b].rest(e, M);
+      if (threadIdx.x % 8 == 0) norms[b * 32 + threadIdx.x / 8] = early[b].norm;
+    }
   }
   meet();
-  // chunk c, of which `w` holds W and then W of chunk c + 2
-  auto step = [&](W &w, int c, auto whole) {
+  // chunk c, of which `w` holds W and then W of chunk c + 2; `xr` holds x of chunk
+  // c + 1 and then of chunk c + 1 + FAR
+  auto step = [&](W &w, X &xr, int c, auto whole) {
     const int s = s0 + c * CH;
     put_x(xr, mine + (~c & 1) * KG * TILE);
-    load_x(xr, s + 2 * CH);
+    load_x(xr, s + (1 + FAR) * CH);
     const char *tile = mine + (c & 1) * KG * TILE;
     bf16x8v xv[CH][RB];
 #pragma unroll
@@ -363,12 +379,12 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
   };
   int c = 0;
   for (; c + 2 <= full; c += 2) {
-    step(w0, c, std::true_type{});
-    step(w1, c + 1, std::true_type{});
+    step(w0, FAR == 2 ? x1 : x0, c, std::true_type{});
+    step(w1, x0, c + 1, std::true_type{});
   }
   for (; c < chunks; c += 2) {
-    step(w0, c, std::false_type{});
-    step(w1, c + 1, std::false_type{});
+    step(w0, FAR == 2 ? x1 : x0, c, std::false_type{});
+    step(w1, x0, c + 1, std::false_type{});
   }
   // sum of the groups
   if constexpr (KG > 1) {
@@ -393,7 +409,9 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
   if (nblk >= blocks) return;
   if constexpr (NORM) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[0][r] *= norms[col];
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[b][r] *= norms[b * 32 + col];
   }
   if constexpr (KIND == ends::GLU || KIND == ends::QKV) {
     // registers r and r + 8 of a lane are a pair, 4 neighbours at a time
@@ -943,14 +961,15 @@ at::Tensor decode_gemm_rows(at::Tensor x, at::Tensor ws, int64_t N,
   return y;
 }
 
-// decode_glu of 1 to 128 rows x as they lie: the gated rows [M, N / 2], or,
-// of up to 32 rows (which may come without their 1 / rms), an operand.
+// decode_glu of 1 to 128 rows x as they lie (up to 64 may come without their 1 /
+// rms): the gated rows [M, N / 2], or, of up to 32 rows, an operand.
 at::Tensor rows_glu(at::Tensor x, at::Tensor ws, int64_t N, bool gelu,
                     bool operand, c10::optional<at::Tensor> squares,
                     double eps) {
   check_rows(x, ws, N, N / 2);
   const int64_t M = x.size(0), K = x.size(1);
-  TORCH_CHECK(M <= MMAX || !(operand || squares.has_value()),
+  TORCH_CHECK((M <= MMAX || !operand) &&
+              (M <= 2 * MMAX || !squares.has_value()),
               "rows_glu: operand, squares");
   Ends e{};
   e.half = (int)(N / 2);
@@ -963,16 +982,19 @@ at::Tensor rows_glu(at::Tensor x, at::Tensor ws, int64_t N, bool gelu,
   return out;
 }
 
-// decode_heads of 1 to 128 rows x as they lie: rotated q [M, hq, dh], or, in
-// rows, q and k rotated and v side by side [M, N].
+// decode_heads of 1 to 128 rows x as they lie (up to 64 may come without their 1 /
+// rms): rotated q [M, hq, dh], or, in rows, q and k rotated and v side by side [M,
+// N].
 at::Tensor rows_heads(at::Tensor x, at::Tensor ws, int64_t N, at::Tensor cos,
                       at::Tensor sin, at::Tensor positions, at::Tensor k_cache,
                       at::Tensor v_cache, at::Tensor slots, int64_t hq,
-                      bool rows) {
+                      bool rows, c10::optional<at::Tensor> squares, double eps) {
   Ends e{};
   const int64_t M = x.size(0), K = x.size(1);
   set_heads(e, M, N, cos, sin, positions, k_cache, v_cache, slots, hq);
   check_rows(x, ws, N, e.half);
+  TORCH_CHECK(M <= 2 * MMAX || !squares.has_value(), "rows_heads: squares");
+  set_squares(e, squares, M, K, eps);
   auto out = rows ? at::empty({M, N}, x.options())
                   : at::empty({M, hq, (int64_t)e.dh}, x.options());
   (rows ? e.y : e.q) = (uint16_t *)out.data_ptr();

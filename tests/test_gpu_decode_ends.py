@@ -352,3 +352,126 @@ def test_shortest_prompts(monkeypatch, tokens, kv, inter, eight_bit):
         monkeypatch.setattr(ops, name, lambda *a, **k: None)
     for a, b in zip(got, prompt()):
         assert _rel(a, b.double()) < 2e-2
+
+
+@pytest.mark.parametrize("m", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("n,k", [(32, 1024), (1024, 1088), (4096, 8192)])
+def test_residual_sum_of_rows(m, n, k):
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    res = (torch.randn(m, n, device=DEV) * k ** 0.5).bfloat16()
+    gamma = torch.randn(n, device=DEV).bfloat16()
+    ws, _, w = _weight(n, k, 0, False)
+    assert ops.ext().rows_res_supported(m, n, k)
+    out, y, squares = ops.ext().rows_res(x, ws, res, gamma)
+    want = res.double() + x.double() @ w.t()
+    assert _rel(out, want) < BF16
+    assert _rel(y, want * gamma.double()) < BF16
+    assert _rel(squares.sum(1), want.square().sum(1)) < 1e-5
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 1024, 1024), (65, 1024, 1024),
+                                   (48, 1040, 1024), (48, 1024, 1056),
+                                   (48, 4128, 1024)])
+def test_refused_residual_sums_of_rows(m, n, k):
+    assert not ops.ext().rows_res_supported(m, n, k)
+    x = torch.zeros(m, k, device=DEV).bfloat16()
+    res = torch.zeros(m, n, device=DEV).bfloat16()
+    ws = torch.zeros(n * k, device=DEV).bfloat16()
+    with pytest.raises(RuntimeError):
+        ops.ext().rows_res(x, ws, res, res[0])
+
+
+@pytest.mark.parametrize("m", [33, 64])
+@pytest.mark.parametrize("parts,n", [(1, 1024), (2, 1280), (4, 4096), (8, 8192)])
+def test_residual_of_parts(m, parts, n):
+    """Sums of parts and residual with the norm's squares, fp32 throughout."""
+    assert ops.ext().parts_res_supported(n)
+    p = torch.randn(parts, m, n, device=DEV)
+    res = torch.randn(m, n, device=DEV).bfloat16()
+    gamma = torch.randn(n, device=DEV).bfloat16()
+    out, y, squares = ops.ext().parts_res(p, res, gamma)
+    want = res.double() + p.double().sum(0)
+    assert _rel(out, want) < BF16
+    assert _rel(y, want * gamma.double()) < BF16
+    assert _rel(squares.sum(1), want.square().sum(1)) < 1e-5
+
+
+@pytest.mark.parametrize("m", [33, 48, 64])
+@pytest.mark.parametrize("inter,k,parts", [(2048, 1024, 4), (5504, 4096, 128),
+                                           (2064, 1056, 256)])
+def test_units_of_rows_normed_late(m, inter, k, parts):
+    """rows_glu and rows_heads of 33 to 64 rows that still lack their 1 / rms."""
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    squares = _squares(x, parts)
+    w = (torch.randn(2 * inter, k, device=DEV) / k ** 0.5).bfloat16()
+    ws = ops.ext().decode_swizzle_w(w, inter)
+    both = (x.double() * _inverse_rms(x)) @ w.double().t()
+    want = _act(both[:, :inter], False) * both[:, inter:]
+    h = ops.ext().rows_glu(x, ws, 2 * inter, False, False, squares, 1e-5)
+    assert _rel(h, want) < BF16
+
+    dh, hq, hkv = 128, 16, 4
+    n = (hq + 2 * hkv) * dh
+    w = torch.randn(n, k, device=DEV).bfloat16()
+    ws = ops.ext().decode_swizzle_w(w, dh // 2)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    kc = torch.zeros(8, hkv, 16, dh, device=DEV).bfloat16()
+    vc = torch.zeros_like(kc)
+    ones = torch.ones(8, dh // 2, device=DEV)
+    y = ops.ext().rows_heads(x, ws, n, ones, ones * 0, torch.zeros(m, **i32),
+                             kc, vc, torch.arange(m, **i32), hq, True, squares,
+                             1e-5)
+    want = (x.double() * _inverse_rms(x)) @ w.double().t()
+    assert _rel(y.reshape(m, -1), want) < BF16
+
+
+def _served_by_rows(monkeypatch):
+    """Blocks that run_rows took, call by call."""
+    from runbooks_amd.models import decode_chain
+    seen, plain = [], decode_chain.run_rows
+
+    def run(*args):
+        out = plain(*args)
+        seen.append(out[2])
+        return out
+    monkeypatch.setattr(decode_chain, "run_rows", run)
+    return seen
+
+
+@pytest.mark.parametrize("tokens", [33, 48, 64])
+@pytest.mark.parametrize("kv,inter,hidden", [(8, 2048, 1024), (2, 6144, 1024),
+                                             (8, 12288, 1024), (8, 2048, 4096)])
+@pytest.mark.parametrize("decode", [False, True])
+def test_steps_of_rows(monkeypatch, tokens, kv, inter, hidden, decode):
+    """A prompt and a step of 33 to 64 rows on these kernels and on the modules,
+    bound as in test_decode_step, and with a hook on the second block, which is
+    called in its place and gets the first one's result."""
+    m = _model(kv, inter, hidden)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    seen = _served_by_rows(monkeypatch)
+
+    def step():
+        if decode:
+            args = _step(m, tokens, False)
+            caches = args[2]
+        else:
+            caches = m.alloc_caches(16, DEV)
+            args = (torch.arange(tokens, device=DEV)[None] % 50,
+                    torch.arange(tokens, **i32), caches,
+                    torch.arange(tokens, **i32) + 5)
+        with torch.no_grad():
+            logits = m.decode(*args) if decode else m.prefill(*args)
+        return [logits] + [c for layer in caches for c in layer]
+
+    got = step()
+    called = []
+    hook = m.blocks[1].mlp.register_forward_hook(
+        lambda mod, x, y: called.append(y.shape))
+    mixed = step()
+    hook.remove()
+    monkeypatch.setattr(type(m), "_few_rows",
+                        lambda self, x, *a: self._blocks(x, a[-1]))
+    ref = step()
+    assert seen == [2, 1] and len(called) == 1
+    for a, b, c in zip(got, mixed, ref):
+        assert _rel(a, c.double()) < 2e-2 and _rel(b, c.double()) < 2e-2

@@ -6,21 +6,21 @@
 // Bound by L2, which feeds LDS at 16 TB/s (62 GB/s a CU: what is left of a
 // product of 8192 x 8192 x 4096 without its matrix instructions takes 269 us in
 // tiles of 256 x 256 and 554 in those of 128 x 128), and by the matrix cores
-// (without loads 312 us, 1760 TFLOP/s; both together 401). So tiles are as large
+// (without loads 312 us, 1760 TFLOP/s; both together 382). So tiles are as large
 // as their number allows; where it does not, for prompts of some hundred rows,
 // workgroups share the sums.
 //
-// us in the library and here, weights out of cache: 256 x 4096 x 11008 51 and 36
-// (4 parts), 512 x 4096 x 11008 75 and 47 (4), 1021 x 4096 x 11008 105 and 80 (2),
-// 512 x 3072 x 24576 267 and 82 (4), 512 x 22016 x 4096 80 and 77, 1021 x 49152 x
-// 3072 240 and 235, 2048 x 4096 x 14336 205 and 180, 7931 x 28672 x 4096 1300 and
-// 1340 (1420 and 1340 with the gated unit).
-
+// us in the library and here, weights out of cache: 256 x 4096 x 11008 52 and 37
+// (4 parts), 512 x 4096 x 11008 78 and 48 (4), 1021 x 4096 x 11008 110 and 84 (2),
+// 512 x 3072 x 24576 261 and 88 (4), 512 x 22016 x 4096 92 and 80, 1021 x 49152 x
+// 3072 250 and 229, 2048 x 4096 x 14336 207 and 188, 7931 x 28672 x 4096 1292 and
+// 1276 (1427 and 1306 with the gated unit).
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "decode_ends.h"
@@ -32,16 +32,70 @@ using ends::f32x4v;
 using rb::buffer;
 using rb::u32x4v;
 
-__device__ __forceinline__ void put(uint16_t *p, const float (&f)[4]) {
+typedef __attribute__((ext_vector_type(2))) uint32_t u32x2v;
+
+__device__ __forceinline__ u32x2v packed(const float (&f)[4]) {
   typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4v;
-  *reinterpret_cast<bf16x4v *>(p) =
-      __builtin_convertvector((f32x4v){f[0], f[1], f[2], f[3]}, bf16x4v);
+  return __builtin_bit_cast(
+      u32x2v, __builtin_convertvector((f32x4v){f[0], f[1], f[2], f[3]}, bf16x4v));
+}
+
+// Four columns of a lane from n on in each of two neighbouring 16 x 16 results, a
+// and b, the first at column `first` of y, a row of `cols`: after an exchange
+// between neighbouring fours, a lane stores eight. In pieces of 8 bytes a wave's
+// store filled 32 of a line of 128 (us of zeros in these and in pieces of 16: 4096 x
+// 4096 x 512 23.4 and 21.2, 8192 x 8192 x 1024 102 and 88, 2048 x 12288 x 4096 128
+// and 122, 512 x 12288 x 4096 67 and 63).
+__device__ __forceinline__ void put(uint16_t *y, u32x2v a, u32x2v b, int first,
+                                    int fk, int cols, bool there) {
+  const auto lo = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  const int n = first + (fk & 1) * 16 + (fk >> 1) * 8;
+  if (!there || n >= cols) return;
+  if (cols % 8 == 0) {
+    *reinterpret_cast<u32x4v *>(y + n) = (u32x4v){lo[0], hi[0], lo[1], hi[1]};
+  } else {
+    *reinterpret_cast<u32x2v *>(y + n) = (u32x2v){lo[0], hi[0]};
+    if (n + 4 < cols)
+      *reinterpret_cast<u32x2v *>(y + n + 4) = (u32x2v){lo[1], hi[1]};
+  }
+}
+
+// The same of one result.
+__device__ __forceinline__ void put(uint16_t *y, u32x2v a, int first, int fk,
+                                    int cols, bool there) {
+  if (there && first + fk * 4 < cols)
+    *reinterpret_cast<u32x2v *>(y + first + fk * 4) = a;
 }
 
 // As text, for the compiler copies sums between the register files otherwise.
 __device__ __forceinline__ void mma(f32x4v &c, bf16x8v a, bf16x8v b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
                : "+a"(c) : "v"(a), "v"(b));
+}
+
+// The same beside a load of 16 bytes a lane into LDS at lds + MORE. Of one text, for
+// the product then stands between the write of m0 and its use, which have to be an
+// instruction apart: a wave issues one in four clocks, and a product takes 16.
+template <unsigned MORE>
+__device__ __forceinline__ void mma_load(f32x4v &c, bf16x8v a, bf16x8v b,
+                                         u32x4v from, unsigned voff,
+                                         unsigned soff, unsigned lds) {
+  asm volatile(
+      "s_add_u32 m0, %6, %7\n\t"
+      "v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\t"
+      "buffer_load_dwordx4 %3, %4, %5 offen lds"
+      : "+a"(c)
+      : "v"(a), "v"(b), "v"(voff), "s"(from), "s"(soff), "s"(lds), "n"(MORE)
+      : "memory", "m0", "scc");
+}
+
+template <class F, int... Q>
+__device__ __forceinline__ void each_of(F &f, std::integer_sequence<int, Q...>) {
+  (f(std::integral_constant<int, Q>()), ...);
+}
+template <int N, class F> __device__ __forceinline__ void each(F &f) {
+  each_of(f, std::make_integer_sequence<int, N>());
 }
 
 // A product by itself, outside of the matrix registers, which the sums fill.
@@ -74,6 +128,12 @@ __device__ __forceinline__ int sibling(const Adapters &a, int n) {
 }
 
 constexpr unsigned NOWHERE = 0x80000000;    // past the end of every such buffer
+
+// i, known from here on: what is computed of it stays behind this.
+__device__ __forceinline__ int pinned(int i) {
+  asm volatile("" : "+s"(i));
+  return i;
+}
 
 // Waits until the last products are in their registers, if `left` is 0. The
 // compiler does not know what mma() takes, and may move sums about right behind
@@ -121,14 +181,15 @@ __device__ __forceinline__ void end_lora(const Adapters &a,
   // for all loads in the loop over K that follows
   constexpr int loaded = 0x0f70;        // vmcnt(0)
   __builtin_amdgcn_s_waitcnt(loaded);
-  int now = -1;
+  int of = -1;
+  u32x2v held[FM];
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
     const int n = __builtin_amdgcn_readfirstlane(n0 + j * 16);
     if (n >= N) continue;
     const int s = sibling(a, n);
-    if (s != now) {
-      now = s;
+    if (s != of) {
+      of = s;
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
         const bf16x8v v = ends::load8v(
@@ -145,7 +206,13 @@ __device__ __forceinline__ void end_lora(const Adapters &a,
       take(f, acc[i][j]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) f[e] += a.scale * d[e];
-      if (m < M) put(y + (int64_t)m * N + n + fk * 4, f);
+      const u32x2v now = packed(f);
+      if (j % 2 == 0)
+        held[i] = now;
+      else
+        put(y + (int64_t)m * N, held[i], now, n - 16, fk, N, m < M);
+      if (j % 2 == 0 && (j + 1 == FN || n + 16 >= N))
+        put(y + (int64_t)m * N, now, n, fk, N, m < M);
     }
   }
 }
@@ -162,6 +229,15 @@ __device__ __forceinline__ void end_lora(const Adapters &a,
 // operands of the second are read; from slot B1, when all waves have read theirs
 // and the buffer is free, it is filled for the K-tile SX (SW) on; from slot B2,
 // when the next K-tile is there, that one's first operands are read.
+//
+// A slot is 16 clocks, in which a wave issues three instructions beside the product.
+// So a load has one beside it (mma_load), and what its addresses take, some 30
+// scalar instructions a K-tile, is spread over the slots in front of B1 instead of
+// standing before the first (pinned(); us of normal data and of zeros, before and
+// now: 2048 x 12288 x 4096 165 and 162, 132 and 128; 7931 x 28672 x 4096 with the
+// gated unit 1334 and 1305, 1044 and 1005; 2048 x 22016 x 4096 279 and 273, 227 and
+// 219). With wider stores a step of llama2-7b, 4 x 512 tokens, takes 59.0 ms, 60.5
+// before.
 //
 // Workgroups stay for all of their tiles, and the buffers are filled for the
 // next one during the end of the one before. Tiles go to XCDs in runs, down
@@ -377,7 +453,9 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
   constexpr int D = (2 * F - B1) / LOADS;
   constexpr int BEFORE =
       (B2 - B1 + D - 1) / D < LOADS ? (B2 - B1 + D - 1) / D : LOADS;
-  static_assert(D > 0 && (R - 1) * R1 < B1 && B2 + 1 + (R - 1) * R2 < 2 * F,
+  // slots for what the loads' addresses take
+  constexpr int A = 1, AD = (B1 - 1 - A) / 5;
+  static_assert(D > 0 && AD > 0 && (R - 1) * R1 < B1 && B2 + 1 + (R - 1) * R2 < 2 * F,
                 "slots");
   int bx = 0, bw = 0;
   while (true) {
@@ -385,37 +463,61 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
     const bool more = then < end;
     const Place next = more ? place(then) : here;
     for (int t = 0; t < kn; ++t) {
-      const int nx = bx + 1 == SX ? 0 : bx + 1, nw = bw + 1 == SW ? 0 : bw + 1;
+      int nx, nw;
+      unsigned lx, lw;
       Place p;                        // of the K-tiles that are fetched now
-      p.rx = t + SX < kn ? here.rx : next.rx;
-      p.rw = t + SW < kn ? here.rw : next.rw;
-      p.m0 = t + SX < kn ? here.m0 : next.m0;
-      p.n0 = t + SW < kn ? here.n0 : next.n0;
-      const int tx = t + SX < kn ? t + SX : t + SX - kn;
-      const int tw = t + SW < kn ? t + SW : t + SW - kn;
-      aim_x(p, tx);
-      aim_w(p, tw);
+      auto slot = [&](auto at) __attribute__((always_inline)) {
+        constexpr int q = decltype(at)::value;
+        constexpr int set = q / F, i = q / FN % FM, j = q % FN;
+        if constexpr (q == A) {
+          const int u = pinned(t + SX);
 #pragma unroll
-      for (int set = 0; set < 2; ++set)
+          for (int e = 0; e < 3; ++e) p.rx[e] = u < kn ? here.rx[e] : next.rx[e];
+          p.rx[3] = here.rx[3];
+          p.m0 = u < kn ? here.m0 : next.m0;
+        }
+        if constexpr (q == A + AD) {
+          const int u = pinned(t + SX);
+          aim_x(p, u < kn ? u : u - kn);
+        }
+        if constexpr (q == A + 2 * AD) {
+          lx = pinned(bx) * XS + wid * 1024;
+          lw = SX * XS - XS + bw * WS + wid * 1024;
+        }
+        if constexpr (q == A + 3 * AD) {
+          const int u = pinned(t + SW);
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            const int q = (set * FM + i) * FN + j;
-            if (q == B1)
-              asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (q == B2) wait(std::integral_constant<int, AHEAD + BEFORE>());
-            mma(acc[i][j], fw[set][j], fx[set][i]);
-            __builtin_amdgcn_sched_barrier(0);
-            if (q % R1 == 0 && q / R1 < R) frag(1, bx, bw, q / R1);
-            if (q > B2 && (q - B2 - 1) % R2 == 0 && (q - B2 - 1) / R2 < R)
-              frag(0, nx, nw, (q - B2 - 1) / R2);
-            if (q >= B1 && (q - B1) % D == 0 && (q - B1) / D < LOADS) {
-              const int l = (q - B1) / D;
-              load(p, l < XL ? bx : bw, l);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-          }
+          for (int e = 0; e < 3; ++e) p.rw[e] = u < kn ? here.rw[e] : next.rw[e];
+          p.rw[3] = here.rw[3];
+          p.n0 = u < kn ? here.n0 : next.n0;
+        }
+        if constexpr (q == A + 4 * AD) {
+          const int u = pinned(t + SW);
+          aim_w(p, u < kn ? u : u - kn);
+        }
+        if constexpr (q == A + 5 * AD) {
+          nx = pinned(bx + 1), nw = pinned(bw + 1);
+          nx = nx == SX ? 0 : nx;
+          nw = nw == SW ? 0 : nw;
+        }
+        if constexpr (q == B1)
+          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if constexpr (q == B2) wait(std::integral_constant<int, AHEAD + BEFORE>());
+        if constexpr (q >= B1 && (q - B1) % D == 0 && (q - B1) / D < LOADS) {
+          constexpr int l = (q - B1) / D;
+          mma_load<l * WAVES * 1024>(
+              acc[i][j], fw[set][j], fx[set][i], l < XL ? p.rx : p.rw,
+              voff[l], l < XL ? p.sx : p.sw, l < XL ? lx : lw);
+        } else {
+          mma(acc[i][j], fw[set][j], fx[set][i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (q % R1 == 0 && q / R1 < R) frag(1, bx, bw, q / R1);
+        if constexpr (q > B2 && (q - B2 - 1) % R2 == 0 && (q - B2 - 1) / R2 < R)
+          frag(0, nx, nw, (q - B2 - 1) / R2);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      each<2 * F>(slot);
       bx = nx;
       bw = nw;
       settle(__builtin_amdgcn_readfirstlane(kn - 1 - t));
@@ -429,33 +531,34 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tiles_kernel(
     for (int i = 0; i < FM; ++i) {
       const int m = here.m0 + (wm * FM + i) * 16 + fr;
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (GLU) {
+      constexpr int RESULTS = GLU ? FN / 2 : FN;
+      const int n0 = (GLU ? here.n0 / 2 : here.n0) + wn * RESULTS * 16;
+      const int cols = GLU ? N / 2 : N;
+      u32x2v held = {};
 #pragma unroll
-        for (int j = 0; j < FN / 2; ++j) {
-          const int n = here.n0 / 2 + (wn * FN / 2 + j) * 16 + fk * 4;
-          if (m >= M || n >= N / 2) continue;
-          float g[4], u[4];
-          take(g, acc[i][j]);
-          take(u, acc[i][j + FN / 2]);
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            g[e] = ends::gate(g[e], u[e], KIND == GELU);
-          put((uint16_t *)y + (int64_t)m * (N / 2) + n, g);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const int n = here.n0 + (wn * FN + j) * 16 + fk * 4;
-          if (m >= M || n >= N) continue;
-          float f[4];
-          take(f, acc[i][j]);
-          if constexpr (KIND == PARTS) {
+      for (int j = 0; j < RESULTS; ++j) {
+        float f[4];
+        take(f, acc[i][j]);
+        if constexpr (KIND == PARTS) {
+          const int n = n0 + j * 16 + fk * 4;
+          if (m < M && n < N)
             *reinterpret_cast<f32x4v *>(
                 (float *)y + ((int64_t)blockIdx.y * M + m) * N + n) =
                 (f32x4v){f[0], f[1], f[2], f[3]};
-          } else {
-            put((uint16_t *)y + (int64_t)m * N + n, f);
+        } else {
+          if constexpr (GLU) {
+            float u[4];
+            take(u, acc[i][j + FN / 2]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              f[e] = ends::gate(f[e], u[e], KIND == GELU);
           }
+          uint16_t *row = (uint16_t *)y + (int64_t)m * cols;
+          if (j % 2 == 1)
+            put(row, held, packed(f), n0 + j * 16 - 16, fk, cols, m < M);
+          else if (j + 1 == RESULTS)
+            put(row, packed(f), n0 + j * 16, fk, cols, m < M);
+          held = packed(f);
         }
       }
     }

@@ -408,3 +408,32 @@ def test_parts_are_not_differentiated():
     ref = x.float() + parts.sum(0)
     # one rounding, and the order of three fp32 terms of up to 5
     assert bool(((s.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2e-6).all())
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("n", [8, 24, 264, 1048])
+def test_stores_of_eight_columns(tile, n):
+    """Rows of whole pieces of 16 bytes that end within a pair of 16 x 16 results,
+    and behind the first of one: y and its unit."""
+    from runbooks_amd import ops
+    x, w = _inputs(131, 2 * n, 320)
+    _check(ops.ext().tile_gemm(x, w[:n].contiguous(), tile=tile), x, w[:n],
+           2.0 ** -8)
+    g, u = (x.float() @ w.float().t()).chunk(2, 1)
+    ref = torch.nn.functional.silu(g) * u
+    got = ops.ext().tile_gemm(x, w, glu=1, tile=tile).float()
+    assert bool(((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4).all())
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("widths", [[48], [16, 32], [208, 16, 48]])
+def test_adapters_of_odd_results(tile, widths):
+    """An odd number of 16 x 16 results, and siblings that meet within a pair."""
+    from runbooks_amd import ops
+    x, w = _inputs(131, sum(widths), 320)
+    t = torch.randn(len(widths), 131, 16, device="cuda").bfloat16()
+    bs = [torch.randn(n, 16, device="cuda").bfloat16() for n in widths]
+    got = ops.ext().tile_lora(x, w, t, bs, 0.3, tile=tile)
+    ref = _with_adapters(x, w, t, bs, 0.3)
+    bound = 2.0 ** -8 * ref.abs() + 2.0 ** -24 * (2 * 320 ** 1.5 + 2 * 16 * 16)
+    assert bool(((got.float() - ref).abs() <= bound).all())

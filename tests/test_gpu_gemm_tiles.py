@@ -437,3 +437,18 @@ def test_adapters_of_odd_results(tile, widths):
     ref = _with_adapters(x, w, t, bs, 0.3)
     bound = 2.0 ** -8 * ref.abs() + 2.0 ** -24 * (2 * 320 ** 1.5 + 2 * 16 * 16)
     assert bool(((got.float() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m,n,k,tiles", [
+    (321, 8192, 4096, True), (512, 6144, 4096, False), (900, 4096, 4096, True),
+    (513, 3328, 256, False), (1030, 2052, 2048, True), (1400, 20484, 512, False),
+    (1400, 4096, 8256, False)])
+def test_wide_products(monkeypatch, m, n, k, tiles):
+    """wide_linear and wide_product, on either side of the rule for tiles."""
+    from runbooks_amd import ops
+    from runbooks_amd.ops import linear
+    x, w = _inputs(m, n, k)
+    assert linear._wide_in_tiles(m, n, k) is tiles
+    with torch.no_grad():
+        _check(ops.wide_linear(x, w), x, w, 2.0 ** -8)
+        _check(linear.wide_product(x, w), x, w, 2.0 ** -8)

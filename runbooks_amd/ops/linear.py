@@ -324,7 +324,7 @@ def wide_product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """x @ weight^T on the GPU for a result that is not differentiated, in
     whole rounds of tiles."""
     rows, cols = x.shape[0], weight.shape[0]
-    if rows > 320 and _wide_in_tiles(rows, cols, x.shape[1]) and \
+    if _many_in_tiles(rows, cols, x.shape[1]) and \
             _backend.ext().tile_gemm_takes(x, weight):
         return _backend.ext().tile_gemm(x, weight)
     y = _one_round(x, weight)
@@ -347,21 +347,24 @@ def _wide_in_tiles(m: int, n: int, k: int) -> bool:
     and 64; 18432 x 3072 256 51 and 45; 12288 x 1024 256 17 and 16, 320 17 and 18).
     Wider ones the library takes in whole rounds (24576 x 4096 192 58 and 60,
     320 72 and 79; 32768 x 1024 320 26 and 31; 24576 x 8192 129 100 and 119), of
-    narrower ones there are too few tiles (6144 x 4096 200 25 and 34).
-
-    More rows: wherever they make up 64 tiles of 256 x 256, or 40 of short sums,
-    which the library takes long to begin and end (6144 x 4096 512 36 and 39, 900
-    51 and 45, 2048 81 and 75, 7931 271 and 268; 12288 x 3072 512 43 and 42, 1021 67
-    and 59, 3001 193 and 173; 15360 x 5120 1021 144 and 118; 4608 x 3584 640 30 and
-    36, 900 41 and 35, 1100 41 and 43, 2500 68 and 65; 3072 x 2048 512 14 and 17, 1021
-    21 and 17, 2048 26 and 25; 4096 x 4096 768 33 and 38, 900 37 and 33, 1280 46 and
-    48, 2048 59 and 57; 10240 x 8192 1021 146 and 143). Of 182 sizes of 2304 to 20480
-    columns and sums of 768 to 8192 25 are slower, by up to 6%, the mean is 0.95."""
-    if m > 320:
-        tiles = -(-m // 256) * -(-n // 256)
-        return n <= 20480 and 256 <= k <= 8192 and tiles >= (64 if k > 2048 else 40)
+    narrower ones there are too few tiles (6144 x 4096 200 25 and 34)."""
     return 12288 <= n < 20480 and \
         (m <= 256 or (m <= 320 and n < 15360 and 2048 <= k < 8192))
+
+
+def _many_in_tiles(m: int, n: int, k: int) -> bool:
+    """The same of more rows: wherever they make up 64 tiles of 256 x 256, or 40 of
+    short sums, which the library takes long to begin and end (us there and in tiles:
+    6144 x 4096 512 rows 36 and 39, 900 51 and 45, 2048 81 and 75, 7931 271 and 268;
+    12288 x 3072 512 43 and 42, 1021 67 and 59, 3001 193 and 173; 15360 x 5120 1021
+    144 and 118; 4608 x 3584 640 30 and 36, 900 41 and 35, 1100 41 and 43, 2500 68 and
+    65; 3072 x 2048 512 14 and 17, 1021 21 and 17, 2048 26 and 25; 4096 x 4096 768 33
+    and 38, 900 37 and 33, 1280 46 and 48, 2048 59 and 57; 10240 x 8192 1021 146 and
+    143). Of 182 sizes of 2304 to 20480 columns and sums of 768 to 8192 25 are slower,
+    by up to 6%, the mean is 0.95."""
+    tiles = -(-m // 256) * -(-n // 256)
+    return m > 320 and n <= 20480 and 256 <= k <= 8192 and \
+        tiles >= (64 if k > 2048 else 40)
 
 
 def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -374,7 +377,8 @@ def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     6144 x 4096 15.9 and 15.4, of 24 rows 47.9 and 52.6, 14.7 and 15.0)."""
     if x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2:
         (m, k), n = x.shape, weight.shape[0]
-        if _wide_in_tiles(m, n, k) and _tiles_serve(x, weight):
+        if (_wide_in_tiles(m, n, k) or _many_in_tiles(m, n, k)) and \
+                _tiles_serve(x, weight):
             return _backend.ext().tile_gemm(x, weight)
         if m > 1280:
             return wide_product(x, weight)

@@ -448,7 +448,7 @@ def test_wide_products(monkeypatch, m, n, k, tiles):
     from runbooks_amd import ops
     from runbooks_amd.ops import linear
     x, w = _inputs(m, n, k)
-    assert linear._wide_in_tiles(m, n, k) is tiles
+    assert linear._many_in_tiles(m, n, k) is tiles
     with torch.no_grad():
         _check(ops.wide_linear(x, w), x, w, 2.0 ** -8)
         _check(linear.wide_product(x, w), x, w, 2.0 ** -8)

@@ -396,11 +396,10 @@ def _lora_in_tiles(m: int, n: int, k: int) -> bool:
 
     Rows of up to 5120: where the result is wide or has more than 32 tiles of 256 x
     256 (us in the library with the pass and in tiles: 12288 x 4096 129 rows 44 and
-    38, 2048 174 and 163, 3001 258 and 242; 6144 x 4096 129 44 and 34, 3001 143 and
-    135; 22016 x 4096 700 149 and 127, 2600 394 and 391; 28672 x 4096 2048 388 and
-    393; 27648 x 5120 1536 393 and 346; 4096 x 4096 900 42 and 36, 512 34 and 39;
-    2048 x 2048 1800 25 and 20), up to where the library has whole rounds of its
-    larger tiles (22016 x 4096 3001 436 and 478, 4096 588 and 614).
+    38, 2048 169 and 169, 3001 251 and 232; 6144 x 4096 129 44 and 34, 3001 143 and
+    135; 22016 x 4096 700 149 and 127, 2300 359 and 334; 28672 x 4096 2048 385 and
+    364; 27648 x 5120 1536 393 and 346; 4096 x 4096 900 42 and 36, 512 34 and 39;
+    2048 x 2048 1800 25 and 20), of up to 60 million results (_large_lora_in_tiles).
 
     Longer rows: where one round of tiles does (4096 x 11008 1800 158 and 139, 2048
     164 and 146, 3001 209 and 201; 4096 x 14336 2048 205 and 185; 5120 x 13824 1536
@@ -418,12 +417,23 @@ def _lora_in_tiles(m: int, n: int, k: int) -> bool:
         any(224 <= t <= 256 for t in (tiles(256, 128), tiles(192, 256)))
 
 
+def _large_lora_in_tiles(m: int, n: int, k: int) -> bool:
+    """The same of results of more than 60 million (us in the library with the pass and
+    in tiles: 22016 x 4096 3001 rows 447 and 430, 8192 1129 and 1072; 28672 x 4096 2300
+    420 and 387, 3001 564 and 543, 8192 1438 and 1342; 27648 x 5120 4096 915 and 825;
+    12288 x 4096 8192 631 and 608; 11264 x 2048 6000 257 and 241; a step of mistral-7b,
+    3001 tokens, 97.7 ms and 96.1)."""
+    return m * n > 60_000_000 and n >= 6144 and 256 <= k <= 5120
+
+
 def wide_product_lora(x: torch.Tensor, weight: torch.Tensor, t: torch.Tensor,
                       bs: list, scale: float) -> torch.Tensor:
     """wide_product(x, weight) + scale t_i B_i^T of adapters side by side
     (csrc/lora_group.hip)."""
     ext, (n, k) = _backend.ext(), weight.shape
-    if _lora_in_tiles(x.shape[0], n, k) and ext.tile_gemm_takes(x, weight):
+    m = x.shape[0]
+    if (_lora_in_tiles(m, n, k) or _large_lora_in_tiles(m, n, k)) and \
+            ext.tile_gemm_takes(x, weight):
         return ext.tile_lora(x, weight, t, bs, scale)
     y = wide_product(x, weight)
     ext.lora_add_(y, t, bs, scale, False)

@@ -452,3 +452,21 @@ def test_wide_products(monkeypatch, m, n, k, tiles):
     with torch.no_grad():
         _check(ops.wide_linear(x, w), x, w, 2.0 ** -8)
         _check(linear.wide_product(x, w), x, w, 2.0 ** -8)
+
+
+@pytest.mark.parametrize("m,n,k,tiles", [
+    (3001, 20480, 256, True), (9800, 6144, 320, True), (2900, 20480, 256, False),
+    (9800, 6140, 256, False), (3001, 20480, 5184, False)])
+def test_large_products_with_adapters(m, n, k, tiles):
+    from runbooks_amd.ops import linear
+    assert linear._large_lora_in_tiles(m, n, k) is \
+        (tiles and not linear._lora_in_tiles(m, n, k))
+    if not tiles:
+        return
+    x, w = _inputs(m, n, k)
+    t = torch.randn(1, m, 16, device="cuda").bfloat16()
+    bs = [torch.randn(n, 16, device="cuda").bfloat16()]
+    ref = _with_adapters(x, w, t, bs, 0.3)
+    bound = 2.0 ** -8 * ref.abs() + 2.0 ** -24 * (2 * k ** 1.5 + 2 * 16 * 16)
+    got = linear.wide_product_lora(x, w, t, bs, 0.3)
+    assert bool(((got.float() - ref).abs() <= bound).all())

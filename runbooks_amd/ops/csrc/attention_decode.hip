@@ -95,7 +95,9 @@ RB_DEV Place shifted_place() {
 // 1000 to 4003 128 and 118 (5.7 TB/s), 32 of 100 to 4000 in two parts 61 and 55; 16
 // heads of 256: 7 of 90 to 1801 in parts 32.4 and 29.1, 16 of 100 to 2000 60 and 57.
 // Where nothing is uneven it costs 0.2 to 0.4 us (32 of 100 with a table of 4096
-// 14.0 and 14.2, 8 of 400 18.0 and 18.2), so tables of up to 512 tokens go by shifts.
+// 14.0 and 14.2, 8 of 400 18.0 and 18.2), so tables of up to 512 tokens go by shifts,
+// as do up to four sequences, whose parts are all begun at once (of two and three
+// within 1% either way).
 RB_DEV Place sorted_place(const int32_t *lens, const int32_t *starts) {
   __shared__ int found;
   const int B = gridDim.x, hkv = gridDim.y, of_each = hkv * gridDim.z;
@@ -842,7 +844,7 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
   uint16_t *swz = out_swz.has_value() ? (uint16_t *)out_swz->data_ptr()
                                       : nullptr;
   const int64_t longest = (int64_t)max_blocks * bs;
-  const bool sorted = B > 1 && B <= 64 && longest > 512;
+  const bool sorted = B > 4 && B <= 64 && longest > 512;
   // MFMA route: keyed on the TRANSPOSED V layout (bf16 [Dh, BS] /
   // fp8 [Dh+4, BS] blocks) the allocator chooses for MFMA-eligible
   // models (G >= 4, DH <= 128, 16-token blocks — RB_DECODE_MFMA=0 at

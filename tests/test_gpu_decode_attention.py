@@ -61,7 +61,7 @@ def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
 
 @pytest.mark.parametrize("hq,hkv,nsplit", [(3, 3, 1), (5, 5, 3), (8, 2, 1),
                                            (8, 2, 2)])
-@pytest.mark.parametrize("batch", [2, 31, 64, 65])
+@pytest.mark.parametrize("batch", [2, 4, 5, 31, 64, 65])
 def test_sorted_sequences(batch, hq, hkv, nsplit):
     """Every sequence and head is somebody's, whatever the lengths (of some the
     same, of one none that its window sees), whole and in parts, in rounds of

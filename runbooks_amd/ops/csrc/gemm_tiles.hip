@@ -242,7 +242,7 @@ __device__ __forceinline__ void end_lora(const Adapters &a,
 // Workgroups stay for all of their tiles, and the buffers are filled for the
 // next one during the end of the one before. Tiles go to XCDs in runs, down
 // bands of 8, so that those that run together share rows in its L2 (7931 x 28672
-// x 4096: 1432 us down all rows and one tile a workgroup, 1330 now).
+// x 4096: 1432 us down all rows and one tile a workgroup, 1330 so).
 //
 // DOWN: W is [K, N] and lies in LDS as it does in memory, a row of BN columns for
 // each of a K-tile's 64; ds_read_b64_tr takes operands out of it, four of a column

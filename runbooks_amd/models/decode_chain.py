@@ -229,5 +229,8 @@ def run_rows(model, x, positions, caches, slots, attend, joint: bool, *types):
         layer = _rows_layer(blocks[i], m, caches[i][0], types) \
             if i < len(blocks) else None
         if layer is None:
-            return x, ext.decode_gemm_rows(h, down.ws, down.n, down.half), i
+            # fp32 parts where a norm adds them up, as Transformer._blocks has it
+            parts = i < len(blocks) and blocks[i].fuses_residual()
+            return x, ext.decode_gemm_rows(h, down.ws, down.n, down.half,
+                                           parts), i
         x, y = _add_rows(x, h, down, layer.blk.norm1)

@@ -475,3 +475,47 @@ def test_steps_of_rows(monkeypatch, tokens, kv, inter, hidden, decode):
     assert seen == [2, 1] and len(called) == 1
     for a, b, c in zip(got, mixed, ref):
         assert _rel(a, c.double()) < 2e-2 and _rel(b, c.double()) < 2e-2
+
+
+@pytest.mark.parametrize("decode", [False, True])
+@pytest.mark.parametrize("why", ["hook", "copy", "norm"])
+def test_rows_handed_over(monkeypatch, decode, why):
+    """What run_rows leaves to the modules, of a block whose MLP has a hook, one
+    whose copy is older than its weight, and one whose norm has a hook: to a norm
+    that adds them up, the last product's sums in fp32 parts, unrounded."""
+    from runbooks_amd.models import decode_chain
+    m = _model(8, 2048)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    if decode:
+        args = _step(m, 40, False)
+    else:
+        args = (torch.arange(40, device=DEV)[None], torch.arange(40, **i32),
+                m.alloc_caches(16, DEV), torch.arange(40, **i32))
+    blk = m.blocks[1]
+    if why == "hook":
+        blk.mlp.register_forward_hook(lambda *a: None)
+    elif why == "copy":
+        with torch.no_grad():
+            blk.mlp.down_proj.weight.mul_(0.5)
+    else:
+        blk.norm2.register_forward_hook(lambda *a: None)
+    seen, given = [], []
+    run, product = decode_chain.run_rows, ops.ext().decode_gemm_rows
+
+    def run_rows(*a):
+        monkeypatch.setattr(ops.ext(), "decode_gemm_rows", lambda x, *b:
+                            given.append(x) or product(x, *b))
+        seen.append(run(*a))
+        monkeypatch.setattr(ops.ext(), "decode_gemm_rows", product)
+        return seen[-1]
+    monkeypatch.setattr(decode_chain, "run_rows", run_rows)
+    with torch.no_grad():
+        (m.decode if decode else m.prefill)(*args)
+    _, delta, blocks = seen[0]
+    assert blocks == 1
+    want = given[-1].double() @ m.blocks[0].mlp.down_proj.weight.double().t()
+    if why == "norm":           # adds no parts up
+        assert delta.dtype == torch.bfloat16 and _rel(delta, want) < BF16
+    else:
+        assert delta.dtype == torch.float32 and delta.shape[1:] == want.shape
+        assert _rel(delta.sum(0), want) < 1e-5

@@ -320,9 +320,15 @@ def _whole_rounds(rows: int, cols: int) -> int:
     return min(across // step * step * 256 or cols, cols)
 
 
+def _differentiated(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    return torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)
+
+
 def wide_product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """x @ weight^T on the GPU for a result that is not differentiated, in
-    whole rounds of tiles."""
+    """x @ weight^T on the GPU, in whole rounds of tiles; one call where the result
+    is differentiated."""
+    if _differentiated(x, weight):
+        return x @ weight.t()
     rows, cols = x.shape[0], weight.shape[0]
     if _many_in_tiles(rows, cols, x.shape[1]) and \
             _backend.ext().tile_gemm_takes(x, weight):
@@ -368,14 +374,15 @@ def _many_in_tiles(m: int, n: int, k: int) -> bool:
 
 
 def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """fast_linear for a result that is not differentiated, of rows x that are
-    there also where they have a decode operand; of many rows a wide_product.
+    """fast_linear of rows x that are there also where they have a decode operand;
+    of many rows a wide_product. A result that is differentiated is fast_linear's.
 
     From 17 to 32 rows the kernel that shares x is the faster one where it has
     about one workgroup for every CU (us without and with it, 32 rows: 22016 x
     4096 34.9 and 31.2, 12288 x 4096 23.2 and 21.7; 49152 x 3072 52.7 and 53.0,
     6144 x 4096 15.9 and 15.4, of 24 rows 47.9 and 52.6, 14.7 and 15.0)."""
-    if x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2:
+    if x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and \
+            not _differentiated(x, weight):
         (m, k), n = x.shape, weight.shape[0]
         if (_wide_in_tiles(m, n, k) or _many_in_tiles(m, n, k)) and \
                 _tiles_serve(x, weight):

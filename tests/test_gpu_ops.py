@@ -1303,6 +1303,34 @@ def test_wide_products(rows, n, k):
         assert (got.double() - ref).norm() < (2 ** -9 + 1e-5) * ref.norm()
 
 
+@pytest.mark.parametrize("rows,n,k", [
+    (20, 10240, 1024),              # a registered copy that shares x
+    (1400, 4096, 1024),             # tiles
+    (2048, 3584, 8256),             # one round of tiles
+    (1536, 11008, 64)])             # two calls
+@pytest.mark.parametrize("which", ["x", "weight"])
+def test_wide_products_are_differentiated(rows, n, k, which):
+    """Gradients of what wide_linear and wide_product return, whichever way the
+    product would take without them: one rounding, fp32 sums."""
+    from runbooks_amd.ops.linear import (register_decode_weight, wide_linear,
+                                         wide_product)
+    torch.manual_seed(rows)
+    x = torch.randn(rows, k, device=DEV).bfloat16()
+    w = torch.randn(n, k, device=DEV).bfloat16()
+    dy = torch.randn(rows, n, device=DEV).bfloat16()
+    if rows <= 32:
+        register_decode_weight(w)
+    (x if which == "x" else w).requires_grad_()
+    want = dy.double() @ w.double() if which == "x" else \
+        dy.double().t() @ x.double()
+    ref = x.detach().double() @ w.detach().double().t()
+    for product in (wide_linear, wide_product):
+        y = product(x, w)
+        assert (y.double() - ref).norm() < 2 ** -8 * ref.norm()
+        got, = torch.autograd.grad(y, x if which == "x" else w, dy)
+        assert (got.double() - want).norm() < 2 ** -8 * want.norm()
+
+
 @pytest.mark.parametrize("M", [1, 32, 33, 64, 65, 128])
 @pytest.mark.parametrize("N,K", [(32, 1024), (96, 1040), (20512, 1024),
                                  (160, 8208), (4096, 4096)])

@@ -467,7 +467,21 @@ def wide_product_grad(dy: torch.Tensor, weight: torch.Tensor,
 def _library_grad(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """Wide results in whole rounds of tiles, like wide_product's (2048 rows of
     4096 to 11008 columns: 284 and 171 us; to 4096 and 6144 columns 3 to 14%
-    slower in two calls)."""
+    slower in two calls). Long sums with few tiles in two fp32 halves, rounded
+    once: there the library keeps tiles of 256 x 256, of which there are not
+    enough (us in one sum and in two, to 4096 columns: 2048 rows of 22016 453
+    and 372, 512 213 and 163, 1024 rows of 28672 359 and 307, 2048 401 and 463;
+    2049 rows of 17408 325 and 300, 2304 367 and 314; with more tiles, 2560 rows
+    of 22016, 372 and 390; of 12288 and 2048 rows 195 and 213). From 60 to 2300
+    rows two are 20% faster of 22016, 17% of 24576 to 3072 columns, 5% of 28672,
+    if 16384 < n <= 32768 and k % 4 == 0 and \
+            -(-rows // 256) * -(-k // 256) <= 144:
+        half = n // 128 * 64
+        parts = torch.empty(2, rows, k, dtype=torch.float32, device=dy.device)
+        for part, at in zip(parts, (slice(0, half), slice(half, n))):
+            torch.mm(dy[:, at], weight[at], out_dtype=torch.float32, out=part)
+        return _backend.ext().sum_parts(parts)
+    and 11% slower of 49152 to 3072 (1024 rows 435 and 516, 2048 523 and 885)."""
     rows, (n, k) = dy.shape[0], weight.shape
     if k >= 8192:
         main = _whole_rounds(rows, k)

@@ -1331,6 +1331,25 @@ def test_wide_products_are_differentiated(rows, n, k, which):
         assert (got.double() - want).norm() < 2 ** -8 * want.norm()
 
 
+@pytest.mark.parametrize("rows,n,k,halves", [
+    (20, 16448, 64, True), (2304, 17408, 4096, True), (300, 32768, 60, True),
+    (20, 16384, 64, False), (20, 32832, 64, False), (20, 16448, 62, False)])
+def test_long_sums_of_input_gradients(monkeypatch, rows, n, k, halves):
+    """Sums that are left to the library and long go in two fp32 halves, rounded
+    once: on either side of the rule."""
+    from runbooks_amd.ops import linear
+    torch.manual_seed(rows)
+    dy = torch.randn(rows, n, device=DEV).bfloat16()
+    w = torch.randn(n, k, device=DEV).bfloat16()
+    summed, sum_parts = [], ops.ext().sum_parts
+    monkeypatch.setattr(ops.ext(), "sum_parts",
+                        lambda p: summed.append(p.shape) or sum_parts(p))
+    got = linear.wide_product_grad(dy, w)
+    assert summed == ([(2, rows, k)] if halves else [])
+    ref = dy.double() @ w.double()
+    assert (got.double() - ref).norm() < (2 ** -9 + 1e-5) * ref.norm()
+
+
 @pytest.mark.parametrize("M", [1, 32, 33, 64, 65, 128])
 @pytest.mark.parametrize("N,K", [(32, 1024), (96, 1040), (20512, 1024),
                                  (160, 8208), (4096, 4096)])

@@ -41,6 +41,7 @@ void affine_add_(at::Tensor x, at::Tensor w, c10::optional<at::Tensor> bias, at:
 at::Tensor embed_res32(at::Tensor tokens, at::Tensor positions, at::Tensor table, at::Tensor places);
 at::Tensor sum_parts(at::Tensor parts);
 bool tile_gemm_takes(at::Tensor x, at::Tensor w, bool glu);
+bool tile_gemm_pays(int64_t M, int64_t N, int64_t K);
 bool rows_res_supported(int64_t M, int64_t N, int64_t K);
 bool parts_res_supported(int64_t N);
 std::vector<at::Tensor> parts_res(at::Tensor parts, at::Tensor res, at::Tensor norm);
@@ -178,6 +179,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sum_parts", &sum_parts, "fp32 [P, M, N] -> their sum [M, N] bf16");
   m.def("tile_gemm_takes", &tile_gemm_takes, py::arg("x"), py::arg("w"),
         py::arg("glu") = false, "whether tile_gemm takes x and W");
+  m.def("tile_gemm_pays", &tile_gemm_pays, py::arg("M"), py::arg("N"),
+        py::arg("K"), "whether it is as good as the library");
   m.def("parts_res_supported", &parts_res_supported);
   m.def("parts_res", &parts_res, "the same of fp32 parts of the product");
   m.def("rows_res_supported", &rows_res_supported);

@@ -757,6 +757,51 @@ bool tile_gemm_takes(at::Tensor x, at::Tensor w, bool glu) {
          (!glu || w.size(0) * w.size(1) * 2 < ((int64_t)1 << 32));
 }
 
+// Whether a product of more than 320 rows is as good in tiles as in the library, which
+// has tiles of 256 x 256 and others, is slow at columns that are no multiple of 256,
+// and takes short sums (up to 512) long to begin and end.
+//
+// Up to one round of 256 x 256: where columns are a multiple, tiles that fill the CUs
+// (85% of a round; small ones 70%), or whole bands of rows (1, 2, 4, 8) of which the
+// library pads more than a tenth. us there and in tiles: 1021 x 12288 x 3072 65 and 59,
+// 400 x 10240 x 4096 48 and 42, 512 x 12288 x 4096 55 and 53; not: 1280 x 4096 x 4096
+// 47 and 49, 640 x 8192 x 3072 38 and 40, 330 x 8192 x 4096 33 and 35.
+//
+// More rounds: not where they are whole or nearly whole for the library (7931 x 6144 x
+// 4096 275 and 283, 2048 x 8192 x 2560 65 and 69), nor of sums past 6144, which it
+// takes as fast (mean 1.00 of 641 sizes).
+//
+// Of 15098 sizes, 321 to 24576 rows, 256 to 20480 columns and sums of 256 to 8192, 12347
+// go by tiles: the mean is 0.87 of the library's time, 414 are slower by more than 3%
+// and 106 by more than 6%. Of the others the mean would be 0.99, 917 and 414.
+bool tile_gemm_pays(int64_t M, int64_t N, int64_t K) {
+  const int64_t down = (M + 255) / 256, across = (N + 255) / 256;
+  const int64_t all = down * across;
+  if (M <= 320 || M > 24576 || N < 256 || N > 20480 || K < 256 || K > 8192 ||
+      all < (K > 2048 ? 64 : 40))
+    return false;
+  if (K <= 512) return true;
+  const bool padded = N % 256 != 0;
+  const Choice c = choose_two(M, N, K);
+  const Tile &t = TILES[c.tile];
+  const bool large = t.bm == 256 && t.bn == 256;
+  if (all <= 256) {
+    if (c.rest >= 0 || padded || large) return c.rest < 0 && padded;
+    const int64_t tm = (M + t.bm - 1) / t.bm, tn = (N + t.bn - 1) / t.bn;
+    const int64_t slots = (tm * tn + 255) / 256 * 256;
+    const double fill = (double)(M * N) / (double)(slots * t.bm * t.bn);
+    if (t.bm == 128 && t.bn == 128) return K <= 2048 || fill >= 0.7;
+    return fill >= 0.85 || (t.bm != 192 && 8 % tm == 0 &&
+                            M * 10 < down * 2304 && tm * tn * 4 >= slots * 3);
+  }
+  if (all % 256 == 0) return padded && K <= 6144;
+  if (down <= 5) return true;
+  if (K > 6144) return false;
+  const int64_t step = 256 / down;      // columns of tiles in a round
+  if (c.rest >= 0) return down * step < 256;
+  return padded || !large || down * step < 230 || across % step != 0;
+}
+
 // Parts that tile_gemm makes of sums where it may.
 int64_t tile_gemm_parts(int64_t M, int64_t N, int64_t K) {
   return choose(M, N, K, MAX_PARTS, -1).parts;

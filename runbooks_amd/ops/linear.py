@@ -359,18 +359,8 @@ def _wide_in_tiles(m: int, n: int, k: int) -> bool:
 
 
 def _many_in_tiles(m: int, n: int, k: int) -> bool:
-    """The same of more rows: wherever they make up 64 tiles of 256 x 256, or 40 of
-    short sums, which the library takes long to begin and end (us there and in tiles:
-    6144 x 4096 512 rows 36 and 39, 900 51 and 45, 2048 81 and 75, 7931 271 and 268;
-    12288 x 3072 512 43 and 42, 1021 67 and 59, 3001 193 and 173; 15360 x 5120 1021
-    144 and 118; 4608 x 3584 640 30 and 36, 900 41 and 35, 1100 41 and 43, 2500 68 and
-    65; 3072 x 2048 512 14 and 17, 1021 21 and 17, 2048 26 and 25; 4096 x 4096 768 33
-    and 38, 900 37 and 33, 1280 46 and 48, 2048 59 and 57; 10240 x 8192 1021 146 and
-    143). Of 182 sizes of 2304 to 20480 columns and sums of 768 to 8192 25 are slower,
-    by up to 6%, the mean is 0.95."""
-    tiles = -(-m // 256) * -(-n // 256)
-    return m > 320 and n <= 20480 and 256 <= k <= 8192 and \
-        tiles >= (64 if k > 2048 else 40)
+    """The same of more rows (tile_gemm_pays in csrc/gemm_tiles.hip)."""
+    return m > 320 and _backend.ext().tile_gemm_pays(m, n, k)
 
 
 def wide_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:

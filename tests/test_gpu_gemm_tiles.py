@@ -440,18 +440,27 @@ def test_adapters_of_odd_results(tile, widths):
 
 
 @pytest.mark.parametrize("m,n,k,tiles", [
-    (321, 8192, 4096, True), (512, 6144, 4096, False), (900, 4096, 4096, True),
+    (321, 8192, 4096, False), (512, 6144, 4096, False), (900, 4096, 4096, True),
     (513, 3328, 256, False), (1030, 2052, 2048, True), (1400, 20484, 512, False),
-    (1400, 4096, 8256, False)])
+    (1400, 4096, 8256, False),
+    (400, 8196, 4096, True),        # no multiple of 256
+    (1280, 4096, 2560, False), (2048, 3072, 2560, True),    # CUs idle, and not
+    (2048, 8192, 1024, False), (1900, 11004, 512, True),    # whole rounds, short
+    (2816, 6144, 1024, True), (2816, 6144, 6208, False),    # more rounds
+    (10300, 256, 1024, True), (16384, 252, 512, False), (24600, 256, 256, False)])
 def test_wide_products(monkeypatch, m, n, k, tiles):
-    """wide_linear and wide_product, on either side of the rule for tiles."""
+    """wide_linear and wide_product go by the rule for tiles, on either side."""
     from runbooks_amd import ops
     from runbooks_amd.ops import linear
     x, w = _inputs(m, n, k)
     assert linear._many_in_tiles(m, n, k) is tiles
+    called, tile_gemm = [], ops.ext().tile_gemm
+    monkeypatch.setattr(ops.ext(), "tile_gemm",
+                        lambda *a, **kw: called.append(1) or tile_gemm(*a, **kw))
     with torch.no_grad():
-        _check(ops.wide_linear(x, w), x, w, 2.0 ** -8)
-        _check(linear.wide_product(x, w), x, w, 2.0 ** -8)
+        for i, product in enumerate((ops.wide_linear, linear.wide_product), 1):
+            _check(product(x, w), x, w, 2.0 ** -8)
+            assert len(called) == (i if tiles else 0)
 
 
 @pytest.mark.parametrize("m,n,k,tiles", [

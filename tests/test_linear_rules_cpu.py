@@ -40,3 +40,24 @@ def test_sums_in_parts(m, n, k, parts):
     (128, 22016, 4096, False)])
 def test_products_with_adapters(m, n, k, tiles):
     assert linear._lora_in_tiles(m, n, k) is tiles
+
+
+@pytest.mark.parametrize("m,n,k,tiles", [
+    # one round of 256 x 256: columns that are a multiple of 256 and others
+    (1021, 12288, 3072, True), (512, 12288, 4096, True), (400, 10240, 4096, True),
+    (900, 4096, 4096, True), (1280, 4096, 4096, False), (640, 8192, 3072, False),
+    (330, 8192, 4096, False), (2048, 6144, 4096, True), (640, 8256, 3072, True),
+    (1280, 4160, 4096, True),
+    # small tiles of short sums
+    (1280, 2048, 2048, True), (330, 5120, 4096, False),
+    # more rounds
+    (900, 18432, 8192, True), (7931, 6144, 4096, False), (7931, 6208, 4096, True),
+    (2048, 8192, 2560, False), (2500, 12288, 6144, True),
+    (2500, 12288, 6208, False), (2048, 9216, 4096, False),
+    # narrow, short, and past what was measured
+    (10300, 256, 1024, True), (10300, 248, 1024, False), (16384, 16, 256, False),
+    (24576, 12288, 512, True), (24577, 12288, 512, False),
+    (2048, 20480, 256, True), (2048, 20736, 256, False), (2048, 12288, 192, False)])
+def test_wide_products_of_many_rows(m, n, k, tiles):
+    pytest.importorskip("runbooks_amd.ops._hip_core")
+    assert linear._many_in_tiles(m, n, k) is tiles

@@ -917,24 +917,35 @@ bool tile_gemm_down_takes(at::Tensor x, at::Tensor w) {
 }
 
 // Whether tile_gemm_down, with the parts' sum, is as good as the library and a pass
-// for the adapters. It is not where one launch leaves CUs idle, of sums that are not
-// much longer than the result is wide: there the library splits them (us there and
-// here: 12288 to 4096 columns, 2500 rows 213 and 238; 4096 to 4096, 1100 rows 51 and
-// 56; 5632 to 2048, 2500 rows 68 and 75; 8192 to 8192, 1100 rows 139 and 148). Of 295
-// other sizes, 33 to 8192 rows of 2048 to 57344 columns, 14 are slower, by 3 to 6%
-// and one by 12 (300 rows, 4096 to 11008, 53 and 59), the mean is 0.78: 12288 to 4096,
-// 300 rows 118 and 56, 2048 198 and 172; 22016 to 4096, 512 rows 202 and 99, 2048 359
-// and 297, 3001 428 and 431; 4096 to 11008, 2048 rows 179 and 168; 4096 to 14336, 3001
-// rows 317 and 292.
+// for the adapters: 300 rows of 12288 to 4096 columns 56 us, 118 there, 2048 rows 172
+// and 198; of 22016 to 4096 512 rows 99 and 202, 2048 297 and 359; of 4096 to 11008
+// 2048 rows 168 and 179. It is not (us there and here)
+//  - of a few rows, and of results of less than 64K in narrow columns, whose sums the
+//    library splits further (33 x 768 of 8192 19 and 23, 129 x 256 of 4096 13 and 17);
+//  - of small results and short sums, where begin and end count (300 x 1024 of 1024
+//    12.2 and 13.6, 400 x 2048 of 2048 17.5 and 19.5);
+//  - where one launch leaves CUs idle, of sums that are not much longer than the result
+//    is wide (2500 x 4096 of 12288 213 and 238, 1100 x 4096 of 4096 51 and 56, 2500 x
+//    2048 of 5632 68 and 75, 1100 x 8192 of 8192 139 and 148).
+// Of 17362 other sizes, 33 to 24576 rows of 64 to 20480 columns and sums of 256 to 57344,
+// with one adapter, the mean is 0.69 of the library's time; 196 are slower by more than
+// 3%, and of those of 2048 columns and more 73 of 9476: long sums whose tiles are as many
+// and as large as the library's (3001 x 4096 of 28672 556 and 579), which it makes up
+// for in a step (two adapters, lower clocks: mistral-7b, 3001 tokens, 96.3 ms and 97.1
+// with the library there).
 bool tile_gemm_down_pays(int64_t M, int64_t N, int64_t K) {
-  if (M <= 32) return false;            // a few rows were not measured
+  if (M <= 32 || M > 24576 || N < 64 || K > 57344) return false;
   const Choice c = choose_down(M, N, K, MAX_PARTS, -1);
   if (c.tile < 0) return false;
   const Tile &t = TILES[c.tile];
   const int64_t tiles = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn);
-  const int64_t rounds = (tiles + 255) / 256;
-  return !(M >= 1024 && c.parts == 1 && c.rest < 0 && tiles * 10 < rounds * 2304 &&
-           N <= K && (N <= 4096 || K < 2 * N));
+  const int64_t rounds = (tiles + 255) / 256, all = M * N;
+  const bool one = c.parts == 1 && c.rest < 0;
+  if (N < 2048 && all < 65536 && K > 1024) return false;
+  if (one && K > 512 && K <= 1024 && all >= 20000 && all < 500000) return false;
+  if (K > 1024 && K <= 2048 && all >= 250000 && all < 1000000) return false;
+  return !(M >= 1024 && one && tiles * 10 < rounds * 2304 && N <= K &&
+           (N <= 4096 || K < 2 * N));
 }
 
 std::vector<int64_t> tile_gemm_down_choice(int64_t M, int64_t N, int64_t K,

@@ -61,3 +61,22 @@ def test_products_with_adapters(m, n, k, tiles):
 def test_wide_products_of_many_rows(m, n, k, tiles):
     pytest.importorskip("runbooks_amd.ops._hip_core")
     assert linear._many_in_tiles(m, n, k) is tiles
+
+
+@pytest.mark.parametrize("m,n,k,tiles", [
+    (2048, 4096, 22016, True), (512, 4096, 22016, True), (300, 4096, 12288, True),
+    (2048, 11008, 4096, True), (3001, 14336, 4096, True),
+    # a few rows, narrow columns
+    (32, 4096, 4096, False), (33, 4096, 4096, True), (33, 768, 8192, False),
+    (129, 256, 4096, False), (2048, 16, 4096, False), (2048, 64, 4096, True),
+    # small results of short sums
+    (300, 1024, 1024, False), (300, 1024, 512, True), (400, 2048, 2048, False),
+    (700, 2048, 2048, True),
+    # few tiles, and enough
+    (1100, 4096, 4096, False), (2304, 4096, 17408, False),
+    (3001, 4096, 28672, True),
+    # past what was measured
+    (24577, 4096, 4096, False), (2048, 4096, 57408, False)])
+def test_gradients_of_inputs(m, n, k, tiles):
+    ext = pytest.importorskip("runbooks_amd.ops._hip_core")
+    assert ext.tile_gemm_down_pays(m, n, k) is tiles

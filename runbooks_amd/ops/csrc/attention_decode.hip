@@ -73,15 +73,20 @@ RB_DEV void store_operand(uint16_t *swz, int kk0, int b, const float (&v)[VE],
 // order share a CU; in plain order those would be heads of one sequence wherever
 // the batch divides 256, and the CUs of the longest ones would run long after the
 // others.
-struct Place { int b, h, split; };
+struct Place { int b, h, split, len, start; };
 
 // The sequences are shifted with head and split, once around over the whole grid:
 // a CU gets sequences spread evenly over the batch.
-RB_DEV Place shifted_place() {
+RB_DEV int shifted() {
   const unsigned y = blockIdx.y + gridDim.y * blockIdx.z;
-  const unsigned b =
-      (blockIdx.x + y * gridDim.x / (gridDim.y * gridDim.z)) % gridDim.x;
-  return {(int)b, (int)blockIdx.y, (int)blockIdx.z};
+  return (int)((blockIdx.x + y * gridDim.x / (gridDim.y * gridDim.z)) %
+               gridDim.x);
+}
+
+RB_DEV Place shifted_place(const int32_t *lens, const int32_t *starts) {
+  const int b = shifted();
+  return {b, (int)blockIdx.y, (int)blockIdx.z, lens[b],
+          starts != nullptr ? starts[b] : 0};
 }
 
 // The longest sequences first, so that none is begun late, and every other 256
@@ -94,22 +99,37 @@ RB_DEV Place shifted_place() {
 // 124, 32 of 1072 each 104 and 104; 8 kv heads of 128 with four queries each: 64 of
 // 1000 to 4003 128 and 118 (5.7 TB/s), 32 of 100 to 4000 in two parts 61 and 55; 16
 // heads of 256: 7 of 90 to 1801 in parts 32.4 and 29.1, 16 of 100 to 2000 60 and 57.
-// Where nothing is uneven it costs 0.2 to 0.4 us (32 of 100 with a table of 4096
-// 14.0 and 14.2, 8 of 400 18.0 and 18.2), so tables of up to 512 tokens go by shifts,
+// Where nothing is uneven that cost 0.3 to 0.8 us, so lengths within 128 tokens of the
+// first one's go by shifts, and what a wave has loaded is not loaded again (us of a
+// table of 4096 by shifts alone, sorted, and so: 32 of 100 13.7, 14.4 and 13.9, 64 of
+// 500 with 8 kv heads 26.9, 27.7 and 26.8, 16 of 100 with 12 heads of 64 9.0, 9.8 and
+// 9.2; 32 of 20 to 500 31.2, 29.7 and 29.5). Tables of up to 512 tokens go by shifts,
 // as do up to four sequences, whose parts are all begun at once (of two and three
-// within 1% either way).
+// within 1% either way), and more than 64, for which a wave has no lanes.
 RB_DEV Place sorted_place(const int32_t *lens, const int32_t *starts) {
-  __shared__ int found;
   const int B = gridDim.x, hkv = gridDim.y, of_each = hkv * gridDim.z;
+  const int lane = threadIdx.x & 63;
+  int len = 0, start = 0;
+  if (lane < B) {
+    len = lens[lane];
+    if (starts != nullptr) start = starts[lane];
+  }
+  const int sees = max(0, len - start);
+  const int off = sees - __builtin_amdgcn_readfirstlane(sees);
+  if (!__any(lane < B && (off > 128 || off < -128))) {
+    const int b = shifted();
+    return {b, (int)blockIdx.y, (int)blockIdx.z,
+            __builtin_amdgcn_readlane(len, b),
+            __builtin_amdgcn_readlane(start, b)};
+  }
+  __shared__ int found;
   const int all = B * of_each;
   const int id = blockIdx.x + B * (blockIdx.y + hkv * blockIdx.z);
   const int round = id & ~255;
   const int at = id & 256 ? round + min(256, all - round) - 1 - (id & 255) : id;
   if (threadIdx.x < 64) {
-    const int lane = threadIdx.x;
-    int key = -1;                       // all of them different
-    if (lane < B)
-      key = max(0, lens[lane] - (starts ? starts[lane] : 0)) * 64 + lane;
+    // all of them different
+    const int key = lane < B ? sees * 64 + lane : -1;
     int longer = 0;
 #pragma unroll
     for (int i0 = 0; i0 < 64; i0 += 8)
@@ -120,8 +140,9 @@ RB_DEV Place sorted_place(const int32_t *lens, const int32_t *starts) {
     if (lane < B && longer == at / of_each) found = lane;
   }
   __syncthreads();
-  const int rest = at % of_each;
-  return {found, rest % hkv, rest / hkv};
+  const int b = __builtin_amdgcn_readfirstlane(found), rest = at % of_each;
+  return {b, rest % hkv, rest / hkv, __builtin_amdgcn_readlane(len, b),
+          __builtin_amdgcn_readlane(start, b)};
 }
 
 // FP8: caches are e4m3 rows of fp8_row_bytes(DH) = DH bytes + f32
@@ -159,18 +180,19 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
   constexpr bool HS = (G >= NW);
   constexpr int GW = HS ? G / NW : G;
   const Place place =
-      sorted ? sorted_place(seq_lens, seq_starts) : shifted_place();
+      sorted ? sorted_place(seq_lens, seq_starts)
+             : shifted_place(seq_lens, seq_starts);
   const int b = place.b, h_kv = place.h, split = place.split;
   const int hq0 = h_kv * G;
   const int Hq = hkv * G;
 
-  const int seq_len = seq_lens[b];
+  const int seq_len = place.len;
   // Strict sliding windows: seq_starts[b] (0 when null) is the first
   // VIRTUAL position this query attends to — mistral attends to exactly
   // W trailing tokens, not the engine's retained block-aligned W..W+15.
   // Index math pre-validated on CPU: tests/test_decode_sim_cpu.py
   // (simulate_decode seq_starts).
-  const int start = (seq_starts != nullptr) ? seq_starts[b] : 0;
+  const int start = place.start;
   int t_begin = start, t_end = seq_len;
   if (SPLIT) {
     const int len = seq_len - start;
@@ -574,13 +596,14 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
   constexpr int FRW = FP8 ? 2 : 4;        // u32 words per raw fragment
 
   const Place place =
-      sorted ? sorted_place(seq_lens, seq_starts) : shifted_place();
+      sorted ? sorted_place(seq_lens, seq_starts)
+             : shifted_place(seq_lens, seq_starts);
   const int b = place.b, h_kv = place.h, split = place.split;
   const int hq0 = h_kv * G;
   const int Hq = hkv * G;
 
-  const int seq_len = seq_lens[b];
-  const int start = (seq_starts != nullptr) ? seq_starts[b] : 0;
+  const int seq_len = place.len;
+  const int start = place.start;
   int t_begin = start, t_end = seq_len;
   if (SPLIT) {
     const int len = seq_len - start;

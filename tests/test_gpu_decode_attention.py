@@ -94,6 +94,35 @@ def test_sorted_sequences(batch, hq, hkv, nsplit):
                 assert _rel(got[i], ref[i].double()) < (4 if vt else 2) * BF16
 
 
+@pytest.mark.parametrize("hq,hkv,nsplit", [(5, 5, 3), (8, 2, 1)])
+@pytest.mark.parametrize("batch", [5, 40, 64])
+@pytest.mark.parametrize("spread", [0, 128, 129])
+def test_even_sequences_of_a_wide_table(hq, hkv, nsplit, batch, spread):
+    """Lengths that are within 128 of the first one's, and just not, with windows
+    and without: every sequence's own result."""
+    torch.manual_seed(batch)
+    dh, blocks = 64, 33
+    lens = torch.full((batch,), 300)
+    lens[1], lens[-1] = 300 + spread, 300 - spread
+    vt = hq // hkv >= 4
+    kc, vc = ops.alloc_kv_cache(batch * blocks, hkv, dh, DEV,
+                                dtype=torch.bfloat16, v_transposed=vt)
+    kc.normal_()
+    vc.normal_()
+    i32 = dict(dtype=torch.int32, device=DEV)
+    tables = torch.randperm(batch * blocks, device=DEV).to(torch.int32) \
+        .view(batch, blocks)
+    q = torch.randn(batch, hq, dh, device=DEV).bfloat16()
+    for s in (None, torch.arange(batch) % 7 * 20):
+        got = ops.ext().paged_decode_swz(
+            q, kc, vc, tables, lens.to(**i32), nsplit, dh ** -0.5,
+            None if s is None else s.to(**i32))[0].cpu()
+        ref = ops.paged_decode_ref(q.cpu(), kc.cpu(), vc.cpu(), tables.cpu(),
+                                   lens, dh ** -0.5, s)
+        for i in range(batch):          # 16-bit probabilities in matrix products
+            assert _rel(got[i], ref[i].double()) < (4 if vt else 2) * BF16
+
+
 def test_uneven_captured_bucket():
     """One long sequence among short ones and rows that pad the batch, by the
     split of a captured step: each the plain result."""

@@ -185,7 +185,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("parts_res", &parts_res, "the same of fp32 parts of the product");
   m.def("rows_res_supported", &rows_res_supported);
   m.def("rows_res", &rows_res,
-        "x W^T + residual of 17 to 64 rows x, times the next norm's weight, and "
+        "x W^T + residual of 33 to 64 rows x, times the next norm's weight, and "
         "parts of its squares");
   m.def("tile_lora", &tile_lora, py::arg("x"), py::arg("w"), py::arg("t"),
         py::arg("bs"), py::arg("scale"), py::arg("tile") = -1,

@@ -148,7 +148,7 @@ __global__ __launch_bounds__(BLOCK, 1) void decode_res_kernel(Sum a) {
   if (en == 0) a.squares[(int64_t)em * gridDim.x + blockIdx.x] = ss;
 }
 
-// The same of 17 to 64 rows x as they lie, B blocks of 16. x is as long as W's share
+// The same of 33 to 64 rows x as they lie, B blocks of 16. x is as long as W's share
 // of a workgroup and longer, so all loads go past the registers: a wave has a ring
 // of its own in LDS, of AHEAD pieces of 64 columns of x and W, and waits for no
 // other. Rows of x go by 128 bytes, their pieces of 16 at their index ^ (row / 2) %
@@ -161,7 +161,7 @@ constexpr int ROW_WAVES = 4;
 
 template <int B> struct Ring {
   static constexpr int STAGE = (B + 1) * 2048, LOADS = 2 * B + 2;
-  static constexpr int AHEAD = B == 4 ? 3 : B == 3 ? 4 : 5;
+  static constexpr int AHEAD = B == 4 ? 3 : 4;
   static constexpr int LDS = ROW_WAVES * AHEAD * STAGE;
 };
 
@@ -364,7 +364,7 @@ std::vector<at::Tensor> decode_res(at::Tensor xs, at::Tensor ws,
 // Whether rows_res takes rows [M, K] of W [N, K] in the decode layout: its parts of
 // the squares are one per 16 columns, 256 at most.
 bool rows_res_supported(int64_t M, int64_t N, int64_t K) {
-  return M >= 17 && M <= 64 && N > 0 && N % 32 == 0 && N <= 4096 &&
+  return M >= 33 && M <= 64 && N > 0 && N % 32 == 0 && N <= 4096 &&
          K % 64 == 0 && K >= 1024 && K < (1 << 22);
 }
 
@@ -406,8 +406,7 @@ std::vector<at::Tensor> rows_res(at::Tensor x, at::Tensor ws, at::Tensor res,
     hipLaunchKernelGGL(kernel, dim3((unsigned)(N / 16)), dim3(ROW_WAVES * 64),
                        Ring<B>::LDS, at::cuda::getCurrentHIPStream(), a);
   };
-  if (M <= 32) go(std::integral_constant<int, 2>{});
-  else if (M <= 48) go(std::integral_constant<int, 3>{});
+  if (M <= 48) go(std::integral_constant<int, 3>{});
   else go(std::integral_constant<int, 4>{});
   return {out, y, squares};
 }
@@ -418,7 +417,7 @@ bool parts_res_supported(int64_t N) {
   return N > 0 && N % 256 == 0 && N <= 16384;
 }
 
-// {r', y, squares [M, N / 64]} of parts [P, M, N] of what is added, P 1, 2, 4 or 8.
+// {r', y, squares [M, N / 64]} of parts [P, M, N] of what is added, P 2, 4 or 8.
 std::vector<at::Tensor> parts_res(at::Tensor parts, at::Tensor res,
                                   at::Tensor norm) {
   TORCH_CHECK(res.is_cuda() && res.dim() == 2 && res.is_contiguous() &&
@@ -449,11 +448,10 @@ std::vector<at::Tensor> parts_res(at::Tensor parts, at::Tensor res,
                        squares.data_ptr<float>(), (int)M, (int)N);
   };
   switch (parts.size(0)) {
-    case 1: go(parts_res_kernel<1>); break;
     case 2: go(parts_res_kernel<2>); break;
     case 4: go(parts_res_kernel<4>); break;
     case 8: go(parts_res_kernel<8>); break;
-    default: TORCH_CHECK(false, "parts_res: 1, 2, 4 or 8 parts");
+    default: TORCH_CHECK(false, "parts_res: 2, 4 or 8 parts");
   }
   return {out, y, squares};
 }

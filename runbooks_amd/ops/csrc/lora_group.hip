@@ -624,6 +624,7 @@ static void run_grads(Grad db, Grad da, const Adapters &a, const at::Tensor &x) 
                      dim3(256), 0, stream, db, da);
 }
 
+// One of the two by itself, what lora_grads is tested against (fine-tunes take both).
 // transposed=False: scale x_i^T t_i, [columns, 16]; the columns of x belong to
 // siblings of `widths`. transposed=True: scale t_i^T x, [16 n, columns].
 at::Tensor lora_grad(at::Tensor x, at::Tensor t, std::vector<int64_t> widths,

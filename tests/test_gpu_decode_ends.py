@@ -354,7 +354,7 @@ def test_shortest_prompts(monkeypatch, tokens, kv, inter, eight_bit):
         assert _rel(a, b.double()) < 2e-2
 
 
-@pytest.mark.parametrize("m", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("m", [33, 48, 49, 64])
 @pytest.mark.parametrize("n,k", [(32, 1024), (1024, 1088), (4096, 8192)])
 def test_residual_sum_of_rows(m, n, k):
     x = torch.randn(m, k, device=DEV).bfloat16()
@@ -369,7 +369,8 @@ def test_residual_sum_of_rows(m, n, k):
     assert _rel(squares.sum(1), want.square().sum(1)) < 1e-5
 
 
-@pytest.mark.parametrize("m,n,k", [(16, 1024, 1024), (65, 1024, 1024),
+@pytest.mark.parametrize("m,n,k", [(16, 1024, 1024), (32, 1024, 1024),
+                                   (65, 1024, 1024),
                                    (48, 1040, 1024), (48, 1024, 1056),
                                    (48, 4128, 1024)])
 def test_refused_residual_sums_of_rows(m, n, k):
@@ -382,7 +383,7 @@ def test_refused_residual_sums_of_rows(m, n, k):
 
 
 @pytest.mark.parametrize("m", [33, 64])
-@pytest.mark.parametrize("parts,n", [(1, 1024), (2, 1280), (4, 4096), (8, 8192)])
+@pytest.mark.parametrize("parts,n", [(2, 1280), (4, 4096), (8, 8192)])
 def test_residual_of_parts(m, parts, n):
     """Sums of parts and residual with the norm's squares, fp32 throughout."""
     assert ops.ext().parts_res_supported(n)

@@ -197,14 +197,16 @@ def test_products_of_paired_copies(m, fp8):
                 assert torch.equal(a, b)
 
 
-def _model(kv, inter, hidden=1024, eight_bit=False):
+def _model(kv, inter, hidden=1024, eight_bit=False, heads=8, dh=128,
+           act="silu_glu"):
     from runbooks_amd.models import build_model, get_config
     from runbooks_amd.models.config import register
     from runbooks_amd.models.transformer import fuse_for_inference
     cfg = dataclasses.replace(
-        get_config("smoke-llama"), name=f"ends-{kv}-{inter}-{hidden}",
-        hidden_size=hidden, num_heads=8, num_kv_heads=kv, head_dim=128,
-        intermediate_size=inter, num_layers=2)
+        get_config("smoke-llama"),
+        name=f"ends-{kv}-{inter}-{hidden}-{heads}-{dh}-{act}",
+        hidden_size=hidden, num_heads=heads, num_kv_heads=kv, head_dim=dh,
+        intermediate_size=inter, num_layers=2, act=act)
     register(cfg)
     m = build_model(cfg.name, dtype=torch.bfloat16, tp=1, device=DEV, seed=3)
     return fuse_for_inference(m.eval(), load_in_8bit=eight_bit)
@@ -215,8 +217,8 @@ def _step(m, batch, fp8):
     g = torch.Generator(device=DEV).manual_seed(batch)
     caches = m.alloc_caches(batch * 2 + 1, DEV, fp8=fp8)
     for layer in caches:
-        hkv = layer[0].shape[1]
-        k, v = (torch.randn(batch * 32, hkv, 128, device=DEV,
+        hkv, dh = layer[0].shape[1], layer[0].shape[3]
+        k, v = (torch.randn(batch * 32, hkv, dh, device=DEV,
                             generator=g).bfloat16() for _ in range(2))
         ops.kv_append(k, v, *layer, torch.arange(batch * 32, device=DEV,
                                                  dtype=torch.int32))
@@ -520,3 +522,43 @@ def test_rows_handed_over(monkeypatch, decode, why):
     else:
         assert delta.dtype == torch.float32 and delta.shape[1:] == want.shape
         assert _rel(delta.sum(0), want) < 1e-5
+
+
+@pytest.mark.parametrize("rows", ["step", "prompt", "prompts"])
+@pytest.mark.parametrize("stale", [False, True])
+@pytest.mark.parametrize("kv,inter,hidden,heads,dh,act", [
+    (8, 2048, 1024, 8, 128, "gelu_glu"), (4, 2048, 1024, 16, 64, "silu_glu"),
+    (4, 2048, 1024, 4, 256, "gelu_glu"),
+    (2, 1024, 8448, 8, 128, "silu_glu")])       # a down projection in one part
+def test_rows_of_other_models(monkeypatch, rows, stale, kv, inter, hidden, heads,
+                              dh, act):
+    """As test_steps_of_rows: units of GELU, heads of 64 and 256, sums that no
+    kernel takes in parts, two prompts at once, and a second block whose copies
+    are older than its weights."""
+    m = _model(kv, inter, hidden, heads=heads, dh=dh, act=act)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    seen = _served_by_rows(monkeypatch)
+    if stale:
+        with torch.no_grad():
+            m.blocks[1].mlp._gateup_w.mul_(0.5)
+
+    def step():
+        if rows == "step":
+            args = _step(m, 40, False)
+            caches = args[2]
+        else:
+            caches = m.alloc_caches(16, DEV)
+            n, of = (2, 24) if rows == "prompts" else (1, 47)
+            args = (torch.arange(n * of, device=DEV).view(n, of) % 50,
+                    torch.arange(of, **i32).repeat(n), caches,
+                    torch.arange(n * of, **i32) + 5)
+        with torch.no_grad():
+            logits = (m.decode if rows == "step" else m.prefill)(*args)
+        return [logits] + [c for layer in caches for c in layer]
+
+    got = step()
+    monkeypatch.setattr(type(m), "_few_rows",
+                        lambda self, x, *a: self._blocks(x, a[-1]))
+    assert seen == [1 if stale else 2]
+    for a, b in zip(got, step()):
+        assert _rel(a, b.double()) < 2e-2

@@ -354,12 +354,15 @@ def test_gradients_of_inputs(monkeypatch, m, n, k, siblings, tiles):
         linear._library_grad(x, w)
     if tiles or not taken:
         ext.lora_add_(other, t, As, 1.0, True)
-    product = 2.0 ** -8 * (x.double() @ w.double()).abs().max()
-    for y in (got, other):
-        ref = x.double() @ w.double() + sum(
-            ti.double() @ a.double() for ti, a in zip(t, As))
-        bound = 2.0 ** -8 * ref.abs() + product + 1e-4
-        assert bool(((y.double() - ref).abs() <= bound).all())
+    own, library = (got, other) if tiles else (other, got)
+    if taken:
+        _check_down(own, x, w, t, As, 2.0 ** -8)
+    # the product's rounding, of whatever size it is, and the sum's
+    ref = x.double() @ w.double()
+    product = 2.0 ** -8 * ref.abs()
+    ref = ref + sum(ti.double() @ a.double() for ti, a in zip(t, As))
+    bound = 2.0 ** -8 * ref.abs() + product + 1e-4
+    assert bool(((library.double() - ref).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("change", ["rows", "columns", "aligned", "type", "rank"])

@@ -179,8 +179,8 @@ def _add_rows(x, rows, copy, norm):
     long rows, parts and a launch that adds them up (us of 45 and 64 rows, in parts
     with the norm and whole: 4096 x 4096 15.8 and 12.2, 16.4 and 13.5; 2048 x 2048
     11.2 and 7.6, 11.9 and 8.2; 4096 x 11008 26.6 and 28.6, 28.6 and 32.6; 4096 x
-    14336 28.8 and 37.6, 30.8 and 39.6). A prompt of 45 tokens of llama2-7b, all in
-    all, 3560 -> 3410 us."""
+    14336 28.8 and 37.6, 30.8 and 39.6). Prompts of 45 tokens of llama2-7b, one after
+    the other, take 3457 us in the modules' launches and 3309 in run_rows'."""
     ext, m = ops.ext(), x.shape[0]
     if copy.half == 0 and copy.k <= 8192 and \
             ext.rows_res_supported(m, copy.n, copy.k):
@@ -201,8 +201,9 @@ def run_rows(model, x, positions, caches, slots, attend, joint: bool, *types):
     heads' results as rows; with `joint`, q is q, k and v side by side.
 
     A block is looked at while the GPU is at the one before it: a look at all of
-    llama2-7b takes the host 0.55 ms, for which an idle GPU would wait (one prompt
-    of 45 tokens 4.17 ms, so 3.69)."""
+    llama2-7b takes the host 0.7 ms, for which an idle GPU would wait (a prompt of 45
+    tokens by itself, from the call until its logits are there: 4.22 ms, so 3.52, and
+    3.70 in the modules)."""
     cfg, ext, m = model.cfg, ops.ext(), x.shape[0]
     if not (_served(model) and cfg.norm == "rmsnorm" and
             not cfg.parallel_residual and not cfg.single_norm and

@@ -1,7 +1,7 @@
 // Paged decode attention (one query token per sequence) for CDNA4 (gfx950).
 //
-// The serving hot loop: memory-bound on the KV read (288 GB HBM3E at
-// ~6.3 TB/s achievable). Design, MI355X-first:
+// The serving hot loop: memory-bound on the KV read (HBM3E gives 6.6 TB/s to
+// long reads that pass L2's older lines, 5.9 to others). Design, MI355X-first:
 //  * wave64 split into four 16-lane groups; each group owns ONE kv token
 //    per step at 8 (Dh=128) or 4 (Dh=64) elems/lane, so every wave streams
 //    4 contiguous KV rows per iteration at 16/8 B per lane.
@@ -56,7 +56,7 @@ RB_DEV float rb_dot2(unsigned a, unsigned b, float c) {
 // VE outputs of sequence b from column kk0 of a row (a multiple of VE, as VE is
 // of 4) in the decode GEMM's operand layout, [K/16][2][32][8].
 template <int VE>
-RB_DEV void store_operand(uint16_t *swz, int kk0, int b, const float (&v)[VE],
+RB_DEV void store_operand(uint16_t *swz, int kk0, int b, const float *v,
                           float scale) {
   constexpr int W = VE < 8 ? VE : 8;
 #pragma unroll
@@ -94,7 +94,8 @@ RB_DEV Place shifted_place(const int32_t *lens, const int32_t *starts) {
 // with it. Up to 64 sequences, whose lengths one wave compares for all (B steps of
 // three instructions; all waves of a CU together took 0.8 us).
 //
-// us by shifts and sorted, 32 heads of 128: 32 sequences of 129 to 2015 tokens 108
+// us by shifts and sorted, with loads that stayed in L2 (launch_decode: 10% longer
+// than now), 32 heads of 128: 32 sequences of 129 to 2015 tokens 108
 // and 101 (5.6 TB/s), 16 of 800 to 3900 in e4m3 76 and 69, 64 of 100 to 1200 133 and
 // 124, 32 of 1072 each 104 and 104; 8 kv heads of 128 with four queries each: 64 of
 // 1000 to 4003 128 and 118 (5.7 TB/s), 32 of 100 to 4000 in two parts 61 and 55; 16
@@ -151,7 +152,7 @@ RB_DEV Place sorted_place(const int32_t *lens, const int32_t *starts) {
 // capacity within 288 GB. Dequant rides
 // v_cvt_pk_f32_fp8 in the inner loop.
 template <int DH, int G, bool SPLIT, bool FP8 = false, int WAVES = NW,
-          int PER_SIMD = 1>
+          int PER_SIMD = 1, bool ONCE = !FP8 && G < NW>
 __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k_cache,
     const uint16_t *__restrict__ v_cache, const int32_t *__restrict__ block_tables,
@@ -205,7 +206,13 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
   const int wid = threadIdx.x >> 6;
   const int grp = lane / GL;               // lane group: token sub-index
   const int gl = lane % GL;                // lane within group
-  const int d0 = gl * VE;                  // this lane's Dh slice
+  // This lane's columns: pieces of 16 bytes, those of a group side by side, so
+  // that a load takes whole lines of memory (16 heads of 256, whose rows are two
+  // pieces a lane, us with a lane's pieces side by side and so: 32 sequences of 100
+  // to 2000 tokens 100 and 91, 7 of 90 to 1801 29.5 and 27.3).
+  constexpr int CH = VE < (FP8 ? 16 : 8) ? VE : (FP8 ? 16 : 8);
+  const int d0 = gl * CH;
+  auto column = [&](int e) { return d0 + e / CH * (GL * CH) + e % CH; };
 
   // Q for this wave's GW heads. bf16 caches keep Q as PACKED bf16 pairs: the
   // K dot then runs on v_dot2_f32_bf16 straight from the raw K words — no
@@ -215,18 +222,18 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
   unsigned qpk[GW][VE / 2];
 #pragma unroll
   for (int g = 0; g < GW; ++g) {
-    const uint16_t *qp = q + ((int64_t)b * Hq + hq_base + g) * DH + d0;
+    const uint16_t *qp = q + ((int64_t)b * Hq + hq_base + g) * DH;
 #pragma unroll
     for (int e = 0; e < VE; ++e) qreg[g][e] = 0.f;
     {
       float tmp[VE];
 #pragma unroll
       for (int e8 = 0; e8 < VE; e8 += 8) {
-        if (VE - e8 >= 8) rb::VIO<uint16_t>::load(qp + e8, tmp + e8);
+        if (VE - e8 >= 8) rb::VIO<uint16_t>::load(qp + column(e8), tmp + e8);
         else {
 #pragma unroll
           for (int e = 0; e < VE % 8; ++e)
-            tmp[e8 + e] = rb::bf16_to_f32(qp[e8 + e]);
+            tmp[e8 + e] = rb::bf16_to_f32(qp[column(e8 + e)]);
         }
       }
       if (FP8) {
@@ -305,17 +312,26 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
         const uint8_t *v8 = reinterpret_cast<const uint8_t *>(v_cache);
         const int64_t row =
             (((int64_t)blk * hkv + h_kv) * bs + (tt % bs)) * RB8;
-        rb::ld_words<RW>(kraw[slot][u], k8 + row + d0);
-        rb::ld_words<RW>(vraw[slot][u], v8 + row + d0);
+#pragma unroll
+        for (int c = 0; c < VE; c += CH) {
+          rb::ld_words<CH / 4>(kraw[slot][u] + c / 4, k8 + row + column(c));
+          rb::ld_words<CH / 4>(vraw[slot][u] + c / 4, v8 + row + column(c));
+        }
         kscale[slot][u] = *reinterpret_cast<const float *>(k8 + row + DH);
         vscale[slot][u] = *reinterpret_cast<const float *>(v8 + row + DH);
       } else {
         const int64_t base =
             (((int64_t)blk * hkv + h_kv) * bs + (tt % bs)) * DH + d0;
-        rb::ld_words<RW>(kraw[slot][u],
-                         reinterpret_cast<const uint8_t *>(k_cache + base));
-        rb::ld_words<RW>(vraw[slot][u],
-                         reinterpret_cast<const uint8_t *>(v_cache + base));
+#pragma unroll
+        for (int c = 0; c < VE; c += CH)
+          rb::ld_words<CH / 2, ONCE>(
+              kraw[slot][u] + c / 2,
+              reinterpret_cast<const uint8_t *>(k_cache + base) + c * GL * 2);
+#pragma unroll
+        for (int c = 0; c < VE; c += CH)
+          rb::ld_words<CH / 2, ONCE>(
+              vraw[slot][u] + c / 2,
+              reinterpret_cast<const uint8_t *>(v_cache + base) + c * GL * 2);
       }
     }
   };
@@ -427,16 +443,19 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
           float *pp =
               partial + (((int64_t)b * Hq + h) * nsplit + split) * (DH + 2);
 #pragma unroll
-          for (int e = 0; e < VE; ++e) pp[d0 + e] = acc[g][e];
+          for (int e = 0; e < VE; ++e) pp[column(e)] = acc[g][e];
           if (gl == 0) { pp[DH] = m[g]; pp[DH + 1] = l[g]; }
         } else {
           const float inv_l = (l[g] > 0.f) ? 1.0f / l[g] : 0.f;
-          uint16_t *op = out + ((int64_t)b * Hq + h) * DH + d0;
+          uint16_t *op = out + ((int64_t)b * Hq + h) * DH;
 #pragma unroll
           for (int e = 0; e < VE; ++e)
-            op[e] = rb::f32_to_bf16(acc[g][e] * inv_l);
+            op[column(e)] = rb::f32_to_bf16(acc[g][e] * inv_l);
           if (out_swz != nullptr)
-            store_operand<VE>(out_swz, h * DH + d0, b, acc[g], inv_l);
+#pragma unroll
+            for (int c = 0; c < VE; c += CH)
+              store_operand<CH>(out_swz, h * DH + column(c), b, acc[g] + c,
+                                inv_l);
         }
       }
     }
@@ -450,7 +469,7 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
 #pragma unroll
     for (int g = 0; g < GW; ++g) {
 #pragma unroll
-      for (int e = 0; e < VE; ++e) lds[wid][g][d0 + e] = acc[g][e];
+      for (int e = 0; e < VE; ++e) lds[wid][g][column(e)] = acc[g][e];
       if (gl == 0) { lds[wid][g][DH] = m[g]; lds[wid][g][DH + 1] = l[g]; }
     }
   }
@@ -471,21 +490,25 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
         const float a = __expf(lds[w][g][DH] - mm);
         ll += lds[w][g][DH + 1] * a;
 #pragma unroll
-        for (int e = 0; e < VE; ++e) av[e] += lds[w][g][d0 + e] * a;
+        for (int e = 0; e < VE; ++e) av[e] += lds[w][g][column(e)] * a;
       }
     }
     if (SPLIT) {
       float *pp = partial + (((int64_t)b * Hq + hq0 + g) * nsplit + split) * (DH + 2);
 #pragma unroll
-      for (int e = 0; e < VE; ++e) pp[d0 + e] = av[e];
+      for (int e = 0; e < VE; ++e) pp[column(e)] = av[e];
       if (gl == 0) { pp[DH] = mm; pp[DH + 1] = ll; }
     } else {
       const float inv_l = (ll > 0.f) ? 1.0f / ll : 0.f;
-      uint16_t *op = out + ((int64_t)b * Hq + hq0 + g) * DH + d0;
+      uint16_t *op = out + ((int64_t)b * Hq + hq0 + g) * DH;
 #pragma unroll
-      for (int e = 0; e < VE; ++e) op[e] = rb::f32_to_bf16(av[e] * inv_l);
+      for (int e = 0; e < VE; ++e)
+        op[column(e)] = rb::f32_to_bf16(av[e] * inv_l);
       if (out_swz != nullptr)
-        store_operand<VE>(out_swz, (hq0 + g) * DH + d0, b, av, inv_l);
+#pragma unroll
+        for (int c = 0; c < VE; c += CH)
+          store_operand<CH>(out_swz, (hq0 + g) * DH + column(c), b, av + c,
+                            inv_l);
     }
   }
 }
@@ -701,11 +724,11 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int ks = 0; ks < KS32; ++ks)
-          rb::ld_words<4>(kfr[slot][t][ks],
+          rb::ld_words<4, true>(kfr[slot][t][ks],
                           kb + ((krow + 4 * t) * DH + ks * 32 + h16 * 8) * 2);
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
-        rb::ld_words<4>(vfr[slot][dt],
+        rb::ld_words<4, true>(vfr[slot][dt],
                         vb + ((dt * 16 + i16) * BS + tok0) * 2);
     }
   };
@@ -925,13 +948,24 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                        splits > 1 ? nullptr : swz, partial, hkv, bs, max_blocks,
                        splits, scale, sorted);
   };
+  // Keys and values go past L2's older lines: in a step they are read once (ONCE;
+  // us of caches that lie in memory, without and with it: 32 sequences of 129 to 2015
+  // tokens, 32 heads of 128 104 and 92, 4 of 4000 54 and 49, one of 701 10.9 and 10.2,
+  // of 37 4.8 and 4.5; 64 of 37 to 1400, 12 heads of 64 30.9 and 28.0). Heads of 64 are
+  // those of small models, whose caches a few sequences leave in L2 from step to step:
+  // there not, as far as a layer's table has room for no more than L2's 32 MB (one of
+  // 37 tokens, 12 heads 3.6 and 3.9).
+  constexpr bool EITHER = DH == 64 && !FP8 && G < NW;
+  const bool once =
+      !EITHER || (int64_t)B * hkv * longest * DH * 4 > ((int64_t)32 << 20);
   if constexpr (G < NW) {
     // Whole sequences by 8 waves: of a short one more have nothing to do, and a CU
     // has room for more workgroups (which is why one query head a kv head keeps
     // to 64 registers, of 68). By 16 where long tables and few workgroups leave
     // the longest sequences to the end; by 4 where there are workgroups enough and
     // 8 waves take too many registers (e4m3 107, two query heads 93).
-    // us by 4, 8 and 16 waves, 32 heads of 128 in bf16: 32 sequences of 100 tokens
+    // us by 4, 8 and 16 waves, with loads that stayed in L2, 32 heads of 128 in bf16:
+    // 32 sequences of 100 tokens
     // 14.0, 13.7 and 17.3, of 300 31.9, 31.8 and 33.2, of 129 to 2015 111, 107 and
     // 111, 4000 and 31 of 100 115, 69 and 58; 16 of 100 9.0, 9.3 and 10.3, of 800 to
     // 3900 135, 120 and 117, 4000 and 15 of 100 111, 65 and 50; one of 100 5.8, 5.3
@@ -949,15 +983,33 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
         return go(paged_decode_kernel<DH, G, false, FP8, 16, ROOM>, 16, 1,
                   nullptr);
     const bool many = (FP8 || G > 1) && base > (DH == 64 ? 1023 : 512);
-    if (nsplit <= 1 && longest > 64 && !many)
+    if (nsplit <= 1 && longest > 64 && !many) {
+      if constexpr (EITHER)
+        if (!once)
+          return go(paged_decode_kernel<DH, G, false, FP8, 8, ROOM, false>, 8,
+                    1, nullptr);
       return go(paged_decode_kernel<DH, G, false, FP8, 8, ROOM>, 8, 1, nullptr);
+    }
   }
-  if (nsplit <= 1)
+  if (nsplit <= 1) {
+    if constexpr (EITHER)
+      if (!once)
+        return go(paged_decode_kernel<DH, G, false, FP8, NW, 1, false>, NW, 1,
+                  nullptr);
     return go(paged_decode_kernel<DH, G, false, FP8>, NW, 1, nullptr);
+  }
   auto partial = at::empty({B, Hq, nsplit, DH + 2},
                            q.options().dtype(at::kFloat));
-  go(paged_decode_kernel<DH, G, true, FP8>, NW, nsplit,
-     partial.data_ptr<float>());
+  bool gone = false;
+  if constexpr (EITHER)
+    if (!once) {
+      go(paged_decode_kernel<DH, G, true, FP8, NW, 1, false>, NW, nsplit,
+         partial.data_ptr<float>());
+      gone = true;
+    }
+  if (!gone)
+    go(paged_decode_kernel<DH, G, true, FP8>, NW, nsplit,
+       partial.data_ptr<float>());
   hipLaunchKernelGGL((decode_combine_kernel<DH / 64>),
                      dim3((B * Hq + 3) / 4), dim3(256), 0, stream,
                      partial.data_ptr<float>(), (uint16_t *)out.data_ptr(), swz,
@@ -978,7 +1030,8 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
 // batch takes about as long. In place of more parts it does not, and an engine's
 // tables are wide whatever the lengths.
 //
-// us in parts and whole, 32 heads of 128 in bf16: one sequence of 200 tokens 9.1
+// us in parts and whole, with loads that stayed in L2, 32 heads of 128 in bf16: one
+// sequence of 200 tokens 9.1
 // and 7.1, of 512 9.8 and 9.5, of 1024 12.0 and 16.2; 4 of 512 13.8 and 12.2, one of
 // 512 and 3 of 50 10.1 and 10.5, one of 1024 and 3 of 50 12.7 and 16.6; 16 (two
 // parts) of 800 to 3900 122 and 123, 4000 and 15 of 100 63.7 and 54.3; 8 (four) of

@@ -75,23 +75,30 @@ RB_DEV void fp8w_to_f32(uint32_t w, float *f) {
 }
 
 // raw vector load of RW u32 words (8/16/32 B) — no conversion, so the
-// compiler can keep the s_waitcnt away from the issue point
-template <int RW>
+// compiler can keep the s_waitcnt away from the issue point. ONCE: of what is
+// read once, past L2's older lines (a long read of 1 GB 5.9 TB/s, so 6.6).
+template <int RW, bool ONCE = false>
 RB_DEV void ld_words(uint32_t *dst, const uint8_t *src) {
   typedef __attribute__((ext_vector_type(2))) unsigned int u32x2i;
   typedef __attribute__((ext_vector_type(4))) unsigned int u32x4i;
+  auto ld = [](const auto *p) {
+    if constexpr (ONCE) return __builtin_nontemporal_load(p);
+    else return *p;
+  };
   if constexpr (RW == 1) {
-    *dst = *reinterpret_cast<const uint32_t *>(src);
+    *dst = ld(reinterpret_cast<const uint32_t *>(src));
   } else if constexpr (RW == 2) {
-    *reinterpret_cast<u32x2i *>(dst) = *reinterpret_cast<const u32x2i *>(src);
+    *reinterpret_cast<u32x2i *>(dst) =
+        ld(reinterpret_cast<const u32x2i *>(src));
   } else if constexpr (RW == 4) {
-    *reinterpret_cast<u32x4i *>(dst) = *reinterpret_cast<const u32x4i *>(src);
+    *reinterpret_cast<u32x4i *>(dst) =
+        ld(reinterpret_cast<const u32x4i *>(src));
   } else {
     static_assert(RW == 8, "unsupported row width");
     reinterpret_cast<u32x4i *>(dst)[0] =
-        reinterpret_cast<const u32x4i *>(src)[0];
+        ld(reinterpret_cast<const u32x4i *>(src));
     reinterpret_cast<u32x4i *>(dst)[1] =
-        reinterpret_cast<const u32x4i *>(src)[1];
+        ld(reinterpret_cast<const u32x4i *>(src) + 1);
   }
 }
 

@@ -24,7 +24,9 @@ def _rel(a, b):
     (2, 8, 4, 128, 40, 1), (3, 4, 4, 256, 17, 1), (2, 4, 4, 256, 16, 8),
     # as many workgroups as change the number of waves, and one more sequence
     (16, 32, 32, 128, 33, 1), (17, 32, 32, 128, 33, 1),
-    (43, 24, 24, 64, 5, 1), (17, 64, 32, 128, 5, 1)])
+    (43, 24, 24, 64, 5, 1), (17, 64, 32, 128, 5, 1),
+    # heads of 64 in tables of more than 32 MB, whole by 8 and by 4 waves
+    (43, 24, 24, 64, 8, 1), (90, 24, 24, 64, 4, 1)])
 def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
     """By 4, 8 or 16 waves or in parts, with and without a window's start, and
     with sequences as short and as long as the table: the plain result but for

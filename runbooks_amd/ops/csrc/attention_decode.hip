@@ -23,6 +23,7 @@
 #include <ATen/hip/HIPContext.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -513,6 +514,296 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
   }
 }
 
+// e4m3 caches of blocks of 16, up to two query heads a kv head: whole blocks of a head,
+// which are contiguous, go to LDS past the registers, and their rows of DH + 16 bytes
+// (values, scale) are read there. Loaded by rows, which begin and end within lines of
+// memory, scales apart, a line was asked for up to three times and could not pass L2.
+// A wave has a ring of its own and waits for no other; a lane group of eight takes a
+// row, 16 tokens a step. Keys are multiplied as bf16 pairs, which they are exactly.
+//
+// Bound by memory. us by rows and so, 32 heads of 128: 16 sequences of 800 to 3900
+// tokens 68.5 and 60.6 (5.7 TB/s), 32 of 1000 58.9 and 53.9, 64 of 1000 110 and 99, 32
+// of 50 to 1000 34.1 and 31.9, of 100 11.6 and 11.0, 8 of 400 in four parts 15.1 and
+// 14.1, one of 700 10.7 and 9.8, of 50 4.8 and 4.3; 4000 and 15 of 100, where few CUs
+// have anything to do, 39.5 and 40.1. Two queries each: 32 of 50 to 1000 51 and 34.
+// Four workgroups of four waves fill a CU, as two of eight do (with the longer ring of
+// two, 32 of 100 took 14.4, 8 of 400 17.3). 16 heads of 256: 16 of 100 to 2000 in
+// four parts 42.6 and 38.7.
+template <int DH, int WAVES> struct Blocks8 {
+  static constexpr int PART = (DH + 16) * 16, STAGE = 2 * PART;   // K, then V
+  static constexpr int FULL = PART / 1024, LOADS = 2 * FULL + 1;
+  static constexpr int PER_CU = WAVES == 8 || DH == 256 ? 2 : 4;
+  static constexpr int AHEAD = (160 / PER_CU - 3) * 1024 / STAGE / WAVES;
+  static constexpr int LDS = WAVES * AHEAD * STAGE;
+  static_assert(PART % 1024 == 256 && AHEAD >= 2, "pieces, ring");
+};
+
+template <int DH, int G, bool SPLIT, int WAVES, bool ONCE>
+__global__ __launch_bounds__(WAVES * 64, DH == 256 ? 2 : 4) void paged_decode8_kernel(
+    const uint16_t *__restrict__ q, const uint8_t *__restrict__ k_cache,
+    const uint8_t *__restrict__ v_cache,
+    const int32_t *__restrict__ block_tables,
+    const int32_t *__restrict__ seq_lens,
+    const int32_t *__restrict__ seq_starts, uint16_t *__restrict__ out,
+    uint16_t *__restrict__ out_swz, float *__restrict__ partial, int hkv,
+    int max_blocks, int nsplit, float scale, bool sorted) {
+  using R = Blocks8<DH, WAVES>;
+  constexpr int BS = 16, GL = 8, VE = DH / GL, TPW = 64 / GL, U = BS / TPW;
+  constexpr int CH = VE < 16 ? VE : 16, RW = VE / 4;
+  constexpr float LOG2E = 1.4426950408889634f;
+  constexpr float RISE = 8.0f;          // of a maximum before it is moved
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const Place place =
+      sorted ? sorted_place(seq_lens, seq_starts)
+             : shifted_place(seq_lens, seq_starts);
+  const int b = place.b, h_kv = place.h, split = place.split;
+  const int hq0 = h_kv * G, Hq = hkv * G;
+  int t_begin = place.start, t_end = place.len;
+  if (SPLIT) {
+    const int chunk = (place.len - place.start + nsplit - 1) / nsplit;
+    t_begin = place.start + split * chunk;
+    t_end = min(place.len, t_begin + chunk);
+  }
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = lane / GL, gl = lane % GL;
+  // this lane's columns, as in paged_decode_kernel
+  auto column = [&](int e) { return e / CH * (GL * CH) + gl * CH + e % CH; };
+
+  const int32_t *bt = block_tables + (int64_t)b * max_blocks;
+  constexpr int BT_LDS = 512;
+  __shared__ int32_t bt_lds[BT_LDS];
+  const int lo = t_begin / BS, hi = t_end > t_begin ? (t_end - 1) / BS : lo - 1;
+  for (int i = (int)threadIdx.x; i < min(hi - lo + 1, BT_LDS); i += WAVES * 64)
+    bt_lds[i] = bt[lo + i];
+
+  unsigned qpk[G][VE / 2];              // the rows' own bits; scaled in fp32
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int c = 0; c < VE; c += CH)
+#pragma unroll
+      for (int e = 0; e < CH; e += 8) {
+        const uint4 w = *reinterpret_cast<const uint4 *>(
+            q + ((int64_t)b * Hq + hq0 + g) * DH + column(c + e));
+        qpk[g][(c + e) / 2] = w.x;
+        qpk[g][(c + e) / 2 + 1] = w.y;
+        qpk[g][(c + e) / 2 + 2] = w.z;
+        qpk[g][(c + e) / 2 + 3] = w.w;
+      }
+  __syncthreads();
+
+  const unsigned mine = wid * (R::AHEAD * R::STAGE);
+  const unsigned ring =
+      mine + (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem;
+  auto fetch = [&](int bi, int stage) {
+    const int blk = __builtin_amdgcn_readfirstlane(
+        bi - lo < BT_LDS ? bt_lds[bi - lo] : bt[bi]);
+    const int64_t at = ((int64_t)blk * hkv + h_kv) * R::PART;
+    const uint8_t *k = k_cache + at, *v = v_cache + at;
+    const unsigned to =
+        __builtin_amdgcn_readfirstlane(ring + stage * R::STAGE);
+#pragma unroll
+    for (int i = 0; i < R::FULL; ++i)
+      rb::lds_load_from<ONCE>(k + i * 1024 + lane * 16, to + i * 1024);
+    // the last 16 pieces of K and the first of V
+    if (lane < 32)
+      rb::lds_load_from<ONCE>(
+          (lane < 16 ? k + R::FULL * 1024 : v - 256) + lane * 16,
+          to + R::FULL * 1024);
+#pragma unroll
+    for (int i = 0; i < R::FULL; ++i)
+      rb::lds_load_from<ONCE>(v + 256 + i * 1024 + lane * 16,
+                              to + R::PART + 256 + i * 1024);
+  };
+
+  float m[G], l[G], acc[G][VE];         // maxima in exponents of 2
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    m[g] = -INFINITY;
+    l[g] = 0.0f;
+#pragma unroll
+    for (int e = 0; e < VE; ++e) acc[g][e] = 0.0f;
+  }
+  const float to2 = scale * LOG2E;
+#pragma unroll
+  for (int j = 0; j < R::AHEAD; ++j)
+    if (lo + wid + j * WAVES <= hi) fetch(lo + wid + j * WAVES, j);
+  int stage = 0;
+  for (int bi = lo + wid; bi <= hi; bi += WAVES) {
+    if (bi + (R::AHEAD - 1) * WAVES <= hi)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R::AHEAD - 1) * R::LOADS)
+                   : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    uint32_t kw[U][RW], vw[U][RW];
+    float ks[U], vs[U];
+    const char *at = smem + mine + stage * R::STAGE + grp * (DH + 16);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const char *k = at + u * TPW * (DH + 16), *v = k + R::PART;
+#pragma unroll
+      for (int c = 0; c < VE; c += CH) {
+        rb::ld_words<CH / 4>(kw[u] + c / 4, (const uint8_t *)k + column(c));
+        rb::ld_words<CH / 4>(vw[u] + c / 4, (const uint8_t *)v + column(c));
+      }
+      ks[u] = *reinterpret_cast<const float *>(k + DH);
+      vs[u] = *reinterpret_cast<const float *>(v + DH);
+    }
+    // read before it is written again
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (bi + R::AHEAD * WAVES <= hi) fetch(bi + R::AHEAD * WAVES, stage);
+    stage = stage + 1 == R::AHEAD ? 0 : stage + 1;
+    if (bi * BS < t_begin || (bi + 1) * BS > t_end) {
+      // rows that are not the sequence's may hold anything
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int t = bi * BS + u * TPW + grp;
+        const bool there = t >= t_begin && t < t_end;
+        vs[u] = there ? vs[u] : 0.0f;
+#pragma unroll
+        for (int w = 0; w < RW; ++w) vw[u][w] = there ? vw[u][w] : 0;
+      }
+    }
+
+    float x[G][U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) x[g][u] = 0.0f;
+#pragma unroll
+      for (int w = 0; w < RW; ++w) {
+        const unsigned a = rb::fp8_pair_bf16<false>(kw[u][w]);
+        const unsigned c = rb::fp8_pair_bf16<true>(kw[u][w]);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          x[g][u] = rb_dot2(a, qpk[g][2 * w], x[g][u]);
+          x[g][u] = rb_dot2(c, qpk[g][2 * w + 1], x[g][u]);
+        }
+      }
+    }
+    float p[G][U];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      rb::lane_sums<GL>(x[g]);
+      float mx = -INFINITY;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int t = bi * BS + u * TPW + grp;
+        x[g][u] = t >= t_begin && t < t_end ? x[g][u] * (ks[u] * to2)
+                                            : -INFINITY;
+        mx = fmaxf(mx, x[g][u]);
+      }
+      if (__any(mx > m[g] + RISE)) {
+        const float mn = fmaxf(m[g], mx);
+        // groups that have seen no key keep a finite reference
+        const float alpha =
+            __builtin_amdgcn_exp2f(m[g] - (mn == -INFINITY ? 0.0f : mn));
+        l[g] *= alpha;
+#pragma unroll
+        for (int e = 0; e < VE; ++e) acc[g][e] *= alpha;
+        m[g] = mn;
+      }
+      const float ref = m[g] == -INFINITY ? 0.0f : m[g];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        p[g][u] = __builtin_amdgcn_exp2f(x[g][u] - ref);
+        l[g] += p[g][u];
+        p[g][u] *= vs[u];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int w = 0; w < RW; ++w) {
+        float f[4];
+        rb::fp8w_to_f32(vw[u][w], f);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int g = 0; g < G; ++g) acc[g][w * 4 + e] += p[g][u] * f[e];
+      }
+  }
+
+  // the lane groups of a wave, then the waves
+  auto merge = [&](auto bit) {
+    constexpr int OFF = decltype(bit)::value;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const float mo = rb::lane_xor<OFF>(m[g]), lo = rb::lane_xor<OFF>(l[g]);
+      const float mn = fmaxf(m[g], mo), ref = mn == -INFINITY ? 0.0f : mn;
+      const float a1 = __builtin_amdgcn_exp2f(m[g] - ref);
+      const float a2 = __builtin_amdgcn_exp2f(mo - ref);
+#pragma unroll
+      for (int e = 0; e < VE; ++e)
+        acc[g][e] = acc[g][e] * a1 + rb::lane_xor<OFF>(acc[g][e]) * a2;
+      l[g] = l[g] * a1 + lo * a2;
+      m[g] = mn;
+    }
+  };
+  merge(std::integral_constant<int, 8>{});
+  merge(std::integral_constant<int, 16>{});
+  merge(std::integral_constant<int, 32>{});
+  static_assert(WAVES * G * (DH + 2) * 4 <= R::LDS, "merge buffer");
+  float *ex = reinterpret_cast<float *>(smem);      // [wave][head][DH + 2]
+  __syncthreads();                      // the last blocks have been read
+  if (grp == 0) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      float *r = ex + (wid * G + g) * (DH + 2);
+#pragma unroll
+      for (int e = 0; e < VE; ++e) r[column(e)] = acc[g][e];
+      if (gl == 0) {
+        r[DH] = m[g];
+        r[DH + 1] = l[g];
+      }
+    }
+  }
+  __syncthreads();
+  // a wave a head, a lane DH / 64 columns
+  constexpr int V = DH / 64;
+  const int d0 = lane * V;
+  for (int g = wid; g < G; g += WAVES) {
+    float mm = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+      mm = fmaxf(mm, ex[(w * G + g) * (DH + 2) + DH]);
+    const float ref = mm == -INFINITY ? 0.0f : mm;
+    float ll = 0.0f, o[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) o[e] = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float *r = ex + (w * G + g) * (DH + 2);
+      const float a = __builtin_amdgcn_exp2f(r[DH] - ref);
+      ll += r[DH + 1] * a;
+#pragma unroll
+      for (int e = 0; e < V; ++e) o[e] += r[d0 + e] * a;
+    }
+    const int h = hq0 + g;
+    if (SPLIT) {
+      float *pp = partial +
+                  (((int64_t)b * Hq + h) * nsplit + split) * (DH + 2);
+#pragma unroll
+      for (int e = 0; e < V; ++e) pp[d0 + e] = o[e];
+      if (lane == 0) {
+        pp[DH] = mm / LOG2E;
+        pp[DH + 1] = ll;
+      }
+    } else {
+      const float inv_l = ll > 0.0f ? 1.0f / ll : 0.0f;
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const int kk = h * DH + d0 + e;
+        const uint16_t y = rb::f32_to_bf16(o[e] * inv_l);
+        out[(int64_t)b * Hq * DH + kk] = y;
+        if (out_swz != nullptr)
+          out_swz[(kk >> 4) * 512 + (kk >> 3 & 1) * 256 + b * 8 + (kk & 7)] = y;
+      }
+    }
+  }
+}
+
 // Second pass for SPLIT mode: a wave merges the nsplit partials of one (b, hq)
 // row. The maxima and sums are one load of the wave, the rows (VE = dh / 64
 // values a lane) are loaded eight at a time: two round trips to memory where
@@ -956,8 +1247,56 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
   // there not, as far as a layer's table has room for no more than L2's 32 MB (one of
   // 37 tokens, 12 heads 3.6 and 3.9).
   constexpr bool EITHER = DH == 64 && !FP8 && G < NW;
-  const bool once =
-      !EITHER || (int64_t)B * hkv * longest * DH * 4 > ((int64_t)32 << 20);
+  const bool once = DH != 64 || (int64_t)B * hkv * longest *
+                                        (FP8 ? DH + 16 : DH * 2) * 2 >
+                                    ((int64_t)32 << 20);
+  if constexpr (FP8 && G < NW) {
+    if (bs == 16) {
+      const int splits = std::max(nsplit, 1);
+      at::Tensor partial;
+      if (splits > 1)
+        partial = at::empty({B, Hq, splits, DH + 2},
+                            q.options().dtype(at::kFloat));
+      auto go8 = [&](auto part, auto waves, auto past) {
+        constexpr int WAVES = decltype(waves)::value;
+        constexpr int lds = Blocks8<DH, WAVES>::LDS;
+        auto kernel = paged_decode8_kernel<DH, G, decltype(part)::value, WAVES,
+                                           decltype(past)::value>;
+        static const bool ready =
+            hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                lds) == hipSuccess;
+        TORCH_CHECK(ready, "paged_decode: LDS size");
+        hipLaunchKernelGGL(kernel, dim3(B, hkv, splits), dim3(WAVES * 64), lds,
+                           stream, (const uint16_t *)q.data_ptr(),
+                           (const uint8_t *)k_cache.data_ptr(),
+                           (const uint8_t *)v_cache.data_ptr(),
+                           block_tables.data_ptr<int32_t>(),
+                           seq_lens.data_ptr<int32_t>(), starts,
+                           splits > 1 ? nullptr : (uint16_t *)out.data_ptr(),
+                           splits > 1 ? nullptr : swz,
+                           splits > 1 ? partial.data_ptr<float>() : nullptr,
+                           hkv, max_blocks, splits, scale, sorted);
+      };
+      auto by_cache = [&](auto part, auto waves) {
+        if constexpr (DH == 64)
+          if (!once) return go8(part, waves, std::false_type{});
+        go8(part, waves, std::true_type{});
+      };
+      using Four = std::integral_constant<int, 4>;
+      using Most = std::integral_constant<int, DH == 256 ? 4 : 8>;
+      if (splits > 1) by_cache(std::true_type{}, Four{});
+      else if (longest > 64 && (int64_t)B * hkv <= (DH == 64 ? 1023 : 512))
+        by_cache(std::false_type{}, Most{});
+      else by_cache(std::false_type{}, Four{});
+      if (splits > 1)
+        hipLaunchKernelGGL((decode_combine_kernel<DH / 64>),
+                           dim3((B * Hq + 3) / 4), dim3(256), 0, stream,
+                           partial.data_ptr<float>(),
+                           (uint16_t *)out.data_ptr(), swz, B * Hq, Hq, splits);
+      return;
+    }
+  }
   if constexpr (G < NW) {
     // Whole sequences by 8 waves: of a short one more have nothing to do, and a CU
     // has room for more workgroups (which is why one query head a kv head keeps

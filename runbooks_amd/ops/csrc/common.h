@@ -74,6 +74,12 @@ RB_DEV void fp8w_to_f32(uint32_t w, float *f) {
   f[0] = a[0]; f[1] = a[1]; f[2] = b[0]; f[3] = b[1];
 }
 
+// two of a word's e4m3 -> packed bf16 (exact)
+template <bool HIGH> RB_DEV unsigned fp8_pair_bf16(uint32_t w) {
+  return __builtin_bit_cast(
+      unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, HIGH));
+}
+
 // raw vector load of RW u32 words (8/16/32 B) — no conversion, so the
 // compiler can keep the s_waitcnt away from the issue point. ONCE: of what is
 // read once, past L2's older lines (a long read of 1 GB 5.9 TB/s, so 6.6).
@@ -328,6 +334,19 @@ RB_DEV void lds_load_once(u32x4v from, unsigned voff, unsigned soff,
       "s_mov_b32 m0, %3\n\ts_nop 0\n\t"
       "buffer_load_dwordx4 %0, %1, %2 offen nt lds"
       :: "v"(voff), "s"(from), "s"(soff), "s"(lds) : "memory", "m0");
+}
+
+// The same from an address of each lane (those that are active).
+template <bool ONCE>
+RB_DEV void lds_load_from(const void *p, unsigned lds) {
+  if constexpr (ONCE)
+    asm volatile(
+        "s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
+        :: "v"(p), "s"(lds) : "memory", "m0");
+  else
+    asm volatile(
+        "s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+        :: "v"(p), "s"(lds) : "memory", "m0");
 }
 
 // two floats -> packed bf16 words (round to nearest even)

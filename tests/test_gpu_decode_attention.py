@@ -61,6 +61,37 @@ def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
                                operand.view(-1, 32, 8)[:, :batch])
 
 
+@pytest.mark.parametrize("batch,hq,hkv,dh,blocks,nsplit", [
+    (3, 4, 4, 128, 9, 1), (2, 8, 4, 128, 33, 3), (3, 4, 4, 64, 9, 1),
+    (3, 2, 2, 256, 40, 2), (17, 32, 32, 128, 33, 1)])
+def test_rows_of_nobody_8bit(batch, hq, hkv, dh, blocks, nsplit):
+    """What lies in a block beside a sequence's rows, ahead of its window and past
+    its end, may be anything: the same bits as with zeros there."""
+    torch.manual_seed(dh)
+    lens = torch.randint(1, blocks * 16 + 1, (batch,))
+    lens[0], lens[1] = 1, blocks * 16 - 7
+    starts = torch.clamp(lens - 45, min=0)
+    tokens = torch.cat([torch.arange(int(a), int(n)) + i * blocks * 16
+                        for i, (a, n) in enumerate(zip(starts, lens))])
+    k, v = (torch.randn(len(tokens), hkv, dh, device=DEV).bfloat16()
+            for _ in "kv")
+    i32 = dict(dtype=torch.int32, device=DEV)
+    q = torch.randn(batch, hq, dh, device=DEV).bfloat16()
+    tables = torch.arange(batch * blocks, **i32).view(batch, blocks)
+    results = []
+    for filled in (0, 255):
+        kc, vc = ops.alloc_kv_cache(batch * blocks, hkv, dh, DEV,
+                                    dtype=torch.bfloat16, fp8=True)
+        kc.fill_(filled)
+        vc.fill_(filled)
+        ops.kv_append(k, v, kc, vc, tokens.to(**i32))
+        results.append(ops.ext().paged_decode_swz(
+            q, kc, vc, tables, lens.to(**i32), nsplit, dh ** -0.5,
+            starts.to(**i32))[0])
+    assert bool(results[0].isfinite().all())
+    assert torch.equal(*results)
+
+
 @pytest.mark.parametrize("hq,hkv,nsplit", [(3, 3, 1), (5, 5, 3), (8, 2, 1),
                                            (8, 2, 2)])
 @pytest.mark.parametrize("batch", [2, 4, 5, 31, 64, 65])

@@ -39,16 +39,11 @@ RB_DEV bf16x8v load8v(const uint16_t *p) {
 
 // Two words of e4m3 -> 8 bf16 (exact).
 RB_DEV bf16x8v fp8_to_bf16(unsigned lo, unsigned up) {
-  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2v;
-  union { bf16x2v h[4]; bf16x8v v; } c;
-  c.h[0] = __builtin_convertvector(
-      __builtin_amdgcn_cvt_pk_f32_fp8(lo, false), bf16x2v);
-  c.h[1] = __builtin_convertvector(
-      __builtin_amdgcn_cvt_pk_f32_fp8(lo, true), bf16x2v);
-  c.h[2] = __builtin_convertvector(
-      __builtin_amdgcn_cvt_pk_f32_fp8(up, false), bf16x2v);
-  c.h[3] = __builtin_convertvector(
-      __builtin_amdgcn_cvt_pk_f32_fp8(up, true), bf16x2v);
+  union { unsigned u[4]; bf16x8v v; } c;
+  c.u[0] = rb::fp8_pair_bf16<false>(lo);
+  c.u[1] = rb::fp8_pair_bf16<true>(lo);
+  c.u[2] = rb::fp8_pair_bf16<false>(up);
+  c.u[3] = rb::fp8_pair_bf16<true>(up);
   return c.v;
 }
 

@@ -52,6 +52,7 @@ constexpr int MMAX = 32;
 using ends::bf16x8v;
 using ends::Ends;
 using ends::f32x16v;
+using ends::f32x4v;
 using ends::fp8_to_bf16;
 using ends::Kind;
 using ends::load8v;
@@ -59,13 +60,18 @@ using ends::u32x4v;
 
 // What a thread needs for its ends besides the sums; issued before the stream
 // of W (begin) and behind its first loads (rest), so that their ways to memory
-// lie beside its own. A thread's row m is that of its place in finish().
+// lie beside its own. A thread's row m is that of its place in finish(); waves that
+// have none there, of up to 16 rows, need nothing (`mine`).
 template <Kind KIND> struct Early {
   static constexpr int PARTS = 8;       // of 4 squares, for up to 256 in all
   float4 squares[PARTS];
   float norm;
+  float scale[4];                       // of the rows of W in finish()
   int position;
   ends::Turn<2> turn;
+  RB_DEV static bool mine(int M) {
+    return (__builtin_amdgcn_readfirstlane(threadIdx.x) >> 3) < M;
+  }
   RB_DEV void begin(const Ends &e, int M, int base = 0) {
     const int m = min(base + ((int)threadIdx.x >> 3), M - 1);
     const int i = threadIdx.x & 7;
@@ -77,6 +83,14 @@ template <Kind KIND> struct Early {
             e.squares + (int64_t)m * e.parts +
             min((j * 8 + i) * 4, e.parts - 4));
     }
+  }
+  RB_DEV void begin_scale(const Ends &e) {
+    constexpr bool PAIRS = KIND == ends::GLU || KIND == ends::QKV;
+    const int c = (threadIdx.x & 7) * (PAIRS ? 2 : 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      scale[j] = e.scale[ends::column(
+          e.half, blockIdx.x, PAIRS ? c + (j & 1) + (j >> 1) * 16 : c + j)];
   }
   RB_DEV void rest(const Ends &e, int M) {
     const int m = min((int)threadIdx.x >> 3, M - 1), i = threadIdx.x & 7;
@@ -96,34 +110,29 @@ template <Kind KIND> struct Early {
   }
 };
 
-// Sums the four waves' accumulators of 32 rows of W, times the rows' scales
-// where there are any, and hands them on.
-template <Kind KIND>
-__device__ __forceinline__ void finish(const f32x16v &acc, const Ends &e,
-                                       const Early<KIND> &early, int M, int N) {
-  const int tid = threadIdx.x, wid = tid >> 6;
-  const int hi = (tid & 63) >> 5, col = tid & 31;
+// Sums the four waves' parts of 32 rows of W, red[wave][row][m], times the rows'
+// scales where there are any (FP8), and hands them on.
+template <bool FP8, Kind KIND, int RED>
+__device__ __forceinline__ void finish(const float (&red)[4][32][RED],
+                                       const Ends &e, const Early<KIND> &early,
+                                       int M, int N) {
+  const int tid = threadIdx.x;
   const int nblk = blockIdx.x;
-  __shared__ __attribute__((aligned(16))) float red[4][32][MMAX];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int n_local = (r & 3) + 8 * (r >> 2) + 4 * hi;
-    red[wid][n_local][col] = acc[r];
-  }
   __syncthreads();
 
   // 1024 outputs, 4 per thread, n fastest so bf16 stores coalesce 8 B.
   const int em = tid >> 3;               // 0..31
   if (em >= M) return;
-  auto sum = [&](int r) {
+  auto sum = [&](int r, int j) {
     float x = red[0][r][em] + red[1][r][em] + red[2][r][em] + red[3][r][em];
     if (KIND != ends::SLAB) x *= early.norm;
-    if (e.scale != nullptr) x *= e.scale[ends::column(e.half, nblk, r)];
+    if (FP8) x *= early.scale[j];
     return x;
   };
   if constexpr (KIND == ends::GLU || KIND == ends::QKV) {
     const int c = (tid & 7) * 2;
-    float a[2] = {sum(c), sum(c + 1)}, b[2] = {sum(16 + c), sum(17 + c)};
+    float a[2] = {sum(c, 0), sum(c + 1, 1)};
+    float b[2] = {sum(16 + c, 2), sum(17 + c, 3)};
     if constexpr (KIND == ends::GLU)
       ends::put_gated<2>(e, em, nblk * 16 + c, N, a, b);
     else
@@ -131,7 +140,8 @@ __device__ __forceinline__ void finish(const f32x16v &acc, const Ends &e,
   } else {
     const int en = (tid & 7) * 4;        // 0,4,..,28
     const int n = ends::column(e.half, nblk, en);
-    const float f[4] = {sum(en), sum(en + 1), sum(en + 2), sum(en + 3)};
+    const float f[4] = {sum(en, 0), sum(en + 1, 1), sum(en + 2, 2),
+                        sum(en + 3, 3)};
     if constexpr (KIND == ends::PLAIN) {
       ends::put<4>(e.y + (int64_t)em * N + n, f);
     } else {
@@ -148,6 +158,40 @@ template <bool FP8> struct Step {
   u32x4v w;
   bf16x8v x[X];
 };
+
+// Steps s0 .. s1 - 1 by two chunks of U in turn. BOTH: both are on their way before
+// `meanwhile` waits for anything; of 17 to 32 rows, whose chunks are long, that costs
+// 1 to 3%.
+template <bool BOTH, int U, typename Step, typename Load, typename Multiply,
+          typename Meanwhile>
+__device__ __forceinline__ void stream_chunks(Step (&a)[U], Step (&b)[U],
+                                              int s0, int s1, Load load,
+                                              Multiply multiply,
+                                              Meanwhile meanwhile) {
+  if (s0 < s1) {
+    load(a, s0);
+    if (BOTH) load(b, s0 + U);
+  }
+  meanwhile();
+  if (s0 >= s1) return;
+  int s = s0;
+  for (; s + 2 * U < s1; s += 2 * U) {
+    if (!BOTH) load(b, s + U);
+#pragma unroll
+    for (int u = 0; u < U; ++u) multiply(a[u]);
+    load(a, s + 2 * U);
+#pragma unroll
+    for (int u = 0; u < U; ++u) multiply(b[u]);
+    if (BOTH) load(b, s + 3 * U);
+  }
+  if (!BOTH) load(b, s + U);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (s + u < s1) multiply(a[u]);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (s + U + u < s1) multiply(b[u]);
+}
 
 // W nontemporal (streamed once, must not evict L2); x plain (re-read by every
 // n-block: L2 is exactly where it wants to live). Columns past M read the last
@@ -167,9 +211,9 @@ template <bool FP8> struct Step {
 //         16 rows  32.5 -> 14.1  49.3 -> 20.8  17.7 -> 6.5  37.7 -> 12.8
 //         32 rows  34.7 -> 17.7  56.5 -> 26.4  18.1 -> 7.7  38.1 -> 16.0
 template <bool FP8, typename Meanwhile>
-__device__ __forceinline__ f32x16v weight_stream(
+__device__ __forceinline__ void weight_stream(
     const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws, int M,
-    int K, Meanwhile meanwhile) {
+    int K, float (&red)[4][32][MMAX], Meanwhile meanwhile) {
   constexpr int X = Step<FP8>::X, U = FP8 ? 4 : 8;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -207,38 +251,99 @@ __device__ __forceinline__ f32x16v weight_stream(
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w.v, c.x[0], acc, 0, 0, 0);
     }
   };
-  if (s0 < s1) load(a, s0);
-  meanwhile();
-  if (s0 < s1) {
-    int s = s0;
-    for (; s + 2 * U < s1; s += 2 * U) {
-      load(b, s + U);
+  stream_chunks<false>(a, b, s0, s1, load, multiply, meanwhile);
 #pragma unroll
-      for (int u = 0; u < U; ++u) multiply(a[u]);
-      load(a, s + 2 * U);
-#pragma unroll
-      for (int u = 0; u < U; ++u) multiply(b[u]);
-    }
-    load(b, s + U);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (s + u < s1) multiply(a[u]);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (s + U + u < s1) multiply(b[u]);
-  }
-  return acc;
+  for (int r = 0; r < 16; ++r)
+    red[wid][(r & 3) + 8 * (r >> 2) + 4 * hi][col] = acc[r];
 }
 
-template <bool FP8, Kind KIND>
+// The same of up to 16 rows x: products of 16 x 16, two of which share an operand of
+// x, so half as many loads of x go with one of W. A step is two kilobytes of W, 32
+// columns (e4m3: 64), its operands as in decode_res.hip.
+//
+// With that, what the ends need behind two chunks of W in place of one, and the scales
+// of W's rows loaded ahead of it and not behind it, us in a graph with the norm left out
+// of x and the ends, of 1 and 16 rows before and now: 12288 x 4096 and rotation 20.3 and
+// 19.3, 21.1 and 20.2 (W alone takes 17.8); 6144 x 4096 11.7 and 11.2, 12.4 and 11.9;
+// 22016 x 4096 and unit 31.4 and 30.7, 32.4 and 31.3 (29.3); 49152 x 3072 47.9 and
+// 46.8, 46.2 and 44.5; in e4m3 12288 x 4096 14.4 and 12.7, 14.4 and 13.4 (9.5), 22016 x
+// 4096 20.4 and 17.3, 20.9 and 19.6 (16).
+template <bool FP8, typename Meanwhile>
+__device__ __forceinline__ void weight_stream16(
+    const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws, int M,
+    int K, float (&red)[4][32][17], Meanwhile meanwhile) {
+  constexpr int X = FP8 ? 2 : 1, U = 4;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, i16 = lane & 15, grp = lane >> 4;
+  const int steps = K / (32 * X), groups = gridDim.y * 4;
+  const int g = blockIdx.y * 4 + wid;
+  const int s0 = (int)((int64_t)steps * g / groups);
+  const int s1 = (int)((int64_t)steps * (g + 1) / groups);
+  const uint8_t *w = ws + (int64_t)blockIdx.x * steps * 2048 + grp * 512 +
+                     i16 * 16;
+  const uint8_t *x = reinterpret_cast<const uint8_t *>(xs) +
+                     (FP8 ? (grp >> 1) * 2048 + (grp & 1) * 512 : grp * 512) +
+                     min(i16, M - 1) * 16;
+  struct Both { u32x4v w[2]; bf16x8v x[X]; };
+  Both a[U], b[U];
+  f32x4v acc[2] = {(f32x4v)(0.0f), (f32x4v)(0.0f)};
+  auto load = [&](Both (&c)[U], int s) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t at = min(s + u, s1 - 1);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        c[u].w[h] = __builtin_nontemporal_load(
+            reinterpret_cast<const u32x4v *>(w + at * 2048 + h * 256));
+#pragma unroll
+      for (int i = 0; i < X; ++i)
+        c[u].x[i] = load8v(reinterpret_cast<const uint16_t *>(
+            x + at * (2048 * X) + i * 1024));
+    }
+  };
+  auto multiply = [&](const Both &c) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if constexpr (FP8) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              fp8_to_bf16(c.w[h][2 * i], c.w[h][2 * i + 1]), c.x[i], acc[h], 0,
+              0, 0);
+      } else {
+        union { u32x4v u; bf16x8v v; } t;
+        t.u = c.w[h];
+        acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t.v, c.x[0], acc[h],
+                                                         0, 0, 0);
+      }
+    }
+  };
+  stream_chunks<true>(a, b, s0, s1, load, multiply, meanwhile);
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      red[wid][h * 16 + grp * 4 + r][i16] = acc[h][r];
+}
+
+// FEW: up to 16 rows, K a multiple of 32 (e4m3: 64).
+template <bool FP8, Kind KIND, bool FEW>
 __global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
     const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws, int M,
     int N, int K, Ends e) {
+  __shared__ __attribute__((aligned(16))) float red[4][32][FEW ? 17 : MMAX];
   Early<KIND> early;
-  early.begin(e, M);
-  const f32x16v acc =
-      weight_stream<FP8>(xs, ws, M, K, [&] { early.rest(e, M); });
-  finish<KIND>(acc, e, early, M, N);
+  const bool mine = !FEW || Early<KIND>::mine(M);
+  if (mine) {
+    early.begin(e, M);
+    if constexpr (FP8) early.begin_scale(e);
+  }
+  auto meanwhile = [&] {
+    if (mine) early.rest(e, M);
+  };
+  if constexpr (FEW) weight_stream16<FP8>(xs, ws, M, K, red, meanwhile);
+  else weight_stream<FP8>(xs, ws, M, K, red, meanwhile);
+  finish<FP8, KIND, FEW ? 17 : MMAX>(red, e, early, M, N);
 }
 
 // 17 to 128 rows (RB blocks of 32): x is longer than W's share of a workgroup, so
@@ -601,12 +706,17 @@ static void launch(Kind kind, const at::Tensor &xs, const at::Tensor &ws,
                        (const uint8_t *)ws.data_ptr(), (int)M, (int)N, (int)K,
                        e);
   };
-  switch (kind) {
-    case ends::SLAB: return go(decode_gemm_kernel<FP8, ends::SLAB>);
-    case ends::PLAIN: return go(decode_gemm_kernel<FP8, ends::PLAIN>);
-    case ends::GLU: return go(decode_gemm_kernel<FP8, ends::GLU>);
-    case ends::QKV: return go(decode_gemm_kernel<FP8, ends::QKV>);
-  }
+  auto of = [&](auto few) {
+    constexpr bool FEW = decltype(few)::value;
+    switch (kind) {
+      case ends::SLAB: return go(decode_gemm_kernel<FP8, ends::SLAB, FEW>);
+      case ends::PLAIN: return go(decode_gemm_kernel<FP8, ends::PLAIN, FEW>);
+      case ends::GLU: return go(decode_gemm_kernel<FP8, ends::GLU, FEW>);
+      case ends::QKV: return go(decode_gemm_kernel<FP8, ends::QKV, FEW>);
+    }
+  };
+  if (M <= 16 && K % (FP8 ? 64 : 32) == 0) of(std::true_type{});
+  else of(std::false_type{});
 }
 
 // The sums of a product as slabs [split, M, N], or, unsplit, y [M, N] bf16.

@@ -46,11 +46,11 @@ struct Sum {
 //   4096 x 4096        12.0  8.1   13.2  8.4   13.8 10.1
 //   4096 x 11008       21.0 19.1   22.0 20.5   23.8 24.0
 //   3072 x 24576       34.9 31.5   34.2 33.7   39.7 45.7
-//   4096 x 4096  e4m3  10.1  6.3   11.2  7.5   12.4  8.6
+//   4096 x 4096  e4m3  10.1  5.6   11.2  6.7   12.4  8.1
 //   4096 x 11008 e4m3  16.0 12.3   16.4 13.0   18.4 17.8
 template <bool FP8, int B>
 __global__ __launch_bounds__(BLOCK, 1) void decode_res_kernel(Sum a) {
-  constexpr int X = FP8 ? 2 : 1, U = B == 1 ? (FP8 ? 6 : 8) : 4;
+  constexpr int X = FP8 ? 2 : 1, U = B == 1 ? 8 : 4;
   const int tid = threadIdx.x;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, i16 = lane & 15, grp = lane >> 4;

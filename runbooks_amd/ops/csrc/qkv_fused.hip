@@ -145,12 +145,17 @@ __global__ __launch_bounds__(BLOCK) void qkv_rope_append_kernel(Args a) {
     Chunk<V> x, z;
     x.load(src);
     z.load(src + half);
+    // before the rotation waits for the position
+    const int slot = a.slots[t];
     if (h < a.hq + a.hkv) {
       const int64_t p = (int64_t)a.pos[t] * half + d;
+      float cs[V], sn[V];
+      __builtin_memcpy(cs, a.cs + p, sizeof(cs));   // tables begin anywhere
+      __builtin_memcpy(sn, a.sn + p, sizeof(sn));
 #pragma unroll
       for (int e = 0; e < V; ++e) {
         const float u = rb::bf16_to_f32(x.v[e]), w = rb::bf16_to_f32(z.v[e]);
-        const float c = a.cs[p + e], s = a.sn[p + e];
+        const float c = cs[e], s = sn[e];
         x.v[e] = rb::f32_to_bf16(u * c - w * s);
         z.v[e] = rb::f32_to_bf16(w * c + u * s);
       }
@@ -166,7 +171,6 @@ __global__ __launch_bounds__(BLOCK) void qkv_rope_append_kernel(Args a) {
     }
     const bool is_v = h >= a.hq + a.hkv;
     const int kh = h - a.hq - (is_v ? a.hkv : 0);
-    const int slot = a.slots[t];
     uint8_t qx[V], qz[V];
     float scale = 0.0f;
     // all lanes of a row take part, whatever its slot
@@ -188,11 +192,8 @@ __global__ __launch_bounds__(BLOCK) void qkv_rope_append_kernel(Args a) {
       } else {
         uint8_t *dst = (uint8_t *)(is_v ? a.v_cache : a.k_cache) +
                        (head * a.bs + off) * (a.dh + 16) + d;
-#pragma unroll
-        for (int e = 0; e < V; ++e) {
-          dst[e] = qx[e];
-          dst[half + e] = qz[e];
-        }
+        __builtin_memcpy(dst, qx, V);
+        __builtin_memcpy(dst + half, qz, V);
         if (d == 0) *reinterpret_cast<float *>(dst + a.dh) = scale;
       }
     } else if (VT && is_v) {

@@ -72,6 +72,26 @@ def test_gated_unit(m, inter, k, parts, fp8, gelu):
         assert _rel(_rows(h, inter, m), ref) < BF16
 
 
+@pytest.mark.parametrize("m", [1, 15, 16, 17])
+@pytest.mark.parametrize("n,k,fp8", [
+    (64, 1040, False), (64, 1056, False), (4096, 1088, False),
+    (64, 1056, True), (64, 1088, True), (4096, 4160, True), (96, 64, True)])
+def test_few_rows(m, n, k, fp8):
+    """Products of 16 x 16 and, of more rows or odd lengths of sums, of 32 x 32, whole
+    and in parts, of fewer columns of x than there are waves too."""
+    torch.manual_seed(m + k)
+    ws, scale, w = _weight(n, k, 0, fp8)
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    e, ref = ops.ext(), x.double() @ w.t()
+    args = (e.decode_swizzle_x(x), ws) + ((scale,) if fp8 else ()) + (m, n, k)
+    y = (e.decode_gemm_fp8 if fp8 else e.decode_gemm)(*args)
+    assert _rel(y, ref) < BF16
+    raw = e.decode_gemm_fp8(*args, raw=True) if fp8 else \
+        e.decode_gemm_raw(*args, True)
+    if raw.dtype == torch.float32:
+        assert _rel(raw.double().sum(0), ref) < 1e-5
+
+
 @pytest.mark.parametrize("m", [1, 33, 64, 65, 128])
 @pytest.mark.parametrize("inter,k", [(16, 1024), (10256, 1040)])
 def test_gated_unit_of_rows(m, inter, k):

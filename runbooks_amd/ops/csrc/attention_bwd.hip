@@ -29,6 +29,10 @@
 //   3001 tokens, 32 query and 8 kv heads of 128    1864 -> 344 us, 751 TF/s
 //   4 x 512 tokens, 32 heads of 128                 284 ->  79 us
 //   4000 tokens, 32 heads of 64                     941 -> 260 us, 883 TF/s
+// Since then, with loads to LDS that the compiler does not wait for, operands read
+// ahead, and dK/dV's whole tiles in slots of a product and what stands beside it: 302 ->
+// 283, 71 -> 69; 512 tokens, 32 heads of 128 42.5 -> 39.6. dQ in slots spills (256
+// registers, two waves a SIMD): 333 us both kernels.
 //
 // mfma_f32_32x32x16_bf16 layouts:
 //   A[i][k]: i = lane&31, k = (lane>>5)*8 + e
@@ -116,10 +120,10 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
   const int64_t kv_stride = a.kv_stride;
   const int64_t kv0 = (int64_t)at.batch * S * kv_stride + h_kv * DH;
   const uint16_t *kb = a.k + kv0, *vb = a.v + kv0;
-  const TileLoad<DH, NW> load(wid, lane);
+  const TileLoad<DH, NW> load(wid, lane, kv_stride);
   const int n_tiles = (min(S, at.tile * QT + QT) + ROWS - 1) / ROWS;
-  load(kb, kv_stride, 0, S, smem, wid);
-  load(vb, kv_stride, 0, S, smem + TILE, wid);
+  load(kb, 0, S, smem, wid);
+  load(vb, 0, S, smem + TILE, wid);
 
   const int64_t token = (int64_t)at.batch * S + (q_valid ? qrow : 0);
   const int64_t row0 = (token * a.Hq + at.head) * DH;    // of dout, out
@@ -174,6 +178,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
       dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
           row_frag<DH>(vt, r0, ks, col, hi), dof[ks], dp, 0, 0, 0);
     }
+    if constexpr (!ORDERED) reads_ahead<2 * KSTEPS, 4>();
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       float p = ORDERED ? __expf(s[r] * by - lse)
@@ -198,8 +203,8 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_bwd_dq_kernel(Args a) {
     __syncthreads();                    // nobody reads the other buffer any more
     if (t + 1 < n_tiles) {
       char *next = smem + (~t & 1) * 2 * TILE;
-      load(kb, kv_stride, (t + 1) * ROWS, S, next, wid);
-      load(vb, kv_stride, (t + 1) * ROWS, S, next + TILE, wid);
+      load(kb, (t + 1) * ROWS, S, next, wid);
+      load(vb, (t + 1) * ROWS, S, next + TILE, wid);
     }
   };
   const Walk mine = walk(wrow, S);
@@ -249,14 +254,15 @@ void fa_bwd_dkdv_kernel(Args a) {
   const uint16_t *ob = a.dout + token0 * o_stride + at.head * DH;
   const int64_t stat = ((int64_t)at.batch * a.Hq + at.head) * S;
   const float by = unit(a.scale), to2 = by * LOG2E;
-  const TileLoad<DH, NW> load(wid, lane);
+  const TileLoad<DH, NW> load_q(wid, lane, a.q_stride);
+  const TileLoad<DH, NW> load_o(wid, lane, o_stride);
   const int tile0 = at.tile * KT / ROWS, n_tiles = (S + ROWS - 1) / ROWS;
 
   // tile t's rows and statistics; the latter through registers, stored when
   // the tile before it has been worked on
   auto send = [&](int t, char *tile) {
-    load(qb, a.q_stride, t * ROWS, S, tile, wid);
-    load(ob, o_stride, t * ROWS, S, tile + TILE, wid);
+    load_q(qb, t * ROWS, S, tile, wid);
+    load_o(ob, t * ROWS, S, tile + TILE, wid);
   };
   char *stats = smem + 4 * TILE;        // two buffers, like the tiles
   auto stat_of = [&](int t) {
@@ -285,6 +291,9 @@ void fa_bwd_dkdv_kernel(Args a) {
     load_row<DH>(kf, a.k + row0, hi);
     clear_if<DH>(a.scale == 0.0f, kf);
     load_row<DH>(vf, a.v + row0, hi);
+    // where the compiler sees it: otherwise it waits for these in the loop, and with
+    // them for the tiles that are on their way
+    __builtin_amdgcn_s_waitcnt(0x0f70);         // vmcnt(0)
   }
   f32x16v acc_dk[DTILES], acc_dv[DTILES];
 #pragma unroll
@@ -293,11 +302,9 @@ void fa_bwd_dkdv_kernel(Args a) {
     acc_dv[dt] = (f32x16v)(0.0f);
   }
 
-  // queries qbase .. qbase + 31, rows r0 .. of the tile
-  auto queries = [&](const char *qt, const float *st, int qbase, int r0,
-                     auto masked) {
-    const char *ot = qt + TILE;
-    f32x16v s = (f32x16v)(0.0f), dp = (f32x16v)(0.0f), lse, dvec;
+  // scores and dP of queries r0 .. r0 + 31 of a tile
+  auto products = [&](f32x16v &s, f32x16v &dp, f32x16v &lse, f32x16v &dvec,
+                      const char *qt, const float *st, int r0) {
 #pragma unroll
     for (int rq = 0; rq < 4; ++rq) {
       const float4 l = *reinterpret_cast<const float4 *>(
@@ -309,17 +316,19 @@ void fa_bwd_dkdv_kernel(Args a) {
       dvec[rq * 4] = d.x; dvec[rq * 4 + 1] = d.y;
       dvec[rq * 4 + 2] = d.z; dvec[rq * 4 + 3] = d.w;
     }
-    if constexpr (!ORDERED) {
-      s = lse;
-      dp = dvec;
-    }
+    s = ORDERED ? (f32x16v)(0.0f) : lse;
+    dp = ORDERED ? (f32x16v)(0.0f) : dvec;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
       s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
           row_frag<DH>(qt, r0, ks, col, hi), kf[ks], s, 0, 0, 0);
       dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-          row_frag<DH>(ot, r0, ks, col, hi), vf[ks], dp, 0, 0, 0);
+          row_frag<DH>(qt + TILE, r0, ks, col, hi), vf[ks], dp, 0, 0, 0);
     }
+  };
+  // P and dS, of queries qbase ..
+  auto weigh = [&](f32x16v &s, f32x16v &dp, const f32x16v &lse,
+                   const f32x16v &dvec, int qbase, auto masked) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       float p = ORDERED ? __expf(s[r] * by - lse[r])
@@ -329,6 +338,8 @@ void fa_bwd_dkdv_kernel(Args a) {
       s[r] = p;
       dp[r] = ORDERED ? p * (dp[r] - dvec[r]) * a.scale : dp[r] * p;
     }
+  };
+  auto add = [&](const f32x16v &s, const f32x16v &dp, const char *qt, int r0) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       const bf16x8v pf = score_frag<ORDERED>(s, ks);
@@ -336,13 +347,93 @@ void fa_bwd_dkdv_kernel(Args a) {
 #pragma unroll
       for (int dt = 0; dt < DTILES; ++dt) {
         acc_dv[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            column_frag<DH, ORDERED>(ot, r0 + ks * 16, dt, lane), pf,
+            column_frag<DH, ORDERED>(qt + TILE, r0 + ks * 16, dt, lane), pf,
             acc_dv[dt], 0, 0, 0);
         acc_dk[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
             column_frag<DH, ORDERED>(qt, r0 + ks * 16, dt, lane), dsf,
             acc_dk[dt], 0, 0, 0);
       }
     }
+  };
+  auto queries = [&](const char *qt, const float *st, int qbase, int r0,
+                     auto masked) {
+    f32x16v s, dp, lse, dvec;
+    products(s, dp, lse, dvec, qt, st, r0);
+    weigh(s, dp, lse, dvec, qbase, masked);
+    add(s, dp, qt, r0);
+  };
+  // A whole tile that is seen whole: its 8 KSTEPS products, each with what is issued
+  // beside it. A SIMD has one wave of these, whose vector instructions (weights of a
+  // half, 32 queries) take half as long as its products, and which does both at a
+  // time only where they stand in turns; operands are read AHEAD products ahead.
+  auto tile_of = [&](const char *qt, const float *st) {
+    constexpr int N = 2 * KSTEPS, AHEAD = 8, SUMS = 2 * DTILES;
+    static_assert(N == 2 * SUMS && 16 % N == 0, "as many products either way");
+    f32x16v s[2], dp[2];
+    bf16x8v ring[AHEAD], pf[2][2], df[2][2];
+    auto statistics = [&](auto half) {
+      constexpr int u = decltype(half)::value;
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq) {
+        const float4 l = *reinterpret_cast<const float4 *>(
+            st + u * 32 + 8 * rq + 4 * hi);
+        const float4 d = *reinterpret_cast<const float4 *>(
+            st + ROWS + u * 32 + 8 * rq + 4 * hi);
+        s[u][rq * 4] = l.x; s[u][rq * 4 + 1] = l.y;
+        s[u][rq * 4 + 2] = l.z; s[u][rq * 4 + 3] = l.w;
+        dp[u][rq * 4] = d.x; dp[u][rq * 4 + 1] = d.y;
+        dp[u][rq * 4 + 2] = d.z; dp[u][rq * 4 + 3] = d.w;
+      }
+    };
+    auto read = [&](auto at) {
+      constexpr int q = decltype(at)::value, u = q / N % 2, i = q % N;
+      const char *tile = qt + (q < 2 * N ? i % 2 : 1 - i % 2) * TILE;
+      if constexpr (q < 2 * N)
+        ring[q % AHEAD] = row_frag<DH>(tile, u * 32, i / 2, col, hi);
+      else
+        ring[q % AHEAD] = column_frag<DH>(tile, u * 32 + i / SUMS * 16,
+                                          i % SUMS / 2, lane);
+    };
+    // elements of half u that stand beside product i
+    auto weights = [&](auto half, auto at) {
+      constexpr int u = decltype(half)::value, i = decltype(at)::value;
+      constexpr int E = 16 / N, r0 = (i - 2) * E, r1 = i + 1 == N ? 16 : r0 + E;
+#pragma unroll
+      for (int r = r0; r < r1; ++r) {
+        s[u][r] = __builtin_amdgcn_exp2f(s[u][r] * to2);
+        dp[u][r] *= s[u][r];
+        if (r % 8 == 7) {
+          pf[u][r / 8] = score_frag(s[u], r / 8);
+          df[u][r / 8] = score_frag(dp[u], r / 8);
+        }
+      }
+    };
+    auto slot = [&](auto at) __attribute__((always_inline)) {
+      constexpr int q = decltype(at)::value, u = q / N % 2, i = q % N;
+      __builtin_amdgcn_sched_barrier(0);
+      const bf16x8v x = ring[q % AHEAD];
+      if constexpr (q < 2 * N) {
+        f32x16v &c = i % 2 == 0 ? s[u] : dp[u];
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            x, i % 2 == 0 ? kf[i / 2] : vf[i / 2], c, 0, 0, 0);
+      } else {
+        f32x16v &c = i % 2 == 0 ? acc_dv[i % SUMS / 2] : acc_dk[i % SUMS / 2];
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            x, i % 2 == 0 ? pf[u][i / SUMS] : df[u][i / SUMS], c, 0, 0, 0);
+      }
+      if constexpr (q + AHEAD < 4 * N)
+        read(std::integral_constant<int, q + AHEAD>());
+      if constexpr (q == 2) statistics(std::integral_constant<int, 1>());
+      // of the first half beside the second one's scores, of the second beside the
+      // first one's sums, two products behind the last that they need
+      if constexpr ((q / N == 1 || q / N == 2) && i >= 2)
+        weights(std::integral_constant<int, q / N - 1>(),
+                std::integral_constant<int, i>());
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    statistics(std::integral_constant<int, 0>());
+    each<AHEAD>(read);
+    each<4 * N>(slot);
   };
   auto step = [&](int t, auto masked) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -355,10 +446,14 @@ void fa_bwd_dkdv_kernel(Args a) {
     const char *qt = smem + (t & 1) * 2 * TILE;
     const float *st = reinterpret_cast<const float *>(stats +
                                                       (t & 1) * STATS);
+    if constexpr (!ORDERED && !decltype(masked)::value) {
+      tile_of(qt, st);
+    } else {
 #pragma unroll
-    for (int r0 = 0; r0 < ROWS; r0 += 32)
-      if (!decltype(masked)::value || t * ROWS + r0 + 31 >= wkey)
-        queries(qt, st, t * ROWS + r0, r0, masked);
+      for (int r0 = 0; r0 < ROWS; r0 += 32)
+        if (!decltype(masked)::value || t * ROWS + r0 + 31 >= wkey)
+          queries(qt, st, t * ROWS + r0, r0, masked);
+    }
     if (t + 1 < n_tiles) keep(t + 1, next);
   };
   // tiles that some of the workgroup's keys do not see whole, then the others

@@ -21,6 +21,14 @@
 //   512 tokens, 32 heads of 128                      43 ->  13 us
 //   1021 tokens, 16 heads of 256                    133 ->  36 us
 //   4000 tokens, 32 heads of 64                     288 ->  89 us,  737 TF/s
+// Since then, with loads to LDS that the compiler does not wait for, operands read
+// ahead (flash_tile.h) and, of heads of 256, sums that stay in the matrix registers, on
+// another card: 7931 tokens 510 -> 491, 2048 of 32 heads 54 -> 49, 1021 of 32 heads
+// 22.7 -> 21.5; 16 heads of 256, 7931 713 -> 650, 3000 138 -> 129, 1021 36 -> 35. What is
+// left: the two waves of a SIMD do the same at the same time, so that products and
+// vector instructions take turns (48% of the time each). Two groups of waves a half-step
+// apart, a barrier between half-steps, took as long: a half-step of products then waits
+// for LDS (1860 clocks, 1024 of products).
 //
 // mfma_f32_32x32x16_bf16 layouts:
 //   A[i][k]: i = lane&31, k = (lane>>5)*8 + e (e = 0..7)
@@ -43,6 +51,26 @@ using namespace flash;
 
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float RISE = 8.0f;           // of a maximum before it is moved
+
+// c += a b, c in the matrix registers: as text, for with more sums than there are
+// vector registers the compiler moves them back and forth in every step. FRESH: b has
+// just been computed.
+template <bool FRESH>
+RB_DEV void add_product(f32x16v &c, bf16x8v a, bf16x8v b) {
+  if constexpr (FRESH)
+    asm volatile("s_nop 3\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
+                 : "+a"(c) : "v"(a), "v"(b));
+  else
+    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
+                 : "+a"(c) : "v"(a), "v"(b));
+}
+
+RB_DEV void scale_sum(float &c, float by) {
+  float t;
+  asm volatile(
+      "v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %2, %1\n\t"
+      "v_accvgpr_write_b32 %0, %1" : "+a"(c), "=&v"(t) : "v"(by));
+}
 
 // SPLIT 2: two waves share 32 query rows, one takes the lower and one the upper
 // 32 keys of every tile; their results meet in LDS at the end.
@@ -85,11 +113,11 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
 
   const uint16_t *kb = kp + (int64_t)b * S * kv_stride + h_kv * DH;
   const uint16_t *vb = vp + (int64_t)b * S * kv_stride + h_kv * DH;
-  const TileLoad<DH, NW> load(wid, lane);
+  const TileLoad<DH, NW> load(wid, lane, kv_stride);
   const int kv_end = min(S, q0 + QT);       // causal upper bound for this WG
   const int n_tiles = (kv_end + ROWS - 1) / ROWS;
-  load(kb, kv_stride, 0, S, smem, wid);
-  load(vb, kv_stride, 0, S, smem + TILE, wid);
+  load(kb, 0, S, smem, wid);
+  load(vb, 0, S, smem + TILE, wid);
 
   // ---- Q fragments (B operand of K Q^T); a factor below zero goes into
   // their signs, so that scores and their maxima have one order, and a factor
@@ -121,6 +149,18 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
   float m_run = -INFINITY;                  // in exponents of 2 (ORDERED: of e)
   float l_run = 0.0f;
 
+  // Wide heads have more sums than there is room for among the vector registers. The
+  // last products that the compiler does not see are done where a step's scores are,
+  // behind them in the same unit; elsewhere this waits for them.
+  constexpr bool TEXT = DH == 256;
+  auto settle = [&] {
+    if constexpr (TEXT)
+#pragma unroll
+      for (int dt = 0; dt < DTILES; ++dt)
+        asm volatile("s_nop 15" : "+a"(acc_o[dt]));
+  };
+  settle();
+
   // Keys kbase .. kbase + 32 SUB - 1 of the tile, from row r0 on; `masked`:
   // some of them are hidden from some row
   constexpr int SUB = DH == 256 || SPLIT == 2 || ORDERED ? 1 : 2;
@@ -135,6 +175,8 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
         s[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
             row_frag<DH>(kt, r0 + u * 32, ks, col, hi), qf[ks], s[u], 0, 0, 0);
     }
+    // (of heads of 64 it changes nothing, of 256 it costs 4%)
+    if constexpr (DH == 128) reads_ahead<SUB * KSTEPS, 8>();
     if constexpr (decltype(masked)::value) {
 #pragma unroll
       for (int u = 0; u < SUB; ++u)
@@ -190,8 +232,16 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
 #pragma unroll
       for (int dt = 0; dt < DTILES; ++dt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc_o[dt][r] *= alpha;
+        for (int r = 0; r < 16; ++r) {
+          if constexpr (TEXT) {
+            float c = acc_o[dt][r];
+            scale_sum(c, alpha);
+            acc_o[dt][r] = c;
+          }
+          else acc_o[dt][r] *= alpha;
+        }
       m_run = mn;
+      settle();
     }
     const float ref = m_run == -INFINITY ? 0.0f : m_run;
 #pragma unroll
@@ -205,10 +255,16 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
       for (int ks = 0; ks < 2; ++ks) {
         const bf16x8v pf = score_frag(s[u], ks);
 #pragma unroll
-        for (int dt = 0; dt < DTILES; ++dt)
-          acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              column_frag<DH>(vt, r0 + u * 32 + ks * 16, dt, lane), pf,
-              acc_o[dt], 0, 0, 0);
+        for (int dt = 0; dt < DTILES; ++dt) {
+          const bf16x8v vf =
+              column_frag<DH>(vt, r0 + u * 32 + ks * 16, dt, lane);
+          if constexpr (TEXT)
+            dt == 0 ? add_product<true>(acc_o[dt], vf, pf)
+                    : add_product<false>(acc_o[dt], vf, pf);
+          else
+            acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf, acc_o[dt],
+                                                                0, 0, 0);
+        }
       }
     }
   };
@@ -219,8 +275,8 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
     __syncthreads();                    // nobody reads the other buffer any more
     if (t + 1 < n_tiles) {
       char *next = smem + (~t & 1) * 2 * TILE;
-      load(kb, kv_stride, (t + 1) * ROWS, S, next, wid);
-      load(vb, kv_stride, (t + 1) * ROWS, S, next + TILE, wid);
+      load(kb, (t + 1) * ROWS, S, next, wid);
+      load(vb, (t + 1) * ROWS, S, next + TILE, wid);
     }
   };
   // first all-visible tiles, then those on the diagonal, then those that only
@@ -235,17 +291,22 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
       keys(kt, kt + TILE, t * ROWS + i + part * 32, i + part * 32,
            std::false_type{});
   }
-  for (; t < n_tiles; ++t) {
+  // (TEXT: a branch around the sums would have them moved, so that a half that is
+  // hidden from all rows of a wave is computed too)
+  const int seen = TEXT ? min(n_tiles, (mine.last + ROWS) / ROWS) : n_tiles;
+  for (; t < seen; ++t) {
     arrive(t);
     const char *kt = smem + (t & 1) * 2 * TILE;
 #pragma unroll
     for (int i = 0; i < ROWS; i += SUB * 32 * SPLIT) {
       const int r0 = i + part * 32, kbase = t * ROWS + r0;
-      if (kbase <= mine.last)
+      if (TEXT || kbase <= mine.last)
         keys(kt, kt + TILE, kbase, r0, std::true_type{});
     }
   }
+  for (; t < n_tiles; ++t) arrive(t);
 
+  settle();
   if constexpr (SPLIT == 2) {
     // lane-major pieces of 16 bytes: the result, maximum and sum of part 1
     constexpr int PIECES = DTILES * 4;

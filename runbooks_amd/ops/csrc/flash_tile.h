@@ -12,6 +12,9 @@
 
 #include <torch/extension.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "common.h"
 
 namespace flash {
@@ -23,6 +26,7 @@ static inline at::Tensor aligned16(const at::Tensor &t) {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8v;
 typedef __attribute__((ext_vector_type(16))) float f32x16v;
+using rb::u32x4v;
 
 constexpr int ROWS = 64;               // of a tile
 
@@ -35,6 +39,29 @@ RB_DEV unsigned pack2(float lo, float hi) {
   return c.u;
 }
 
+// The order of a block's instructions: N products, an operand of each read from LDS
+// AHEAD products before it. Left to itself the compiler has every product wait for a
+// read of its own. us, 32 heads of 128, with that and without: 1021 tokens 21.5 and
+// 22.9, 2000 (four waves of whole keys) 50 and 55.
+template <int N, int AHEAD> RB_DEV void reads_ahead() {
+  __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+  for (int i = 0; i < N - AHEAD; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
+}
+
+// f of 0 .. N - 1, known where it is compiled.
+template <class F, int... Q>
+RB_DEV void each_of(F &f, std::integer_sequence<int, Q...>) {
+  (f(std::integral_constant<int, Q>()), ...);
+}
+template <int N, class F> RB_DEV void each(F &f) {
+  each_of(f, std::make_integer_sequence<int, N>());
+}
+
 template <int DH> RB_DEV constexpr int mix(int row) {
   return DH == 64 ? ((row >> 1 & 1) << 2) | (row >> 2 & 3)
                   : ((row & 3) << 2) | (row >> 2 & 3);
@@ -44,33 +71,39 @@ template <int DH> constexpr int tile_bytes() { return ROWS * DH * 2; }
 
 // Loads of a tile by NW waves: piece i of wave w is the kilobyte (1024 bytes
 // of LDS) i * NW + w of the tile, STEP rows after the one before; mix() is
-// linear in the bits of a row.
+// linear in the bits of a row. Rows `stride` elements apart.
 template <int DH, int NW> struct TileLoad {
   static constexpr int PIECES = tile_bytes<DH>() / 1024 / NW;
   static constexpr int CHUNKS = DH / 8;          // of a row
   static constexpr int STEP = NW * 64 / CHUNKS;
-  int row, off;                                  // of piece 0 (off: elements)
+  unsigned at[PIECES];                           // bytes from a tile's first row
+  int64_t stride;
 
-  RB_DEV TileLoad(int wid, int lane) {
-    const int at = wid * 64 + lane;
-    row = at / CHUNKS;
-    off = (at % CHUNKS ^ mix<DH>(row)) * 8;
+  RB_DEV TileLoad(int wid, int lane, int64_t stride) : stride(stride) {
+    const int piece = wid * 64 + lane;
+    const int row = piece / CHUNKS, off = piece % CHUNKS ^ mix<DH>(row);
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+      at[i] = (unsigned)(row + i * STEP) * (unsigned)(stride * 2) +
+              (off ^ mix<DH>(i * STEP)) * 16;
   }
 
-  // Rows r0 .. r0 + 63 of `rows` rows, `stride` elements apart from `base`
-  // on; rows past the end are the last one again. `tile` is uniform.
-  RB_DEV void operator()(const uint16_t *base, int64_t stride, int r0,
-                         int rows, char *tile, int wid) const {
+  // Rows r0 .. r0 + 63 of `rows` rows from `base` on; rows past the end are zeros.
+  // `tile` is uniform. The caller waits (vmcnt): the compiler, which would wait for
+  // all loads to LDS before the next read of it, does not see these. Addresses are
+  // the tile's, in scalar registers, and these. us before, with loads that it saw
+  // and addresses of each lane, and now: the forward of 7931 tokens, 16 heads of
+  // 256 714 and 682, 5000 tokens, 16 heads of 64 81 and 79.
+  RB_DEV void operator()(const uint16_t *base, int r0, int rows, char *tile,
+                         int wid) const {
+    const int n = min(rows - r0, ROWS);
+    const u32x4v from = rb::buffer(
+        base + r0 * stride, n > 0 ? (uint32_t)((n - 1) * stride + DH) * 2 : 0);
+    const unsigned to = __builtin_amdgcn_readfirstlane(
+        (unsigned)(size_t)(__attribute__((address_space(3))) char *)tile);
 #pragma unroll
-    for (int i = 0; i < PIECES; ++i) {
-      const uint16_t *p =
-          base + (int64_t)min(r0 + row + i * STEP, rows - 1) * stride +
-          (off ^ mix<DH>(i * STEP) * 8);
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) uint32_t *)(const void *)p,
-          (__attribute__((address_space(3))) uint32_t *)(void *)(
-              tile + (i * NW + wid) * 1024), 16, 0, 0);
-    }
+    for (int i = 0; i < PIECES; ++i)
+      rb::lds_load(from, at[i], 0, to + (i * NW + wid) * 1024);
   }
 };
 

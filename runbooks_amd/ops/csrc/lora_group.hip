@@ -318,11 +318,11 @@ RB_DEV void lora_grad_tile(const Grad &g, const Adapters &a, int64_t T, int c0,
   const int b1 = (int)(blocks * (share + 1) / g.shares);
 
   // columns past the end: the last ones again, not stored
-  const flash::TileLoad<64, 4> load(wid, lane);
+  const flash::TileLoad<64, 4> load(wid, lane, C);
   const uint16_t *xc = x + min(c0, C - 64);
   auto send = [&](int b, char *buf) {
-    load(xc, C, b * 128, (int)T, buf, wid);
-    load(xc, C, b * 128 + 64, (int)T, buf + TILE, wid);
+    load(xc, b * 128, (int)T, buf, wid);
+    load(xc, b * 128 + 64, (int)T, buf + TILE, wid);
     // m's rows: 16 bytes a lane, rows past the end as zeros
     for (int n = 0; n < mats; ++n) {
       const uint16_t *src = m + (of + n) * T * R;

@@ -423,6 +423,26 @@ def _hashed(n, salt):
     return ((h & 0xffff).float() / 65536 - 0.5) * 4
 
 
+@pytest.mark.parametrize("S,hq,dh", [(160, 4, 64), (160, 4, 128), (97, 4, 256),
+                                     (330, 4, 256), (1313, 32, 256)])
+def test_flash_rising_scores(S, hq, dh):
+    """Scores that rise with the key, so that every tile moves the maximum and with it
+    the sums before it, to nearly nothing: rounded probabilities and results."""
+    _assert_hip()
+    torch.manual_seed(dh)
+    q = torch.full((1, S, hq, dh), 0.5, device=DEV).bfloat16()
+    k = (torch.arange(S, device=DEV) / (8 * dh ** 0.5))[None, :, None, None] \
+        .expand(1, S, hq, dh).bfloat16().contiguous()
+    v = torch.randn(1, S, hq, dh, device=DEV).bfloat16()
+    out = ops.ext().flash_prefill(q, k, v, 4.0)
+    for h in range(0, hq, 7):
+        s = q[0, :, h].double() @ k[0, :, h].double().t() * 4.0
+        s = s.masked_fill(torch.ones(S, S, dtype=torch.bool, device=DEV).triu(1),
+                          -torch.inf)
+        ref = s.softmax(-1) @ v[0, :, h].double()
+        assert (out[0, :, h].double() - ref).norm() <= 2 ** -7 * ref.norm()
+
+
 @pytest.mark.parametrize("B,S,Hq,Hkv,bits", [
     (1, 1, 1, 1, (4093165637, 932004135, 3265854109, 3265854109, 34914089)),
     (2, 31, 3, 3, (2980831709, 3346004597, 2951792153, 627292471,

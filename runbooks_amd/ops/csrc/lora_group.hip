@@ -21,7 +21,7 @@
 //   lora_down          19, 18, 7.7    19, 14, 6.5    -, 22, 11
 //   lora_add (columns) 26, 18, 18     53, 42, 42
 //   lora_down_columns  70, 13, 10     57, 25, 22     -, 7.2, 5.3
-//   dB and dA          96, 29, 25     71, 40, 33     -, 30, 22
+//   dB and dA          96, 29, 23     71, 40, 32     -, 30, 21
 //   lora_add (sum)     18, 8, 8       18, 8, 8
 // and no additions of dx, copies of t or transposes of A around them.
 //
@@ -323,15 +323,17 @@ RB_DEV void lora_grad_tile(const Grad &g, const Adapters &a, int64_t T, int c0,
   auto send = [&](int b, char *buf) {
     load(xc, b * 128, (int)T, buf, wid);
     load(xc, b * 128 + 64, (int)T, buf + TILE, wid);
-    // m's rows: 16 bytes a lane, rows past the end as zeros
-    for (int n = 0; n < mats; ++n) {
-      const uint16_t *src = m + (of + n) * T * R;
-      const int64_t row = (int64_t)b * 128 + tid / 2;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (row < T)
-        v = *reinterpret_cast<const uint4 *>(src + row * R + tid % 2 * 8);
-      *reinterpret_cast<uint4 *>(buf + 2 * TILE + n * MB + tid * 16) = v;
-    }
+    // m's rows past the registers too: by them, they were waited for as soon as they
+    // were sent for, and what is ahead of them with them (dB and dA of 2048 rows, q, k, v
+    // 27.2 and 25.3 us, gate and up 33.7 and 32.8, down 22.9 and 21.4)
+    const int64_t row = (int64_t)b * 128;
+    const uint32_t bytes = (uint32_t)max(min((int)(T - row), 128), 0) * (R * 2);
+    const unsigned to = __builtin_amdgcn_readfirstlane(
+        (unsigned)(size_t)(__attribute__((address_space(3))) char *)buf +
+        2 * TILE + wid * 1024);
+    for (int n = 0; n < mats; ++n)
+      rb::lds_load(rb::buffer(m + ((of + n) * T + row) * R, bytes), tid * 16, 0,
+                   to + n * MB);
   };
   f32x16v acc[2][NB];
 #pragma unroll
@@ -343,14 +345,6 @@ RB_DEV void lora_grad_tile(const Grad &g, const Adapters &a, int64_t T, int c0,
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     char *buf = smem + ((b - b0) & 1) * BUF;
-    if ((b + 1) * 128 > T) {
-      // rows past the end, which m's zeros would not hide if the last row,
-      // which they repeat, is not finite
-      for (int at = (int)(T - b * 128) * 128 + tid * 16; at < 2 * TILE;
-           at += 256 * 16)
-        *reinterpret_cast<uint4 *>(buf + at) = make_uint4(0, 0, 0, 0);
-      __syncthreads();
-    }
     if (b + 1 < b1) send(b + 1, smem + ((b - b0 + 1) & 1) * BUF);
     const char *tile = buf + (wid >> 1) * TILE;
 #pragma unroll

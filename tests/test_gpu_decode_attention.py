@@ -61,6 +61,29 @@ def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
                                operand.view(-1, 32, 8)[:, :batch])
 
 
+@pytest.mark.parametrize("parts", [15, 16, 17, 64, 65, 81])
+@pytest.mark.parametrize("dh", [64, 128, 256])
+def test_many_parts(dh, parts):
+    """The merge takes 16 rows at a time and 64 weights: around both, with a sequence
+    that has keys in the first parts only and one without any."""
+    torch.manual_seed(dh + parts)
+    blocks = parts * 4
+    assert ops.ext().paged_decode_parts(parts, blocks * 16, dh, 1, False) == parts
+    lens = torch.tensor([blocks * 16, blocks * 16 - 61, 3, 0])
+    kc, vc = ops.alloc_kv_cache(4 * blocks, 3, dh, DEV, dtype=torch.bfloat16)
+    kc.normal_()
+    vc.normal_()
+    q = 2 * torch.randn(4, 3, dh, device=DEV).bfloat16()
+    i32 = dict(dtype=torch.int32, device=DEV)
+    tables = torch.arange(4 * blocks, **i32).view(4, blocks)
+    got = ops.ext().paged_decode_swz(q, kc, vc, tables, lens.to(**i32), parts,
+                                     dh ** -0.5, None)[0]
+    ref = ops.paged_decode_ref(q[:3].cpu(), kc.cpu(), vc.cpu(), tables[:3].cpu(),
+                               lens[:3], dh ** -0.5)
+    assert _rel(got[:3].cpu(), ref.double()) < 2 * BF16
+    assert not bool(got[3].any())
+
+
 @pytest.mark.parametrize("batch,hq,hkv,dh,blocks,nsplit", [
     (3, 4, 4, 128, 9, 1), (2, 8, 4, 128, 33, 3), (3, 4, 4, 64, 9, 1),
     (3, 2, 2, 256, 40, 2), (17, 32, 32, 128, 33, 1)])

@@ -359,6 +359,13 @@ __global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
 // rows by the tiles of x (3.8 TB/s). W two chunks ahead and a chunk's operands
 // of x read at once: 22016 x 4096 of 45 rows 40.6 -> 34.0 us, 4096 x 4096 15.0 ->
 // 13.5 (library 43 and 23).
+// Of the ends, which took 1.3 to 3 us behind the stream where one group's wave had
+// them all, every group takes a share, with its angles loaded ahead of the sums; a
+// wave that shares its tile with no other waits for none. 12288 x 4096 and rotation of
+// 32, 45 and 64 rows 21.8 -> 21.1, 24.5 -> 23.4, 26.4 -> 25.4 us, 6144 x 4096 of 45
+// 19.1 -> 17.6, 3072 x 1024 of 64 10.0 -> 8.6. W four chunks ahead in place of two
+// changes nothing: with 64 rows a CU's loads of x, all of which every workgroup needs,
+// are the bound.
 template <int RB, int NWN, int CH, Kind KIND>
 __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
     const uint16_t *__restrict__ x, const uint8_t *__restrict__ ws, int M,
@@ -366,8 +373,8 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
   constexpr int KG = 4 / NWN, P = 2 * CH;          // pieces of a row
   constexpr int XL = RB * CH / NWN;                // of x, a lane and chunk
   constexpr int TILE = RB * 32 * P * 16;
-  static_assert(XL * NWN == RB * CH &&
-                2 * KG * TILE >= (KG - 1) * NWN * RB * 4096, "tiles");
+  static_assert(XL * NWN == RB * CH && (KG == 1 || 2 * KG * TILE >= RB * 16384),
+                "tiles");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, hi = lane >> 5, col = lane & 31;
@@ -388,6 +395,24 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
   if constexpr (NORM)
 #pragma unroll
     for (int b = 0; b < RB; ++b) early[b].begin(e, M, b * 32);
+  // A sum's 8 registers 4 q .. 4 q + 3 and 8 more, of RB blocks of rows: shares of the
+  // groups by turns, which end them side by side
+  constexpr int SHARES = RB * 2, OWN = (SHARES + KG - 1) / KG;
+  constexpr bool HEADS = KIND == ends::QKV;
+  ends::Turn<4> turn[HEADS ? OWN : 1];
+  int position[HEADS ? OWN : 1];
+  auto row_of = [&](int i) { return min((kg + i * KG) / 2 * 32 + col, M - 1); };
+  auto turns = [&] {
+    if constexpr (HEADS)
+#pragma unroll
+      for (int i = 0; i < OWN; ++i)
+        turn[i].load(e, row_of(i),
+                     min(nblk, blocks - 1) * 16 + 8 * ((kg + i * KG) & 1) + 4 * hi,
+                     position[i]);
+  };
+  if constexpr (HEADS)
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) position[i] = e.pos[row_of(i)];
 
   struct X { u32x4v v[XL]; };
   struct W { u32x4v v[CH]; };
@@ -417,10 +442,14 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
     for (int i = 0; i < XL; ++i)
       *reinterpret_cast<u32x4v *>(tile + xput[i]) = d.v[i];
   };
-  auto meet = [] {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  auto meet = [] {                                 // those that share a tile
+    if constexpr (NWN > 1) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    }
   };
   f32x16v acc[RB];
 #pragma unroll
@@ -456,6 +485,8 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
       if (threadIdx.x % 8 == 0) norms[b * 32 + threadIdx.x / 8] = early[b].norm;
     }
   }
+  constexpr bool AHEAD = OWN <= 2;                 // more have no registers for it
+  if constexpr (AHEAD) turns();
   meet();
   // chunk c, of which `w` holds W and then W of chunk c + 2; `xr` holds x of chunk
   // c + 1 and then of chunk c + 1 + FAR
@@ -491,80 +522,78 @@ __global__ __launch_bounds__(BLOCK, 2) void decode_gemm_rows_kernel(
     step(w0, FAR == 2 ? x1 : x0, c, std::false_type{});
     step(w1, x0, c + 1, std::false_type{});
   }
-  // sum of the groups
+  if constexpr (!AHEAD) turns();
+  if constexpr (NWN == 1) __syncthreads();         // every wave's tiles, norms
+  // sum of the groups: what is another's share goes to LDS
+  float *red = reinterpret_cast<float *>(smem) + wn * SHARES * KG * 512 + lane * 4;
   if constexpr (KG > 1) {
-    float *red = reinterpret_cast<float *>(smem) + wn * RB * 1024 + lane;
-    if (kg > 0) {
 #pragma unroll
-      for (int b = 0; b < RB; ++b)
+    for (int i = 0; i < SHARES; ++i)
+      if (i % KG != kg)
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-          red[((kg - 1) * NWN * RB + b) * 1024 + r * 64] = acc[b][r];
-    }
+        for (int h = 0; h < 2; ++h) {
+          const int r = h * 8 + i % 2 * 4;
+          *reinterpret_cast<float4 *>(red + (i * KG + kg) * 512 + h * 256) =
+              make_float4(acc[i / 2][r], acc[i / 2][r + 1], acc[i / 2][r + 2],
+                          acc[i / 2][r + 3]);
+        }
     __syncthreads();
-    if (kg > 0) return;
-#pragma unroll
-    for (int g = 0; g < KG - 1; ++g)
-#pragma unroll
-      for (int b = 0; b < RB; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          acc[b][r] += red[(g * NWN * RB + b) * 1024 + r * 64];
   }
   if (nblk >= blocks) return;
-  if constexpr (NORM) {
 #pragma unroll
-    for (int b = 0; b < RB; ++b)
+  for (int i = 0; i < SHARES; ++i) {
+    if (i % KG != kg) continue;
+    const int b = i / 2, q = i % 2, m = b * 32 + col;
+    float f[2][4];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[b][r] *= norms[b * 32 + col];
-  }
-  if constexpr (KIND == ends::GLU || KIND == ends::QKV) {
-    // registers r and r + 8 of a lane are a pair, 4 neighbours at a time
-    constexpr bool HEADS = KIND == ends::QKV;
-    ends::Turn<4> turn[HEADS ? RB : 1][2];
-    if constexpr (HEADS) {
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int b = 0; b < RB; ++b) {
-        const int m = min(b * 32 + col, M - 1), position = e.pos[m];
+      for (int j = 0; j < 4; ++j) f[h][j] = acc[b][h * 8 + q * 4 + j];
+    if constexpr (KG > 1) {
+      float4 other[2][KG];
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
-          turn[b][q].load(e, m, nblk * 16 + 8 * q + 4 * hi, position);
-      }
-    }
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int b = 0; b < RB; ++b) {
-      const int m = b * 32 + col;
-      if (m >= M) continue;
+        for (int g = 0; g < KG; ++g)
+          other[h][g] = g == i % KG
+              ? make_float4(f[h][0], f[h][1], f[h][2], f[h][3])
+              : *reinterpret_cast<float4 *>(red + (i * KG + g) * 512 + h * 256);
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int p = nblk * 16 + 8 * q + 4 * hi;
-        float f[4], g[4];
+      for (int h = 0; h < 2; ++h) {
+        float4 sum = other[h][0];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          f[j] = acc[b][4 * q + j];
-          g[j] = acc[b][8 + 4 * q + j];
+        for (int g = 1; g < KG; ++g) {
+          sum.x += other[h][g].x; sum.y += other[h][g].y;
+          sum.z += other[h][g].z; sum.w += other[h][g].w;
         }
-        if constexpr (HEADS) ends::put_heads<4>(e, turn[b][q], m, p, N, f, g);
-        else ends::put_gated<4>(e, m, p, N, f, g);
+        f[h][0] = sum.x; f[h][1] = sum.y; f[h][2] = sum.z; f[h][3] = sum.w;
       }
     }
-    return;
-  }
+    if constexpr (NORM) {
+      const float norm = norms[m];
 #pragma unroll
-  for (int b = 0; b < RB; ++b) {
-    const int m = b * 32 + col;
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) f[h][j] *= norm;
+    }
     if (m >= M) continue;
+    // registers r and r + 8 of a lane are a pair, 4 neighbours at a time
+    const int p = nblk * 16 + 8 * q + 4 * hi;
+    if constexpr (HEADS) {
+      ends::put_heads<4>(e, turn[i / KG], m, p, N, f[0], f[1]);
+    } else if constexpr (KIND == ends::GLU) {
+      ends::put_gated<4>(e, m, p, N, f[0], f[1]);
+    } else {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int n = ends::column(e.half, nblk, 8 * q + 4 * hi);
-      const float f[4] = {acc[b][4 * q], acc[b][4 * q + 1], acc[b][4 * q + 2],
-                          acc[b][4 * q + 3]};
-      if constexpr (KIND == ends::PLAIN)
-        ends::put<4>(e.y + (int64_t)m * N + n, f);
-      else
-        *reinterpret_cast<float4 *>(
-            e.slabs + ((int64_t)blockIdx.y * M + m) * N + n) =
-            make_float4(f[0], f[1], f[2], f[3]);
+      for (int h = 0; h < 2; ++h) {
+        const int n = ends::column(e.half, nblk, 16 * h + 8 * q + 4 * hi);
+        if constexpr (KIND == ends::PLAIN)
+          ends::put<4>(e.y + (int64_t)m * N + n, f[h]);
+        else
+          *reinterpret_cast<float4 *>(
+              e.slabs + ((int64_t)blockIdx.y * M + m) * N + n) =
+              make_float4(f[h][0], f[h][1], f[h][2], f[h][3]);
+      }
     }
   }
 }

@@ -100,17 +100,17 @@ def _heads(layer, y, m, cos, sin, positions, kc, vc, slots):
             out = ops.wide_linear(y.rows, layer.attn._qkv_w)
         return ext.qkv_rope_append(out, cos, sin, positions.to(torch.int32),
                                    kc, vc, slots.to(torch.int32), hq)
-    if y.squares is None and c.shares_x(m):
+    if y.swz is None or (y.squares is None and c.shares_x(m)):
         return ext.rows_heads(y.rows, c.ws, c.n, cos, sin, positions, kc, vc,
-                              slots, hq)
+                              slots, hq, False, y.squares, y.eps)
     return ext.decode_heads(y.swz, c.ws, c.scale, m, c.n, c.k, y.squares, y.eps,
                             cos, sin, positions, kc, vc, slots, hq)
 
 
-def _gated(layer, y, m):
+def _gated(layer, y, m, operand: bool):
     ext, c = ops.ext(), layer.gate_up
     if y.rows is not None and c.shares_x(m):
-        return ext.rows_glu(y.rows, c.ws, c.n, layer.gelu, True, y.squares,
+        return ext.rows_glu(y.rows, c.ws, c.n, layer.gelu, operand, y.squares,
                             y.eps)
     return ext.decode_glu(y.swz, c.ws, c.scale, m, c.n, c.k, layer.gelu,
                           y.squares, y.eps)
@@ -123,7 +123,7 @@ def _add(x, operand, copy, norm, rows: bool):
     # which is what it takes with many long rows (us in parts and whole, with
     # the norm: 32 rows, 4096 x 4096 13.8 and 10.1, 4096 x 11008 23.8 and 24.0,
     # 4096 x 14336 27.1 and 29.6, 3072 x 24576 39.7 and 45.7; 16 rows 13.2 and
-    # 8.4, 22.0 and 20.5, 25.4 and 24.2, 34.2 and 33.7)
+    # 8.4, 22.0 and 20.5, 25.4 and 24.2, 34.2 and 33.7); most of those are _long_rows'
     if (m <= 16 or copy.k <= 8192) and \
             ext.decode_res_supported(m, copy.n, copy.k, copy.fp8):
         x, y, squares = ext.decode_res(operand, copy.ws, copy.scale, x,
@@ -135,6 +135,24 @@ def _add(x, operand, copy, norm, rows: bool):
            ext.rmsnorm_res_fwd_dec)
     x, rows_, swz = add(x, delta, norm.weight, norm.eps)
     return x, _Normed(swz, rows_)
+
+
+def _long_rows(layer, after, m: int, kc) -> bool:
+    """Whether the long sums of the down projection of 17 to 32 rows go as 33 to 64
+    do, in parts by the kernel whose waves share x and with a launch that adds them up
+    (_add_rows); then the gated unit and q, k and v of the layer behind them, which
+    reads keys `kc`, take rows. us in parts of the kernel for operands with the norm,
+    and so, weights out of cache, 17 and 32 rows: 2048 x 8208 23.0 and 11.8, 24.8 and
+    12.3; 4096 x 14336 of 32 28.4 and 23.7; 5120 x 13824 38.6 and 31.2, 42.2 and 32.2;
+    1024 x 16384 13.3 and 11.7, 14.0 and 12.6. A step of 32 sequences of llama2-7b
+    5958 -> 5701."""
+    down, heads, norm = layer.down, after.qkv, after.blk.norm1.weight
+    return (m > 16 and down.k > 8192 and down.half == 0 and
+            layer.gate_up.shares_x(m) and not (down.fp8 or heads.fp8) and
+            heads.k >= 1024 and kc.dtype == torch.bfloat16 and
+            norm.data_ptr() % 16 == 0 and
+            ops.ext().parts_res_supported(down.n) and
+            ops.ext().rows_ends_pay(m, heads.n, heads.k))
 
 
 def run(model, layers, x, positions, caches, slots, tables, seq_lens, nsplit,
@@ -153,9 +171,14 @@ def run(model, layers, x, positions, caches, slots, tables, seq_lens, nsplit,
             q, kc, vc, tables, seq_lens, scale=attn.scale, nsplit=nsplit,
             seq_starts=seq_starts)
         x, y = _add(x, o, layer.o, blk.norm2, layer.gate_up.shares_x(m))
-        h = _gated(layer, y, m)
-        if i + 1 < len(layers):
-            x, y = _add(x, h, layer.down, layers[i + 1].blk.norm1, False)
+        after = layers[i + 1] if i + 1 < len(layers) else None
+        rows = after is not None and _long_rows(layer, after, m,
+                                                caches[i + 1][0])
+        h = _gated(layer, y, m, not rows)
+        if rows:
+            x, y = _add_rows(x, h, layer.down, after.blk.norm1)
+        elif after is not None:
+            x, y = _add(x, h, layer.down, after.blk.norm1, False)
     return x, layers[-1].down.product(h, m)
 
 

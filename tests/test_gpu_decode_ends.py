@@ -268,6 +268,29 @@ def test_decode_step(monkeypatch, batch, kv, inter, hidden, eight_bit):
     assert _rel(got, ref.double()) < 2e-2
 
 
+@pytest.mark.parametrize("batch", [16, 17, 32])
+@pytest.mark.parametrize("kv,inter,fp8", [
+    (8, 8208, False), (2, 16384, False), (8, 8192, False), (8, 8208, True)])
+def test_long_rows_step(monkeypatch, batch, kv, inter, fp8):
+    """As test_decode_step, with down projections from where on 17 to 32 rows take
+    parts of their sums and rows; not one short of it, nor ahead of 8-bit caches."""
+    from runbooks_amd.models import decode_chain
+    m = _model(kv, inter)
+    args = _step(m, batch, fp8)
+    seen, plain = [], ops.ext().parts_res
+
+    def parts_res(*a):
+        seen.append(1)
+        return plain(*a)
+    with torch.no_grad():
+        monkeypatch.setattr(ops.ext(), "parts_res", parts_res)
+        got = m.decode(*args)
+        assert len(seen) == (batch > 16 and inter > 8192 and not fp8)
+        monkeypatch.setattr(decode_chain, "layers_of", lambda *a: None)
+        ref = m.decode(*args)
+    assert _rel(got, ref.double()) < 2e-2
+
+
 def test_hooked_modules_are_called():
     m = _model(8, 2048)
     args = _step(m, 3, False)

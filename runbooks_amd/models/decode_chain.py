@@ -109,11 +109,11 @@ def _heads(layer, y, m, cos, sin, positions, kc, vc, slots):
 
 def _gated(layer, y, m, operand: bool):
     ext, c = ops.ext(), layer.gate_up
-    if y.rows is not None and c.shares_x(m):
+    if y.rows is not None and (y.swz is None or c.shares_x(m)):
         return ext.rows_glu(y.rows, c.ws, c.n, layer.gelu, operand, y.squares,
                             y.eps)
     return ext.decode_glu(y.swz, c.ws, c.scale, m, c.n, c.k, layer.gelu,
-                          y.squares, y.eps)
+                          y.squares, y.eps, not operand)
 
 
 def _add(x, operand, copy, norm, rows: bool):
@@ -123,7 +123,7 @@ def _add(x, operand, copy, norm, rows: bool):
     # which is what it takes with many long rows (us in parts and whole, with
     # the norm: 32 rows, 4096 x 4096 13.8 and 10.1, 4096 x 11008 23.8 and 24.0,
     # 4096 x 14336 27.1 and 29.6, 3072 x 24576 39.7 and 45.7; 16 rows 13.2 and
-    # 8.4, 22.0 and 20.5, 25.4 and 24.2, 34.2 and 33.7); most of those are _long_rows'
+    # 8.4, 22.0 and 20.5, 25.4 and 24.2, 34.2 and 33.7); long ones are _in_parts'
     if (m <= 16 or copy.k <= 8192) and \
             ext.decode_res_supported(m, copy.n, copy.k, copy.fp8):
         x, y, squares = ext.decode_res(operand, copy.ws, copy.scale, x,
@@ -137,22 +137,39 @@ def _add(x, operand, copy, norm, rows: bool):
     return x, _Normed(swz, rows_)
 
 
-def _long_rows(layer, after, m: int, kc) -> bool:
-    """Whether the long sums of the down projection of 17 to 32 rows go as 33 to 64
-    do, in parts by the kernel whose waves share x and with a launch that adds them up
-    (_add_rows); then the gated unit and q, k and v of the layer behind them, which
-    reads keys `kc`, take rows. us in parts of the kernel for operands with the norm,
-    and so, weights out of cache, 17 and 32 rows: 2048 x 8208 23.0 and 11.8, 24.8 and
-    12.3; 4096 x 14336 of 32 28.4 and 23.7; 5120 x 13824 38.6 and 31.2, 42.2 and 32.2;
-    1024 x 16384 13.3 and 11.7, 14.0 and 12.6. A step of 32 sequences of llama2-7b
-    5958 -> 5701."""
-    down, heads, norm = layer.down, after.qkv, after.blk.norm1.weight
-    return (m > 16 and down.k > 8192 and down.half == 0 and
-            layer.gate_up.shares_x(m) and not (down.fp8 or heads.fp8) and
-            heads.k >= 1024 and kc.dtype == torch.bfloat16 and
-            norm.data_ptr() % 16 == 0 and
-            ops.ext().parts_res_supported(down.n) and
-            ops.ext().rows_ends_pay(m, heads.n, heads.k))
+def _in_parts(copy, m: int) -> bool:
+    """Whether the sums of up to 32 rows that get the residual go as those of 33 to 64
+    do: in parts by the kernel whose waves share x, and a launch that adds them up
+    (_add_rows). us of the product and the norm by operands in parts, so, and in whole
+    sums, weights out of cache, of 1, 16, 17 and 32 rows:
+      3072 x 24576  33.6 27.8 30.8  34.3 27.5 32.8  35.3 27.6 38.6  38.7 29.4 45.0
+      4096 x 11008  20.2 18.6 18.6  21.3 18.4 19.4  21.8 18.4 20.7  23.7 19.9 23.8
+      4096 x 8192   19.2 16.4 13.6  20.0 16.6 13.9  20.0 16.7 15.8  20.3 17.1 17.9
+      5120 x 5120   16.7 13.0       18.2 14.0       19.6 14.1       21.6 15.6
+      5120 x 13824  33.5 28.7       35.8 31.1       37.6 29.0       42.0 32.1
+    Of up to 16 rows what the products around it lose by rows (0 to 0.7 us) is more
+    than 4096 x 11008 gains."""
+    ext = ops.ext()
+    return (not copy.fp8 and copy.half == 0 and copy.n <= 8192 and
+            ext.parts_res_supported(copy.n) and copy.k >= 1024 and
+            (copy.k > (16384 if m <= 16 else 8192) or
+             not ext.decode_res_supported(m, copy.n, copy.k, False)))
+
+
+def _heads_by_rows(layer, m: int, kc) -> bool:
+    c = layer.qkv
+    return (not c.fp8 and c.k >= 1024 and kc.dtype == torch.bfloat16 and
+            layer.blk.norm1.weight.data_ptr() % 16 == 0 and
+            ops.ext().rows_ends_pay(m, c.n, c.k))
+
+
+def _gate_by_rows(layer, m: int) -> bool:
+    """us by operands and by rows, of 1, 8 and 16 rows: 27648 x 5120 48.0 44.1, 45.8
+    43.8, 46.3 44.3; 28672 x 4096 40.1 41.1, 39.2 38.9, 39.4 39.6; 49152 x 3072 47.0
+    52.4, 45.1 50.9, 44.6 51.5."""
+    c = layer.gate_up
+    return (not c.fp8 and c.k >= 1024 and 10240 <= c.n <= 32768 and
+            layer.blk.norm2.weight.data_ptr() % 16 == 0)
 
 
 def run(model, layers, x, positions, caches, slots, tables, seq_lens, nsplit,
@@ -167,13 +184,17 @@ def run(model, layers, x, positions, caches, slots, tables, seq_lens, nsplit,
     for i, (layer, (kc, vc)) in enumerate(zip(layers, caches)):
         blk, attn = layer.blk, layer.attn
         q = _heads(layer, y, m, cos, sin, positions, kc, vc, slots)
-        _, o = ops.paged_decode_with_operand(
+        o, operand = ops.paged_decode_with_operand(
             q, kc, vc, tables, seq_lens, scale=attn.scale, nsplit=nsplit,
             seq_starts=seq_starts)
-        x, y = _add(x, o, layer.o, blk.norm2, layer.gate_up.shares_x(m))
+        if _in_parts(layer.o, m) and _gate_by_rows(layer, m):
+            x, y = _add_rows(x, o.view(m, -1), layer.o, blk.norm2)
+        else:
+            x, y = _add(x, operand, layer.o, blk.norm2,
+                        layer.gate_up.shares_x(m))
         after = layers[i + 1] if i + 1 < len(layers) else None
-        rows = after is not None and _long_rows(layer, after, m,
-                                                caches[i + 1][0])
+        rows = (after is not None and _in_parts(layer.down, m) and
+                _heads_by_rows(after, m, caches[i + 1][0]))
         h = _gated(layer, y, m, not rows)
         if rows:
             x, y = _add_rows(x, h, layer.down, after.blk.norm1)

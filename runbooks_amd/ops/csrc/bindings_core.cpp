@@ -21,7 +21,7 @@ std::vector<at::Tensor> swiglu_packed_dec(at::Tensor y);
 std::vector<at::Tensor> geglu_packed_dec(at::Tensor y);
 at::Tensor decode_gemm_raw(at::Tensor xs, at::Tensor ws, int64_t M, int64_t N, int64_t K, bool f32, int64_t half);
 at::Tensor decode_gemm(at::Tensor xs, at::Tensor ws, int64_t M, int64_t N, int64_t K, int64_t force_split, int64_t half);
-at::Tensor decode_glu(at::Tensor xs, at::Tensor ws, c10::optional<at::Tensor> scale, int64_t M, int64_t N, int64_t K, bool gelu, c10::optional<at::Tensor> squares, double eps);
+at::Tensor decode_glu(at::Tensor xs, at::Tensor ws, c10::optional<at::Tensor> scale, int64_t M, int64_t N, int64_t K, bool gelu, c10::optional<at::Tensor> squares, double eps, bool rows);
 at::Tensor decode_heads(at::Tensor xs, at::Tensor ws, c10::optional<at::Tensor> scale, int64_t M, int64_t N, int64_t K, c10::optional<at::Tensor> squares, double eps, at::Tensor cos, at::Tensor sin, at::Tensor positions, at::Tensor k_cache, at::Tensor v_cache, at::Tensor slots, int64_t hq);
 at::Tensor decode_normed(at::Tensor xs, at::Tensor ws, c10::optional<at::Tensor> scale, int64_t M, int64_t N, int64_t K, at::Tensor squares, double eps, int64_t half);
 bool rows_ends_pay(int64_t M, int64_t N, int64_t K);
@@ -119,10 +119,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("xs"), py::arg("ws"), py::arg("M"), py::arg("N"),
         py::arg("K"), py::arg("force_split") = -1, py::arg("half") = 0);
   m.def("decode_glu", &decode_glu,
-        "gated unit of a decode product, as the next one's operand",
+        "gated unit of a decode product, as the next one's operand or rows",
         py::arg("xs"), py::arg("ws"), py::arg("scale"), py::arg("M"),
         py::arg("N"), py::arg("K"), py::arg("gelu"),
-        py::arg("squares") = py::none(), py::arg("eps") = 0.0);
+        py::arg("squares") = py::none(), py::arg("eps") = 0.0,
+        py::arg("rows") = false);
   m.def("decode_heads", &decode_heads,
         "decode product of q, k and v -> rotated q, keys and values cached",
         py::arg("xs"), py::arg("ws"), py::arg("scale"), py::arg("M"),

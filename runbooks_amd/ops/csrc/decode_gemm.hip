@@ -939,15 +939,16 @@ static void launch_ends(Kind kind, const at::Tensor &xs, const at::Tensor &ws,
 at::Tensor decode_glu(at::Tensor xs, at::Tensor ws,
                       c10::optional<at::Tensor> scale, int64_t M, int64_t N,
                       int64_t K, bool gelu, c10::optional<at::Tensor> squares,
-                      double eps) {
+                      double eps, bool rows) {
   check_product(xs, ws, scale, M, N, K, N / 2);
   TORCH_CHECK(N > 0, "decode_glu: rows");
   Ends e{};
   e.half = (int)(N / 2);
   e.gelu = gelu;
   set_squares(e, squares, M, K, eps);
-  auto out = at::empty({N / 32 * 512}, xs.options());
-  e.operand = (uint16_t *)out.data_ptr();
+  auto out = rows ? at::empty({M, N / 2}, xs.options())
+                  : at::empty({N / 32 * 512}, xs.options());
+  (rows ? e.y : e.operand) = (uint16_t *)out.data_ptr();
   launch_ends(ends::GLU, xs, ws, scale, e, M, N, K);
   return out;
 }

@@ -268,14 +268,17 @@ def test_decode_step(monkeypatch, batch, kv, inter, hidden, eight_bit):
     assert _rel(got, ref.double()) < 2e-2
 
 
-@pytest.mark.parametrize("batch", [16, 17, 32])
-@pytest.mark.parametrize("kv,inter,fp8", [
-    (8, 8208, False), (2, 16384, False), (8, 8192, False), (8, 8208, True)])
-def test_long_rows_step(monkeypatch, batch, kv, inter, fp8):
-    """As test_decode_step, with down projections from where on 17 to 32 rows take
-    parts of their sums and rows; not one short of it, nor ahead of 8-bit caches."""
+@pytest.mark.parametrize("batch", [1, 16, 17, 32])
+@pytest.mark.parametrize("kv,inter,hidden,fp8,few,many", [
+    (8, 8192, 1024, False, 0, 0), (8, 8224, 1024, False, 0, 1),
+    (2, 16384, 1024, False, 0, 1), (8, 16400, 1024, False, 1, 1),
+    (8, 16400, 1024, True, 0, 0), (8, 5120, 4352, False, 3, 3)])
+def test_sums_in_parts(monkeypatch, batch, kv, inter, hidden, fp8, few, many):
+    """As test_decode_step, around the lengths from where on the sums of up to 16 and
+    of more rows go in parts (`few` and `many` of two layers' four, the last of which
+    is another kernel's), with wide residuals and ahead of 8-bit caches."""
     from runbooks_amd.models import decode_chain
-    m = _model(kv, inter)
+    m = _model(kv, inter, hidden)
     args = _step(m, batch, fp8)
     seen, plain = [], ops.ext().parts_res
 
@@ -285,7 +288,7 @@ def test_long_rows_step(monkeypatch, batch, kv, inter, fp8):
     with torch.no_grad():
         monkeypatch.setattr(ops.ext(), "parts_res", parts_res)
         got = m.decode(*args)
-        assert len(seen) == (batch > 16 and inter > 8192 and not fp8)
+        assert len(seen) == (few if batch <= 16 else many)
         monkeypatch.setattr(decode_chain, "layers_of", lambda *a: None)
         ref = m.decode(*args)
     assert _rel(got, ref.double()) < 2e-2

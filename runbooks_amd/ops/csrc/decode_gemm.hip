@@ -1020,10 +1020,16 @@ static void launch_rows(Kind kind, const at::Tensor &x, const at::Tensor &ws,
 // four for long rows, of which splits to fill the CUs cost less (us with two
 // and four at their best split: 4096 x 11008 of 64 rows 25 and 26, of 100 rows
 // 32 and 30; 3072 x 24576 38 and 34, 50 and 41; 4096 x 4096 14 and 16, 17 and
-// 20; 22016 x 4096 of 64 rows 45 and 36, 12288 x 4096 25 and 26).
+// 20; 22016 x 4096 of 64 rows 45 and 36, 12288 x 4096 25 and 26). Where four blocks
+// have up to half of the CUs take a second workgroup and the others none, two are
+// spread better, except that with more rows what x takes of a CU grows (four and two:
+// 36864 x 2048 of 17, 45 and 64 rows 35.4 and 30.5, 39.1 and 34.8, 40.6 and 37.2, of
+// 100 the same; 49152 x 3072 52.4 and 48.0, 56.7 and 52.9, 59.0 and 58.9, 67 and 72;
+// 65536 x 4096, two workgroups on every CU, 87 and 90, 88 and 96).
 struct Cut { int blocks, split; };
 static Cut cut_of(int64_t M, int64_t N, int64_t K) {
-  Cut c{N >= 20480 || K >= (M <= 64 ? 20480 : 8192) ? 4 : 2, 1};
+  const bool spill = M <= 64 && N > 32768 && N <= 49152;
+  Cut c{(N >= 20480 && !spill) || K >= (M <= 64 ? 20480 : 8192) ? 4 : 2, 1};
   const int64_t wgs = (N / 32 + c.blocks - 1) / c.blocks;
   while (c.split < 8 && wgs * c.split * 2 <= 256 && K / (c.split * 2) >= 256)
     c.split *= 2;

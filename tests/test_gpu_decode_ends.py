@@ -103,6 +103,13 @@ def test_gated_unit_of_rows(m, inter, k):
     assert _rel(ops.ext().rows_glu(x, ws, 2 * inter, False), ref) < BF16
 
 
+@pytest.mark.parametrize("m", [17, 64, 65])
+@pytest.mark.parametrize("inter", [16384, 16400, 24576, 24592])
+def test_wide_gated_unit_of_rows(m, inter):
+    """Around the widths from where on a workgroup has two blocks of W and not four."""
+    test_gated_unit_of_rows(m, inter, 1024)
+
+
 def _heads_case(m, hq, hkv, dh, vt):
     n, k = (hq + 2 * hkv) * dh, 1056
     cos, sin = ops.rope_tables(dh, 50, device=DEV)

@@ -804,20 +804,19 @@ __global__ __launch_bounds__(WAVES * 64, DH == 256 ? 2 : 4) void paged_decode8_k
   }
 }
 
-// Second pass for SPLIT mode: a wave merges the nsplit partials of one (b, hq)
+// Second pass for SPLIT mode: a workgroup of a wave merges the nsplit partials of one (b, hq)
 // row. Maxima and sums are one load of the wave (a lane a partial), and the rows (VE =
 // dh / 64 values a lane) are loaded 16 at a time beside it: one round trip to memory up
 // to 16 splits, where rows behind their weights made two (both kernels, one sequence of
 // 701 tokens, 32 heads, 12 splits: 10.2 us, 8.6 so) and loops over the splits three per
 // split.
 template <int VE>
-__global__ __launch_bounds__(256) void decode_combine_kernel(
+__global__ __launch_bounds__(64) void decode_combine_kernel(
     const float *__restrict__ partial, uint16_t *__restrict__ out,
-    uint16_t *__restrict__ out_swz, int rows, int Hq, int nsplit) {
+    uint16_t *__restrict__ out_swz, int Hq, int nsplit) {
   constexpr int DH = VE * 64, CHUNK = 16;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);  // b * Hq + hq
-  if (row >= rows) return;
-  const int lane = threadIdx.x & 63, d0 = lane * VE;
+  const int row = blockIdx.x;           // b * Hq + hq
+  const int lane = threadIdx.x, d0 = lane * VE;
   const float *p = partial + (int64_t)row * nsplit * (DH + 2);
   float x[CHUNK][VE];
   auto load = [&](int s0) {             // past the end: the last one again
@@ -859,16 +858,17 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(
   }
   rb::lane_sums<64>(ll);
   const float inv_l = (ll[0] > 0.f) ? 1.0f / ll[0] : 0.f;
-  const int b = row / Hq, h = row % Hq;
+  auto put = [&](uint16_t *at) {
+    if constexpr (VE == 1) *at = rb::f32_to_bf16(o[0] * inv_l);
 #pragma unroll
-  for (int e = 0; e < VE; ++e) {
-    const uint16_t ob = rb::f32_to_bf16(o[e] * inv_l);
-    out[(int64_t)row * DH + d0 + e] = ob;
-    if (out_swz != nullptr) {
-      const int kk = h * DH + d0 + e;
-      out_swz[(kk >> 4) * 512 + ((kk >> 3) & 1) * 256 + b * 8 +
-              (kk & 7)] = ob;
-    }
+    for (int e = 0; e + 1 < VE; e += 2)
+      *reinterpret_cast<uint32_t *>(at + e) =
+          rb::pack_bf16x2(o[e] * inv_l, o[e + 1] * inv_l);
+  };
+  put(out + (int64_t)row * DH + d0);
+  if (out_swz != nullptr) {
+    const int b = row / Hq, kk = row % Hq * DH + d0;
+    put(out_swz + (kk >> 4) * 512 + ((kk >> 3) & 1) * 256 + b * 8 + (kk & 7));
   }
 }
 
@@ -1232,9 +1232,9 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                            nullptr, nullptr, partial.data_ptr<float>(), hkv,
                            max_blocks, nsplit, scale, sorted);
         hipLaunchKernelGGL((decode_combine_kernel<DH / 64>),
-                           dim3((B * Hq + 3) / 4), dim3(256), 0, stream,
+                           dim3(B * Hq), dim3(64), 0, stream,
                            partial.data_ptr<float>(),
-                           (uint16_t *)out.data_ptr(), swz, B * Hq, Hq,
+                           (uint16_t *)out.data_ptr(), swz, Hq,
                            nsplit);
       }
       return;
@@ -1306,9 +1306,9 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
       else by_cache(std::false_type{}, Four{});
       if (splits > 1)
         hipLaunchKernelGGL((decode_combine_kernel<DH / 64>),
-                           dim3((B * Hq + 3) / 4), dim3(256), 0, stream,
+                           dim3(B * Hq), dim3(64), 0, stream,
                            partial.data_ptr<float>(),
-                           (uint16_t *)out.data_ptr(), swz, B * Hq, Hq, splits);
+                           (uint16_t *)out.data_ptr(), swz, Hq, splits);
       return;
     }
   }
@@ -1365,9 +1365,9 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
     go(paged_decode_kernel<DH, G, true, FP8>, NW, nsplit,
        partial.data_ptr<float>());
   hipLaunchKernelGGL((decode_combine_kernel<DH / 64>),
-                     dim3((B * Hq + 3) / 4), dim3(256), 0, stream,
+                     dim3(B * Hq), dim3(64), 0, stream,
                      partial.data_ptr<float>(), (uint16_t *)out.data_ptr(), swz,
-                     B * Hq, Hq, nsplit);
+                     Hq, nsplit);
 }
 
 }  // namespace

@@ -7,9 +7,10 @@
   * gate and up projection with the gated unit;
   * the down projection with the residual and the next norm's sums.
 
-A norm's 1 / rms is left to the product that reads its result. Where a step has
-no kernel of this kind (8-bit caches, wide residuals, long sums of many rows) it
-is the launches of Block.forward_decode_fused.
+A norm's 1 / rms is left to the product that reads its result. Long sums and wide
+residuals go in parts, with a launch that adds them up (_in_parts). Where a step has
+no kernel of either kind (8-bit caches and weights with such sums) it is the launches
+of Block.forward_decode_fused.
 
 33 to 64 rows, sequences or tokens of a prompt, go the same way with rows in place
 of operands (run_rows).

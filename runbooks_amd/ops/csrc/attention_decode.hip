@@ -808,7 +808,7 @@ __global__ __launch_bounds__(WAVES * 64, DH == 256 ? 2 : 4) void paged_decode8_k
 // row. Maxima and sums are one load of the wave (a lane a partial), and the rows (VE =
 // dh / 64 values a lane) are loaded 16 at a time beside it: one round trip to memory up
 // to 16 splits, where rows behind their weights made two (both kernels, one sequence of
-// 701 tokens, 32 heads, 12 splits: 10.2 us, 8.6 so) and loops over the splits three per
+// 701 tokens, 32 heads, 12 splits: 10.2 us, 8.6 so, 8.0 and loops over the splits three per
 // split.
 template <int VE>
 __global__ __launch_bounds__(64) void decode_combine_kernel(
@@ -1384,8 +1384,8 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
 // batch takes about as long. In place of more parts it does not, and an engine's
 // tables are wide whatever the lengths.
 //
-// us in parts and whole, with loads that stayed in L2, 32 heads of 128 in bf16: one
-// sequence of 200 tokens 9.1
+// us in parts and whole, with loads that stayed in L2 and a merge that took 2 us
+// longer than now, 32 heads of 128 in bf16: one sequence of 200 tokens 9.1
 // and 7.1, of 512 9.8 and 9.5, of 1024 12.0 and 16.2; 4 of 512 13.8 and 12.2, one of
 // 512 and 3 of 50 10.1 and 10.5, one of 1024 and 3 of 50 12.7 and 16.6; 16 (two
 // parts) of 800 to 3900 122 and 123, 4000 and 15 of 100 63.7 and 54.3; 8 (four) of

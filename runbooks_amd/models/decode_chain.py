@@ -108,9 +108,20 @@ def _heads(layer, y, m, cos, sin, positions, kc, vc, slots):
                             cos, sin, positions, kc, vc, slots, hq)
 
 
+def _gate_shares_x(c, m: int) -> bool:
+    """shares_x of a gated unit, which the kernel whose waves share x also wins where it
+    is wider, unless the sums are short or it is wider still (us by operands and by
+    rows, of 17, 24 and 32 rows: 36864 x 2048 28.2 30.5, 28.2 31.1, 30.1 31.8; 49152 x
+    3072 48.0 47.5, 48.1 48.1, 52.2 48.7; 57344 x 8192 145.7 139.4, 145.8 139.8, 157.7
+    141.1; 65536 x 4096 83.5 85.6, 83.7 84.6, 90.5 84.5). Results in rows take the kernel
+    for operands 0.5 to 7 us more."""
+    return c.shares_x(m) or (16 < m <= 32 and not c.fp8 and
+                             32768 < c.n <= 57344 and c.k >= 3072)
+
+
 def _gated(layer, y, m, operand: bool):
     ext, c = ops.ext(), layer.gate_up
-    if y.rows is not None and (y.swz is None or c.shares_x(m)):
+    if y.rows is not None and (y.swz is None or _gate_shares_x(c, m)):
         return ext.rows_glu(y.rows, c.ws, c.n, layer.gelu, operand, y.squares,
                             y.eps)
     return ext.decode_glu(y.swz, c.ws, c.scale, m, c.n, c.k, layer.gelu,
@@ -192,7 +203,7 @@ def run(model, layers, x, positions, caches, slots, tables, seq_lens, nsplit,
             x, y = _add_rows(x, o.view(m, -1), layer.o, blk.norm2)
         else:
             x, y = _add(x, operand, layer.o, blk.norm2,
-                        layer.gate_up.shares_x(m))
+                        _gate_shares_x(layer.gate_up, m))
         after = layers[i + 1] if i + 1 < len(layers) else None
         rows = (after is not None and _in_parts(layer.down, m) and
                 _heads_by_rows(after, m, caches[i + 1][0]))

@@ -52,17 +52,26 @@ using namespace flash;
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float RISE = 8.0f;           // of a maximum before it is moved
 
-// c += a b, c in the matrix registers: as text, for with more sums than there are
-// vector registers the compiler moves them back and forth in every step. FRESH: b has
-// just been computed.
-template <bool FRESH>
-RB_DEV void add_product(f32x16v &c, bf16x8v a, bf16x8v b) {
-  if constexpr (FRESH)
-    asm volatile("s_nop 3\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
-                 : "+a"(c) : "v"(a), "v"(b));
-  else
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
-                 : "+a"(c) : "v"(a), "v"(b));
+// c[i] += a[i] b, c in the matrix registers: as text, for with more sums than there are
+// vector registers the compiler moves them back and forth in every step. It does not see
+// these products, so what it would wait for ahead of one is in the text: a and b may
+// have just been computed, moved or put together (up to 4 wait states; behind the first
+// product nothing comes in between). Whoever else reads or writes c settles it first.
+//
+// Four at a time share the wait. us of 16 heads of 256 with products by themselves, a
+// wait in each (of four and of two states) and so: 7931 tokens 731, 704 and 632, 1021
+// 37.3, 35.7 and 33.3; and with a wait in the first of eight only, which what the
+// compiler puts ahead of the others would have broken, 688 and 36.2.
+constexpr int TEXT_PRODUCTS = 4;
+RB_DEV void add_products(f32x16v *c, const bf16x8v *a, bf16x8v b) {
+  asm volatile(
+      "s_nop 3\n\t"
+      "v_mfma_f32_32x32x16_bf16 %0, %4, %8, %0\n\t"
+      "v_mfma_f32_32x32x16_bf16 %1, %5, %8, %1\n\t"
+      "v_mfma_f32_32x32x16_bf16 %2, %6, %8, %2\n\t"
+      "v_mfma_f32_32x32x16_bf16 %3, %7, %8, %3"
+      : "+a"(c[0]), "+a"(c[1]), "+a"(c[2]), "+a"(c[3])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b));
 }
 
 RB_DEV void scale_sum(float &c, float by) {
@@ -149,21 +158,23 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
   float m_run = -INFINITY;                  // in exponents of 2 (ORDERED: of e)
   float l_run = 0.0f;
 
-  // Wide heads have more sums than there is room for among the vector registers. The
-  // last products that the compiler does not see are done where a step's scores are,
-  // behind them in the same unit; elsewhere this waits for them.
+  // Wide heads have more sums than there is room for among the vector registers. Where
+  // anything but a product reads or writes them, this is ahead of it and behind it, as
+  // the compiler waits for neither (20 wait states at most).
   constexpr bool TEXT = DH == 256;
   auto settle = [&] {
     if constexpr (TEXT)
-#pragma unroll
-      for (int dt = 0; dt < DTILES; ++dt)
-        asm volatile("s_nop 15" : "+a"(acc_o[dt]));
+      asm volatile("s_nop 15\n\ts_nop 15"
+                   : "+a"(acc_o[0]), "+a"(acc_o[1]), "+a"(acc_o[2]),
+                     "+a"(acc_o[3]), "+a"(acc_o[4]), "+a"(acc_o[5]),
+                     "+a"(acc_o[6]), "+a"(acc_o[7]));
   };
   settle();
 
   // Keys kbase .. kbase + 32 SUB - 1 of the tile, from row r0 on; `masked`:
   // some of them are hidden from some row
   constexpr int SUB = DH == 256 || SPLIT == 2 || ORDERED ? 1 : 2;
+  constexpr int AT_ONCE = TEXT ? TEXT_PRODUCTS : 1;
   auto keys = [&](const char *kt, const char *vt, int kbase, int r0,
                   auto masked) {
     f32x16v s[SUB];
@@ -229,6 +240,7 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
       const float alpha = __builtin_amdgcn_exp2f(
           m_run - (mn == -INFINITY ? 0.0f : mn));
       l_run *= alpha;
+      settle();
 #pragma unroll
       for (int dt = 0; dt < DTILES; ++dt)
 #pragma unroll
@@ -255,15 +267,16 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
       for (int ks = 0; ks < 2; ++ks) {
         const bf16x8v pf = score_frag(s[u], ks);
 #pragma unroll
-        for (int dt = 0; dt < DTILES; ++dt) {
-          const bf16x8v vf =
-              column_frag<DH>(vt, r0 + u * 32 + ks * 16, dt, lane);
+        for (int dt = 0; dt < DTILES; dt += AT_ONCE) {
+          bf16x8v vf[AT_ONCE];
+#pragma unroll
+          for (int j = 0; j < AT_ONCE; ++j)
+            vf[j] = column_frag<DH>(vt, r0 + u * 32 + ks * 16, dt + j, lane);
           if constexpr (TEXT)
-            dt == 0 ? add_product<true>(acc_o[dt], vf, pf)
-                    : add_product<false>(acc_o[dt], vf, pf);
+            add_products(&acc_o[dt], vf, pf);
           else
-            acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf, acc_o[dt],
-                                                                0, 0, 0);
+            acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                vf[0], pf, acc_o[dt], 0, 0, 0);
         }
       }
     }

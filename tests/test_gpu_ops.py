@@ -443,6 +443,35 @@ def test_flash_rising_scores(S, hq, dh):
         assert (out[0, :, h].double() - ref).norm() <= 2 ** -7 * ref.norm()
 
 
+@pytest.mark.parametrize("dh", [64, 128, 256])
+@pytest.mark.parametrize("S,hq", [(33, 1), (160, 4), (330, 4), (1313, 32)])
+def test_flash_rows_beside_one_that_jumps(S, hq, dh):
+    """One row of every 32 whose scores rise by 12 exponents of 2 with each 32 keys,
+    which moves the maxima of all of them, while the others rise by 0.5 to 3: their sums
+    so far are scaled by 0.125 to 0.7 each time, and stay part of the result."""
+    _assert_hip()
+    torch.manual_seed(dh)
+    steps = torch.arange(S, device=DEV) // 32
+    rise = (0.5 + 2.5 * torch.rand(int(steps[-1]) + 1, device=DEV)).cumsum(0)
+    q = 0.3 * torch.randn(1, S, hq, dh, device=DEV)
+    k = 0.3 * torch.randn(1, S, hq, dh, device=DEV)
+    jumps = torch.arange(S, device=DEV) % 32 == 9
+    q[..., 0], q[..., 1] = (~jumps)[None, :, None], jumps[None, :, None]
+    unit = math.log(2) * dh ** 0.5
+    k[..., 0] = (rise[steps] * unit)[None, :, None]
+    k[..., 1] = (12 * steps * unit)[None, :, None]
+    q, k = q.bfloat16(), k.bfloat16()
+    v = torch.randn(1, S, hq, dh, device=DEV).bfloat16()
+    out = ops.ext().flash_prefill(q, k, v, dh ** -0.5)
+    for h in range(0, hq, 7):
+        s = q[0, :, h].double() @ k[0, :, h].double().t() * dh ** -0.5
+        s = s.masked_fill(torch.ones(S, S, dtype=torch.bool, device=DEV).triu(1),
+                          -torch.inf)
+        ref = s.softmax(-1) @ v[0, :, h].double()
+        off = (out[0, :, h].double() - ref).norm(dim=-1)
+        assert bool((off <= 2 ** -6 * ref.norm(dim=-1)).all())
+
+
 @pytest.mark.parametrize("B,S,Hq,Hkv,bits", [
     (1, 1, 1, 1, (4093165637, 932004135, 3265854109, 3265854109, 34914089)),
     (2, 31, 3, 3, (2980831709, 3346004597, 2951792153, 627292471,

@@ -240,20 +240,26 @@ __global__ __launch_bounds__(NW * 64, DH == 256 ? 1 : 2) void flash_prefill_kern
       const float alpha = __builtin_amdgcn_exp2f(
           m_run - (mn == -INFINITY ? 0.0f : mn));
       l_run *= alpha;
-      settle();
+      // (TEXT: three instructions a sum, 0.9 us, where the others take one. The first
+      // time there is nothing to scale; us of 16 heads of 256, 33 tokens 9.6 and 8.6,
+      // 100 11.4 and 10.4, 250 15.3 and 14.1)
+      if (!TEXT || __any(m_run != -INFINITY)) {
+        settle();
 #pragma unroll
-      for (int dt = 0; dt < DTILES; ++dt)
+        for (int dt = 0; dt < DTILES; ++dt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          if constexpr (TEXT) {
-            float c = acc_o[dt][r];
-            scale_sum(c, alpha);
-            acc_o[dt][r] = c;
+          for (int r = 0; r < 16; ++r) {
+            if constexpr (TEXT) {
+              float c = acc_o[dt][r];
+              scale_sum(c, alpha);
+              acc_o[dt][r] = c;
+            } else {
+              acc_o[dt][r] *= alpha;
+            }
           }
-          else acc_o[dt][r] *= alpha;
-        }
+        settle();
+      }
       m_run = mn;
-      settle();
     }
     const float ref = m_run == -INFINITY ? 0.0f : m_run;
 #pragma unroll

@@ -1266,7 +1266,11 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                                         (FP8 ? DH + 16 : DH * 2) * 2 >
                                     ((int64_t)32 << 20);
   if constexpr (FP8 && G < NW) {
-    if (bs == 16) {
+    // (loads to LDS take addresses that are multiples of their 16 bytes; a cache that
+    // begins anywhere, or has other blocks, is read through registers)
+    const auto begin = reinterpret_cast<uintptr_t>(k_cache.data_ptr()) |
+                       reinterpret_cast<uintptr_t>(v_cache.data_ptr());
+    if (bs == 16 && begin % 16 == 0) {
       const int splits = std::max(nsplit, 1);
       at::Tensor partial;
       if (splits > 1)

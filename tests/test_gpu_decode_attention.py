@@ -115,6 +115,37 @@ def test_rows_of_nobody_8bit(batch, hq, hkv, dh, blocks, nsplit):
     assert torch.equal(*results)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("batch,hq,hkv,dh,blocks,nsplit", [
+    (3, 4, 4, 128, 9, 1), (2, 8, 4, 128, 33, 3), (3, 4, 4, 64, 9, 1),
+    (40, 32, 32, 64, 3, 1), (3, 2, 2, 256, 40, 2)])
+def test_caches_that_begin_anywhere(batch, hq, hkv, dh, blocks, nsplit, fp8):
+    """Parts of one buffer that no block begins on a multiple of 16 bytes of: the result
+    of the same caches by themselves."""
+    torch.manual_seed(dh)
+    tokens = blocks * 16
+    whole = ops.alloc_kv_cache(batch * blocks, hkv, dh, DEV, dtype=torch.bfloat16,
+                               fp8=fp8)
+    k, v = (torch.randn(batch * tokens, hkv, dh, device=DEV).bfloat16()
+            for _ in "kv")
+    i32 = dict(dtype=torch.int32, device=DEV)
+    ops.kv_append(k, v, *whole, torch.arange(batch * tokens, **i32))
+    beside = []
+    for cache, at in zip(whole, (4, 8)):
+        flat = torch.zeros(cache.numel() * cache.element_size() + 16,
+                           dtype=torch.uint8, device=DEV)[at:at - 16]
+        assert flat.data_ptr() % 16 == at
+        beside.append(flat.view(cache.dtype).view(cache.shape).copy_(cache))
+    q = torch.randn(batch, hq, dh, device=DEV).bfloat16()
+    tables = torch.randperm(batch * blocks, device=DEV).to(torch.int32) \
+        .view(batch, blocks)
+    lens = torch.randint(1, tokens + 1, (batch,)).to(**i32)
+    args = (tables, lens, nsplit, dh ** -0.5, None)
+    got = ops.ext().paged_decode_swz(q, *beside, *args)[0]
+    ref = ops.ext().paged_decode_swz(q, *whole, *args)[0]
+    assert _rel(got, ref.double()) < 2 * BF16
+
+
 @pytest.mark.parametrize("hq,hkv,nsplit", [(3, 3, 1), (5, 5, 3), (8, 2, 1),
                                            (8, 2, 2)])
 @pytest.mark.parametrize("batch", [2, 4, 5, 31, 64, 65])

@@ -518,17 +518,18 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
 // which are contiguous, go to LDS past the registers, and their rows of DH + 16 bytes
 // (values, scale) are read there. Loaded by rows, which begin and end within lines of
 // memory, scales apart, a line was asked for up to three times and could not pass L2.
-// A wave has a ring of its own and waits for no other; a lane group of eight takes a
-// row, 16 tokens a step. Keys are multiplied as bf16 pairs, which they are exactly.
+// A wave has a ring of its own and waits for no other, nor for more of its blocks than
+// the one it reads; a lane group of eight takes a row, 16 tokens a step. Keys are
+// multiplied as bf16 pairs, which they are exactly.
 //
-// Bound by memory. us by rows and so, 32 heads of 128: 16 sequences of 800 to 3900
-// tokens 68.5 and 60.6 (5.7 TB/s), 32 of 1000 58.9 and 53.9, 64 of 1000 110 and 99, 32
-// of 50 to 1000 34.1 and 31.9, of 100 11.6 and 11.0, 8 of 400 in four parts 15.1 and
-// 14.1, one of 700 10.7 and 9.8, of 50 4.8 and 4.3; 4000 and 15 of 100, where few CUs
-// have anything to do, 39.5 and 40.1. Two queries each: 32 of 50 to 1000 51 and 34.
-// Four workgroups of four waves fill a CU, as two of eight do (with the longer ring of
-// two, 32 of 100 took 14.4, 8 of 400 17.3). 16 heads of 256: 16 of 100 to 2000 in
-// four parts 42.6 and 38.7.
+// Bound by memory. us by rows and so, whole sequences, 32 heads of 128: 16 of 800 to
+// 3900 tokens 68.9 and 59.5 (5.8 TB/s), 32 of 1000 59.1 and 51.8, 64 of 1000 111 and
+// 96, 32 of 50 to 1000 34.0 and 30.3, of 100 11.7 and 10.3, of 20 6.9 and 6.9, one of 50
+// 4.8 and 4.3; where few CUs have anything to do, 4000 and 15 of 100 39.5 and 30.6, 4000
+// and 31 of 100 58.0 and 40.9 (40.1 and 69.7 where a step waited for every block that was
+// on its way). Two queries each: 32 of 50 to 1000 51 and 34. 12 heads of 64: 64 of 500
+// 17.5 and 15.6. Four workgroups of four waves fill a CU, as two of eight do; the longer
+// ring that two of four have room for is slower.
 template <int DH, int WAVES> struct Blocks8 {
   static constexpr int PART = (DH + 16) * 16, STAGE = 2 * PART;   // K, then V
   static constexpr int FULL = PART / 1024, LOADS = 2 * FULL + 1;
@@ -591,15 +592,26 @@ __global__ __launch_bounds__(WAVES * 64, DH == 256 ? 2 : 4) void paged_decode8_k
         qpk[g][(c + e) / 2 + 2] = w.z;
         qpk[g][(c + e) / 2 + 3] = w.w;
       }
+  // where the compiler sees it: otherwise it waits for these in the loop, and with them
+  // for the blocks that are on their way
+  __builtin_amdgcn_s_waitcnt(0x0f70);             // vmcnt(0)
   __syncthreads();
 
   const unsigned mine = wid * (R::AHEAD * R::STAGE);
   const unsigned ring =
       mine + (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem;
+  // a block's number, from LDS alone where it lies there: of a pointer to either place
+  // the load would wait for all blocks that are on their way
+  auto block_of = [&](int bi) {
+    int blk = bt_lds[min(bi - lo, BT_LDS - 1)];
+    if (bi - lo >= BT_LDS) {
+      blk = bt[bi];
+      asm volatile("" : "+v"(blk));
+    }
+    return __builtin_amdgcn_readfirstlane(blk);
+  };
   auto fetch = [&](int bi, int stage) {
-    const int blk = __builtin_amdgcn_readfirstlane(
-        bi - lo < BT_LDS ? bt_lds[bi - lo] : bt[bi]);
-    const int64_t at = ((int64_t)blk * hkv + h_kv) * R::PART;
+    const int64_t at = ((int64_t)block_of(bi) * hkv + h_kv) * R::PART;
     const uint8_t *k = k_cache + at, *v = v_cache + at;
     const unsigned to =
         __builtin_amdgcn_readfirstlane(ring + stage * R::STAGE);

@@ -1,6 +1,6 @@
-"""Matrix products that stand as text in a kernel (csrc/attention_prefill.hip, heads of
-256) are not seen by the compiler, which puts no wait states around them: looked for in
-what it made of this repository's source."""
+"""What the compiler made of this repository's kernels, where their source cannot say it
+all: waits around matrix products that stand as text, which it does not see, and loads
+that would wait for others to be done."""
 import re
 import shutil
 import subprocess
@@ -15,7 +15,7 @@ DUMP = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
 DONE = 20
 
 
-def _kernels(tmp_path):
+def _kernels(tmp_path, kernel):
     built = list(OPS.glob("_hip.cpython*.so"))
     if not built or not Path(DUMP).exists():
         pytest.skip("nothing built, or no llvm-objdump")
@@ -27,7 +27,9 @@ def _kernels(tmp_path):
         names = subprocess.run([DUMP, "-t", part], capture_output=True,
                                text=True).stdout
         for name in sorted(set(re.findall(
-                r"\S*flash_prefill_kernelILi256E\S*f(?=\n)", names))):
+                rf"\S*{kernel}\S*(?=\n)", names))):
+            if "." in name:
+                continue
             text = subprocess.run(
                 [DUMP, "-d", f"--disassemble-symbols={name}", part],
                 capture_output=True, text=True, check=True).stdout
@@ -47,7 +49,7 @@ def _sums(args):
 
 def test_products_as_text_wait(tmp_path):
     seen = 0
-    for code in _kernels(tmp_path):
+    for code in _kernels(tmp_path, "flash_prefill_kernelILi256E"):
         # four products behind a wait of four states
         inside, sums = set(), set()
         for i, (op, args) in enumerate(code):
@@ -69,3 +71,13 @@ def test_products_as_text_wait(tmp_path):
             since += int(args) + 1 if op == "s_nop" else 1
         seen += 1
     assert seen == 2                        # by whole and by half keys
+
+
+def test_blocks_of_8_bits_stay_on_their_way(tmp_path):
+    """A load from a pointer that may be one to LDS or to memory waits for all loads
+    ahead of it, and so for every block that the ring has asked for."""
+    seen = 0
+    for code in _kernels(tmp_path, "paged_decode8_kernel"):
+        assert not any(op.startswith("flat_load") for op, _ in code)
+        seen += 1
+    assert seen > 0

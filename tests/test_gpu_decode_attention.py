@@ -116,6 +116,32 @@ def test_rows_of_nobody_8bit(batch, hq, hkv, dh, blocks, nsplit):
 
 
 @pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hq,hkv,dh", [(2, 2, 64), (2, 2, 128), (4, 2, 128),
+                                       (1, 1, 256), (8, 2, 128)])
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_more_blocks_than_are_kept(hq, hkv, dh, nsplit, fp8):
+    """Sequences whose blocks' numbers lie in LDS (512 of a part), just not, and three
+    times as many: rows of a table that nothing else has."""
+    torch.manual_seed(dh)
+    lens = torch.tensor([512 * 16, 512 * 16 + 1, 1537 * 16, 40])
+    blocks, vt = 1537, hq // hkv >= 4
+    kc, vc = ops.alloc_kv_cache(4 * blocks, hkv, dh, DEV, dtype=torch.bfloat16,
+                                fp8=fp8, v_transposed=vt)
+    k, v = (torch.randn(4 * blocks * 16, hkv, dh, device=DEV).bfloat16()
+            for _ in "kv")
+    i32 = dict(dtype=torch.int32, device=DEV)
+    ops.kv_append(k, v, kc, vc, torch.arange(len(k), **i32))
+    tables = torch.randperm(4 * blocks, device=DEV).to(torch.int32).view(4, blocks)
+    q = torch.randn(4, hq, dh, device=DEV).bfloat16()
+    got = ops.ext().paged_decode_swz(q, kc, vc, tables, lens.to(**i32), nsplit,
+                                     dh ** -0.5, None)[0].cpu()
+    ref = ops.paged_decode_ref(q.cpu(), kc.cpu(), vc.cpu(), tables.cpu(), lens,
+                               dh ** -0.5)
+    for i in range(4):                  # 16-bit probabilities in matrix products
+        assert _rel(got[i], ref[i].double()) < (4 if vt else 2) * BF16
+
+
+@pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("batch,hq,hkv,dh,blocks,nsplit", [
     (3, 4, 4, 128, 9, 1), (2, 8, 4, 128, 33, 3), (3, 4, 4, 64, 9, 1),
     (40, 32, 32, 64, 3, 1), (3, 2, 2, 256, 40, 2)])

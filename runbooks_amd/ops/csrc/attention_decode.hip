@@ -147,21 +147,109 @@ RB_DEV Place sorted_place(const int32_t *lens, const int32_t *starts) {
           __builtin_amdgcn_readlane(start, b)};
 }
 
+// Blocks of sequence b, from the first one of its part on, that another sequence of the
+// batch reads too (a prefix that their requests share): those stay in L2 for the
+// others, while what one sequence reads goes past L2's older lines.
+//
+// For a workgroup that has own[i] = block lo + i of its part's `n` blocks on their way
+// to LDS. A wave asks for the other sequences' block lo ahead of these (Ask), and looks
+// at them behind these and ahead of the barrier that these need anyway (before). Only
+// where there is another one are the two rows compared (after).
+//
+// us of 32 sequences, 512 shared tokens and 100 of their own, all read past L2, none, and
+// so; 3600 and 100: 32 heads of 128 44.2, 31.4 and 28.6; 257, 142 and 120; in e4m3 27.5,
+// 23.9 and 20.2; 137, 105 and 78; 8 kv heads of 128 with four queries each 18.9, 15.4 and
+// 14.8; 74.6, 43.7 and 43.4; 16 heads of 256 42.0, 29.6 and 27.9; 238, 115 and 112. Where
+// nothing is shared it takes up to 0.5 us (32 of 100 tokens 13.4 and 13.9), so parts of
+// up to four blocks, whose loads are little, are not looked at.
+struct Shared {
+  int other, same;
+  RB_DEV static bool asked(int n) { return n > 4 && gridDim.x > 1; }
+  RB_DEV static bool first_wave() {
+    return __builtin_amdgcn_readfirstlane(threadIdx.x) < 64;
+  }
+  // of one wave: what it compares, asked for ahead of `own`
+  struct Ask {
+    int mine = 0, len = 0, block = 0;
+    RB_DEV Ask(const int32_t *tables, const int32_t *lens, int max_blocks, int b,
+               int lo, int n) {
+      if (!asked(n) || !first_wave()) return;
+      const int i = min((int)threadIdx.x & 63, (int)gridDim.x - 1);
+      mine = tables[(int64_t)b * max_blocks + lo];
+      len = lens[i];
+      block = tables[(int64_t)i * max_blocks + lo];
+    }
+  };
+  RB_DEV void before(const Ask &ask, const int32_t *tables, const int32_t *lens,
+                     int max_blocks, int bs, int b, int lo, int n) {
+    const int B = gridDim.x, lane = threadIdx.x & 63;
+    if (!asked(n) || !first_wave()) return;
+    int found = -1, len = ask.len, block = ask.block;
+    for (int i0 = 0;;) {
+      const unsigned long long those =
+          __ballot(i0 + lane < B && i0 + lane != b && len > lo * bs &&
+                   block == ask.mine);
+      if (those != 0) found = i0 + __builtin_ctzll(those);
+      i0 += 64;
+      if (found >= 0 || i0 >= B) break;
+      const int i = min(i0 + lane, B - 1);
+      len = lens[i];
+      block = tables[(int64_t)i * max_blocks + lo];
+    }
+    if (lane == 0) {
+      other = found;
+      same = n;
+    }
+  }
+  template <int THREADS>
+  RB_DEV int after(const int32_t *tables, const int32_t *lens, int max_blocks,
+                   int bs, int lo, int n, const int32_t *own) {
+    if (!asked(n)) return 0;
+    const int who = __builtin_amdgcn_readfirstlane(other);
+    if (who < 0) return 0;
+    const int32_t *at = tables + (int64_t)who * max_blocks + lo;
+    const int theirs = (lens[who] + bs - 1) / bs - lo;
+    for (int i = threadIdx.x; i < n; i += THREADS)
+      if (i >= theirs || at[i] != own[i]) {
+        atomicMin(&same, i);
+        break;
+      }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(same);
+  }
+};
+
+// load(true) or load(false), whose instructions differ in what they say to L2 alone:
+// taken for the same ones, they would become one that says nothing.
+template <typename Load> RB_DEV void by_policy(bool past, Load load) {
+  if (past) {
+    asm volatile("; past L2" ::: "memory");
+    load(std::true_type{});
+    asm volatile("; past L2" ::: "memory");
+  } else {
+    load(std::false_type{});
+  }
+}
+
 // FP8: caches are e4m3 rows of fp8_row_bytes(DH) = DH bytes + f32
 // scale (+pad): decode attention is KV-bandwidth bound at long context,
 // so halving cache bytes halves the dominant stream AND doubles KV
 // capacity within 288 GB. Dequant rides
 // v_cvt_pk_f32_fp8 in the inner loop.
+//
+// BS: tokens of a block, where that is known (0: any number). With it the first form's
+// two kinds of loads fit the 64 registers of eight waves a SIMD.
 template <int DH, int G, bool SPLIT, bool FP8 = false, int WAVES = NW,
-          int PER_SIMD = 1, bool ONCE = !FP8 && G < NW>
+          int PER_SIMD = 1, bool ONCE = false, int BS = 0>
 __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k_cache,
     const uint16_t *__restrict__ v_cache, const int32_t *__restrict__ block_tables,
     const int32_t *__restrict__ seq_lens,
     const int32_t *__restrict__ seq_starts, uint16_t *__restrict__ out,
     uint16_t *__restrict__ out_swz,
-    float *__restrict__ partial, int hkv, int bs, int max_blocks, int nsplit,
-    float scale, bool sorted) {
+    float *__restrict__ partial, int hkv, int block_size, int max_blocks,
+    int nsplit, float scale, bool sorted) {
+  const int bs = BS != 0 ? BS : block_size;
   // Lane-group geometry: GL lanes cover one token's Dh. bf16 reads 2 B
   // per element, so 16 lanes x VE=DH/16 elems = 16 B/lane; fp8 reads
   // 1 B per element, so 8-lane groups with VE=DH/8 keep the loads at
@@ -266,12 +354,26 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
   constexpr int BT_LDS = 512;
   __shared__ int32_t bt_lds[BT_LDS];
   const int blk0 = t_begin / bs;
-  if (t_begin < t_end) {
-    const int nbt = min((t_end - 1) / bs - blk0 + 1, BT_LDS);
+  const int nbt =
+      t_begin < t_end ? min((t_end - 1) / bs - blk0 + 1, BT_LDS) : 0;
+  __shared__ Shared shared;
+  auto numbers = [&] {
     for (int i = (int)threadIdx.x; i < nbt; i += WAVES * 64)
       bt_lds[i] = bt[blk0 + i];
+  };
+  if constexpr (ONCE) {
+    const Shared::Ask ask(block_tables, seq_lens, max_blocks, b, blk0,
+                          nbt);
+    numbers();
+    shared.before(ask, block_tables, seq_lens, max_blocks, bs, b, blk0, nbt);
+  } else {
+    numbers();
   }
   __syncthreads();
+  int alone = 0;                           // from this token on
+  if constexpr (ONCE)
+    alone = (blk0 + shared.after<WAVES * 64>(block_tables, seq_lens, max_blocks,
+                                             bs, blk0, nbt, bt_lds)) * bs;
 
   // Software-pipelined KV stream: the K/V rows of later steps are issued as
   // RAW bytes while one is computed. (Converting at load time puts an
@@ -301,40 +403,48 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
   uint32_t kraw[DEPTH][TPS][RW], vraw[DEPTH][TPS][RW];
   float kscale[DEPTH][TPS], vscale[DEPTH][TPS];
 
+  const int uw = __builtin_amdgcn_readfirstlane(wid);
   auto fetch = [&](int i, int slot) {
+    auto load = [&](auto past) {
+      constexpr bool PAST = decltype(past)::value;
 #pragma unroll
-    for (int u = 0; u < TPS; ++u) {
-      const int tt = min(t_base + i * stride + u * TPW, t_end - 1);
-      const int bi = tt / bs - blk0;
-      const int blk = (bi < BT_LDS) ? bt_lds[bi] : bt[tt / bs];
-      if (FP8) {
-        constexpr int RB8 = DH + 16;
-        const uint8_t *k8 = reinterpret_cast<const uint8_t *>(k_cache);
-        const uint8_t *v8 = reinterpret_cast<const uint8_t *>(v_cache);
-        const int64_t row =
-            (((int64_t)blk * hkv + h_kv) * bs + (tt % bs)) * RB8;
-#pragma unroll
-        for (int c = 0; c < VE; c += CH) {
-          rb::ld_words<CH / 4>(kraw[slot][u] + c / 4, k8 + row + column(c));
-          rb::ld_words<CH / 4>(vraw[slot][u] + c / 4, v8 + row + column(c));
+      for (int u = 0; u < TPS; ++u) {
+        const int tt = min(t_base + i * stride + u * TPW, t_end - 1);
+        const int bi = (unsigned)tt / (unsigned)bs - blk0;
+        int blk = bt_lds[min(bi, BT_LDS - 1)];
+        if (bi >= BT_LDS) {
+          blk = bt[blk0 + bi];
+          asm volatile("" : "+v"(blk));
         }
-        kscale[slot][u] = *reinterpret_cast<const float *>(k8 + row + DH);
-        vscale[slot][u] = *reinterpret_cast<const float *>(v8 + row + DH);
-      } else {
-        const int64_t base =
-            (((int64_t)blk * hkv + h_kv) * bs + (tt % bs)) * DH + d0;
+        const unsigned head = (unsigned)blk * (unsigned)hkv + h_kv;
+        const int64_t row = (int64_t)head * bs + (unsigned)tt % (unsigned)bs;
+        const uint8_t *k = reinterpret_cast<const uint8_t *>(k_cache);
+        const uint8_t *v = reinterpret_cast<const uint8_t *>(v_cache);
+        if constexpr (FP8) {
+          const int64_t at = row * (DH + 16);
 #pragma unroll
-        for (int c = 0; c < VE; c += CH)
-          rb::ld_words<CH / 2, ONCE>(
-              kraw[slot][u] + c / 2,
-              reinterpret_cast<const uint8_t *>(k_cache + base) + c * GL * 2);
+          for (int c = 0; c < VE; c += CH) {
+            rb::ld_words<CH / 4>(kraw[slot][u] + c / 4, k + at + column(c));
+            rb::ld_words<CH / 4>(vraw[slot][u] + c / 4, v + at + column(c));
+          }
+          kscale[slot][u] = *reinterpret_cast<const float *>(k + at + DH);
+          vscale[slot][u] = *reinterpret_cast<const float *>(v + at + DH);
+        } else {
+          const int64_t at = (row * DH + d0) * 2;
 #pragma unroll
-        for (int c = 0; c < VE; c += CH)
-          rb::ld_words<CH / 2, ONCE>(
-              vraw[slot][u] + c / 2,
-              reinterpret_cast<const uint8_t *>(v_cache + base) + c * GL * 2);
+          for (int c = 0; c < VE; c += CH)
+            rb::ld_words<CH / 2, PAST>(kraw[slot][u] + c / 2,
+                                       k + at + c * GL * 2);
+#pragma unroll
+          for (int c = 0; c < VE; c += CH)
+            rb::ld_words<CH / 2, PAST>(vraw[slot][u] + c / 2,
+                                       v + at + c * GL * 2);
+        }
       }
-    }
+    };
+    const int first = t_begin + (HS ? 0 : uw * TPW * TPS) + i * stride;
+    if constexpr (ONCE) by_policy(first >= alone, load);
+    else load(std::false_type{});
   };
 
   // cur is a compile-time constant at every call site below, so the
@@ -575,8 +685,20 @@ __global__ __launch_bounds__(WAVES * 64, DH == 256 ? 2 : 4) void paged_decode8_k
   constexpr int BT_LDS = 512;
   __shared__ int32_t bt_lds[BT_LDS];
   const int lo = t_begin / BS, hi = t_end > t_begin ? (t_end - 1) / BS : lo - 1;
-  for (int i = (int)threadIdx.x; i < min(hi - lo + 1, BT_LDS); i += WAVES * 64)
-    bt_lds[i] = bt[lo + i];
+  const int staged = min(hi - lo + 1, BT_LDS);
+  __shared__ Shared shared;
+  auto numbers = [&] {
+    for (int i = (int)threadIdx.x; i < staged; i += WAVES * 64)
+      bt_lds[i] = bt[lo + i];
+  };
+  if constexpr (ONCE) {
+    const Shared::Ask ask(block_tables, seq_lens, max_blocks, b, lo,
+                          staged);
+    numbers();
+    shared.before(ask, block_tables, seq_lens, max_blocks, BS, b, lo, staged);
+  } else {
+    numbers();
+  }
 
   unsigned qpk[G][VE / 2];              // the rows' own bits; scaled in fp32
 #pragma unroll
@@ -596,6 +718,10 @@ __global__ __launch_bounds__(WAVES * 64, DH == 256 ? 2 : 4) void paged_decode8_k
   // for the blocks that are on their way
   __builtin_amdgcn_s_waitcnt(0x0f70);             // vmcnt(0)
   __syncthreads();
+  int alone = 0;                                  // from this block on
+  if constexpr (ONCE)
+    alone = lo + shared.after<WAVES * 64>(block_tables, seq_lens, max_blocks, BS,
+                                          lo, staged, bt_lds);
 
   const unsigned mine = wid * (R::AHEAD * R::STAGE);
   const unsigned ring =
@@ -610,23 +736,28 @@ __global__ __launch_bounds__(WAVES * 64, DH == 256 ? 2 : 4) void paged_decode8_k
     }
     return __builtin_amdgcn_readfirstlane(blk);
   };
-  auto fetch = [&](int bi, int stage) {
+  auto send = [&](int bi, int stage, auto past) {
+    constexpr bool PAST = decltype(past)::value;
     const int64_t at = ((int64_t)block_of(bi) * hkv + h_kv) * R::PART;
     const uint8_t *k = k_cache + at, *v = v_cache + at;
     const unsigned to =
         __builtin_amdgcn_readfirstlane(ring + stage * R::STAGE);
 #pragma unroll
     for (int i = 0; i < R::FULL; ++i)
-      rb::lds_load_from<ONCE>(k + i * 1024 + lane * 16, to + i * 1024);
+      rb::lds_load_from<PAST>(k + i * 1024 + lane * 16, to + i * 1024);
     // the last 16 pieces of K and the first of V
     if (lane < 32)
-      rb::lds_load_from<ONCE>(
+      rb::lds_load_from<PAST>(
           (lane < 16 ? k + R::FULL * 1024 : v - 256) + lane * 16,
           to + R::FULL * 1024);
 #pragma unroll
     for (int i = 0; i < R::FULL; ++i)
-      rb::lds_load_from<ONCE>(v + 256 + i * 1024 + lane * 16,
+      rb::lds_load_from<PAST>(v + 256 + i * 1024 + lane * 16,
                               to + R::PART + 256 + i * 1024);
+  };
+  auto fetch = [&](int bi, int stage) {
+    if (ONCE && bi >= alone) send(bi, stage, std::true_type{});
+    else send(bi, stage, std::false_type{});
   };
 
   float m[G], l[G], acc[G][VE];         // maxima in exponents of 2
@@ -965,13 +1096,27 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
   constexpr int BT_LDS = 512;
   __shared__ int32_t bt_lds[BT_LDS];
   const int blk0 = t_begin / BS;
-  if (t_begin < t_end) {
-    const int nbt = min((t_end - 1) / BS - blk0 + 1, BT_LDS);
+  const int nbt =
+      t_begin < t_end ? min((t_end - 1) / BS - blk0 + 1, BT_LDS) : 0;
+  __shared__ Shared shared;
+  auto numbers = [&] {
     for (int i = tid; i < nbt; i += BLOCK) bt_lds[i] = bt[blk0 + i];
+  };
+  if constexpr (!FP8) {
+    const Shared::Ask ask(block_tables, seq_lens, max_blocks, b, blk0,
+                          nbt);
+    numbers();
+    shared.before(ask, block_tables, seq_lens, max_blocks, BS, b, blk0, nbt);
+  } else {
+    numbers();
   }
   // cross-wave merge region
   __shared__ float mlds[NW][G][DH + 2];
   __syncthreads();
+  int alone = 0;                          // from this block on
+  if constexpr (!FP8)
+    alone = blk0 + shared.after<BLOCK>(block_tables, seq_lens, max_blocks, BS,
+                                       blk0, nbt, bt_lds);
 
   // Q fragments (B of the swapped QK^T); head = i16.
   rb_bf16x8v qf[KS32];
@@ -1038,16 +1183,20 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
       // v block is [DH][BS] (transposed layout)
       const uint8_t *vb = reinterpret_cast<const uint8_t *>(
           v_cache + vblk * DH * BS);
+      auto load = [&](auto past) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int ks = 0; ks < KS32; ++ks)
-          rb::ld_words<4, true>(kfr[slot][t][ks],
-                          kb + ((krow + 4 * t) * DH + ks * 32 + h16 * 8) * 2);
+          for (int ks = 0; ks < KS32; ++ks)
+            rb::ld_words<4, decltype(past)::value>(
+                kfr[slot][t][ks],
+                kb + ((krow + 4 * t) * DH + ks * 32 + h16 * 8) * 2);
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-        rb::ld_words<4, true>(vfr[slot][dt],
-                        vb + ((dt * 16 + i16) * BS + tok0) * 2);
+        for (int dt = 0; dt < DT; ++dt)
+          rb::ld_words<4, decltype(past)::value>(
+              vfr[slot][dt], vb + ((dt * 16 + i16) * BS + tok0) * 2);
+      };
+      by_policy(bi >= alone, load);
     }
   };
 
@@ -1130,7 +1279,7 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_mfma_kernel(
           frag(vfr[cur][dt]), pf.v, acc_o[dt], 0, 0, 0);
   };
 
-  const int bi0 = blk_lo + 2 * wid;
+  const int bi0 = blk_lo + 2 * __builtin_amdgcn_readfirstlane(wid);
   if (bi0 <= blk_hi) fetch(bi0, 0);
   for (int bi = bi0; bi <= blk_hi; bi += 2 * PAIR) {
     step(bi, 0);
@@ -1266,14 +1415,14 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
                        splits > 1 ? nullptr : swz, partial, hkv, bs, max_blocks,
                        splits, scale, sorted);
   };
-  // Keys and values go past L2's older lines: in a step they are read once (ONCE;
-  // us of caches that lie in memory, without and with it: 32 sequences of 129 to 2015
-  // tokens, 32 heads of 128 104 and 92, 4 of 4000 54 and 49, one of 701 10.9 and 10.2,
-  // of 37 4.8 and 4.5; 64 of 37 to 1400, 12 heads of 64 30.9 and 28.0). Heads of 64 are
-  // those of small models, whose caches a few sequences leave in L2 from step to step:
-  // there not, as far as a layer's table has room for no more than L2's 32 MB (one of
-  // 37 tokens, 12 heads 3.6 and 3.9).
-  constexpr bool EITHER = DH == 64 && !FP8 && G < NW;
+  // Keys and values go past L2's older lines, as in a step a sequence's are read once
+  // (ONCE; us of caches that lie in memory, without and with it: 32 sequences of 129 to
+  // 2015 tokens, 32 heads of 128 104 and 92, 4 of 4000 54 and 49, one of 701 10.9 and
+  // 10.2, of 37 4.8 and 4.5; 64 of 37 to 1400, 12 heads of 64 30.9 and 28.0). What
+  // sequences share does not (Shared). Heads of 64 are those of small models, whose
+  // caches a few sequences leave in L2 from step to step: there not, as far as a
+  // layer's table has room for no more than L2's 32 MB (one of 37 tokens, 12 heads 3.6
+  // and 3.9).
   const bool once = DH != 64 || (int64_t)B * hkv * longest *
                                         (FP8 ? DH + 16 : DH * 2) * 2 >
                                     ((int64_t)32 << 20);
@@ -1328,6 +1477,17 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
       return;
     }
   }
+  // blocks of 16 tokens, as caches have them, or any
+  auto by_block = [&](auto launch) {
+    using Any = std::integral_constant<int, 0>;
+    using Sixteen = std::integral_constant<int, 16>;
+    if constexpr (!FP8 && G < NW) {
+      if (bs == 16 && once) return launch(std::true_type{}, Sixteen{});
+      if constexpr (DH == 64)
+        if (bs == 16) return launch(std::false_type{}, Sixteen{});
+    }
+    launch(std::false_type{}, Any{});
+  };
   if constexpr (G < NW) {
     // Whole sequences by 8 waves: of a short one more have nothing to do, and a CU
     // has room for more workgroups (which is why one query head a kv head keeps
@@ -1350,36 +1510,32 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
     const int64_t base = (int64_t)B * hkv;
     if constexpr (ROOM == 8 && DH == 128)
       if (nsplit <= 1 && longest > 512 && base <= 512)
-        return go(paged_decode_kernel<DH, G, false, FP8, 16, ROOM>, 16, 1,
-                  nullptr);
+        return by_block([&](auto past, auto block) {
+          go(paged_decode_kernel<DH, G, false, FP8, 16, ROOM,
+                                 decltype(past)::value, decltype(block)::value>,
+             16, 1, nullptr);
+        });
     const bool many = (FP8 || G > 1) && base > (DH == 64 ? 1023 : 512);
-    if (nsplit <= 1 && longest > 64 && !many) {
-      if constexpr (EITHER)
-        if (!once)
-          return go(paged_decode_kernel<DH, G, false, FP8, 8, ROOM, false>, 8,
-                    1, nullptr);
-      return go(paged_decode_kernel<DH, G, false, FP8, 8, ROOM>, 8, 1, nullptr);
-    }
+    if (nsplit <= 1 && longest > 64 && !many)
+      return by_block([&](auto past, auto block) {
+        go(paged_decode_kernel<DH, G, false, FP8, 8, ROOM, decltype(past)::value,
+                               decltype(block)::value>,
+           8, 1, nullptr);
+      });
   }
-  if (nsplit <= 1) {
-    if constexpr (EITHER)
-      if (!once)
-        return go(paged_decode_kernel<DH, G, false, FP8, NW, 1, false>, NW, 1,
-                  nullptr);
-    return go(paged_decode_kernel<DH, G, false, FP8>, NW, 1, nullptr);
-  }
+  if (nsplit <= 1)
+    return by_block([&](auto past, auto block) {
+      go(paged_decode_kernel<DH, G, false, FP8, NW, 1, decltype(past)::value,
+                             decltype(block)::value>,
+         NW, 1, nullptr);
+    });
   auto partial = at::empty({B, Hq, nsplit, DH + 2},
                            q.options().dtype(at::kFloat));
-  bool gone = false;
-  if constexpr (EITHER)
-    if (!once) {
-      go(paged_decode_kernel<DH, G, true, FP8, NW, 1, false>, NW, nsplit,
-         partial.data_ptr<float>());
-      gone = true;
-    }
-  if (!gone)
-    go(paged_decode_kernel<DH, G, true, FP8>, NW, nsplit,
-       partial.data_ptr<float>());
+  by_block([&](auto past, auto block) {
+    go(paged_decode_kernel<DH, G, true, FP8, NW, 1, decltype(past)::value,
+                           decltype(block)::value>,
+       NW, nsplit, partial.data_ptr<float>());
+  });
   hipLaunchKernelGGL((decode_combine_kernel<DH / 64>),
                      dim3(B * Hq), dim3(64), 0, stream,
                      partial.data_ptr<float>(), (uint16_t *)out.data_ptr(), swz,

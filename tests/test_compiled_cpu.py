@@ -81,3 +81,16 @@ def test_blocks_of_8_bits_stay_on_their_way(tmp_path):
         assert not any(op.startswith("flat_load") for op, _ in code)
         seen += 1
     assert seen > 0
+
+
+def test_loads_of_both_kinds(tmp_path):
+    """Past L2 and not: two loads that differ in that alone are one to the compiler
+    where it may have them so, and neither."""
+    seen = 0
+    for code in _kernels(tmp_path, "paged_decode_(?:mfma_)?kernel"):
+        wide = [args.split()[-1] == "nt" for op, args in code
+                if op == "global_load_dwordx4"]
+        if any(wide):
+            assert 3 * wide.count(False) > wide.count(True) > wide.count(False) / 3
+            seen += 1
+    assert seen > 0

@@ -159,15 +159,27 @@ template <bool FP8> struct Step {
   bf16x8v x[X];
 };
 
-// Steps s0 .. s1 - 1 by two chunks of U in turn. BOTH: both are on their way before
-// `meanwhile` waits for anything; of 17 to 32 rows, whose chunks are long, that costs
-// 1 to 3%.
-template <bool BOTH, int U, typename Step, typename Load, typename Multiply,
-          typename Meanwhile>
+// Steps s0 .. s1 - 1 by two chunks of U in turn.
+//
+// BOTH: both are on their way before `meanwhile` waits for anything, and what is past
+// the end is not loaded behind the first two; of 17 to 32 rows, whose chunks are long,
+// that costs 1 to 3%. APART: loads and products stay in this order. Left to itself the
+// compiler puts the loads of the loop behind all of its products, so that none is on
+// its way meanwhile.
+template <bool BOTH, bool APART, int U, typename Step, typename Load,
+          typename Multiply, typename Meanwhile>
 __device__ __forceinline__ void stream_chunks(Step (&a)[U], Step (&b)[U],
                                               int s0, int s1, Load load,
                                               Multiply multiply,
                                               Meanwhile meanwhile) {
+  auto apart = [] {
+    if (APART) __builtin_amdgcn_sched_barrier(0);
+  };
+  auto up_to_end = [&](Step (&c)[U], int s) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (s + u < s1) multiply(c[u]);
+  };
   if (s0 < s1) {
     load(a, s0);
     if (BOTH) load(b, s0 + U);
@@ -175,22 +187,33 @@ __device__ __forceinline__ void stream_chunks(Step (&a)[U], Step (&b)[U],
   meanwhile();
   if (s0 >= s1) return;
   int s = s0;
-  for (; s + 2 * U < s1; s += 2 * U) {
+  for (; s + (BOTH ? 3 : 2) * U < s1; s += 2 * U) {
     if (!BOTH) load(b, s + U);
 #pragma unroll
     for (int u = 0; u < U; ++u) multiply(a[u]);
+    apart();
     load(a, s + 2 * U);
+    apart();
 #pragma unroll
     for (int u = 0; u < U; ++u) multiply(b[u]);
+    apart();
     if (BOTH) load(b, s + 3 * U);
+    apart();
+  }
+  if (BOTH && s + 2 * U < s1) {                    // three chunks are left
+#pragma unroll
+    for (int u = 0; u < U; ++u) multiply(a[u]);
+    apart();
+    load(a, s + 2 * U);
+    apart();
+#pragma unroll
+    for (int u = 0; u < U; ++u) multiply(b[u]);
+    up_to_end(a, s + 2 * U);
+    return;
   }
   if (!BOTH) load(b, s + U);
-#pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (s + u < s1) multiply(a[u]);
-#pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (s + U + u < s1) multiply(b[u]);
+  up_to_end(a, s);
+  up_to_end(b, s + U);
 }
 
 // W nontemporal (streamed once, must not evict L2); x plain (re-read by every
@@ -251,7 +274,7 @@ __device__ __forceinline__ void weight_stream(
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w.v, c.x[0], acc, 0, 0, 0);
     }
   };
-  stream_chunks<false>(a, b, s0, s1, load, multiply, meanwhile);
+  stream_chunks<false, false>(a, b, s0, s1, load, multiply, meanwhile);
 #pragma unroll
   for (int r = 0; r < 16; ++r)
     red[wid][(r & 3) + 8 * (r >> 2) + 4 * hi][col] = acc[r];
@@ -261,13 +284,17 @@ __device__ __forceinline__ void weight_stream(
 // x, so half as many loads of x go with one of W. A step is two kilobytes of W, 32
 // columns (e4m3: 64), its operands as in decode_res.hip.
 //
-// With that, what the ends need behind two chunks of W in place of one, and the scales
-// of W's rows loaded ahead of it and not behind it, us in a graph with the norm left out
-// of x and the ends, of 1 and 16 rows before and now: 12288 x 4096 and rotation 20.3 and
-// 19.3, 21.1 and 20.2 (W alone takes 17.8); 6144 x 4096 11.7 and 11.2, 12.4 and 11.9;
-// 22016 x 4096 and unit 31.4 and 30.7, 32.4 and 31.3 (29.3); 49152 x 3072 47.9 and
-// 46.8, 46.2 and 44.5; in e4m3 12288 x 4096 14.4 and 12.7, 14.4 and 13.4 (9.5), 22016 x
-// 4096 20.4 and 17.3, 20.9 and 19.6 (16).
+// us in a graph with the norm left out of x and the ends, of 1 and 16 rows, by products
+// of 32 x 32 with the ends behind one chunk of W, and so: 12288 x 4096 and rotation 20.1
+// and 19.3, 21.0 and 20.3 (W alone takes 17.8); 6144 x 4096 11.8 and 11.2, 12.4 and 11.7;
+// 22016 x 4096 and unit 32.1 and 31.0, 32.5 and 31.2 (29.3); 49152 x 3072 46.0 and 45.1,
+// 46.0 and 44.4; in e4m3 12288 x 4096 14.0 and 11.6, 14.6 and 13.0 (9.5), 22016 x 4096
+// 20.4 and 16.9, 19.4 and 17.7 (16).
+// In e4m3, whose conversions the compiler gathers with the products, loads are kept apart
+// from these (APART; 9 to 16 rows of 12288 x 3072 11.4 us by 32 x 32, 11.8 with loads
+// behind the products, 10.7 apart and with nothing loaded past the end). In bf16 they
+// stand behind a loop's products as compiled, 24 loads after a wait for all: apart, q, k
+// and v take 1 to 6% less and heads of 128256 rows 1 to 3% more.
 template <bool FP8, typename Meanwhile>
 __device__ __forceinline__ void weight_stream16(
     const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws, int M,
@@ -318,7 +345,7 @@ __device__ __forceinline__ void weight_stream16(
       }
     }
   };
-  stream_chunks<true>(a, b, s0, s1, load, multiply, meanwhile);
+  stream_chunks<true, FP8>(a, b, s0, s1, load, multiply, meanwhile);
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -744,7 +771,13 @@ static void launch(Kind kind, const at::Tensor &xs, const at::Tensor &ws,
       case ends::QKV: return go(decode_gemm_kernel<FP8, ends::QKV, FEW>);
     }
   };
-  if (M <= 16 && K % (FP8 ? 64 : 32) == 0) of(std::true_type{});
+  // Of e4m3 columns a wave has one chunk of these where there are up to 1024 of them, and
+  // its second one is loaded for nothing: no matter where a CU has no more than one
+  // workgroup (us of the products of 16 x 16 and of 32 x 32, 1024 columns: 4096 and 8192
+  // rows 4.4 and 4.6, 4.7 and 4.9; 49152 14.9 and 13.3)
+  const bool few = M <= 16 && K % (FP8 ? 64 : 32) == 0 &&
+                   (!FP8 || K > 1024 * split || N / 32 * split <= 256);
+  if (few) of(std::true_type{});
   else of(std::false_type{});
 }
 

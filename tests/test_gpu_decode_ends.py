@@ -75,7 +75,12 @@ def test_gated_unit(m, inter, k, parts, fp8, gelu):
 @pytest.mark.parametrize("m", [1, 15, 16, 17])
 @pytest.mark.parametrize("n,k,fp8", [
     (64, 1040, False), (64, 1056, False), (4096, 1088, False),
-    (64, 1056, True), (64, 1088, True), (4096, 4160, True), (96, 64, True)])
+    (64, 1056, True), (64, 1088, True), (4096, 4160, True), (96, 64, True),
+    # two to six chunks of a wave, whole and not, and e4m3 sums of one
+    (64, 1536, False), (64, 1568, False), (64, 2080, False), (64, 3072, False),
+    (64, 2048, True), (64, 2112, True), (64, 3072, True), (64, 3136, True),
+    (64, 4096, True), (64, 5184, True), (64, 6144, True), (8192, 1024, True),
+    (8224, 1024, True), (8224, 1088, True)])
 def test_few_rows(m, n, k, fp8):
     """Products of 16 x 16 and, of more rows or odd lengths of sums, of 32 x 32, whole
     and in parts, of fewer columns of x than there are waves too."""

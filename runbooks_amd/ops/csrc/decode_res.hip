@@ -36,7 +36,7 @@ struct Sum {
 
 // A workgroup takes 16 rows of W and all of their sums, so that nothing is left
 // to add up: of a width of 4096 that is a workgroup for every CU. Its eight
-// waves take parts of the sums, a kilobyte of W an instruction; B blocks of 16
+// waves take parts of the sums, U kilobytes of W at a time; B blocks of 16
 // rows of x (16x16x32 products: A[i=l&15][k=(l>>4)*8+e], B[k][j=l&15],
 // C[j=l&15][i=(l>>4)*4+r]). A lane's 16 bytes of e4m3 are of two products.
 //
@@ -48,9 +48,9 @@ struct Sum {
 //   3072 x 24576       34.9 31.5   34.2 33.7   39.7 45.7
 //   4096 x 4096  e4m3  10.1  5.6   11.2  6.7   12.4  8.1
 //   4096 x 11008 e4m3  16.0 12.3   16.4 13.0   18.4 17.8
-template <bool FP8, int B>
+template <bool FP8, int B, int U>
 __global__ __launch_bounds__(BLOCK, 1) void decode_res_kernel(Sum a) {
-  constexpr int X = FP8 ? 2 : 1, U = B == 1 ? 8 : 4;
+  constexpr int X = FP8 ? 2 : 1;
   const int tid = threadIdx.x;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, i16 = lane & 15, grp = lane >> 4;
@@ -356,8 +356,19 @@ std::vector<at::Tensor> decode_res(at::Tensor xs, at::Tensor ws,
     hipLaunchKernelGGL(kernel, dim3((unsigned)(N / 16)), dim3(BLOCK), 0,
                        at::cuda::getCurrentHIPStream(), a);
   };
-  if (M <= 16) fp8 ? go(decode_res_kernel<true, 1>) : go(decode_res_kernel<false, 1>);
-  else fp8 ? go(decode_res_kernel<true, 2>) : go(decode_res_kernel<false, 2>);
+  // Loads past the end of a wave's sums are made for nothing: of e4m3, whose waves have
+  // few steps, by six or by eight, as fewer are loaded (us by six and by eight, of one
+  // row and 2048, 4096, 5632, 11008 and 14336 columns, 4, 8, 11, 22 and 28 steps: 2048
+  // rows 3.9 4.2, -, 6.0 6.8, 4096 rows -, 6.2 5.6, -, 12.3 12.4, 13.1 13.9).
+  const int64_t steps = (K / 64 + WAVES - 1) / WAVES;
+  if (M > 16)
+    fp8 ? go(decode_res_kernel<true, 2, 4>) : go(decode_res_kernel<false, 2, 4>);
+  else if (!fp8)
+    go(decode_res_kernel<false, 1, 8>);
+  else if ((steps + 7) / 8 * 8 <= (steps + 5) / 6 * 6)
+    go(decode_res_kernel<true, 1, 8>);
+  else
+    go(decode_res_kernel<true, 1, 6>);
   return {out, y, squares};
 }
 

@@ -179,7 +179,8 @@ def test_heads(m, hq, hkv, dh, vt, fp8):
 
 @pytest.mark.parametrize("m", [1, 15, 16, 17, 32])
 @pytest.mark.parametrize("n,k", [(64, 64), (64, 2080), (4096, 4096),
-                                 (3072, 11008)])
+                                 (3072, 11008), (64, 3072), (64, 5632),
+                                 (64, 6208), (64, 14336)])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_residual_sum(m, n, k, fp8):
     e = ops.ext()

@@ -354,8 +354,12 @@ __device__ __forceinline__ void weight_stream16(
 }
 
 // FEW: up to 16 rows, K a multiple of 32 (e4m3: 64).
+// In bf16 the 32 x 32 kernel is kept to registers for three workgroups a CU, which it has
+// without being told in e4m3 (148): left alone it takes 176, room for two (us of 17 rows
+// with two and three, norm and ends included: 22016 x 4096 33.1 and 32.5, 6144 x 4096
+// 12.7 and 12.5, 36864 x 2048 29.1 and 28.1, 34816 x 1024 16.9 and 15.6).
 template <bool FP8, Kind KIND, bool FEW>
-__global__ __launch_bounds__(BLOCK, 1) void decode_gemm_kernel(
+__global__ __launch_bounds__(BLOCK, FEW || FP8 ? 1 : 3) void decode_gemm_kernel(
     const uint16_t *__restrict__ xs, const uint8_t *__restrict__ ws, int M,
     int N, int K, Ends e) {
   __shared__ __attribute__((aligned(16))) float red[4][32][FEW ? 17 : MMAX];

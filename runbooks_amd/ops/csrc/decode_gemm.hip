@@ -1059,13 +1059,25 @@ static void launch_rows(Kind kind, const at::Tensor &x, const at::Tensor &ws,
 // 32 and 30; 3072 x 24576 38 and 34, 50 and 41; 4096 x 4096 14 and 16, 17 and
 // 20; 22016 x 4096 of 64 rows 45 and 36, 12288 x 4096 25 and 26). Where four blocks
 // have up to half of the CUs take a second workgroup and the others none, two are
-// spread better, except that with more rows what x takes of a CU grows (four and two:
-// 36864 x 2048 of 17, 45 and 64 rows 35.4 and 30.5, 39.1 and 34.8, 40.6 and 37.2, of
-// 100 the same; 49152 x 3072 52.4 and 48.0, 56.7 and 52.9, 59.0 and 58.9, 67 and 72;
-// 65536 x 4096, two workgroups on every CU, 87 and 90, 88 and 96).
+// spread better, except that with more rows what x takes of a CU grows, the more the
+// longer they are. us of a gated unit (of a product as it is) with four and two blocks,
+// of 48 and 64 rows:
+//   34816 x  1024   22.8  20.4 ( 23.2  20.5)   23.8  21.8 ( 24.2  21.9)
+//   49152 x  2048   42.8  39.6 ( 44.1  39.8)   43.7  41.7 ( 44.8  42.8)
+//   49152 x  3072   56.8  54.3 ( 57.5  55.5)   59.0  57.4 ( 60.2  59.4)
+//   36864 x  4096   69.5  64.8 ( 69.8  66.0)   71.3  68.9 ( 71.7  70.5)
+//   40960 x  4096   70.9  67.0 ( 71.1  68.6)   72.6  71.3 ( 73.1  73.3)
+//   49152 x  4096   73.9  72.5 ( 74.6  75.1)   75.6  77.1 ( 77.0  80.9)
+//   43008 x  5120   87.1  83.3 ( 87.4  85.2)   91.2  92.2 ( 91.9  95.0)
+//   35840 x  6656  107.0  99.4 (107.3 100.5)  110.5 107.5 (111.2 109.9)
+//   44032 x  8192  134.1 124.7 (134.8 128.5)  138.2 136.0 (139.1 140.0)
+//   49152 x 12288  209.0 200.8 (212.7 206.9)  218.2 216.4 (221.5 226.1)
+// Of 17 rows two blocks take 3 to 15% less, of 100 the same or more, and two workgroups
+// on every CU have nothing to spread (65536 x 4096 of 45 rows 87 and 90).
 struct Cut { int blocks, split; };
 static Cut cut_of(int64_t M, int64_t N, int64_t K) {
-  const bool spill = M <= 64 && N > 32768 && N <= 49152;
+  const bool spill = M <= (K <= 3072 || N <= 36864 ? 64 : 48) && N > 32768 &&
+                     N <= 49152;
   Cut c{(N >= 20480 && !spill) || K >= (M <= 64 ? 20480 : 8192) ? 4 : 2, 1};
   const int64_t wgs = (N / 32 + c.blocks - 1) / c.blocks;
   while (c.split < 8 && wgs * c.split * 2 <= 256 && K / (c.split * 2) >= 256)

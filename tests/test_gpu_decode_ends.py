@@ -115,6 +115,14 @@ def test_wide_gated_unit_of_rows(m, inter):
     test_gated_unit_of_rows(m, inter, 1024)
 
 
+@pytest.mark.parametrize("m", [48, 49, 64])
+@pytest.mark.parametrize("inter,k", [(18432, 3072), (18432, 3104), (18448, 3072),
+                                     (18448, 3104)])
+def test_wide_gated_unit_of_long_rows(m, inter, k):
+    """Around the sizes from where on more than 48 rows have four all the same."""
+    test_gated_unit_of_rows(m, inter, k)
+
+
 def _heads_case(m, hq, hkv, dh, vt):
     n, k = (hq + 2 * hkv) * dh, 1056
     cos, sin = ops.rope_tables(dh, 50, device=DEV)

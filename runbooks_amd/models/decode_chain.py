@@ -110,13 +110,19 @@ def _heads(layer, y, m, cos, sin, positions, kc, vc, slots):
 
 def _gate_shares_x(c, m: int) -> bool:
     """shares_x of a gated unit, which the kernel whose waves share x also wins where it
-    is wider, unless the sums are short or it is wider still (us by operands and by
-    rows, of 17, 24 and 32 rows: 36864 x 2048 28.2 30.5, 28.2 31.1, 30.1 31.8; 49152 x
-    3072 48.0 47.5, 48.1 48.1, 52.2 48.7; 57344 x 8192 145.7 139.4, 145.8 139.8, 157.7
-    141.1; 65536 x 4096 83.5 85.6, 83.7 84.6, 90.5 84.5). Results in rows take the kernel
+    is wider, of more than 24 rows or of long sums. us by operands and by rows, of 17 to
+    24 and of 32 rows:
+      36864 x 3072  39.1 41.9  42.4 43.2    49152 x 4096  63.9 67.4  69.0 69.1
+      40960 x 3072  40.5 43.1  44.0 44.4    57344 x 4096  74.1 74.4  80.4 74.9
+      49152 x 3072  48.0 47.3  52.2 47.9    35840 x 6656  83.0 85.2  91.4 88.7
+      57344 x 3072  55.5 55.5  60.8 56.0    43008 x 5120  74.0 70.4  81.5 73.8
+      36864 x 4096  51.9 59.3  56.4 60.5    57344 x 5120  90.2 88.3  98.6 89.6
+      43008 x 4096  60.6 61.4  66.4 62.7    44032 x 8192 120.7 113.1 130.9 114.3
+    and of 65536 x 4096 83.5 and 84.6, 90.5 and 84.5. Results in rows take the kernel
     for operands 0.5 to 7 us more."""
     return c.shares_x(m) or (16 < m <= 32 and not c.fp8 and
-                             32768 < c.n <= 57344 and c.k >= 3072)
+                             43008 <= c.n <= 57344 and
+                             c.k >= (3072 if m > 24 else 5120))
 
 
 def _gated(layer, y, m, operand: bool):

@@ -289,12 +289,13 @@ def test_decode_step(monkeypatch, batch, kv, inter, hidden, eight_bit):
     assert _rel(got, ref.double()) < 2e-2
 
 
-@pytest.mark.parametrize("batch", [16, 17, 32])
-@pytest.mark.parametrize("inter,hidden,shared", [
-    (16400, 3072, True), (16400, 3040, False), (28672, 3072, True),
-    (28688, 3072, False)])
-def test_wide_gated_unit_of_a_step(monkeypatch, batch, inter, hidden, shared):
-    """As test_decode_step, around the sizes of wide gated units that take rows."""
+@pytest.mark.parametrize("batch", [16, 17, 24, 25, 32])
+@pytest.mark.parametrize("inter,hidden,first", [
+    (21488, 3072, 33), (21504, 3040, 33), (21504, 3072, 25), (28672, 3072, 25),
+    (28688, 3072, 33), (21504, 5088, 25), (21504, 5120, 17)])
+def test_wide_gated_unit_of_a_step(monkeypatch, batch, inter, hidden, first):
+    """As test_decode_step, around the sizes of wide gated units that take rows, from
+    `first` on."""
     from runbooks_amd.models import decode_chain
     m = _model(8, inter, hidden)
     args = _step(m, batch, False)
@@ -306,7 +307,7 @@ def test_wide_gated_unit_of_a_step(monkeypatch, batch, inter, hidden, shared):
     with torch.no_grad():
         monkeypatch.setattr(ops.ext(), "rows_glu", rows_glu)
         got = m.decode(*args)
-        assert len(seen) == (2 if batch > 16 and shared else 0)
+        assert len(seen) == (2 if batch >= first else 0)
         monkeypatch.setattr(decode_chain, "layers_of", lambda *a: None)
         ref = m.decode(*args)
     assert _rel(got, ref.double()) < 2e-2

@@ -110,19 +110,27 @@ def _heads(layer, y, m, cos, sin, positions, kc, vc, slots):
 
 def _gate_shares_x(c, m: int) -> bool:
     """shares_x of a gated unit, which the kernel whose waves share x also wins where it
-    is wider, of more than 24 rows or of long sums. us by operands and by rows, of 17 to
-    24 and of 32 rows:
-      36864 x 3072  39.1 41.9  42.4 43.2    49152 x 4096  63.9 67.4  69.0 69.1
-      40960 x 3072  40.5 43.1  44.0 44.4    57344 x 4096  74.1 74.4  80.4 74.9
-      49152 x 3072  48.0 47.3  52.2 47.9    35840 x 6656  83.0 85.2  91.4 88.7
-      57344 x 3072  55.5 55.5  60.8 56.0    43008 x 5120  74.0 70.4  81.5 73.8
-      36864 x 4096  51.9 59.3  56.4 60.5    57344 x 5120  90.2 88.3  98.6 89.6
-      43008 x 4096  60.6 61.4  66.4 62.7    44032 x 8192 120.7 113.1 130.9 114.3
-    and of 65536 x 4096 83.5 and 84.6, 90.5 and 84.5. Results in rows take the kernel
+    is wider: of more than 24 rows, unless rows of x begin a multiple of 2 kB apart (few of
+    L2's channels have them all) and there is not much of W; of fewer with long sums. us
+    by operands and by rows, of 24 and of 32 rows:
+      36864 x 3072  39.1 42.0  42.4 43.2    36864 x 3328  45.8 45.9  50.4 47.4
+      40960 x 3072  40.6 43.5  44.0 44.4    33792 x 3584  46.2 47.9  51.1 49.3
+      49152 x 3072  48.0 47.1  52.2 47.9    40960 x 3584  49.0 50.0  53.9 51.3
+      57344 x 3072  55.6 55.6  60.8 56.0    40960 x 3840  51.6 53.2  56.2 55.1
+      36864 x 4096  51.9 59.7  56.4 60.5    36864 x 4352  58.0 58.3  63.6 60.4
+      43008 x 4096  60.7 61.6  66.4 62.7    40960 x 4608  61.4 63.0  67.3 64.6
+      49152 x 4096  63.8 67.8  69.0 69.1    36864 x 5632  71.2 73.9  78.5 75.8
+      57344 x 4096  74.1 74.5  80.4 74.9    33792 x 6656  81.5 85.0  89.9 87.0
+      40960 x 5120  65.1 70.2  70.7 73.1    40960 x 6656  86.8 89.0  95.0 91.5
+      43008 x 5120  74.2 71.4  81.5 73.8    36864 x 6144  74.4 80.3  81.6 82.9
+      57344 x 5120  90.5 88.6  98.6 89.6    44032 x 8192 120.8 113.0 130.9 114.3
+    and of 65536 x 4096 83.7 and 84.6, 90.5 and 84.5. Results in rows take the kernel
     for operands 0.5 to 7 us more."""
-    return c.shares_x(m) or (16 < m <= 32 and not c.fp8 and
-                             43008 <= c.n <= 57344 and
-                             c.k >= (3072 if m > 24 else 5120))
+    wide = 16 < m <= 32 and not c.fp8 and 32768 < c.n <= 57344
+    if m <= 24:
+        return c.shares_x(m) or (wide and c.n >= 43008 and c.k >= 5120)
+    return c.shares_x(m) or (wide and c.k >= 3072 and
+                             (c.n >= 43008 or c.k % 1024 != 0))
 
 
 def _gated(layer, y, m, operand: bool):

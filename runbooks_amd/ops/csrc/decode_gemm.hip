@@ -1076,8 +1076,8 @@ static void launch_rows(Kind kind, const at::Tensor &x, const at::Tensor &ws,
 // on every CU have nothing to spread (65536 x 4096 of 45 rows 87 and 90).
 struct Cut { int blocks, split; };
 static Cut cut_of(int64_t M, int64_t N, int64_t K) {
-  const bool spill = M <= (K <= 3072 || N <= 36864 ? 64 : 48) && N > 32768 &&
-                     N <= 49152;
+  const bool spill = N > 32768 && N <= 49152 &&
+                     M <= (N <= 36864 || N * K <= 40960 * 4096 ? 64 : 48);
   Cut c{(N >= 20480 && !spill) || K >= (M <= 64 ? 20480 : 8192) ? 4 : 2, 1};
   const int64_t wgs = (N / 32 + c.blocks - 1) / c.blocks;
   while (c.split < 8 && wgs * c.split * 2 <= 256 && K / (c.split * 2) >= 256)

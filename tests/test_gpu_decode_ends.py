@@ -116,8 +116,9 @@ def test_wide_gated_unit_of_rows(m, inter):
 
 
 @pytest.mark.parametrize("m", [48, 49, 64])
-@pytest.mark.parametrize("inter,k", [(18432, 3072), (18432, 3104), (18448, 3072),
-                                     (18448, 3104)])
+@pytest.mark.parametrize("inter,k", [(18432, 4096), (18432, 6656), (20480, 4096),
+                                     (20480, 4128), (20496, 4096), (24576, 3408),
+                                     (24576, 3424)])
 def test_wide_gated_unit_of_long_rows(m, inter, k):
     """Around the sizes from where on more than 48 rows have four all the same."""
     test_gated_unit_of_rows(m, inter, k)
@@ -292,7 +293,8 @@ def test_decode_step(monkeypatch, batch, kv, inter, hidden, eight_bit):
 @pytest.mark.parametrize("batch", [16, 17, 24, 25, 32])
 @pytest.mark.parametrize("inter,hidden,first", [
     (21488, 3072, 33), (21504, 3040, 33), (21504, 3072, 25), (28672, 3072, 25),
-    (28688, 3072, 33), (21504, 5088, 25), (21504, 5120, 17)])
+    (28688, 3072, 33), (21504, 5088, 25), (21504, 5120, 17), (16400, 3584, 25),
+    (16400, 4096, 33), (16384, 3584, 17)])
 def test_wide_gated_unit_of_a_step(monkeypatch, batch, inter, hidden, first):
     """As test_decode_step, around the sizes of wide gated units that take rows, from
     `first` on."""

@@ -26,7 +26,9 @@ def _rel(a, b):
     (16, 32, 32, 128, 33, 1), (17, 32, 32, 128, 33, 1),
     (43, 24, 24, 64, 5, 1), (17, 64, 32, 128, 5, 1),
     # heads of 64 in tables of more than 32 MB, whole by 8 and by 4 waves
-    (43, 24, 24, 64, 8, 1), (90, 24, 24, 64, 4, 1)])
+    (43, 24, 24, 64, 8, 1), (90, 24, 24, 64, 4, 1),
+    # and of as many in e4m3, in parts too
+    (42, 24, 24, 64, 14, 1), (90, 24, 24, 64, 7, 1), (16, 24, 24, 64, 36, 3)])
 def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
     """By 4, 8 or 16 waves or in parts, with and without a window's start, and
     with sequences as short and as long as the table: the plain result but for
@@ -59,6 +61,69 @@ def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
             operand = ops.ext().decode_swizzle_x(got[0].view(batch, -1))
             assert torch.equal(got[1].view(-1, 32, 8)[:, :batch],
                                operand.view(-1, 32, 8)[:, :batch])
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("batch,hq,hkv,dh,blocks,nsplit,size", [
+    (3, 4, 4, 128, 9, 1, 8), (17, 32, 32, 128, 9, 1, 32), (2, 8, 4, 64, 40, 3, 32),
+    (43, 24, 24, 64, 5, 1, 8), (90, 24, 24, 64, 4, 1, 32), (3, 2, 2, 256, 40, 3, 32),
+    (3, 4, 2, 128, 300, 1, 4)])
+def test_blocks_of_other_sizes(batch, hq, hkv, dh, blocks, nsplit, size, fp8):
+    torch.manual_seed(size)
+    tokens = blocks * size
+    kc, vc = ops.alloc_kv_cache(batch * blocks, hkv, dh, DEV, dtype=torch.bfloat16,
+                                block_size=size, fp8=fp8)
+    k, v = (torch.randn(batch * tokens, hkv, dh, device=DEV).bfloat16()
+            for _ in "kv")
+    i32 = dict(dtype=torch.int32, device=DEV)
+    ops.kv_append(k, v, kc, vc, torch.arange(batch * tokens, **i32))
+    q = torch.randn(batch, hq, dh, device=DEV).bfloat16()
+    tables = torch.randperm(batch * blocks, device=DEV).to(torch.int32) \
+        .view(batch, blocks)
+    lens = torch.randint(1, tokens + 1, (batch,))
+    got = ops.ext().paged_decode_swz(q, kc, vc, tables, lens.to(**i32), nsplit,
+                                     dh ** -0.5, None)[0]
+    pick = sorted({0, batch // 2, batch - 1})
+    ref = ops.paged_decode_ref(q[pick].cpu(), kc.cpu(), vc.cpu(), tables[pick].cpu(),
+                               lens[pick], dh ** -0.5)
+    assert _rel(got[pick].cpu(), ref.double()) < 2 * BF16
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hq,hkv,dh", [(2, 2, 64), (4, 2, 64), (2, 2, 128),
+                                       (4, 2, 128), (1, 1, 256), (2, 1, 256),
+                                       (8, 2, 128)])
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_tokens_beside_one_that_jumps(hq, hkv, dh, nsplit, fp8):
+    """One token of every eight whose scores rise by 2.5 exponents of 2 a block, 10 and
+    more a step of a wave, which moves the maxima of all lane groups, while the others
+    rise by a quarter: their sums so far are scaled by 0.25 to 0.5 each time. All end as
+    high and are part of the result."""
+    torch.manual_seed(dh)
+    blocks = 40
+    t = torch.arange(blocks * 16, device=DEV)
+    left = blocks - 1 - t // 16
+    exponent = torch.where(t % 8 == 3, -2.5 * left, -0.25 * left)
+    exponent = exponent + torch.rand(len(t), device=DEV)
+    k = 0.3 * torch.randn(2 * len(t), hkv, dh, device=DEV)
+    k[..., 0] = (exponent * (0.6931 * dh ** 0.5)).repeat(2)[:, None]
+    v = torch.randn_like(k).bfloat16()
+    vt = hq // hkv >= 4
+    kc, vc = ops.alloc_kv_cache(2 * blocks, hkv, dh, DEV, dtype=torch.bfloat16,
+                                fp8=fp8, v_transposed=vt)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    ops.kv_append(k.bfloat16(), v, kc, vc, torch.arange(len(k), **i32))
+    q = 0.1 * torch.randn(2, hq, dh, device=DEV)
+    q[..., 0] = 1
+    q = q.bfloat16()
+    lens = torch.tensor([blocks * 16, blocks * 16 - 21])
+    tables = torch.arange(2 * blocks, **i32).view(2, blocks)
+    got = ops.ext().paged_decode_swz(q, kc, vc, tables, lens.to(**i32), nsplit,
+                                     dh ** -0.5, None)[0].cpu()
+    ref = ops.paged_decode_ref(q.cpu(), kc.cpu(), vc.cpu(), tables.cpu(), lens,
+                               dh ** -0.5)
+    for i in range(2):                  # 16-bit probabilities in matrix products
+        assert _rel(got[i], ref[i].double()) < (4 if vt else 2) * BF16
 
 
 @pytest.mark.parametrize("parts", [15, 16, 17, 64, 65, 81])

@@ -147,9 +147,9 @@ def _add(x, operand, copy, norm, rows: bool):
     ext, m = ops.ext(), x.shape[0]
     # the kernel whose workgroups have whole sums reads x once for 16 columns,
     # which is what it takes with many long rows (us in parts and whole, with
-    # the norm: 32 rows, 4096 x 4096 13.8 and 10.1, 4096 x 11008 23.8 and 24.0,
-    # 4096 x 14336 27.1 and 29.6, 3072 x 24576 39.7 and 45.7; 16 rows 13.2 and
-    # 8.4, 22.0 and 20.5, 25.4 and 24.2, 34.2 and 33.7); long ones are _in_parts'
+    # the norm: 32 rows, 4096 x 4096 13.8 and 10.3, 4096 x 11008 25.2 and 25.1,
+    # 4096 x 14336 29.7 and 33.5, 3072 x 24576 42.1 and 49.5; 16 rows 12.7 and
+    # 8.5, 22.3 and 21.0, 25.4 and 24.1, 37.2 and 37.6); long ones are _in_parts'
     if (m <= 16 or copy.k <= 8192) and \
             ext.decode_res_supported(m, copy.n, copy.k, copy.fp8):
         x, y, squares = ext.decode_res(operand, copy.ws, copy.scale, x,

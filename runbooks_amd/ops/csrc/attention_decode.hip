@@ -2,9 +2,11 @@
 //
 // The serving hot loop: memory-bound on the KV read (HBM3E gives 6.6 TB/s to
 // long reads that pass L2's older lines, 5.9 to others). Design, MI355X-first:
-//  * wave64 split into four 16-lane groups; each group owns ONE kv token
-//    per step at 8 (Dh=128) or 4 (Dh=64) elems/lane, so every wave streams
-//    4 contiguous KV rows per iteration at 16/8 B per lane.
+//  * wave64 split into lane groups, each of which owns one kv token at 16 bytes
+//    a lane and load: 16 lanes for rows of 256 and 512 bytes (heads of 128 and
+//    256), 8 for rows of 128 (heads of 64, up to two query heads a kv head) and
+//    for e4m3, so every wave streams 4 or 8 contiguous KV rows at a time. (Heads
+//    of 64 with four query heads or more keep 16 lanes of 8 bytes, for registers.)
 //  * GQA/MQA-native: a workgroup handles one (seq, kv_head); its G query
 //    heads share each K/V read (falcon-40b MQA G=16, llama2-70b G=8,
 //    llama2-7b MHA G=1).
@@ -95,12 +97,11 @@ RB_DEV Place shifted_place(const int32_t *lens, const int32_t *starts) {
 // with it. Up to 64 sequences, whose lengths one wave compares for all (B steps of
 // three instructions; all waves of a CU together took 0.8 us).
 //
-// us by shifts and sorted, with loads that stayed in L2 (launch_decode: 10% longer
-// than now), 32 heads of 128: 32 sequences of 129 to 2015 tokens 108
-// and 101 (5.6 TB/s), 16 of 800 to 3900 in e4m3 76 and 69, 64 of 100 to 1200 133 and
-// 124, 32 of 1072 each 104 and 104; 8 kv heads of 128 with four queries each: 64 of
-// 1000 to 4003 128 and 118 (5.7 TB/s), 32 of 100 to 4000 in two parts 61 and 55; 16
-// heads of 256: 7 of 90 to 1801 in parts 32.4 and 29.1, 16 of 100 to 2000 60 and 57.
+// us by shifts and sorted, 32 heads of 128: 32 sequences of 129 to 2015 tokens 101
+// and 94 (6.0 TB/s), 16 of 800 to 3900 in e4m3 66 and 62, 64 of 100 to 1200 120 and 113,
+// 32 of 1072 each 93.5 and 93.1; 8 kv heads of 128 with four queries each: 64 of 1000 to
+// 4003 122 and 106 (6.2 TB/s), 32 of 100 to 4000 in two parts 63 and 52; 16 heads of 256:
+// 7 of 90 to 1801 in parts 27.4 and 26.2, 16 of 100 to 2000 57.8 and 58.1.
 // Where nothing is uneven that cost 0.3 to 0.8 us, so lengths within 128 tokens of the
 // first one's go by shifts, and what a wave has loaded is not loaded again (us of a
 // table of 4096 by shifts alone, sorted, and so: 32 of 100 13.7, 14.4 and 13.9, 64 of
@@ -250,13 +251,13 @@ __global__ __launch_bounds__(WAVES * 64, PER_SIMD) void paged_decode_kernel(
     float *__restrict__ partial, int hkv, int block_size, int max_blocks,
     int nsplit, float scale, bool sorted) {
   const int bs = BS != 0 ? BS : block_size;
-  // Lane-group geometry: GL lanes cover one token's Dh. bf16 reads 2 B
-  // per element, so 16 lanes x VE=DH/16 elems = 16 B/lane; fp8 reads
-  // 1 B per element, so 8-lane groups with VE=DH/8 keep the loads at
-  // the full 16 B width (8 B accesses run 0.54-0.70x on gfx950 — the
-  // first fp8 cut used 16-lane groups and showed ZERO long-context win).
-  // (G > 4 keeps 16-lane groups even for fp8: qreg[G][VE]+acc[G][VE]
-  // at VE=16 would spill past 256 VGPRs)
+  // Lane-group geometry: GL lanes cover one token's Dh, with 16 B a lane and
+  // load (8 B accesses run 0.54-0.70x on gfx950 — the first fp8 cut used
+  // 16-lane groups and showed ZERO long-context win): 16 lanes for bf16 rows of
+  // heads of 128 and, by two loads, 256; 8 lanes for e4m3 rows, of 1 B an
+  // element, and for bf16 rows of heads of 64, of 128 B.
+  // (More query heads keep 16-lane groups, G > 4 for fp8 and G >= NW for heads
+  // of 64: qreg[G][VE]+acc[G][VE] of twice the VE would spill past 256 VGPRs)
   constexpr int GL = (FP8 && G <= 4) || (DH == 64 && G < NW) ? 8 : 16;
   constexpr int VE = DH / GL;              // elems per lane
   constexpr int TPW = 64 / GL;             // tokens per wave pass
@@ -947,12 +948,12 @@ __global__ __launch_bounds__(WAVES * 64, DH == 256 ? 2 : 4) void paged_decode8_k
   }
 }
 
-// Second pass for SPLIT mode: a workgroup of a wave merges the nsplit partials of one (b, hq)
-// row. Maxima and sums are one load of the wave (a lane a partial), and the rows (VE =
-// dh / 64 values a lane) are loaded 16 at a time beside it: one round trip to memory up
-// to 16 splits, where rows behind their weights made two (both kernels, one sequence of
-// 701 tokens, 32 heads, 12 splits: 10.2 us, 8.6 so, 8.0 and loops over the splits three per
-// split.
+// Second pass for SPLIT mode: a workgroup of one wave merges the nsplit partials of one
+// (b, hq) row. Maxima and sums are one load of the wave (a lane a partial), and the rows
+// (VE = dh / 64 values a lane) are loaded 16 at a time beside it: one round trip to memory
+// up to 16 splits. us of both kernels, one sequence of 701 tokens, 32 heads, 12 splits:
+// 10.2 with rows loaded by eights behind their weights, 8.6 with rows beside them and
+// four rows of the output a workgroup of four waves, 8.0 so.
 template <int VE>
 __global__ __launch_bounds__(64) void decode_combine_kernel(
     const float *__restrict__ partial, uint16_t *__restrict__ out,
@@ -1493,19 +1494,18 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
     // has room for more workgroups (which is why one query head a kv head keeps
     // to 64 registers, of 68). By 16 where long tables and few workgroups leave
     // the longest sequences to the end; by 4 where there are workgroups enough and
-    // 8 waves take too many registers (e4m3 107, two query heads 93).
-    // us by 4, 8 and 16 waves, with loads that stayed in L2, 32 heads of 128 in bf16:
-    // 32 sequences of 100 tokens
-    // 14.0, 13.7 and 17.3, of 300 31.9, 31.8 and 33.2, of 129 to 2015 111, 107 and
-    // 111, 4000 and 31 of 100 115, 69 and 58; 16 of 100 9.0, 9.3 and 10.3, of 800 to
-    // 3900 135, 120 and 117, 4000 and 15 of 100 111, 65 and 50; one of 100 5.8, 5.3
-    // and 6.1, of 512 13.2, 9.6 and 9.5; 12 heads of 64, 64 of 37 to 1400 33, 32 and
-    // 34. By 4 and 8 waves, e4m3: 32 of 100 11.0 and 14.9, of 50 to 1000 32.0 and
-    // 35.7, 64 of 300 34.9 and 40.4, of 1000 104 and 103, 16 of 1000 27.0 and 28.2,
-    // 4000 and 15 of 100 55 and 39; 12 heads of 64, 64 of 50 to 1000 20.9 and 18.8,
-    // 128 of them 28.8 and 29.2. 32 kv heads with two queries each, 64 sequences of
-    // 100 27 and 33, of 50 to 1000 113 and 108. 16 heads of 256, 40 sequences of 100
-    // 17.6 and 18.7, of 50 to 1000 84 and 73.
+    // 8 waves take too many registers (two query heads).
+    // us by 4, 8 and 16 waves, caches out of L2, 32 heads of 128 in bf16: 32 sequences of
+    // 100 tokens 13.9, 14.0 and 17.5, of 300 30.7, 30.6 and 33.1, of 129 to 2015 100, 94
+    // and 97, 4000 and 31 of 100 112, 64 and 49; 16 of 100 9.2, 9.3 and 9.6, of 800 to
+    // 3900 129, 103 and 102, 4000 and 15 of 100 109, 61 and 47; one of 100 6.1, 5.2 and
+    // 5.9, of 512 16.2, 10.6 and 10.1. By 4 and 8 waves: 12 heads of 64, 64 of 37 to 1400
+    // 32.0 and 28.5; 32 kv heads with two queries each, 64 of 100 25.3 and 31.5, of 50 to
+    // 1000 93 and 99; 16 heads of 256, 40 of 100 16.2 and 18.6, of 50 to 1000 62.4 and
+    // 59.3. e4m3 by whole blocks (above) has the same line: 32 heads of 128, 32 of 100
+    // 10.7 and 14.4, of 50 to 1000 31.6 and 34.5, 64 of 300 33.8 and 39.6, of 1000 99.9
+    // and 98.1, 16 of 1000 29.3 and 28.9, 4000 and 15 of 100 41.1 and 30.3; 12 heads of
+    // 64, 64 of 50 to 1000 16.4 and 18.8, 128 of them 30.7 and 30.6.
     constexpr int ROOM = !FP8 && G == 1 && DH <= 128 ? 8 : 1;
     const int64_t base = (int64_t)B * hkv;
     if constexpr (ROOM == 8 && DH == 128)
@@ -1556,18 +1556,31 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
 // batch takes about as long. In place of more parts it does not, and an engine's
 // tables are wide whatever the lengths.
 //
-// us in parts and whole, with loads that stayed in L2 and a merge that took 2 us
-// longer than now, 32 heads of 128 in bf16: one sequence of 200 tokens 9.1
-// and 7.1, of 512 9.8 and 9.5, of 1024 12.0 and 16.2; 4 of 512 13.8 and 12.2, one of
-// 512 and 3 of 50 10.1 and 10.5, one of 1024 and 3 of 50 12.7 and 16.6; 16 (two
-// parts) of 800 to 3900 122 and 123, 4000 and 15 of 100 63.7 and 54.3; 8 (four) of
-// 384 16.8 and 13.9, of 129 to 2015 34.5 and 34.4, 5 of 2000 and 3 that pad the batch
-// 38.2 and 33.4, 4000 and 7 of 100 35.8 and 47.3. e4m3: 16 (two) of 256 15.9 and 12.4,
-// of 800 to 3900 74.5 and 75.4, 4000 and 15 of 100 36.1 and 39.3; 8 (four) of 384 14.4
-// and 10.0, 4000 and 7 of 100 22.6 and 37.5. 16 heads of 256: 4 of 256 12.9 and 10.7,
-// one of 256 and 7 of 50 11.0 and 9.9, one of 512 and 7 of 50 12.2 and 15.2; 32 (two)
-// of 100 to 2000 110 and 108, 4000 and 31 of 100 79 and 84; 16 (four), 4000 and 15 of
-// 100 44 and 80.
+// us whole and in parts, caches out of L2, 32 heads of 128 in bf16, and in e4m3:
+//   one (16 parts at most)  100 tokens  5.2  7.0   5.4  6.8   256   7.3  7.2   6.2  6.8
+//                           384         9.0  7.4   7.1  7.1   512  10.6  7.6   7.8  7.2
+//                           768        12.7  8.3   9.3  8.2  1024  15.0  8.6  10.8  8.2
+//   two (16)                256         7.6  7.8   6.4  7.2   384   9.5  8.6   7.4  8.4
+//                           512        11.2  9.1   8.1  8.5  1024  16.1 11.8  11.2 10.7
+//   4 (8)                   256         8.1  9.2   6.9  8.6   512  12.1 11.8   8.6 10.6
+//                          1024        18.8 18.2  12.2 13.4
+//     1024 and 3 of 50                 15.6 11.0  11.1 10.6
+//   8 (4)                   256        10.0 11.7   8.2 10.9   512  15.3 17.6  10.9 13.6
+//                          1024        26.9 28.1  17.8 20.0
+//     129 to 2015                      31.8 30.0  21.4 21.6
+//     4000 and 7 of 100                45.5 35.6  29.5 17.6
+//   16 (2)                  256        15.5 17.6  11.3 13.8   512  26.2 28.8  17.4 20.2
+//     800 to 3900                       104  111  62.7 64.8
+//     4000 and 15 of 100               47.1 61.7  30.5 26.9
+// 16 heads of 256:
+//   one (16)                256         9.8  8.2   8.3  8.4   384  11.9  8.5  10.0  8.5
+//   8 (8)                   256        11.7 12.4   9.1 11.6   384  15.6 15.3  10.6 15.1
+//     512 and 7 of 50                  14.9 10.2  12.2 15.1
+//   16 (4)  4000 and 15 of 100         77.7 41.0  60.1 23.5
+//   32 (2)  100 to 2000                93.1 94.7  54.6 60.6
+//           4000 and 31 of 100         82.9 73.5  62.1 37.6
+// The lines lie where even batches of four and more have them. One or two sequences in
+// bf16 would gain 1 to 3 us in parts in tables of 384 to 512 tokens (256: 192 to 256).
 int64_t paged_decode_parts(int64_t nsplit, int64_t longest, int64_t dh,
                            int64_t group, bool transposed) {
   const int64_t parts =

@@ -24,7 +24,7 @@
 // Since then, with loads to LDS that the compiler does not wait for, operands read
 // ahead (flash_tile.h) and, of heads of 256, sums that stay in the matrix registers, on
 // another card: 7931 tokens 510 -> 491, 2048 of 32 heads 54 -> 49, 1021 of 32 heads
-// 22.7 -> 21.5; 16 heads of 256, 7931 713 -> 650, 3000 138 -> 129, 1021 36 -> 35. What is
+// 22.7 -> 21.5; 16 heads of 256, 7931 713 -> 632, 1021 36 -> 33 (add_products). What is
 // left: the two waves of a SIMD do the same at the same time, so that products and
 // vector instructions take turns (48% of the time each). Two groups of waves a half-step
 // apart, a barrier between half-steps, took as long: a half-step of products then waits

@@ -225,7 +225,8 @@ __device__ __forceinline__ void stream_chunks(Step (&a)[U], Step (&b)[U],
 //
 // Bound by the weight stream, and with 32 rows by x (as long as W, or twice as
 // long as e4m3). us before -> now, weights out of cache, for N x K of
-// 12288 x 4096, 22016 x 4096, 4096 x 4096 and 4096 x 11008:
+// 12288 x 4096, 22016 x 4096, 4096 x 4096 and 4096 x 11008 (up to 16 rows of such sizes
+// are weight_stream16's since; of 1 and 16 rows this is what it was chosen over):
 //   bf16  1 row    23.1 -> 20.0  36.9 -> 32.3  8.9 -> 8.2  21.3 -> 17.3
 //         16 rows  24.3 -> 22.5  37.5 -> 33.1  9.1 -> 8.6  21.6 -> 17.7
 //         32 rows  23.5 -> 23.6  37.5 -> 38.3  9.3 -> 9.3  21.9 -> 20.2

@@ -43,11 +43,11 @@ struct Sum {
 // Bound by the weight stream, by x with many long rows. us in a graph, weights
 // out of cache, in parts that the norm's kernel adds up, and here, of 1, 16 and
 // 32 rows:
-//   4096 x 4096        12.0  8.1   13.2  8.4   13.8 10.1
-//   4096 x 11008       21.0 19.1   22.0 20.5   23.8 24.0
-//   3072 x 24576       34.9 31.5   34.2 33.7   39.7 45.7
-//   4096 x 4096  e4m3  10.1  5.6   11.2  6.7   12.4  8.1
-//   4096 x 11008 e4m3  16.0 12.3   16.4 13.0   18.4 17.8
+//   4096 x 4096        11.8  7.7   12.7  8.5   13.8 10.3
+//   4096 x 11008       21.2 19.3   22.3 21.0   25.2 25.1
+//   3072 x 24576       34.5 31.9   37.2 37.6   42.1 49.5
+//   4096 x 4096  e4m3   8.8  5.7    9.8  6.1   11.6  8.3
+//   4096 x 11008 e4m3  14.0 12.5   15.0 13.0   18.4 18.0
 template <bool FP8, int B, int U>
 __global__ __launch_bounds__(BLOCK, 1) void decode_res_kernel(Sum a) {
   constexpr int X = FP8 ? 2 : 1;

@@ -21,9 +21,10 @@
 //   lora_down          19, 18, 7.7    19, 14, 6.5    -, 22, 11
 //   lora_add (columns) 26, 18, 18     53, 42, 42
 //   lora_down_columns  70, 13, 10     57, 25, 22     -, 7.2, 5.3
-//   dB and dA          96, 29, 23     71, 40, 32     -, 30, 21
+//   dB and dA          96, 29, 25     71, 40, 33     -, 30, 22
 //   lora_add (sum)     18, 8, 8       18, 8, 8
-// and no additions of dx, copies of t or transposes of A around them.
+// and no additions of dx, copies of t or transposes of A around them. (dB and dA take 2, 1
+// and 1.5 us less since rows of t and dt go to LDS past the registers, lora_grad_tile.)
 //
 // mfma layouts: 16x16x32 A[i=l&15][k=(l>>4)*8+e], B[k][j=l&15],
 // C[j=l&15][i=(l>>4)*4+r]; 32x32x16 as in flash_tile.h.

@@ -1464,10 +1464,15 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
           if (!once) return go8(part, waves, std::false_type{});
         go8(part, waves, std::true_type{});
       };
+      // By 8 waves where two workgroups a CU are all there are. With more the others
+      // would be begun when these end, and four of 4 waves fit a CU (us by 4 and 8, 12
+      // heads of 64: 64 sequences of 100 tokens 7.1 and 9.2, of 300 11.1 and 13.1, of 50 to
+      // 1000 17.0 and 19.5, 2000 and 63 of 100 20.7 and 14.7; by rows 7.8, 11.7, 18.6, 19.2;
+      // 43 sequences 6.6 8.6, 10.1 11.4, 13.9 14.2, 20.3 14.4 and 7.3, 10.4, 14.4, 17.6).
       using Four = std::integral_constant<int, 4>;
       using Most = std::integral_constant<int, DH == 256 ? 4 : 8>;
       if (splits > 1) by_cache(std::true_type{}, Four{});
-      else if (longest > 64 && (int64_t)B * hkv <= (DH == 64 ? 1023 : 512))
+      else if (longest > 64 && (int64_t)B * hkv <= 512)
         by_cache(std::false_type{}, Most{});
       else by_cache(std::false_type{}, Four{});
       if (splits > 1)
@@ -1502,10 +1507,9 @@ void launch_decode(const at::Tensor &q, const at::Tensor &k_cache,
     // 5.9, of 512 16.2, 10.6 and 10.1. By 4 and 8 waves: 12 heads of 64, 64 of 37 to 1400
     // 32.0 and 28.5; 32 kv heads with two queries each, 64 of 100 25.3 and 31.5, of 50 to
     // 1000 93 and 99; 16 heads of 256, 40 of 100 16.2 and 18.6, of 50 to 1000 62.4 and
-    // 59.3. e4m3 by whole blocks (above) has the same line: 32 heads of 128, 32 of 100
-    // 10.7 and 14.4, of 50 to 1000 31.6 and 34.5, 64 of 300 33.8 and 39.6, of 1000 99.9
-    // and 98.1, 16 of 1000 29.3 and 28.9, 4000 and 15 of 100 41.1 and 30.3; 12 heads of
-    // 64, 64 of 50 to 1000 16.4 and 18.8, 128 of them 30.7 and 30.6.
+    // 59.3. e4m3 by whole blocks (above): 32 heads of 128, 32 of 100 10.7 and 14.4, of 50
+    // to 1000 31.6 and 34.5, 64 of 300 33.8 and 39.6, of 1000 99.9 and 98.1, 16 of 1000
+    // 29.3 and 28.9, 4000 and 15 of 100 41.1 and 30.3.
     constexpr int ROOM = !FP8 && G == 1 && DH <= 128 ? 8 : 1;
     const int64_t base = (int64_t)B * hkv;
     if constexpr (ROOM == 8 && DH == 128)

@@ -29,7 +29,10 @@ def _rel(a, b):
     (43, 24, 24, 64, 8, 1), (90, 24, 24, 64, 4, 1),
     # and of as many in e4m3, in parts too
     (21, 24, 24, 64, 27, 1), (42, 24, 24, 64, 14, 1), (90, 24, 24, 64, 7, 1),
-    (16, 24, 24, 64, 36, 3)])
+    (16, 24, 24, 64, 36, 3),
+    # eight query heads by rows, numbers of blocks in LDS and past it
+    (5, 16, 2, 128, 33, 1), (2, 64, 8, 128, 40, 4), (3, 8, 1, 64, 33, 1),
+    (1, 8, 1, 128, 530, 1)])
 def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
     """By 4, 8 or 16 waves or in parts, with and without a window's start, and
     with sequences as short and as long as the table: the plain result but for
@@ -68,7 +71,7 @@ def test_whole_sequences(batch, hq, hkv, dh, blocks, nsplit, fp8):
 @pytest.mark.parametrize("batch,hq,hkv,dh,blocks,nsplit,size", [
     (3, 4, 4, 128, 9, 1, 8), (17, 32, 32, 128, 9, 1, 32), (2, 8, 4, 64, 40, 3, 32),
     (43, 24, 24, 64, 5, 1, 8), (90, 24, 24, 64, 4, 1, 32), (3, 2, 2, 256, 40, 3, 32),
-    (3, 4, 2, 128, 300, 1, 4)])
+    (3, 4, 2, 128, 300, 1, 4), (3, 16, 2, 128, 9, 1, 32)])
 def test_blocks_of_other_sizes(batch, hq, hkv, dh, blocks, nsplit, size, fp8):
     torch.manual_seed(size)
     tokens = blocks * size
